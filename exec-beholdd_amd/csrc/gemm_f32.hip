@@ -1,0 +1,285 @@
+// Matrix products of float32 operands on the float32 matrix instructions: C[M, N] (+)= A[M, K] W[N, K]^T, and the gated form
+// out[M, F] = act(A W[:F]^T) * (A W[F:]^T).  Every product is a 32-bit fused multiply-add with a 32-bit sum, as in the plain FMA
+// kernel (generic.hip); only the order of the sums differs, and it is blocked here as there.
+//
+// Two kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`.  More rows are
+// matrix-core work: `gemm_f32_tiles`.
+#include "common.h"
+#include "gemm_f32.h"
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+__device__ static inline floatx4 load4(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
+
+// ---- few rows ------------------------------------------------------------------------------------------
+// v_mfma_f32_4x4x1_16B multiplies 16 independent 4 x 4 blocks: lane 4 b + i holds row i of block b of either operand.  A block is
+// a slice of k here: lane 4 b + i loads 16 bytes of weight row i at k = k0 + 4 b, so that a wave's load covers four rows of 256
+// contiguous bytes, the next four products take their four elements in turn, and the 16 blocks' sums (every 16th group of four k)
+// are added at the end, then those of the workgroup's waves, which share K.  The activations are loaded the same way, from the L2.
+// Bound by the weights' stream; against 64 bits the sum of K terms is one of K / (16 WAVES) and one of 16 WAVES.
+// Measured at 4 rows: 1,024 x 3,072 in 6.2 us and 32,768 x 1,024 in 29 us (4.6 TB/s); the FMA tiles of generic.hip, whose
+// workgroups of 64 weight rows do 16 times the products and number 16 there, took 150 to 290 us.
+//   R: groups of four weight rows a wave, C: groups of four activation rows, WAVES: waves that share K.
+template <int R, int C, int WAVES, bool GATED>
+__global__ __launch_bounds__(64 * WAVES) void gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                  float* __restrict__ c, int M, int N, int K, int accumulate,
+                                                                  GateForm form) {
+  constexpr int GROUPS = GATED ? R / 2 : R;   // groups of outputs; GATED: the first half of the R groups are gates, the rest ups
+  constexpr int U = C >= 4 ? 2 : 4;           // chunks of 64 k whose loads are in flight together
+  __shared__ float sums[WAVES][R * C][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 3, b = lane >> 2;
+  const int n0 = blockIdx.x * 4 * GROUPS;
+  const float* w_row[R];
+  const float* a_row[C];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int n = min(n0 + 4 * (r % GROUPS) + i, N - 1);      // rows beyond the last one repeat it and are not written
+    w_row[r] = w + (size_t)(GATED && r >= GROUPS ? N + n : n) * K + 4 * b;
+  }
+#pragma unroll
+  for (int j = 0; j < C; ++j) a_row[j] = a + (size_t)min(4 * j + i, M - 1) * K + 4 * b;
+  floatx4 acc[R][C] = {};
+  int k0 = 64 * wave;
+  for (; k0 + 64 * WAVES * (U - 1) + 64 <= K; k0 += 64 * WAVES * U) {
+    floatx4 wv[U][R], av[U][C];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[u][r] = load4(w_row[r] + k0 + 64 * WAVES * u);
+#pragma unroll
+      for (int j = 0; j < C; ++j) av[u][j] = load4(a_row[j] + k0 + 64 * WAVES * u);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int j = 0; j < C; ++j) acc[r][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(wv[u][r][t], av[u][j][t], acc[r][j], 0, 0, 0);
+  }
+  for (; k0 < K; k0 += 64 * WAVES) {
+    const bool inside = k0 + 4 * b < K;       // K is a multiple of 4
+    floatx4 wv[R], av[C];
+#pragma unroll
+    for (int r = 0; r < R; ++r) wv[r] = inside ? load4(w_row[r] + k0) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < C; ++j) av[j] = inside ? load4(a_row[j] + k0) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < C; ++j) acc[r][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(wv[r][t], av[j][t], acc[r][j], 0, 0, 0);
+  }
+  // a lane's four numbers are rows 0..3 of its block's result, column i.  Over the blocks: halves of the lanes take half of the
+  // rows each, twice, then the rest of the blocks are added, so that lane 32 h + 16 q + .. + i holds row 2 h + q, column i.
+  const bool high = lane & 32, odd = lane & 16;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const floatx4 v = acc[r][j];
+      const float x0 = (high ? v[2] : v[0]) + __shfl_xor(high ? v[0] : v[2], 32, BH_WAVE);
+      const float x1 = (high ? v[3] : v[1]) + __shfl_xor(high ? v[1] : v[3], 32, BH_WAVE);
+      float x = (odd ? x1 : x0) + __shfl_xor(odd ? x0 : x1, 16, BH_WAVE);
+      x += __shfl_xor(x, 8, BH_WAVE);
+      x += __shfl_xor(x, 4, BH_WAVE);
+      if ((lane & 12) == 0) sums[wave][r * C + j][4 * (lane >> 4) + i] = x;
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < GROUPS * C * 16; e += 64 * WAVES) {
+    const int row = e % (4 * GROUPS), m = e / (4 * GROUPS);   // neighbouring threads: neighbouring outputs of one activation row
+    const int n = n0 + row;
+    if (n >= N || m >= M) continue;
+    const int place = 4 * (row % 4) + m % 4, at = (row / 4) * C + m / 4;
+    float v = 0.f;
+#pragma unroll
+    for (int s = 0; s < WAVES; ++s) v += sums[s][at][place];
+    if (GATED) {
+      float up = 0.f;
+#pragma unroll
+      for (int s = 0; s < WAVES; ++s) up += sums[s][at + GROUPS * C][place];
+      v = gate_mul(v, up, form);
+    }
+    const size_t to = (size_t)m * N + n;
+    c[to] = accumulate ? v + c[to] : v;
+  }
+}
+
+// ---- many rows -----------------------------------------------------------------------------------------
+// Four waves own 64 B x 64 B outputs (B = 1 or 2), a wave B x B tiles of v_mfma_f32_32x32x2_f32; a workgroup is one such group, or
+// KG of them that take the slices of k in turn (B = 1).  Slices of 32 k go through two LDS buffers, the next slice's loads on their way while one is multiplied.  A row of a slice takes 36 floats of
+// LDS, so that the 16-byte reads of 16 neighbouring rows fall on different banks; lane (row, half) reads four k at once and the
+// matrix instructions take k in that order, the same for both operands.  Every slice is summed on its own and then added.
+// Bound by the matrix instructions (64 cycles a tile and two k) where the tiles fill the chip.
+// Measured: 695 x 6,144 x 1,024 in 104 us (84 TFLOP/s), 2,048 x 32,768 x 1,024 in 1.12 ms (122 TFLOP/s; a library product of 8,192
+// cubed reaches 154); 695 x 1,024 x 3,072 in 70 us, 87 with one group of waves a workgroup.
+#define F32_SLICE 32
+#define F32_STRIDE 36
+
+template <int B, int KG, bool ACCUMULATE>
+__global__ __launch_bounds__(256 * KG) void gemm_f32_tiles_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                  float* __restrict__ c, int M, int N, int K) {
+  constexpr int TILE = 64 * B, LOADS = TILE / 32;
+  __shared__ __attribute__((aligned(16))) float slices[KG][2][2][TILE * F32_STRIDE];   // [group][buffer][activations, weights]
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, group = threadIdx.x >> 8;
+  auto& lds = slices[group];
+  const int m0 = blockIdx.y * TILE, n0 = blockIdx.x * TILE;
+  const int l_row = tid >> 3, l_k = 4 * (tid & 7);
+  const float *a_from[LOADS], *w_from[LOADS];
+#pragma unroll
+  for (int s = 0; s < LOADS; ++s) {
+    a_from[s] = a + (size_t)min(m0 + l_row + 32 * s, M - 1) * K + l_k;
+    w_from[s] = w + (size_t)min(n0 + l_row + 32 * s, N - 1) * K + l_k;
+  }
+  floatx4 next_a[LOADS], next_w[LOADS];
+  auto fetch = [&](int k0) {
+    const bool inside = k0 + l_k < K;      // K is a multiple of 4
+#pragma unroll
+    for (int s = 0; s < LOADS; ++s) {
+      next_a[s] = inside ? load4(a_from[s] + k0) : floatx4{0.f, 0.f, 0.f, 0.f};
+      next_w[s] = inside ? load4(w_from[s] + k0) : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto put = [&](int buffer) {
+#pragma unroll
+    for (int s = 0; s < LOADS; ++s) {
+      *reinterpret_cast<floatx4*>(&lds[buffer][0][(l_row + 32 * s) * F32_STRIDE + l_k]) = next_a[s];
+      *reinterpret_cast<floatx4*>(&lds[buffer][1][(l_row + 32 * s) * F32_STRIDE + l_k]) = next_w[s];
+    }
+  };
+  const int wm = (wave >> 1) * 32 * B, wn = (wave & 1) * 32 * B;
+  const int half = lane >> 5, at_row = lane & 31;
+  floatx16 acc[B][B] = {};
+  fetch(F32_SLICE * group);
+  put(0);
+  __syncthreads();
+  int buffer = 0;
+  for (int k0 = 0; k0 < K; k0 += KG * F32_SLICE, buffer ^= 1) {     // every group as often; a slice beyond K is zeros
+    const bool more = k0 + KG * F32_SLICE < K;
+    if (more) fetch(k0 + (KG + group) * F32_SLICE);
+    const float* as = &lds[buffer][0][(wm + at_row) * F32_STRIDE + 4 * half];
+    const float* ws = &lds[buffer][1][(wn + at_row) * F32_STRIDE + 4 * half];
+    floatx16 part[B][B] = {};
+#pragma unroll
+    for (int kk = 0; kk < F32_SLICE; kk += 8) {
+      floatx4 av[B], wv[B];
+#pragma unroll
+      for (int x = 0; x < B; ++x) {
+        av[x] = load4(as + 32 * x * F32_STRIDE + kk);
+        wv[x] = load4(ws + 32 * x * F32_STRIDE + kk);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int x = 0; x < B; ++x)
+#pragma unroll
+          for (int y = 0; y < B; ++y) part[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[x][t], wv[y][t], part[x][y], 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < B; ++x)
+#pragma unroll
+      for (int y = 0; y < B; ++y) acc[x][y] += part[x][y];
+    if (more) put(buffer ^ 1);     // its readers passed the barrier that ended the slice before
+    __syncthreads();
+  }
+  if constexpr (KG > 1) {          // the groups' sums, lane by lane, through their own slices' memory
+    floatx16* mine = reinterpret_cast<floatx16*>(&slices[group][0][0][0]) + tid;
+    if (group > 0) *mine = acc[0][0];
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int s = 1; s < KG; ++s) acc[0][0] += *(reinterpret_cast<const floatx16*>(&slices[s][0][0][0]) + tid);
+  }
+#pragma unroll
+  for (int x = 0; x < B; ++x)
+#pragma unroll
+    for (int y = 0; y < B; ++y) {
+      const int n = n0 + wn + 32 * y + at_row;
+      if (n >= N) continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = m0 + wm + 32 * x + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (m >= M) continue;
+        const size_t to = (size_t)m * N + n;
+        c[to] = ACCUMULATE ? acc[x][y][r] + c[to] : acc[x][y][r];
+      }
+    }
+}
+
+// ---- which products go where ---------------------------------------------------------------------------
+
+bool bh_gemm_f32_takes(const void* a, const void* w, const void* c, int K) {
+  return K % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) % 16) == 0 && ((uintptr_t)c % 4) == 0;
+}
+
+template <int R, int C, bool GATED>
+static void few_waves(const float* a, const float* w, float* c, int M, int N, int K, int accumulate, GateForm form, hipStream_t stream) {
+  const int outputs = 4 * (GATED ? R / 2 : R), blocks = (N + outputs - 1) / outputs;
+  if constexpr (R == 4) {
+    // Many rows: a wave alone walks all of K, so that its loads run on behind one another (32,768 x 1,024 at 32 rows 61 us, 105
+    // where four waves share K), as long as that leaves four workgroups a compute unit.
+    if (blocks >= 4 * bh_compute_units()) {
+      gemm_f32_few_kernel<R, C, 1, GATED><<<blocks, 64, 0, stream>>>(a, w, c, M, N, K, accumulate, form);
+      return;
+    }
+  } else if (K >= 2048 && blocks < 2 * bh_compute_units()) {
+    // Eight waves share a long K where four would leave a compute unit with fewer than two workgroups.
+    gemm_f32_few_kernel<R, C, 8, GATED><<<blocks, 512, 0, stream>>>(a, w, c, M, N, K, accumulate, form);
+    return;
+  }
+  gemm_f32_few_kernel<R, C, 4, GATED><<<blocks, 256, 0, stream>>>(a, w, c, M, N, K, accumulate, form);
+}
+
+template <int R, bool GATED>
+static void few_rows(const float* a, const float* w, float* c, int M, int N, int K, int accumulate, GateForm form, hipStream_t stream) {
+  if (M <= 4) few_waves<R, 1, GATED>(a, w, c, M, N, K, accumulate, form, stream);
+  else if (M <= 8) few_waves<R, 2, GATED>(a, w, c, M, N, K, accumulate, form, stream);
+  else if (M <= 16) few_waves<R, 4, GATED>(a, w, c, M, N, K, accumulate, form, stream);
+  else few_waves<R, 8, GATED>(a, w, c, M, N, K, accumulate, form, stream);
+}
+
+int bh_gemm_f32(const float* a, const float* w, float* c, int accumulate, int M, int N, int K, hipStream_t stream) {
+  const int units = bh_compute_units();
+  if (M <= BH_F32_FEW_ROWS) {
+    const GateForm none = {0.f, 0.f};
+    // as many weight rows a workgroup as leave two workgroups a compute unit
+    if (N >= 32 * units) few_rows<4, false>(a, w, c, M, N, K, accumulate, none, stream);
+    else if (N >= 16 * units) few_rows<2, false>(a, w, c, M, N, K, accumulate, none, stream);
+    else few_rows<1, false>(a, w, c, M, N, K, accumulate, none, stream);
+    return bh_check_launch("gemm_f32_few");
+  }
+  // Tiles of 128 x 128 read half as much a product, but only four of them a compute unit and more level out (695 x 6,144 x 1,024,
+  // 1.1 a unit: 141 us, 104 in tiles of 64 x 64); where tiles of 64 x 64 are not even two a unit, a second group of waves hides the
+  // first one's waits for its slices.
+  const long units4 = 4L * units, wide = (long)((N + 127) / 128) * ((M + 127) / 128);
+  const bool big = wide >= units4;
+  const int tile = big ? 128 : 64;
+  BH_REQUIRE((M + tile - 1) / tile <= 65535, "gemm: M=%d needs more than 65535 row tiles", M);
+  const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile);
+  const bool groups = (long)grid.x * grid.y < 2L * units && K >= 4 * F32_SLICE;
+#define BH_F32_TILES(B, KG)                                                                                          \
+  do {                                                                                                               \
+    if (accumulate) gemm_f32_tiles_kernel<B, KG, true><<<grid, 256 * KG, 0, stream>>>(a, w, c, M, N, K);             \
+    else gemm_f32_tiles_kernel<B, KG, false><<<grid, 256 * KG, 0, stream>>>(a, w, c, M, N, K);                       \
+  } while (0)
+  if (big) BH_F32_TILES(2, 1);
+  else if (groups) BH_F32_TILES(1, 2);
+  else BH_F32_TILES(1, 1);
+#undef BH_F32_TILES
+  return bh_check_launch("gemm_f32_tiles");
+}
+
+// The gated form of few rows in one launch.  bh_gemm_f32_takes_gated: whether these sizes go (else: the product, then its activation).
+extern "C" int bh_gemm_f32_takes_gated(int M, int F, int K) { return M > 0 && M <= BH_F32_FEW_ROWS && F > 0 && K > 0 && K % 4 == 0 ? 1 : 0; }
+extern "C" int bh_gemm_f32_gated(const float* a, const float* w, float* out, int M, int F, int K, int gate, hipStream_t stream) {
+  BH_REQUIRE(bh_gemm_f32_takes_gated(M, F, K) && bh_gemm_f32_takes(a, w, out, K),
+             "gemm: a gated float32 product takes up to %d rows, K a multiple of 4 and 16-byte aligned operands (M=%d K=%d)",
+             BH_F32_FEW_ROWS, M, K);
+  const GateForm form = bh_gate_form(gate);
+  if (F >= 16 * bh_compute_units()) few_rows<4, true>(a, w, out, M, F, K, 0, form, stream);
+  else few_rows<2, true>(a, w, out, M, F, K, 0, form, stream);
+  return bh_check_launch("gemm_f32_few");
+}

@@ -4,6 +4,7 @@
 // no matrix-core mode); the bfloat16 engine uses them wherever no faster kernel fits a size.
 // All reductions, norms, softmax and rotation are computed in float32.
 #include "common.h"
+#include "gemm_f32.h"
 #include <algorithm>
 
 #include <stdarg.h>
@@ -309,8 +310,12 @@ extern "C" int bh_gemm_generic(const void* a, int a_dtype, const void* w, int w_
   BH_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: sizes M=%d N=%d K=%d must be positive", M, N, K);
   BH_REQUIRE((N + GT - 1) / GT <= 2147483647 && (M + GT - 1) / GT <= 65535,
              "gemm: M=%d needs more than 65535 row tiles", M);
-  if (a_dtype == BH_F32 && w_dtype == BH_F32)
+  if (a_dtype == BH_F32 && w_dtype == BH_F32) {
+    // 32-bit operands and result: the float32 matrix instructions (gemm_f32.hip), unless K or an address forbids 16-byte loads
+    if (c_dtype == BH_F32 && bh_gemm_f32_takes(a, w, c, K))
+      return bh_gemm_f32((const float*)a, (const float*)w, (float*)c, accumulate, M, N, K, stream);
     return gemm_generic_out<float, float>(a, w, c, c_dtype, accumulate, M, N, K, stream);
+  }
   if (a_dtype == BH_BF16 && w_dtype == BH_BF16)
     return gemm_generic_out<bf16_t, bf16_t>(a, w, c, c_dtype, accumulate, M, N, K, stream);
   if (a_dtype == BH_BF16 && w_dtype == BH_F32)

@@ -144,6 +144,10 @@ class KernelSizes:
             "bh_gemm_bf16_bare_parts": [i, i, i, i],
             "bh_gemm_bf16_bare": [p, p, p, i, i, i, i, i, p],
             "bh_attention_generic": [p, p, i, p, p, p, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
+            "bh_attention_f32": [p, p, p, p, p, i, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
+            "bh_attention_f32_takes": [i, i, i, i],
+            "bh_gemm_f32_takes_gated": [i, i, i],
+            "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
             "bh_swiglu": [p, p, i, i, i, i, p],
             "bh_sample": [p, p, p, p, p, p, p, p, i, i, p],
             "bh_sample_scratch": [i, i],
@@ -671,6 +675,11 @@ class HipKernels(KernelSizes):
             return
         if isinstance(a, BlockedRows):
             a = self.from_blocked(a)
+        if (a.dtype == w.dtype == torch.float32 and self.lib.bh_gemm_f32_takes_gated(m, width, k)
+                and (a.data_ptr() | w.data_ptr()) % 16 == 0):
+            self._check(self.lib.bh_gemm_f32_gated(self._ptr(a, "gemm a"), self._ptr(w, "gemm w"), self._ptr(out, "gemm out"),
+                                                   m, width, k, self.GATES[gate], self._stream()))
+            return
         both = torch.empty((m, 2 * width), dtype=a.dtype, device=self.device)
         self.gemm(a, w, both)
         self.swiglu(both, out, gate)
@@ -800,11 +809,21 @@ class HipKernels(KernelSizes):
                              n_splits, _block_rows(out), self._ptr(sinks, "sinks", (torch.float32,), True), *gating, *form, float(out_scale),
                              self._stream()))
             return
+        kv_order = self.kv_order(k_pages.dtype, head_dim)
+        if (q.dtype == torch.float32 and self.lib.bh_attention_f32_takes(n_heads, n_kv_heads, head_dim, kv_order)
+                and (q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0):
+            self._check(self.lib.bh_attention_f32(
+                *common, self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
+                self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1], page_table.shape[0],
+                self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(positions, "positions", (torch.int32,)),
+                n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), kv_order,
+                self._ptr(sinks, "sinks", (torch.float32,), True), *gating, *form, float(out_scale), self._stream()))
+            return
         self._check(self.lib.bh_attention_generic(
             *common, _code(q, "q"), self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
             self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1],
             self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(positions, "positions", (torch.int32,)),
-            n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), self.kv_order(k_pages.dtype, head_dim),
+            n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), kv_order,
             self._ptr(sinks, "sinks", (torch.float32,), True), *gating, *form, float(out_scale), self._stream()))
 
     def _score_form(self, softcap, slopes, q_temp, n_heads, what):
