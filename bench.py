@@ -588,8 +588,7 @@ def pudorax_kernels(K, torch, width, heads, context, experts=32, top=4):
 
 def pudorax_expert_calls(K, torch, x, chosen, shares, w_gu, w_d, hidden, active, top, ff, width):
     """(name, call, bytes, operations) of the routed experts' work as a step of these rows runs it: grouped by expert, then for
-    few rows a workgroup per expert and block of outputs, for many rows the framework's products on every expert's stretch."""
-    from types import SimpleNamespace
+    few rows a workgroup per expert and block of outputs, for many rows tiles of pairs of all experts in one launch."""
     from beholdd.parts.experts import RoutedExperts
     rows, experts = x.shape[0], w_gu.shape[0]
     pairs = rows * top
@@ -607,15 +606,17 @@ def pudorax_expert_calls(K, torch, x, chosen, shares, w_gu, w_d, hidden, active,
                2.0 * pairs * ff * width)
         yield ("experts_combine", lambda: K.experts_combine(y, None, shares, hidden), y.numel() * 4 + 2 * hidden.numel() * 4, 0.0)
         return
-    part = RoutedExperts(width, experts, top, ff, 7.0, "m.")
-    part.w_gate_up, part.w_down = w_gu, w_d
-    part.prepare(K)
-    ctx = SimpleNamespace(kernels=K, device=x.device, new_f32=lambda *shape: torch.empty(shape, device=x.device),
-                          new_activations=lambda *shape, reader=None: torch.empty(shape, device=x.device, dtype=x.dtype))
-    one = part.in_one_launch and 6.0 * pairs * ff * width <= part.ONE_LAUNCH_WORK
-    form = "two launches over all experts" if one else f"{2 * experts} products, clamped_glu"
-    yield (f"experts of a prompt (gather, {form}, combine)", lambda: part._as_products(ctx, x, lists, counts, shares, hidden),
-           weights_read + pairs * (2 * width + 3 * ff) * 2 + pairs * width * 8, 6.0 * pairs * ff * width)
+    up, down = K.pack_weight(w_gu.reshape(-1, width)), K.pack_weight(w_d.reshape(-1, ff))
+    inner = torch.empty(pairs, ff, device=x.device, dtype=x.dtype)
+    y = torch.empty(pairs, width, device=x.device)
+
+    def prompt():
+        K.experts_many(x, top, lists, counts, up, inner, gated=True, limit=7.0, alpha=1.702)
+        K.experts_many(inner, 1, lists, counts, down, y)
+        K.experts_combine(y, None, shares, hidden)
+
+    yield ("experts of a prompt (two launches over all experts, combine)", prompt,
+           weights_read + pairs * (width + 2 * ff) * 2 + pairs * width * 8, 6.0 * pairs * ff * width)
 
 
 def pudorax_bench(args, torch):

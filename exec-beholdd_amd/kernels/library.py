@@ -212,6 +212,7 @@ class KernelSizes:
             "bh_experts_rows": [p, i, i, p, i, p, p, p, i, i, i, i, f, f, f, p, p],
             "bh_experts_tiles": [p, i, p, i, p, p, p, i, i, i, i, f, f, f, p, p],
             "bh_experts_tiles_takes": [i, i],
+            "bh_experts_many": [p, i, p, i, p, p, p, i, i, i, i, i, f, f, f, p, p],
             "bh_experts_gather": [p, i, i, p, i, p, p, p, p, i, i, i, p, p],
             "bh_gla_scan": [p, i, i, i, i, i, p, i, p, f, f, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, p],
             "bh_gla_chunk_rows": [i, i, i, i, i],
@@ -1749,15 +1750,23 @@ class HipKernels(KernelSizes):
     def experts_tiles(self, rows, rows_per_pair_row, lists, counts, w, out, gated=False, limit=0.0, alpha=0.0, shift=1.0, in_weights=None):
         """`experts_rows` on the matrix cores: `w` is the PackedWeight of all experts' matrices one below the other ([E * 2 N, K]
         gated, gate rows and then up rows of every expert; otherwise [E * N, K])."""
+        self._experts_packed(False, rows, rows_per_pair_row, lists, counts, w, out, gated, limit, alpha, shift, in_weights)
+
+    def experts_many(self, rows, rows_per_pair_row, lists, counts, w, out, gated=False, limit=0.0, alpha=0.0, shift=1.0, in_weights=None):
+        """`experts_tiles` for steps in which an expert has many pairs: an expert's matrices are read once for 64 or 128 of them."""
+        self._experts_packed(True, rows, rows_per_pair_row, lists, counts, w, out, gated, limit, alpha, shift, in_weights)
+
+    def _experts_packed(self, many, rows, rows_per_pair_row, lists, counts, w, out, gated, limit, alpha, shift, in_weights):
         experts, k = counts.shape[0], rows.shape[1]
         n = out.shape[1]
         if not isinstance(w, PackedWeight) or tuple(w.shape) != (experts * (2 if gated else 1) * n, k) or rows.dtype != torch.bfloat16 \
                 or out.dtype != (torch.bfloat16 if gated else torch.float32) or lists.shape[0] != experts:
             raise KernelError(f"experts_tiles: shapes rows {tuple(rows.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
-        self._check(self.lib.bh_experts_tiles(
+        entry, pairs = (self.lib.bh_experts_many, (out.shape[0],)) if many else (self.lib.bh_experts_tiles, ())
+        self._check(entry(
             self._ptr(rows, "experts rows", (torch.bfloat16,)), int(rows_per_pair_row), self._ptr(lists, "lists", (torch.int32,)), lists.shape[1],
             self._ptr(counts, "counts", (torch.int32,)), self._ptr(w.data, "expert weights", (torch.bfloat16,)), self._ptr(out, "experts out"),
-            experts, k, n, int(bool(gated)), float(limit), float(alpha), float(shift),
+            *pairs, experts, k, n, int(bool(gated)), float(limit), float(alpha), float(shift),
             self._ptr(in_weights, "pair weights", (torch.float32,), True), self._stream()))
 
     def experts_products_take(self, dtype, inputs: int, outputs: int) -> bool:

@@ -19,10 +19,10 @@ The experts' matrices are kept stacked: gate and up rows of an expert in one [2 
 all.  The (row, choice) pairs are grouped by expert on the device (`experts_group`).  A step of few rows then runs a
 workgroup per expert and block of outputs that reads the expert's rows from memory once for all of its pairs (`experts_tiles`
 on the matrix cores from the packed form of the matrices, or `experts_rows` for sizes and element types that one does not take), with nothing that depends on the routing on the host, so that decode steps can be captured.  A step
-of many rows (a prompt) reads the experts' counts on the host (the step waits for the device there), lays the pairs'
-inputs side by side, expert after expert, and runs all experts' products in one launch on the matrix cores
-(`experts_products`, over a table of row tiles made from the counts; the activation rides in the first product), or,
-for sizes and element types that kernel does not take, the framework's matrix products on each expert's stretch.  Sizes
+of many rows (a prompt) runs all experts' products from the packed matrices in two launches too (`experts_many`: the workgroups
+find their tiles of pairs in the counts by themselves, the activation rides in the first product).  For sizes and element types
+that the packed form does not take it reads the experts' counts on the host (the step waits for the device there), lays the pairs'
+inputs side by side, expert after expert, and runs the framework's matrix products on each expert's stretch.  Sizes
 that the grouped kernels do not take go pair by pair (`experts_gate_up`, `experts_down`).  In every form a row's
 experts' shares are added in the order of its own choice, so its result depends on its batch-mates by rounding at most.  The routing is left in
 `ctx.extras["routing"]` ((chosen, weights) of the last layer that ran).  Every size and constant is a constructor
@@ -85,9 +85,6 @@ class RoutedExperts:
     PACK_FOR_PROMPTS = True   # keep a second copy of every expert's matrices in the form the products of many rows read fastest
     WIDE_ROUTER = 128         # a router of fewer outputs is kept with that many for steps of more than WIDE_FROM_ROWS rows: products
     WIDE_FROM_ROWS = 32       # that cut K into parts need a whole tile of outputs (2,048 rows, 40 experts: 71 -> 22 us)
-    ONE_LAUNCH_WORK = 1.5e11  # up to that many operations a layer, a prompt's experts run as one launch over all of them: the
-                              # one kernel reaches about 120 TFLOP/s whatever the size (tiles of 128 x 64 outputs re-read their
-                              # operands through the L2), the products per expert cost about 25 us each and then run faster
 
     def __init__(self, hidden: int, n_experts: int, top: int, ff: int, limit: float, prefix: str, shared=None,
                  alpha: float = GATE_SLOPE, router_bias: bool = True, scoring: str = "softmax", weigh_input: bool = False,
@@ -109,8 +106,7 @@ class RoutedExperts:
         self.has_router_bias = bool(router_bias)
         self.router_bias = self.correction = self.w_gate_up = self.w_down = None
         self.for_products = None      # per expert (gate and up, down) as the matrix products take them
-        self.for_few_rows = None      # all experts' matrices one below the other, packed (gate and up, down), for kernels.experts_tiles
-        self.in_one_launch = False    # a prompt's products run as one launch over all experts (kernels.experts_products)
+        self.packed = None            # all experts' matrices one below the other (gate and up, down), as experts_tiles and experts_many take them
 
     def tensor_specs(self):
         specs = self.router.tensor_specs()
@@ -151,14 +147,9 @@ class RoutedExperts:
         self.router.prepare(kernels)
         if self.shared is not None:
             self.shared.prepare(kernels)
-        takes = getattr(kernels, "experts_products_take", None)
-        self.in_one_launch = bool(takes is not None and takes(self.w_gate_up.dtype, self.hidden, self.ff) and takes(self.w_down.dtype, self.ff, self.hidden))
         tiles = getattr(kernels, "experts_tiles_take", None)
         if tiles is not None and tiles(self.w_gate_up.dtype, self.hidden, self.ff) and tiles(self.w_down.dtype, self.ff, self.hidden):
-            self.for_few_rows = (kernels.pack_weight(self.w_gate_up.view(-1, self.hidden)), kernels.pack_weight(self.w_down.view(-1, self.ff)))
-            # blocks of 16 rows do not straddle experts: an expert's own packed matrices lie side by side in these
-            self.for_products = list(zip(*([type(whole)(part, whole.shape[0] // self.n_experts, whole.shape[1])
-                                            for part in whole.data.view(self.n_experts, -1)] for whole in self.for_few_rows)))
+            self.packed = (kernels.pack_weight(self.w_gate_up.view(-1, self.hidden)), kernels.pack_weight(self.w_down.view(-1, self.ff)))
         elif self.PACK_FOR_PROMPTS and hasattr(kernels, "pack_weight"):
             self.for_products = [(kernels.pack_weight(self.w_gate_up[e]), kernels.pack_weight(self.w_down[e])) for e in range(self.n_experts)]
 
@@ -169,7 +160,8 @@ class RoutedExperts:
         total += 2 * step.matrix(step.rows, self.top, 4)
         pairs = step.rows * self.top
         total += step.matrix(self.n_experts, step.rows, 4) + step.matrix(pairs, self.ff) + step.matrix(pairs, self.hidden, 4)
-        if step.rows > step.seqs and pairs >= self.PRODUCT_PAIRS * self.n_experts:      # a step of many rows: the pairs' inputs, gate and up
+        in_place = step.act_size == 2 and self.hidden % 64 == 0 and self.ff % 64 == 0
+        if not in_place and step.rows > step.seqs and pairs >= self.PRODUCT_PAIRS * self.n_experts:      # a step of many rows: the pairs' inputs, gate and up
             total += step.matrix(pairs, self.hidden) + step.matrix(pairs, 2 * self.ff) + step.matrix(pairs, 1, 4)
         return total + (self.shared.working_bytes(step) if self.shared is not None else 0)
 
@@ -209,10 +201,14 @@ class RoutedExperts:
             lists = torch.empty((self.n_experts, n), dtype=torch.int32, device=ctx.device)
             counts = torch.empty((self.n_experts,), dtype=torch.int32, device=ctx.device)
             k.experts_group(chosen, lists, counts)
-            if ctx.is_decode or pairs < self.PRODUCT_PAIRS * self.n_experts:
+            many = pairs >= self.PRODUCT_PAIRS * self.n_experts
+            if self.packed is not None or ctx.is_decode or not many:
                 inner = ctx.new_activations(pairs, self.ff)
                 y = ctx.new_f32(pairs, self.hidden)
-                product, (up, down) = (k.experts_tiles, self.for_few_rows) if self.for_few_rows is not None else (k.experts_rows, (self.w_gate_up, self.w_down))
+                if self.packed is not None:
+                    product, (up, down) = k.experts_many if many else k.experts_tiles, self.packed
+                else:
+                    product, (up, down) = k.experts_rows, (self.w_gate_up, self.w_down)
                 product(x, self.top, lists, counts, up, inner, gated=True, limit=self.limit, alpha=self.alpha, **ahead)
                 product(inner, 1, lists, counts, down, y)
                 self._combine(k, y, None, behind, hidden, adding)
@@ -245,16 +241,6 @@ class RoutedExperts:
         gathered = ctx.new_activations(pairs, self.hidden)
         place = torch.empty((pairs,), dtype=torch.int32, device=ctx.device)
         k.experts_gather(x, self.top, lists, counts, offsets, gathered, place, **({"in_weights": weights} if self.weigh_input else {}))
-        if self.in_one_launch and 6.0 * pairs * self.ff * self.hidden <= self.ONE_LAUNCH_WORK:
-            tiles = torch.tensor([(e, first + at, min(128, count - at)) for e, (first, count) in enumerate(zip(starts, held))
-                                  for at in range(0, count, 128)], dtype=torch.int32, device=ctx.device)
-            inner = ctx.new_activations(pairs, self.ff)
-            y = ctx.new_f32(pairs, self.hidden)
-            if len(tiles):      # (every choice of the step may have fallen on identity experts)
-                k.experts_products(gathered, self.w_gate_up, tiles, inner, gated=True, limit=self.limit, alpha=self.alpha, **act)
-                k.experts_products(inner, self.w_down, tiles, y)
-            self._combine(k, y, place, behind, hidden, adding)
-            return
         both = ctx.new_activations(pairs, 2 * self.ff)
         for e, (first, count) in enumerate(zip(starts, held)):
             if count:
