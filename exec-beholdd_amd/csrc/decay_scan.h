@@ -1,0 +1,342 @@
+// A linear recurrence with a scalar decay per row and head, for prompts, on the float32 matrix instructions:
+//   S_t = d_t S_(t-1) + w_t k_t v_t^T,   o_t = S_t^T q_t + skip v_t          S [D][V] per (sequence, head)
+// (lightning attention: d the head's constant, w 1, no skip; the state-space recurrence: d and w from the row's step size.)
+//
+// With the rows in chunks of 64 and D(t, j) = d_(j+1) .. d_t, a chunk that starts from the state E has
+//   o_t = D(t, start) E^T q_t + sum_(j <= t) D(t, j) w_j (q_t . k_j) v_j + skip v_t,   S_end = D(end, start) E + sum_j D(end, j) w_j k_j v_j^T,
+// so that all of it but the chain of states is products of matrices, for all chunks at the same time:
+//   scan_states    a workgroup a (chunk, head): Z = sum_j D(end, j) w_j k_j v_j^T and the chunk's whole decay
+//   scan_combine   goes through a sequence's chunks in order: E_(c+1) = D E_c + Z_c, from and to the sequence's region; a thread four elements
+//   scan_outputs   a workgroup a (chunk, head): scores q k^T, times their decays and weights below the diagonal, times v, and E^T q
+// Every product and sum is 32-bit; decays are differences of logarithms summed in 64 bits (or powers of the constant), so that
+// no row's decay is a chain of roundings.  A walk row by row (lightning_scan, ssm_chunk) has the same sums in another order, but as a
+// serial chain of FMAs.
+// A sequence's chunks have places of their own, floor(first row / 64) + sequence onward, which overlap no other sequence's: a step
+// needs rows / 64 + sequences places, and a window of them at a time has memory for its states.
+// Bound by the matrix instructions and the operands' reads from LDS beside them; a state is written once and read twice.
+// Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 83 us in all (26 + 18 +
+// 39), 233 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 163 us, 606.  With the values in LDS beside the
+// keys, one workgroup a compute unit, 102 and 213.
+#pragma once
+
+#include "common.h"
+
+#define DS_ROWS 64                    // rows of a chunk
+#define DS_MOST_VALUES 256             // elements of a value
+#define DS_PSTRIDE 20                   // floats from one row of a 16 x 16 tile of scores to the next: 16 rows' 16 bytes on all banks
+#define DS_SCORES (10 * 16 * DS_PSTRIDE) // the tiles on and below the diagonal, (row, column) at place row (row + 1) / 2 + column
+#define DS_SCRATCH_FLOATS (24L << 20) // states that a window of places may take: 96 MB (36: 8,192 rows of 32 heads 621 -> 878 us)
+
+typedef float ds_f32x4_t __attribute__((ext_vector_type(4)));
+
+struct ScanChunk {
+  int seq, chunk, first, rows;
+};
+
+__device__ inline int ds_place_of(const int32_t* seq_start, int seq) { return seq_start[seq] / DS_ROWS + seq; }
+
+// The chunk at a place; rows 0 where no sequence has one there.  The same for the whole workgroup.
+__device__ inline ScanChunk ds_find(const int32_t* __restrict__ seq_start, int n_seqs, int place) {
+  const int lane = threadIdx.x & 63;
+  int upto = 0;      // sequences whose places start at this one or before
+  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
+    const int s = s0 + lane;
+    upto += __popcll(__ballot(s < n_seqs && ds_place_of(seq_start, s < n_seqs ? s : 0) <= place));
+  }
+  ScanChunk at;
+  at.seq = __builtin_amdgcn_readfirstlane(upto - 1);      // the first sequence starts at place 0
+  at.chunk = place - ds_place_of(seq_start, at.seq);
+  at.first = seq_start[at.seq] + at.chunk * DS_ROWS;
+  at.rows = min(DS_ROWS, seq_start[at.seq + 1] - at.first);
+  if (at.rows < 0) at.rows = 0;
+  return at;
+}
+
+// Rows' decays within a chunk.  POWERS: of one number, pow[n] = d^n; otherwise from the rows' logarithms, summed in 64 bits.
+template <bool POWERS>
+struct ScanDecays;
+template <>
+struct ScanDecays<true> {
+  float pow[DS_ROWS + 1];
+  __device__ float between(int t, int j) const { return pow[t - j]; }
+  __device__ float from_start(int t) const { return pow[t + 1]; }
+};
+template <>
+struct ScanDecays<false> {
+  double sum[DS_ROWS];
+  // e^x of a 64-bit number: what 32 bits of it leave out is below 2^-24 of it, so that one term of the series is enough
+  static __device__ float exponential(double x) {
+    const float head = (float)x, power = expf(head);
+    return fmaf(power, (float)(x - head), power);
+  }
+  __device__ float between(int t, int j) const { return exponential(sum[t] - sum[j]); }
+  __device__ float from_start(int t) const { return exponential(sum[t]); }
+};
+
+// In: what the recurrence reads.  POWERS, SKIPS (with skip(head)), q4 / k4 / v4(row, head, i) (elements i .. i + 3 of the head's vector), and
+// prepare(decays, weights, chunk, head): called by a whole workgroup, which it leaves with a barrier to come.
+template <class In>
+__global__ __launch_bounds__(512) void scan_states_kernel(In in, const int32_t* __restrict__ seq_start, int n_seqs, int place0, int places,
+                                                          float* __restrict__ states, float* __restrict__ factors, int H, int D, int V) {
+  extern __shared__ __align__(16) float ds_lds[];
+  __shared__ ScanDecays<In::POWERS> decays;
+  __shared__ float weights[DS_ROWS];
+  const int head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + blockIdx.x);
+  if (at.rows == 0) return;
+  const int ks = D + 4, vs = V + 4;
+  float* k_lds = ds_lds;
+  float* v_lds = k_lds + DS_ROWS * ks;
+  in.prepare(decays, weights, at, head);
+  for (int e = tid; e < DS_ROWS * V / 4; e += 512) {
+    const int r = e / (V / 4), i = 4 * (e % (V / 4));
+    *reinterpret_cast<float4*>(v_lds + r * vs + i) = r < at.rows ? in.v4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __syncthreads();
+  for (int e = tid; e < DS_ROWS * D / 4; e += 512) {
+    const int r = e / (D / 4), i = 4 * (e % (D / 4));
+    float4 k = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (r < at.rows) {
+      k = in.k4(at.first + r, head, i);
+      const float w = weights[r] * decays.between(at.rows - 1, r);
+      k = make_float4(k.x * w, k.y * w, k.z * w, k.w * w);
+    }
+    *reinterpret_cast<float4*>(k_lds + r * ks + i) = k;
+  }
+  if (tid == 0) factors[(size_t)blockIdx.x * H + head] = decays.from_start(at.rows - 1);
+  __syncthreads();
+  // Z [D][V]: 32 x 16 elements at a time, rows of the chunk as the products' depth
+  const int j = lane & 15, g = lane >> 4, columns = V / 16;
+  float* out = states + ((size_t)blockIdx.x * H + head) * D * V;
+  for (int unit = wave; unit < D / 32 * columns; unit += 8) {
+    const int d0 = unit / columns * 32, c0 = unit % columns * 16;
+    ds_f32x4_t acc[2] = {};
+#pragma unroll
+    for (int s = 0; s < DS_ROWS / 4; ++s) {
+      const int row = 16 * (s / 4) + 4 * g + s % 4;      // four rows of 4 D + 16 floats apart: on banks of their own
+      const float* k_row = k_lds + row * ks + d0 + j;
+      const float v = v_lds[row * vs + c0 + j];
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[0], v, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[16], v, acc[1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[(size_t)(d0 + 16 * x + 4 * g + r) * V + c0 + j] = acc[x][r];
+  }
+}
+
+// grid (sequences, heads, elements / 1024)
+template <int UNUSED = 0>
+__global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                                           int place0, int places, float* __restrict__ states,
+                                                           const float* __restrict__ factors, float* __restrict__ home, long slot_stride,
+                                                           int H, int size) {
+  constexpr int AHEAD = 8;
+  const int seq = blockIdx.x, head = blockIdx.y, e = 4 * (blockIdx.z * 256 + threadIdx.x);
+  if (e >= size) return;
+  const int base = ds_place_of(seq_start, seq), chunks = (seq_start[seq + 1] - seq_start[seq] + DS_ROWS - 1) / DS_ROWS;
+  const int from = max(0, place0 - base), upto = min(chunks, place0 + places - base);
+  if (from >= upto) return;
+  float4* mine = reinterpret_cast<float4*>(home + (size_t)seq_slot[seq] * slot_stride + (size_t)head * size + e);
+  const size_t apart = (size_t)H * size;
+  float* z = states + ((size_t)(base + from - place0) * H + head) * size + e;
+  const float* f = factors + (size_t)(base + from - place0) * H + head;
+  float4 state = *mine;
+  for (int c = 0; c < upto - from; c += AHEAD) {
+    float4 own[AHEAD];
+    float factor[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int at = min(c + u, upto - from - 1);
+      own[u] = *reinterpret_cast<const float4*>(z + at * apart);
+      factor[u] = f[(size_t)at * H];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (c + u >= upto - from) break;
+      *reinterpret_cast<float4*>(z + (c + u) * apart) = state;      // what this chunk starts from
+      state.x = fmaf(factor[u], state.x, own[u].x);
+      state.y = fmaf(factor[u], state.y, own[u].y);
+      state.z = fmaf(factor[u], state.z, own[u].z);
+      state.w = fmaf(factor[u], state.w, own[u].w);
+    }
+  }
+  *mine = state;
+}
+
+template <class In>
+__global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t* __restrict__ seq_start, int n_seqs, int place0,
+                                                           const float* __restrict__ states, float* __restrict__ out, int H, int D, int V) {
+  extern __shared__ __align__(16) float ds_lds[];
+  __shared__ ScanDecays<In::POWERS> decays;
+  __shared__ float weights[DS_ROWS];
+  const int head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + blockIdx.x);
+  if (at.rows == 0) return;
+  const int qs = D + 4, vs = V + 4;
+  // The scores and the values take the keys' place once those have been multiplied (the values wait in registers), which lets two
+  // workgroups of heads of 128 share a compute unit.
+  float* q_lds = ds_lds;
+  float* k_lds = q_lds + DS_ROWS * qs;
+  float* p_lds = k_lds;
+  float* v_lds = p_lds + DS_SCORES;
+  in.prepare(decays, weights, at, head);
+  for (int e = tid; e < DS_ROWS * D / 4; e += 512) {
+    const int r = e / (D / 4), i = 4 * (e % (D / 4));
+    const bool there = r < at.rows;
+    *reinterpret_cast<float4*>(q_lds + r * qs + i) = there ? in.q4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float4*>(k_lds + r * qs + i) = there ? in.k4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  float4 values[DS_MOST_VALUES / 32];
+#pragma unroll
+  for (int u = 0; u < DS_MOST_VALUES / 32; ++u) {
+    const int e = tid + 512 * u, r = e / (V / 4), i = 4 * (e % (V / 4));
+    values[u] = r < at.rows && e < DS_ROWS * V / 4 ? in.v4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __syncthreads();
+  // scores: the ten 16 x 16 tiles on and below the diagonal, a wave one or two.  A lane's 16 bytes are k 16 b + 4 g .. + 3 of its row
+  // for either operand, which the matrix instructions take in turn.
+  const int j = lane & 15, g = lane >> 4;
+  ds_f32x4_t score[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int tile = wave + 8 * u;
+    score[u] = ds_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (tile >= 10) continue;
+    const int tr = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, tc = tile - tr * (tr + 1) / 2;
+    const float* q_row = q_lds + (16 * tr + j) * qs + 4 * g;
+    const float* k_row = k_lds + (16 * tc + j) * qs + 4 * g;
+    ds_f32x4_t chain[4] = {};      // four sums side by side, added at the end
+    for (int b = 0; b < D; b += 32) {
+      const ds_f32x4_t q0 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b), k0 = *reinterpret_cast<const ds_f32x4_t*>(k_row + b);
+      const ds_f32x4_t q1 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b + 16), k1 = *reinterpret_cast<const ds_f32x4_t*>(k_row + b + 16);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        chain[t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q0[t], k0[t], chain[t & 1], 0, 0, 0);
+        chain[2 + (t & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(q1[t], k1[t], chain[2 + (t & 1)], 0, 0, 0);
+      }
+    }
+    score[u] = (chain[0] + chain[1]) + (chain[2] + chain[3]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int tile = wave + 8 * u;
+    if (tile >= 10) continue;
+    const int tr = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, tc = tile - tr * (tr + 1) / 2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * tr + 4 * g + r, c = 16 * tc + j;
+      float p = 0.f;
+      if (c <= t && t < at.rows) {
+        p = score[u][r] * decays.between(t, c) * weights[c];
+      }
+      p_lds[tile * 16 * DS_PSTRIDE + (4 * g + r) * DS_PSTRIDE + j] = p;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < DS_MOST_VALUES / 32; ++u) {
+    const int e = tid + 512 * u;
+    if (e < DS_ROWS * V / 4) *reinterpret_cast<float4*>(v_lds + e / (V / 4) * vs + 4 * (e % (V / 4))) = values[u];
+  }
+  __syncthreads();
+  // outputs: 32 rows x 16 columns at a time
+  const float* start = states + ((size_t)blockIdx.x * H + head) * D * V;
+  for (int unit = wave; unit < 2 * (V / 16); unit += 8) {
+    const int r0 = 32 * (unit & 1), c0 = unit / 2 * 16;
+    ds_f32x4_t acc[2][2] = {}, from_state[2][2] = {};      // [side][upper or lower 16 rows]: two sums side by side
+    const float* q_row = q_lds + (r0 + j) * qs + 4 * g;
+    const float* e_row = start + (size_t)(4 * g) * V + c0 + j;
+#pragma unroll 4
+    for (int b = 0; b < D; b += 16) {
+      float e[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) e[t] = e_row[(size_t)(b + t) * V];
+      const ds_f32x4_t q0 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b), q1 = *reinterpret_cast<const ds_f32x4_t*>(q_row + 16 * qs + b);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        from_state[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(q0[t], e[t], from_state[t & 1][0], 0, 0, 0);
+        from_state[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q1[t], e[t], from_state[t & 1][1], 0, 0, 0);
+      }
+    }
+    const int tr = r0 / 16;
+    const float* p_row = p_lds + tr * (tr + 1) / 2 * 16 * DS_PSTRIDE + j * DS_PSTRIDE + 4 * g;      // the upper 16 rows' tiles; then the lower's
+    const float* p_lower = p_row + (tr + 1) * 16 * DS_PSTRIDE;
+    for (int b = 0; b < r0 + 32; b += 16) {
+      float v[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[t] = v_lds[(b + 4 * g + t) * vs + c0 + j];
+      const ds_f32x4_t p1 = *reinterpret_cast<const ds_f32x4_t*>(p_lower + b * DS_PSTRIDE);
+      if (b <= r0) {      // the upper 16 rows see no later ones
+        const ds_f32x4_t p0 = *reinterpret_cast<const ds_f32x4_t*>(p_row + b * DS_PSTRIDE);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[t], v[t], acc[t & 1][0], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[t], v[t], acc[t & 1][1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = r0 + 16 * x + 4 * g + r;
+        if (t >= at.rows) continue;
+        float total = fmaf(from_state[0][x][r] + from_state[1][x][r], decays.from_start(t), acc[0][x][r] + acc[1][x][r]);
+        if (In::SKIPS) total = fmaf(in.skip(head), v_lds[t * vs + c0 + j], total);
+        out[((size_t)(at.first + t) * H + head) * V + c0 + j] = total;
+      }
+  }
+}
+
+__device__ inline float4 ds_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ inline float4 ds_load4(const bf16_t* p) {
+  const uint2 raw = *reinterpret_cast<const uint2*>(p);
+  return make_float4(bf16_bits_to_f32((uint16_t)raw.x), bf16_bits_to_f32((uint16_t)(raw.x >> 16)), bf16_bits_to_f32((uint16_t)raw.y),
+                     bf16_bits_to_f32((uint16_t)(raw.y >> 16)));
+}
+
+// ---- host side -----------------------------------------------------------------------------------------
+
+inline long ds_places(int n_seqs, int n_rows) {
+  return n_seqs == 1 ? ((long)n_rows + DS_ROWS - 1) / DS_ROWS : (long)n_rows / DS_ROWS + n_seqs;
+}
+inline size_t ds_states_lds(int D, int V) { return ((size_t)DS_ROWS * (D + 4) + (size_t)DS_ROWS * (V + 4)) * sizeof(float); }
+inline size_t ds_outputs_lds(int D, int V) {
+  const size_t keys = (size_t)DS_ROWS * (D + 4), behind = DS_SCORES + (size_t)DS_ROWS * (V + 4);
+  return ((size_t)DS_ROWS * (D + 4) + (keys > behind ? keys : behind)) * sizeof(float);
+}
+// Floats of scratch memory that a step of these sizes takes; 0 where this form does not take it: sizes have to be whole tiles and
+// fit a workgroup's LDS.
+inline long ds_scratch_floats(int n_seqs, int n_rows, int H, int D, int V) {
+  if (V > DS_MOST_VALUES || D % 32 || V % 16 || D < 64 || H > 65535 ||
+      ds_outputs_lds(D, V) > 150 * 1024 || ds_states_lds(D, V) > 150 * 1024)
+    return 0;
+  const long places = ds_places(n_seqs, n_rows), one = (long)H * ((long)D * V + 1);
+  const long most = DS_SCRATCH_FLOATS / one > 1 ? DS_SCRATCH_FLOATS / one : 1;
+  return (places < most ? places : most) * one;
+}
+
+template <class In>
+int ds_launch(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
+              long scratch_floats, int n_seqs, int n_rows, int H, int D, int V, hipStream_t stream) {
+  const long one = (long)H * ((long)D * V + 1), places = ds_places(n_seqs, n_rows);
+  const int window = (int)(scratch_floats / one < places ? scratch_floats / one : places);
+  BH_REQUIRE(window > 0, "scan: no scratch memory for a chunk's states");
+  BH_REQUIRE(n_seqs <= 2147483647 && ((long)D * V + 1023) / 1024 <= 65535, "scan: a state of %d x %d is too large", D, V);
+  const size_t states_lds = ds_states_lds(D, V), outputs_lds = ds_outputs_lds(D, V);
+  bh_allow_lds<scan_states_kernel<In>>(states_lds);
+  bh_allow_lds<scan_outputs_kernel<In>>(outputs_lds);
+  float* factors = scratch + (size_t)window * H * D * V;
+  for (long place = 0; place < places; place += window) {
+    const int here = (int)(places - place < window ? places - place : window);
+    scan_states_kernel<In><<<dim3(here, H), 512, states_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, factors, H, D, V);
+    if (int status = bh_check_launch("scan_states")) return status;
+    scan_combine_kernel<0><<<dim3(n_seqs, H, (D * V + 1023) / 1024), 256, 0, stream>>>(seq_start, seq_slot, (int)place, here, scratch, factors, home,
+                                                                                     slot_stride, H, D * V);
+    if (int status = bh_check_launch("scan_combine")) return status;
+    scan_outputs_kernel<In><<<dim3(here, H), 512, outputs_lds, stream>>>(in, seq_start, n_seqs, (int)place, scratch, out, H, D, V);
+    if (int status = bh_check_launch("scan_outputs")) return status;
+  }
+  return 0;
+}

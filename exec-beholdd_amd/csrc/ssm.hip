@@ -6,6 +6,7 @@
 //                       `gate_after` the statistic is y's alone: out = rms_g(y) * w * silu(z)
 // Everything but the reading of dt_raw and z is float32.
 #include "common.h"
+#include "decay_scan.h"
 
 __device__ inline float softplus_f32(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
@@ -336,6 +337,70 @@ extern "C" int bh_ssm_scan_fast(const float* xbc, int xbc_stride, const void* pr
     BH_SF(bf16_t, 128);
   }
 #undef BH_SF
+  return bh_fail("ssm_scan: unknown dtype %d", dtype);
+}
+
+// ---- prompts as products of matrices (decay_scan.h): q = C, k = B, v = x, weighed by the step size, D x added -----------
+template <typename T>
+struct SsmRows {
+  static constexpr bool POWERS = false, SKIPS = true;
+  const float* xbc;
+  int stride;
+  const T* proj;
+  int proj_stride, dt_first;
+  const float *dt_bias, *a_log, *d_skip;
+  int H, vdim, N, G;
+  __device__ float4 q4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + H * vdim + (G + head / (H / G)) * N + i); }
+  __device__ float4 k4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + H * vdim + head / (H / G) * N + i); }
+  __device__ float4 v4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + head * vdim + i); }
+  __device__ float skip(int head) const { return d_skip[head]; }
+  __device__ void prepare(ScanDecays<false>& decays, float* weights, const ScanChunk& at, int head) const {
+    const int t = threadIdx.x;
+    if (t >= DS_ROWS) return;      // the first wave
+    float dt = 0.f;
+    double sum = 0.0;
+    if (t < at.rows) {
+      dt = softplus_f32(to_f32(proj[(size_t)(at.first + t) * proj_stride + dt_first + head]) + dt_bias[head]);
+      const double log_decay = -(double)expf(a_log[head]) * dt;
+      sum = log_decay < -1e5 ? -1e5 : log_decay;      // forgets everything either way, and differences stay numbers
+    }
+#pragma unroll
+    for (int off = 1; off < DS_ROWS; off <<= 1) {
+      const double lower = __shfl_up(sum, off, BH_WAVE);
+      if (t >= off) sum += lower;
+    }
+    decays.sum[t] = sum;
+    weights[t] = dt;
+  }
+};
+
+// Floats of scratch memory the products take for a step of these sizes; 0 where they do not take it.
+extern "C" long bh_ssm_products_scratch(int n_seqs, int n_rows, int max_rows, int H, int vdim, int N, int G, int xbc_stride) {
+  if (n_seqs < 1 || n_rows < n_seqs || H < 1 || vdim < 1 || N < 1 || G < 1 || H % G || xbc_stride % 4) return 0;
+  // The walk takes the longest sequence's rows at 1.27 us each, or, where sequences and heads fill the chip, about as long as the
+  // products: 1.67 ns a row of a chunk and head, and their launches.  8 sequences of 64 rows: 32 heads 83 us against 51, 128 heads
+  // 128 against 152; 8 of 1,024: 64 heads 1,231 against 763, 128 heads 1,706 against 1,757.
+  const long whole = (long)n_seqs * ((max_rows + DS_ROWS - 1) / DS_ROWS), places = ds_places(n_seqs, n_rows);
+  if (max_rows < DS_ROWS || 760L * max_rows <= (long)DS_ROWS * H * (whole < places ? whole : places) + 10000) return 0;
+  return ds_scratch_floats(n_seqs, n_rows, H, N, vdim);
+}
+// As bh_ssm_scan; xbc, the state and its stride lie on 16 bytes.
+extern "C" int bh_ssm_products(const float* xbc, int xbc_stride, const void* proj, int dtype, int proj_stride, int dt_first,
+                               const float* dt_bias, const float* a_log, const float* d_skip, float* state, long slot_stride,
+                               const int32_t* seq_start, const int32_t* seq_slot, float* y, int n_seqs, int H, int vdim, int N, int G,
+                               int n_rows, int max_rows, float* scratch, long scratch_floats, hipStream_t stream) {
+  const long wanted = bh_ssm_products_scratch(n_seqs, n_rows, max_rows, H, vdim, N, G, xbc_stride);
+  BH_REQUIRE(wanted > 0 && scratch != nullptr && scratch_floats >= wanted, "ssm_scan: %d heads of %d with %d rows do not go as products", H, vdim, N);
+  BH_REQUIRE(xbc_stride >= H * vdim + 2 * G * N, "ssm_scan: a row of %d does not hold x, B and C", xbc_stride);
+  BH_REQUIRE(dt_first >= 0 && dt_first + H <= proj_stride, "ssm_scan: the step sizes lie outside their row");
+  BH_REQUIRE((((uintptr_t)xbc | (uintptr_t)state | (uintptr_t)scratch) % 16) == 0 && slot_stride % 4 == 0,
+             "ssm_scan: operands must be 16-byte aligned");
+  if (dtype == BH_F32)
+    return ds_launch(SsmRows<float>{xbc, xbc_stride, (const float*)proj, proj_stride, dt_first, dt_bias, a_log, d_skip, H, vdim, N, G}, seq_start,
+                     seq_slot, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
+  if (dtype == BH_BF16)
+    return ds_launch(SsmRows<bf16_t>{xbc, xbc_stride, (const bf16_t*)proj, proj_stride, dt_first, dt_bias, a_log, d_skip, H, vdim, N, G}, seq_start,
+                     seq_slot, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
   return bh_fail("ssm_scan: unknown dtype %d", dtype);
 }
 

@@ -175,6 +175,8 @@ class KernelSizes:
             "bh_relu_squared": [p, p, i, i, i, i, p],
             "bh_lightning_scan": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
             "bh_lightning_chunks": [i, i, i, i, i, p],
+            "bh_lightning_products": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
+            "bh_ssm_products": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, ctypes.c_long, p],
             "bh_gated_rmsnorm": [p, p, i, i, p, p, i, i, f, i, p],
             "bh_latent_write": [p, i, i, i, p, f, p, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, i, i, i, i, i, p, ctypes.c_long, i, f, p],
             "bh_heads_linear": [p, ctypes.c_long, i, i, p, p, ctypes.c_long, i, i, i, i, i, i, i, i, p],
@@ -235,6 +237,8 @@ class KernelSizes:
             function.restype = i
         lib.bh_gemm_bf16_scratch.argtypes = [i, i, i, i, i]
         lib.bh_gemm_bf16_scratch.restype = ctypes.c_long
+        lib.bh_lightning_products_scratch.argtypes, lib.bh_lightning_products_scratch.restype = [i] * 10, ctypes.c_long
+        lib.bh_ssm_products_scratch.argtypes, lib.bh_ssm_products_scratch.restype = [i] * 8, ctypes.c_long
         for query in (lib.bh_gemm_bf16_norm_blocks, lib.bh_gemm_bf16_takes_norm, lib.bh_gemm_bf16_turns_blocks,
                       lib.bh_gemm_bf16_reads_blocked, lib.bh_gemm_bf16_writes_blocked):
             query.argtypes, query.restype = [i, i, i, i, i], ctypes.c_int
@@ -297,6 +301,9 @@ class KernelSizes:
 
     def ssm_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, vdim, n_state) -> int:
         """Bytes of scratch memory that `ssm_scan` allocates for a step of these sizes (sequences cut into chunks)."""
+        products = int(self.lib.bh_ssm_products_scratch(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim), int(n_state), 1, 0))
+        if products:
+            return _rounded(products * 4)
         if not self.lib.bh_ssm_fast_takes(int(vdim), int(n_state)):
             return 0
         chunk_rows = int(self.lib.bh_ssm_chunk_rows(int(n_seqs), int(max_rows), int(n_heads)))
@@ -1029,6 +1036,9 @@ class HipKernels(KernelSizes):
         """Bytes of scratch memory that `lightning_scan` allocates for a step of these sizes (the states of the chunks it cuts
         long sequences into)."""
         rows = ctypes.c_int(0)
+        products = int(self.lib.bh_lightning_products_scratch(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(dim), int(vdim), 0, 0, 0, 0))
+        if products:
+            return _rounded(products * 4)
         chunks = int(self.lib.bh_lightning_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim), ctypes.byref(rows)))
         return _rounded(n_seqs * chunks * n_heads * dim * vdim * 4) if chunks > 1 else 0
 
@@ -1037,8 +1047,9 @@ class HipKernels(KernelSizes):
         """For every sequence b of the step (rows seq_start[b] .. seq_start[b + 1] - 1 in order, state row seq_slot[b]) and
         head h: S <- decay[h] * S + k_t v_t^T, out_t = S^T q_t with q, k, v = silu of the row's slices from q_off, k_off,
         v_off of `proj` [n, P].  state f32 [slots, H, dim, vdim] in place, out f32 [n, H * vdim].  `max_rows_per_seq`: no
-        sequence of the step brings more rows (the step's total, if it is not given); long sequences that would leave the
-        chip idle are cut into chunks that run side by side, whose states take scratch memory for the length of the call."""
+        sequence of the step brings more rows (the step's total, if it is not given); long sequences go as products of matrices
+        over chunks of rows where the sizes allow it, or, where they would leave the chip idle, are cut into chunks that are walked
+        side by side; the chunks' states take scratch memory for the length of the call."""
         n_rows, stride = proj.shape
         n_seqs = seq_slot.shape[0]
         if (state.dim() != 4 or tuple(state.shape[1:]) != (n_heads, dim, vdim) or tuple(out.shape) != (n_rows, n_heads * vdim)
@@ -1047,10 +1058,15 @@ class HipKernels(KernelSizes):
                               f"{tuple(out.shape)} do not fit {n_heads} heads of {dim} x {vdim} and {n_seqs} sequences")
         f32, i32 = (torch.float32,), (torch.int32,)
         most = min(int(max_rows_per_seq), n_rows) if max_rows_per_seq else n_rows
-        chunk_rows = ctypes.c_int(0)
-        chunks = int(self.lib.bh_lightning_chunks(n_seqs, n_rows, most, n_heads, vdim, ctypes.byref(chunk_rows)))
-        scratch = torch.empty(n_seqs * chunks * n_heads * dim * vdim, dtype=torch.float32, device=self.device) if chunks > 1 else None
-        self._check(self.lib.bh_lightning_scan(
+        entry, floats = self.lib.bh_lightning_products, 0
+        if (proj.data_ptr() | state.data_ptr()) % 16 == 0:
+            floats = int(self.lib.bh_lightning_products_scratch(n_seqs, n_rows, most, n_heads, dim, vdim, stride, int(q_off), int(k_off), int(v_off)))
+        if not floats:
+            chunk_rows = ctypes.c_int(0)
+            chunks = int(self.lib.bh_lightning_chunks(n_seqs, n_rows, most, n_heads, vdim, ctypes.byref(chunk_rows)))
+            entry, floats = self.lib.bh_lightning_scan, n_seqs * chunks * n_heads * dim * vdim if chunks > 1 else 0
+        scratch = torch.empty(floats, dtype=torch.float32, device=self.device) if floats else None
+        self._check(entry(
             self._ptr(proj, "lightning proj"), _code(proj, "lightning proj"), stride, int(q_off), int(k_off), int(v_off),
             self._ptr(state, "lightning state", f32), self._ptr(decay, "lightning decay", f32),
             self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._ptr(out, "lightning out", f32),
@@ -1630,10 +1646,17 @@ class HipKernels(KernelSizes):
                   self._ptr(d_skip, "D", (torch.float32,)), where, stride)
         rest = (self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)),
                 self._ptr(out, "ssm_scan out", (torch.float32,)), n_seqs, n_heads, vdim, n_state, n_groups)
+        most = int(max_rows_per_seq) if max_rows_per_seq else n_rows
+        floats = 0
+        if (xbc.data_ptr() | where) % 16 == 0 and stride % 4 == 0:
+            floats = int(self.lib.bh_ssm_products_scratch(n_seqs, n_rows, most, n_heads, vdim, n_state, n_groups, xbc.shape[1]))
+        if floats:
+            scratch = torch.empty(floats, dtype=torch.float32, device=self.device)
+            self._check(self.lib.bh_ssm_products(*common, *rest, n_rows, most, self._ptr(scratch, "chunk states"), floats, self._stream()))
+            return
         if not self.lib.bh_ssm_fast_takes(int(vdim), int(n_state)):
             self._check(self.lib.bh_ssm_scan(*common, *rest, self._stream()))
             return
-        most = int(max_rows_per_seq) if max_rows_per_seq else n_rows
         chunk_rows = int(self.lib.bh_ssm_chunk_rows(n_seqs, most, n_heads))
         chunks = -(-most // chunk_rows)
         states = decays = cum = None
