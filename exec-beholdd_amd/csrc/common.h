@@ -23,6 +23,13 @@ __device__ inline bf16_t from_f32<bf16_t>(float x) {
   return r;
 }
 
+// Four neighbouring elements in one store; `to` lies on the bytes of four of them.
+__device__ inline void store_four(float* to, float a, float b, float c, float d) { *reinterpret_cast<float4*>(to) = make_float4(a, b, c, d); }
+__device__ inline void store_four(bf16_t* to, float a, float b, float c, float d) {
+  *reinterpret_cast<uint2*>(to) = make_uint2(f32_to_bf16_bits(a) | ((uint32_t)f32_to_bf16_bits(b) << 16),
+                                             f32_to_bf16_bits(c) | ((uint32_t)f32_to_bf16_bits(d) << 16));
+}
+
 // ---- gated activations ----------------------------------------------------------------------
 // act(gate) * up with act(g) = g / (1 + exp(-g (slope + cube g^2))): silu with slope 1 and cube 0, and with slope
 // 2 sqrt(2/pi) and cube 2 sqrt(2/pi) 0.044715 the tanh form of GELU, since (1 + tanh(y)) / 2 = 1 / (1 + exp(-2y)).
