@@ -23,6 +23,23 @@ __device__ inline bf16_t from_f32<bf16_t>(float x) {
   return r;
 }
 
+// ---- rows that are written in blocks of 16 ---------------------------------------------------------------
+// A row puts 16 bytes into each 128-byte line of such a block; the line is whole when its eight rows are there.  Workgroups go to the
+// eight XCDs in turn, each with an L2 of its own, so with a workgroup a row in order the eight parts of a line meet in no cache and
+// go to memory as parts.  Kernels of a workgroup a row therefore take 16 neighbouring rows to an XCD: workgroup i's place on its XCD
+// is i / 8.  The grid is made of whole rounds of 128 workgroups; those beyond the last row have nothing to do.
+// Measured: rmsnorm of 8,160 rows of 4,096 70 -> 47 us, the squared ReLU of 2,048 x 6,144 23 -> 13, one stream's update and norm of
+// 2,048 rows of 4,096 42 -> 24.
+#define BH_ROWS_ROUND 128
+inline unsigned bh_rows_grid(int n_rows, int block_rows) {
+  return block_rows == 16 && n_rows >= BH_ROWS_ROUND ? ((unsigned)n_rows + BH_ROWS_ROUND - 1) / BH_ROWS_ROUND * BH_ROWS_ROUND : (unsigned)n_rows;
+}
+__device__ inline int bh_row_of_block(int block_rows) {
+  if (block_rows != 16 || gridDim.x % BH_ROWS_ROUND) return blockIdx.x;
+  const int place = blockIdx.x / 8;
+  return (place / 16 * 8 + blockIdx.x % 8) * 16 + place % 16;
+}
+
 // Four neighbouring elements in one store; `to` lies on the bytes of four of them.
 __device__ inline void store_four(float* to, float a, float b, float c, float d) { *reinterpret_cast<float4*>(to) = make_float4(a, b, c, d); }
 __device__ inline void store_four(bf16_t* to, float a, float b, float c, float d) {

@@ -472,9 +472,10 @@ extern "C" int bh_lightning_products(const void* proj, int dtype, int row_stride
 // fused projection's rows (before its sigmoid), out in the activation type (rows, or blocks of rows).
 template <typename T>
 __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __restrict__ gate, int gate_stride,
-                                     const float* __restrict__ w, T* __restrict__ out, int width, float eps, int block_rows) {
+                                     const float* __restrict__ w, T* __restrict__ out, int n_rows, int width, float eps, int block_rows) {
   __shared__ float scratch[16];
-  const int r = blockIdx.x;
+  const int r = bh_row_of_block(block_rows);
+  if (r >= n_rows) return;
   const float* row = o + (size_t)r * width;
   const T* g = gate + (size_t)r * gate_stride;
   float ss = 0.f;
@@ -495,9 +496,9 @@ extern "C" int bh_gated_rmsnorm(const float* o, const void* gate, int dtype, int
              "gated_rmsnorm: rows in blocks of %d need bfloat16 and a width that is a multiple of 32 (got %d)", out_block_rows, width);
   const int threads = width >= 2048 ? 1024 : (width >= 512 ? 512 : 256);
   if (dtype == BH_F32)
-    gated_rmsnorm_kernel<float><<<dim3(n_rows), dim3(threads), 0, stream>>>(o, (const float*)gate, gate_stride, w, (float*)out, width, eps, out_block_rows);
+    gated_rmsnorm_kernel<float><<<dim3(n_rows), dim3(threads), 0, stream>>>(o, (const float*)gate, gate_stride, w, (float*)out, n_rows, width, eps, out_block_rows);
   else if (dtype == BH_BF16)
-    gated_rmsnorm_kernel<bf16_t><<<dim3(n_rows), dim3(threads), 0, stream>>>(o, (const bf16_t*)gate, gate_stride, w, (bf16_t*)out, width, eps, out_block_rows);
+    gated_rmsnorm_kernel<bf16_t><<<dim3(bh_rows_grid(n_rows, out_block_rows)), dim3(threads), 0, stream>>>(o, (const bf16_t*)gate, gate_stride, w, (bf16_t*)out, n_rows, width, eps, out_block_rows);
   else
     return bh_fail("gated_rmsnorm: unknown dtype %d", dtype);
   return bh_check_launch("gated_rmsnorm");

@@ -241,15 +241,16 @@ __global__ void streams_update_rmsnorm_kernel(float* __restrict__ x, const float
 
 // The same for up to four streams whose width is a multiple of 4, in 16-byte pieces: a thread keeps PER pieces between the statistic
 // and the write, and has all of its loads on their way together.
-// Bound by the streams' way from memory and back.  Measured, two streams, bfloat16 out: 2,048 rows of 2,048 21 us (31 with an element a
+// Bound by the streams' way from memory and back.  Measured, two streams, bfloat16 out: 2,048 rows of 2,048 19 us (31 with an element a
 // load and a loop over the streams), 16 rows of 4,096 4.9 us (12.2).
 template <typename TO, int S, int PER>
 __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ mix,
                                                    const float* __restrict__ give, const float* __restrict__ scale,
                                                    const float* __restrict__ take, const float* __restrict__ w, TO* __restrict__ out,
-                                                   int width, float eps, int block_rows) {
+                                                   int n_rows, int width, float eps, int block_rows) {
   __shared__ float scratch[16];
-  const int r = blockIdx.x, pieces = width / 4;
+  const int r = bh_row_of_block(block_rows), pieces = width / 4;
+  if (r >= n_rows) return;
   float4* xr = reinterpret_cast<float4*>(x + (size_t)r * S * width);
   const float4* yr = reinterpret_cast<const float4*>(y + (size_t)r * width);
   const float4* scales = reinterpret_cast<const float4*>(scale);
@@ -323,8 +324,8 @@ extern "C" int bh_streams_update_rmsnorm(float* x, const float* y, const float* 
     const int pieces = width / 4, most = n_rows < bh_compute_units() / 4 ? 1024 : streams > 1 && pieces > 1024 ? 512 : 256;
     const int threads = pieces >= most ? most : (pieces + BH_WAVE - 1) / BH_WAVE * BH_WAVE, per = (pieces + threads - 1) / threads;
 #define BH_WIDE(TO, S, PER)                                                                                                          \
-  streams_update_rmsnorm_wide_kernel<TO, S, PER><<<n_rows, threads, 0, stream>>>(x, y, mix, give, scale, take, w, (TO*)out, width, eps, \
-                                                                                 out_block_rows)
+  streams_update_rmsnorm_wide_kernel<TO, S, PER><<<bh_rows_grid(n_rows, out_block_rows), threads, 0, stream>>>(                        \
+      x, y, mix, give, scale, take, w, (TO*)out, n_rows, width, eps, out_block_rows)
 #define BH_WIDE_SIZES(TO, S)            \
   do {                                  \
     if (per == 1) BH_WIDE(TO, S, 1);    \
@@ -392,12 +393,12 @@ __global__ void relu_squared_kernel(const T* __restrict__ x, T* __restrict__ out
 }
 
 // The same in pieces of 16 bytes (4 or 8 neighbouring columns, which lie together in rows and in blocks alike): a thread one piece.
-// 2,048 x 6,144 bfloat16 into blocks 23 us, 32 with an element a thread (a division and a 2-byte store each).
+// 2,048 x 6,144 bfloat16 into blocks 13 us, 32 with an element a thread (a division and a 2-byte store each).
 template <typename T>
-__global__ __launch_bounds__(256) void relu_squared_pieces_kernel(const T* __restrict__ x, T* __restrict__ out, int width, int block_rows) {
+__global__ __launch_bounds__(256) void relu_squared_pieces_kernel(const T* __restrict__ x, T* __restrict__ out, int n_rows, int width, int block_rows) {
   constexpr int N = 16 / sizeof(T);
-  const int row = blockIdx.y, i = N * (blockIdx.x * 256 + threadIdx.x);
-  if (i >= width) return;
+  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  if (row >= n_rows || i >= width) return;
   union {
     uint4 raw;
     T v[N];
@@ -416,11 +417,11 @@ extern "C" int bh_relu_squared(const void* x, void* out, int dtype, int n_rows, 
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && dtype == BH_BF16 && width % 32 == 0 && x != out),
              "relu_squared: rows in blocks of %d need bfloat16, a width that is a multiple of 32 (got %d) and an output of their own",
              out_block_rows, width);
-  if (n_rows <= 65535 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
+  if (width <= 8 * 256 * 65535 / 2 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
     const int n = dtype == BH_F32 ? 4 : 8;
-    const dim3 grid((width / n + 255) / 256, n_rows);
-    if (dtype == BH_F32) relu_squared_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (float*)out, width, out_block_rows);
-    else relu_squared_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, width, out_block_rows);
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (width / n + 255) / 256);
+    if (dtype == BH_F32) relu_squared_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
+    else relu_squared_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
     return bh_check_launch("relu_squared");
   }
   const size_t total = (size_t)n_rows * width;
