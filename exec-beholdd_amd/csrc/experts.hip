@@ -235,11 +235,36 @@ __global__ __launch_bounds__(256) void clamped_glu_kernel(const T* __restrict__ 
   }
 }
 
+// The same in pieces of 16 bytes (4 or 8 neighbouring columns, which lie together in rows and in blocks alike).
+// 2,100 rows of 3,072, bfloat16 into blocks 12.3 us, 24 with an element a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void clamped_glu_pieces_kernel(const T* __restrict__ gu, T* __restrict__ out, int n_rows, int ff, float limit,
+                                                                 float alpha, int out_block_rows, float shift) {
+  constexpr int N = 16 / sizeof(T);
+  const int row = bh_row_of_block(out_block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  if (row >= n_rows || i >= ff) return;
+  union Piece {
+    uint4 raw;
+    T v[N];
+  } gate, up;
+  gate.raw = *reinterpret_cast<const uint4*>(gu + (size_t)row * 2 * ff + i);
+  up.raw = *reinterpret_cast<const uint4*>(gu + (size_t)row * 2 * ff + ff + i);
+#pragma unroll
+  for (int e = 0; e < N; ++e) gate.v[e] = from_f32<T>(clamped_glu(to_f32(gate.v[e]), to_f32(up.v[e]), limit, alpha, shift));
+  *reinterpret_cast<uint4*>(out + bh_rows_index(out_block_rows, row, i, ff)) = gate.raw;
+}
+
 extern "C" int bh_clamped_glu(const void* gu, int dtype, void* out, int n_rows, int ff, float limit, float alpha, int out_block_rows,
                               float shift, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && ff > 0, "clamped_glu: sizes must be positive");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && ff % 32 == 0 && dtype == BH_BF16),
              "clamped_glu: rows in blocks of %d of width %d are not written", out_block_rows, ff);
+  if (ff <= 4 * 256 * 65535 && (((uintptr_t)gu | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && ff % 4 == 0) || (dtype == BH_BF16 && ff % 8 == 0))) {
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (ff / (dtype == BH_F32 ? 4 : 8) + 255) / 256);
+    if (dtype == BH_F32) clamped_glu_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)gu, (float*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
+    else clamped_glu_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)gu, (bf16_t*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
+    return bh_check_launch("clamped_glu");
+  }
   const size_t n = (size_t)n_rows * ff;
   const int blocks = (int)((n + 255) / 256 < 8192 ? (n + 255) / 256 : 8192);
   if (dtype == BH_F32)
@@ -463,11 +488,49 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
   hidden[(size_t)row * D + d] = fresh ? total : hidden[(size_t)row * D + d] + total;
 }
 
+// The same for widths that are multiples of 4, 16 bytes a thread.  2,100 rows of 2,048, four experts a row 17 us, 27 with an element a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void experts_combine_wide_kernel(const float* __restrict__ y, const int32_t* __restrict__ place,
+                                                                   const float* __restrict__ weights, float* __restrict__ hidden,
+                                                                   const T* __restrict__ through, const int32_t* __restrict__ chosen, int E,
+                                                                   int top, int D, int fresh) {
+  const int row = blockIdx.x, d = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (d >= D) return;
+  float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int j = 0; j < top; ++j) {
+    const int pair = row * top + j;
+    float4 share;
+    if (through && chosen[pair] >= E) {
+      const T* own = through + (size_t)row * D + d;
+      share = make_float4(to_f32(own[0]), to_f32(own[1]), to_f32(own[2]), to_f32(own[3]));
+    } else {
+      share = *reinterpret_cast<const float4*>(y + (size_t)(place ? place[pair] : pair) * D + d);
+    }
+    const float f = weights ? weights[pair] : 1.0f;
+    total = make_float4(fmaf(f, share.x, total.x), fmaf(f, share.y, total.y), fmaf(f, share.z, total.z), fmaf(f, share.w, total.w));
+  }
+  float4* to = reinterpret_cast<float4*>(hidden + (size_t)row * D + d);
+  if (!fresh) {
+    const float4 old = *to;
+    total = make_float4(old.x + total.x, old.y + total.y, old.z + total.z, old.w + total.w);
+  }
+  *to = total;
+}
+
 extern "C" int bh_experts_combine(const float* y, const int32_t* place, const float* weights, float* hidden, const void* through,
                                   int dtype, const int32_t* chosen, int E, int n_rows, int top, int D, int fresh, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && top > 0 && D > 0, "experts_combine: sizes must be positive");
   BH_REQUIRE((D + 255) / 256 <= 65535, "experts_combine: rows of up to 16 million outputs");
   BH_REQUIRE(through == nullptr || (chosen != nullptr && E > 0), "experts_combine: inputs that are handed through come with the choices");
+  if (D % 4 == 0 && (((uintptr_t)y | (uintptr_t)hidden) % 16) == 0 && (dtype == BH_F32 || dtype == BH_BF16)) {
+    const dim3 wide(n_rows, (D / 4 + 255) / 256);
+    if (dtype == BH_F32)
+      experts_combine_wide_kernel<float><<<wide, 256, 0, stream>>>(y, place, weights, hidden, (const float*)through, chosen, E, top, D, fresh);
+    else
+      experts_combine_wide_kernel<bf16_t><<<wide, 256, 0, stream>>>(y, place, weights, hidden, (const bf16_t*)through, chosen, E, top, D, fresh);
+    return bh_check_launch("experts_combine");
+  }
   const dim3 grid(n_rows, (D + 255) / 256);
   if (dtype == BH_F32)
     experts_combine_kernel<float><<<grid, 256, 0, stream>>>(y, place, weights, hidden, (const float*)through, chosen, E, top, D, fresh);

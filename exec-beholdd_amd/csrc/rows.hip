@@ -34,11 +34,74 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
   }
 }
 
+// The same for widths that are multiples of 4, in 16-byte pieces that a thread keeps between the mean, the deviations and the write: the
+// row is read once.  2,100 rows of 2,048, bfloat16 out in blocks 9.3 us (18.4 with three passes of single
+// elements), 16 rows 4.1 us (8.6).
+template <typename TO, int PER>
+__global__ void layernorm_wide_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows, const float* __restrict__ w,
+                                      const float* __restrict__ b, TO* __restrict__ out, int n_rows, int width, float eps, int out_block_rows) {
+  __shared__ float scratch[16];
+  const int r = bh_row_of_block(out_block_rows), pieces = width / 4;
+  if (r >= n_rows) return;
+  const float4* src = reinterpret_cast<const float4*>(x + (size_t)(rows ? rows[r] : r) * width);
+  float4 held[PER];
+  float sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    held[k] = i < pieces ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) sum += (held[k].x + held[k].y) + (held[k].z + held[k].w);
+  const float mean = block_sum(sum, scratch) / (float)width;
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    held[k] = make_float4(held[k].x - mean, held[k].y - mean, held[k].z - mean, held[k].w - mean);
+    if (threadIdx.x + k * blockDim.x < pieces)
+      ss += (held[k].x * held[k].x + held[k].y * held[k].y) + (held[k].z * held[k].z + held[k].w * held[k].w);
+  }
+  const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i >= pieces) continue;
+    const float4 f = reinterpret_cast<const float4*>(w)[i], c = b ? reinterpret_cast<const float4*>(b)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    // four neighbouring columns lie together in rows and in blocks alike
+    store_four(out + bh_rows_index(out_block_rows, r, 4 * i, width), held[k].x * inv * f.x + c.x, held[k].y * inv * f.y + c.y,
+               held[k].z * inv * f.z + c.z, held[k].w * inv * f.w + c.w);
+  }
+}
+
+// Threads and pieces a thread of a row: a row on as many waves as have a piece each where the rows are few (their latency is the
+// time), four pieces a thread where the rows fill the chip.
+static void wide_row(int n_rows, int pieces, int* threads, int* per) {
+  const int most = n_rows <= 64 ? 1024 : 256;
+  *threads = pieces >= most ? most : (pieces + BH_WAVE - 1) / BH_WAVE * BH_WAVE;
+  while ((pieces + *threads - 1) / *threads > 4 && *threads < 1024) *threads *= 2;
+  *per = (pieces + *threads - 1) / *threads;
+}
+
+template <typename TO>
+static bool layernorm_wide(const float* x, const int32_t* rows, const float* w, const float* b, TO* out, int n_rows, int width, float eps,
+                           int out_block_rows, hipStream_t stream) {
+  if (width % 4 || width > 4 * 4 * 1024 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) % 16)) return false;
+  int threads, per;
+  wide_row(n_rows, width / 4, &threads, &per);
+  const unsigned grid = bh_rows_grid(n_rows, out_block_rows);
+  if (per == 1) layernorm_wide_kernel<TO, 1><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
+  else if (per == 2) layernorm_wide_kernel<TO, 2><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
+  else layernorm_wide_kernel<TO, 4><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
+  return true;
+}
+
 extern "C" int bh_layernorm(const float* x, const int32_t* rows, const float* w, const float* b, void* out, int out_dtype,
                             int n_rows, int width, float eps, int out_block_rows, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "layernorm: sizes must be positive");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && width % 32 == 0 && out_dtype == BH_BF16),
              "layernorm: rows in blocks of %d of width %d are not written", out_block_rows, width);
+  if (out_dtype == BH_F32 && layernorm_wide(x, rows, w, b, (float*)out, n_rows, width, eps, out_block_rows, stream)) return bh_check_launch("layernorm");
+  if (out_dtype == BH_BF16 && layernorm_wide(x, rows, w, b, (bf16_t*)out, n_rows, width, eps, out_block_rows, stream)) return bh_check_launch("layernorm");
   if (out_dtype == BH_F32)
     layernorm_kernel<float><<<n_rows, 256, 0, stream>>>(x, rows, w, b, (float*)out, width, eps, out_block_rows);
   else if (out_dtype == BH_BF16)
@@ -243,12 +306,32 @@ __global__ __launch_bounds__(256) void cast_concat_kernel(const float* __restric
   }
 }
 
+// The same for widths that are multiples of 8: a thread eight neighbouring columns of a row, which lie together in rows and in blocks
+// alike.  2,100 rows of 2,048 into blocks 10 us, 14.6 with an element a thread.
+template <typename TO>
+__global__ __launch_bounds__(256) void cast_concat_wide_kernel(const float* __restrict__ a, const float* __restrict__ b, TO* __restrict__ out,
+                                                               int n_rows, int width, int out_block_rows) {
+  const int total = b ? 2 * width : width, r = bh_row_of_block(out_block_rows), i = 8 * (blockIdx.y * 256 + threadIdx.x);
+  if (r >= n_rows || i >= total) return;
+  const float4* from = reinterpret_cast<const float4*>(i < width ? a + (size_t)r * width + i : b + (size_t)r * width + i - width);
+  const float4 low = from[0], high = from[1];
+  TO* to = out + bh_rows_index(out_block_rows, r, i, total);
+  store_four(to, low.x, low.y, low.z, low.w);
+  store_four(to + 4, high.x, high.y, high.z, high.w);
+}
+
 extern "C" int bh_cast_concat(const float* a, const float* b, void* out, int out_dtype, int n_rows, int width,
                               int out_block_rows, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "cast_concat: sizes must be positive");
   const int total = b ? 2 * width : width;
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && total % 32 == 0 && out_dtype == BH_BF16),
              "cast_concat: rows in blocks of %d of width %d are not written", out_block_rows, total);
+  if (width % 8 == 0 && total <= 8 * 256 * 65535 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16) == 0 && (out_dtype == BH_F32 || out_dtype == BH_BF16)) {
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (total / 8 + 255) / 256);
+    if (out_dtype == BH_F32) cast_concat_wide_kernel<float><<<grid, 256, 0, stream>>>(a, b, (float*)out, n_rows, width, out_block_rows);
+    else cast_concat_wide_kernel<bf16_t><<<grid, 256, 0, stream>>>(a, b, (bf16_t*)out, n_rows, width, out_block_rows);
+    return bh_check_launch("cast_concat");
+  }
   const size_t n = (size_t)n_rows * total;
   const int blocks = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
   if (out_dtype == BH_F32)
@@ -284,8 +367,45 @@ __global__ __launch_bounds__(256) void rms_scale_add_kernel(float* __restrict__ 
   for (int i = threadIdx.x; i < width; i += blockDim.x) dst[i] += src[i] * inv * w[i];
 }
 
+// The same for widths that are multiples of 4: pieces of 16 bytes that a thread keeps between the statistic and the sum.
+// 2,100 rows of 2,048 10 us, 15.5 in two passes of single elements; 16 rows 4.1 us (6.6).
+template <int PER>
+__global__ void rms_scale_add_wide_kernel(float* __restrict__ h, const float* __restrict__ y, const float* __restrict__ w, int width, float eps) {
+  __shared__ float scratch[16];
+  const int pieces = width / 4;
+  const float4* src = reinterpret_cast<const float4*>(y + (size_t)blockIdx.x * width);
+  float4* dst = reinterpret_cast<float4*>(h + (size_t)blockIdx.x * width);
+  float4 held[PER], old[PER];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    held[k] = i < pieces ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < pieces) old[k] = dst[i];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) ss += (held[k].x * held[k].x + held[k].y * held[k].y) + (held[k].z * held[k].z + held[k].w * held[k].w);
+  const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i >= pieces) continue;
+    const float4 f = reinterpret_cast<const float4*>(w)[i];
+    dst[i] = make_float4(old[k].x + held[k].x * inv * f.x, old[k].y + held[k].y * inv * f.y, old[k].z + held[k].z * inv * f.z,
+                         old[k].w + held[k].w * inv * f.w);
+  }
+}
+
 extern "C" int bh_rms_scale_add(float* h, const float* y, const float* w, int n_rows, int width, float eps, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "rms_scale_add: sizes must be positive");
+  if (width % 4 == 0 && width <= 4 * 4 * 1024 && (((uintptr_t)h | (uintptr_t)y | (uintptr_t)w) % 16) == 0 && h != y) {
+    int threads, per;
+    wide_row(n_rows, width / 4, &threads, &per);
+    if (per == 1) rms_scale_add_wide_kernel<1><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
+    else if (per == 2) rms_scale_add_wide_kernel<2><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
+    else rms_scale_add_wide_kernel<4><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
+    return bh_check_launch("rms_scale_add");
+  }
   rms_scale_add_kernel<<<n_rows, 256, 0, stream>>>(h, y, w, width, eps);
   return bh_check_launch("rms_scale_add");
 }
@@ -302,11 +422,33 @@ __global__ __launch_bounds__(256) void gelu_tanh_kernel(const T* __restrict__ x,
   out[to] = from_f32<T>(gelu_tanh(to_f32(x[at])));
 }
 
+// The same in pieces of 16 bytes (4 or 8 neighbouring columns, which lie together in rows and in blocks alike).
+template <typename T>
+__global__ __launch_bounds__(256) void gelu_tanh_pieces_kernel(const T* __restrict__ x, T* __restrict__ out, int n_rows, int width, int block_rows) {
+  constexpr int N = 16 / sizeof(T);
+  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  if (row >= n_rows || i >= width) return;
+  union {
+    uint4 raw;
+    T v[N];
+  } piece;
+  piece.raw = *reinterpret_cast<const uint4*>(x + (size_t)row * width + i);
+#pragma unroll
+  for (int e = 0; e < N; ++e) piece.v[e] = from_f32<T>(gelu_tanh(to_f32(piece.v[e])));
+  *reinterpret_cast<uint4*>(out + bh_rows_index(block_rows, row, i, width)) = piece.raw;
+}
+
 extern "C" int bh_gelu_tanh(const void* x, void* out, int dtype, int n_rows, int width, int out_block_rows, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "gelu_tanh: nothing to do");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && dtype == BH_BF16 && width % 32 == 0 && x != out),
              "gelu_tanh: rows in blocks of %d need bfloat16, a width that is a multiple of 32 (got %d) and an output of their own",
              out_block_rows, width);
+  if (width <= 4 * 256 * 65535 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (width / (dtype == BH_F32 ? 4 : 8) + 255) / 256);
+    if (dtype == BH_F32) gelu_tanh_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
+    else gelu_tanh_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
+    return bh_check_launch("gelu_tanh");
+  }
   const size_t total = (size_t)n_rows * width;
   const size_t blocks = (total + 255) / 256;
   BH_REQUIRE(blocks <= 2147483647u, "gelu_tanh: too many elements");

@@ -246,6 +246,34 @@ __global__ __launch_bounds__(256) void gate_heads_kernel(const T* __restrict__ a
   }
 }
 
+// The same in pieces of 16 bytes (4 or 8 neighbouring elements of a head, which lie together in rows and in blocks alike).
+template <typename T>
+__global__ __launch_bounds__(256) void gate_heads_pieces_kernel(const T* __restrict__ attended, int pad, const T* __restrict__ gate,
+                                                                int gate_stride, int gate_first, T* __restrict__ out, int n_rows, int H,
+                                                                int vdim, int out_block_rows, int gate_per_head) {
+  constexpr int N = 16 / sizeof(T);
+  const int width = H * vdim, row = bh_row_of_block(out_block_rows), c = N * (blockIdx.y * 256 + threadIdx.x);
+  if (row >= n_rows || c >= width) return;
+  const int head = c / vdim, i = c % vdim;
+  union Piece {
+    uint4 raw;
+    T v[N];
+  } piece, gates;
+  piece.raw = *reinterpret_cast<const uint4*>(attended + ((size_t)row * H + head) * pad + i);
+  if (gate) {
+    const T* own = gate + (size_t)row * gate_stride + gate_first;
+    if (gate_per_head) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) gates.v[e] = own[head];
+    } else {
+      gates.raw = *reinterpret_cast<const uint4*>(own + c);
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) piece.v[e] = from_f32<T>(to_f32(piece.v[e]) / (1.0f + expf(-to_f32(gates.v[e]))));
+  }
+  *reinterpret_cast<uint4*>(out + bh_rows_index(out_block_rows, row, c, width)) = piece.raw;
+}
+
 extern "C" int bh_gate_heads(const void* attended, int dtype, int pad, const void* gate, int gate_stride, int gate_first,
                              void* out, int n_rows, int H, int vdim, int out_block_rows, int gate_per_head, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && H > 0 && vdim > 0 && pad >= vdim, "gate_heads: sizes do not fit");
@@ -253,6 +281,19 @@ extern "C" int bh_gate_heads(const void* attended, int dtype, int pad, const voi
              "gate_heads: the gate lies outside its row");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && (H * vdim) % 32 == 0 && dtype == BH_BF16),
              "gate_heads: rows in blocks of %d of width %d are not written", out_block_rows, H * vdim);
+  const int piece = dtype == BH_F32 ? 4 : 8;
+  const bool gates_on16 = gate == nullptr || gate_per_head || ((uintptr_t)gate % 16 == 0 && gate_stride % piece == 0 && gate_first % piece == 0);
+  if (vdim % piece == 0 && pad % piece == 0 && gates_on16 && (((uintptr_t)attended | (uintptr_t)out) % 16) == 0 && (long)H * vdim <= 4L * 256 * 65535 &&
+      (dtype == BH_F32 || dtype == BH_BF16)) {
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (H * vdim / piece + 255) / 256);
+    if (dtype == BH_F32)
+      gate_heads_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)attended, pad, (const float*)gate, gate_stride, gate_first, (float*)out,
+                                                               n_rows, H, vdim, out_block_rows, gate_per_head);
+    else
+      gate_heads_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)attended, pad, (const bf16_t*)gate, gate_stride, gate_first,
+                                                                (bf16_t*)out, n_rows, H, vdim, out_block_rows, gate_per_head);
+    return bh_check_launch("gate_heads");
+  }
   const size_t n = (size_t)n_rows * H * vdim;
   const int blocks = (int)((n + 255) / 256 < 8192 ? (n + 255) / 256 : 8192);
   if (dtype == BH_F32)
