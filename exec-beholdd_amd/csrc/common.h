@@ -47,6 +47,22 @@ __device__ inline void store_four(bf16_t* to, float a, float b, float c, float d
                                              f32_to_bf16_bits(c) | ((uint32_t)f32_to_bf16_bits(d) << 16));
 }
 
+// The same as loads.
+__device__ inline float4 load_four(const float* from) { return *reinterpret_cast<const float4*>(from); }
+__device__ inline float4 load_four(const bf16_t* from) {
+  const uint2 v = *reinterpret_cast<const uint2*>(from);
+  return make_float4(bf16_bits_to_f32(v.x & 0xffff), bf16_bits_to_f32(v.x >> 16), bf16_bits_to_f32(v.y & 0xffff), bf16_bits_to_f32(v.y >> 16));
+}
+
+// Threads and pieces a thread of a row: a row on as many waves as have a piece each where the rows are few (their latency is the
+// time), four pieces a thread where the rows fill the chip.
+inline void bh_wide_row(int n_rows, int pieces, int* threads, int* per) {
+  const int most = n_rows <= 64 ? 1024 : 256;
+  *threads = pieces >= most ? most : (pieces + BH_WAVE - 1) / BH_WAVE * BH_WAVE;
+  while ((pieces + *threads - 1) / *threads > 4 && *threads < 1024) *threads *= 2;
+  *per = (pieces + *threads - 1) / *threads;
+}
+
 // ---- gated activations ----------------------------------------------------------------------
 // act(gate) * up with act(g) = g / (1 + exp(-g (slope + cube g^2))): silu with slope 1 and cube 0, and with slope
 // 2 sqrt(2/pi) and cube 2 sqrt(2/pi) 0.044715 the tanh form of GELU, since (1 + tanh(y)) / 2 = 1 / (1 + exp(-2y)).

@@ -488,12 +488,66 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
   }
 }
 
+// The same for widths that are multiples of 4, in pieces of four that a thread keeps between the sum and the write: 2,048 rows of 2,048,
+// bfloat16 13.1 us (20.5 with single elements), 16 rows of 2,048 4.3 us (6.7).
+template <typename T, int PER>
+__global__ void gated_rmsnorm_wide_kernel(const float* __restrict__ o, const T* __restrict__ gate, int gate_stride, const float* __restrict__ w,
+                                          T* __restrict__ out, int n_rows, int width, float eps, int block_rows) {
+  __shared__ float scratch[16];
+  const int r = bh_row_of_block(block_rows), pieces = width / 4;
+  if (r >= n_rows) return;
+  const float4* row = reinterpret_cast<const float4*>(o + (size_t)r * width);
+  const T* g = gate + (size_t)r * gate_stride;
+  float4 held[PER], open[PER];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    held[k] = open[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < pieces) {
+      held[k] = row[i];
+      open[k] = load_four(g + 4 * i);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) ss += (held[k].x * held[k].x + held[k].y * held[k].y) + (held[k].z * held[k].z + held[k].w * held[k].w);
+  const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i >= pieces) continue;
+    const float4 f = w ? reinterpret_cast<const float4*>(w)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+    auto gated = [&](float v, float by, float z) { return v * inv * by * (1.0f / (1.0f + expf(-z))); };
+    store_four(out + bh_rows_index(block_rows, r, 4 * i, width), gated(held[k].x, f.x, open[k].x), gated(held[k].y, f.y, open[k].y),
+               gated(held[k].z, f.z, open[k].z), gated(held[k].w, f.w, open[k].w));
+  }
+}
+
+template <typename T>
+static bool gated_rmsnorm_wide(const float* o, const T* gate, int gate_stride, const float* w, T* out, int n_rows, int width, float eps,
+                               int block_rows, hipStream_t stream) {
+  if (width % 4 || gate_stride % 4 || width > 4 * 4 * 1024 || (uintptr_t)gate % (4 * sizeof(T)) || (uintptr_t)out % (4 * sizeof(T)) ||
+      (((uintptr_t)o | (uintptr_t)w) % 16))
+    return false;
+  int threads, per;
+  bh_wide_row(n_rows, width / 4, &threads, &per);
+  const unsigned grid = bh_rows_grid(n_rows, block_rows);
+  if (per == 1) gated_rmsnorm_wide_kernel<T, 1><<<grid, threads, 0, stream>>>(o, gate, gate_stride, w, out, n_rows, width, eps, block_rows);
+  else if (per == 2) gated_rmsnorm_wide_kernel<T, 2><<<grid, threads, 0, stream>>>(o, gate, gate_stride, w, out, n_rows, width, eps, block_rows);
+  else gated_rmsnorm_wide_kernel<T, 4><<<grid, threads, 0, stream>>>(o, gate, gate_stride, w, out, n_rows, width, eps, block_rows);
+  return true;
+}
+
 extern "C" int bh_gated_rmsnorm(const float* o, const void* gate, int dtype, int gate_stride, const float* w, void* out,
                                 int n_rows, int width, float eps, int out_block_rows, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0 && gate_stride >= width, "gated_rmsnorm: rows %d, width %d, gate stride %d", n_rows,
              width, gate_stride);
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && dtype == BH_BF16 && width % 32 == 0),
              "gated_rmsnorm: rows in blocks of %d need bfloat16 and a width that is a multiple of 32 (got %d)", out_block_rows, width);
+  if (dtype == BH_F32 && gated_rmsnorm_wide(o, (const float*)gate, gate_stride, w, (float*)out, n_rows, width, eps, out_block_rows, stream))
+    return bh_check_launch("gated_rmsnorm");
+  if (dtype == BH_BF16 && gated_rmsnorm_wide(o, (const bf16_t*)gate, gate_stride, w, (bf16_t*)out, n_rows, width, eps, out_block_rows, stream))
+    return bh_check_launch("gated_rmsnorm");
   const int threads = width >= 2048 ? 1024 : (width >= 512 ? 512 : 256);
   if (dtype == BH_F32)
     gated_rmsnorm_kernel<float><<<dim3(n_rows), dim3(threads), 0, stream>>>(o, (const float*)gate, gate_stride, w, (float*)out, n_rows, width, eps, out_block_rows);

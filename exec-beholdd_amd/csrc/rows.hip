@@ -73,21 +73,12 @@ __global__ void layernorm_wide_kernel(const float* __restrict__ x, const int32_t
   }
 }
 
-// Threads and pieces a thread of a row: a row on as many waves as have a piece each where the rows are few (their latency is the
-// time), four pieces a thread where the rows fill the chip.
-static void wide_row(int n_rows, int pieces, int* threads, int* per) {
-  const int most = n_rows <= 64 ? 1024 : 256;
-  *threads = pieces >= most ? most : (pieces + BH_WAVE - 1) / BH_WAVE * BH_WAVE;
-  while ((pieces + *threads - 1) / *threads > 4 && *threads < 1024) *threads *= 2;
-  *per = (pieces + *threads - 1) / *threads;
-}
-
 template <typename TO>
 static bool layernorm_wide(const float* x, const int32_t* rows, const float* w, const float* b, TO* out, int n_rows, int width, float eps,
                            int out_block_rows, hipStream_t stream) {
   if (width % 4 || width > 4 * 4 * 1024 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) % 16)) return false;
   int threads, per;
-  wide_row(n_rows, width / 4, &threads, &per);
+  bh_wide_row(n_rows, width / 4, &threads, &per);
   const unsigned grid = bh_rows_grid(n_rows, out_block_rows);
   if (per == 1) layernorm_wide_kernel<TO, 1><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
   else if (per == 2) layernorm_wide_kernel<TO, 2><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
@@ -400,7 +391,7 @@ extern "C" int bh_rms_scale_add(float* h, const float* y, const float* w, int n_
   BH_REQUIRE(n_rows > 0 && width > 0, "rms_scale_add: sizes must be positive");
   if (width % 4 == 0 && width <= 4 * 4 * 1024 && (((uintptr_t)h | (uintptr_t)y | (uintptr_t)w) % 16) == 0 && h != y) {
     int threads, per;
-    wide_row(n_rows, width / 4, &threads, &per);
+    bh_wide_row(n_rows, width / 4, &threads, &per);
     if (per == 1) rms_scale_add_wide_kernel<1><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
     else if (per == 2) rms_scale_add_wide_kernel<2><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
     else rms_scale_add_wide_kernel<4><<<n_rows, threads, 0, stream>>>(h, y, w, width, eps);
