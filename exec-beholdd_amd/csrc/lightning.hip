@@ -2,7 +2,8 @@
 //   S_t = decay_h * S_(t-1) + k_t v_t^T        S [dim][vdim] per (sequence, head), kept between steps
 //   o_t = S_t^T q_t
 // with q, k, v = silu of the rows of one fused projection.  The state, the decay and both products are float32
-// (plain FMA) whatever type the projection rows have.  A workgroup owns a tile of VT value columns of one
+// whatever type the projection rows have.  Prompts of aligned sizes go through decay_scan.h (chunks of 64 rows as matrix
+// products); what follows is the walk that takes every other call of several rows a sequence.  A workgroup owns a tile of VT value columns of one
 // (sequence, head) and walks that sequence's rows of the step in order; a thread owns a slice of `dim` of one
 // column, so the state lives in registers from the first row to the last and memory sees it once each way.
 // The tile is as narrow as it takes to give every compute unit a workgroup (a prompt of one sequence has only

@@ -4,7 +4,8 @@
 //                       y = S^T C + D x.   S is [N][vdim] float32 and lives in the sequence's state region.
 //   gated_group_rmsnorm out = rms_g(y * silu(z)) * w, the root mean square taken in `groups` equal parts of a row; with
 //                       `gate_after` the statistic is y's alone: out = rms_g(y) * w * silu(z)
-// Everything but the reading of dt_raw and z is float32.
+// Everything but the reading of dt_raw and z is float32.  Prompts of aligned sizes go through decay_scan.h (chunks of 64 rows as
+// matrix products) where that is estimated to be faster than the walks below.
 #include "common.h"
 #include "decay_scan.h"
 

@@ -8,8 +8,8 @@
 The four projections are one stacked product.  The state is a fixed-size float32 region of the cache (kind
 "state"): a step continues from what the sequence's slot holds, whatever the step's cut, and a slot starts at
 zero.  State, decay and both products of the recurrence are float32; the projections and their activations have
-the engine's activation type.  One kernel walks a sequence's rows of the step in order with the state in
-registers (`lightning_scan`, prompts and decode steps alike), one norms and gates (`gated_rmsnorm`).
+the engine's activation type.  `lightning_scan` takes a sequence's rows of the step in order, a decode step's row with
+the state in registers and a prompt's in chunks whose work is matrix products; `gated_rmsnorm` norms and gates.
 Every size and the decays are constructor parameters.
 """
 

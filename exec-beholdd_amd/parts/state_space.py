@@ -9,8 +9,8 @@
 
 Per sequence the layer keeps one float32 region: the heads' states, then the last taps - 1 rows of (x, B, C) as they
 were projected.  The step sizes, decays, the state, both products of the recurrence and the norm are float32; the
-projection and the convolution's inputs have the engine's activation type.  One kernel walks a sequence's rows of the
-step in order, so prompts, portions and decode steps are one code path.  Every size is a constructor parameter.
+projection and the convolution's inputs have the engine's activation type.  `ssm_scan` takes a sequence's rows of
+the step in order (long ones in chunks whose work is matrix products), whatever the step's cut.  Every size is a constructor parameter.
 """
 
 from __future__ import annotations
