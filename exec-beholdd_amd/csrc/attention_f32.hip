@@ -133,7 +133,7 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
       const bool seen = at >= first[r] && at <= pos[r];
       score = seen ? score : -INFINITY;
       const float now = fmaxf(most[r], wave_max(score));
-      const float p = seen ? expf(score - now) : 0.f;
+      const float p = score == -INFINITY ? 0.f : expf(score - now);      // also where a seen key's score is: a page of those has now -inf
       alpha[r] = most[r] == -INFINITY ? 0.f : expf(most[r] - now);
       sum[r] = sum[r] * alpha[r] + p;
       most[r] = now;

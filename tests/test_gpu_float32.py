@@ -112,3 +112,21 @@ def test_float32_attention_score_forms_and_ends(K):
                     dev(table), dev(torch.arange(3, dtype=torch.int32)), dev(positions), n_heads, kv_heads, size, 0.2, **more)
         outs.append(out.reshape(3, n_heads, size)[..., :40].double())
     assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("rows", [1, 12])
+@pytest.mark.parametrize("blind", [(64, 128), (0, 64), (60, 200), (128, 197)])
+def test_float32_attention_pages_of_keys_that_are_infinitely_far(K, rows, blind):
+    """Keys with a score of minus infinity, a wave's whole first page of them, count for nothing beside keys that are seen."""
+    n_heads, kv_heads, head_dim, length = 4, 2, 64, 300
+    kp, vp, table, keys, values = make_cache(1, [length], kv_heads, head_dim, torch.float32, seed=rows)
+    for t in range(*blind):
+        kp[int(table[0, t // 64]), :, t % 64] = keys[0][t] = float("-inf")
+    positions = torch.arange(length - rows, length, dtype=torch.int32)
+    q = torch.rand(rows, n_heads * head_dim, generator=torch.Generator().manual_seed(2)) + 0.1
+    out = torch.full(q.shape, float("nan"), device="cuda:0")
+    layout = Layout(rows == 1, dev(torch.tensor([0, rows], dtype=torch.int32)), 1, rows, length - 1)
+    K.attention(dev(q), out, dev(kp), dev(vp), dev(table), dev(torch.zeros(rows, dtype=torch.int32)), dev(positions), n_heads, kv_heads, head_dim,
+                head_dim ** -0.5, layout=layout)
+    want = attention_reference_rows(q, keys[0], values[0], positions.long(), n_heads, kv_heads, head_dim, head_dim ** -0.5, 0)
+    assert float((out.cpu().double() - want).abs().max() / want.abs().max()) < 1e-5
