@@ -15,11 +15,13 @@
 // needs rows / 64 + sequences places, and a window of them at a time has memory for its states.
 // Bound by the matrix instructions and the operands' reads from LDS beside them; a state is written once and read twice.
 // Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 83 us in all (26 + 18 +
-// 39), 233 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 163 us, 606.  With the values in LDS beside the
+// 39), 233 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 165 us, 606.  With the values in LDS beside the
 // keys, one workgroup a compute unit, 102 and 213.
 #pragma once
 
 #include "common.h"
+
+#include <type_traits>
 
 #define DS_ROWS 64                    // rows of a chunk
 #define DS_MOST_VALUES 256             // elements of a value
@@ -171,6 +173,7 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
   extern __shared__ __align__(16) float ds_lds[];
   __shared__ ScanDecays<In::POWERS> decays;
   __shared__ float weights[DS_ROWS];
+  __shared__ int any_spoilt;      // whether a value of the chunk is not finite
   const int head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const ScanChunk at = ds_find(seq_start, n_seqs, place0 + blockIdx.x);
   if (at.rows == 0) return;
@@ -194,6 +197,7 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
     const int e = tid + 512 * u, r = e / (V / 4), i = 4 * (e % (V / 4));
     values[u] = r < at.rows && e < DS_ROWS * V / 4 ? in.v4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  if (tid == 0) any_spoilt = 0;
   __syncthreads();
   // scores: the ten 16 x 16 tiles on and below the diagonal, a wave one or two.  A lane's 16 bytes are k 16 b + 4 g .. + 3 of its row
   // for either operand, which the matrix instructions take in turn.
@@ -235,12 +239,16 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
       p_lds[tile * 16 * DS_PSTRIDE + (4 * g + r) * DS_PSTRIDE + j] = p;
     }
   }
+  float zero = 0.f;      // zero times every value: NaN where one is not finite
 #pragma unroll
   for (int u = 0; u < DS_MOST_VALUES / 32; ++u) {
     const int e = tid + 512 * u;
     if (e < DS_ROWS * V / 4) *reinterpret_cast<float4*>(v_lds + e / (V / 4) * vs + 4 * (e % (V / 4))) = values[u];
+    zero = fmaf(values[u].w, 0.f, fmaf(values[u].z, 0.f, fmaf(values[u].y, 0.f, fmaf(values[u].x, 0.f, zero))));
   }
+  if (zero != 0.f) any_spoilt = 1;
   __syncthreads();
+  const bool spoilt = any_spoilt;
   // outputs: 32 rows x 16 columns at a time
   const float* start = states + ((size_t)blockIdx.x * H + head) * D * V;
   for (int unit = wave; unit < 2 * (V / 16); unit += 8) {
@@ -263,18 +271,44 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
     const int tr = r0 / 16;
     const float* p_row = p_lds + tr * (tr + 1) / 2 * 16 * DS_PSTRIDE + j * DS_PSTRIDE + 4 * g;      // the upper 16 rows' tiles; then the lower's
     const float* p_lower = p_row + (tr + 1) * 16 * DS_PSTRIDE;
-    for (int b = 0; b < r0 + 32; b += 16) {
-      float v[4];
+    auto add_rows = [&](auto guarded) {
+      for (int b = 0; b < r0 + 32; b += 16) {
+        float v[4], own[4];      // own: what the tile on the diagonal takes
 #pragma unroll
-      for (int t = 0; t < 4; ++t) v[t] = v_lds[(b + 4 * g + t) * vs + c0 + j];
-      const ds_f32x4_t p1 = *reinterpret_cast<const ds_f32x4_t*>(p_lower + b * DS_PSTRIDE);
-      if (b <= r0) {      // the upper 16 rows see no later ones
-        const ds_f32x4_t p0 = *reinterpret_cast<const ds_f32x4_t*>(p_row + b * DS_PSTRIDE);
+        for (int t = 0; t < 4; ++t) {
+          v[t] = v_lds[(b + 4 * g + t) * vs + c0 + j];
+          own[t] = !guarded || isfinite(v[t]) ? v[t] : 0.f;
+        }
+        const ds_f32x4_t p1 = *reinterpret_cast<const ds_f32x4_t*>(p_lower + b * DS_PSTRIDE);
+        if (b <= r0) {      // the upper 16 rows see no later ones
+          const ds_f32x4_t p0 = *reinterpret_cast<const ds_f32x4_t*>(p_row + b * DS_PSTRIDE);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[t], v[t], acc[t & 1][0], 0, 0, 0);
+          for (int t = 0; t < 4; ++t)
+            acc[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[t], guarded && b == r0 ? own[t] : v[t], acc[t & 1][0], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[t], guarded && b == r0 + 16 ? own[t] : v[t], acc[t & 1][1], 0, 0, 0);
       }
+    };
+    if (!spoilt) {
+      add_rows(std::false_type{});
+    } else {
+      // Scores above the diagonal are zeros, but zero times infinity is not: a value that is not finite stays out of the product of
+      // its own rows' tile and is added by itself, to its row and the later ones.
+      add_rows(std::true_type{});
+      for (int x = 0; x < 2; ++x) {
+        const float* p_tile = p_lds + ((tr + x) * (tr + x + 1) / 2 + tr + x) * 16 * DS_PSTRIDE;
+        for (int c = 0; c < 16; ++c) {
+          const float v = v_lds[(r0 + 16 * x + c) * vs + c0 + j];
+          if (isfinite(v)) continue;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[t], v[t], acc[t & 1][1], 0, 0, 0);
+          for (int r = 0; r < 4; ++r) {
+            const float added = fmaf(p_tile[(4 * g + r) * DS_PSTRIDE + c], v, acc[0][x][r]);
+            if (c <= 4 * g + r) acc[0][x][r] = added;
+          }
+        }
+      }
     }
 #pragma unroll
     for (int x = 0; x < 2; ++x)

@@ -97,3 +97,40 @@ def test_scans_of_sizes_that_are_no_whole_tiles_keep_their_walk(K):
         assert K.lib.bh_lightning_products_scratch(1, 500, 500, heads, dim, vdim, 4096, 0, 1024, 2048) == 0
     assert K.lib.bh_lightning_products_scratch(1, 500, 500, 2, 64, 64, 514, 0, 128, 256) == 0       # rows that lie on no 16 bytes
     assert K.lib.bh_lightning_products_scratch(8, 8, 1, 2, 64, 64, 512, 0, 128, 256) == 0           # a decode step
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("row", [0, 16, 37, 63, 64, 111, 190, 199])
+@pytest.mark.parametrize("kind", ["lightning", "state space"])
+def test_a_value_that_is_not_finite_reaches_no_earlier_row(K, kind, row, value):
+    """The rows before it, the other columns' rows, heads and sequences have the bits that they have without it; its own row and the
+    later ones are not finite in its column, as in the recurrence."""
+    heads, dim, vdim, lengths, column = 2, 64, 48, [200, 130], 21
+    total, width = sum(lengths), heads * vdim
+    g = torch.Generator().manual_seed(row)
+    starts, slots = dev(torch.tensor([0, 200, 330], dtype=torch.int32)), dev(torch.tensor([1, 0], dtype=torch.int32))
+    keys = heads * dim
+    rows = torch.randn(total, 2 * keys + width, generator=g).cuda()      # q, k, v, or v, k, q
+    rates, state = torch.randn(total, heads, generator=g).cuda(), torch.randn(2, heads, dim, vdim, generator=g).cuda()
+    first = 2 * keys if kind == "lightning" else 0
+
+    def run(rows):
+        out, held = torch.full((total, width), 7.0, device="cuda:0"), state.clone()
+        if kind == "lightning":
+            K.lightning_scan(rows, 0, keys, 2 * keys, held, dev(torch.tensor([0.9, 0.99])), starts, slots, out, heads, dim, vdim, max_rows_per_seq=200)
+        else:
+            zero = torch.zeros(heads, device="cuda:0")
+            K.ssm_scan(rows, rates, 0, zero - 2.0, zero, zero + 1.0, held.view(2, -1), 0, starts, slots, out, heads, vdim, dim, heads, max_rows_per_seq=200)
+        return out, held
+
+    assert K.lib.bh_lightning_products_scratch(2, total, 200, heads, dim, vdim, rows.shape[1], 0, keys, 2 * keys) > 0
+    assert K.lib.bh_ssm_products_scratch(2, total, 200, heads, vdim, dim, heads, rows.shape[1]) > 0
+    clean, _ = run(rows)
+    spoilt = rows.clone()
+    spoilt[row, first + vdim + column] = value      # head 1
+    got, held = run(spoilt)
+    at = vdim + column
+    assert torch.isfinite(clean).all() and not torch.isfinite(got[row:200, at]).any()
+    assert not torch.isfinite(held[1, 1, :, column]).any()
+    got[row:200, at] = clean[row:200, at]
+    assert torch.equal(got, clean)
