@@ -45,8 +45,9 @@ __device__ inline ScanChunk ds_find(const int32_t* __restrict__ seq_start, int n
     const int s = s0 + lane;
     upto += __popcll(__ballot(s < n_seqs && ds_place_of(seq_start, s < n_seqs ? s : 0) <= place));
   }
-  ScanChunk at;
-  at.seq = __builtin_amdgcn_readfirstlane(upto - 1);      // the first sequence starts at place 0
+  ScanChunk at = {0, 0, 0, 0};
+  if (upto == 0) return at;      // a place before the first sequence's, where rows of nobody lie ahead of it
+  at.seq = __builtin_amdgcn_readfirstlane(upto - 1);
   at.chunk = place - ds_place_of(seq_start, at.seq);
   at.first = seq_start[at.seq] + at.chunk * DS_ROWS;
   at.rows = min(DS_ROWS, seq_start[at.seq + 1] - at.first);

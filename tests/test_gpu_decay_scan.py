@@ -134,3 +134,30 @@ def test_a_value_that_is_not_finite_reaches_no_earlier_row(K, kind, row, value):
     assert not torch.isfinite(held[1, 1, :, column]).any()
     got[row:200, at] = clean[row:200, at]
     assert torch.equal(got, clean)
+
+
+@pytest.mark.parametrize("first", [63, 64, 70, 200])
+def test_scans_of_sequences_that_start_behind_the_step_s_first_row(K, first):
+    """Rows before the first sequence belong to nobody: neither read nor written."""
+    heads, dim, vdim, lengths = 2, 64, 64, [150, 1, 128]
+    total, keys, width = first + sum(lengths), heads * dim, heads * vdim
+    g = torch.Generator().manual_seed(first)
+    rows = torch.randn(total, 2 * keys + width, generator=g).cuda()
+    rows[:first] = float("nan")
+    rates, state = torch.randn(total, heads, generator=g).cuda(), torch.randn(3, heads, dim, vdim, generator=g).cuda()
+    starts = np.concatenate([[first], first + np.cumsum(lengths)]).astype(np.int32)
+    slots, zero = dev(torch.tensor([2, 0, 1], dtype=torch.int32)), torch.zeros(heads, device="cuda:0")
+    for shift in (0, first):      # as they lie, and without those rows
+        at = dev(torch.from_numpy(starts - shift))
+        outs = [torch.full((total - shift, width), 7.0, device="cuda:0") for _ in range(2)]
+        held = [state.clone() for _ in range(2)]
+        K.lightning_scan(rows[shift:].contiguous(), 0, keys, 2 * keys, held[0], dev(torch.tensor([0.9, 0.99])), at, slots, outs[0], heads, dim, vdim,
+                         max_rows_per_seq=150)
+        K.ssm_scan(rows[shift:].contiguous(), rates[shift:].contiguous(), 0, zero - 2.0, zero, zero + 1.0, held[1].view(3, -1), 0, at, slots, outs[1],
+                   heads, vdim, dim, heads, max_rows_per_seq=150)
+        if shift == 0:
+            behind = outs, held
+    for a, b in zip(behind[0], outs):
+        assert bool((a[:first] == 7.0).all()) and torch.isfinite(b).all() and torch.equal(a[first:], b)
+    for a, b in zip(behind[1], held):
+        assert torch.equal(a, b)
