@@ -338,6 +338,20 @@ extern "C" int bh_lightning_chunks(int n_seqs, int n_rows, int max_rows, int H, 
   return (max_rows + rows - 1) / rows;
 }
 
+// Chunks of all sequences together, at most, over the steps of up to n_seqs sequences, n_rows rows and max_rows rows a sequence (0: no
+// such step is cut): fewer sequences are cut into more chunks each.
+extern "C" long bh_lightning_most_chunks(int n_seqs, int n_rows, int max_rows, int H, int vdim) {
+  const long tiles = (vdim + 63) / 64, wanted = 2L * bh_compute_units();
+  long most = 0;
+  for (long n = 1; n <= n_seqs && n * H * tiles < wanted; ++n) {
+    const long longest = n_rows - n + 1 < max_rows ? n_rows - n + 1 : max_rows;      // the other sequences bring a row each
+    if (longest < 128) break;
+    const long cuts = (wanted + n * H * tiles - 1) / (n * H * tiles), pieces = (longest + 63) / 64, chunks = cuts < pieces ? cuts : pieces;
+    if (chunks > 1 && n * chunks > most) most = n * chunks;
+  }
+  return most;
+}
+
 template <typename T, int DPT, int VT>
 static int launch_lightning(const void* proj, int row_stride, int q_off, int k_off, int v_off, float* state,
                             const float* decay, const int32_t* seq_start, const int32_t* seq_slot, float* out, int n_seqs,
@@ -449,7 +463,11 @@ extern "C" long bh_lightning_products_scratch(int n_seqs, int n_rows, int max_ro
   if (max_rows < 128) return 0;
   return ds_scratch_floats(n_seqs, n_rows, H, dim, vdim);
 }
-// As bh_lightning_scan; proj, state and out lie on 16 bytes.
+// The most that it can be for a step of up to so many sequences and rows (more of either never takes less), whichever form is faster.
+extern "C" long bh_lightning_products_most(int n_seqs, int n_rows, int max_rows, int H, int dim, int vdim) {
+  return max_rows < 128 || n_seqs < 1 || n_rows < 128 || H < 1 || dim < 1 || vdim < 1 ? 0 : ds_scratch_floats(n_seqs, n_rows, H, dim, vdim);
+}
+// As bh_lightning_scan; proj, state and scratch lie on 16 bytes.
 extern "C" int bh_lightning_products(const void* proj, int dtype, int row_stride, int q_off, int k_off, int v_off, float* state,
                                      const float* decay, const int32_t* seq_start, const int32_t* seq_slot, float* out, int n_seqs,
                                      int n_rows, int max_rows, int H, int dim, int vdim, float* scratch, long scratch_floats,

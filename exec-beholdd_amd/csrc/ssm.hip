@@ -272,6 +272,20 @@ extern "C" int bh_ssm_chunk_rows(int n_seqs, int max_rows, int H) {
   return (rows + SS_STAGE - 1) / SS_STAGE * SS_STAGE;
 }
 
+// Chunks of all sequences together, at most, over the steps of up to n_seqs sequences, n_rows rows and max_rows rows a sequence (0: no
+// such step is cut).
+extern "C" long bh_ssm_most_chunks(int n_seqs, int n_rows, int max_rows, int H) {
+  const long enough = 2L * bh_compute_units();
+  long most = 0;
+  for (long n = 1; n <= n_seqs; ++n) {
+    const long longest = n_rows - n + 1 < max_rows ? n_rows - n + 1 : max_rows;      // the other sequences bring a row each
+    const long wanted = (enough + n * H - 1) / (n * H), pieces = longest / 64, chunks = wanted < pieces ? wanted : pieces;
+    if (longest <= 128 || wanted < 2) break;
+    if (n * chunks > most) most = n * chunks;
+  }
+  return most;
+}
+
 // Whether the recurrence with the state in registers takes these sizes (otherwise bh_ssm_scan walks with the state in LDS).
 extern "C" int bh_ssm_fast_takes(int vdim, int N) {
   if (vdim > 256 || vdim < 1 || N < 1) return 0;
@@ -384,6 +398,10 @@ extern "C" long bh_ssm_products_scratch(int n_seqs, int n_rows, int max_rows, in
   const long whole = (long)n_seqs * ((max_rows + DS_ROWS - 1) / DS_ROWS), places = ds_places(n_seqs, n_rows);
   if (max_rows < DS_ROWS || 760L * max_rows <= (long)DS_ROWS * H * (whole < places ? whole : places) + 10000) return 0;
   return ds_scratch_floats(n_seqs, n_rows, H, N, vdim);
+}
+// The most that it can be for a step of up to so many sequences and rows (more of either never takes less), whichever form is faster.
+extern "C" long bh_ssm_products_most(int n_seqs, int n_rows, int max_rows, int H, int vdim, int N) {
+  return max_rows < DS_ROWS || n_seqs < 1 || n_rows < DS_ROWS || H < 1 || vdim < 1 || N < 1 ? 0 : ds_scratch_floats(n_seqs, n_rows, H, N, vdim);
 }
 // As bh_ssm_scan; xbc, the state and its stride lie on 16 bytes.
 extern "C" int bh_ssm_products(const float* xbc, int xbc_stride, const void* proj, int dtype, int proj_stride, int dt_first,

@@ -237,8 +237,9 @@ class KernelSizes:
             function.restype = i
         lib.bh_gemm_bf16_scratch.argtypes = [i, i, i, i, i]
         lib.bh_gemm_bf16_scratch.restype = ctypes.c_long
-        lib.bh_lightning_products_scratch.argtypes, lib.bh_lightning_products_scratch.restype = [i] * 10, ctypes.c_long
-        lib.bh_ssm_products_scratch.argtypes, lib.bh_ssm_products_scratch.restype = [i] * 8, ctypes.c_long
+        for query, count in ((lib.bh_lightning_products_scratch, 10), (lib.bh_ssm_products_scratch, 8), (lib.bh_lightning_products_most, 6),
+                             (lib.bh_ssm_products_most, 6), (lib.bh_lightning_most_chunks, 5), (lib.bh_ssm_most_chunks, 4)):
+            query.argtypes, query.restype = [i] * count, ctypes.c_long
         for query in (lib.bh_gemm_bf16_norm_blocks, lib.bh_gemm_bf16_takes_norm, lib.bh_gemm_bf16_turns_blocks,
                       lib.bh_gemm_bf16_reads_blocked, lib.bh_gemm_bf16_writes_blocked):
             query.argtypes, query.restype = [i, i, i, i, i], ctypes.c_int
@@ -300,18 +301,22 @@ class KernelSizes:
         return _rounded(words * 4) + 4 * _rounded(n_rows * 4)
 
     def ssm_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, vdim, n_state) -> int:
-        """Bytes of scratch memory that `ssm_scan` allocates for a step of these sizes (sequences cut into chunks)."""
-        products = int(self.lib.bh_ssm_products_scratch(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim), int(n_state), 1, 0))
-        if products:
-            return _rounded(products * 4)
+        """Bytes of scratch memory that `ssm_scan` allocates at most in a step of up to so many sequences, rows and rows a sequence
+        (fewer sequences may take more than many: what they are cut into, and whether they go as products, depends on both)."""
+        products = _rounded(int(self.lib.bh_ssm_products_most(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim), int(n_state))) * 4)
         if not self.lib.bh_ssm_fast_takes(int(vdim), int(n_state)):
-            return 0
-        chunk_rows = int(self.lib.bh_ssm_chunk_rows(int(n_seqs), int(max_rows), int(n_heads)))
-        chunks = -(-int(max_rows) // chunk_rows)
-        if chunks <= 1:
-            return 0
-        return (_rounded(n_seqs * chunks * n_heads * n_state * vdim * 4) + _rounded(n_seqs * chunks * n_heads * 4)
-                + _rounded(n_rows * n_heads * 4))
+            return products
+        chunks = int(self.lib.bh_ssm_most_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads)))
+        if not chunks:
+            return products
+        return max(products, _rounded(chunks * n_heads * n_state * vdim * 4) + _rounded(chunks * n_heads * 4) + _rounded(n_rows * n_heads * 4))
+
+    def lightning_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, dim, vdim) -> int:
+        """Bytes of scratch memory that `lightning_scan` allocates at most in a step of up to so many sequences, rows and rows a
+        sequence (the states of the chunks it cuts long sequences into; fewer sequences may take more than many)."""
+        products = int(self.lib.bh_lightning_products_most(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(dim), int(vdim)))
+        chunks = int(self.lib.bh_lightning_most_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim)))
+        return _rounded(max(products, chunks * n_heads * dim * vdim) * 4)
 
     def gla_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, dim, vdim) -> int:
         """Bytes of scratch memory that `gla_scan` allocates for a step of these sizes (long sequences cut into chunks)."""
@@ -1032,16 +1037,6 @@ class HipKernels(KernelSizes):
                                              _code(x, "relu_squared x"), x.shape[0], x.shape[1], _block_rows(out), self._stream()))
 
     # ---- linear attention with a decay, as a recurrence over a float32 state ----
-    def lightning_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, dim, vdim) -> int:
-        """Bytes of scratch memory that `lightning_scan` allocates for a step of these sizes (the states of the chunks it cuts
-        long sequences into)."""
-        rows = ctypes.c_int(0)
-        products = int(self.lib.bh_lightning_products_scratch(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(dim), int(vdim), 0, 0, 0, 0))
-        if products:
-            return _rounded(products * 4)
-        chunks = int(self.lib.bh_lightning_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(vdim), ctypes.byref(rows)))
-        return _rounded(n_seqs * chunks * n_heads * dim * vdim * 4) if chunks > 1 else 0
-
     def lightning_scan(self, proj, q_off, k_off, v_off, state, decay, seq_start, seq_slot, out, n_heads, dim, vdim,
                        max_rows_per_seq=None):
         """For every sequence b of the step (rows seq_start[b] .. seq_start[b + 1] - 1 in order, state row seq_slot[b]) and
