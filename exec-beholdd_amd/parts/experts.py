@@ -20,9 +20,9 @@ all.  The (row, choice) pairs are grouped by expert on the device (`experts_grou
 workgroup per expert and block of outputs that reads the expert's rows from memory once for all of its pairs (`experts_tiles`
 on the matrix cores from the packed form of the matrices, or `experts_rows` for sizes and element types that one does not take), with nothing that depends on the routing on the host, so that decode steps can be captured.  A step
 of many rows (a prompt) runs all experts' products from the packed matrices in two launches too (`experts_many`: the workgroups
-find their tiles of pairs in the counts by themselves, the activation rides in the first product).  For sizes and element types
-that the packed form does not take it reads the experts' counts on the host (the step waits for the device there), lays the pairs'
-inputs side by side, expert after expert, and runs the framework's matrix products on each expert's stretch.  Sizes
+find their tiles of pairs in the counts by themselves, the activation rides in the first product), unless an expert's products are
+large.  Those, and sizes and element types that the packed form does not take, wait for the experts' counts on the host, lay the
+pairs' inputs side by side, expert after expert, and run the framework's matrix products on each expert's stretch.  Sizes
 that the grouped kernels do not take go pair by pair (`experts_gate_up`, `experts_down`).  In every form a row's
 experts' shares are added in the order of its own choice, so its result depends on its batch-mates by rounding at most.  The routing is left in
 `ctx.extras["routing"]` ((chosen, weights) of the last layer that ran).  Every size and constant is a constructor
@@ -83,6 +83,12 @@ class RoutedExperts:
     writes_fresh = True       # forward(..., fresh=True) writes its result instead of adding it
     PRODUCT_PAIRS = 16        # from that many pairs an expert on average, a step of many rows runs matrix products
     PACK_FOR_PROMPTS = True   # keep a second copy of every expert's matrices in the form the products of many rows read fastest
+    # A prompt's experts run as one launch over all of them up to so many pairs x hidden x ff an expert on average, beyond that as
+    # products one by one: the one launch reaches 0.37 to 0.55 PFLOP/s whatever the size, a product of its own costs the host's wait
+    # for the counts, the gathered rows and about 25 us, and then reaches 0.8 to 1.0.  One launch / one by one, us, 8 experts: width
+    # 4,096, ff 1,536 at 2,048 pairs an expert 1,057 / 1,254, at 4,096 2,046 / 1,871; ff 4,096 at 1,024 1,320 / 1,384, at 2,048
+    # 2,470 / 2,245; ff 14,336 at 256 1,443 / 1,405, at 2,048 8,532 / 5,681; 4 to 128 experts cross at the same work.
+    ONE_LAUNCH_WORK = 1.8e10
     WIDE_ROUTER = 128         # a router of fewer outputs is kept with that many for steps of more than WIDE_FROM_ROWS rows: products
     WIDE_FROM_ROWS = 32       # that cut K into parts need a whole tile of outputs (2,048 rows, 40 experts: 71 -> 22 us)
 
@@ -105,8 +111,9 @@ class RoutedExperts:
         self.router_wide = None       # the router's matrix with rows of zeros behind it, as the products of many rows take it
         self.has_router_bias = bool(router_bias)
         self.router_bias = self.correction = self.w_gate_up = self.w_down = None
-        self.for_products = None      # per expert (gate and up, down) as the matrix products take them
+        self.for_products = None      # per expert (gate and up, down) as the matrix products take them: its part of `packed` where there is one
         self.packed = None            # all experts' matrices one below the other (gate and up, down), as experts_tiles and experts_many take them
+        self.in_one_launch = False    # a prompt's products may run as one launch over all experts (kernels.experts_many)
 
     def tensor_specs(self):
         specs = self.router.tensor_specs()
@@ -150,6 +157,10 @@ class RoutedExperts:
         tiles = getattr(kernels, "experts_tiles_take", None)
         if tiles is not None and tiles(self.w_gate_up.dtype, self.hidden, self.ff) and tiles(self.w_down.dtype, self.ff, self.hidden):
             self.packed = (kernels.pack_weight(self.w_gate_up.view(-1, self.hidden)), kernels.pack_weight(self.w_down.view(-1, self.ff)))
+            self.in_one_launch = True
+            # blocks of 16 rows do not straddle experts: an expert's own packed matrices lie side by side in these
+            self.for_products = list(zip(*([type(whole)(part, whole.shape[0] // self.n_experts, whole.shape[1])
+                                            for part in whole.data.view(self.n_experts, -1)] for whole in self.packed)))
         elif self.PACK_FOR_PROMPTS and hasattr(kernels, "pack_weight"):
             self.for_products = [(kernels.pack_weight(self.w_gate_up[e]), kernels.pack_weight(self.w_down[e])) for e in range(self.n_experts)]
 
@@ -160,7 +171,7 @@ class RoutedExperts:
         total += 2 * step.matrix(step.rows, self.top, 4)
         pairs = step.rows * self.top
         total += step.matrix(self.n_experts, step.rows, 4) + step.matrix(pairs, self.ff) + step.matrix(pairs, self.hidden, 4)
-        in_place = step.act_size == 2 and self.hidden % 64 == 0 and self.ff % 64 == 0
+        in_place = step.act_size == 2 and self.hidden % 64 == 0 and self.ff % 64 == 0 and self._one_launch_is_faster(pairs)
         if not in_place and step.rows > step.seqs and pairs >= self.PRODUCT_PAIRS * self.n_experts:      # a step of many rows: the pairs' inputs, gate and up
             total += step.matrix(pairs, self.hidden) + step.matrix(pairs, 2 * self.ff) + step.matrix(pairs, 1, 4)
         return total + (self.shared.working_bytes(step) if self.shared is not None else 0)
@@ -202,7 +213,7 @@ class RoutedExperts:
             counts = torch.empty((self.n_experts,), dtype=torch.int32, device=ctx.device)
             k.experts_group(chosen, lists, counts)
             many = pairs >= self.PRODUCT_PAIRS * self.n_experts
-            if self.packed is not None or ctx.is_decode or not many:
+            if ctx.is_decode or not many or (self.in_one_launch and self._one_launch_is_faster(pairs)):
                 inner = ctx.new_activations(pairs, self.ff)
                 y = ctx.new_f32(pairs, self.hidden)
                 if self.packed is not None:
@@ -217,6 +228,9 @@ class RoutedExperts:
         if self.shared is not None:
             self.shared.forward(ctx, x, hidden)
         return None
+
+    def _one_launch_is_faster(self, pairs: int) -> bool:
+        return pairs * self.hidden * self.ff <= self.ONE_LAUNCH_WORK * self.n_experts
 
     def _combine(self, k, y, place, weights, hidden, adding=None):
         adding = adding or {}

@@ -300,7 +300,7 @@ def test_routing_by_corrected_softmax_scores(K, rows, experts, top):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,identity,top,ff", [(1, 64, 4, 2, 1, 40), (37, 192, 8, 3, 3, 96), (5, 130, 5, 1, 6, 33), (700, 256, 16, 4, 2, 64),
                                                                 (300, 128, 4, 4, 1, 128), (260, 72, 2, 6, 2, 24), (64, 1024, 8, 8, 4, 256)])
-def test_experts_some_of_which_hand_their_input_through(K, dtype, rows, width, experts, identity, top, ff):
+def test_experts_some_of_which_hand_their_input_through(K, monkeypatch, dtype, rows, width, experts, identity, top, ff):
     """The part with its forms (pair by pair for odd sizes, an expert's rows at once, products over gathered rows, in one launch and
     one by one) against the plain experts, written over what stood there and added to it; scratch memory that holds nothing
     finite must not reach a row."""
@@ -323,6 +323,13 @@ def test_experts_some_of_which_hand_their_input_through(K, dtype, rows, width, e
     assert (chosen >= experts).any() or rows == 1
     choice = np.sort(plain.softmax(plain.linear(h, names["m.router"])) + names["m.correction"], axis=-1)
     sure = torch.from_numpy(choice[:, -top] - choice[:, -top - 1] > 1e-4 if top < experts + identity else np.ones(rows, bool))
+    called = []
+    for name in ("experts_many", "experts_gather"):
+        def note(*args, _run=getattr(K, name), _name=name, **more):
+            called.append(_name)
+            return _run(*args, **more)
+        monkeypatch.setattr(K, name, note)
+    many, grouped = rows * top >= part.PRODUCT_PAIRS * experts, K.experts_rows_take(width) and K.experts_rows_take(ff)
     for is_decode, one_launch in ((True, None), (False, True), (False, False)):
         if one_launch is False:
             part.in_one_launch = False
@@ -334,7 +341,12 @@ def test_experts_some_of_which_hand_their_input_through(K, dtype, rows, width, e
         del poison                                       # the allocator hands this memory out again
         for fresh in (True, False):
             hidden = torch.full((rows, width), 5.0, device="cuda:0")
+            called.clear()
             part.forward(ctx, dev(h_t), hidden, fresh=fresh)
+            if many and grouped and part.packed is not None:
+                assert called == (["experts_gather"] if one_launch is False else ["experts_many"] * 2), (is_decode, one_launch)
+            elif many and grouped and not is_decode:
+                assert called == ["experts_gather"]
             assert rel(hidden[sure], (want + (0.0 if fresh else 5.0))[sure.numpy()]) < tol(dtype, f32=5e-5, bf16=2e-2), (is_decode, one_launch, fresh)
         got_chosen, got_shares = ctx.extras["routing"]
         assert rel(got_shares.sort(dim=-1).values[sure], np.sort(shares[sure.numpy()], axis=-1)) < 1e-5
