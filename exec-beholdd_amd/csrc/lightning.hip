@@ -459,8 +459,24 @@ struct LightningRows {
 extern "C" long bh_lightning_products_scratch(int n_seqs, int n_rows, int max_rows, int H, int dim, int vdim, int row_stride, int q_off,
                                               int k_off, int v_off) {
   if (n_seqs < 1 || n_rows < n_seqs || H < 1 || dim < 1 || vdim < 1 || (row_stride | q_off | k_off | v_off) % 4) return 0;
+  if (n_rows == n_seqs) return 0;      // a row each: the step kernel's
   // The walk costs a row's latency (0.45 us) and three launches less: one sequence of 96 rows 38 us against 46, of 128 60 against 46.
   if (max_rows < 128) return 0;
+  // A place's latency grows with its state (20 us and 1.6 ns an element for one round of places), the walk's only with the keys' size
+  // as long as its workgroups of 16 columns find room beside one another (one a compute unit, two with few keys): one sequence, 4
+  // heads of 256 x 256 walk 256 rows in 97 us against 125, 320 rows in 140 against 126; 8 heads of 64 x 256 47 against 52 and 65
+  // against 53.
+  int rows = 0;
+  const long chunks = (long)n_seqs * bh_lightning_chunks(n_seqs, n_rows, max_rows, H, vdim, &rows), most = n_rows / rows + n_seqs;
+  const long walkers = (chunks < most ? chunks : most) * H * ((vdim + 15) / 16);
+  if (walkers <= (dim <= 64 ? 2L : 1L) * bh_compute_units() && (long)dim * (vdim - 156) > 6250) return 0;
+  // Many sequences of a row beside a few long ones: each takes a place of 64 rows and has its state written twice and read twice more
+  // than by the walk, whose time is the longest sequence's rows.  One sequence of max_rows among n of a row, walk / products us: 32
+  // heads of 128 x 128 with 128 rows n 192 1,212 / 1,069, 256 1,414 / 1,415, 401 1,345 / 2,152; 64 heads with 300 rows n 256
+  // 4,437 / 3,137, 512 6,042 / 7,162; 128 heads of 64 x 16 with 128 rows n 96 426 / 387, 192 636 / 787.  With keys of 192 and more the walk is
+  // the slower one at every count measured.
+  const int lasting = vdim <= 32 ? 9 : (long)H * ((vdim + 63) / 64) >= 64 ? 17 : 22;      // tenths of a row of the longest sequence
+  if (dim <= 128 && (long)n_seqs * H >= 1024 && 10L * n_seqs > (long)lasting * max_rows) return 0;
   return ds_scratch_floats(n_seqs, n_rows, H, dim, vdim);
 }
 // The most that it can be for a step of up to so many sequences and rows (more of either never takes less), whichever form is faster.
