@@ -395,6 +395,11 @@ extern "C" long bh_ssm_products_scratch(int n_seqs, int n_rows, int max_rows, in
   // The walk takes the longest sequence's rows at 1.27 us each, or, where sequences and heads fill the chip, about as long as the
   // products: 1.67 ns a row of a chunk and head, and their launches.  8 sequences of 64 rows: 32 heads 83 us against 51, 128 heads
   // 128 against 152; 8 of 1,024: 64 heads 1,231 against 763, 128 heads 1,706 against 1,757.
+  // The figures are those of states of 128 x 64; up to 256 x 128 and down to 64 x 64 the line lies in the same place (walk / products
+  // us, 64 rows: 8 sequences of 64 heads of 64 x 64 68 / 63, of 128 x 64 95 / 91), below that a row of the walk is quicker: 8
+  // sequences of 64 heads of 64 x 32 45 / 51, of 64 x 16 39 / 43.
+  if (n_rows == n_seqs) return 0;      // a row each
+  if (max_rows == DS_ROWS && N * vdim <= 64 * 32 && (long)n_rows * H >= 512L * DS_ROWS) return 0;
   const long whole = (long)n_seqs * ((max_rows + DS_ROWS - 1) / DS_ROWS), places = ds_places(n_seqs, n_rows);
   if (max_rows < DS_ROWS || 760L * max_rows <= (long)DS_ROWS * H * (whole < places ? whole : places) + 10000) return 0;
   return ds_scratch_floats(n_seqs, n_rows, H, N, vdim);

@@ -21,3 +21,10 @@ def lib():
 def test_lightning(lib, seqs, rows, longest, heads, dim, vdim, products):
     stride = 2 * heads * (dim + vdim)
     assert (lib.bh_lightning_products_scratch(seqs, rows, longest, heads, dim, vdim, stride, 0, heads * dim, 2 * heads * dim) > 0) == products
+
+
+@pytest.mark.parametrize("seqs,rows,longest,heads,vdim,n_state,products", [
+    (1, 63, 63, 32, 64, 128, False), (1, 64, 64, 32, 64, 128, True), (100, 100, 100, 8, 64, 128, False), (8, 512, 64, 64, 64, 64, True),
+    (8, 512, 64, 64, 32, 64, False), (7, 448, 64, 64, 32, 64, True), (8, 520, 65, 8, 32, 64, True), (8, 512, 64, 128, 64, 128, False)])
+def test_state_space(lib, seqs, rows, longest, heads, vdim, n_state, products):
+    assert (lib.bh_ssm_products_scratch(seqs, rows, longest, heads, vdim, n_state, 1, heads * vdim + 2 * n_state) > 0) == products
