@@ -241,12 +241,23 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(F32Attention 
 }
 
 template <int P>
-void launch(const F32Attention& t, int n_rows, int n_seqs, hipStream_t stream) {
+void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, hipStream_t stream) {
   constexpr int NR = P <= 4 ? 4 : P <= 7 ? 2 : 1;      // what the registers hold without spilling
+  const bool prompts = n_rows >= 8 * n_seqs;
+  // Rows that see one page have work for one wave a row and head, and rows that see a few have it where they and the heads fill the
+  // chip: waves of their own leave no wave without a page.  Four waves on four rows / a wave a row, us, 16 heads of 128 on 8: one
+  // prompt of 33 rows 15.9 / 6.8, 16 of 40 172 / 52, one of 256 61 / 40; 8 heads of 256 on 2: 4 prompts of 64 47 / 17, but 30 rows
+  // behind 100 cached keys (240 workgroups) 8.5 / 12.3.
+  if (most_pages <= 1 || (most_pages <= 4 && (long)n_rows * t.H >= (prompts ? 2L : 4L) * bh_compute_units())) {
+    constexpr int FEW = P <= 4 ? 1 : NR;
+    if (prompts) attention_f32_kernel<P, FEW, 1><<<dim3((n_rows + FEW - 1) / FEW, t.H), 64, 0, stream>>>(t, n_rows);
+    else attention_f32_kernel<P, 1, 1><<<dim3(n_rows, t.H), 64, 0, stream>>>(t, n_rows);
+    return;
+  }
   // Prompts: rows of one sequence share the pages' reads.  Else a row a workgroup, of eight waves where the rows and heads alone
   // leave compute units idle and the registers allow it: as many pages are then on their way together.
   constexpr int MANY = P <= 3 ? 8 : 4;
-  if (n_rows >= 8 * n_seqs) attention_f32_kernel<P, NR, 4><<<dim3((n_rows + NR - 1) / NR, t.H), 256, 0, stream>>>(t, n_rows);
+  if (prompts) attention_f32_kernel<P, NR, 4><<<dim3((n_rows + NR - 1) / NR, t.H), 256, 0, stream>>>(t, n_rows);
   else if ((long)n_rows * t.H < 2 * bh_compute_units())
     attention_f32_kernel<P, 1, MANY><<<dim3(n_rows, t.H), 64 * MANY, 0, stream>>>(t, n_rows);
   else attention_f32_kernel<P, 1, 4><<<dim3(n_rows, t.H), 256, 0, stream>>>(t, n_rows);
@@ -258,10 +269,10 @@ void launch(const F32Attention& t, int n_rows, int n_seqs, hipStream_t stream) {
 extern "C" int bh_attention_f32_takes(int H, int KVH, int hd, int kv_order) {
   return hd % 32 == 0 && hd >= 32 && hd <= 256 && KVH > 0 && H % KVH == 0 && H <= 65535 && kv_order == BH_KV_ROWS ? 1 : 0;
 }
-// `n_seqs`: the rows of the page table.
+// `n_seqs`: the rows of the page table.  `most_pages`: how many pages a row sees at most, as far as the caller knows.
 extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages, const float* v_pages, const int32_t* page_table,
-                                int table_stride, int n_seqs, const int32_t* row_seq, const int32_t* positions, int n_rows, int H,
-                                int KVH, int hd, float scale, int window, int kv_order, const float* sinks, const void* gates,
+                                int table_stride, int n_seqs, int most_pages, const int32_t* row_seq, const int32_t* positions,
+                                int n_rows, int H, int KVH, int hd, float scale, int window, int kv_order, const float* sinks, const void* gates,
                                 int gate_stride, float cap, const float* slopes, float temp_coef, int temp_every, float out_scale,
                                 hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && H > 0 && KVH > 0 && hd > 0 && n_seqs > 0, "attention: sizes must be positive");
@@ -273,14 +284,14 @@ extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages
   const F32Attention t = {q, out, k_pages, v_pages, page_table, table_stride, row_seq, positions, H, KVH, form, window,
                           {sinks, gates, gate_stride, out_scale}};
   switch (hd / 32) {
-    case 1: launch<1>(t, n_rows, n_seqs, stream); break;
-    case 2: launch<2>(t, n_rows, n_seqs, stream); break;
-    case 3: launch<3>(t, n_rows, n_seqs, stream); break;
-    case 4: launch<4>(t, n_rows, n_seqs, stream); break;
-    case 5: launch<5>(t, n_rows, n_seqs, stream); break;
-    case 6: launch<6>(t, n_rows, n_seqs, stream); break;
-    case 7: launch<7>(t, n_rows, n_seqs, stream); break;
-    default: launch<8>(t, n_rows, n_seqs, stream); break;
+    case 1: launch<1>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 2: launch<2>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 3: launch<3>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 4: launch<4>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 5: launch<5>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 6: launch<6>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 7: launch<7>(t, n_rows, n_seqs, most_pages, stream); break;
+    default: launch<8>(t, n_rows, n_seqs, most_pages, stream); break;
   }
   return bh_check_launch("attention_f32");
 }

@@ -144,7 +144,7 @@ class KernelSizes:
             "bh_gemm_bf16_bare_parts": [i, i, i, i],
             "bh_gemm_bf16_bare": [p, p, p, i, i, i, i, i, p],
             "bh_attention_generic": [p, p, i, p, p, p, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
-            "bh_attention_f32": [p, p, p, p, p, i, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
+            "bh_attention_f32": [p, p, p, p, p, i, i, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32_takes": [i, i, i, i],
             "bh_gemm_f32_takes_gated": [i, i, i],
             "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
@@ -828,6 +828,7 @@ class HipKernels(KernelSizes):
             self._check(self.lib.bh_attention_f32(
                 *common, self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
                 self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1], page_table.shape[0],
+                furthest // self.page_size + 1 if layout is not None else page_table.shape[1],
                 self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(positions, "positions", (torch.int32,)),
                 n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), kv_order,
                 self._ptr(sinks, "sinks", (torch.float32,), True), *gating, *form, float(out_scale), self._stream()))

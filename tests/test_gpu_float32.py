@@ -130,3 +130,28 @@ def test_float32_attention_pages_of_keys_that_are_infinitely_far(K, rows, blind)
                 head_dim ** -0.5, layout=layout)
     want = attention_reference_rows(q, keys[0], values[0], positions.long(), n_heads, kv_heads, head_dim, head_dim ** -0.5, 0)
     assert float((out.cpu().double() - want).abs().max() / want.abs().max()) < 1e-5
+
+
+# a page at most (prompts, a row a sequence, both ends of a page), four pages in enough rows and heads for a wave a row, and five
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim", [(4, 2, 32), (8, 4, 128), (6, 3, 160), (8, 2, 256)])
+@pytest.mark.parametrize("pasts,news", [([0, 5, 63], [1, 1, 1]), ([0, 10], [64, 33]), ([0], [3]), ([0, 200, 100], [190, 56, 30]), ([0, 200], [190, 57]),
+                                        ([50] * 150 + [255] * 20, [1] * 170)])
+def test_float32_attention_of_few_pages(K, n_heads, kv_heads, head_dim, pasts, news):
+    lengths = [p + n for p, n in zip(pasts, news)]
+    kp, vp, table, keys, values = make_cache(len(lengths), lengths, kv_heads, head_dim, torch.float32, seed=head_dim)
+    for s, n in enumerate(lengths):
+        if n % 64:
+            kp[int(table[s, (n - 1) // 64]), :, n % 64:, :] = float("nan")
+            vp[int(table[s, (n - 1) // 64]), :, :, n % 64:] = float("nan")
+    positions = torch.tensor([p + t for p, n in zip(pasts, news) for t in range(n)], dtype=torch.int32)
+    row_seq = torch.tensor([s for s, n in enumerate(news) for _ in range(n)], dtype=torch.int32)
+    q = torch.randn(len(positions), n_heads * head_dim, generator=torch.Generator().manual_seed(1))
+    out = torch.full(q.shape, float("nan"), device="cuda:0")
+    starts = torch.tensor([0] + [sum(news[:i + 1]) for i in range(len(news))], dtype=torch.int32)
+    layout = Layout(max(news) == 1, dev(starts), len(news), max(news), max(lengths) - 1)
+    K.attention(dev(q), out, dev(kp), dev(vp), dev(table), dev(row_seq), dev(positions), n_heads, kv_heads, head_dim, head_dim ** -0.5, layout=layout)
+    got = out.cpu().double()
+    for s in range(len(news)):
+        rows = row_seq == s
+        want = attention_reference_rows(q[rows], keys[s], values[s], positions[rows].long(), n_heads, kv_heads, head_dim, head_dim ** -0.5, 0)
+        assert float((got[rows] - want).abs().max() / want.abs().max()) < 1e-5, s      # as in test_float32_attention_rows_of_a_step
