@@ -40,6 +40,16 @@ __device__ inline int bh_row_of_block(int block_rows) {
   return (place / 16 * 8 + blockIdx.x % 8) * 16 + place % 16;
 }
 
+// ---- element-wise kernels in pieces of 16 bytes --------------------------------------------------------------
+// A thread's 8 elements of bfloat16 are a chain of as many exponentials or stores: worth it from the size on at which an element a
+// thread would keep the chip busy (1,536 threads a compute unit), not below it, where the chain is the time.  An element / a piece a
+// thread, us: gated heads of 65 x 2,048 2.9 / 3.5, of 2,000 x 256 4.8 / 3.8 into blocks, clamped gate of 300 x 1,000 2.8 / 3.2, of
+// 300 x 2,048 3.6 / 3.3, squared ReLU of 65 x 5,120 2.8 / 3.0, of 2,000 x 256 3.6 / 2.9 into blocks.  Four of float32 cost nothing.
+int bh_compute_units();
+inline bool bh_pieces_pay(long elements) { return elements >= 1536L * bh_compute_units(); }
+// A row's pieces go to workgroups of up to four waves, of fewer where the row has no more (8,160 rows of 256, gelu 7.0 us with four).
+inline unsigned bh_piece_threads(int pieces) { return pieces >= 256 ? 256u : ((unsigned)pieces + 63) / 64 * 64; }
+
 // Four neighbouring elements in one store; `to` lies on the bytes of four of them.
 __device__ inline void store_four(float* to, float a, float b, float c, float d) { *reinterpret_cast<float4*>(to) = make_float4(a, b, c, d); }
 __device__ inline void store_four(bf16_t* to, float a, float b, float c, float d) {

@@ -241,7 +241,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void clamped_glu_pieces_kernel(const T* __restrict__ gu, T* __restrict__ out, int n_rows, int ff, float limit,
                                                                  float alpha, int out_block_rows, float shift) {
   constexpr int N = 16 / sizeof(T);
-  const int row = bh_row_of_block(out_block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  const int row = bh_row_of_block(out_block_rows), i = N * (blockIdx.y * blockDim.x + threadIdx.x);
   if (row >= n_rows || i >= ff) return;
   union Piece {
     uint4 raw;
@@ -259,10 +259,11 @@ extern "C" int bh_clamped_glu(const void* gu, int dtype, void* out, int n_rows, 
   BH_REQUIRE(n_rows > 0 && ff > 0, "clamped_glu: sizes must be positive");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && ff % 32 == 0 && dtype == BH_BF16),
              "clamped_glu: rows in blocks of %d of width %d are not written", out_block_rows, ff);
-  if (ff <= 4 * 256 * 65535 && (((uintptr_t)gu | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && ff % 4 == 0) || (dtype == BH_BF16 && ff % 8 == 0))) {
-    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (ff / (dtype == BH_F32 ? 4 : 8) + 255) / 256);
-    if (dtype == BH_F32) clamped_glu_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)gu, (float*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
-    else clamped_glu_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)gu, (bf16_t*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
+  if ((dtype == BH_F32 || bh_pieces_pay((long)n_rows * ff)) && ff <= 4 * 256 * 65535 && (((uintptr_t)gu | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && ff % 4 == 0) || (dtype == BH_BF16 && ff % 8 == 0))) {
+    const int pieces = ff / (dtype == BH_F32 ? 4 : 8);
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (pieces + 255) / 256), block(bh_piece_threads(pieces));
+    if (dtype == BH_F32) clamped_glu_pieces_kernel<float><<<grid, block, 0, stream>>>((const float*)gu, (float*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
+    else clamped_glu_pieces_kernel<bf16_t><<<grid, block, 0, stream>>>((const bf16_t*)gu, (bf16_t*)out, n_rows, ff, limit, alpha, out_block_rows, shift);
     return bh_check_launch("clamped_glu");
   }
   const size_t n = (size_t)n_rows * ff;

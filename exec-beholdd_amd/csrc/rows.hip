@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void cast_concat_kernel(const float* __restric
 template <typename TO>
 __global__ __launch_bounds__(256) void cast_concat_wide_kernel(const float* __restrict__ a, const float* __restrict__ b, TO* __restrict__ out,
                                                                int n_rows, int width, int out_block_rows) {
-  const int total = b ? 2 * width : width, r = bh_row_of_block(out_block_rows), i = 8 * (blockIdx.y * 256 + threadIdx.x);
+  const int total = b ? 2 * width : width, r = bh_row_of_block(out_block_rows), i = 8 * (blockIdx.y * blockDim.x + threadIdx.x);
   if (r >= n_rows || i >= total) return;
   const float4* from = reinterpret_cast<const float4*>(i < width ? a + (size_t)r * width + i : b + (size_t)r * width + i - width);
   const float4 low = from[0], high = from[1];
@@ -317,10 +317,11 @@ extern "C" int bh_cast_concat(const float* a, const float* b, void* out, int out
   const int total = b ? 2 * width : width;
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && total % 32 == 0 && out_dtype == BH_BF16),
              "cast_concat: rows in blocks of %d of width %d are not written", out_block_rows, total);
-  if (width % 8 == 0 && total <= 8 * 256 * 65535 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16) == 0 && (out_dtype == BH_F32 || out_dtype == BH_BF16)) {
-    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (total / 8 + 255) / 256);
-    if (out_dtype == BH_F32) cast_concat_wide_kernel<float><<<grid, 256, 0, stream>>>(a, b, (float*)out, n_rows, width, out_block_rows);
-    else cast_concat_wide_kernel<bf16_t><<<grid, 256, 0, stream>>>(a, b, (bf16_t*)out, n_rows, width, out_block_rows);
+  // (nothing to compute: two thirds of that size are enough, 65 x 5,120 3.2 us an element a thread and 3.0 in pieces)
+  if ((out_dtype == BH_F32 || bh_pieces_pay((long)n_rows * total * 3 / 2)) && width % 8 == 0 && total <= 8 * 256 * 65535 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16) == 0 && (out_dtype == BH_F32 || out_dtype == BH_BF16)) {
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (total / 8 + 255) / 256), block(bh_piece_threads(total / 8));
+    if (out_dtype == BH_F32) cast_concat_wide_kernel<float><<<grid, block, 0, stream>>>(a, b, (float*)out, n_rows, width, out_block_rows);
+    else cast_concat_wide_kernel<bf16_t><<<grid, block, 0, stream>>>(a, b, (bf16_t*)out, n_rows, width, out_block_rows);
     return bh_check_launch("cast_concat");
   }
   const size_t n = (size_t)n_rows * total;
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_kernel(const T* __restrict__ x,
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_tanh_pieces_kernel(const T* __restrict__ x, T* __restrict__ out, int n_rows, int width, int block_rows) {
   constexpr int N = 16 / sizeof(T);
-  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * blockDim.x + threadIdx.x);
   if (row >= n_rows || i >= width) return;
   union {
     uint4 raw;
@@ -434,10 +435,14 @@ extern "C" int bh_gelu_tanh(const void* x, void* out, int dtype, int n_rows, int
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && dtype == BH_BF16 && width % 32 == 0 && x != out),
              "gelu_tanh: rows in blocks of %d need bfloat16, a width that is a multiple of 32 (got %d) and an output of their own",
              out_block_rows, width);
-  if (width <= 4 * 256 * 65535 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
-    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (width / (dtype == BH_F32 ? 4 : 8) + 255) / 256);
-    if (dtype == BH_F32) gelu_tanh_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
-    else gelu_tanh_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
+  // (its chain is the longest, and into rows an element a thread writes whole lines too: 2,000 x 1,000 4.4 us, 4.5 in pieces, 8,160 x
+  // 256, where a row's pieces are half a wave, 4.4 and 6.2)
+  const long elements = (long)n_rows * width / (out_block_rows ? 1 : dtype == BH_F32 ? 2 : 4);
+  if (bh_pieces_pay(elements) && (out_block_rows || width >= 8 * BH_WAVE) && width <= 4 * 256 * 65535 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
+    const int pieces = width / (dtype == BH_F32 ? 4 : 8);
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (pieces + 255) / 256), block(bh_piece_threads(pieces));
+    if (dtype == BH_F32) gelu_tanh_pieces_kernel<float><<<grid, block, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
+    else gelu_tanh_pieces_kernel<bf16_t><<<grid, block, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
     return bh_check_launch("gelu_tanh");
   }
   const size_t total = (size_t)n_rows * width;

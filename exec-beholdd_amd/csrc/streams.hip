@@ -397,7 +397,7 @@ __global__ void relu_squared_kernel(const T* __restrict__ x, T* __restrict__ out
 template <typename T>
 __global__ __launch_bounds__(256) void relu_squared_pieces_kernel(const T* __restrict__ x, T* __restrict__ out, int n_rows, int width, int block_rows) {
   constexpr int N = 16 / sizeof(T);
-  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * 256 + threadIdx.x);
+  const int row = bh_row_of_block(block_rows), i = N * (blockIdx.y * blockDim.x + threadIdx.x);
   if (row >= n_rows || i >= width) return;
   union {
     uint4 raw;
@@ -417,11 +417,12 @@ extern "C" int bh_relu_squared(const void* x, void* out, int dtype, int n_rows, 
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && dtype == BH_BF16 && width % 32 == 0 && x != out),
              "relu_squared: rows in blocks of %d need bfloat16, a width that is a multiple of 32 (got %d) and an output of their own",
              out_block_rows, width);
-  if (width <= 8 * 256 * 65535 / 2 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
-    const int n = dtype == BH_F32 ? 4 : 8;
-    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (width / n + 255) / 256);
-    if (dtype == BH_F32) relu_squared_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
-    else relu_squared_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
+  // (rows of bfloat16 that are less than a wave's pieces: 8,160 x 256 4.0 us an element a thread, 4.3 in pieces)
+  if ((dtype == BH_F32 || (bh_pieces_pay((long)n_rows * width) && (out_block_rows || width >= 8 * BH_WAVE))) && width <= 8 * 256 * 65535 / 2 && (((uintptr_t)x | (uintptr_t)out) % 16) == 0 && ((dtype == BH_F32 && width % 4 == 0) || (dtype == BH_BF16 && width % 8 == 0))) {
+    const int pieces = width / (dtype == BH_F32 ? 4 : 8);
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (pieces + 255) / 256), block(bh_piece_threads(pieces));
+    if (dtype == BH_F32) relu_squared_pieces_kernel<float><<<grid, block, 0, stream>>>((const float*)x, (float*)out, n_rows, width, out_block_rows);
+    else relu_squared_pieces_kernel<bf16_t><<<grid, block, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, n_rows, width, out_block_rows);
     return bh_check_launch("relu_squared");
   }
   const size_t total = (size_t)n_rows * width;

@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void gate_heads_pieces_kernel(const T* __restr
                                                                 int gate_stride, int gate_first, T* __restrict__ out, int n_rows, int H,
                                                                 int vdim, int out_block_rows, int gate_per_head) {
   constexpr int N = 16 / sizeof(T);
-  const int width = H * vdim, row = bh_row_of_block(out_block_rows), c = N * (blockIdx.y * 256 + threadIdx.x);
+  const int width = H * vdim, row = bh_row_of_block(out_block_rows), c = N * (blockIdx.y * blockDim.x + threadIdx.x);
   if (row >= n_rows || c >= width) return;
   const int head = c / vdim, i = c % vdim;
   union Piece {
@@ -283,14 +283,14 @@ extern "C" int bh_gate_heads(const void* attended, int dtype, int pad, const voi
              "gate_heads: rows in blocks of %d of width %d are not written", out_block_rows, H * vdim);
   const int piece = dtype == BH_F32 ? 4 : 8;
   const bool gates_on16 = gate == nullptr || gate_per_head || ((uintptr_t)gate % 16 == 0 && gate_stride % piece == 0 && gate_first % piece == 0);
-  if (vdim % piece == 0 && pad % piece == 0 && gates_on16 && (((uintptr_t)attended | (uintptr_t)out) % 16) == 0 && (long)H * vdim <= 4L * 256 * 65535 &&
+  if ((dtype == BH_F32 || bh_pieces_pay((long)n_rows * H * vdim)) && vdim % piece == 0 && pad % piece == 0 && gates_on16 && (((uintptr_t)attended | (uintptr_t)out) % 16) == 0 && (long)H * vdim <= 4L * 256 * 65535 &&
       (dtype == BH_F32 || dtype == BH_BF16)) {
-    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (H * vdim / piece + 255) / 256);
+    const dim3 grid(bh_rows_grid(n_rows, out_block_rows), (H * vdim / piece + 255) / 256), block(bh_piece_threads(H * vdim / piece));
     if (dtype == BH_F32)
-      gate_heads_pieces_kernel<float><<<grid, 256, 0, stream>>>((const float*)attended, pad, (const float*)gate, gate_stride, gate_first, (float*)out,
+      gate_heads_pieces_kernel<float><<<grid, block, 0, stream>>>((const float*)attended, pad, (const float*)gate, gate_stride, gate_first, (float*)out,
                                                                n_rows, H, vdim, out_block_rows, gate_per_head);
     else
-      gate_heads_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)attended, pad, (const bf16_t*)gate, gate_stride, gate_first,
+      gate_heads_pieces_kernel<bf16_t><<<grid, block, 0, stream>>>((const bf16_t*)attended, pad, (const bf16_t*)gate, gate_stride, gate_first,
                                                                 (bf16_t*)out, n_rows, H, vdim, out_block_rows, gate_per_head);
     return bh_check_launch("gate_heads");
   }

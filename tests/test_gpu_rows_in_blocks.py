@@ -43,3 +43,31 @@ def test_rows_and_blocks_agree(K, rows, width):
         call(in_blocks)
         got = K.from_blocked(in_blocks)
         assert bool(torch.isfinite(in_rows.float()).all()) and torch.equal(got, in_rows), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width", [(128, 4096), (129, 4128), (2049, 256), (2100, 264), (530, 1000), (530, 4096), (40, 16640), (16, 33280)])
+def test_pieces_and_elements_agree(K, dtype, rows, width):
+    """Element-wise kernels take a thread a piece of 16 bytes from a size on and a thread an element below it: the step's first rows
+    alone are below it, so that both run the same rows; widths of fewer pieces than a workgroup's threads and of more, a last piece in
+    the middle of one.  Bit for bit."""
+    g = torch.Generator().manual_seed(rows + width)
+    few = max(1, 400_000 // (8 * width))
+    x, both = (torch.randn(rows, n, generator=g).to(dtype).cuda() for n in (width, 2 * width))
+    f32 = torch.randn(rows, width, generator=g).cuda()
+    calls = {
+        "relu_squared": lambda n, out: K.relu_squared(x[:n], out),
+        "gelu_tanh": lambda n, out: K.gelu_tanh(x[:n], out),
+        "clamped_glu": lambda n, out: K.clamped_glu(both[:n], out, 1.5, 1.702),
+        "cast_concat": lambda n, out: K.cast_concat(f32[:n], None, out),
+        "gate_heads": lambda n, out: K.gate_heads(x[:n], width // 8, both[:n], width, out, 8, width // 8),
+    }
+    for name, call in calls.items():
+        whole, part = (torch.full((n, width), float("nan"), dtype=dtype, device="cuda:0") for n in (rows, few))
+        call(rows, whole)
+        call(few, part)
+        assert bool(torch.isfinite(whole.float()).all()) and torch.equal(whole[:few], part), name
+        if dtype == torch.bfloat16 and width % 32 == 0:
+            out = blocked(K, rows, width)
+            call(rows, out)
+            assert torch.equal(K.from_blocked(out), whole), name
