@@ -135,13 +135,13 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const int32_t* __res
 // (a thread adds its four elements first), like that kernel's differs between widths.
 typedef float norm_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint16_t norm_u16x4_t __attribute__((ext_vector_type(4)));
-template <typename TW, typename TO, int NV>
+template <typename TW, typename TO, int NV, bool SPREAD>
 __global__ void rmsnorm_wide_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows,
                                     const TW* __restrict__ w, TO* __restrict__ out, int n_rows, int width, float eps,
                                     int block_rows) {
   __shared__ float scratch[16];
-  const int r = bh_row_of_block(block_rows);
-  if (r >= n_rows) return;
+  const int r = bh_row_of_block<SPREAD>();
+  if (SPREAD && r >= n_rows) return;
   const int src = rows ? rows[r] : r;
   const norm_f32x4_t* xr = reinterpret_cast<const norm_f32x4_t*>(x + (size_t)src * width);
   const int fours = width / 4;
@@ -191,9 +191,9 @@ static void launch_rmsnorm(const float* x, const int32_t* rows, const void* w, v
     const int fours = width / 4;
     const int wide_threads = std::min(1024, ((fours + 3) / 4 + 63) / 64 * 64);   // four groups per thread where that fits
     const int each = (fours + wide_threads - 1) / wide_threads;
-    dim3 grid(bh_rows_grid(n_rows, block_rows)), block(wide_threads);
-#define BH_NORM_WIDE(NV) \
-  rmsnorm_wide_kernel<TW, TO, NV><<<grid, block, 0, stream>>>(x, rows, (const TW*)w, (TO*)out, n_rows, width, eps, block_rows)
+#define BH_NORM_WIDE(NV)                                                                                                            \
+  BH_BY_ROWS(TO, n_rows, block_rows, wide_threads, stream, (x, rows, (const TW*)w, (TO*)out, n_rows, width, eps, block_rows),       \
+             rmsnorm_wide_kernel, TW, TO, NV)
     if (each == 1) BH_NORM_WIDE(1);
     else if (each == 2) BH_NORM_WIDE(2);
     else BH_NORM_WIDE(4);

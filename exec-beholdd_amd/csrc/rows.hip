@@ -135,13 +135,13 @@ __global__ __launch_bounds__(256) void sum_layernorm_kernel(float* __restrict__ 
 
 // The same for rows of up to THREADS * PER elements: a thread keeps its PER elements of the sum in registers, so the row is read
 // once and written once and nothing waits for its own stores (a step of few rows is three trips to memory shorter).
-template <typename TO, int PER, int THREADS>
+template <typename TO, int PER, int THREADS, bool SPREAD>
 __global__ __launch_bounds__(THREADS) void sum_layernorm_held_kernel(float* __restrict__ h, const float* __restrict__ y, float alpha,
                                                                  const float* __restrict__ w, const float* __restrict__ b,
                                                                  TO* __restrict__ rounded, int n_rows, int width, float eps, int out_block_rows) {
   __shared__ float scratch[THREADS / BH_WAVE];
-  const int r = bh_row_of_block(out_block_rows);
-  if (r >= n_rows) return;
+  const int r = bh_row_of_block<SPREAD>();
+  if (SPREAD && r >= n_rows) return;
   float* row = h + (size_t)r * width;
   const float* add = y + (size_t)r * width;
   float held[PER];
@@ -174,8 +174,9 @@ __global__ __launch_bounds__(THREADS) void sum_layernorm_held_kernel(float* __re
 template <typename TO>
 static void sum_layernorm_launch(float* h, const float* y, float alpha, const float* w, const float* b, TO* rounded, int n_rows,
                                  int width, float eps, int out_block_rows, hipStream_t stream) {
-#define BH_SL(PER, THREADS) \
-  sum_layernorm_held_kernel<TO, PER, THREADS><<<bh_rows_grid(n_rows, out_block_rows), THREADS, 0, stream>>>(h, y, alpha, w, b, rounded, n_rows, width, eps, out_block_rows)
+#define BH_SL(PER, THREADS)                                                                                                       \
+  BH_BY_ROWS(TO, n_rows, out_block_rows, THREADS, stream, (h, y, alpha, w, b, rounded, n_rows, width, eps, out_block_rows),       \
+             sum_layernorm_held_kernel, TO, PER, THREADS)
   if (n_rows <= 64 && width > 1024 && width <= 1024 * 8) {      // few rows: a row on sixteen waves, a few elements a thread
     if (width <= 1024 * 4) BH_SL(4, 1024);
     else BH_SL(8, 1024);
@@ -208,12 +209,12 @@ extern "C" int bh_sum_layernorm(float* h, const float* y, float alpha, const flo
 
 // h <- h + y / sqrt(mean(y^2) + eps) * w: the norm of what a sublayer gave, added to the residual.  One workgroup a row; a thread
 // keeps its PER elements of y and h in registers (PER 0: rows longer than that are read twice).  w: float32 or bfloat16.
-template <typename TO, typename TW, int PER, int THREADS>
+template <typename TO, typename TW, int PER, int THREADS, bool SPREAD>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ y, const TW* __restrict__ w,
                                                               TO* __restrict__ rounded, int n_rows, int width, float eps, int out_block_rows) {
   __shared__ float scratch[THREADS / BH_WAVE];
-  const int r = bh_row_of_block(out_block_rows);
-  if (r >= n_rows) return;
+  const int r = bh_row_of_block<SPREAD>();
+  if (SPREAD && r >= n_rows) return;
   float* row = h + (size_t)r * width;
   const float* add = y + (size_t)r * width;
   constexpr int HELD = PER ? PER : 1;
@@ -251,7 +252,9 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(float* __restrict_
 template <typename TO, typename TW>
 static void add_rmsnorm_launch(float* h, const float* y, const TW* w, TO* rounded, int n_rows, int width, float eps, int out_block_rows,
                                hipStream_t stream) {
-#define BH_AN(PER, THREADS) add_rmsnorm_kernel<TO, TW, PER, THREADS><<<bh_rows_grid(n_rows, out_block_rows), THREADS, 0, stream>>>(h, y, w, rounded, n_rows, width, eps, out_block_rows)
+#define BH_AN(PER, THREADS)                                                                                              \
+  BH_BY_ROWS(TO, n_rows, out_block_rows, THREADS, stream, (h, y, w, rounded, n_rows, width, eps, out_block_rows), add_rmsnorm_kernel, \
+             TO, TW, PER, THREADS)
   if (n_rows <= 64 && width > 1024 && width <= 1024 * 8) {      // few rows: a row on sixteen waves, a few elements a thread
     if (width <= 1024 * 4) BH_AN(4, 1024);
     else BH_AN(8, 1024);

@@ -454,13 +454,13 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(const float* _
 
 // The same with a wave a group, for groups of up to 512 elements (the heads of a row normed one by one): a workgroup takes a
 // row, its four waves the row's groups in turn, a lane keeps its elements in registers between the statistic and the write.
-template <typename T>
+template <typename T, bool SPREAD>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_waves_kernel(const float* __restrict__ y, const T* __restrict__ z, int z_stride,
                                                                         int z_first, const float* __restrict__ w, float eps,
                                                                         T* __restrict__ out, int n_rows, int width, int groups, int out_block_rows,
                                                                         int gate_after) {
-  const int row = bh_row_of_block(out_block_rows), per = width / groups, lane = threadIdx.x % BH_WAVE;
-  if (row >= n_rows) return;
+  const int row = bh_row_of_block<SPREAD>(), per = width / groups, lane = threadIdx.x % BH_WAVE;
+  if (SPREAD && row >= n_rows) return;
   for (int group = threadIdx.x / BH_WAVE; group < groups; group += 4) {
     const int c0 = group * per;
     const float* src = y + (size_t)row * width + c0;
@@ -498,11 +498,13 @@ extern "C" int bh_gated_group_rmsnorm(const float* y, const void* z, int dtype, 
   dim3 grid(n_rows, groups);
   if (groups > 1 && width / groups <= 8 * BH_WAVE && n_rows >= bh_compute_units() / 2) {      // many rows of small groups: a wave a group
     if (dtype == BH_F32)
-      gated_group_rmsnorm_waves_kernel<float><<<n_rows, 256, 0, stream>>>(y, (const float*)z, z_stride, z_first, w, eps, (float*)out, n_rows, width,
-                                                                          groups, out_block_rows, gate_after);
+      BH_BY_ROWS(float, n_rows, out_block_rows, 256, stream,
+                 (y, (const float*)z, z_stride, z_first, w, eps, (float*)out, n_rows, width, groups, out_block_rows, gate_after),
+                 gated_group_rmsnorm_waves_kernel, float);
     else if (dtype == BH_BF16)
-      gated_group_rmsnorm_waves_kernel<bf16_t><<<bh_rows_grid(n_rows, out_block_rows), 256, 0, stream>>>(
-          y, (const bf16_t*)z, z_stride, z_first, w, eps, (bf16_t*)out, n_rows, width, groups, out_block_rows, gate_after);
+      BH_BY_ROWS(bf16_t, n_rows, out_block_rows, 256, stream,
+                 (y, (const bf16_t*)z, z_stride, z_first, w, eps, (bf16_t*)out, n_rows, width, groups, out_block_rows, gate_after),
+                 gated_group_rmsnorm_waves_kernel, bf16_t);
     else
       return bh_fail("gated_group_rmsnorm: unknown dtype %d", dtype);
     return bh_check_launch("gated_group_rmsnorm");

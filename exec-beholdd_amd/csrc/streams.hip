@@ -243,14 +243,14 @@ __global__ void streams_update_rmsnorm_kernel(float* __restrict__ x, const float
 // and the write, and has all of its loads on their way together.
 // Bound by the streams' way from memory and back.  Measured, two streams, bfloat16 out: 2,048 rows of 2,048 19 us (31 with an element a
 // load and a loop over the streams), 16 rows of 4,096 4.9 us (12.2).
-template <typename TO, int S, int PER>
+template <typename TO, int S, int PER, bool SPREAD>
 __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ mix,
                                                    const float* __restrict__ give, const float* __restrict__ scale,
                                                    const float* __restrict__ take, const float* __restrict__ w, TO* __restrict__ out,
                                                    int n_rows, int width, float eps, int block_rows) {
   __shared__ float scratch[16];
-  const int r = bh_row_of_block(block_rows), pieces = width / 4;
-  if (r >= n_rows) return;
+  const int r = bh_row_of_block<SPREAD>(), pieces = width / 4;
+  if (SPREAD && r >= n_rows) return;
   float4* xr = reinterpret_cast<float4*>(x + (size_t)r * S * width);
   const float4* yr = reinterpret_cast<const float4*>(y + (size_t)r * width);
   const float4* scales = reinterpret_cast<const float4*>(scale);
@@ -324,8 +324,8 @@ extern "C" int bh_streams_update_rmsnorm(float* x, const float* y, const float* 
     const int pieces = width / 4, most = n_rows < bh_compute_units() / 4 ? 1024 : streams > 1 && pieces > 1024 ? 512 : 256;
     const int threads = pieces >= most ? most : (pieces + BH_WAVE - 1) / BH_WAVE * BH_WAVE, per = (pieces + threads - 1) / threads;
 #define BH_WIDE(TO, S, PER)                                                                                                          \
-  streams_update_rmsnorm_wide_kernel<TO, S, PER><<<bh_rows_grid(n_rows, out_block_rows), threads, 0, stream>>>(                        \
-      x, y, mix, give, scale, take, w, (TO*)out, n_rows, width, eps, out_block_rows)
+  BH_BY_ROWS(TO, n_rows, out_block_rows, threads, stream, (x, y, mix, give, scale, take, w, (TO*)out, n_rows, width, eps, out_block_rows), \
+             streams_update_rmsnorm_wide_kernel, TO, S, PER)
 #define BH_WIDE_SIZES(TO, S)            \
   do {                                  \
     if (per == 1) BH_WIDE(TO, S, 1);    \
