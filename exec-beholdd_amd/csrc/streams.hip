@@ -255,7 +255,8 @@ __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const 
   const float4* yr = reinterpret_cast<const float4*>(y + (size_t)r * width);
   const float4* scales = reinterpret_cast<const float4*>(scale);
   const float4* weights = reinterpret_cast<const float4*>(w);
-  float4 old[PER][S], add[PER];
+  constexpr bool SOON = S <= 2;      // whether the registers hold the scales beside the streams
+  float4 old[PER][S], add[PER], by[SOON ? PER : 1];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int i = threadIdx.x + j * blockDim.x;
@@ -263,6 +264,7 @@ __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const 
 #pragma unroll
       for (int s = 0; s < S; ++s) old[j][s] = xr[s * pieces + i];
       add[j] = yr[i];
+      if constexpr (SOON) by[j] = scales ? scales[i] : float4{1.f, 1.f, 1.f, 1.f};
     }
   }
   float m[S][S], g[S], share[S];
@@ -280,7 +282,9 @@ __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const 
     const int i = threadIdx.x + j * blockDim.x;
     kept[j] = float4{0.f, 0.f, 0.f, 0.f};
     if (i < pieces) {
-      const float4 c = scales ? scales[i] : float4{1.f, 1.f, 1.f, 1.f};
+      float4 c;
+      if constexpr (SOON) c = by[j];
+      else c = scales ? scales[i] : float4{1.f, 1.f, 1.f, 1.f};
       const float4 a = {c.x * add[j].x, c.y * add[j].y, c.z * add[j].z, c.w * add[j].w};
 #pragma unroll
       for (int t = 0; t < S; ++t) {
