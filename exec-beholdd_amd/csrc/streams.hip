@@ -297,7 +297,7 @@ __global__ void streams_update_rmsnorm_wide_kernel(float* __restrict__ x, const 
         kept[j] = float4{fmaf(share[t], v.x, kept[j].x), fmaf(share[t], v.y, kept[j].y), fmaf(share[t], v.z, kept[j].z), fmaf(share[t], v.w, kept[j].w)};
       }
     }
-    ss += kept[j].x * kept[j].x + kept[j].y * kept[j].y + kept[j].z * kept[j].z + kept[j].w * kept[j].w;
+    ss += fmaf(kept[j].w, kept[j].w, fmaf(kept[j].z, kept[j].z, fmaf(kept[j].x, kept[j].x, kept[j].y * kept[j].y)));
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.0f / sqrtf(ss / (float)width + eps);
