@@ -2,14 +2,15 @@
 // same scores, masks, sinks and gates as attention_generic (generic.hip), which takes every other size.
 //
 // A workgroup takes one query head of one row, or of NR neighbouring rows where they belong to one sequence (prompts), and its
-// waves take the visible pages in turn.  Keys lie [token][dim]: eight lanes share a key, 16 bytes each, so that a wave's load
+// waves (one, where the pages are few) take the visible pages in turn.  Keys lie [token][dim]: eight lanes share a key, 16 bytes each, so that a wave's load
 // covers eight keys' whole 128-byte lines; their shares are added crosswise, which leaves lane l with the score of one key of the
 // page.  Values lie [dim][token]: 16 lanes share a dimension, so that a load is 1 KB of contiguous memory, and every lane keeps
 // its own sums over its four tokens of each page; they are added over the lanes once, behind the last page.  The waves' softmax
 // sums are merged through LDS.
 // Bound by the pages' way from memory or the L2 (a page of a head of 128 is 64 KB): NR rows share it.
 // Measured (8 heads of 128 on 4): a decode step of 4 rows at 40 to 300 keys 8.2 us, 54 with a thread a key (generic.hip: every
-// lane its own line), 20 before a page's keys and values were asked for together; prompts of 695 rows in all 94 us, 120 there.
+// lane its own line), 20 before a page's keys and values were asked for together; four prompts of 695 rows in all, up to 256 each,
+// 41 us in waves of their own, 94 in workgroups of four waves on four rows, 120 there.
 #include "common.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));

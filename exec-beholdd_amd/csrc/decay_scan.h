@@ -14,9 +14,9 @@
 // A sequence's chunks have places of their own, floor(first row / 64) + sequence onward, which overlap no other sequence's: a step
 // needs rows / 64 + sequences places, and a window of them at a time has memory for its states.
 // Bound by the matrix instructions and the operands' reads from LDS beside them; a state is written once and read twice.
-// Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 83 us in all (26 + 18 +
-// 39), 233 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 165 us, 606.  With the values in LDS beside the
-// keys, one workgroup a compute unit, 102 and 213.
+// Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 88 us in all (26 + 18 +
+// 40 and the gaps between), 240 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 165 us, 610.  With the
+// values in LDS beside the keys, one workgroup a compute unit, about 20 and 50 us more.
 #pragma once
 
 #include "common.h"

@@ -13,7 +13,7 @@
 // in the tiles of experts_mfma.hip from row-major matrices, whose 128 weight rows a slice of k lie 4 KB apart; 16 pairs 45 / 21
 // (201 MB at 4.5 TB/s), 56 / 35 with experts_tiles, which reads the weights once for 16 pairs and is still ahead at 8 (35 / 21
 // against 42 / 21).  Width 4,096, ff 1,536, 256 pairs 379 / 219, where a product an expert of the kernels for one matrix took about
-// 25 us each.
+// 25 us each; those reach twice the rate on large matrices, and the caller takes them there.
 #include "common.h"
 
 typedef __bf16 xm_bf16x8_t __attribute__((ext_vector_type(8)));

@@ -1,5 +1,6 @@
-// The routed experts' products of a prompt on the matrix cores, all experts in one launch, from weights as they lie.  The model's own
-// prompts run experts_many.hip (packed weights, no table from the host), which is faster at every size measured.
+// The routed experts' products of a prompt on the matrix cores, all experts in one launch, from weights as they lie and a table of tiles
+// from the host: an entry point of the library for callers who keep no packed copy of their matrices.  The parts do keep one and run
+// experts_many.hip, or large experts one by one; both were ahead of this at every size they are taken for.
 // The pairs' inputs lie side by side, expert after expert (experts_gather); a table made from the experts' counts names
 // every tile of up to 128 rows: {expert, first row, rows}.  A workgroup of four waves takes one tile of rows and
 // 128 weight rows; a wave owns 32 of the tile's rows against all 128 weight rows (four blocks of v_mfma_f32_32x32x16_bf16).

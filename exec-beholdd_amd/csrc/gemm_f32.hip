@@ -1,9 +1,9 @@
-// Matrix products of float32 operands on the float32 matrix instructions: C[M, N] (+)= A[M, K] W[N, K]^T, and the gated form
-// out[M, F] = act(A W[:F]^T) * (A W[F:]^T).  Every product is a 32-bit fused multiply-add with a 32-bit sum, as in the plain FMA
+// Matrix products of float32 operands on the float32 matrix instructions: C[M, N] (+)= A[M, K] W[N, K]^T, and for few rows the gated
+// form out[M, F] = act(A W[:F]^T) * (A W[F:]^T).  Every product is a 32-bit fused multiply-add with a 32-bit sum, as in the plain FMA
 // kernel (generic.hip); only the order of the sums differs, and it is blocked here as there.
 //
-// Two kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`.  More rows are
-// matrix-core work: `gemm_f32_tiles`.
+// Two kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`, gated or not.  More rows are
+// matrix-core work: `gemm_f32_tiles`, whose gated products are followed by an activation of their own.
 #include "common.h"
 #include "gemm_f32.h"
 

@@ -1,7 +1,8 @@
 // Kernels that take every size and both element types: embedding gather, RMSNorm, a tiled
 // FMA matrix product, per-head q/k norm + rotation + cache write, attention over the paged
-// cache, SwiGLU.  The float32 engine runs on these alone (true 32-bit arithmetic: plain FMA,
-// no matrix-core mode); the bfloat16 engine uses them wherever no faster kernel fits a size.
+// cache, SwiGLU.  The float32 engine runs on these and on the kernels of gemm_f32.hip and
+// attention_f32.hip, which take most of its products and attention (true 32-bit arithmetic in
+// all of them); the bfloat16 engine uses them wherever no faster kernel fits a size.
 // All reductions, norms, softmax and rotation are computed in float32.
 #include "common.h"
 #include "gemm_f32.h"
