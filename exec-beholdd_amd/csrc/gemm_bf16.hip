@@ -31,7 +31,7 @@
 // Which 8 of the k values a lane group multiplies is free as long as both operands agree.
 #include "common.h"
 #include "gemm_bf16_slices.h"
-#include "gemm_bf16_turns.h"
+#include "gemm_bf16_ring.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_span_kernel(const uint
 // 64 * blockIdx.x + 4 col .. + 3 of row 16 * blockIdx.y + r (N is a multiple of 16 here).  All of a thread's
 // loads are asked for before the first is used.  A norm behind gets one partial sum per row and block.
 #define MAX_PARTS 16
-#define MAX_TURNS_PARTS 8   // what gemm_turns_parts cuts K into at most
+#define MAX_RING_PARTS 8    // what gemm_ring_plan cuts K into at most
 #define FINISH_COLUMNS 64
 typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
 // blocks.c: a SwiGLU's bfloat16 output goes out in blocks of that many rows (bh_rows_index; 0: rows); blocks.behind: so do
@@ -616,9 +616,9 @@ __global__ __launch_bounds__(256) void gemm_parts_finish_kernel(const float* __r
 // ---- tiled -----------------------------------------------------------------------------------
 
 // The same for a product that completes the float32 residual right before an RMSNorm reads it, with many rows
-// (the parts come from the kernel whose wave groups take turns): a block owns eight whole rows, so it can finish
+// (the parts come from the kernel for many rows, gemm_bf16_ring.hip): a block owns eight whole rows, so it can finish
 // the norm itself and the norm needs no launch and no second pass over the residual.  Lane l of wave w has row
-// l % 8 of the block's rows and the pieces of eight columns 8 w + l / 8, + 128, ...: a wave reads 256 contiguous
+// l % 8 of the block's rows and the pieces of eight columns 8 w + l / 8, + 128, ... (here of 8 rows and 16 waves): a wave reads 256 contiguous
 // bytes of each of its rows and writes 128 contiguous bytes of the norm's output per row, or, with
 // normed_blocked (the output in blocks of 16 rows x 32 columns, bh_blocked_index, for a product that reads it
 // that way), the 128 bytes that eight rows' pieces of the same columns fill there.  The parts are added in their
@@ -626,23 +626,24 @@ __global__ __launch_bounds__(256) void gemm_parts_finish_kernel(const float* __r
 // order that depends on the width only.
 #define FINISH_NORM_PIECES 8   // pieces of eight columns per thread: rows of up to 8,192
 typedef uint32_t finish_u32x4_t __attribute__((ext_vector_type(4)));
-template <int PARTS, int ROWS>   // PARTS: at least `parts`, what the loop over them is unrolled to; ROWS per block, 128 threads each
-__global__ __launch_bounds__(128 * ROWS) void gemm_parts_finish_norm_kernel(const float* __restrict__ sums, float* __restrict__ c,
+template <int PARTS, int ROWS, int ROW_WAVES>   // PARTS: at least `parts`, what the loop over them is unrolled to; ROWS per block, ROW_WAVES waves each
+__global__ __launch_bounds__(64 * ROW_WAVES * ROWS) void gemm_parts_finish_norm_kernel(const float* __restrict__ sums, float* __restrict__ c,
                                                                       int M, int N, int parts, const void* __restrict__ weight,
                                                                       int weight_f32, float eps, uint16_t* __restrict__ normed,
                                                                       int normed_blocked) {
-  constexpr int WAVES = 2 * ROWS, WAVE_PIECES = 64 / ROWS;   // a step over the row is 128 pieces wide
+  constexpr int WAVES = ROW_WAVES * ROWS, WAVE_PIECES = 64 / ROWS, STEP = WAVES * WAVE_PIECES;   // a step over the row is STEP pieces wide
+  constexpr int STEPS = (FINISH_NORM_PIECES * 128 + STEP - 1) / STEP;
   __shared__ float partial[WAVES][ROWS];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int r = lane % ROWS, row = blockIdx.x * ROWS + r, pieces = N / 8;
   const bool row_there = row < M;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   constexpr bool KEEP = PARTS <= 4;   // with more parts the registers do not hold the new values too: they are read again
-  f32x4_t value[KEEP ? FINISH_NORM_PIECES : 1][2];
+  f32x4_t value[KEEP ? STEPS : 1][2];
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < FINISH_NORM_PIECES; ++j) {
-    const int piece = WAVE_PIECES * wave + lane / ROWS + 128 * j;
+  for (int j = 0; j < STEPS; ++j) {
+    const int piece = WAVE_PIECES * wave + lane / ROWS + STEP * j;
     const bool there = row_there && piece < pieces;
     if (KEEP) value[j][0] = value[j][1] = zero;
     if (!there) continue;
@@ -682,8 +683,8 @@ __global__ __launch_bounds__(128 * ROWS) void gemm_parts_finish_norm_kernel(cons
   for (int w = 0; w < WAVES; ++w) total += partial[w][r];
   const float inv = 1.0f / sqrtf(total / (float)N + eps);
 #pragma unroll
-  for (int j = 0; j < FINISH_NORM_PIECES; ++j) {
-    const int piece = WAVE_PIECES * wave + lane / ROWS + 128 * j;
+  for (int j = 0; j < STEPS; ++j) {
+    const int piece = WAVE_PIECES * wave + lane / ROWS + STEP * j;
     if (!row_there || piece >= pieces) continue;
     f32x4_t g[2];
     if (weight_f32) {
@@ -1295,6 +1296,8 @@ static void launch_tiled(const void* a, const void* w, void* c, int M, int N, in
 #undef BH_TILED
 }
 
+static RingOutput ring_output(int activation, bool f32) { return activation ? RING_GATED : f32 ? RING_F32 : RING_BF16; }
+
 // How many partial sums per row a product of these sizes writes when a norm rides behind it (0: it cannot
 // carry one), and whether it can take prepared norm rows as its activations.
 // Beyond 256 rows a product carries no norm: at the Qwen3-8B shapes, whole model, the prompt of 128 tokens
@@ -1305,6 +1308,7 @@ extern "C" int bh_gemm_bf16_norm_blocks(int M, int N, int K, int layout, int act
   if (activation || M <= 0 || M > NORM_RIDES_UP_TO_ROWS || N <= 0 || K % 8 != 0) return 0;
   int rows, columns, parts, each;
   if (gemm_slices_takes(M, N, K, layout, 0)) return (N + FINISH_COLUMNS - 1) / FINISH_COLUMNS;   // always finished by that kernel
+  if (const RingPlan ring = gemm_ring_plan(M, N, K, layout, RING_F32); ring.tile >= 0) return ring.parts > 1 ? (N + FINISH_COLUMNS - 1) / FINISH_COLUMNS : 0;
   tiled_config(M, N, false, &rows, &columns);
   if (!tiled_whole(M, N, K, layout, rows, columns)) {   // the skinny kernel's blocks, or its workgroups of wider spans
     if (layout == 1 && skinny_first(M, N, K, layout, 0))
@@ -1324,10 +1328,10 @@ extern "C" int bh_gemm_bf16_takes_norm(int M, int N, int K, int layout, int acti
 
 // The rows per block (16 or 8) if a product of these sizes reads its activations faster from blocks of that
 // many rows x 32 columns (bh_rows_index, layout.h) and takes them that way, else 0: the products of the kernel
-// whose wave groups take turns (16), and those of up to 32 rows of the skinny kernel (8 up to 8 rows, else 16).
+// for many rows (16), and those of up to 32 rows of the skinny kernel (8 up to 8 rows, else 16).
 extern "C" int bh_gemm_bf16_reads_blocked(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0) return 0;
-  if (gemm_turns_blocks(M, N, K, layout, activation) || gemm_turns_parts(M, N, K, layout, activation) > 1) return 16;
+  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return 16;
   if (skinny_first(M, N, K, layout, activation)) return M <= 8 ? 8 : 16;
   if (gemm_slices_takes(M, N, K, layout, activation)) return 16;
   return 0;
@@ -1335,10 +1339,10 @@ extern "C" int bh_gemm_bf16_reads_blocked(int M, int N, int K, int layout, int a
 
 // In what form a product of these sizes can write the bfloat16 rows it produces for the next product (a SwiGLU's
 // output, the rows prepared for a norm behind it): 2 = rows or blocks of 8 or 16 rows (the skinny kernel),
-// 1 = rows or, for SwiGLU, blocks of 16 (the kernel whose wave groups take turns), 0 = rows only.
+// 1 = rows or, for SwiGLU, blocks of 16 (the kernel for many rows), 0 = rows only.
 extern "C" int bh_gemm_bf16_writes_blocked(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 32 != 0) return 0;
-  if (gemm_turns_blocks(M, N, K, layout, activation)) return activation ? 1 : 0;
+  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return activation ? 1 : 0;
   if (gemm_slices_takes(M, N, K, layout, activation)) return 2;    // the finishing kernel writes any blocks
   int rows, columns;
   tiled_config(M, N, activation != 0, &rows, &columns);
@@ -1348,18 +1352,16 @@ extern "C" int bh_gemm_bf16_writes_blocked(int M, int N, int K, int layout, int 
 // layout: 0 = rows, 1 = tiles.  activation: 0 = none; 1 = SwiGLU (W has 2 * N rows: gate rows then up rows); to bh_gemm_bf16
 // itself also 2: the same with GELU's tanh form on the gate (BhGate; what the queries say of SwiGLU goes for it too).
 // Bytes of scratch memory that bh_gemm_bf16 wants for this product (0: none).
-// In how many parts of K the tiled kernels (whole tiles, or the kernel whose wave groups take turns) multiply a
-// product when they are given scratch memory (1: in one go).
-static int tiled_or_turns_parts(int M, int N, int K, int layout, int activation) {
-  if (gemm_turns_blocks(M, N, K, layout, activation)) return 1;
-  if (const int turns_parts = gemm_turns_parts(M, N, K, layout, activation); turns_parts > 1) return turns_parts;
+// In how many parts of K the kernel for many rows, or whole tiles, multiply a product when they are given scratch memory (1: in one go).
+static int tiled_or_ring_parts(int M, int N, int K, int layout, int activation, bool f32) {
+  if (const RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32)); ring.tile >= 0) return ring.parts;
   int parts, each;
   tiled_parts(M, N, K, layout, activation != 0, &parts, &each);
   return parts;
 }
 extern "C" long bh_gemm_bf16_scratch(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  int parts = tiled_or_turns_parts(M, N, K, layout, activation);
+  int parts = std::max(tiled_or_ring_parts(M, N, K, layout, activation, true), tiled_or_ring_parts(M, N, K, layout, activation, false));
   if (gemm_slices_takes(M, N, K, layout, activation))   // (a caller whose activations lie in rows gets the tiles: room for either)
     parts = std::max(parts, gemm_slices_parts(M, N, K, activation, nullptr));
   else if (parts == 1) return 0;
@@ -1415,7 +1417,7 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
   }();
   // 33 to 128 rows from blocks of 16: the kernel whose waves share the activations through LDS, then the finishing kernel
   const bool slices = scratch != nullptr && a_block_rows == 16 && !skinny && gemm_slices_takes(M, N, K, layout, activation);
-  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || gemm_turns_blocks(M, N, K, layout, activation))),
+  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0)),
              "gemm_bf16: a product of M=%d N=%d K=%d does not write these blocks", M, N, K);
   dim3 finish_grid((N + FINISH_COLUMNS - 1) / FINISH_COLUMNS, (M + 15) / 16);
   const RowBlocks finish_blocks = {0, slices ? c_block_rows : 0, slices ? behind_block_rows : 0};
@@ -1438,27 +1440,30 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
     return bh_check_launch("gemm_parts_finish");
   }
   const int a_blocked = a_block_rows == 16 && !skinny, c_blocked = c_block_rows == 16 && !skinny;
-  if (!ahead_ss && !behind_weight && (f32 || !accumulate)) {   // many rows: the kernel whose wave groups take turns
-    if (const int blocks = gemm_turns_blocks(M, N, K, layout, activation))
-      return gemm_turns_launch(a, w, c, c_dtype, accumulate, M, N, K, activation, blocks, a_blocked, c_blocked, form, stream);
-  }
+  // (what the kernel for many rows does not finish itself, rows of a norm ahead or adding into bfloat16, takes a plan with parts if there is one)
+  RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32));
+  if (ring.parts == 1 && !activation && (ahead_ss || (accumulate && !f32)))
+    if (const RingPlan other = gemm_ring_plan(M, N, K, layout, ring_output(0, !f32)); other.parts > 1) ring = other;
+  if (a_blocked && !behind_weight && ring.tile >= 0 && ring.parts == 1)   // many rows (what cannot run there comes in rows)
+    return gemm_ring_launch(a, w, c, c_dtype, accumulate, M, N, K, activation, ring.tile, c_blocked, form, stream);
 #define BH_PICK(FN, TILES, EXTRA, ...)                                             \
   do {                                                                              \
     if (f32) FN<TILES, EXTRA, float>(__VA_ARGS__);                                  \
     else FN<TILES, EXTRA, bf16_t>(__VA_ARGS__);                                     \
   } while (0)
-  const bool in_parts = scratch != nullptr && tiled_or_turns_parts(M, N, K, layout, activation) > 1;
-  BH_REQUIRE(!a_blocked || (in_parts && gemm_turns_parts(M, N, K, layout, activation) > 1),
+  const bool in_parts = scratch != nullptr && (ring.tile >= 0 ? ring.parts : tiled_or_ring_parts(M, N, K, layout, activation, f32)) > 1;
+  BH_REQUIRE(!a_blocked || (in_parts && ring.tile >= 0 && ring.parts > 1),
              "gemm_bf16: a product of M=%d N=%d K=%d that reads rows in blocks needs its scratch memory", M, N, K);
-  BH_REQUIRE(in_parts || !behind_weight || tiled_or_turns_parts(M, N, K, layout, activation) == 1,
+  BH_REQUIRE(in_parts || !behind_weight || tiled_or_ring_parts(M, N, K, layout, activation, f32) == 1,
              "gemm_bf16: a product of M=%d N=%d K=%d carries a norm through its finishing kernel and needs scratch memory", M, N, K);
   if (in_parts) {   // K in parts, then the finishing kernel
     BH_REQUIRE(((uintptr_t)c | (uintptr_t)scratch | (uintptr_t)behind_rows) % 16 == 0,
                "gemm_bf16: output, scratch memory and norm rows must be 16-byte aligned");
     int parts, each;
-    if (const int turns_parts = gemm_turns_parts(M, N, K, layout, activation); turns_parts > 1) {
-      parts = turns_parts;
-      if (int status = gemm_turns_launch_parts(a, w, (float*)scratch, M, N, K, parts, a_blocked, stream)) return status;
+    if (ring.tile >= 0) {
+      BH_REQUIRE(a_blocked, "gemm_bf16: a product of M=%d N=%d K=%d in parts reads its activations in blocks of 16 rows", M, N, K);
+      parts = ring.parts;
+      if (int status = gemm_ring_launch_parts(a, w, (float*)scratch, M, N, K, ring, stream)) return status;
     } else {
       tiled_parts(M, N, K, layout, activation != 0, &parts, &each);
       const RidingNorm none = {};
@@ -1494,43 +1499,52 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
   return bh_check_launch("gemm_tiled");
 }
 
-// residual[M, N] += A W^T and normed = RMSNorm(residual; weight, eps) as bfloat16, in one go: for the products of
-// many rows whose K the turns kernel multiplies in parts (bh_gemm_bf16_finishes_norm says which), whose finishing
-// kernel streams the residual anyway.  `scratch`: bh_gemm_bf16_scratch() bytes.
+extern "C" int bh_rmsnorm(const float* x, const int32_t* rows, const void* w, int w_dtype, void* out, int out_dtype, int n_rows, int width,
+                          float eps, int out_block_rows, hipStream_t stream);      // generic.hip
+// residual[M, N] += A W^T and normed = RMSNorm(residual; weight, eps) as bfloat16: for the products of the kernel for many rows
+// (bh_gemm_bf16_finishes_norm says which).  Where K goes in parts the finishing kernel streams the residual anyway and finishes the
+// norm; where it does not the norm is a launch of its own.  `scratch`: bh_gemm_bf16_scratch() bytes.
 extern "C" int bh_gemm_bf16_finishes_norm(int M, int N, int K, int layout) {
-  if (M <= 0 || N <= 0 || K <= 0 || N % 8 != 0 || N > 8 * 128 * FINISH_NORM_PIECES) return 0;
-  const int parts = gemm_turns_parts(M, N, K, layout, 0);
-  return parts > 1 && parts <= MAX_TURNS_PARTS ? 1 : 0;
+  if (M <= 0 || N <= 0 || K < 512 || N % 8 != 0 || N > 8 * 128 * FINISH_NORM_PIECES) return 0;
+  return gemm_ring_plan(M, N, K, layout, RING_F32).tile >= 0 ? 1 : 0;
 }
 extern "C" int bh_gemm_bf16_then_norm(const void* a, const void* w, float* residual, int M, int N, int K, int layout,
                                       const void* norm_weight, int norm_weight_dtype, float eps, void* normed,
                                       void* scratch, int a_blocked, int normed_blocked, hipStream_t stream) {
   BH_REQUIRE(bh_gemm_bf16_finishes_norm(M, N, K, layout),
              "gemm_bf16_then_norm: a product of M=%d N=%d K=%d does not finish a norm (bh_gemm_bf16_finishes_norm)", M, N, K);
-  BH_REQUIRE(a && w && residual && norm_weight && normed && scratch, "gemm_bf16_then_norm: every operand is needed");
+  const RingPlan ring = gemm_ring_plan(M, N, K, layout, RING_F32);
+  const int parts = ring.parts;
+  BH_REQUIRE(a && w && residual && norm_weight && normed && (scratch || parts == 1), "gemm_bf16_then_norm: every operand is needed");
+  BH_REQUIRE(a_blocked, "gemm_bf16_then_norm: the activations lie in blocks of 16 rows");
   BH_REQUIRE(norm_weight_dtype == BH_F32 || norm_weight_dtype == BH_BF16, "gemm_bf16_then_norm: unknown norm weight dtype %d", norm_weight_dtype);
   BH_REQUIRE(eps >= 0.f, "gemm_bf16_then_norm: eps must not be negative");
   BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)residual | (uintptr_t)normed | (uintptr_t)scratch | (uintptr_t)norm_weight) % 16 == 0,
              "gemm_bf16_then_norm: operands must be 16-byte aligned");
   BH_REQUIRE(!normed_blocked || N % 32 == 0, "gemm_bf16_then_norm: rows in blocks need N=%d to be a multiple of 32", N);
-  const int parts = gemm_turns_parts(M, N, K, layout, 0);
-  if (int status = gemm_turns_launch_parts(a, w, (float*)scratch, M, N, K, parts, a_blocked, stream)) return status;
-#define BH_FINISH_NORM_ROWS(PARTS, ROWS)                                                                              \
-  gemm_parts_finish_norm_kernel<PARTS, ROWS><<<(M + ROWS - 1) / ROWS, 128 * ROWS, 0, stream>>>(                        \
+  if (parts == 1) {
+    if (int status = gemm_ring_launch(a, w, residual, BH_F32, 1, M, N, K, 0, ring.tile, 0, GateForm{}, stream)) return status;
+    return bh_rmsnorm(residual, nullptr, norm_weight, norm_weight_dtype, normed, BH_BF16, M, N, eps, normed_blocked ? 16 : 0, stream);
+  }
+  if (int status = gemm_ring_launch_parts(a, w, (float*)scratch, M, N, K, ring, stream)) return status;
+#define BH_FINISH_NORM_ROWS(PARTS, ROWS, ROW_WAVES)                                                                    \
+  gemm_parts_finish_norm_kernel<PARTS, ROWS, ROW_WAVES><<<(M + ROWS - 1) / ROWS, 64 * ROW_WAVES * ROWS, 0, stream>>>(  \
       (const float*)scratch, residual, M, N, parts, norm_weight, norm_weight_dtype == BH_F32, eps, (uint16_t*)normed, \
       normed_blocked)
   // Rows per block: at 1,024 rows two ran 4 % faster than eight (more and smaller blocks), from 2,048 rows on all ran
-  // alike; full 128-byte lines of the blocked output take eight.
-  const int rows_per_block = M >= 4096 ? 8 : M >= 2048 ? 4 : 2;
+  // alike; full 128-byte lines of the blocked output take eight.  Rows that are fewer than twice the compute units: a row a block and
+  // eight waves on it (252 rows of 5,120 from eight parts of 17,408, the product with this kernel behind it 75.9 -> 73.6 us).
+  const int rows_per_block = M >= 4096 ? 8 : M >= 2048 ? 4 : M >= 2 * bh_compute_units() ? 2 : 1;
 #define BH_FINISH_NORM(PARTS)                          \
   do {                                                 \
-    if (rows_per_block == 8) BH_FINISH_NORM_ROWS(PARTS, 8); \
-    else if (rows_per_block == 4) BH_FINISH_NORM_ROWS(PARTS, 4); \
-    else BH_FINISH_NORM_ROWS(PARTS, 2); \
+    if (rows_per_block == 8) BH_FINISH_NORM_ROWS(PARTS, 8, 2); \
+    else if (rows_per_block == 4) BH_FINISH_NORM_ROWS(PARTS, 4, 2); \
+    else if (rows_per_block == 2) BH_FINISH_NORM_ROWS(PARTS, 2, 2); \
+    else BH_FINISH_NORM_ROWS(PARTS, 1, 8); \
   } while (0)
   if (parts <= 2) BH_FINISH_NORM(2);
   else if (parts <= 4) BH_FINISH_NORM(4);
-  else BH_FINISH_NORM(MAX_TURNS_PARTS);
+  else BH_FINISH_NORM(MAX_RING_PARTS);
 #undef BH_FINISH_NORM_ROWS
 #undef BH_FINISH_NORM
   return bh_check_launch("gemm_parts_finish_norm");
@@ -1542,8 +1556,8 @@ extern "C" int bh_gemm_bf16_then_norm(const void* a, const void* w, float* resid
 // K goes in parts through the kernel for many rows.  `sums`: parts * M * N floats.
 extern "C" int bh_gemm_bf16_bare_parts(int M, int N, int K, int layout) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int parts = gemm_turns_parts(M, N, K, layout, 0);
-  return parts > 1 && parts <= MAX_TURNS_PARTS ? parts : 0;
+  const RingPlan ring = gemm_ring_bare_plan(M, N, K, layout);
+  return ring.tile >= 0 && ring.parts > 1 && ring.parts <= MAX_RING_PARTS ? ring.parts : 0;
 }
 extern "C" int bh_gemm_bf16_bare(const void* a, const void* w, float* sums, int M, int N, int K, int layout, int a_blocked,
                                  hipStream_t stream) {
@@ -1551,5 +1565,6 @@ extern "C" int bh_gemm_bf16_bare(const void* a, const void* w, float* sums, int 
   BH_REQUIRE(parts > 0, "gemm_bf16_bare: a product of M=%d N=%d K=%d is not left in parts (bh_gemm_bf16_bare_parts)", M, N, K);
   BH_REQUIRE(a && w && sums, "gemm_bf16_bare: every operand is needed");
   BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)sums) % 16 == 0, "gemm_bf16_bare: operands must be 16-byte aligned");
-  return gemm_turns_launch_parts(a, w, sums, M, N, K, parts, a_blocked, stream);
+  BH_REQUIRE(a_blocked, "gemm_bf16_bare: the activations lie in blocks of 16 rows");
+  return gemm_ring_launch_parts(a, w, sums, M, N, K, gemm_ring_bare_plan(M, N, K, layout), stream);
 }

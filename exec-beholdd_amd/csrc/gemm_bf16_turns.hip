@@ -1,8 +1,8 @@
 // bfloat16 matrix products of many rows, C[M, N] (+)= A[M, K] * W[N, K]^T with W in the tiles layout
-// (see gemm_bf16.hip), for the shapes where a 256-row tile fills the chip: prompts from 320 tokens on.
+// (see gemm_bf16.hip), for the shapes where a 256-row tile fills the chip: prompts from 129 tokens on.
 //
 // A workgroup of eight waves owns 256 rows x 32 YB weight rows.  Its waves form two groups of four (one wave
-// of each group per SIMD) that take turns: while one group multiplies (32, 24 or 16 MFMAs on operands it holds
+// of each group per SIMD) that take turns: while one group multiplies (32 or 24 MFMAs on operands it holds
 // in registers), the other reads its next operands from LDS and asks for data that is three steps ahead; a
 // barrier ends every turn.  So the matrix cores always have one wave per SIMD that does nothing but multiply,
 // and no wave waits for memory in the middle of its multiplies.  A step is half a 64-wide k slice: the 32 k
@@ -10,23 +10,20 @@
 //
 // Global memory goes to LDS directly (16-byte loads that write LDS at the wave's base + 16 * lane): 1 KB per
 // load, which is one operand of 16 rows x 32 k in lane order, so that reading it back is one conflict-free
-// 16-byte read per lane.  Four lanes bring 256 bytes of a block of W; of A they bring 64 consecutive bytes of a
-// row when A lies in rows, so that a quarter of a wave touches 16 cache lines, each for a quarter of its bytes,
-// and every line is asked for again by the next step.  A in blocks of 16 rows x 32 k in operand order
-// (bh_blocked_index in layout.h; the kernels that produce activations write it that way for this reader) makes
-// an operand 1 KB of contiguous memory like W's: gate/up at 2,048 rows 333 -> 293 us (1.41 PFLOP/s), qkv 100 -> 85,
-// down with 128-wide tiles 247 -> 181, with 256-wide tiles at 4,096 rows 348 -> 284 (1.45).  The vendor library's
+// 16-byte read per lane.  A lies in blocks of 16 rows x 32 k in operand order (bh_blocked_index in layout.h; the
+// kernels that produce activations write it that way for this reader), so that an operand is 1 KB of contiguous
+// memory like W's; from plain rows, of which a quarter of a wave touched 16 cache lines for a quarter of their
+// bytes each, gate/up at 2,048 rows took 333 us instead of 293 (1.41 PFLOP/s).  The vendor library's
 // product (torch.matmul, bfloat16) takes 287 us for the gate/up shape without the gate (1.44 PFLOP/s), 81 us for qkv,
 // and reaches 1.51 to 1.55 at its best shapes (4,096 and 8,192 rows): that, not 2.5, is what these matrix cores
 // give with operands from memory.
 // LDS holds four steps (4 x (16 + 2 YB) KB); a step's region is loaded again as soon as both groups have read
 // it, which is five to six turns before it is read next.
 //
-// Measured at the Qwen3-8B shapes, 2,048 rows, activations in rows, each product alone: gate/up with SwiGLU 404 -> 330 us
-// (1.25 PFLOP/s), qkv 132 -> 104 us with tiles of 192 weight rows (256 of them, one per compute unit), o 102 ->
-// 84 us with 128; in the whole model 381 -> 338, 115 -> 101 and 87 -> 94 us (which is why the o and down
-// projections there go through K in parts of the widest tile instead, see turns_plan: 77 us for o, finishing
-// kernel included).
+// It stands beside the ring of gemm_bf16_ring.hip, which keeps both waves of a SIMD busy at once: with tiles of 256 x 256 and 256 x 192 the
+// matrix cores' power sets the clock, and taking turns is the more frugal way (8,160 rows, us here / there: gate and up of 12,288 x 4,096
+// 1,170 / 1,235, 4,096 x 12,288 551 / 585, 6,144 x 4,096 293 / 303; 2,048 x 8,192 x 2,048 56 / 58); with narrower tiles, which wait for their
+// operands more than for the matrix cores, the ring wins (256 x 128 at 2,048 x 4,096 x 4,096: 84 / 63).
 // What bounds it (activations in rows): the loads alone (no multiplies) take 0.9 of the whole kernel's time, the
 // multiplies alone 0.6, the multiplies with their operand reads from LDS 0.8 (1.46 to 1.58 PFLOP/s).  It is not the loads' latency (five or six steps in LDS instead of four changed nothing; touching the
 // lines three slices ahead with 4-byte loads made it slower, 0.9 PFLOP/s for gate/up: loads retire in order, so
@@ -36,10 +33,6 @@
 // would be all that its 16 channels of 64 bytes per clock can give; a compute unit alone gets at most about
 // 43 bytes per clock out of L1 and L2 (loads only, to LDS or to registers alike), and a tile of 256 x 128 asks
 // for 47 where 256 x 256 asks for 32, which is why the narrower tiles lose.
-// Tried for the products with 4,096 weight rows, which have only 128 tiles of 256 x 256: a tile of 256 x 128
-// in which the two groups divide the k steps between them (every wave 64 x 128, sums exchanged through LDS at
-// the end) ran like the 128-wide tile (0.8 PFLOP/s); A brought in whole 128-byte lines and kept permuted in
-// LDS was slower (its slice buffer is free only four turns before it is read again).
 #include "gemm_bf16_turns.h"
 #include <type_traits>
 
@@ -71,10 +64,9 @@ __device__ inline bf16x8_t as_bf16x8(u32x4_t v) { return __builtin_bit_cast(bf16
 // first): a slice of rows is then fetched once for four compute units and a slice of weights once for eight,
 // 12 slices for 32 tiles, where a whole column of row tiles under one weight tile would fetch 33 (measured
 // with the chip full: L2 delivers 26 TB/s to the compute units, what lies beyond it 7; at 149,070 rows x
-// 51,200 weight rows the column order read 305 GB per product and ran at 1.14 PFLOP/s).  Up to eight row tiles
-// (2,048 rows) both orders are the same; at 8,192 rows x 4,096 the gate and up product went from 1,245 to
-// 1,165 us (1.42 PFLOP/s) and the down projection from 600 to 563 us (1.46).  Only speed depends on where
-// the workgroups really run.
+// 51,200 weight rows the column order read 305 GB per product and ran at 1.14 PFLOP/s).  At 8,192 rows x 4,096
+// the gate and up product went from 1,245 to 1,165 us (1.42 PFLOP/s) and the down projection from 600 to 563 us
+// (1.46).  Only speed depends on where the workgroups really run.
 __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int* tile_n, int* tile_m) {
   constexpr int BM = 8, BN = 4;
   const int total = n_tiles * m_tiles, xcd = blockIdx.x % 8, each = total / 8, more = total % 8;
@@ -98,14 +90,13 @@ __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int* tile_n, 
 // MODE 0: bfloat16 output.  1: float32 output, optionally added to what is there.  2: SwiGLU (the gate as `form` says), bfloat16 output
 // (N outputs; W has 2 N rows, gate rows then up rows; a wave's weight rows are the gate and the up rows of
 // the same outputs).  YB: blocks of 16 weight rows per wave.
-// A tile that would stick out of the matrix is moved back inside and stores only what it owns.
-// a_blocked: A lies in blocks of 16 rows x 32 k in operand order (bh_blocked_index), so that a wave's load of an
-// operand is 1 KB of contiguous memory; its buffer holds whole tiles of 256 rows, and a tile that sticks out
-// below stays where it is and stores only the rows that exist.  c_blocked (MODE 2): the output likewise.
+// A tile that would stick out of the weight rows is moved back inside and stores only what it owns.
+// A's buffer holds whole tiles of 256 rows, and a tile that sticks out below stays where it is and stores only the rows
+// that exist.  c_blocked (MODE 2): the output lies in blocks of 16 rows.
 template <int MODE, int YB>
 __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ w,
                                                       void* __restrict__ c, int M, int N, int K, int accumulate,
-                                                      int a_blocked, int c_blocked, GateForm form) {
+                                                      int c_blocked, GateForm form) {
   constexpr int OUTS = MODE == 2 ? 16 * YB : 32 * YB;
   constexpr int CHUNKS = 16 + 2 * YB;
   constexpr int WL = YB / 2;   // W chunks per loading wave
@@ -116,8 +107,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
   const int g = wave / 4, i4 = wave % 4;
   int tile_n, tile_m;
   tile_of_workgroup((N + OUTS - 1) / OUTS, (M + 255) / 256, &tile_n, &tile_m);
-  const int m_own = tile_m * 256, n_own = tile_n * OUTS;
-  const int m0 = a_blocked ? m_own : min(m_own, M - 256), n0 = min(n_own, N - OUTS);
+  const int m0 = tile_m * 256, n_own = tile_n * OUTS, n0 = min(n_own, N - OUTS);
   // K in parts (blockIdx.y, MODE 1 only): part p multiplies its share of k and leaves the bare sums at
   // c + p * M * N for the finishing kernel of gemm_bf16.hip; one part is the whole product.
   const int k_part = K / gridDim.y, k_first = blockIdx.y * k_part;
@@ -125,11 +115,10 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 
   // The first group brings A (four blocks of 16 rows per wave), the second W (YB / 2 blocks per wave).
   // A step takes 32 consecutive k: lane (row r = lane % 16, group q = lane / 16) holds k 8 q .. 8 q + 7 of them,
-  // so four lanes bring 64 consecutive bytes of a row.  In W's tiles layout those are the 16-byte pieces
+  // 1 KB of contiguous memory of a block of A.  In W's tiles layout those are the 16-byte pieces
   // 4 v + q of the row (v: first or second step of the slice), piece p at half p % 2, lane 16 (p / 2) + r.
-  const uint16_t* a_src = a_blocked ? a + ((size_t)((m0 + 64 * i4) / 16) * (K / 32) + k_first / 32) * 512 + lane * 8
-                                    : a + (size_t)(m0 + 64 * i4 + lane % 16) * K + k_first + 8 * (lane / 16);
-  const size_t a_block = a_blocked ? (size_t)(K / 32) * 512 : (size_t)16 * K;   // from 16 rows to the next
+  const uint16_t* a_src = a + ((size_t)((m0 + 64 * i4) / 16) * (K / 32) + k_first / 32) * 512 + lane * 8;
+  const size_t a_block = (size_t)(K / 32) * 512;   // from 16 rows to the next
   const int w_lane = ((lane / 16) % 2) * 512 + (16 * (lane / 32) + lane % 16) * 8;   // + 256 elements for the second step
   const uint16_t* w_src[WL];
 #pragma unroll
@@ -138,14 +127,13 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
     const int nb = MODE == 2 ? (y < YB / 2 ? 0 : N / 16) + n0 / 16 + (YB / 2) * gg + y % (YB / 2) : n0 / 16 + rb;
     w_src[b] = w + ((size_t)nb * (K / 64) + k_first / 64) * 1024 + w_lane;
   }
-  auto fetch_a = [&](int j, int region) {   // step j = half u of slice s
-    const int s = j >> 1, u = j & 1;
+  auto fetch_a = [&](int j, int region) {
 #pragma unroll
     for (int b = 0; b < 4; ++b)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a_src + b * a_block + (a_blocked ? j * 512 : s * 64 + u * 32)),
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a_src + b * a_block + j * 512),
                                        (__attribute__((address_space(3))) void*)&lds[(region * CHUNKS + 4 * i4 + b) * 64], 16, 0, 0);
   };
-  auto fetch_w = [&](int j, int region) {
+  auto fetch_w = [&](int j, int region) {   // step j = half u of slice s
     const int s = j >> 1, u = j & 1;
 #pragma unroll
     for (int b = 0; b < WL; ++b)
@@ -226,7 +214,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int row = m + 16 * x;
-      if (row < m_own || row >= M) continue;
+      if (row >= M) continue;
 #pragma unroll
       for (int y = 0; y < YB / 2; ++y) {
         const int n = n0 + 8 * YB * g + 16 * y + 4 * (lane / 16);
@@ -241,7 +229,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int row = m + 16 * x;
-      if (row < m_own || row >= M) continue;
+      if (row >= M) continue;
 #pragma unroll
       for (int y = 0; y < YB; ++y) {
         const int n = n0 + 16 * YB * g + 16 * y + 4 * (lane / 16);
@@ -268,136 +256,30 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 #undef TICK
 
 template <int MODE>
-void launch(const void* a, const void* w, void* c, int blocks, int M, int N, int K, int accumulate, int a_blocked,
-            int c_blocked, GateForm form, hipStream_t stream, int parts = 1) {
+void launch(const void* a, const void* w, void* c, int blocks, int M, int N, int K, int accumulate, int parts, int c_blocked, GateForm form,
+            hipStream_t stream) {
   const int outs = (MODE == 2 ? 16 : 32) * blocks;
   dim3 grid(((N + outs - 1) / outs) * ((M + 255) / 256), parts);
-#define BH_TURNS(YB) \
-  gemm_turns_kernel<MODE, YB><<<grid, 512, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, c, M, N, K, accumulate, a_blocked, c_blocked, form)
-  if (blocks == 8) BH_TURNS(8);
-  else if (blocks == 6) BH_TURNS(6);
-  else BH_TURNS(4);
-#undef BH_TURNS
+  if (blocks == 8)
+    gemm_turns_kernel<MODE, 8><<<grid, 512, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, c, M, N, K, accumulate, c_blocked, form);
+  else
+    gemm_turns_kernel<MODE, 6><<<grid, 512, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, c, M, N, K, accumulate, c_blocked, form);
 }
 
 }  // namespace
 
-bool gemm_turns_can(int M, int N, int K, int layout, int activation, int blocks) {
-  if (blocks != 8 && blocks != 6 && blocks != 4) return false;
-  const int outs = (activation ? 16 : 32) * blocks;
-  return layout == 1 && M >= 256 && N >= outs && N % 16 == 0 && K >= 128 && K % 128 == 0 &&
+bool gemm_turns_can(int M, int N, int K, int mode, int blocks, int parts) {
+  if (blocks != 8 && blocks != 6) return false;
+  const int outs = (mode == 2 ? 16 : 32) * blocks;
+  return M > 0 && N >= outs && N % 16 == 0 && parts >= 1 && (mode == 1 || parts == 1) && K >= 128 * parts && K % (128 * parts) == 0 &&
          (long)((N + outs - 1) / outs) * ((M + 255) / 256) < (1L << 31);   // offsets into A, W and C are 64-bit
 }
 
-// Which way, if any.  A tile of YB blocks per wave costs a compute unit YB x cost(YB) units of time, where cost
-// is what the narrower tiles lose (measured 1.43, 1.16 and 1.07 PFLOP/s for 8, 6 and 4 with the chip full and the
-// activations in blocks; 1.25, 1.11 and 0.90 with activations in rows), and
-// the chip works in rounds of 256 tiles; a tile of its own is taken if that estimate reaches 0.6 PFLOP/s, which
-// the other tiled kernels stay below at these sizes (with 0.8 as the bar, prefill steps of 320 to 768 tokens were 2 to
-// 18 % slower at the Qwen3-8B, 14B and 32B widths, and no length was faster).  Products with so few of the widest tiles that much of the
-// chip would idle can instead cut K into parts over as many times the workgroups, each leaving its bare sums in
-// scratch memory ([part][row][weight row], float32) for a finishing kernel of gemm_bf16.hip; that costs about
-// 0.85 of the tile's rate (for the o projection of the Qwen3-8B shape at 2,048 rows the parts and the 128-wide
-// tile run alike alone, but the whole prefill went 31.8 -> 30.5 ms with the parts).
-namespace {
-struct TurnsPlan {
-  int blocks;   // tile width for the product in one launch, or 0
-  int parts;    // parts of K, or 1
-  int part_blocks = 8;   // the tile width of the parts
-};
-TurnsPlan turns_plan(int M, int N, int K, int layout, int activation) {
-  TurnsPlan plan = {0, 1};
-  if (M <= 256) return plan;   // up to there a norm may ride on the product, which this kernel does not carry
-  double best_rate = 600.0;    // TFLOP/s: what a tile of its own has to reach
-  double direct_rate = 0.0;
-  const double work = (double)M * (activation ? 2.0 * N : (double)N);   // rows x weight rows
-  const int units = bh_compute_units();   // a round is one tile per compute unit (the rates below were measured with 256)
-  for (int blocks = 8; blocks >= 4; blocks -= 2) {
-    if (!gemm_turns_can(M, N, K, layout, activation, blocks)) continue;
-    const int outs = (activation ? 16 : 32) * blocks;
-    const long tiles = (long)((N + outs - 1) / outs) * ((M + 255) / 256);
-    const long rounds = (tiles + units - 1) / units;
-    const double cost = blocks == 8 ? 1.0 : blocks == 6 ? 1.23 : 1.34;
-    const double rate = 1430.0 * (units / 256.0) * work / ((double)rounds * units * 256 * (activation ? 2 : 1) * outs * cost);
-    if (rate >= best_rate) best_rate = direct_rate = rate, plan.blocks = blocks;
-  }
-  if (!activation && M >= 320 && gemm_turns_can(M, N, K, layout, 0, 8)) {
-    // As many parts (8, 4 or 2) as keep the workgroups within one round and every part at least 512 long; worth
-    // it from about five eighths of the chip on.  Measured at the Qwen3-8B widths against the other kernels, us:
-    // 512 rows: down in 8 parts 88 -> 72 (o in 4 parts, half the chip, 41 -> 45; in 8 parts of 512 the prefill step of
-    // 512 tokens is 0.5 % faster than with the older tiles); 768 rows: o 71 -> 53,
-    // down 195 -> 102 in 4; 1,024 rows: o 72 -> 57, down 196 -> 111 in 4; 1,536 rows: o 93 -> 77, down 219 -> 173 in 2;
-    // 2,048 rows: down 240 -> 199 in 2.  From 320 rows on (a whole prefill step of the Qwen3-8B shape with the parts from 257
-    // rows on instead of from 512 on: 272 tokens 9.15 -> 9.24 ms, 320 tokens 9.34 -> 9.25, 384 tokens 9.62 -> 9.48, 448 tokens
-    // 10.88 -> 9.77).
-    // With the widest tile first; where that needs eight parts (257 to 512 rows at these widths), four parts of the
-    // 128-wide tile instead: half the bare sums to write and to read again (512 rows at the Qwen3-8B widths, product +
-    // finishing kernel, o and down on average: 42.5 + 19.9 -> 40.9 + 14.1 us; where the widest tile needs four parts or
-    // two, the narrower one lost: 640 rows 51.8 + 16.0 -> 64.0 + 13.1, 1,024 rows 60.8 + 21.7 -> 73.8 + 17.4; the
-    // 192-wide tile lost everywhere).
-    auto parts_of = [&](int pb) {
-      const int outs = 32 * pb;
-      const long tiles = (long)((N + outs - 1) / outs) * ((M + 255) / 256);
-      int parts = 8;
-      while (parts > 1 && (tiles * parts > units || K / parts < 512 || K % (128 * parts) != 0)) parts /= 2;
-      return parts > 1 && tiles * parts >= units * 5 / 8 ? parts : 1;
-    };
-    int pb = 8, parts = parts_of(8);
-    if (parts == 8 && gemm_turns_can(M, N, K, layout, 0, 4) && parts_of(4) == 4) pb = 4, parts = 4;
-    // Where the widest tile finds no cut that fills five eighths of the chip within one round (the q/k/v projection of the
-    // Qwen3-8B shape at 513 to 768 rows: 72 tiles, 144 workgroups in two parts, 288 in four) and no tile of its own is worth it
-    // either, the 192-wide tile may (96 tiles, 192 workgroups in two parts), then the 128-wide one.
-    if (parts == 1 && plan.blocks == 0)
-      for (int narrower = 6; narrower >= 4 && parts == 1; narrower -= 2)
-        if (gemm_turns_can(M, N, K, layout, 0, narrower) && parts_of(narrower) > 1) pb = narrower, parts = parts_of(narrower);
-    if (parts > 1) {
-      const double rate = 0.85 * 1430.0 * (units / 256.0) * work / ((double)units * 256 * 32 * pb / parts * (pb == 8 ? 1.0 : pb == 6 ? 1.23 : 1.34));
-      if (rate > direct_rate) plan.blocks = 0, plan.parts = parts, plan.part_blocks = pb;
-    }
-  }
-  return plan;
-}
-}  // namespace
-
-int gemm_turns_blocks(int M, int N, int K, int layout, int activation) {
-  return turns_plan(M, N, K, layout, activation).blocks;
-}
-int gemm_turns_parts(int M, int N, int K, int layout, int activation) {
-  return turns_plan(M, N, K, layout, activation).parts;
-}
-
-int gemm_turns_launch_parts(const void* a, const void* w, float* sums, int M, int N, int K, int parts, int a_blocked,
-                            hipStream_t stream) {
-  const int pb = turns_plan(M, N, K, 1, 0).part_blocks;
-  BH_REQUIRE(parts >= 1 && K % (128 * parts) == 0 && gemm_turns_can(M, N, K / parts, 1, 0, pb),
-             "gemm_turns: M=%d N=%d K=%d cannot be multiplied in %d parts of K", M, N, K, parts);
-  BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)sums) % 16 == 0, "gemm_turns: operands must be 16-byte aligned");
-  launch<1>(a, w, sums, pb, M, N, K, 0, a_blocked, 0, GateForm{}, stream, parts);
+int gemm_turns_launch(const void* a, const void* w, void* c, int mode, int accumulate, int M, int N, int K, int blocks, int parts,
+                      int c_blocked, GateForm form, hipStream_t stream) {
+  BH_REQUIRE(gemm_turns_can(M, N, K, mode, blocks, parts), "gemm_turns: M=%d N=%d K=%d with %d blocks per wave in %d parts of K is not a product this kernel takes", M, N, K, blocks, parts);
+  if (mode == 2) launch<2>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
+  else if (mode == 1) launch<1>(a, w, c, blocks, M, N, K, accumulate, parts, 0, form, stream);
+  else launch<0>(a, w, c, blocks, M, N, K, 0, 1, 0, form, stream);
   return bh_check_launch("gemm_turns");
-}
-
-int gemm_turns_launch(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K,
-                      int activation, int blocks, int a_blocked, int c_blocked, GateForm form, hipStream_t stream) {
-  BH_REQUIRE(gemm_turns_can(M, N, K, 1, activation, blocks),
-             "gemm_turns: a product of M=%d N=%d K=%d with %d blocks per wave is not one this kernel takes "
-             "(M >= 256, K a multiple of 128, N a multiple of 16 and at least a tile)", M, N, K, blocks);
-  BH_REQUIRE(c_dtype == BH_F32 || (c_dtype == BH_BF16 && !accumulate),
-             "gemm_turns: output float32, or bfloat16 without accumulation");
-  BH_REQUIRE(!activation || c_dtype == BH_BF16, "gemm_turns: SwiGLU writes bfloat16");
-  BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0 && (c_dtype == BH_F32 || N % 4 == 0),
-             "gemm_turns: operands and output must be 16-byte aligned");
-  BH_REQUIRE(!c_blocked || (activation && N % 32 == 0), "gemm_turns: only SwiGLU writes its output in blocks, and N=%d must be a multiple of 32", N);
-  if (activation) launch<2>(a, w, c, blocks, M, N, K, 0, a_blocked, c_blocked, form, stream);
-  else if (c_dtype == BH_F32) launch<1>(a, w, c, blocks, M, N, K, accumulate, a_blocked, 0, form, stream);
-  else launch<0>(a, w, c, blocks, M, N, K, 0, a_blocked, 0, form, stream);
-  return bh_check_launch("gemm_turns");
-}
-
-// For tests and measurements: the kernel at a given tile width, whatever gemm_turns_blocks would choose.
-extern "C" int bh_gemm_bf16_turns(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N,
-                                  int K, int activation, int blocks, int a_blocked, int c_blocked, hipStream_t stream) {
-  return gemm_turns_launch(a, w, c, c_dtype, accumulate, M, N, K, activation != 0, blocks, a_blocked, c_blocked, bh_gate_form(activation), stream);
-}
-extern "C" int bh_gemm_bf16_turns_blocks(int M, int N, int K, int layout, int activation) {
-  return gemm_turns_blocks(M, N, K, layout, activation);
 }

@@ -443,7 +443,7 @@ __device__ inline float head_sum(float v) {
 }
 
 // PARTS: `qkv` holds no bfloat16 rows but the float32 sums of a product whose K was cut into parts,
-// [parts][n_rows][(H + 2 KVH) * HD], as the kernel left them whose wave groups take turns: an element is the sum
+// [parts][n_rows][(H + 2 KVH) * HD], as the kernels for many rows left them: an element is the sum
 // of its parts in their order, rounded to bfloat16 (what that product's finishing kernel would have written, which
 // this takes the place of, and the bfloat16 rows' trip to memory and back with it).
 template <bool PARTS, int RN>

@@ -542,15 +542,15 @@ class HipKernels(KernelSizes):
         if (then_norm is not None and ahead is None and accumulate and packed and out.dtype == torch.float32
                 and not activation and then_norm.weight.shape == (n,) and then_norm.weight.dtype in _CODES
                 and finishes_norm):
-            # many rows, K in parts: the finishing kernel owns whole rows and finishes the norm itself
+            # many rows: with K in parts the finishing kernel owns whole rows and finishes the norm itself, else its launch follows
             normed = self.new_rows(m, n, torch.bfloat16, *self._reader_of(then_norm))
             if _block_rows(normed) not in (0, 16):
                 normed = torch.empty((m, n), dtype=torch.bfloat16, device=self.device)
-            scratch = torch.empty(scratch_bytes // 4, dtype=torch.float32, device=self.device)
+            scratch = torch.empty(scratch_bytes // 4, dtype=torch.float32, device=self.device) if scratch_bytes else None
             self._check(self.lib.bh_gemm_bf16_then_norm(
                 self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out", (torch.float32,)), m, n, k, 1,
                 self._ptr(then_norm.weight, "norm weight"), _code(then_norm.weight, "norm weight"), float(then_norm.eps),
-                self._ptr(normed, "norm rows"), self._ptr(scratch, "gemm scratch"), int(a_block_rows == 16),
+                self._ptr(normed, "norm rows"), self._ptr(scratch, "gemm scratch", None, True), int(a_block_rows == 16),
                 int(isinstance(normed, BlockedRows)), self._stream()))
             return True, normed
         behind = None
@@ -636,8 +636,8 @@ class HipKernels(KernelSizes):
         return bool(self.lib.bh_qk_norm_rope_cache_takes_sums(int(n_rows), int(head_dim), int(rot)))
 
     def gemm_turns(self, a, w, out, blocks, accumulate=False, swiglu=False):
-        """The product for many rows whose wave groups take turns, at a given tile width (`blocks` of 16
-        weight rows per wave: 8, 6 or 4), whatever `gemm` would choose for these sizes: out[M, N] (+)= a @ w^T,
+        """The product for many rows on tiles of 256 rows at a given width (`blocks` of 32 weight rows: 8, 6 or 4),
+        whatever `gemm` would choose for these sizes: out[M, N] (+)= a @ w^T,
         or with `swiglu` out[M, F] = silu(a @ w[:F]^T) * (a @ w[F:]^T).  `w` is a PackedWeight."""
         if (not isinstance(w, PackedWeight) or a.dim() != 2 or out.dim() != 2 or a.dtype != torch.bfloat16
                 or _block_rows(a) not in (0, 16) or _block_rows(out) not in (0, 16)):
@@ -646,13 +646,16 @@ class HipKernels(KernelSizes):
         n = out.shape[1]
         if w.shape[1] != k or w.shape[0] != (2 * n if swiglu else n) or out.shape[0] != m:
             raise KernelError(f"gemm_turns: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
+        if k % 32 == 0:
+            a = self._in_blocks_of(a, 16)
         self._check(self.lib.bh_gemm_bf16_turns(
             self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), _code(out, "gemm out"),
             int(bool(accumulate)), m, n, k, int(bool(swiglu)), int(blocks), int(_block_rows(a) == 16),
             int(_block_rows(out) == 16), self._stream()))
 
     def gemm_turns_blocks(self, m, n, k, swiglu=False):
-        """The tile width `gemm` uses for a packed product of these sizes (0: another kernel runs it)."""
+        """The width of the tiles of 256 rows on which `gemm` runs a packed product of these sizes in one go, in blocks of 32
+        weight rows (0: it runs otherwise)."""
         return int(self.lib.bh_gemm_bf16_turns_blocks(m, n, k, 1, int(bool(swiglu))))
 
     def _takes_norm(self, a, w, n, activation):
