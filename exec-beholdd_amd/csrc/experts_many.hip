@@ -4,17 +4,21 @@
 // A workgroup of four waves owns 32 XB pairs of one expert and 128 of its weight rows (gated: the gate and the up rows of the same 64
 // outputs, so that a lane holds both sums of an output), a wave 16 XB pairs x 64 weight rows.  Which ones, every workgroup finds by
 // itself from the experts' counts: the grid is as large as the pairs allow at most, and what lies beyond the last tile ends at once.
-// A step is 32 k: operands go from global memory straight to LDS in lane order (1 KB a load; a pair's input row is found through
-// its list, 64 bytes of it a load), three steps ahead in a ring of four, a barrier a step; two workgroups share a compute unit and
-// hide each other's barriers.
+// Operands go from global memory straight to LDS (1 KB a load): a pair's input row, found through its list, in units of 64 k, so that a
+// load takes whole cache lines, into a ring of three; weight rows in steps of 32 k, the k of one matrix instruction, in lane order into a
+// ring of four.  While step j is multiplied from registers, the operands of step j + 1 are read from LDS into the other set of registers
+// and what comes up to four steps later is asked for, a read, a load and a group of MFMAs in turn; a barrier a step.  Two workgroups
+// share a compute unit and hide each other's barriers.
 // Bound by the operands' way from the L2 and memory: weights are read once a tile of pairs, and neighbours on an XCD are the tiles
-// of pairs of the same weight rows.
-// Measured (32 experts, gate and up / down, us): width 2,048, ff 768, 262 pairs an expert 112 / 71 (0.47 and 0.37 PFLOP/s), 474 / 239
-// in the tiles of experts_mfma.hip from row-major matrices, whose 128 weight rows a slice of k lie 4 KB apart; 16 pairs 45 / 21
-// (201 MB at 4.5 TB/s), 56 / 35 with experts_tiles, which reads the weights once for 16 pairs and is still ahead at 8 (35 / 21
-// against 42 / 21).  Width 4,096, ff 1,536, 256 pairs 379 / 219, where a product an expert of the kernels for one matrix took about
-// 25 us each; those reach twice the rate on large matrices, and the caller takes them there.
+// of pairs of the same weight rows.  Tiles of few steps (down: 24 for ff 768) pay for their start and their float32 output beside it.
+// Measured (32 experts, gate and up / down, us), in brackets with rows loaded in steps of 32 k, half a line a row and load, whose other
+// half came from the L2 once more, and each step's operands read from LDS before its MFMAs: width 2,048, ff 768, 263 pairs an expert
+// 87 / 63 (116 / 74), 0.61 and 0.42 PFLOP/s; 512 pairs 139 / 100 (176 / 117); 16 pairs 45 / 21 (47 / 21; 201 MB at 4.5 TB/s), where
+// experts_tiles, which reads the weights once for 16 pairs, takes 56 / 35 and is ahead up to 8 pairs.  Width 4,096, ff 1,536, 256 pairs
+// 290 / 170 (372 / 210).  8 experts, width 4,096, ff 4,096, 1,024 pairs 573 / 305 (748 / 405), 0.96 and 0.90 PFLOP/s.  The registers
+// in turn without the whole lines: 112 / 75 at the first size.
 #include "common.h"
+#include <type_traits>
 
 typedef __bf16 xm_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float xm_f32x4_t __attribute__((ext_vector_type(4)));
@@ -34,14 +38,24 @@ __device__ inline float activation(float g, float u, float limit, float alpha, f
 // s_waitcnt of gfx9: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8; waits for all LDS reads and until at most `vm` of the
 // wave's global loads are on their way.
 #define XM_WAIT(vm) __builtin_amdgcn_s_waitcnt(((vm) & 15) | (((vm) >> 4) << 14) | (7 << 4) | (0 << 8))
+// Every wave has waited for its loads.  Nothing may be moved across it by the compiler.
+#define XM_MEET()                         \
+  do {                                    \
+    __builtin_amdgcn_sched_barrier(0);    \
+    __builtin_amdgcn_s_barrier();         \
+    __builtin_amdgcn_sched_barrier(0);    \
+  } while (0)
 
 template <bool GATED, int XB>
-__global__ __launch_bounds__(256) void experts_many_kernel(const uint16_t* __restrict__ in, int in_div, const int32_t* __restrict__ list,
+__global__ __launch_bounds__(256, 2) void experts_many_kernel(const uint16_t* __restrict__ in, int in_div, const int32_t* __restrict__ list,
                                                            int capacity, const int32_t* __restrict__ counts, int E,
                                                            const uint16_t* __restrict__ w, void* __restrict__ out_raw, int K, int N,
                                                            float limit, float alpha, float shift, const float* __restrict__ in_weights) {
-  constexpr int ROWS = 32 * XB, OUTS = GATED ? 64 : 128, REGIONS = 4, CHUNKS = 2 * XB + 8;
-  __shared__ __attribute__((aligned(16))) xm_u32x4_t lds[REGIONS * CHUNKS * 64];   // [region][2 XB blocks of pairs, 8 of weights][lane]
+  constexpr int ROWS = 32 * XB, OUTS = GATED ? 64 : 128, STEPS = 4;
+  // [3 units of 64 k in turn][block of 16 pairs][16 rows x 8 pieces], then [STEPS steps of 32 k in turn][block of 16 weight rows][lane]; one
+  // array, for before a read from one of two arrays the compiler waits for all loads on their way to that one
+  __shared__ __attribute__((aligned(16))) xm_u32x4_t lds[3 * 2 * XB * 128 + STEPS * 8 * 64];
+  constexpr int W_RING = 3 * 2 * XB * 128;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_tiles = (N + OUTS - 1) / OUTS;
 
@@ -52,9 +66,9 @@ __global__ __launch_bounds__(256) void experts_many_kernel(const uint16_t* __res
   for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, BH_WAVE);
   total *= n_tiles;
   // workgroups go to the eight XCDs in turn; every XCD takes a stretch of (expert, weight tile, tile of pairs) in this order
-  const int each = (total + 7) / 8, place = blockIdx.x / 8;
-  const int id = (blockIdx.x % 8) * each + place;
-  if (place >= each || id >= total) return;      // the whole workgroup
+  const int each = (total + 7) / 8, turn = blockIdx.x / 8;
+  const int id = (blockIdx.x % 8) * each + turn;
+  if (turn >= each || id >= total) return;      // the whole workgroup
   int expert = -1, before = 0, count = 0, at = 0;
   for (int e0 = 0; e0 < E && expert < 0; e0 += 64) {
     const int mine = e0 + lane < E ? counts[e0 + lane] : 0, tiles = (mine + ROWS - 1) / ROWS * n_tiles;
@@ -81,16 +95,21 @@ __global__ __launch_bounds__(256) void experts_many_kernel(const uint16_t* __res
   const int p0 = (at % row_tiles) * ROWS, n0 = (at / row_tiles) * OUTS;
   const int32_t* pairs = list + (size_t)expert * capacity;
 
-  // What this wave brings every step: XB / 2 blocks of 16 pairs and two of 16 weight rows.  Lane (r = lane % 16, q = lane / 16) holds
-  // k 8 q .. 8 q + 7 of row r; in the weights' layout those are the pieces 4 v + q of the row (v: first or second step of a chunk of
-  // 64), piece p at half p % 2, lane 16 (p / 2) + r.  Pairs beyond the last one and weight rows beyond the last block repeat it.
-  constexpr int AL = XB / 2;
-  const uint16_t* from_in[AL];
+  // What this wave brings: of the pairs, XB / 2 blocks of 16 rows x a unit of 64 k, a whole cache line of eight rows a load (32 k would be
+  // half a line, whose other half the next step fetches from the L2 again); of the weights two blocks of 16 rows x a step of 32 k in
+  // the weights' own operand order: lane (r = lane % 16, q = lane / 16) takes the pieces 4 v + q of row r (v: first or second step of a
+  // chunk of 64), piece p at half p % 2, lane 16 (p / 2) + r.  Pairs beyond the last one and weight rows beyond the last block repeat it.
+  // The 16-byte piece c of row r of a block of pairs lies at place c ^ (r % 8) ^ (r / 8) of the row's eight, so that the 16 rows whose
+  // piece c a quarter of a wave reads lie in different banks.
+  constexpr int AL = XB / 2, EACH = AL + 2;      // a wave's loads a step: half its blocks' rows of a unit, and its weights of a step
+  const uint16_t* from_in[AL][2];
 #pragma unroll
-  for (int b = 0; b < AL; ++b) {
-    const int p = min(p0 + 16 * (AL * wave + b) + lane % 16, count - 1);
-    from_in[b] = in + (size_t)(pairs[p] / in_div) * K + 8 * (lane / 16);
-  }
+  for (int b = 0; b < AL; ++b)
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int p = min(p0 + 16 * (AL * wave + b) + 8 * half + lane / 8, count - 1);
+      from_in[b][half] = in + (size_t)(pairs[p] / in_div) * K + 8 * ((lane % 8) ^ (lane / 8) ^ half);
+    }
   const uint16_t* from_w[2];
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -101,48 +120,86 @@ __global__ __launch_bounds__(256) void experts_many_kernel(const uint16_t* __res
     from_w[b] = w + ((size_t)expert * (GATED ? 2 : 1) * (N / 16) + block) * (K / 64) * 1024 + ((lane / 16) % 2) * 512 +
                 (16 * (lane / 32) + lane % 16) * 8;
   }
-  auto fetch = [&](int j) {
-    const int region = (j & (REGIONS - 1)) * CHUNKS;
-#pragma unroll
-    for (int b = 0; b < AL; ++b)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from_in[b] + j * 32),
-                                       (__attribute__((address_space(3))) void*)&lds[(region + AL * wave + b) * 64], 16, 0, 0);
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from_w[b] + (size_t)(j >> 1) * 1024 + (j & 1) * 256),
-                                       (__attribute__((address_space(3))) void*)&lds[(region + 2 * XB + 2 * wave + b) * 64], 16, 0, 0);
+  auto ask_rows = [&](int b, int half, int unit, int place) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from_in[b][half] + (size_t)unit * 64),
+                                     (__attribute__((address_space(3))) void*)&lds[((place * 2 * XB + AL * wave + b) * 2 + half) * 64], 16, 0, 0);
+  };
+  auto ask_weights = [&](int b, int step) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from_w[b] + (size_t)(step >> 1) * 1024 + (step & 1) * 256),
+                                     (__attribute__((address_space(3))) void*)&lds[W_RING + ((step % STEPS) * 8 + 2 * wave + b) * 64], 16, 0, 0);
   };
 
-  const int wm = wave / 2, wn = wave % 2, J = K / 32;
+  const int wm = wave / 2, wn = wave % 2, steps = K / 32, units = K / 64;
   xm_f32x4_t acc[XB][4];
 #pragma unroll
   for (int x = 0; x < XB; ++x)
 #pragma unroll
     for (int y = 0; y < 4; ++y) acc[x][y] = xm_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // K is a multiple of 64: at least two steps
-  for (int j = 0; j < 3 && j < J; ++j) fetch(j);
-  constexpr int EACH = AL + 2;      // a wave's loads a step
-  for (int j = 0; j < J; ++j) {
-    // step j has landed for this wave when at most the later steps' loads are on their way, and for all behind the barrier, which
-    // every wave reaches with its reads of step j - 1 done: that region is asked for again
-    const int later = min(2, J - 1 - j);
-    if (later == 2) XM_WAIT(2 * EACH);
-    else if (later == 1) XM_WAIT(EACH);
+  xm_u32x4_t af[2][XB], wf[2][4];      // the operands of an even and of an odd step
+  // the first two units and half of the third, and four steps of weights; what follows is asked for as places become free
+  for (int unit = 0; unit < 3 && unit < units; ++unit)
+#pragma unroll
+    for (int b = 0; b < AL; ++b) {
+      ask_rows(b, 0, unit, unit);
+      if (unit < 2) ask_rows(b, 1, unit, unit);
+    }
+  for (int j = 0; j < STEPS && j < steps; ++j) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) ask_weights(b, j);
+  }
+  XM_WAIT(0);
+  XM_MEET();
+  const int r = lane % 16, read_at = (r / 8) * 64 + (r % 8) * 8 + ((lane / 16) ^ (r % 8) ^ (r / 8));     // ^ 4 for a unit's second step
+#pragma unroll
+  for (int y = 0; y < 4; ++y) wf[0][y] = lds[W_RING + (4 * wn + y) * 64 + lane];
+#pragma unroll
+  for (int x = 0; x < XB; ++x) af[0][x] = lds[(XB * wm + x) * 128 + read_at];
+  int unit_place = 0;      // of the unit of the step that is multiplied
+  // Step j, its operands in registers or on their way there; it reads those of step j + 1.  STEADY: it asks for the weights of step
+  // j + 4, in the place of step j's, and for half a unit of rows: in an even step the second half of the unit two ahead of its own, in
+  // an odd step the first half of the unit three ahead, which takes its own unit's place (beyond the last unit that one again, which
+  // nobody reads).  Every wave waited for its reads of either place before the barrier here.  What step j + 1 needs was asked for in
+  // step j - 3 or before, so the loads of two steps may still be on their way.
+  auto multiply = [&](int j, auto odd, auto steady) {
+    constexpr int U = decltype(odd)::value;
+    constexpr bool STEADY = decltype(steady)::value;
+    if (STEADY) XM_WAIT(2 * EACH);
     else XM_WAIT(0);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (j + 3 < J) fetch(j + 3);
-    const int region = (j & (REGIONS - 1)) * CHUNKS;
-    xm_u32x4_t af[XB], wf[4];
+    XM_MEET();
+    const int after = unit_place == 2 ? 0 : unit_place + 1, ahead = unit_place == 0 ? 2 : unit_place - 1;
+    const int rows_at = (U == 0 ? unit_place : after) * XB * 256 + (U == 0 ? read_at ^ 4 : read_at);
+    constexpr int READS = XB + 4, MFMAS = XB * 4, GROUP = (MFMAS + READS - 1) / READS;
 #pragma unroll
-    for (int x = 0; x < XB; ++x) af[x] = lds[(region + XB * wm + x) * 64 + lane];
+    for (int g = 0; g < READS; ++g) {
+      // (beyond the last step this reads what an earlier one has left there, and nobody uses it)
+      if (g < 4) wf[1 - U][g] = lds[W_RING + (((j + 1) % STEPS) * 8 + 4 * wn + g) * 64 + lane];
+      else af[1 - U][g - 4] = lds[rows_at + (XB * wm + g - 4) * 128];
+      if (STEADY) {
 #pragma unroll
-    for (int y = 0; y < 4; ++y) wf[y] = lds[(region + 2 * XB + 4 * wn + y) * 64 + lane];
+        for (int i = 0; i < EACH; ++i)
+          if (i * READS / EACH == g) {
+            if (i < 2) ask_weights(i, j + STEPS);
+            else if (U == 0) ask_rows(i - 2, 1, j / 2 + 2, ahead);
+            else ask_rows(i - 2, 0, min(j / 2 + 3, units - 1), unit_place);
+          }
+      }
 #pragma unroll
-    for (int x = 0; x < XB; ++x)
-#pragma unroll
-      for (int y = 0; y < 4; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_operand(wf[y]), as_operand(af[x]), acc[x][y], 0, 0, 0);
+      for (int q = g * GROUP; q < (g + 1) * GROUP && q < MFMAS; ++q)
+        acc[q / 4][q % 4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_operand(wf[U][q % 4]), as_operand(af[U][q / 4]), acc[q / 4][q % 4], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (U == 1) unit_place = after;
+  };
+  const std::integral_constant<int, 0> even;
+  const std::integral_constant<int, 1> odd;
+  int j = 0;
+  for (; j + STEPS < steps; j += 2) {
+    multiply(j, even, std::true_type());
+    multiply(j + 1, odd, std::true_type());
+  }
+  for (; j < steps; j += 2) {
+    multiply(j, even, std::false_type());
+    multiply(j + 1, odd, std::false_type());
   }
 
   // acc[x][y][i]: pair 16 (XB wm + x) + lane % 16 of the tile, row 4 (lane / 16) + i of the wave's y-th block of weight rows
@@ -174,6 +231,7 @@ __global__ __launch_bounds__(256) void experts_many_kernel(const uint16_t* __res
   }
 }
 #undef XM_WAIT
+#undef XM_MEET
 
 template <bool GATED, int XB>
 int launch(const void* in, int in_div, const int32_t* list, int capacity, const int32_t* counts, const void* w, void* out, int pairs, int E,
@@ -199,9 +257,9 @@ extern "C" int bh_experts_many(const void* in, int in_div, const int32_t* list, 
   BH_REQUIRE(((uintptr_t)in | (uintptr_t)w | (uintptr_t)out) % 16 == 0, "experts_many: operands must be 16-byte aligned");
   BH_REQUIRE(gated || in_weights == nullptr, "experts_many: weights on the input go with the gated product");
   // Tiles of 128 pairs read the weights half as often as tiles of 64, which leave less of a last tile empty.  Gate and up,
-  // tiles of 64 / 128, us: width 2,048 at 48 pairs an expert 49 / 55, at 96 58 / 63, at 192 107 / 86; width 4,096 at 48 152 / 181,
-  // at 96 213 / 183, at 192 349 / 289.
-  const bool wide = (long)pairs >= 96L * E;
+  // tiles of 64 / 128, us: width 2,048 at 48 pairs an expert 48 / 52, at 64 58 / 52, at 96 64 / 55, at 128 68 / 73, at 192 87 / 76;
+  // width 4,096 at 48 155 / 162, at 64 182 / 160, at 96 198 / 166; width 1,024 at 48 15 / 18, at 64 18 / 18, at 96 17 / 18, at 192 26 / 24.
+  const bool wide = (long)pairs >= 56L * E;
 #define BH_XM(GATED, XB) launch<GATED, XB>(in, in_div, list, capacity, counts, w, out, pairs, E, K, N, limit, alpha, shift, in_weights, stream)
   if (gated) return wide ? BH_XM(true, 4) : BH_XM(true, 2);
   return wide ? BH_XM(false, 4) : BH_XM(false, 2);

@@ -84,11 +84,12 @@ class RoutedExperts:
     PRODUCT_PAIRS = 16        # from that many pairs an expert on average, a step of many rows runs matrix products
     PACK_FOR_PROMPTS = True   # keep a second copy of every expert's matrices in the form the products of many rows read fastest
     # A prompt's experts run as one launch over all of them up to so many pairs x hidden x ff an expert on average, beyond that as
-    # products one by one: the one launch reaches 0.37 to 0.55 PFLOP/s whatever the size, a product of its own costs the host's wait
+    # products one by one: the one launch reaches 0.5 to 0.9 PFLOP/s whatever the size, a product of its own costs the host's wait
     # for the counts, the gathered rows and about 25 us, and then reaches 0.8 to 1.0.  One launch / one by one, us, 8 experts: width
-    # 4,096, ff 1,536 at 2,048 pairs an expert 1,057 / 1,254, at 4,096 2,046 / 1,871; ff 4,096 at 1,024 1,320 / 1,384, at 2,048
-    # 2,470 / 2,245; ff 14,336 at 256 1,443 / 1,405, at 2,048 8,532 / 5,681; 4 to 128 experts cross at the same work.
-    ONE_LAUNCH_WORK = 1.8e10
+    # 4,096, ff 1,536 at 2,048 pairs an expert 913 / 1,170, at 4,096 1,925 / 1,975; ff 4,096 at 1,024 985 / 1,242, at 2,048
+    # 2,044 / 2,151; ff 14,336 at 256 1,121 / 1,387, at 1,024 3,282 / 3,233, at 2,048 6,746 / 5,803; 32 experts, ff 1,536 at 4,096
+    # 7,265 / 7,317; 4 experts, ff 1,536 at 8,192 2,097 / 2,012.
+    ONE_LAUNCH_WORK = 4e10
     WIDE_ROUTER = 128         # a router of fewer outputs is kept with that many for steps of more than WIDE_FROM_ROWS rows: products
     WIDE_FROM_ROWS = 32       # that cut K into parts need a whole tile of outputs (2,048 rows, 40 experts: 71 -> 22 us)
 

@@ -10,10 +10,12 @@ pytestmark = pytest.mark.gpu
 
 
 # pairs an expert: none, one, a tile's edges (64 and 128), several tiles; experts: one, more than a wave's lanes; outputs: less than
-# a tile's, remainders of one; the average decides between tiles of 64 pairs (below 96) and of 128
+# a tile's, remainders of one; the average decides between tiles of 64 pairs (below 56) and of 128; widths of 1 to 5, 7, 12 and 32 units
+# of 64 k, the ring of three units among them
 @pytest.mark.parametrize("counts,width,ff", [([1], 64, 64), ([64, 0, 65, 1], 128, 192), ([0, 63, 127, 0, 30], 192, 64), ([300], 64, 128),
                                              ([128, 129, 127, 257, 0], 256, 64), ([0] * 69 + [200, 3] + [0] * 5 + [40], 64, 64),
-                                             ([150] * 66, 64, 64), ([97, 512], 2048, 768)])
+                                             ([150] * 66, 64, 64), ([97, 512], 2048, 768),
+                                             ([130, 5], 320, 448), ([33, 70, 2], 448, 320)])
 @pytest.mark.parametrize("weighed", [False, True])
 def test_experts_of_many_pairs(K, counts, width, ff, weighed):
     g = torch.Generator().manual_seed(sum(counts) + width)
