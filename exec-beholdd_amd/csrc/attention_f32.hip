@@ -10,7 +10,7 @@
 // Bound by the pages' way from memory or the L2 (a page of a head of 128 is 64 KB): NR rows share it.
 // Measured (8 heads of 128 on 4): a decode step of 4 rows at 40 to 300 keys 8.2 us, 54 with a thread a key (generic.hip: every
 // lane its own line), 20 before a page's keys and values were asked for together; four prompts of 695 rows in all, up to 256 each,
-// 41 us in waves of their own, 94 in workgroups of four waves on four rows, 120 there.
+// 41 us in waves of their own (30 in tiles of columns, see there), 94 in workgroups of four waves on four rows, 120 there.
 #include "common.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -241,10 +241,197 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(F32Attention 
   }
 }
 
+// ---- prompts -------------------------------------------------------------------------------------------
+// Sixteen columns, (row, query head) pairs of one kv head in order, a workgroup, on the float32 matrix instructions (every product a
+// 32-bit fused multiply-add): a page's keys and values are read once for all of them.  Each of its four waves takes 16 of a page's
+// tokens, so that short prompts keep all four busy, and loads the next page's keys while it works on this one's.  With
+// v_mfma_f32_16x16x4_f32, whose operands are an element of 16 rows and four k a lane,
+//     S^T[key, column] = K[key, :] . Q[column, :]        O^T[d, column] += V^T[d, key] . P^T[key, column]
+// lane (i = lane % 16, g = lane / 16) loads 16 bytes of row i of an operand at 16 s + 4 g and gives its four elements to four
+// instructions in turn, which take k in that order on both sides.  A lane then holds the scores of column i and keys 4 g .. 4 g + 3
+// of the 16: the P^T operands of the second product as they are.  The columns may belong to several sequences, which are walked
+// one after another with the others' columns masked.  A page's sums are made apart and then added, as the walk above adds blocks.
+// Bound by a wave's chain of a page: its loads, 64 (heads of 128) matrix instructions of 32 clocks, and the softmax between them.
+// Measured: four prompts of 744 rows in all, 8 heads of 128 on 4: 30 us, 102 in waves of a row each, which read 8 times as much;
+// error against 64 bits 1.14e-7 there (1.20e-7 in the waves), 1.33e-7 for 1,000 rows of 8 heads of 256 (1.48e-7).
+template <int P>
+__global__ __launch_bounds__(256, P <= 4 ? 2 : 1) void attention_f32_tiles_kernel(F32Attention t, int n_rows) {
+  constexpr int HD = 32 * P, CHUNKS = 2 * P, STRIDE = HD + 4, WAVES = 4;
+  __shared__ float o[WAVES][16][STRIDE];
+  __shared__ float tops[WAVES][16], sums[WAVES][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int group = t.H / t.KVH, kv_head = blockIdx.y;
+  const long column = 16L * blockIdx.x + i;
+  const int row = (int)(column / group), head = kv_head * group + (int)(column % group);
+  const bool exists = row < n_rows;
+  const int seq = exists ? t.row_seq[row] : -1, pos = exists ? t.positions[row] : -1;
+  const int first = bh_first_visible(pos < 0 ? 0 : pos, t.window);
+  const float scale = query_scale(t.form, pos < 0 ? 0 : pos), slope = t.form.slopes && exists ? t.form.slopes[head] : 0.f;
+  floatx4 q[CHUNKS];
+#pragma unroll
+  for (int s = 0; s < CHUNKS; ++s)
+    q[s] = exists ? load4(t.q + ((size_t)row * t.H + head) * HD + 16 * s + 4 * g) : floatx4{0.f, 0.f, 0.f, 0.f};
+
+  float most = -INFINITY, sum = 0.f;
+  floatx4 acc[CHUNKS];
+#pragma unroll
+  for (int d = 0; d < CHUNKS; ++d) acc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+  unsigned long long left = __ballot(exists);      // the lanes whose columns are still to be walked
+  while (left) {
+    const int seq_now = __builtin_amdgcn_readfirstlane(__shfl(seq, __ffsll(left) - 1, BH_WAVE));
+    const bool mine = exists && seq == seq_now;
+    left &= ~__ballot(mine);
+    int from = mine ? first : 0x7fffffff, upto = mine ? pos : -1;
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+      from = min(from, __shfl_xor(from, off, BH_WAVE));
+      upto = max(upto, __shfl_xor(upto, off, BH_WAVE));
+    }
+    from = __builtin_amdgcn_readfirstlane(from);
+    upto = __builtin_amdgcn_readfirstlane(upto);
+    const int32_t* table = t.page_table + (size_t)seq_now * t.table_stride;
+    // the wave's pages: those in which some column sees one of its 16 tokens
+    const int tokens = 16 * wave;
+    int page = (from - tokens - 15 + BH_PAGE - 1) / BH_PAGE;
+    if (from < tokens + 15) page = 0;
+    const int last = upto < tokens ? -1 : (upto - tokens) / BH_PAGE;
+    floatx4 k[CHUNKS];
+    auto load_keys = [&](int of) {
+      const float* keys = t.k_pages + (((size_t)table[of] * t.KVH + kv_head) * BH_PAGE + tokens + i) * HD + 4 * g;
+#pragma unroll
+      for (int s = 0; s < CHUNKS; ++s) k[s] = load4(keys + 16 * s);
+    };
+    if (page <= last) load_keys(page);
+    for (; page <= last; ++page) {
+      const size_t block = ((size_t)table[page] * t.KVH + kv_head) * BH_PAGE * HD;
+      const float* values = t.v_pages + block + i * BH_PAGE + tokens + 4 * g;
+      floatx4 v[CHUNKS];
+#pragma unroll
+      for (int d = 0; d < CHUNKS; ++d) v[d] = load4(values + 16 * d * BH_PAGE);
+      // eight chains of half of k, then eight of the other half: no chain is longer than those of the walk above
+      floatx4 p = {0.f, 0.f, 0.f, 0.f};
+      constexpr int MIDDLE = (P + 1) / 2 * 2;
+#pragma unroll
+      for (int from_s = 0; from_s < CHUNKS; from_s += MIDDLE) {
+        floatx4 chain[8] = {};
+#pragma unroll
+        for (int s = from_s; s < from_s + MIDDLE && s < CHUNKS; s += 2)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              chain[2 * e + h] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s + h][e], q[s + h][e], chain[2 * e + h], 0, 0, 0);
+        p += ((chain[0] + chain[1]) + (chain[2] + chain[3])) + ((chain[4] + chain[5]) + (chain[6] + chain[7]));
+      }
+      if (page < last) load_keys(page + 1);
+      float top = -INFINITY;
+      bool whole = mine;
+      const int at = page * BH_PAGE + tokens + 4 * g;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float score = p[e] * scale;
+        if (t.form.cap > 0.f) score = t.form.cap * tanhf(score / t.form.cap);
+        score -= slope * (float)(pos - at - e);
+        const bool seen = mine && at + e >= first && at + e <= pos;
+        whole = whole && seen;
+        p[e] = seen ? score : -INFINITY;
+        top = fmaxf(top, p[e]);
+      }
+      top = fmaxf(top, __shfl_xor(top, 16, BH_WAVE));
+      top = fmaxf(top, __shfl_xor(top, 32, BH_WAVE));
+      const float now = fmaxf(most, top);
+      const float alpha = most == -INFINITY ? 0.f : expf(most - now);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[e] = p[e] == -INFINITY ? 0.f : expf(p[e] - now);
+      sum = sum * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+      most = now;
+      // A key that a column does not see may hold anything (behind a sequence's end, or a later row's): it must not reach that
+      // column's sums, not even times zero.  Where a column does not see all of the tokens, numbers that are not finite are set aside
+      // and then given to those who see them, one by one.
+      bool odd_ones = false;
+      if (!__all(whole)) {
+#pragma unroll
+        for (int d = 0; d < CHUNKS; ++d)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const bool finite = fabsf(v[d][e]) < INFINITY;
+            odd_ones = odd_ones || !finite;
+            v[d][e] = finite ? v[d][e] : 0.f;
+          }
+      }
+#pragma unroll
+      for (int d = 0; d < CHUNKS; d += 2) {
+        floatx4 part[2][2] = {};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) part[h][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[d + h][e], p[e], part[h][e & 1], 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[d + h][e] = fmaf(acc[d + h][e], alpha, part[h][0][e] + part[h][1][e]);
+      }
+      if (__any(odd_ones)) {
+        for (int token = 0; token < 16; ++token) {
+          const int e = token & 3, place = page * BH_PAGE + tokens + token;
+          const float w = __shfl(e == 0 ? p[0] : e == 1 ? p[1] : e == 2 ? p[2] : p[3], i + 16 * (token >> 2), BH_WAVE);
+          if (mine && place >= first && place <= pos) {
+#pragma unroll
+            for (int d = 0; d < CHUNKS; ++d)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const float one = t.v_pages[block + (size_t)(16 * d + 4 * g + r) * BH_PAGE + tokens + token];
+                if (!(fabsf(one) < INFINITY)) acc[d][r] = fmaf(w, one, acc[d][r]);
+              }
+          }
+        }
+      }
+    }
+  }
+
+  sum += __shfl_xor(sum, 16, BH_WAVE);
+  sum += __shfl_xor(sum, 32, BH_WAVE);
+#pragma unroll
+  for (int d = 0; d < CHUNKS; ++d) *reinterpret_cast<floatx4*>(&o[wave][i][16 * d + 4 * g]) = acc[d];
+  if (g == 0) {
+    tops[wave][i] = most;
+    sums[wave][i] = sum;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 16 * HD; e += 64 * WAVES) {
+    const int c = e / HD, d = e % HD;
+    const long of = 16L * blockIdx.x + c;
+    const int to_row = (int)(of / group), to_head = kv_head * group + (int)(of % group);
+    if (to_row >= n_rows) break;      // so are all that follow
+    float top = tops[0][c];
+#pragma unroll
+    for (int s = 1; s < WAVES; ++s) top = fmaxf(top, tops[s][c]);
+    float total = 0.f, all = 0.f;
+#pragma unroll
+    for (int s = 0; s < WAVES; ++s) {
+      const float share = tops[s][c] == -INFINITY ? 0.f : expf(tops[s][c] - top);
+      all += sums[s][c] * share;
+      total += o[s][c][d] * share;
+    }
+    if (t.finish.sinks) all += expf(t.finish.sinks[to_head] - top);
+    t.out[((size_t)to_row * t.H + to_head) * HD + d] = total / all * head_gate<float>(t.finish, to_row, to_head);
+  }
+}
+
 template <int P>
 void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, hipStream_t stream) {
   constexpr int NR = P <= 4 ? 4 : P <= 7 ? 2 : 1;      // what the registers hold without spilling
   const bool prompts = n_rows >= 8 * n_seqs;
+  // Columns in tiles where (rows, heads) are more than the waves of two a SIMD, so that a wave a row would come in rounds, and the step
+  // is prompts: a tile walks its sequences one after another.  As below / in tiles, us: 300, 186, 200 and 58 rows of 8 heads of 128 on 4
+  // 102 / 30, on 16 heads 198 / 40, 16 prompts of 40 rows of 16 heads 52 / 23, one of 256 40 / 18, of 2,048 of 8 heads 724 / 216, of
+  // 1,000 of 8 heads of 256 on 1 400 / 129; but 4 prompts of 64 of 8 heads of 256 17 / 19, one of 33 of 16 heads 6.8 / 10.2, and one of
+  // 512 beside 63 sequences that bring a row behind 1,000 keys 170 / 404.
+  if (n_rows >= 32 * n_seqs && (long)n_rows * t.H > 8L * bh_compute_units() && t.KVH <= 65535) {
+    const long tiles = ((long)n_rows * (t.H / t.KVH) + 15) / 16;
+    attention_f32_tiles_kernel<P><<<dim3((unsigned)tiles, t.KVH), 256, 0, stream>>>(t, n_rows);
+    return;
+  }
   // Rows that see one page have work for one wave a row and head, and rows that see a few have it where they and the heads fill the
   // chip: waves of their own leave no wave without a page.  Four waves on four rows / a wave a row, us, 16 heads of 128 on 8: one
   // prompt of 33 rows 15.9 / 6.8, 16 of 40 172 / 52, one of 256 61 / 40; 8 heads of 256 on 2: 4 prompts of 64 47 / 17, but 30 rows

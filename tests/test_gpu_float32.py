@@ -155,3 +155,68 @@ def test_float32_attention_of_few_pages(K, n_heads, kv_heads, head_dim, pasts, n
         rows = row_seq == s
         want = attention_reference_rows(q[rows], keys[s], values[s], positions[rows].long(), n_heads, kv_heads, head_dim, head_dim ** -0.5, 0)
         assert float((got[rows] - want).abs().max() / want.abs().max()) < 1e-5, s      # as in test_float32_attention_rows_of_a_step
+
+
+# tiles of 16 columns: groups of 1, 3, 8 and 24 heads (columns of a row in two tiles), ends of sequences inside a tile, single rows
+# between prompts, the last tile's columns that do not exist; the wave's 16 tokens before, at and behind a page's, window's or chunk's end
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim", [(16, 16, 32), (9, 3, 64), (16, 2, 128), (24, 1, 96), (8, 2, 256)])
+@pytest.mark.parametrize("window,chunk", [(0, 0), (17, 0), (130, 0), (0, 48)])
+def test_float32_attention_of_prompts_in_tiles(K, n_heads, kv_heads, head_dim, window, chunk):
+    """Many columns of prompts; what a row does not see stays out although its neighbours in the tile see it: an infinite value of a
+    later row's, NaN behind a sequence's end."""
+    pasts, news = [0, 15, 0, 64, 130], [16, 1, 190, 3, 77]
+    lengths = [p + n for p, n in zip(pasts, news)]
+    kp, vp, table, keys, values = make_cache(len(lengths), lengths, kv_heads, head_dim, torch.float32, seed=head_dim + window)
+    for s, n in enumerate(lengths):
+        if n % 64:
+            kp[int(table[s, (n - 1) // 64]), :, n % 64:, :] = float("nan")
+            vp[int(table[s, (n - 1) // 64]), :, :, n % 64:] = float("nan")
+    far, dim = 100, head_dim - 3       # the third sequence's row 100 holds an infinite value
+    vp[int(table[2, far // 64]), :, dim, far % 64] = values[2][far][:, dim] = float("inf")
+    positions = torch.tensor([p + t for p, n in zip(pasts, news) for t in range(n)], dtype=torch.int32)
+    row_seq = torch.tensor([s for s, n in enumerate(news) for _ in range(n)], dtype=torch.int32)
+    q = torch.randn(len(positions), n_heads * head_dim, generator=torch.Generator().manual_seed(1))
+    out = torch.full(q.shape, float("nan"), device="cuda:0")
+    starts = torch.tensor([0] + [sum(news[:i + 1]) for i in range(len(news))], dtype=torch.int32)
+    layout = Layout(False, dev(starts), len(news), max(news), max(lengths) - 1)
+    assert len(positions) >= 32 * len(news) and len(positions) * n_heads > 2048
+    K.attention(dev(q), out, dev(kp), dev(vp), dev(table), dev(row_seq), dev(positions), n_heads, kv_heads, head_dim, head_dim ** -0.5, window,
+                layout=layout, chunk=chunk)
+    got = out.cpu().double().reshape(len(positions), n_heads, head_dim)
+    finite = [v.clone() for v in values]
+    finite[2][far][:, dim] = 0.0
+    for s in range(len(news)):
+        rows = (row_seq == s).nonzero()[:, 0]
+        at = positions[rows].long()
+        first = at // chunk * chunk if chunk else (at - window + 1 if window else at * 0)
+        for part in ([rows] if not chunk else [rows[at // chunk == c] for c in sorted(set((at // chunk).tolist()))]):
+            lead = int(positions[part[0]]) // chunk * chunk if chunk else 0
+            want = attention_reference_rows(q[part], keys[s][lead:], finite[s][lead:], positions[part].long() - lead,
+                                            n_heads, kv_heads, head_dim, head_dim ** -0.5, window).reshape(len(part), n_heads, head_dim)
+            mine = got[part].clone()
+            if s == 2:
+                sees = ((positions[part].long() >= far) & (first[torch.isin(rows, part)] <= far))
+                assert bool((mine[sees][:, :, dim] == float("inf")).all())
+                mine[sees, :, dim], want[sees, :, dim] = 0.0, 0.0
+            # as in test_float32_attention_rows_of_a_step
+            assert float((mine - want).abs().max() / want.abs().max()) < 1e-5, s
+
+
+def test_float32_attention_of_prompts_in_tiles_score_forms_and_ends(K):
+    """Cap, slopes, temperature, sinks, gates and a factor, as the kernel for every size gives them."""
+    n_heads, kv_heads, length = 12, 4, 200
+    kp, vp, table, _, _ = make_cache(1, [length], kv_heads, 64, torch.float32, seed=5)
+    kp[..., 40:], vp[:, :, 40:] = 0.0, 0.0
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn(length, n_heads, 64, generator=g)
+    q[..., 40:] = 0.0
+    more = dict(sinks=dev(torch.randn(n_heads, generator=g)), gates=dev(torch.randn(length, n_heads, generator=g)), softcap=3.0,
+                slopes=dev(torch.rand(n_heads, generator=g)), q_temp=(0.5, 16), out_scale=0.7)
+    outs = []
+    for size in (64, 40):
+        out = torch.empty(length, n_heads * size, device="cuda:0")
+        K.attention(dev(q[..., :size].reshape(length, -1).contiguous()), out, dev(kp[..., :size].contiguous()), dev(vp[:, :, :size].contiguous()),
+                    dev(table), dev(torch.zeros(length, dtype=torch.int32)), dev(torch.arange(length, dtype=torch.int32)), n_heads, kv_heads,
+                    size, 0.2, **more)
+        outs.append(out.reshape(length, n_heads, size)[..., :40].double())
+    assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 1e-5
