@@ -2,10 +2,22 @@
 // form out[M, F] = act(A W[:F]^T) * (A W[F:]^T).  Every product is a 32-bit fused multiply-add with a 32-bit sum, as in the plain FMA
 // kernel (generic.hip); only the order of the sums differs, and it is blocked here as there.
 //
-// Two kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`, gated or not.  More rows are
-// matrix-core work: `gemm_f32_tiles`, whose gated products are followed by an activation of their own.
+// Three kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`, gated or not.  More rows are
+// matrix-core work: `gemm_f32_ring` where K is a multiple of 32, else `gemm_f32_tiles`; gated products are followed by an activation of
+// their own.
 #include "common.h"
 #include "gemm_f32.h"
+#include <type_traits>
+
+// s_waitcnt of gfx9 (vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8): all LDS reads are back, and at most `vm` of the wave's
+// global loads are still on their way.  F32_MEET: every wave has waited; nothing may be moved across it by the compiler.
+#define F32_WAIT(vm) __builtin_amdgcn_s_waitcnt(((vm) & 15) | (((vm) >> 4) << 14) | (7 << 4) | (0 << 8))
+#define F32_MEET()                        \
+  do {                                    \
+    __builtin_amdgcn_sched_barrier(0);    \
+    __builtin_amdgcn_s_barrier();         \
+    __builtin_amdgcn_sched_barrier(0);    \
+  } while (0)
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -108,7 +120,126 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_few_kernel(const float* _
   }
 }
 
-// ---- many rows -----------------------------------------------------------------------------------------
+// ---- many rows, K a multiple of 32 ---------------------------------------------------------------------
+// A workgroup of four waves owns 32 WM x 32 WN outputs, a wave 32 x 32 of them for one of KG shares of k (WM WN KG = 4): the fewer the
+// outputs, the more of the waves share k, so that few rows fill the chip too.  Slices of 32 k go from global memory straight to LDS
+// (1 KB a load: eight whole rows of a slice) into a ring of R, R steps ahead; a step's operands are read from LDS into registers while
+// the step before is multiplied.  The 16-byte piece c of row r of a slice lies at place c ^ (r % 8) of the row's eight, so that the
+// eight rows that a read takes at a time lie in different banks.  A slice is summed on its own and then added, as below, the even and
+// the odd ones apart: error against 64 bits of 744 rows of 6,144 x 1,024 1.31e-7 (below 1.48e-7), of 1,024 x 3,072 1.67e-7 on both.
+// Bound by the matrix instructions (64 cycles an instruction, 16 a slice and wave), the last round of workgroups, and their start.
+template <int WM, int WN, int KG, int R, bool ACCUMULATE>
+__global__ __launch_bounds__(256, KG == 4 ? 1 : 2) void gemm_f32_ring_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                             float* __restrict__ c, int M, int N, int K) {
+  static_assert(WM * WN * KG == 4 && R >= 3, "four waves; a step's loads, the next one's and one more");
+  constexpr int WAVES = WM * WN, A_PIECES = 4 * WM, PIECES = 4 * (WM + WN), EACH = PIECES / WAVES;
+  // one array: before a read from one of several the compiler waits for all loads on their way to that one
+  __shared__ __attribute__((aligned(16))) floatx4 ring[KG * R * PIECES * 64];      // [share][step in turn][8 rows of A, then of W][lane]
+  const int lane = threadIdx.x & 63, wave_of_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_of_all % WAVES, share = wave_of_all / WAVES, wm = wave / WN, wn = wave % WN;
+  const int m0 = blockIdx.y * 32 * WM, n0 = blockIdx.x * 32 * WN, steps = K / 32 / KG;
+  const float* from[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int piece = wave * EACH + i, row = 8 * (piece < A_PIECES ? piece : piece - A_PIECES) + lane / 8;      // rows beyond the last one repeat it
+    from[i] = (piece < A_PIECES ? a + (size_t)min(m0 + row, M - 1) * K : w + (size_t)min(n0 + row, N - 1) * K) + 32 * share +
+              4 * ((lane & 7) ^ (lane / 8));
+  }
+  auto ask = [&](int i, int step, int place) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from[i] + (size_t)step * (32 * KG)),
+                                     (__attribute__((address_space(3))) void*)&ring[((share * R + place) * PIECES + wave * EACH + i) * 64], 16, 0, 0);
+  };
+  const int half = lane >> 5, row = lane & 31;
+  int at[4];      // the lane's pieces of its row, one for every 8 k
+#pragma unroll
+  for (int t = 0; t < 4; ++t) at[t] = (row / 8) * 64 + (row & 7) * 8 + ((2 * t + half) ^ (row & 7));
+  for (int j = 0; j < R && j < steps; ++j) {
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) ask(i, j, j);
+  }
+  F32_WAIT(0);
+  F32_MEET();
+  floatx4 av[2][4], wv[2][4];      // the operands of an even and of an odd step
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    av[0][t] = ring[(share * R * PIECES + 4 * wm) * 64 + at[t]];
+    wv[0][t] = ring[(share * R * PIECES + A_PIECES + 4 * wn) * 64 + at[t]];
+  }
+  // the sums of even and of odd steps, added at the end; a step's own sum is added while the next step's is made
+  floatx16 sum[2] = {}, part[2] = {};
+  int place = 0;                         // of the step that is multiplied
+  // Step j: its operands are in registers or on their way there, and every wave has waited for its reads of them before the barrier, so
+  // step j + R may take their place.  STEADY: it does, and what step j + 1 needs was asked for before the loads of the R - 2 steps
+  // behind it; otherwise (the last R steps) everything asked for is waited for.
+  auto multiply = [&](int j, auto odd, auto steady) {
+    constexpr int U = decltype(odd)::value;
+    constexpr bool STEADY = decltype(steady)::value;
+    if (STEADY) F32_WAIT(EACH * (R - 2));
+    else F32_WAIT(0);
+    F32_MEET();
+    const int next = place == R - 1 ? 0 : place + 1, base = (share * R + next) * PIECES;
+    if (!STEADY && j + R < steps) {
+#pragma unroll
+      for (int i = 0; i < EACH; ++i) ask(i, j + R, place);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      // (beyond the last step this reads what an earlier one has left there, and nobody uses it)
+      av[1 - U][t] = ring[(base + 4 * wm) * 64 + at[t]];
+      wv[1 - U][t] = ring[(base + A_PIECES + 4 * wn) * 64 + at[t]];
+      if (STEADY) {
+#pragma unroll
+        for (int i = 0; i < EACH; ++i)
+          if (i * 4 / EACH == t) ask(i, j + R, place);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        part[U] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[U][t][e], wv[U][t][e], t + e == 0 ? floatx16{} : part[U], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[1 - U][4 * t + e] += part[1 - U][4 * t + e];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    place = next;
+  };
+  const std::integral_constant<int, 0> even;
+  const std::integral_constant<int, 1> odd;
+  int j = 0;
+  for (; j + 1 + R < steps; j += 2) {
+    multiply(j, even, std::true_type());
+    multiply(j + 1, odd, std::true_type());
+  }
+  for (; j + 1 < steps; j += 2) {
+    multiply(j, even, std::false_type());
+    multiply(j + 1, odd, std::false_type());
+  }
+  if (j < steps) multiply(j, even, std::false_type());
+  if (steps % 2) sum[0] += part[0];
+  else sum[1] += part[1];
+  floatx16 acc = sum[0] + sum[1];
+  if constexpr (KG > 1) {      // the shares' sums, lane by lane
+    F32_WAIT(0);
+    F32_MEET();
+    floatx16* sums = reinterpret_cast<floatx16*>(ring) + wave * 64 + lane;
+    if (share > 0) sums[(share - 1) * WAVES * 64] = acc;
+    __syncthreads();
+    if (share > 0) return;
+#pragma unroll
+    for (int s = 0; s < KG - 1; ++s) acc += sums[s * WAVES * 64];
+  }
+  const int n = n0 + 32 * wn + row;
+  if (n >= N) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int m = m0 + 32 * wm + 8 * (r >> 2) + 4 * half + (r & 3);
+    if (m >= M) continue;
+    const size_t to = (size_t)m * N + n;
+    c[to] = ACCUMULATE ? acc[r] + c[to] : acc[r];
+  }
+}
+#undef F32_WAIT
+#undef F32_MEET
+
+// ---- many rows, any K ----------------------------------------------------------------------------------
 // Four waves own 64 B x 64 B outputs (B = 1 or 2), a wave B x B tiles of v_mfma_f32_32x32x2_f32; a workgroup is one such group, or
 // KG of them that take the slices of k in turn (B = 1).  Slices of 32 k go through two LDS buffers, the next slice's loads on their way while one is multiplied.  A row of a slice takes 36 floats of
 // LDS, so that the 16-byte reads of 16 neighbouring rows fall on different banks; lane (row, half) reads four k at once and the
@@ -251,6 +382,33 @@ int bh_gemm_f32(const float* a, const float* w, float* c, int accumulate, int M,
     else few_rows<1, false>(a, w, c, M, N, K, accumulate, none, stream);
     return bh_check_launch("gemm_f32_few");
   }
+  if (K % 32 == 0 && (M + 31) / 32 <= 65535) {
+    // The waves' split with the least estimated time: rounds of workgroups, one a compute unit at a time (two share it and take as long),
+    // of so many slices at what a slice takes, and the start; a smaller tile has to be 5 % ahead, for it reads more.  64 x 64 / 32 x 64 /
+    // 32 x 32 outputs, us, weights from memory (1 to 3 % less than now, before the sums of even and odd steps were kept apart), in
+    // brackets the tiles of gemm_f32_tiles: 744 rows of 6,144 x 1,024 104 / 106 / 173 (120), of 2,048 x 1,024 42 / 38 / 55 (49), of
+    // 1,024 x 3,072 66 / 67 / 72 (75); 1,500 of 1,024 x 3,072 112 / 97 / 139 (132); 300 of 1,024 x 3,072 63 / 38 / 48 (74); 100 of it
+    // 60 / 35 / 22 (71); 64 of 3,000 x 1,024 22 / 14 / 11 (26); 3,200 of 6,144 x 1,024 334 / 373 / 629 (392); 2,048 of 4,096 x 4,096
+    // 563 / 608 / 803 (620), 122 TFLOP/s.
+    const auto rounds = [&](int rows, int columns) {
+      return (double)(((long)((M + rows - 1) / rows) * ((N + columns - 1) / columns) + units - 1) / units);
+    };
+    const double whole = rounds(64, 64) * (K / 32) * 0.58 + 4.0;
+    const double in_two = K % 64 ? 1e30 : rounds(32, 64) * (K / 64) * 0.64 + 4.0;
+    const double in_four = K % 128 ? 1e30 : rounds(32, 32) * ((K / 128) * 0.75 + 4.0);
+#define BH_F32_RING(WM, WN, KG, R)                                                                                                 \
+  do {                                                                                                                             \
+    const dim3 grid((N + 32 * WN - 1) / (32 * WN), (M + 32 * WM - 1) / (32 * WM));                                                 \
+    if (accumulate) gemm_f32_ring_kernel<WM, WN, KG, R, true><<<grid, 256, 0, stream>>>(a, w, c, M, N, K);                         \
+    else gemm_f32_ring_kernel<WM, WN, KG, R, false><<<grid, 256, 0, stream>>>(a, w, c, M, N, K);                                   \
+    return bh_check_launch("gemm_f32_ring");                                                                                       \
+  } while (0)
+    if (in_four < 0.95 * in_two && in_four < 0.95 * whole) BH_F32_RING(1, 1, 4, 4);      // rings of 128, 72 and 48 KB
+    if (in_two < 0.95 * whole) BH_F32_RING(1, 2, 2, 3);
+    BH_F32_RING(2, 2, 1, 3);
+#undef BH_F32_RING
+  }
+  // Other K.
   // Tiles of 128 x 128 read half as much a product, but only four of them a compute unit and more level out (695 x 6,144 x 1,024,
   // 1.1 a unit: 141 us, 104 in tiles of 64 x 64); where tiles of 64 x 64 are not even two a unit, a second group of waves hides the
   // first one's waits for its slices.

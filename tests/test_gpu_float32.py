@@ -33,6 +33,23 @@ def test_float32_products(K, m, n, k):
     assert bool(((summed.cpu().double() - want - c).abs() <= product_bound(a, w, k) + 2.0 ** -24 * (want.abs() + c.abs() + 1)).all())
 
 
+# slices of 32 k: one to nine for waves that own 64 x 64 outputs, the same for two (K a multiple of 64) and four (of 128) shares of k, in
+# fewer and more steps than a ring holds; tiles' remainders; more tiles than compute units
+@pytest.mark.parametrize("m,n,k", [(33, 70, 32), (70, 33, 96), (100, 100, 160), (64, 64, 224), (65, 129, 288), (33, 65, 64), (40, 100, 192),
+                                   (70, 70, 320), (90, 64, 448), (33, 33, 128), (50, 40, 256), (64, 100, 384), (33, 95, 640), (40, 40, 1152),
+                                   (744, 2048, 1024), (2049, 1025, 96), (1100, 2100, 64)])
+def test_float32_products_in_a_ring_of_slices(K, m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w, c = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g), torch.randn(m, n, generator=g)
+    want = a.double() @ w.double().T
+    out = torch.full((m, n), float("nan"), device="cuda:0")
+    K.gemm(dev(a), dev(w), out)
+    assert bool(((out.cpu().double() - want).abs() <= product_bound(a, w, k)).all())
+    summed = dev(c)
+    K.gemm(dev(a), dev(w), summed, accumulate=True)
+    assert bool(((summed.cpu().double() - want - c).abs() <= product_bound(a, w, k) + 2.0 ** -24 * (want.abs() + c.abs() + 1)).all())
+
+
 @pytest.mark.parametrize("gate", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("m,width,k", [(1, 3, 8), (4, 96, 128), (7, 4097, 68), (20, 40, 2304), (32, 8, 60), (33, 72, 64)])
 def test_float32_gated_products(K, m, width, k, gate):
