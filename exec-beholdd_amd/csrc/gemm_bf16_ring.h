@@ -15,7 +15,8 @@ RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output);
 // one part where neither.
 RingPlan gemm_ring_bare_plan(int M, int N, int K, int layout);
 // The activations lie in blocks of 16 rows x 32 columns (bh_blocked_index).  c_dtype BH_F32 (accumulate allowed) or BH_BF16 (no
-// accumulate); activation 1 = gated, bfloat16 output only, in blocks of 16 rows if c_blocked; form: what stands on its gate.
+// accumulate); activation 1 = gated, bfloat16 output only; form: what stands on its gate, or that a plain product squares its bfloat16
+// output behind a ReLU; c_blocked: the output of either in blocks of 16 rows.
 int gemm_ring_launch(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K, int activation, int tile,
                      int c_blocked, GateForm form, hipStream_t stream);
 int gemm_ring_launch_parts(const void* a, const void* w, float* sums, int M, int N, int K, const RingPlan& plan, hipStream_t stream);

@@ -173,6 +173,8 @@ class KernelSizes:
             "bh_streams_update_rmsnorm": [p, p, p, p, p, p, p, p, i, i, i, i, f, i, p],
             "bh_scale": [p, ctypes.c_long, f, p],
             "bh_relu_squared": [p, p, i, i, i, i, p],
+            "bh_gemm_bf16_squared": [p, p, p, i, i, i, i, i, p],
+            "bh_gemm_bf16_squares": [i, i, i],
             "bh_lightning_scan": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
             "bh_lightning_chunks": [i, i, i, i, i, p],
             "bh_lightning_products": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
@@ -359,6 +361,7 @@ class HipKernels(KernelSizes):
         self.device = torch.device("cuda", self._device_index)
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         self._plans: dict = {}      # (m, n, k, packed, activation) -> what the library says of such a product
+        self._squares: dict = {}    # (m, n, k) -> which product squares its output (`gemm_relu_squared`), or 0
         self._bare: dict = {}       # (m, n, k) -> the parts that `gemm_bare` leaves such a product in, or 0
         self.page_size = int(self.lib.bh_page_size())
         if self.page_size != _build.source_page_size():
@@ -608,6 +611,27 @@ class HipKernels(KernelSizes):
             self._ptr(a, "gemm a"), _code(a, "gemm a"), self._ptr(w, "gemm w"), _code(w, "gemm w"),
             self._ptr(out, "gemm out"), _code(out, "gemm out"), int(bool(accumulate)), m, n, k, self._stream()))
         return None
+
+    def gemm_relu_squared(self, a, w, out) -> bool:
+        """out[M, N] = max(a[M, K] @ w[N, K]^T, 0)^2 in one launch, where the library has a product of these operands that does
+        so; False where it has not (then call `gemm` and `relu_squared`)."""
+        if (not isinstance(w, PackedWeight) or isinstance(a, NormedRows) or a.dim() != 2 or a.dtype != torch.bfloat16
+                or out.dtype != torch.bfloat16 or a.shape[1] != w.shape[1]):
+            return False
+        m, k = a.shape
+        n = w.shape[0]
+        if tuple(out.shape) != (m, n):
+            raise KernelError(f"gemm_relu_squared: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
+        squares = self._squares.get((m, n, k))
+        if squares is None:
+            squares = self._squares[(m, n, k)] = int(self.lib.bh_gemm_bf16_squares(m, n, k))
+        if not squares or _block_rows(out) not in ((0, 16) if squares == 1 else (0, 8, 16)):
+            return False
+        a_block_rows = self._product(m, n, k, 1, 0)[0]
+        a = self._in_blocks_of(a, a_block_rows)
+        self._check(self.lib.bh_gemm_bf16_squared(self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), m, n, k,
+                                                  a_block_rows, _block_rows(out), self._stream()))
+        return True
 
     def gemm_bare(self, a, w):
         """a[M, K] @ w[N, K]^T left as `PartSums`, where the product of these operands is one of many rows whose K the

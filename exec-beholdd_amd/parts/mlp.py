@@ -107,9 +107,10 @@ class SquaredReLU:
                 + self.down.working_bytes(step, step.rows, accumulate=True))
 
     def forward(self, ctx, x, hidden, fresh=False):
-        inner = self.up.forward(ctx, x)
-        activated = ctx.new_activations(inner.shape[0], self.inner, reader=self.down.reader())      # as the down product reads it
-        ctx.kernels.relu_squared(inner, activated)
+        activated = ctx.new_activations(x.shape[0], self.inner, reader=self.down.reader())      # as the down product reads it
+        in_one = getattr(ctx.kernels, "gemm_relu_squared", None)
+        if in_one is None or not in_one(x, self.up.weight, activated):
+            ctx.kernels.relu_squared(self.up.forward(ctx, x), activated)
         self.down.forward(ctx, activated, out=hidden, accumulate=not fresh)
 
 

@@ -75,3 +75,28 @@ def test_products_of_many_rows_and_the_norm_behind_them(K, m, n, k):
     got = residual.double()
     want = got / torch.sqrt((got ** 2).mean(-1, keepdim=True) + 1e-5) * weight.double()
     assert rel(K.from_blocked(normed) if isinstance(normed, BlockedRows) else normed, want.cpu()) < 4e-3
+
+
+# few rows (blocks of 8 and of 16, one and two blocks of rows), 33 to 128 rows and spans of 24 weight rows (two launches), many rows on
+# every kind of tile, K in parts (two launches); rows and columns that no tile divides
+@pytest.mark.parametrize("m,n,k", [(1, 96, 128), (8, 544, 192), (9, 4096, 256), (16, 160, 64), (17, 96, 1088), (32, 12288, 128), (16, 6144, 128),
+                                   (40, 512, 256), (129, 1056, 1024), (257, 1600, 1088), (300, 17408, 256), (1000, 4128, 2048),
+                                   (2100, 6144, 256), (4100, 8224, 128), (256, 2048, 4096)])
+def test_products_squared_behind_a_relu(K, m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) / k ** 0.5).bfloat16()
+    packed, a_rows = K.pack_weight(w.cuda()), a.cuda()
+    exact = (a_rows.double() @ w.cuda().double().T).clamp(min=0.0)
+    # float32 sums of k products, squared; the result rounded to 8 bits
+    error = 2.0 ** -23 * k ** 0.5 * 4.0
+    bound = 2.0 ** -8 * exact ** 2 + 2 * exact * error + error ** 2 + 1e-30
+    for block_rows in (0, 8, 16):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda:0") if not block_rows else K.to_blocked(
+            torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda:0"), block_rows=block_rows)
+        taken = K.gemm_relu_squared(a_rows, packed, out)
+        kind = int(K.lib.bh_gemm_bf16_squares(m, n, k))
+        assert taken == (kind == 2 or (kind == 1 and block_rows != 8))
+        assert kind == (0 if (m, n) in ((16, 6144), (40, 512), (129, 1056), (256, 2048)) else 2 if m <= 32 else 1)
+        if taken:
+            got = (K.from_blocked(out) if block_rows else out).double()
+            assert bool(((got - exact ** 2).abs() <= bound).all()), block_rows
