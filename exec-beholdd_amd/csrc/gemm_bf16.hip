@@ -1323,6 +1323,9 @@ extern "C" int bh_gemm_bf16_norm_blocks(int M, int N, int K, int layout, int act
 extern "C" int bh_gemm_bf16_takes_norm(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K % 8 != 0 || (activation && N % 16 != 0)) return 0;
   if (M <= 64) return 1;
+  // The kernel for many rows does not scale its sums: of its products those take prepared rows whose finishing kernel does.
+  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0)
+    return !activation && (gemm_ring_plan(M, N, K, layout, RING_F32).parts > 1 || gemm_ring_plan(M, N, K, layout, RING_BF16).parts > 1) ? 1 : 0;
   int rows, columns;
   tiled_config(M, N, activation != 0, &rows, &columns);
   return tiled_whole(M, N, K, layout, rows, columns) ? 1 : 0;
@@ -1419,7 +1422,16 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
   }();
   // 33 to 128 rows from blocks of 16: the kernel whose waves share the activations through LDS, then the finishing kernel
   const bool slices = scratch != nullptr && a_block_rows == 16 && !skinny && gemm_slices_takes(M, N, K, layout, activation);
-  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0)),
+  // Many rows.  What that kernel does not finish itself, rows of a norm ahead or adding into bfloat16, takes a plan with parts if there
+  // is one; what is left of that comes in rows, to the tiles.
+  RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32));
+  const bool ring_finishes = !ahead_ss && !behind_weight && (f32 || !accumulate);
+  if (ring.parts == 1 && !activation && !ring_finishes)
+    if (const RingPlan other = gemm_ring_plan(M, N, K, layout, ring_output(0, !f32)); other.parts > 1) ring = other;
+  const bool ring_whole = a_block_rows == 16 && ring.tile >= 0 && ring.parts == 1 && ring_finishes;
+  // blocks go out only where the launch that follows writes them: the skinny kernel, the finishing kernel of the slices, and a gated
+  // product of the kernel for many rows (not the tiles, which run what that kernel does not take)
+  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || ring_whole)),
              "gemm_bf16: a product of M=%d N=%d K=%d does not write these blocks", M, N, K);
   dim3 finish_grid((N + FINISH_COLUMNS - 1) / FINISH_COLUMNS, (M + 15) / 16);
   const RowBlocks finish_blocks = {0, slices ? c_block_rows : 0, slices ? behind_block_rows : 0};
@@ -1442,11 +1454,7 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
     return bh_check_launch("gemm_parts_finish");
   }
   const int a_blocked = a_block_rows == 16 && !skinny, c_blocked = c_block_rows == 16 && !skinny;
-  // (what the kernel for many rows does not finish itself, rows of a norm ahead or adding into bfloat16, takes a plan with parts if there is one)
-  RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32));
-  if (ring.parts == 1 && !activation && (ahead_ss || (accumulate && !f32)))
-    if (const RingPlan other = gemm_ring_plan(M, N, K, layout, ring_output(0, !f32)); other.parts > 1) ring = other;
-  if (a_blocked && !behind_weight && ring.tile >= 0 && ring.parts == 1)   // many rows (what cannot run there comes in rows)
+  if (ring_whole)
     return gemm_ring_launch(a, w, c, c_dtype, accumulate, M, N, K, activation, ring.tile, c_blocked, form, stream);
 #define BH_PICK(FN, TILES, EXTRA, ...)                                             \
   do {                                                                              \

@@ -528,7 +528,7 @@ class HipKernels(KernelSizes):
         n = out.shape[1]
         sizes = (m, n, k, int(packed), int(activation))
         a_block_rows, writes, takes_norm, norm_blocks, scratch_bytes, finishes_norm = self._product(*sizes)
-        if a_block_rows == 16 and m > 32 and not scratch_bytes and (ahead is not None or (accumulate and out.dtype != torch.float32)):
+        if a_block_rows == 16 and m > 32 and not scratch_bytes and accumulate and out.dtype != torch.float32:
             a_block_rows = 0      # the kernel for many rows that reads blocks does not take these operands; the tiles read rows
         # the activations in the form this product reads: whoever produced them for this reader wrote them so
         if ahead is not None:
@@ -559,7 +559,8 @@ class HipKernels(KernelSizes):
         behind = None
         if (then_norm is not None and out.dtype == torch.float32 and not activation
                 and then_norm.weight.shape == (n,) and then_norm.weight.dtype in _CODES):
-            blocks = norm_blocks      # 0: this product carries no norm
+            # 0: this product carries no norm, or the product that reads it takes no prepared rows
+            blocks = norm_blocks if self._reader_takes_norm(then_norm, m, n) else 0
             if blocks:
                 rows = self.new_rows(m, n, torch.bfloat16, *self._reader_of(then_norm)) if writes == 2 else \
                     torch.empty((m, n), dtype=torch.bfloat16, device=self.device)
@@ -601,7 +602,7 @@ class HipKernels(KernelSizes):
         if w.shape[1] != k or tuple(out.shape) != (m, n):
             raise KernelError(f"gemm: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
         if isinstance(a, NormedRows) and not self._takes_norm(a, w, n, 0):
-            a = self._run_norm(a)
+            a = self._run_norm(a, w, n, 0)
         done, prepared = self._gemm_fast(a, w, out, accumulate, 0, then_norm)
         if done:
             return prepared
@@ -688,9 +689,21 @@ class HipKernels(KernelSizes):
         return bool(w.dtype == torch.bfloat16 and k % 8 == 0 and (not activation or n % 16 == 0)
                     and self._product(m, n, k, int(isinstance(w, PackedWeight)), int(activation))[2])
 
-    def _run_norm(self, prepared):
-        """The norm that `prepared` stands for, as a step of its own."""
-        out = torch.empty(tuple(prepared.shape), dtype=prepared.dtype, device=self.device)
+    def _reader_takes_norm(self, then_norm, m, n):
+        """Whether prepared norm rows [m, n] are of use to the product that the request names as their reader, if it names one."""
+        reader = self._reader_of(then_norm)
+        if not reader or not reader[2] or n % 64:
+            return True
+        outputs, gated = int(reader[0]), bool(reader[1])
+        if gated and outputs % 16:      # a plain product of both halves
+            outputs, gated = 2 * outputs, False
+        return self._product(m, outputs, n, 1, int(gated))[2]
+
+    def _run_norm(self, prepared, w, n, activation):
+        """The norm that `prepared` stands for, as a step of its own, in the form its reader takes: the product with `w` of `n`
+        outputs."""
+        m, k = prepared.shape
+        out = self.new_rows(m, k, prepared.dtype, n, activation, isinstance(w, PackedWeight))
         self.rmsnorm(prepared.source, prepared.weight, prepared.eps, out)
         return out
 
@@ -705,7 +718,7 @@ class HipKernels(KernelSizes):
             raise KernelError(f"gemm_swiglu: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} "
                               "do not fit")
         if isinstance(a, NormedRows) and width % 16 == 0 and not self._takes_norm(a, w, width, 1):
-            a = self._run_norm(a)
+            a = self._run_norm(a, w, width, 1)
         if self._gemm_fast(a, w, out, False, 1, gate=self.GATES[gate])[0]:
             return
         if isinstance(out, BlockedRows):      # this product writes rows, or not these blocks: regroup them afterwards

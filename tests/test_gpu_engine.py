@@ -166,6 +166,21 @@ def test_prompts_of_many_rows(large_expected):
     check("together against alone", together, alone, TOLERANCE["bfloat16"] / 2)
 
 
+def test_prompts_of_129_to_256_rows_behind_a_narrow_attention(tmp_path):
+    """An attention width below 1,024 at a hidden size of 1,024: the output projection is one of the tiles', which carry the norm
+    behind them, the gate and up product behind it one for many rows, which takes no prepared rows."""
+    import beholdd
+    config = {"architectures": ["Qwen3ForCausalLM"], "num_hidden_layers": 2, "hidden_size": 1024, "num_attention_heads": 4,
+              "num_key_value_heads": 2, "head_dim": 128, "intermediate_size": 3072, "vocab_size": 1000, "rope_theta": 1000000.0,
+              "rms_norm_eps": 1e-6, "max_position_embeddings": 8192, "tie_word_embeddings": False}
+    beholdd.write_random_model(str(tmp_path), config, seed=1, dtype="bfloat16")
+    cfg, weights = plain.load_plain(str(tmp_path))
+    requests = schedules.random_requests(cfg.vocab, [129, 200, 256], seed=5)
+    want = [plain.forward_logits(cfg, weights, r) for r in requests]
+    engine = engine_for(str(tmp_path), "bfloat16")
+    check("whole", schedules.whole(engine, requests), want, TOLERANCE["bfloat16"])
+
+
 @pytest.mark.parametrize("batch", [1, 8, 24])
 def test_every_product_gets_its_rows_the_way_it_reads_them(large_expected, batch):
     """At the Qwen3-8B layer sizes the products of a prompt of 1,500 rows and of decode steps of 1, 8 and 24

@@ -100,3 +100,34 @@ def test_products_squared_behind_a_relu(K, m, n, k):
         if taken:
             got = (K.from_blocked(out) if block_rows else out).double()
             assert bool(((got - exact ** 2).abs() <= bound).all()), block_rows
+
+
+# hidden and attention widths whose output projection prepares the norm behind it (K below 1,024: tiles; more than 8,192 outputs: parts
+# of K and their finishing kernel) in front of a gated product of the kernel for many rows
+@pytest.mark.parametrize("hidden,attention,inter", [(1024, 512, 3072), (9216, 9216, 2048)])
+@pytest.mark.parametrize("m", [129, 200, 256])
+def test_norms_between_products_of_129_to_256_rows(K, m, hidden, attention, inter):
+    """o -> norm -> gate and up into the down product's blocks -> down, with and without the norm's reader named, against float64."""
+    from beholdd.parts.base import NormRequest, ProductReader
+    g = torch.Generator(device="cuda:0").manual_seed(m + hidden)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device="cuda:0")
+    attended = normal(m, attention).to(torch.bfloat16)
+    w_o, w_gate_up, w_down = ((normal(rows, cols) / cols ** 0.5).to(torch.bfloat16)
+                              for rows, cols in ((hidden, attention), (2 * inter, hidden), (hidden, inter)))
+    base, weight = normal(m, hidden), 1 + 0.3 * normal(hidden)
+    o, gate_up, down = K.pack_weight(w_o), K.pack_weight(w_gate_up), K.pack_weight(w_down)
+    residual64 = base.double() + attended.double() @ w_o.double().t()
+    normed64 = residual64 / torch.sqrt((residual64 ** 2).mean(-1, keepdim=True) + 1e-5) * weight.double()
+    both = normed64 @ w_gate_up.double().t()
+    want = residual64 + (both[:, :inter] / (1 + torch.exp(-both[:, :inter])) * both[:, inter:]) @ w_down.double().t()
+    for reader in (None, ProductReader(inter, True)):
+        residual = base.clone()
+        x = K.gemm(attended, o, residual, accumulate=True, then_norm=NormRequest(weight, 1e-5, reader))
+        if x is None:
+            x = K.new_rows(m, hidden, torch.bfloat16, inter, True)
+            K.rmsnorm(residual, weight, 1e-5, x)
+        activated = K.new_rows(m, inter, torch.bfloat16, hidden)
+        K.gemm_swiglu(x, gate_up, activated)
+        K.gemm(activated, down, residual, accumulate=True)
+        # three bfloat16 roundings on the way (the norm's rows, the gated output, and once more where a norm rides)
+        assert rel(residual, want.cpu()) < 1e-2

@@ -2,6 +2,7 @@
 (`KernelSizes`), at the compute-unit count it assumes there (256)."""
 
 import pytest
+import torch
 
 from beholdd.kernels import KernelSizes
 
@@ -50,3 +51,27 @@ def test_the_norm_that_rides_counts_the_workgroups_of_wider_spans(sizes):
     assert blocks(32, 6144, 4096) == 256           # 384 blocks: spans of 24 rows
     assert blocks(8, 7168, 5120) == 448            # 28 rows could lie in three blocks: left to the blocks of 16
     assert blocks(8, 8192, 4096) == 512 and blocks(8, 2560, 4096) == 160
+
+
+def test_prepared_rows_reach_no_product_that_does_not_scale(sizes):
+    """From 129 rows on the kernel for many rows takes a gated product, whose output it may write in blocks but whose sums it does
+    not scale: it takes no prepared rows; plain products take them where K goes in parts."""
+    takes, writes, scratch = sizes.lib.bh_gemm_bf16_takes_norm, sizes.lib.bh_gemm_bf16_writes_blocked, sizes.lib.bh_gemm_bf16_scratch
+    for m in (129, 160, 200, 256, 300, 1000):
+        for k in (64, 512, 1024, 2048, 4096, 9216):
+            for n in (128, 512, 1024, 3072, 9216, 27648):
+                assert not (takes(m, n, k, 1, 1) and writes(m, n, k, 1, 1)), (m, n, k)
+                if sizes.lib.bh_gemm_bf16_reads_blocked(m, n, k, 1, 0) and takes(m, n, k, 1, 0):
+                    assert scratch(m, n, k, 1, 0) > 0, (m, n, k)
+
+
+def test_a_launch_that_writes_rows_refuses_an_output_in_blocks(sizes):
+    """The tiles know rows only: the entry for all products refuses what would reach them with an output in blocks, prepared rows or
+    activations in rows, before anything is launched."""
+    if torch.cuda.is_available():
+        pytest.skip("made-up addresses: only where nothing can be launched")
+    at = 1 << 20
+    for ahead, why in ((at, "cannot take prepared norm rows"), (None, "does not write these blocks")):
+        status = sizes.lib.bh_gemm_bf16(at, at, at, 1, 0, 200, 3072, 1024, 1, 1, ahead, 16 if ahead else 0, 1e-6 if ahead else 0.0,
+                                        None, 0, None, None, None, 0, 16, 0, None)
+        assert status != 0 and why in sizes.lib.bh_last_error().decode(), ahead
