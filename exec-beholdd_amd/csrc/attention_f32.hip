@@ -12,6 +12,7 @@
 // lane its own line), 20 before a page's keys and values were asked for together; four prompts of 695 rows in all, up to 256 each,
 // 41 us in waves of their own (30 in tiles of columns, see there), 94 in workgroups of four waves on four rows, 120 there.
 #include "common.h"
+#include <algorithm>
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
@@ -418,16 +419,44 @@ __global__ __launch_bounds__(256, P <= 4 ? 2 : 1) void attention_f32_tiles_kerne
   }
 }
 
+// Whether a step of prompts goes in tiles.  A tile walks its sequences one after another, a page of a sequence after the other, where
+// the walk above has every row's pages in waves of their own: rows of several sequences that look far back, one behind the other in a
+// tile, are a chain of all their pages (a prompt of 512 rows beside 14 rows behind 1,000 keys, 8 heads of 128 on 4: 138 us, 406 in
+// tiles), and it may begin when all other tiles are done.  So the longest such chain, at what a page of it takes (1.5 us a page of a
+// head of 32, 2.05 of 64, 3.2 of 128, 5.4 of 256), has to fit in what the tiles save of the walk's time for all rows' pages together.
+// That is SAVED, ns a row, head and page (the walk's four waves share a row's pages, so that 1.5 more are waited for on average), from
+// 2,048 rows alone, walk / tiles, us: 16 heads of 32 200 / 115, of 64 345 / 205; 8 heads of 96 544 / 174, 128 724 / 217, 160 651 / 287,
+// 192 1,296 / 330, 224 1,634 / 355, 256 1,376 / 398.
+// `start` and `past`: the step's sequences as the host knows them, or null: then the average is all there is to go by.
+bool tiles_pay(int n_rows, int n_seqs, int H, int KVH, int hd, int span, const int32_t* start, const int32_t* past) {
+  if (n_rows < 32 * n_seqs || (long)n_rows * H <= 8L * bh_compute_units() || KVH > 65535) return false;
+  if (!start || !past) return true;
+  const int group = H / KVH, seen = span ? (span > 0 ? span : -span) / BH_PAGE + 2 : 0x7fffffff;      // pages that a window or chunk touches
+  double row_pages = 0.;
+  long chain = 0, tile = -1, walked = 0;      // the tile that the sequences so far end in, and the pages it walks for them
+  for (int s = 0; s < n_seqs; ++s) {
+    const int rows = start[s + 1] - start[s], pages = std::min((past[s] + rows - 1) / BH_PAGE + 1, seen);
+    if (rows <= 0) continue;
+    row_pages += rows * (0.5 * (std::min(past[s] / BH_PAGE + 1, seen) + pages) + 1.5);
+    const long first = (long)start[s] * group / 16, last = ((long)start[s + 1] * group - 1) / 16;
+    walked = (first == tile ? walked : 0) + pages;
+    chain = std::max(chain, walked);
+    if (last != first) walked = pages;
+    tile = last;
+  }
+  constexpr double SAVED[8] = {0.15, 0.27, 1.2, 1.7, 1.2, 3.2, 4.2, 3.3};
+  return chain * (1.0 + hd / 58.) <= 1e-3 * SAVED[hd / 32 - 1] * row_pages * H + 12.0;
+}
+
 template <int P>
-void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, hipStream_t stream) {
+void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, bool tiled, hipStream_t stream) {
   constexpr int NR = P <= 4 ? 4 : P <= 7 ? 2 : 1;      // what the registers hold without spilling
   const bool prompts = n_rows >= 8 * n_seqs;
   // Columns in tiles where (rows, heads) are more than the waves of two a SIMD, so that a wave a row would come in rounds, and the step
-  // is prompts: a tile walks its sequences one after another.  As below / in tiles, us: 300, 186, 200 and 58 rows of 8 heads of 128 on 4
-  // 102 / 30, on 16 heads 198 / 40, 16 prompts of 40 rows of 16 heads 52 / 23, one of 256 40 / 18, of 2,048 of 8 heads 724 / 216, of
-  // 1,000 of 8 heads of 256 on 1 400 / 129; but 4 prompts of 64 of 8 heads of 256 17 / 19, one of 33 of 16 heads 6.8 / 10.2, and one of
-  // 512 beside 63 sequences that bring a row behind 1,000 keys 170 / 404.
-  if (n_rows >= 32 * n_seqs && (long)n_rows * t.H > 8L * bh_compute_units() && t.KVH <= 65535) {
+  // is prompts.  As below / in tiles, us: 300, 186, 200 and 58 rows of 8 heads of 128 on 4 102 / 30, on 16 heads 198 / 40, 16 prompts of
+  // 40 rows of 16 heads 52 / 23, one of 256 40 / 18, of 2,048 of 8 heads 724 / 216, of 1,000 of 8 heads of 256 on 1 400 / 129; but
+  // 4 prompts of 64 of 8 heads of 256 17 / 19, and one of 33 of 16 heads 6.8 / 10.2.
+  if (tiled) {
     const long tiles = ((long)n_rows * (t.H / t.KVH) + 15) / 16;
     attention_f32_tiles_kernel<P><<<dim3((unsigned)tiles, t.KVH), 256, 0, stream>>>(t, n_rows);
     return;
@@ -457,10 +486,15 @@ void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, hipSt
 extern "C" int bh_attention_f32_takes(int H, int KVH, int hd, int kv_order) {
   return hd % 32 == 0 && hd >= 32 && hd <= 256 && KVH > 0 && H % KVH == 0 && H <= 65535 && kv_order == BH_KV_ROWS ? 1 : 0;
 }
-// `n_seqs`: the rows of the page table.  `most_pages`: how many pages a row sees at most, as far as the caller knows.
+// Whether a step's rows go in tiles of columns: start [n_seqs + 1] and past [n_seqs] on the host, or null.
+extern "C" int bh_attention_f32_tiles(int n_rows, int n_seqs, int H, int KVH, int hd, int window, const int32_t* start, const int32_t* past) {
+  return n_rows > 0 && n_seqs > 0 && bh_attention_f32_takes(H, KVH, hd, BH_KV_ROWS) && tiles_pay(n_rows, n_seqs, H, KVH, hd, window, start, past) ? 1 : 0;
+}
+// `n_seqs`: the rows of the page table.  `most_pages`: how many pages a row sees at most, as far as the caller knows.  `host_start`
+// [n_seqs + 1] and `host_past` [n_seqs]: where each sequence's rows begin and what its cache held before them, in host memory, or null.
 extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages, const float* v_pages, const int32_t* page_table,
-                                int table_stride, int n_seqs, int most_pages, const int32_t* row_seq, const int32_t* positions,
-                                int n_rows, int H, int KVH, int hd, float scale, int window, int kv_order, const float* sinks, const void* gates,
+                                int table_stride, int n_seqs, int most_pages, const int32_t* host_start, const int32_t* host_past,
+                                const int32_t* row_seq, const int32_t* positions, int n_rows, int H, int KVH, int hd, float scale, int window, int kv_order, const float* sinks, const void* gates,
                                 int gate_stride, float cap, const float* slopes, float temp_coef, int temp_every, float out_scale,
                                 hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && H > 0 && KVH > 0 && hd > 0 && n_seqs > 0, "attention: sizes must be positive");
@@ -471,15 +505,16 @@ extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages
   if (const char* fault = bh_score_form_fault(form)) return bh_fail("attention: %s", fault);
   const F32Attention t = {q, out, k_pages, v_pages, page_table, table_stride, row_seq, positions, H, KVH, form, window,
                           {sinks, gates, gate_stride, out_scale}};
+  const bool tiled = tiles_pay(n_rows, n_seqs, H, KVH, hd, window, host_start, host_past);
   switch (hd / 32) {
-    case 1: launch<1>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 2: launch<2>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 3: launch<3>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 4: launch<4>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 5: launch<5>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 6: launch<6>(t, n_rows, n_seqs, most_pages, stream); break;
-    case 7: launch<7>(t, n_rows, n_seqs, most_pages, stream); break;
-    default: launch<8>(t, n_rows, n_seqs, most_pages, stream); break;
+    case 1: launch<1>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 2: launch<2>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 3: launch<3>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 4: launch<4>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 5: launch<5>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 6: launch<6>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    case 7: launch<7>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
+    default: launch<8>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
   }
   return bh_check_launch("attention_f32");
 }

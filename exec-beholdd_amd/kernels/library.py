@@ -144,8 +144,9 @@ class KernelSizes:
             "bh_gemm_bf16_bare_parts": [i, i, i, i],
             "bh_gemm_bf16_bare": [p, p, p, i, i, i, i, i, p],
             "bh_attention_generic": [p, p, i, p, p, p, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
-            "bh_attention_f32": [p, p, p, p, p, i, i, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
+            "bh_attention_f32": [p, p, p, p, p, i, i, i, p, p, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32_takes": [i, i, i, i],
+            "bh_attention_f32_tiles": [i, i, i, i, i, i, p, p],
             "bh_gemm_f32_takes_gated": [i, i, i],
             "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
             "bh_swiglu": [p, p, i, i, i, i, p],
@@ -808,7 +809,8 @@ class HipKernels(KernelSizes):
         the sequence's position 0), else 0 .. p; not both.  `layout`, when given,
         says how rows group into sequences (seq_start int32 [n_seqs + 1] on the device, n_seqs,
         max_rows_per_seq, max_position), which the matrix-core kernel needs; rows of one sequence
-        are consecutive and in position order.  `sinks` (float32 [n_heads]): exp(sinks[head]) is one more term of the
+        are consecutive and in position order.  Its host_seq_start and host_seq_past, where it has them, are the same in lists: the
+        float32 kernels choose by them how the rows are cut up.  `sinks` (float32 [n_heads]): exp(sinks[head]) is one more term of the
         head's softmax sums, with no key and no value.  `gates` [n, P] of q's type: a finished head is multiplied by
         sigmoid(gates[row, gate_first + head]), and by `out_scale`.  Scores are softcap * tanh(score / softcap) where `softcap` is
         given; `slopes` (float32 [n_heads]): slopes[head] * (p - j) is taken off the score of a key at j; `q_temp` = (coef, every):
@@ -865,10 +867,16 @@ class HipKernels(KernelSizes):
         kv_order = self.kv_order(k_pages.dtype, head_dim)
         if (q.dtype == torch.float32 and self.lib.bh_attention_f32_takes(n_heads, n_kv_heads, head_dim, kv_order)
                 and (q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0):
+            # the sequences as the host has them, if it does and they are the page table's: how the rows are best cut up
+            starts, pasts = getattr(layout, "host_seq_start", None), getattr(layout, "host_seq_past", None)
+            if starts is None or pasts is None or len(pasts) != page_table.shape[0] or len(starts) != len(pasts) + 1 or starts[-1] != n_rows:
+                starts = pasts = None
+            else:
+                starts, pasts = (ctypes.c_int32 * len(starts))(*starts), (ctypes.c_int32 * len(pasts))(*pasts)
             self._check(self.lib.bh_attention_f32(
                 *common, self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
                 self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1], page_table.shape[0],
-                furthest // self.page_size + 1 if layout is not None else page_table.shape[1],
+                furthest // self.page_size + 1 if layout is not None else page_table.shape[1], starts, pasts,
                 self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(positions, "positions", (torch.int32,)),
                 n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), kv_order,
                 self._ptr(sinks, "sinks", (torch.float32,), True), *gating, *form, float(out_scale), self._stream()))

@@ -237,3 +237,30 @@ def test_float32_attention_of_prompts_in_tiles_score_forms_and_ends(K):
                     size, 0.2, **more)
         outs.append(out.reshape(length, n_heads, size)[..., :40].double())
     assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("pasts,tiled", [([0] + [900] * 6, False), ([0] * 7, True)])
+def test_float32_attention_of_a_prompt_beside_decoding_rows(K, pasts, tiled):
+    """A step that says how its rows group into sequences: rows behind many keys keep the step out of the tiles, rows behind few do not;
+    the results are the same sums either way."""
+    import ctypes
+    from types import SimpleNamespace
+    n_heads, kv_heads, head_dim, news = 16, 8, 128, [300] + [1] * 6
+    lengths = [p + n for p, n in zip(pasts, news)]
+    kp, vp, table, keys, values = make_cache(len(lengths), lengths, kv_heads, head_dim, torch.float32, seed=3)
+    starts = [sum(news[:i]) for i in range(len(news) + 1)]
+    assert bool(K.lib.bh_attention_f32_tiles(starts[-1], len(news), n_heads, kv_heads, head_dim, 0, (ctypes.c_int32 * len(starts))(*starts),
+                                             (ctypes.c_int32 * len(pasts))(*pasts))) == tiled
+    positions = torch.tensor([p + t for p, n in zip(pasts, news) for t in range(n)], dtype=torch.int32)
+    row_seq = torch.tensor([s for s, n in enumerate(news) for _ in range(n)], dtype=torch.int32)
+    layout = SimpleNamespace(is_decode=False, seq_start=dev(torch.tensor(starts, dtype=torch.int32)), n_seqs=len(news), max_rows_per_seq=max(news),
+                             max_position=max(lengths) - 1, host_seq_start=starts, host_seq_past=pasts)
+    q = torch.randn(len(positions), n_heads * head_dim, generator=torch.Generator().manual_seed(1))
+    out = torch.full(q.shape, float("nan"), device="cuda:0")
+    K.attention(dev(q), out, dev(kp), dev(vp), dev(table), dev(row_seq), dev(positions), n_heads, kv_heads, head_dim, head_dim ** -0.5,
+                layout=layout)
+    for s in range(len(news)):
+        rows = slice(starts[s], starts[s + 1])
+        want = attention_reference_rows(q[rows], keys[s], values[s], positions[rows].long(), n_heads, kv_heads, head_dim, head_dim ** -0.5, 0)
+        # as in test_float32_attention_rows_of_a_step
+        assert float((out[rows].cpu().double() - want).abs().max() / want.abs().max()) < 1e-5, s

@@ -75,3 +75,31 @@ def test_a_launch_that_writes_rows_refuses_an_output_in_blocks(sizes):
         status = sizes.lib.bh_gemm_bf16(at, at, at, 1, 0, 200, 3072, 1024, 1, 1, ahead, 16 if ahead else 0, 1e-6 if ahead else 0.0,
                                         None, 0, None, None, None, 0, 16, 0, None)
         assert status != 0 and why in sizes.lib.bh_last_error().decode(), ahead
+
+
+def float32_tiles(sizes, lengths, pasts, heads, kv_heads, head_dim, window=0):
+    import ctypes
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    return bool(sizes.lib.bh_attention_f32_tiles(starts[-1], len(lengths), heads, kv_heads, head_dim, window,
+                                                 (ctypes.c_int32 * len(starts))(*starts), (ctypes.c_int32 * len(pasts))(*pasts)))
+
+
+def test_float32_prompts_go_in_tiles_unless_short_rows_look_far(sizes):
+    """A tile of 16 columns walks its sequences one after another: prompts go in tiles, and so do rows that share a sequence behind any
+    number of keys, but not decoding rows one behind the other in a tile behind many keys."""
+    alone = lambda *lengths: (list(lengths), [0] * len(lengths))
+    for lengths, pasts in (alone(2048), alone(300, 186, 200, 58), alone(700, 300), alone(*[120] * 8), ([64] * 8, [1000] * 8), ([64] * 8, [8000] * 8)):
+        for heads, kv_heads, head_dim in ((8, 4, 128), (16, 2, 128), (32, 8, 128), (8, 2, 256), (16, 16, 64)):
+            assert float32_tiles(sizes, lengths, pasts, heads, kv_heads, head_dim), (lengths, heads, kv_heads, head_dim)
+    # 8 rows of a sequence each in a tile, 2, 4 and 16
+    for heads, kv_heads, head_dim in ((8, 4, 128), (16, 2, 128), (32, 8, 128), (16, 16, 64)):
+        assert not float32_tiles(sizes, [500] + [1] * 14, [0] + [8000] * 14, heads, kv_heads, head_dim)
+        assert not float32_tiles(sizes, [512, 1], [0, 8000], heads, kv_heads, head_dim)
+    # a window or a chunk bounds what a row sees
+    assert float32_tiles(sizes, [500] + [1] * 14, [0] + [8000] * 14, 32, 8, 128, 64)
+    assert float32_tiles(sizes, [500] + [1] * 14, [0] + [8000] * 14, 32, 8, 128, -64)
+    assert not float32_tiles(sizes, [2000] + [1] * 60, [0] + [4000] * 60, 8, 4, 128)
+    assert float32_tiles(sizes, [2000] + [1] * 60, [0] + [500] * 60, 8, 4, 128)
+    assert float32_tiles(sizes, [2000] + [1] * 60, [0] + [4000] * 60, 32, 8, 128)
+    # few rows a sequence, or few rows and heads: never
+    assert not float32_tiles(sizes, [31] * 8, [0] * 8, 32, 8, 128) and not float32_tiles(sizes, [64], [0], 16, 8, 128)
