@@ -22,7 +22,6 @@
 // 192 x 128 (no faster than 128 x 128 and 256 x 128 at any size) and 256 x 160.
 #include "gemm_bf16_ring.h"
 #include "gemm_bf16_turns.h"
-#include <algorithm>
 #include <type_traits>
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -232,36 +231,38 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
 #undef WAIT_VM_LGKM0
 #undef MEET
 
-// A tile's sizes and what a step of 32 k costs a compute unit that has one, or two, workgroups of it (us; from the products named at the
-// top of this file, weights from memory).  Two workgroups of the tile of four waves share a compute unit.
+// A tile's sizes, what a step of 32 k costs a compute unit that has one, or two, workgroups of it, and what their start and end cost (us).
+// Two workgroups of the tile of four waves share a compute unit.  From the times of every tile and cut of K for 34 products of 1,024 to
+// 17,408 weight rows and 17 numbers of rows from 129 to 4,100 (625 sizes, weights from memory, with the norm, finishing or rotation
+// behind them): what this chooses there takes 1 % (float32), 2 % (bfloat16) and 1 % (gated) longer than the best of them on average.
+// One process differs from another by up to 8 % where a product takes more than 80 us (the clock that the power leaves).
 struct TileShape {
   int rows, columns, share;
-  double step, step_shared;
+  double step, step_shared, start_and_end;
 };
-constexpr TileShape SHAPES[RING_TILES] = {{128, 128, 2, 0.28, 0.50}, {128, 128, 1, 0.25, 0.}, {256, 128, 1, 0.475, 0.}, {256, 192, 1, 0.65, 0.}, {256, 256, 1, 0.81, 0.}};
+constexpr TileShape SHAPES[RING_TILES] = {
+    {128, 128, 2, 0.245, 0.43, 4.0}, {128, 128, 1, 0.23, 0., 5.0}, {256, 128, 1, 0.36, 0., 4.0}, {256, 192, 1, 0.51, 0., 5.3}, {256, 256, 1, 0.594, 0., 5.0}};
 constexpr int MOST_PARTS = 8;
 
 double cost_us(int tile, int parts, int M, int W, int K, RingOutput output) {
   const TileShape& s = SHAPES[tile];
   const long units = bh_compute_units(), workgroups = (long)((M + s.rows - 1) / s.rows) * ((W + s.columns - 1) / s.columns) * parts;
-  const double steps = K / 32.0 / parts, start_and_end = tile == RING_128x128_HALVES ? 5.0 : 4.0;
-  const double alone = steps * s.step + start_and_end;
+  const double steps = K / 32.0 / parts, alone = steps * s.step + s.start_and_end;
   double t;
   if (s.share == 1) {
     t = (double)((workgroups + units - 1) / units) * alone;
-  } else {
-    // Whole rounds of two a compute unit, then a last one: of one each, or of two on some (which run the faster the fewer they are).
-    const double both = steps * s.step_shared + start_and_end;
+  } else {      // whole rounds of two a compute unit, then a last one: of two, which take as long on some units as on all, or of one
+    const double both = steps * s.step_shared + s.start_and_end;
     const long rest = workgroups % (2 * units);
-    t = (double)(workgroups / (2 * units)) * both;
-    if (rest > units) t += alone + (both - alone) * (0.5 + 0.5 * (double)(rest - units) / units);
-    else if (rest > 0) t += alone;
+    t = (double)(workgroups / (2 * units)) * both + (rest > units ? both : rest > 0 ? alone : 0.);
   }
-  t = std::max(t, (double)W * K * 2.0 / 6.0e6);      // the weights once at 6 TB/s
-  // The parts' sums are written at 5.5 TB/s and read again at 6.5 by a second launch.  A plain bfloat16 product in parts is the queries',
-  // keys' and values' projection as a rule, whose reader takes the parts as they are (gemm_ring_bare_plan): only their way to memory counts, in part hidden behind the next tiles.
-  if (parts > 1) t += output == RING_BF16 ? parts * (double)M * W * 4.0 / 7e6 : parts * (double)M * W * 4.0 * (1.0 / 5.5e6 + 1.0 / 6.5e6) + 2.0;
-  return t;
+  if (parts == 1) return t;
+  // The parts' sums on their way to memory and back.  float32: the finishing kernel takes the place of the norm's launch.  bfloat16: it
+  // is a launch more; wide products are the queries', keys' and values' projection as a rule, whose reader takes the parts as they are
+  // (gemm_ring_bare_plan), and at those what hides behind the next tiles is more: cheaper from 6,144 weight rows on (rather than
+  // at the price of the others: 768 x 7,168 x 5,120 75.9 against 79.9 us, 1,000 x 6,144 x 4,096 70.1 against 69.5).
+  const double sums = parts * (double)M * W * 4.0;
+  return t + (output == RING_F32 ? sums / 3.0e6 : W >= 6144 ? sums / 7.0e6 : sums / 3.8e6 + 4.0);
 }
 
 template <int MODE>
@@ -284,8 +285,7 @@ int launch(int tile, int parts, const void* a, const void* w, void* c, int M, in
 
 }  // namespace
 
-// The tile and the parts of K with the least of the estimate above; of the plans without parts a larger tile is taken if its estimate
-// is within 6 % (it asks less of L2, which the estimate does not see where the chip is full many times over).  Up to 256 rows, and for short K there, a norm may ride on the
+// The tile and the parts of K with the least of the estimate above.  Up to 256 rows, and for short K there, a norm may ride on the
 // product (gemm_bf16.hip), which this kernel does not carry; up to 128 rows the kernel of gemm_bf16_slices.hip is the faster one.
 RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
   RingPlan plan = {-1, 1};
@@ -303,13 +303,17 @@ RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
       if (parts > 1 && (K % (64 * parts) != 0 || K / parts < 256)) continue;
       if (tile >= RING_256x192 && !gemm_turns_can(M, N, K, parts > 1 ? 1 : mode, blocks, parts)) continue;
       const double cost = cost_us(tile, parts, M, W, K, output);
-      if (plan.tile < 0 || cost < least || (parts == 1 && plan.parts == 1 && tile >= RING_256x128 && cost < 1.06 * least)) {
-        least = plan.tile < 0 ? cost : std::min(cost, least);
-        plan.tile = tile, plan.parts = parts;
-      }
+      if (plan.tile < 0 || cost < least) least = cost, plan.tile = tile, plan.parts = parts;
     }
   }
   return plan;
+}
+
+// For tests: 16 times the tile (enum RingTile) + the parts of K, or -1; output: enum RingOutput.
+extern "C" int bh_gemm_bf16_plan(int M, int N, int K, int layout, int output) {
+  if (M <= 0 || N <= 0 || K <= 0 || output < RING_F32 || output > RING_BF16) return -1;
+  const RingPlan plan = gemm_ring_plan(M, N, K, layout, (RingOutput)output);
+  return plan.tile < 0 ? -1 : 16 * plan.tile + plan.parts;
 }
 
 RingPlan gemm_ring_bare_plan(int M, int N, int K, int layout) {

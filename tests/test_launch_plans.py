@@ -103,3 +103,27 @@ def test_float32_prompts_go_in_tiles_unless_short_rows_look_far(sizes):
     assert float32_tiles(sizes, [2000] + [1] * 60, [0] + [4000] * 60, 32, 8, 128)
     # few rows a sequence, or few rows and heads: never
     assert not float32_tiles(sizes, [31] * 8, [0] * 8, 32, 8, 128) and not float32_tiles(sizes, [64], [0], 16, 8, 128)
+
+
+TILES = ["128x128", "128x128 in halves", "256x128", "256x192", "256x256"]
+
+
+def many_rows_plan(sizes, m, n, k, output):
+    """(tile, parts of K) of a product of many rows, or None; `output`: "float32", "gated" or "bfloat16"."""
+    plan = sizes.lib.bh_gemm_bf16_plan(m, n, k, 1, ["float32", "gated", "bfloat16"].index(output))
+    return (TILES[plan // 16], plan % 16) if plan >= 0 else None
+
+
+def test_products_of_many_rows_take_the_tiles_that_were_measured_fastest(sizes):
+    """Sizes at which the choice matters: what is chosen / the next best of another kind, us, the launches behind them included."""
+    plan = lambda *size: many_rows_plan(sizes, *size)
+    assert plan(768, 4096, 12288, "float32") == ("256x256", 4)              # 88 / 105 on 128 x 128 in 4 parts
+    assert plan(1500, 4096, 12288, "float32") == ("256x256", 2)             # 143 / 159 on 256 x 128
+    assert plan(1500, 4096, 4096, "float32") == ("256x128", 1)              # 70 / 78 on 128 x 128 in 2 parts
+    assert plan(1000, 5120, 5120, "float32") == ("256x192", 2)              # 72 / 78 on 256 x 128, 98 on 128 x 128 in 2
+    assert plan(1300, 2048, 2048, "bfloat16") == ("128x128", 1)             # 23 / 27 in 2 parts
+    assert plan(2100, 1024, 1024, "bfloat16") == ("128x128", 1)             # 14 / 19 on 256 x 128
+    assert plan(1800, 3072, 2048, "bfloat16")[0] in ("128x128", "256x128")  # 32 / 40 in halves
+    assert plan(640, 17408, 5120, "gated") == ("256x256", 1)                # 231 / 253 on 128 x 128
+    assert plan(256, 12288, 4096, "gated") == ("256x128", 1)                # 66 / 78 on 128 x 128
+    assert plan(128, 4096, 4096, "float32") is None and plan(256, 4096, 512, "float32") is None      # for the slices; the tiles
