@@ -33,6 +33,7 @@
 #include "gemm_bf16_slices.h"
 #include "gemm_bf16_ring.h"
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -1300,6 +1301,31 @@ static void launch_tiled(const void* a, const void* w, void* c, int M, int N, in
 
 static RingOutput ring_output(int activation, bool f32) { return activation ? RING_GATED : f32 ? RING_F32 : RING_BF16; }
 
+// How a product of many rows runs on the kernel for them, or (tile -1) not there.  That kernel multiplies a gated product in one go; few
+// outputs or few rows leave it few tiles, where the whole tiles above with K in parts and their finishing kernel are faster (us, there /
+// here: 256 rows of 1,024 gated outputs x 4,096 37.3 / 19.6, 129 of 2,048 x 2,048 20.2 / 16.3, 512 of 768 x 2,048 19.7 / 18.1; 400 rows of
+// 2,048 x 2,048 20.5 / 24.7, 129 of 6,912 x 2,560 31 / 40).  Theirs is estimated from rounds of two workgroups a compute unit, a slice
+// of 64 k at 0.88 us, or up to 1.6 where two share a unit, 6.2 us for the start and the second launch, and the sums' way; both estimates
+// are within 7 % of 126 measured sizes.  An 8 % lead of the kernel for many rows is asked for: with 256 and 512 rows it is slower than
+// its estimate.
+static RingPlan many_rows_plan(int M, int N, int K, int layout, RingOutput output) {
+  const RingPlan plan = gemm_ring_plan(M, N, K, layout, output);
+  if (output != RING_GATED || plan.tile < 0) return plan;
+  int rows, columns, parts, slices;
+  tiled_config(M, N, true, &rows, &columns);
+  tiled_parts(M, N, K, layout, true, &parts, &slices);
+  if (parts == 1) return plan;
+  const double each = (double)((N + columns - 1) / columns) * ((M + rows - 1) / rows) * parts / bh_compute_units();      // workgroups a compute unit
+  const double slice = 0.88 + 0.72 * std::min(std::max(each - 1.0, 0.0), 1.0), rounds = std::max(std::ceil(each / 2.0), 1.0);
+  const double tiles = rounds * slices * slice + 6.2 + parts * (double)M * 2 * N * 4.0 * 0.25e-6;
+  return tiles < 1.08 * (plan.us + 1.3 + 1.7e-6 * M * N) ? RingPlan{-1, 1} : plan;
+}
+// A gated product that the tiles run in parts where the kernel for many rows could run it: the finishing kernel writes its output, in
+// blocks of 16 rows too.
+static bool gated_in_parts(int M, int N, int K, int layout, int activation) {
+  return activation && gemm_ring_plan(M, N, K, layout, RING_GATED).tile >= 0 && many_rows_plan(M, N, K, layout, RING_GATED).tile < 0;
+}
+
 // How many partial sums per row a product of these sizes writes when a norm rides behind it (0: it cannot
 // carry one), and whether it can take prepared norm rows as its activations.
 // Beyond 256 rows a product carries no norm: at the Qwen3-8B shapes, whole model, the prompt of 128 tokens
@@ -1310,7 +1336,7 @@ extern "C" int bh_gemm_bf16_norm_blocks(int M, int N, int K, int layout, int act
   if (activation || M <= 0 || M > NORM_RIDES_UP_TO_ROWS || N <= 0 || K % 8 != 0) return 0;
   int rows, columns, parts, each;
   if (gemm_slices_takes(M, N, K, layout, 0)) return (N + FINISH_COLUMNS - 1) / FINISH_COLUMNS;   // always finished by that kernel
-  if (const RingPlan ring = gemm_ring_plan(M, N, K, layout, RING_F32); ring.tile >= 0) return ring.parts > 1 ? (N + FINISH_COLUMNS - 1) / FINISH_COLUMNS : 0;
+  if (const RingPlan ring = many_rows_plan(M, N, K, layout, RING_F32); ring.tile >= 0) return ring.parts > 1 ? (N + FINISH_COLUMNS - 1) / FINISH_COLUMNS : 0;
   tiled_config(M, N, false, &rows, &columns);
   if (!tiled_whole(M, N, K, layout, rows, columns)) {   // the skinny kernel's blocks, or its workgroups of wider spans
     if (layout == 1 && skinny_first(M, N, K, layout, 0))
@@ -1324,8 +1350,8 @@ extern "C" int bh_gemm_bf16_takes_norm(int M, int N, int K, int layout, int acti
   if (M <= 0 || N <= 0 || K % 8 != 0 || (activation && N % 16 != 0)) return 0;
   if (M <= 64) return 1;
   // The kernel for many rows does not scale its sums: of its products those take prepared rows whose finishing kernel does.
-  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0)
-    return !activation && (gemm_ring_plan(M, N, K, layout, RING_F32).parts > 1 || gemm_ring_plan(M, N, K, layout, RING_BF16).parts > 1) ? 1 : 0;
+  if (many_rows_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0)
+    return !activation && (many_rows_plan(M, N, K, layout, RING_F32).parts > 1 || many_rows_plan(M, N, K, layout, RING_BF16).parts > 1) ? 1 : 0;
   int rows, columns;
   tiled_config(M, N, activation != 0, &rows, &columns);
   return tiled_whole(M, N, K, layout, rows, columns) ? 1 : 0;
@@ -1336,7 +1362,7 @@ extern "C" int bh_gemm_bf16_takes_norm(int M, int N, int K, int layout, int acti
 // for many rows (16), and those of up to 32 rows of the skinny kernel (8 up to 8 rows, else 16).
 extern "C" int bh_gemm_bf16_reads_blocked(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0) return 0;
-  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return 16;
+  if (many_rows_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return 16;
   if (skinny_first(M, N, K, layout, activation)) return M <= 8 ? 8 : 16;
   if (gemm_slices_takes(M, N, K, layout, activation)) return 16;
   return 0;
@@ -1344,26 +1370,39 @@ extern "C" int bh_gemm_bf16_reads_blocked(int M, int N, int K, int layout, int a
 
 // In what form a product of these sizes can write the bfloat16 rows it produces for the next product (a SwiGLU's
 // output, the rows prepared for a norm behind it): 2 = rows or blocks of 8 or 16 rows (the skinny kernel),
-// 1 = rows or, for SwiGLU, blocks of 16 (the kernel for many rows), 0 = rows only.
+// 1 = rows or, for SwiGLU, blocks of 16 (the products of many rows), 0 = rows only.
 extern "C" int bh_gemm_bf16_writes_blocked(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 32 != 0) return 0;
-  if (gemm_ring_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return activation ? 1 : 0;
+  if (many_rows_plan(M, N, K, layout, ring_output(activation, true)).tile >= 0) return activation ? 1 : 0;
   if (gemm_slices_takes(M, N, K, layout, activation)) return 2;    // the finishing kernel writes any blocks
+  if (gated_in_parts(M, N, K, layout, activation)) return 1;
   int rows, columns;
   tiled_config(M, N, activation != 0, &rows, &columns);
   return M <= 64 && !tiled_whole(M, N, K, layout, rows, columns) ? 2 : 0;
 }
 
-// layout: 0 = rows, 1 = tiles.  activation: 0 = none; 1 = SwiGLU (W has 2 * N rows: gate rows then up rows); to bh_gemm_bf16
-// itself also 2: the same with GELU's tanh form on the gate (BhGate; what the queries say of SwiGLU goes for it too).
-// Bytes of scratch memory that bh_gemm_bf16 wants for this product (0: none).
 // In how many parts of K the kernel for many rows, or whole tiles, multiply a product when they are given scratch memory (1: in one go).
 static int tiled_or_ring_parts(int M, int N, int K, int layout, int activation, bool f32) {
-  if (const RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32)); ring.tile >= 0) return ring.parts;
+  if (const RingPlan ring = many_rows_plan(M, N, K, layout, ring_output(activation, f32)); ring.tile >= 0) return ring.parts;
   int parts, each;
   tiled_parts(M, N, K, layout, activation != 0, &parts, &each);
   return parts;
 }
+// The width (8, 6 or 4 blocks) with which a product of these sizes runs on tiles of 256 rows in one go, else 0.
+extern "C" int bh_gemm_bf16_turns_blocks(int M, int N, int K, int layout, int activation) {
+  const RingPlan plan = many_rows_plan(M, N, K, layout, activation ? RING_GATED : RING_F32);
+  if (plan.parts != 1) return 0;
+  return plan.tile == RING_256x256 ? 8 : plan.tile == RING_256x192 ? 6 : plan.tile == RING_256x128 ? 4 : 0;
+}
+// For tests: 16 times the tile (enum RingTile) + the parts of K, or -1; output: enum RingOutput.
+extern "C" int bh_gemm_bf16_plan(int M, int N, int K, int layout, int output) {
+  if (M <= 0 || N <= 0 || K <= 0 || output < RING_F32 || output > RING_BF16) return -1;
+  const RingPlan plan = many_rows_plan(M, N, K, layout, (RingOutput)output);
+  return plan.tile < 0 ? -1 : 16 * plan.tile + plan.parts;
+}
+// layout: 0 = rows, 1 = tiles.  activation: 0 = none; 1 = SwiGLU (W has 2 * N rows: gate rows then up rows); to bh_gemm_bf16
+// itself also 2: the same with GELU's tanh form on the gate (BhGate; what the queries say of SwiGLU goes for it too).
+// Bytes of scratch memory that bh_gemm_bf16 wants for this product (0: none).
 extern "C" long bh_gemm_bf16_scratch(int M, int N, int K, int layout, int activation) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   int parts = std::max(tiled_or_ring_parts(M, N, K, layout, activation, true), tiled_or_ring_parts(M, N, K, layout, activation, false));
@@ -1424,17 +1463,18 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
   const bool slices = scratch != nullptr && a_block_rows == 16 && !skinny && gemm_slices_takes(M, N, K, layout, activation);
   // Many rows.  What that kernel does not finish itself, rows of a norm ahead or adding into bfloat16, takes a plan with parts if there
   // is one; what is left of that comes in rows, to the tiles.
-  RingPlan ring = gemm_ring_plan(M, N, K, layout, ring_output(activation, f32));
+  RingPlan ring = many_rows_plan(M, N, K, layout, ring_output(activation, f32));
   const bool ring_finishes = !ahead_ss && !behind_weight && (f32 || !accumulate);
   if (ring.parts == 1 && !activation && !ring_finishes)
-    if (const RingPlan other = gemm_ring_plan(M, N, K, layout, ring_output(0, !f32)); other.parts > 1) ring = other;
+    if (const RingPlan other = many_rows_plan(M, N, K, layout, ring_output(0, !f32)); other.parts > 1) ring = other;
   const bool ring_whole = a_block_rows == 16 && ring.tile >= 0 && ring.parts == 1 && ring_finishes;
-  // blocks go out only where the launch that follows writes them: the skinny kernel, the finishing kernel of the slices, and a gated
-  // product of the kernel for many rows (not the tiles, which run what that kernel does not take)
-  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || ring_whole)),
+  // Blocks go out only where the launch that follows writes them: the skinny kernel, the finishing kernel of the slices or of a gated
+  // product's parts, and a gated product of the kernel for many rows (not the tiles that finish a product themselves).
+  const bool tiles_finished = scratch != nullptr && !skinny && !slices && gated_in_parts(M, N, K, layout, activation);
+  BH_REQUIRE(skinny || slices || (c_block_rows != 8 && behind_block_rows == 0 && (c_block_rows == 0 || ring_whole || tiles_finished)),
              "gemm_bf16: a product of M=%d N=%d K=%d does not write these blocks", M, N, K);
   dim3 finish_grid((N + FINISH_COLUMNS - 1) / FINISH_COLUMNS, (M + 15) / 16);
-  const RowBlocks finish_blocks = {0, slices ? c_block_rows : 0, slices ? behind_block_rows : 0};
+  const RowBlocks finish_blocks = {0, slices || tiles_finished ? c_block_rows : 0, slices ? behind_block_rows : 0};
 #define BH_FINISH(SWIGLU, TC)                                                                                \
   gemm_parts_finish_kernel<SWIGLU, TC><<<finish_grid, 256, 0, stream>>>((const float*)scratch, (TC*)c, M, N, K, \
                                                                          parts, accumulate, norm, finish_blocks, form)
@@ -1515,7 +1555,7 @@ extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, 
 // which run the product and the activation one after the other.
 extern "C" int bh_gemm_bf16_squares(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || N % 16 != 0) return 0;
-  if (const RingPlan ring = gemm_ring_plan(M, N, K, 1, RING_BF16); ring.tile >= 0) return ring.parts == 1 ? 1 : 0;
+  if (const RingPlan ring = many_rows_plan(M, N, K, 1, RING_BF16); ring.tile >= 0) return ring.parts == 1 ? 1 : 0;
   return skinny_first(M, N, K, 1, 0) && !skinny_span_rows(M, N, K) ? 2 : 0;
 }
 extern "C" int bh_gemm_bf16_squared(const void* a, const void* w, void* c, int M, int N, int K, int a_block_rows, int c_block_rows,
@@ -1529,7 +1569,7 @@ extern "C" int bh_gemm_bf16_squared(const void* a, const void* w, void* c, int M
   GateForm form = bh_gate_form(0);
   form.squared = true;
   if (kind == 1) {
-    const RingPlan ring = gemm_ring_plan(M, N, K, 1, RING_BF16);
+    const RingPlan ring = many_rows_plan(M, N, K, 1, RING_BF16);
     return gemm_ring_launch(a, w, c, BH_BF16, 0, M, N, K, 0, ring.tile, c_block_rows == 16, form, stream);
   }
   launch_skinny<true, 1, bf16_t>(a, w, c, M, N, K, 0, 0, RidingNorm{}, RowBlocks{a_block_rows, c_block_rows, 0}, form, stream);
@@ -1543,14 +1583,14 @@ extern "C" int bh_rmsnorm(const float* x, const int32_t* rows, const void* w, in
 // norm; where it does not the norm is a launch of its own.  `scratch`: bh_gemm_bf16_scratch() bytes.
 extern "C" int bh_gemm_bf16_finishes_norm(int M, int N, int K, int layout) {
   if (M <= 0 || N <= 0 || K < 512 || N % 8 != 0 || N > 8 * 128 * FINISH_NORM_PIECES) return 0;
-  return gemm_ring_plan(M, N, K, layout, RING_F32).tile >= 0 ? 1 : 0;
+  return many_rows_plan(M, N, K, layout, RING_F32).tile >= 0 ? 1 : 0;
 }
 extern "C" int bh_gemm_bf16_then_norm(const void* a, const void* w, float* residual, int M, int N, int K, int layout,
                                       const void* norm_weight, int norm_weight_dtype, float eps, void* normed,
                                       void* scratch, int a_blocked, int normed_blocked, hipStream_t stream) {
   BH_REQUIRE(bh_gemm_bf16_finishes_norm(M, N, K, layout),
              "gemm_bf16_then_norm: a product of M=%d N=%d K=%d does not finish a norm (bh_gemm_bf16_finishes_norm)", M, N, K);
-  const RingPlan ring = gemm_ring_plan(M, N, K, layout, RING_F32);
+  const RingPlan ring = many_rows_plan(M, N, K, layout, RING_F32);
   const int parts = ring.parts;
   BH_REQUIRE(a && w && residual && norm_weight && normed && (scratch || parts == 1), "gemm_bf16_then_norm: every operand is needed");
   BH_REQUIRE(a_blocked, "gemm_bf16_then_norm: the activations lie in blocks of 16 rows");

@@ -9,6 +9,7 @@ enum RingTile { RING_128x128 = 0, RING_128x128_HALVES, RING_256x128, RING_256x19
 enum RingOutput { RING_F32 = 0, RING_GATED = 1, RING_BF16 = 2 };
 struct RingPlan {
   int tile, parts;
+  double us = 0.;      // the estimate it was chosen by
 };
 RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output);
 // The sums of a plain bfloat16 product left apart: its plan if that has parts, the two halves of k of a plan that adds them up itself;

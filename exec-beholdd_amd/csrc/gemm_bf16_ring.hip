@@ -292,7 +292,6 @@ RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
   const int W = output == RING_GATED ? 2 * N : N;
   if (layout != 1 || M <= 128 || N % 16 != 0 || K % 64 != 0 || K < 128 || N < 128) return plan;
   if (M <= 256 && (K < 1024 || W < 1024)) return plan;
-  double least = 0.;
   for (int tile = 0; tile < RING_TILES; ++tile) {
     if (tile == RING_128x128_HALVES && (K % 128 != 0 || K < 512)) continue;
     const int mode = output == RING_GATED ? 2 : output == RING_F32 ? 1 : 0, blocks = tile == RING_256x256 ? 8 : 6;
@@ -303,22 +302,15 @@ RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
       if (parts > 1 && (K % (64 * parts) != 0 || K / parts < 256)) continue;
       if (tile >= RING_256x192 && !gemm_turns_can(M, N, K, parts > 1 ? 1 : mode, blocks, parts)) continue;
       const double cost = cost_us(tile, parts, M, W, K, output);
-      if (plan.tile < 0 || cost < least) least = cost, plan.tile = tile, plan.parts = parts;
+      if (plan.tile < 0 || cost < plan.us) plan = {tile, parts, cost};
     }
   }
   return plan;
 }
 
-// For tests: 16 times the tile (enum RingTile) + the parts of K, or -1; output: enum RingOutput.
-extern "C" int bh_gemm_bf16_plan(int M, int N, int K, int layout, int output) {
-  if (M <= 0 || N <= 0 || K <= 0 || output < RING_F32 || output > RING_BF16) return -1;
-  const RingPlan plan = gemm_ring_plan(M, N, K, layout, (RingOutput)output);
-  return plan.tile < 0 ? -1 : 16 * plan.tile + plan.parts;
-}
-
 RingPlan gemm_ring_bare_plan(int M, int N, int K, int layout) {
   const RingPlan plan = gemm_ring_plan(M, N, K, layout, RING_BF16);
-  return plan.tile == RING_128x128_HALVES ? RingPlan{RING_128x128, 2} : plan;
+  return plan.tile == RING_128x128_HALVES ? RingPlan{RING_128x128, 2, plan.us} : plan;
 }
 
 static bool ring_can(int M, int N, int K, int tile, int parts) {
@@ -356,10 +348,4 @@ extern "C" int bh_gemm_bf16_turns(const void* a, const void* w, void* c, int c_d
   BH_REQUIRE(a_blocked, "gemm_turns: the activations lie in blocks of 16 rows");
   return gemm_ring_launch(a, w, c, c_dtype, accumulate, M, N, K, activation != 0, blocks == 8 ? RING_256x256 : blocks == 6 ? RING_256x192 : RING_256x128,
                           c_blocked, bh_gate_form(activation), stream);
-}
-// The width (8, 6 or 4 blocks) with which a product of these sizes runs on tiles of 256 rows in one go, else 0.
-extern "C" int bh_gemm_bf16_turns_blocks(int M, int N, int K, int layout, int activation) {
-  const RingPlan plan = gemm_ring_plan(M, N, K, layout, activation ? RING_GATED : RING_F32);
-  if (plan.parts != 1) return 0;
-  return plan.tile == RING_256x256 ? 8 : plan.tile == RING_256x192 ? 6 : plan.tile == RING_256x128 ? 4 : 0;
 }

@@ -102,9 +102,26 @@ def test_products_squared_behind_a_relu(K, m, n, k):
             assert bool(((got - exact ** 2).abs() <= bound).all()), block_rows
 
 
+# gated products whose K the whole tiles cut into parts: the finishing kernel writes rows or the blocks that a product of many rows reads
+@pytest.mark.parametrize("m,inter,k", [(129, 1024, 1024), (200, 1056, 4096), (256, 2048, 2048), (400, 768, 2048)])
+def test_gated_products_of_few_tiles(K, m, inter, k):
+    from beholdd.kernels.library import BlockedRows
+    assert int(K.lib.bh_gemm_bf16_plan(m, inter, k, 1, 1)) < 0 and K.lib.bh_gemm_bf16_scratch(m, inter, k, 1, 1) > 0
+    g = torch.Generator(device="cuda:0").manual_seed(m + inter)
+    a = torch.randn(m, k, generator=g, device="cuda:0").to(torch.bfloat16)
+    w = (torch.randn(2 * inter, k, generator=g, device="cuda:0") / k ** 0.5).to(torch.bfloat16)
+    gate, up = (a.double() @ half.double().t() for half in (w[:inter], w[inter:]))
+    packed, rows = K.pack_weight(w), torch.full((m, inter), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    K.gemm_swiglu(a, packed, rows)
+    assert rel(rows, (gate / (1 + torch.exp(-gate)) * up).cpu()) < 6e-3
+    blocks = K.to_blocked(torch.full((m, inter), float("nan"), dtype=torch.bfloat16, device="cuda:0"))
+    K.gemm_swiglu(K.to_blocked(a), packed, blocks)
+    assert isinstance(blocks, BlockedRows) and torch.equal(K.from_blocked(blocks), rows)
+
+
 # hidden and attention widths whose output projection prepares the norm behind it (K below 1,024: tiles; more than 8,192 outputs: parts
 # of K and their finishing kernel) in front of a gated product of the kernel for many rows
-@pytest.mark.parametrize("hidden,attention,inter", [(1024, 512, 3072), (9216, 9216, 2048)])
+@pytest.mark.parametrize("hidden,attention,inter", [(1024, 512, 3072), (1024, 512, 1024), (9216, 9216, 2048)])
 @pytest.mark.parametrize("m", [129, 200, 256])
 def test_norms_between_products_of_129_to_256_rows(K, m, hidden, attention, inter):
     """o -> norm -> gate and up into the down product's blocks -> down, with and without the norm's reader named, against float64."""

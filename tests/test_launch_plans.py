@@ -55,12 +55,13 @@ def test_the_norm_that_rides_counts_the_workgroups_of_wider_spans(sizes):
 
 def test_prepared_rows_reach_no_product_that_does_not_scale(sizes):
     """From 129 rows on the kernel for many rows takes a gated product, whose output it may write in blocks but whose sums it does
-    not scale: it takes no prepared rows; plain products take them where K goes in parts."""
+    not scale: it takes no prepared rows; products take them where K goes in parts, whose finishing kernel scales."""
     takes, writes, scratch = sizes.lib.bh_gemm_bf16_takes_norm, sizes.lib.bh_gemm_bf16_writes_blocked, sizes.lib.bh_gemm_bf16_scratch
     for m in (129, 160, 200, 256, 300, 1000):
         for k in (64, 512, 1024, 2048, 4096, 9216):
             for n in (128, 512, 1024, 3072, 9216, 27648):
-                assert not (takes(m, n, k, 1, 1) and writes(m, n, k, 1, 1)), (m, n, k)
+                if takes(m, n, k, 1, 1) and writes(m, n, k, 1, 1):
+                    assert sizes.lib.bh_gemm_bf16_plan(m, n, k, 1, 1) < 0 and scratch(m, n, k, 1, 1) > 0, (m, n, k)
                 if sizes.lib.bh_gemm_bf16_reads_blocked(m, n, k, 1, 0) and takes(m, n, k, 1, 0):
                     assert scratch(m, n, k, 1, 0) > 0, (m, n, k)
 
@@ -126,4 +127,7 @@ def test_products_of_many_rows_take_the_tiles_that_were_measured_fastest(sizes):
     assert plan(1800, 3072, 2048, "bfloat16")[0] in ("128x128", "256x128")  # 32 / 40 in halves
     assert plan(640, 17408, 5120, "gated") == ("256x256", 1)                # 231 / 253 on 128 x 128
     assert plan(256, 12288, 4096, "gated") == ("256x128", 1)                # 66 / 78 on 128 x 128
+    # gated products of few tiles: the whole tiles with K in parts
+    assert plan(256, 1024, 4096, "gated") is None and plan(129, 2048, 2048, "gated") is None and plan(512, 768, 2048, "gated") is None
+    assert plan(400, 2048, 2048, "gated") is not None and plan(129, 6912, 2560, "gated") is not None
     assert plan(128, 4096, 4096, "float32") is None and plan(256, 4096, 512, "float32") is None      # for the slices; the tiles
