@@ -70,9 +70,10 @@ __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int parts, in
   *tile_n = first_n + within / rows;
 }
 
-// MODE 0: bfloat16 output, squared behind a ReLU if `form` says so.  1: float32 output, optionally added to what is there; with parts, part p leaves the bare sums of its share
+// MODE 0: bfloat16 output.  1: float32 output, optionally added to what is there; with parts, part p leaves the bare sums of its share
 // of k at c + p M N.  2: gated (the gate as `form` says), bfloat16 output of N columns; W has 2 N rows, gate rows then up rows, and a
-// wave's weight rows are the gate and the up rows of the same outputs.  c_blocked (MODE 0 and 2): the output in blocks of 16 rows.
+// wave's weight rows are the gate and the up rows of the same outputs.  3: as 0, squared behind a ReLU.  c_blocked (MODE 2 and 3): the
+// output in blocks of 16 rows.
 // A tile that sticks out of the matrix repeats its last blocks and stores only what exists; no block of A beyond the last row's is read.
 // K a multiple of 64 per part, so that a part has an even number of steps.
 // KG = 2: two such groups of waves, each with a ring of its own, take half of k each, and the second hands its sums to the first through
@@ -218,12 +219,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          v[i] = MODE == 2 ? gate_mul(acc[x][y][i], acc[x][MODE == 2 ? y + YB / 2 : y][i], form) : form.squared ? relu_squared(acc[x][y][i]) : acc[x][y][i];
+          v[i] = MODE == 2 ? gate_mul(acc[x][y][i], acc[x][MODE == 2 ? y + YB / 2 : y][i], form) : MODE == 3 ? relu_squared(acc[x][y][i]) : acc[x][y][i];
         u32x2_t packed;
         packed[0] = f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
         packed[1] = f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
         *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(c) +
-                                    (c_blocked ? (size_t)bh_blocked_index(row, n, N) : (size_t)row * N + n)) = packed;
+                                    (MODE >= 2 && c_blocked ? (size_t)bh_blocked_index(row, n, N) : (size_t)row * N + n)) = packed;
       }
     }
   }
@@ -335,7 +336,8 @@ int gemm_ring_launch(const void* a, const void* w, void* c, int c_dtype, int acc
              "gemm_ring: only a gated or squared product writes its output in blocks, and N=%d must be a multiple of 32", N);
   if (activation) return launch<2>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);
   if (c_dtype == BH_F32) return launch<1>(tile, 1, a, w, c, M, N, K, accumulate, 0, form, stream);
-  return launch<0>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);
+  if (form.squared) return launch<3>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);
+  return launch<0>(tile, 1, a, w, c, M, N, K, 0, 0, form, stream);
 }
 
 // For tests and measurements: the tiles of 256 rows at a given width of 32 `blocks` weight rows, whatever gemm_ring_plan would choose.

@@ -87,12 +87,12 @@ __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int* tile_n, 
   *tile_n = first_n + within / rows;
 }
 
-// MODE 0: bfloat16 output, squared behind a ReLU if `form` says so.  1: float32 output, optionally added to what is there.  2: SwiGLU (the gate as `form` says), bfloat16 output
+// MODE 0: bfloat16 output.  1: float32 output, optionally added to what is there.  2: SwiGLU (the gate as `form` says), bfloat16 output
 // (N outputs; W has 2 N rows, gate rows then up rows; a wave's weight rows are the gate and the up rows of
-// the same outputs).  YB: blocks of 16 weight rows per wave.
+// the same outputs).  3: as 0, squared behind a ReLU.  YB: blocks of 16 weight rows per wave.
 // A tile that would stick out of the weight rows is moved back inside and stores only what it owns.
 // A's buffer holds whole tiles of 256 rows, and a tile that sticks out below stays where it is and stores only the rows
-// that exist.  c_blocked (MODE 0 and 2): the output lies in blocks of 16 rows.
+// that exist.  c_blocked (MODE 2 and 3): the output lies in blocks of 16 rows.
 template <int MODE, int YB>
 __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ w,
                                                       void* __restrict__ c, int M, int N, int K, int accumulate,
@@ -242,11 +242,11 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
         } else {
           float v[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = form.squared ? relu_squared(acc[x][y][i]) : acc[x][y][i];
+          for (int i = 0; i < 4; ++i) v[i] = MODE == 3 ? relu_squared(acc[x][y][i]) : acc[x][y][i];
           u32x2_t packed;
           packed[0] = f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
           packed[1] = f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
-          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(c) + (c_blocked ? (size_t)bh_blocked_index(row, n, N) : (size_t)row * N + n)) = packed;
+          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(c) + (MODE == 3 && c_blocked ? (size_t)bh_blocked_index(row, n, N) : (size_t)row * N + n)) = packed;
         }
       }
     }
@@ -283,6 +283,7 @@ int gemm_turns_launch(const void* a, const void* w, void* c, int mode, int accum
   BH_REQUIRE(gemm_turns_can(M, N, K, mode, blocks, parts), "gemm_turns: M=%d N=%d K=%d with %d blocks per wave in %d parts of K is not a product this kernel takes", M, N, K, blocks, parts);
   if (mode == 2) launch<2>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
   else if (mode == 1) launch<1>(a, w, c, blocks, M, N, K, accumulate, parts, 0, form, stream);
-  else launch<0>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
+  else if (mode == 3) launch<3>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
+  else launch<0>(a, w, c, blocks, M, N, K, 0, 1, 0, form, stream);
   return bh_check_launch("gemm_turns");
 }
