@@ -257,16 +257,19 @@ class KernelSizes:
                 return _rounded(BlockedRows.padded_rows(rows, block_rows) * width * 2)
         return _rounded(rows * width * act_size)
 
-    def gemm_working_bytes(self, m, n, k, act_size, packed=True, swiglu=False, then_norm=False) -> int:
+    def gemm_working_bytes(self, m, n, k, act_size, packed=True, swiglu=False, then_norm=False, bare=False) -> int:
         """Bytes that `gemm` (or `gemm_swiglu`) of these sizes allocates for the length of the call or returns
         as a prepared norm: partial sums of K in parts, the rows and sums of a norm behind it, a regrouped copy
         of activations that came in another form than the product reads, SwiGLU's two halves where the fused
-        epilogue does not apply."""
+        epilogue does not apply.  `bare`: the product may be left as `PartSums` (`gemm_bare`), also where `gemm` needs no scratch."""
         m, n, k = int(m), int(n), int(k)
         if act_size != 2 or k % 8:
             return _rounded(m * 2 * n * act_size) if swiglu else 0
         sizes = (m, n, k, int(bool(packed)), int(bool(swiglu)))
-        total = _rounded(int(self.lib.bh_gemm_bf16_scratch(*sizes)))
+        scratch = int(self.lib.bh_gemm_bf16_scratch(*sizes))
+        if bare and packed:
+            scratch = max(scratch, int(self.lib.bh_gemm_bf16_bare_parts(m, n, k, 1)) * m * n * 4)
+        total = _rounded(scratch)
         if k % 32 == 0:
             total += 2 * _rounded(BlockedRows.padded_rows(m, 16) * k * 2)      # regrouping: out of blocks, into others
         if then_norm:

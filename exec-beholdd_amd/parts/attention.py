@@ -73,7 +73,7 @@ class GQAAttention:
 
     def working_bytes(self, step) -> int:
         q_width = self.n_heads * self.head_dim
-        total = self.qkv.working_bytes(step, step.rows)
+        total = self.qkv.working_bytes(step, step.rows, bare=True)
         total += step.matrix(step.rows, q_width, reader=self.out.reader_for_plan(step.act_size))     # attended
         total += step.matrix(step.rows, q_width)                                                     # normed, rotated queries
         if step.sizes is not None:

@@ -174,11 +174,11 @@ class StepSize:
         return -(-int(rows) * int(width) * size // 512) * 512
 
     def product(self, rows: int, outputs: int, inputs: int, packed: bool = True, swiglu: bool = False,
-                then_norm: bool = False) -> int:
+                then_norm: bool = False, bare: bool = False) -> int:
         """Bytes that a matrix product of the kernel library allocates beside its output."""
         if self.sizes is None:
             return 0
-        return self.sizes.gemm_working_bytes(rows, outputs, inputs, self.act_size, packed, swiglu, then_norm)
+        return self.sizes.gemm_working_bytes(rows, outputs, inputs, self.act_size, packed, swiglu, then_norm, bare)
 
 
 @dataclass

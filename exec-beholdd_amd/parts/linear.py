@@ -68,12 +68,12 @@ class Linear:
         return ProductReader(self.out_features // 2 if swiglu else self.out_features, swiglu, packed=self.packs(act_size))
 
     def working_bytes(self, step, rows: int, out_size: int | None = None, accumulate: bool = False,
-                      then_norm: bool = False, swiglu: bool = False) -> int:
+                      then_norm: bool = False, swiglu: bool = False, bare: bool = False) -> int:
         """Bytes one product of `rows` rows allocates: its output unless it adds into one, and what the
-        kernel library allocates on the way."""
+        kernel library allocates on the way (`bare`: `forward_bare` may be called in place of `forward`)."""
         outputs = self.out_features // 2 if swiglu else self.out_features
         total = 0 if accumulate else step.matrix(rows, outputs, out_size)
-        return total + step.product(rows, outputs, self.in_features, self.packs(step.act_size), swiglu, then_norm)
+        return total + step.product(rows, outputs, self.in_features, self.packs(step.act_size), swiglu, then_norm, bare)
 
     def prepare(self, kernels):
         """Let the kernel library regroup the matrix into the layout it reads fastest."""

@@ -131,3 +131,18 @@ def test_products_of_many_rows_take_the_tiles_that_were_measured_fastest(sizes):
     assert plan(256, 1024, 4096, "gated") is None and plan(129, 2048, 2048, "gated") is None and plan(512, 768, 2048, "gated") is None
     assert plan(400, 2048, 2048, "gated") is not None and plan(129, 6912, 2560, "gated") is not None
     assert plan(128, 4096, 4096, "float32") is None and plan(256, 4096, 512, "float32") is None      # for the slices; the tiles
+
+
+def test_sums_left_in_parts_are_in_the_byte_plan(sizes):
+    """`gemm_bare` hands out the sums of K's parts, also where the product itself adds up two halves of k and needs no scratch memory:
+    what a projection that may be left in parts is planned with covers them, beside its regrouped activations."""
+    from beholdd.kernels.library import BlockedRows
+    halves = 0
+    for width, outputs in ((1024, 2048), (2048, 4096), (2560, 3584), (4096, 2048), (4096, 6144), (4096, 8192), (5120, 7168)):
+        for m in list(range(129, 1100, 23)) + [1500, 2048, 3000]:
+            parts = sizes.lib.bh_gemm_bf16_bare_parts(m, outputs, width, 1)
+            sums = parts * m * outputs * 4
+            halves += parts == 2 and sizes.lib.bh_gemm_bf16_scratch(m, outputs, width, 1, 0) < sums
+            planned = sizes.gemm_working_bytes(m, outputs, width, 2, bare=True)
+            assert planned >= sums + 2 * BlockedRows.padded_rows(m, 16) * width * 2, (m, outputs, width, parts)
+    assert halves > 0      # sizes among them that scratch memory alone does not cover
