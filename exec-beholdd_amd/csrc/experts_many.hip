@@ -136,18 +136,36 @@ __global__ __launch_bounds__(256, 2) void experts_many_kernel(const uint16_t* __
 #pragma unroll
     for (int y = 0; y < 4; ++y) acc[x][y] = xm_f32x4_t{0.f, 0.f, 0.f, 0.f};
   xm_u32x4_t af[2][XB], wf[2][4];      // the operands of an even and of an odd step
-  // the first two units and half of the third, and four steps of weights; what follows is asked for as places become free
-  for (int unit = 0; unit < 3 && unit < units; ++unit)
+  // The first two units and half of the third, and four steps of weights; what follows is asked for as places become free.  In the order
+  // of their use, so that the first step waits for its own only.
+  auto ask_unit = [&](int unit) {
 #pragma unroll
     for (int b = 0; b < AL; ++b) {
       ask_rows(b, 0, unit, unit);
       if (unit < 2) ask_rows(b, 1, unit, unit);
     }
-  for (int j = 0; j < STEPS && j < steps; ++j) {
+  };
+  auto ask_step = [&](int step) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) ask_weights(b, j);
+    for (int b = 0; b < 2; ++b) ask_weights(b, step);
+  };
+  ask_unit(0);
+  ask_step(0);
+  ask_step(1);
+  if (units >= 3) {
+    ask_unit(1);
+    ask_step(2);
+    ask_unit(2);
+    ask_step(3);
+    XM_WAIT(2 + 2 * AL + 2 + AL + 2);
+  } else {
+    if (units == 2) {
+      ask_unit(1);
+      ask_step(2);
+      ask_step(3);
+    }
+    XM_WAIT(0);
   }
-  XM_WAIT(0);
   XM_MEET();
   const int r = lane % 16, read_at = (r / 8) * 64 + (r % 8) * 8 + ((lane / 16) ^ (r % 8) ^ (r / 8));     // ^ 4 for a unit's second step
 #pragma unroll
