@@ -18,6 +18,7 @@
 // 290 / 170 (372 / 210).  8 experts, width 4,096, ff 4,096, 1,024 pairs 573 / 305 (748 / 405), 0.96 and 0.90 PFLOP/s.  The registers
 // in turn without the whole lines: 112 / 75 at the first size.
 #include "common.h"
+#include <cmath>
 #include <type_traits>
 
 typedef __bf16 xm_bf16x8_t __attribute__((ext_vector_type(8)));
@@ -251,6 +252,27 @@ __global__ __launch_bounds__(256, 2) void experts_many_kernel(const uint16_t* __
 #undef XM_WAIT
 #undef XM_MEET
 
+// Whether tiles of 128 pairs are the faster ones.  They read the weights half as often as tiles of 64, and a compute unit that has one of
+// either takes 1.12 times as long for it; one that has two takes 1.3 times as long as for one.  So it is the rounds of two a compute
+// unit that decide, at as many tiles an expert as the average lets expect (counts differ: from about 0.81 of a tile on some experts
+// need one more, behind that half a tile more).  Gate and up + down, tiles of 64 / 128, us, 32 experts: width 1,024, ff 384 at 56 pairs
+// 25.5 / 27.5, at 80 27.9 / 28.5, at 128 33.7 / 39.0, at 192 44.7 / 40.2; width 2,048, ff 768 at 48 70.5 / 76.0, at 56 46.8 + 29.0 /
+// 51.1 + 24.1, at 64 89.2 / 77.2, at 128 112 / 115; width 4,096, ff 1,536 at 56 264 / 251, at 96 316 / 268.
+// With more tiles than places and k of 4,096 the weights' way from memory is the time, and the wider tiles' steps hide more of it: 16
+// pairs 158 / 149 (768 tiles), where 128 experts of 2,048 x 768 take 146 / 148 (1,536).
+bool tiles_of_128(int pairs, int E, int K, int n_tiles) {
+  const double units = bh_compute_units(), average = (double)pairs / E;
+  const auto tiles = [&](int size) {
+    const double q = average / size, spill = 0.81;
+    return (double)E * n_tiles * (q <= spill ? 1.0 : q < 1.0 ? 1.0 + 0.5 * (q - spill) / (1.0 - spill) : q + 0.5);
+  };
+  const auto time = [&](double count) {
+    const double r = count / units, full = std::floor(r / 2.0), rest = r - 2.0 * full;
+    return 1.3 * full + (rest < 0.02 ? 0.0 : rest <= 1.0 ? 1.0 : 1.3);
+  };
+  return (K >= 4096 && (double)E * n_tiles > 2.0 * units) || 1.12 * time(tiles(128)) < time(tiles(64));
+}
+
 template <bool GATED, int XB>
 int launch(const void* in, int in_div, const int32_t* list, int capacity, const int32_t* counts, const void* w, void* out, int pairs, int E,
            int K, int N, float limit, float alpha, float shift, const float* in_weights, hipStream_t stream) {
@@ -267,6 +289,10 @@ int launch(const void* in, int in_div, const int32_t* list, int capacity, const 
 }  // namespace
 
 // As bh_experts_tiles; `pairs`: how many pairs all experts have together at most (identity experts' may be missing from the lists).
+// For tests: the pairs of a tile.
+extern "C" int bh_experts_many_tile(int pairs, int E, int K, int N, int gated) {
+  return pairs > 0 && E > 0 && N > 0 && tiles_of_128(pairs, E, K, gated ? (N + 63) / 64 : (N + 127) / 128) ? 128 : 64;
+}
 extern "C" int bh_experts_many(const void* in, int in_div, const int32_t* list, int capacity, const int32_t* counts, const void* w, void* out,
                                int pairs, int E, int K, int N, int gated, float limit, float alpha, float shift, const float* in_weights,
                                hipStream_t stream) {
@@ -274,10 +300,7 @@ extern "C" int bh_experts_many(const void* in, int in_div, const int32_t* list, 
              "experts_many: K must be a multiple of 64 and N of 16, got %d and %d", K, N);
   BH_REQUIRE(((uintptr_t)in | (uintptr_t)w | (uintptr_t)out) % 16 == 0, "experts_many: operands must be 16-byte aligned");
   BH_REQUIRE(gated || in_weights == nullptr, "experts_many: weights on the input go with the gated product");
-  // Tiles of 128 pairs read the weights half as often as tiles of 64, which leave less of a last tile empty.  Gate and up,
-  // tiles of 64 / 128, us: width 2,048 at 48 pairs an expert 48 / 52, at 64 58 / 52, at 96 64 / 55, at 128 68 / 73, at 192 87 / 76;
-  // width 4,096 at 48 155 / 162, at 64 182 / 160, at 96 198 / 166; width 1,024 at 48 15 / 18, at 64 18 / 18, at 96 17 / 18, at 192 26 / 24.
-  const bool wide = (long)pairs >= 56L * E;
+  const bool wide = tiles_of_128(pairs, E, K, gated ? (N + 63) / 64 : (N + 127) / 128);
 #define BH_XM(GATED, XB) launch<GATED, XB>(in, in_div, list, capacity, counts, w, out, pairs, E, K, N, limit, alpha, shift, in_weights, stream)
   if (gated) return wide ? BH_XM(true, 4) : BH_XM(true, 2);
   return wide ? BH_XM(false, 4) : BH_XM(false, 2);

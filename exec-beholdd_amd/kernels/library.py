@@ -219,6 +219,7 @@ class KernelSizes:
             "bh_experts_tiles": [p, i, p, i, p, p, p, i, i, i, i, f, f, f, p, p],
             "bh_experts_tiles_takes": [i, i],
             "bh_experts_many": [p, i, p, i, p, p, p, i, i, i, i, i, f, f, f, p, p],
+            "bh_experts_many_tile": [i, i, i, i, i],
             "bh_experts_gather": [p, i, i, p, i, p, p, p, p, i, i, i, p, p],
             "bh_gla_scan": [p, i, i, i, i, i, p, i, p, f, f, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, p],
             "bh_gla_chunk_rows": [i, i, i, i, i],

@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 # pairs an expert: none, one, a tile's edges (64 and 128), several tiles; experts: one, more than a wave's lanes; outputs: less than
-# a tile's, remainders of one; the average decides between tiles of 64 pairs (below 56) and of 128; widths of 1 to 5, 7, 12 and 32 units
-# of 64 k, the ring of three units among them
+# a tile's, remainders of one; widths of 1 to 5, 7, 12 and 32 units of 64 k, the ring of three units among them; so few workgroups run on
+# tiles of 64 pairs
 @pytest.mark.parametrize("counts,width,ff", [([1], 64, 64), ([64, 0, 65, 1], 128, 192), ([0, 63, 127, 0, 30], 192, 64), ([300], 64, 128),
                                              ([128, 129, 127, 257, 0], 256, 64), ([0] * 69 + [200, 3] + [0] * 5 + [40], 64, 64),
                                              ([150] * 66, 64, 64), ([97, 512], 2048, 768),
@@ -48,6 +48,17 @@ def test_experts_of_many_pairs(K, counts, width, ff, weighed):
         assert float(((got_inner[rows] - want).abs() - 2.0 ** -8 * want.abs()).max()) < 1e-4, e
         want = got_inner[rows] @ down[e].double().T
         assert float((got[rows] - want).abs().max()) < 2.0 ** -24 * (ff + 8) * float((got_inner[rows].abs() @ down[e].double().abs().T).max()), e
+
+
+# more workgroups than a round holds, on tiles of 128 pairs: one beyond and one short of a tile, empty and lone ones; 1, 2, 3, 5 and 7 units
+# of 64 k on either product
+@pytest.mark.parametrize("repeats,width,ff,both", [(9, 64, 512, False), (9, 128, 576, False), (9, 192, 512, False), (9, 320, 448, True),
+                                                   (18, 448, 320, True), (20, 320, 64, True), (20, 320, 128, True), (20, 384, 192, True)])
+def test_experts_of_many_pairs_in_tiles_of_128(K, repeats, width, ff, both):
+    counts = [130, 5, 64, 128, 129, 257, 0, 127] * repeats
+    assert K.lib.bh_experts_many_tile(sum(counts), len(counts), width, ff, 1) == 128
+    assert not both or K.lib.bh_experts_many_tile(sum(counts), len(counts), ff, width, 0) == 128
+    test_experts_of_many_pairs(K, counts, width, ff, False)
 
 
 def test_experts_of_many_pairs_take_rows_shared_by_choices(K):

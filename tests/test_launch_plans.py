@@ -146,3 +146,14 @@ def test_sums_left_in_parts_are_in_the_byte_plan(sizes):
             planned = sizes.gemm_working_bytes(m, outputs, width, 2, bare=True)
             assert planned >= sums + 2 * BlockedRows.padded_rows(m, 16) * width * 2, (m, outputs, width, parts)
     assert halves > 0      # sizes among them that scratch memory alone does not cover
+
+
+def test_experts_tiles_of_pairs_follow_the_rounds(sizes):
+    """Pairs of a tile of the routed experts' products: where both widths were timed (32 experts unless said)."""
+    gate_up = lambda pairs, width, ff, experts=32: sizes.lib.bh_experts_many_tile(pairs * experts, experts, width, ff, 1)
+    down = lambda pairs, width, ff, experts=32: sizes.lib.bh_experts_many_tile(pairs * experts, experts, ff, width, 0)
+    assert [gate_up(n, 1024, 384) for n in (16, 48, 56, 128)] == [64] * 4 and gate_up(192, 1024, 384) == 128
+    assert [gate_up(n, 2048, 768) for n in (16, 48, 56)] == [64] * 3 and [gate_up(n, 2048, 768) for n in (64, 96, 192)] == [128] * 3
+    assert down(48, 2048, 768) == 64 and down(56, 2048, 768) == 128
+    assert [gate_up(n, 4096, 1536) for n in (16, 96, 256)] == [128] * 3
+    assert gate_up(56, 2048, 1408, 8) == 64 and gate_up(64, 2048, 1408, 8) == 128 and gate_up(40, 2048, 768, 128) == 64
