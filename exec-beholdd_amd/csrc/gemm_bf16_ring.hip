@@ -286,13 +286,10 @@ int launch(int tile, int parts, const void* a, const void* w, void* c, int M, in
 
 }  // namespace
 
-// The tile and the parts of K with the least of the estimate above.  Up to 256 rows, and for short K there, a norm may ride on the
-// product (gemm_bf16.hip), which this kernel does not carry; up to 128 rows the kernel of gemm_bf16_slices.hip is the faster one.
-RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
+// The tile and the parts of K with the least of the estimate above.
+static RingPlan best_plan(int M, int N, int K, RingOutput output) {
   RingPlan plan = {-1, 1};
   const int W = output == RING_GATED ? 2 * N : N;
-  if (layout != 1 || M <= 128 || N % 16 != 0 || K % 64 != 0 || K < 128 || N < 128) return plan;
-  if (M <= 256 && (K < 1024 || W < 1024)) return plan;
   for (int tile = 0; tile < RING_TILES; ++tile) {
     if (tile == RING_128x128_HALVES && (K % 128 != 0 || K < 512)) continue;
     const int mode = output == RING_GATED ? 2 : output == RING_F32 ? 1 : 0, blocks = tile == RING_256x256 ? 8 : 6;
@@ -307,6 +304,23 @@ RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
     }
   }
   return plan;
+}
+
+// Up to 256 rows, for short K or few outputs there, a norm may ride on the product (gemm_bf16.hip), which this kernel does not carry; up
+// to 128 rows the kernel of gemm_bf16_slices.hip is the faster one.
+// A product asks for its plan several times and a model for the same few over and over; a search takes 0.3 us of the host, which is what
+// bounds a step of few rows.  So a thread keeps the last plans it was asked for.
+RingPlan gemm_ring_plan(int M, int N, int K, int layout, RingOutput output) {
+  if (layout != 1 || M <= 128 || N % 16 != 0 || K % 64 != 0 || K < 128 || N < 128) return {-1, 1};
+  if (M <= 256 && (K < 1024 || (output == RING_GATED ? 2 * N : N) < 1024)) return {-1, 1};
+  struct Kept {
+    int M, N, K, output;
+    RingPlan plan;
+  };
+  static thread_local Kept kept[64] = {};
+  Kept& one = kept[((unsigned)M * 31u + (unsigned)(N / 16) * 17u + (unsigned)(K / 64) * 7u + (unsigned)output) % 64];
+  if (one.M != M || one.N != N || one.K != K || one.output != output) one = {M, N, K, output, best_plan(M, N, K, output)};
+  return one.plan;
 }
 
 RingPlan gemm_ring_bare_plan(int M, int N, int K, int layout) {
