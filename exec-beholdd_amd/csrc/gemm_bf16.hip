@@ -619,14 +619,15 @@ __global__ __launch_bounds__(256) void gemm_parts_finish_kernel(const float* __r
 // ---- tiled -----------------------------------------------------------------------------------
 
 // The same for a product that completes the float32 residual right before an RMSNorm reads it, with many rows
-// (the parts come from the kernel for many rows, gemm_bf16_ring.hip): a block owns eight whole rows, so it can finish
-// the norm itself and the norm needs no launch and no second pass over the residual.  Lane l of wave w has row
-// l % 8 of the block's rows and the pieces of eight columns 8 w + l / 8, + 128, ... (here of 8 rows and 16 waves): a wave reads 256 contiguous
-// bytes of each of its rows and writes 128 contiguous bytes of the norm's output per row, or, with
+// (the parts come from the kernel for many rows, gemm_bf16_ring.hip): a block owns ROWS whole rows, so it can finish
+// the norm itself and the norm needs no launch and no second pass over the residual.  With eight rows and 16 waves,
+// lane l of wave w has row l % 8 of the block's rows and the pieces of eight columns 8 w + l / 8, + 128, ...: a wave
+// reads 256 contiguous bytes of each of its rows and writes 128 contiguous bytes of the norm's output per row, or, with
 // normed_blocked (the output in blocks of 16 rows x 32 columns, bh_blocked_index, for a product that reads it
 // that way), the 128 bytes that eight rows' pieces of the same columns fill there.  The parts are added in their
-// order, then the residual's old values, as the kernel above does; a row's sum of squares is added up in an
-// order that depends on the width only.
+// order, then the residual's old values, as the kernel above does.  A row's sum of squares is added up in an order
+// that depends on the width and on ROWS, and so on the number of rows (bh_gemm_bf16_then_norm, where a product
+// without parts leaves the norm to bh_rmsnorm): in another step the same row's norm may end in another last bit.
 #define FINISH_NORM_PIECES 8   // pieces of eight columns per thread: rows of up to 8,192
 typedef uint32_t finish_u32x4_t __attribute__((ext_vector_type(4)));
 template <int PARTS, int ROWS, int ROW_WAVES>   // PARTS: at least `parts`, what the loop over them is unrolled to; ROWS per block, ROW_WAVES waves each

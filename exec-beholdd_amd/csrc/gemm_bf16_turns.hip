@@ -24,15 +24,6 @@
 // matrix cores' power sets the clock, and taking turns is the more frugal way (8,160 rows, us here / there: gate and up of 12,288 x 4,096
 // 1,170 / 1,235, 4,096 x 12,288 551 / 585, 6,144 x 4,096 293 / 303; 2,048 x 8,192 x 2,048 56 / 58); with narrower tiles, which wait for their
 // operands more than for the matrix cores, the ring wins (256 x 128 at 2,048 x 4,096 x 4,096: 84 / 63).
-// What bounds it (activations in rows): the loads alone (no multiplies) take 0.9 of the whole kernel's time, the
-// multiplies alone 0.6, the multiplies with their operand reads from LDS 0.8 (1.46 to 1.58 PFLOP/s).  It is not the loads' latency (five or six steps in LDS instead of four changed nothing; touching the
-// lines three slices ahead with 4-byte loads made it slower, 0.9 PFLOP/s for gate/up: loads retire in order, so
-// the loads for LDS waited behind the touches), not LDS (a compute unit reads 256 bytes per clock from it and
-// needs a third of that) and not memory beyond L2 (87 % of the L2 requests hit; 0.3 to 0.6 GB come from beyond
-// it).  The 32 compute units of an XCD ask its L2 for 1 MB per step, which at the matrix cores' full speed
-// would be all that its 16 channels of 64 bytes per clock can give; a compute unit alone gets at most about
-// 43 bytes per clock out of L1 and L2 (loads only, to LDS or to registers alike), and a tile of 256 x 128 asks
-// for 47 where 256 x 256 asks for 32, which is why the narrower tiles lose.
 #include "gemm_bf16_turns.h"
 #include <type_traits>
 

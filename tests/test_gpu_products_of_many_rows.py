@@ -19,11 +19,11 @@ def rel(got, want):
     return float((got - want).abs().max() / want.abs().max())
 
 
-# rows, weight rows and k one beyond and one short of whole tiles, of whole steps in the ring (64 k are two), of parts and halves of K
-SIZES = [(129, 1024, 1024), (129, 1040, 1088), (256, 1024, 1152), (257, 128, 128), (257, 144, 192), (383, 1008, 320),      # few tiles
-         (2049, 2064, 1088), (2049, 2032, 1152), (2048, 2048, 2048),                                                      # 128 x 128, whole K and in halves
-         (2096, 3088, 512), (2047, 4096, 640), (1025, 4112, 256),                                                         # 256 x 128
-         (2049, 6128, 256), (251, 5120, 2048), (140, 7168, 1280), (700, 6160, 2048), (8193, 4080, 128)]                   # 256 rows, and parts of K
+# rows, weight rows and k one beyond and one short of whole tiles, of whole steps in the ring (64 k are two), of parts of K; which tiles
+# they run on is an estimate's choice (`test_every_tile_and_cut_of_the_products_of_many_rows` holds sizes to theirs)
+SIZES = [(129, 1024, 1024), (129, 1040, 1088), (256, 1024, 1152), (257, 128, 128), (257, 144, 192), (383, 1008, 320),
+         (2049, 2064, 1088), (2049, 2032, 1152), (2048, 2048, 2048), (2096, 3088, 512), (2047, 4096, 640), (1025, 4112, 256),
+         (2049, 6128, 256), (251, 5120, 2048), (140, 7168, 1280), (700, 6160, 2048), (8193, 4080, 128)]
 
 
 @pytest.mark.parametrize("m,n,k", SIZES)
@@ -75,6 +75,74 @@ def test_products_of_many_rows_and_the_norm_behind_them(K, m, n, k):
     got = residual.double()
     want = got / torch.sqrt((got ** 2).mean(-1, keepdim=True) + 1e-5) * weight.double()
     assert rel(K.from_blocked(normed) if isinstance(normed, BlockedRows) else normed, want.cpu()) < 4e-3
+
+
+TILES = ["128x128", "128x128 in halves", "256x128", "256x192", "256x256"]
+
+
+def plan(K, m, n, k, output):
+    """(tile, parts of K) on the kernel for many rows; `output`: float32, gated or bfloat16."""
+    code = int(K.lib.bh_gemm_bf16_plan(m, n, k, 1, ["float32", "gated", "bfloat16"].index(output)))
+    return (TILES[code // 16], code % 16) if code >= 0 else None
+
+
+# every tile with K whole and in parts, where it is compiled for that output, at sizes that no tile divides; the plan is asserted, so that
+# another estimate cannot empty this
+@pytest.mark.parametrize("output,tile,parts,m,n,k", [
+    ("float32", "128x128", 1, 257, 144, 128), ("float32", "128x128", 2, 257, 144, 512), ("float32", "128x128 in halves", 1, 257, 8208, 3072),
+    ("float32", "256x128", 1, 385, 8208, 128), ("float32", "256x128", 4, 129, 4112, 2048), ("float32", "256x192", 1, 900, 8208, 128),
+    ("float32", "256x192", 4, 129, 8208, 4096), ("float32", "256x256", 1, 1300, 8208, 128), ("float32", "256x256", 5, 257, 6160, 5120),
+    ("gated", "128x128", 1, 257, 144, 128), ("gated", "128x128 in halves", 1, 129, 5136, 3072), ("gated", "256x128", 1, 257, 6160, 128),
+    ("gated", "256x192", 1, 385, 8208, 128), ("gated", "256x256", 1, 257, 12304, 128),
+    ("bfloat16", "128x128", 1, 257, 144, 128), ("bfloat16", "128x128", 4, 257, 144, 1024), ("bfloat16", "128x128 in halves", 1, 520, 4112, 3072),
+    ("bfloat16", "256x128", 1, 385, 8208, 128), ("bfloat16", "256x128", 4, 129, 6160, 1024), ("bfloat16", "256x192", 1, 900, 8208, 128),
+    ("bfloat16", "256x192", 4, 129, 8208, 2048), ("bfloat16", "256x256", 1, 1300, 8208, 128), ("bfloat16", "256x256", 3, 385, 8208, 1536)])
+def test_every_tile_and_cut_of_the_products_of_many_rows(K, output, tile, parts, m, n, k):
+    """From activations whose buffer holds NaN behind the last row; the bounds are those of `test_products_of_many_rows`."""
+    from beholdd.kernels.library import BlockedRows
+    assert plan(K, m, n, k, output) == (tile, parts)
+    g = torch.Generator(device="cuda:0").manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g, device="cuda:0").to(torch.bfloat16)
+    w = (torch.randn((2 if output == "gated" else 1) * n, k, generator=g, device="cuda:0") * 0.05).to(torch.bfloat16)
+    in_blocks = BlockedRows(torch.full((BlockedRows.padded_rows(m, 16) * k,), float("nan"), dtype=torch.bfloat16, device="cuda:0"), m, k)
+    K.to_blocked(a, in_blocks)
+    want = a.double() @ w[:n].double().t()
+    if output == "gated":
+        want = want / (1 + torch.exp(-want)) * (a.double() @ w[n:].double().t())
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+        K.gemm_swiglu(in_blocks, K.pack_weight(w), out)
+        assert rel(out, want.cpu()) < 6e-3
+        return
+    base = torch.randn(m, n, generator=g, device="cuda:0")
+    out = base.clone() if output == "float32" else torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    K.gemm(in_blocks, K.pack_weight(w), out, accumulate=output == "float32")
+    if output == "float32":
+        assert rel(out, (want + base.double()).cpu()) < 4 * math.sqrt(k) * 2.0 ** -24
+    else:
+        assert rel(out, want.cpu()) < 4e-3
+
+
+# the kernel that adds up the parts and finishes the norm, with one, two, four and eight rows a block, for up to two, four and eight parts
+@pytest.mark.parametrize("m,n,k,parts", [(257, 192, 512, 2), (257, 192, 768, 3), (333, 4096, 12288, 4), (257, 192, 1536, 6),
+                                         (520, 192, 512, 2), (520, 192, 768, 3), (520, 192, 1536, 6), (2049, 192, 512, 2), (2049, 192, 768, 3),
+                                         (2049, 128, 1536, 6), (2056, 2048, 6144, 3), (4097, 192, 768, 2), (4097, 192, 1536, 3), (4097, 192, 5120, 5)])
+@pytest.mark.parametrize("blocked", [False, True])
+def test_norm_finished_from_parts_with_every_number_of_rows_a_block(K, m, n, k, parts, blocked):
+    """The residual as without the norm bit for bit; the norm within a bfloat16 rounding of float64's, in rows and in its reader's blocks."""
+    from beholdd.kernels.library import BlockedRows
+    from beholdd.parts.base import NormRequest, ProductReader
+    assert plan(K, m, n, k, "float32")[1] == parts
+    g = torch.Generator(device="cuda:0").manual_seed(m + k)
+    a = torch.randn(m, k, generator=g, device="cuda:0").to(torch.bfloat16)
+    packed = K.pack_weight((torch.randn(n, k, generator=g, device="cuda:0") / k ** 0.5).to(torch.bfloat16))
+    base, weight = torch.randn(m, n, generator=g, device="cuda:0"), 1 + 0.3 * torch.randn(n, generator=g, device="cuda:0")
+    without, residual = base.clone(), base.clone()
+    K.gemm(a, packed, without, accumulate=True)
+    normed = K.gemm(a, packed, residual, accumulate=True, then_norm=NormRequest(weight, 1e-5, ProductReader(4096) if blocked else None))
+    assert torch.equal(without, residual) and isinstance(normed, BlockedRows) == blocked
+    got = residual.double()
+    want = got / torch.sqrt((got ** 2).mean(-1, keepdim=True) + 1e-5) * weight.double()
+    assert rel(K.from_blocked(normed) if blocked else normed, want.cpu()) < 4e-3
 
 
 # few rows (blocks of 8 and of 16, one and two blocks of rows), 33 to 128 rows and spans of 24 weight rows (two launches), many rows on
