@@ -3,7 +3,7 @@
 // kernel (generic.hip); only the order of the sums differs, and it is blocked here as there.
 //
 // Three kernels.  Up to 32 rows (decode steps, short steps) a product is its weights, read once: `gemm_f32_few`, gated or not.  More rows are
-// matrix-core work: `gemm_f32_ring` where K is a multiple of 32, else `gemm_f32_tiles`; gated products are followed by an activation of
+// matrix-core work: `gemm_f32_ring` where K is a multiple of 32 and not short, else `gemm_f32_tiles`; gated products are followed by an activation of
 // their own.
 #include "common.h"
 #include "gemm_f32.h"
@@ -382,7 +382,13 @@ int bh_gemm_f32(const float* a, const float* w, float* c, int accumulate, int M,
     else few_rows<1, false>(a, w, c, M, N, K, accumulate, none, stream);
     return bh_check_launch("gemm_f32_few");
   }
-  if (K % 32 == 0 && (M + 31) / 32 <= 65535) {
+  // Few slices in more than one round: a workgroup of the ring pays for its start (three slices asked for, the shares' sums) what it saves
+  // behind it, and the tiles are ahead where they are not the wide ones.  Ring / tiles, us: 4,096 rows of 1,024 x 32 11.6 / 9.8, x 128
+  // 22.4 / 19.7, x 192 26.6 / 25.7, x 256 29.4 / 30.4; 600 of 4,096 x 128 18.4 / 13.8, x 192 21.3 / 17.8; 1,500 of 1,024 x 64 10.0 / 7.9; one
+  // round, 1,000 of 1,024 x 64 6.4 / 6.4, 300 of 1,024 x 128 6.2 / 7.1; wide ones, 4,096 of 4,096 x 128 64 / 83.
+  const long wide = (long)((N + 127) / 128) * ((M + 127) / 128);      // tiles of 128 x 128
+  const bool short_k = K < 256 && (long)((N + 63) / 64) * ((M + 63) / 64) > units && wide < 4L * units;
+  if (K % 32 == 0 && !short_k && (M + 31) / 32 <= 65535) {
     // The waves' split with the least estimated time: rounds of workgroups, one a compute unit at a time (two share it and take as long),
     // of so many slices at what a slice takes, and the start; a smaller tile has to be 5 % ahead, for it reads more.  64 x 64 / 32 x 64 /
     // 32 x 32 outputs, us, weights from memory (1 to 3 % less than now, before the sums of even and odd steps were kept apart), in
@@ -393,8 +399,8 @@ int bh_gemm_f32(const float* a, const float* w, float* c, int accumulate, int M,
     const auto rounds = [&](int rows, int columns) {
       return (double)(((long)((M + rows - 1) / rows) * ((N + columns - 1) / columns) + units - 1) / units);
     };
-    const double whole = rounds(64, 64) * (K / 32) * 0.58 + 4.0;
-    const double in_two = K % 64 ? 1e30 : rounds(32, 64) * (K / 64) * 0.64 + 4.0;
+    const double whole = rounds(64, 64) * ((K / 32) * 0.58 + 1.0) + 3.0;
+    const double in_two = K % 64 ? 1e30 : rounds(32, 64) * ((K / 64) * 0.64 + 1.0) + 3.0;
     const double in_four = K % 128 ? 1e30 : rounds(32, 32) * ((K / 128) * 0.75 + 4.0);
 #define BH_F32_RING(WM, WN, KG, R)                                                                                                 \
   do {                                                                                                                             \
@@ -408,12 +414,11 @@ int bh_gemm_f32(const float* a, const float* w, float* c, int accumulate, int M,
     BH_F32_RING(2, 2, 1, 3);
 #undef BH_F32_RING
   }
-  // Other K.
+  // Other K, and those few slices.
   // Tiles of 128 x 128 read half as much a product, but only four of them a compute unit and more level out (695 x 6,144 x 1,024,
   // 1.1 a unit: 141 us, 104 in tiles of 64 x 64); where tiles of 64 x 64 are not even two a unit, a second group of waves hides the
   // first one's waits for its slices.
-  const long units4 = 4L * units, wide = (long)((N + 127) / 128) * ((M + 127) / 128);
-  const bool big = wide >= units4;
+  const bool big = wide >= 4L * units;
   const int tile = big ? 128 : 64;
   BH_REQUIRE((M + tile - 1) / tile <= 65535, "gemm: M=%d needs more than 65535 row tiles", M);
   const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile);

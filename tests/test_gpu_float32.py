@@ -50,6 +50,12 @@ def test_float32_products_in_a_ring_of_slices(K, m, n, k):
     assert bool(((summed.cpu().double() - want - c).abs() <= product_bound(a, w, k) + 2.0 ** -24 * (want.abs() + c.abs() + 1)).all())
 
 
+# more than a round of workgroups, K shorter than 256 (tiles) and from 256 on (slices), where the tiles' wide form is ahead of neither
+@pytest.mark.parametrize("m,n,k", [(1100, 1100, 32), (1100, 1100, 224), (2049, 1025, 256), (600, 4100, 256), (1100, 2100, 288), (4100, 4097, 96)])
+def test_float32_products_on_both_sides_of_short_k(K, m, n, k):
+    test_float32_products_in_a_ring_of_slices(K, m, n, k)
+
+
 @pytest.mark.parametrize("gate", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("m,width,k", [(1, 3, 8), (4, 96, 128), (7, 4097, 68), (20, 40, 2304), (32, 8, 60), (33, 72, 64)])
 def test_float32_gated_products(K, m, width, k, gate):
