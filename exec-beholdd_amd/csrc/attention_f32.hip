@@ -13,6 +13,7 @@
 // 41 us in waves of their own (30 in tiles of columns, see there), 94 in workgroups of four waves on four rows, 120 there.
 #include "common.h"
 #include <algorithm>
+#include <cmath>
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
@@ -422,30 +423,37 @@ __global__ __launch_bounds__(256, P <= 4 ? 2 : 1) void attention_f32_tiles_kerne
 // Whether a step of prompts goes in tiles.  A tile walks its sequences one after another, a page of a sequence after the other, where
 // the walk above has every row's pages in waves of their own: rows of several sequences that look far back, one behind the other in a
 // tile, are a chain of all their pages (a prompt of 512 rows beside 14 rows behind 1,000 keys, 8 heads of 128 on 4: 138 us, 406 in
-// tiles), and it may begin when all other tiles are done.  So the longest such chain, at what a page of it takes (1.5 us a page of a
-// head of 32, 2.05 of 64, 3.2 of 128, 5.4 of 256), has to fit in what the tiles save of the walk's time for all rows' pages together.
-// That is SAVED, ns a row, head and page (the walk's four waves share a row's pages, so that 1.5 more are waited for on average), from
-// 2,048 rows alone, walk / tiles, us: 16 heads of 32 200 / 115, of 64 345 / 205; 8 heads of 96 544 / 174, 128 724 / 217, 160 651 / 287,
-// 192 1,296 / 330, 224 1,634 / 355, 256 1,376 / 398.
+// tiles).  So both times are estimated, each from its longest chain of pages and from all its pages together (us a page of the chain; ns
+// a compute unit and page of a tile, ns a row, head and page of the walk, whose four waves share a row's pages, so that 1.5 more are
+// waited for on average; they add as squares do).  Fitted to 304 steps of 1 to 13 sequences, prompts alone, behind up to 3,000 keys and
+// beside decoding rows behind up to 4,000, of 16 head counts and sizes, to 13 % (tiles) and 17 % (walk): with 15 % asked of the tiles
+// the choice takes 0.2 % longer than the better one on average, and one step of the 304 was 9 % slower than walked.
 // `start` and `past`: the step's sequences as the host knows them, or null: then the average is all there is to go by.
 bool tiles_pay(int n_rows, int n_seqs, int H, int KVH, int hd, int span, const int32_t* start, const int32_t* past) {
   if (n_rows < 32 * n_seqs || (long)n_rows * H <= 8L * bh_compute_units() || KVH > 65535) return false;
   if (!start || !past) return true;
+  constexpr double TILE_PAGE[8] = {0.8, 1.6, 2.4, 2.9, 5.4, 6.5, 6.8, 7.8}, WALK_PAGE[8] = {0.43, 0.75, 2.44, 3.49, 3.13, 6.6, 8.88, 5.6};
   const int group = H / KVH, seen = span ? (span > 0 ? span : -span) / BH_PAGE + 2 : 0x7fffffff;      // pages that a window or chunk touches
-  double row_pages = 0.;
-  long chain = 0, tile = -1, walked = 0;      // the tile that the sequences so far end in, and the pages it walks for them
+  double row_pages = 0., tile_pages = 0.;
+  long chain = 0, tile = -1, walked = 0, most = 0;      // tile: the one that the sequences so far end in; walked: the pages it walks for them
   for (int s = 0; s < n_seqs; ++s) {
-    const int rows = start[s + 1] - start[s], pages = std::min((past[s] + rows - 1) / BH_PAGE + 1, seen);
+    const int rows = start[s + 1] - start[s];
     if (rows <= 0) continue;
-    row_pages += rows * (0.5 * (std::min(past[s] / BH_PAGE + 1, seen) + pages) + 1.5);
+    const int pages = std::min((past[s] + rows - 1) / BH_PAGE + 1, seen);
+    const double average = 0.5 * (std::min(past[s] / BH_PAGE + 1, seen) + pages);
     const long first = (long)start[s] * group / 16, last = ((long)start[s + 1] * group - 1) / 16;
+    row_pages += rows * (average + 1.5);
+    tile_pages += (double)(last - first + 1) * average;
     walked = (first == tile ? walked : 0) + pages;
     chain = std::max(chain, walked);
+    most = std::max(most, (long)pages);
     if (last != first) walked = pages;
     tile = last;
   }
-  constexpr double SAVED[8] = {0.15, 0.27, 1.2, 1.7, 1.2, 3.2, 4.2, 3.3};
-  return chain * (1.0 + hd / 58.) <= 1e-3 * SAVED[hd / 32 - 1] * row_pages * H + 12.0;
+  const int size = hd / 32 - 1;
+  const double in_tiles = 6.0 + std::hypot(chain * (0.67 + 0.018 * hd), tile_pages * KVH * TILE_PAGE[size] / bh_compute_units());
+  const double by_rows = 18.0 + std::hypot((0.25 * most + 1.0) * 0.049 * hd, 1e-3 * row_pages * H * WALK_PAGE[size]);
+  return 1.15 * in_tiles <= by_rows;
 }
 
 template <int P>
