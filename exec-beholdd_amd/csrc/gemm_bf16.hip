@@ -1588,13 +1588,12 @@ extern "C" int bh_gemm_bf16_finishes_norm(int M, int N, int K, int layout) {
 }
 extern "C" int bh_gemm_bf16_then_norm(const void* a, const void* w, float* residual, int M, int N, int K, int layout,
                                       const void* norm_weight, int norm_weight_dtype, float eps, void* normed,
-                                      void* scratch, int a_blocked, int normed_blocked, hipStream_t stream) {
+                                      void* scratch, int normed_blocked, hipStream_t stream) {
   BH_REQUIRE(bh_gemm_bf16_finishes_norm(M, N, K, layout),
              "gemm_bf16_then_norm: a product of M=%d N=%d K=%d does not finish a norm (bh_gemm_bf16_finishes_norm)", M, N, K);
   const RingPlan ring = many_rows_plan(M, N, K, layout, RING_F32);
   const int parts = ring.parts;
   BH_REQUIRE(a && w && residual && norm_weight && normed && (scratch || parts == 1), "gemm_bf16_then_norm: every operand is needed");
-  BH_REQUIRE(a_blocked, "gemm_bf16_then_norm: the activations lie in blocks of 16 rows");
   BH_REQUIRE(norm_weight_dtype == BH_F32 || norm_weight_dtype == BH_BF16, "gemm_bf16_then_norm: unknown norm weight dtype %d", norm_weight_dtype);
   BH_REQUIRE(eps >= 0.f, "gemm_bf16_then_norm: eps must not be negative");
   BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)residual | (uintptr_t)normed | (uintptr_t)scratch | (uintptr_t)norm_weight) % 16 == 0,
@@ -1637,12 +1636,10 @@ extern "C" int bh_gemm_bf16_bare_parts(int M, int N, int K, int layout) {
   const RingPlan ring = gemm_ring_bare_plan(M, N, K, layout);
   return ring.tile >= 0 && ring.parts > 1 && ring.parts <= MAX_RING_PARTS ? ring.parts : 0;
 }
-extern "C" int bh_gemm_bf16_bare(const void* a, const void* w, float* sums, int M, int N, int K, int layout, int a_blocked,
-                                 hipStream_t stream) {
+extern "C" int bh_gemm_bf16_bare(const void* a, const void* w, float* sums, int M, int N, int K, int layout, hipStream_t stream) {
   const int parts = bh_gemm_bf16_bare_parts(M, N, K, layout);
   BH_REQUIRE(parts > 0, "gemm_bf16_bare: a product of M=%d N=%d K=%d is not left in parts (bh_gemm_bf16_bare_parts)", M, N, K);
   BH_REQUIRE(a && w && sums, "gemm_bf16_bare: every operand is needed");
   BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)sums) % 16 == 0, "gemm_bf16_bare: operands must be 16-byte aligned");
-  BH_REQUIRE(a_blocked, "gemm_bf16_bare: the activations lie in blocks of 16 rows");
   return gemm_ring_launch_parts(a, w, sums, M, N, K, gemm_ring_bare_plan(M, N, K, layout), stream);
 }

@@ -356,12 +356,11 @@ int gemm_ring_launch(const void* a, const void* w, void* c, int c_dtype, int acc
 
 // For tests and measurements: the tiles of 256 rows at a given width of 32 `blocks` weight rows, whatever gemm_ring_plan would choose.
 extern "C" int bh_gemm_bf16_turns(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K, int activation,
-                                  int blocks, int a_blocked, int c_blocked, hipStream_t stream) {
+                                  int blocks, int c_blocked, hipStream_t stream) {
   const int outs = (activation ? 16 : 32) * blocks;
   BH_REQUIRE((blocks == 8 || blocks == 6 || blocks == 4) && M >= 256 && N >= outs && N % 16 == 0 && K >= 128 && K % 128 == 0,
              "gemm_turns: a product of M=%d N=%d K=%d with %d blocks per wave is not one this kernel takes "
              "(M >= 256, K a multiple of 128, N a multiple of 16 and at least a tile)", M, N, K, blocks);
-  BH_REQUIRE(a_blocked, "gemm_turns: the activations lie in blocks of 16 rows");
   return gemm_ring_launch(a, w, c, c_dtype, accumulate, M, N, K, activation != 0, blocks == 8 ? RING_256x256 : blocks == 6 ? RING_256x192 : RING_256x128,
                           c_blocked, bh_gate_form(activation), stream);
 }

@@ -143,7 +143,7 @@ class KernelSizes:
             "bh_qk_norm_rope_cache_takes_sums": [i, i, i],
             "bh_gemm_bf16_plan": [i, i, i, i, i],
             "bh_gemm_bf16_bare_parts": [i, i, i, i],
-            "bh_gemm_bf16_bare": [p, p, p, i, i, i, i, i, p],
+            "bh_gemm_bf16_bare": [p, p, p, i, i, i, i, p],
             "bh_attention_generic": [p, p, i, p, p, p, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32": [p, p, p, p, p, i, i, i, p, p, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32_takes": [i, i, i, i],
@@ -156,8 +156,8 @@ class KernelSizes:
             "bh_sample_draw_scratch": [i, i],
             "bh_sample_top_k_scratch": [i, i],
             "bh_gemm_bf16": [p, p, p, i, i, i, i, i, i, i, p, i, f, p, i, p, p, p, i, i, i, p],
-            "bh_gemm_bf16_turns": [p, p, p, i, i, i, i, i, i, i, i, i, p],
-            "bh_gemm_bf16_then_norm": [p, p, p, i, i, i, i, p, i, f, p, p, i, i, p],
+            "bh_gemm_bf16_turns": [p, p, p, i, i, i, i, i, i, i, i, p],
+            "bh_gemm_bf16_then_norm": [p, p, p, i, i, i, i, p, i, f, p, p, i, p],
             "bh_rows_blocked": [p, p, i, i, i, i, p],
             "bh_gemm_bf16_finishes_norm": [i, i, i, i],
             "bh_attention_bf16": [p, p, p, p, p, p, p, i, p, p, i, i, i, i, i, i, f, i, i, i, i, p, p, i, f, p, f, i, f, p],
@@ -559,8 +559,8 @@ class HipKernels(KernelSizes):
             self._check(self.lib.bh_gemm_bf16_then_norm(
                 self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out", (torch.float32,)), m, n, k, 1,
                 self._ptr(then_norm.weight, "norm weight"), _code(then_norm.weight, "norm weight"), float(then_norm.eps),
-                self._ptr(normed, "norm rows"), self._ptr(scratch, "gemm scratch", None, True), int(a_block_rows == 16),
-                int(isinstance(normed, BlockedRows)), self._stream()))
+                self._ptr(normed, "norm rows"), self._ptr(scratch, "gemm scratch", None, True), int(isinstance(normed, BlockedRows)),
+                self._stream()))
             return True, normed
         behind = None
         if (then_norm is not None and out.dtype == torch.float32 and not activation
@@ -659,7 +659,7 @@ class HipKernels(KernelSizes):
         a = self._in_blocks_of(a, a_block_rows)
         sums = torch.empty((parts, m, n), dtype=torch.float32, device=self.device)
         self._check(self.lib.bh_gemm_bf16_bare(self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(sums, "gemm sums"),
-                                               m, n, k, 1, int(a_block_rows == 16), self._stream()))
+                                               m, n, k, 1, self._stream()))
         return PartSums(sums)
 
     def qk_norm_rope_takes_sums(self, n_rows, head_dim, rot) -> bool:
@@ -681,8 +681,7 @@ class HipKernels(KernelSizes):
             a = self._in_blocks_of(a, 16)
         self._check(self.lib.bh_gemm_bf16_turns(
             self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), _code(out, "gemm out"),
-            int(bool(accumulate)), m, n, k, int(bool(swiglu)), int(blocks), int(_block_rows(a) == 16),
-            int(_block_rows(out) == 16), self._stream()))
+            int(bool(accumulate)), m, n, k, int(bool(swiglu)), int(blocks), int(_block_rows(out) == 16), self._stream()))
 
     def gemm_turns_blocks(self, m, n, k, swiglu=False):
         """The width of the tiles of 256 rows on which `gemm` runs a packed product of these sizes in one go, in blocks of 32
