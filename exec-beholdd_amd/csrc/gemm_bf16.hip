@@ -1302,24 +1302,34 @@ static void launch_tiled(const void* a, const void* w, void* c, int M, int N, in
 
 static RingOutput ring_output(int activation, bool f32) { return activation ? RING_GATED : f32 ? RING_F32 : RING_BF16; }
 
-// How a product of many rows runs on the kernel for them, or (tile -1) not there.  That kernel multiplies a gated product in one go; few
-// outputs or few rows leave it few tiles, where the whole tiles above with K in parts and their finishing kernel are faster (us, there /
-// here: 256 rows of 1,024 gated outputs x 4,096 37.3 / 19.6, 129 of 2,048 x 2,048 20.2 / 16.3, 512 of 768 x 2,048 19.7 / 18.1; 400 rows of
-// 2,048 x 2,048 20.5 / 24.7, 129 of 6,912 x 2,560 31 / 40).  Theirs is estimated from rounds of two workgroups a compute unit, a slice
-// of 64 k at 0.88 us, or up to 1.6 where two share a unit, 6.2 us for the start and the second launch, and the sums' way; both estimates
-// are within 7 % of 126 measured sizes.  An 8 % lead of the kernel for many rows is asked for: with 256 and 512 rows it is slower than
-// its estimate.
+// How a product of many rows runs on the kernel for them, or (tile -1) not there, but on the whole tiles above with K in parts and their
+// finishing kernel.  Those are faster where that kernel has few tiles and cannot cut K, or not so finely: a gated product it multiplies
+// in one go, and others only into parts of whole slices that are all alike.  us, there / here: gated, 256 rows of 1,024 outputs x 4,096
+// 37.3 / 19.6, 129 of 2,048 x 2,048 20.2 / 16.3, 512 of 768 x 2,048 19.7 / 18.1, but 400 of 2,048 x 2,048 20.5 / 24.7, 129 of 6,912 x 2,560
+// 31 / 40; float32, 278 rows of 960 x 4,544 (71 slices) 35.6 / 18.0, 478 of 768 x 7,232 54 / 28.7; bfloat16, 148 of 2,816 x 4,544 39.7 / 21.6.
+// Theirs is estimated from rounds of two workgroups a compute unit, what a slice of 64 k takes one that has a unit alone or shares it,
+// the start and the second launch, and the sums' way; within 7 % of 126 (gated) and 196 measured sizes.  A lead is asked of the kernel
+// for many rows with a gated product of up to 512 rows, for with 256 and 512 it is slower than its estimate, and of the tiles beyond
+// 512 rows (616 rows of 1,408 x 2,304, gated, 21.2 / 26.2; 641 of 512 x 3,392, float32, 27.6 / 16.6).  (What a plain product writes may
+// not decide: its activations come in one form.)
+static bool whole_tiles_win(int M, int N, int K, int layout, bool gated, const RingPlan& f32, const RingPlan& other) {
+  int rows, columns, parts, slices;
+  tiled_config(M, N, gated, &rows, &columns);
+  tiled_parts(M, N, K, layout, gated, &parts, &slices);
+  if (parts == 1) return false;
+  const double each = (double)((N + columns - 1) / columns) * ((M + rows - 1) / rows) * parts / bh_compute_units();      // workgroups a compute unit
+  const double sharing = std::min(std::max(each - 1.0, 0.0), 1.0), rounds = std::max(std::ceil(each / 2.0), 1.0), outputs = 1e-6 * M * N;
+  if (gated) return rounds * slices * (0.88 + 0.72 * sharing) + 6.2 + parts * outputs * 2.0 < (M <= TILED_FEW_ROWS ? 1.08 : 0.95) * (f32.us + 1.3 + 1.7 * outputs);
+  const double tiles = rounds * slices * (0.9 + 0.45 * sharing) + 8.3 + parts * outputs * 1.27;
+  const bool few = M <= TILED_FEW_ROWS;
+  return tiles < (few ? 1.0 : 0.9) * (f32.us + 3.0 + 2.8 * outputs) && tiles < (few ? 1.05 : 0.9) * (other.us + 0.5 + 0.7 * outputs);
+}
 static RingPlan many_rows_plan(int M, int N, int K, int layout, RingOutput output) {
   const RingPlan plan = gemm_ring_plan(M, N, K, layout, output);
-  if (output != RING_GATED || plan.tile < 0) return plan;
-  int rows, columns, parts, slices;
-  tiled_config(M, N, true, &rows, &columns);
-  tiled_parts(M, N, K, layout, true, &parts, &slices);
-  if (parts == 1) return plan;
-  const double each = (double)((N + columns - 1) / columns) * ((M + rows - 1) / rows) * parts / bh_compute_units();      // workgroups a compute unit
-  const double slice = 0.88 + 0.72 * std::min(std::max(each - 1.0, 0.0), 1.0), rounds = std::max(std::ceil(each / 2.0), 1.0);
-  const double tiles = rounds * slices * slice + 6.2 + parts * (double)M * 2 * N * 4.0 * 0.25e-6;
-  return tiles < 1.08 * (plan.us + 1.3 + 1.7e-6 * M * N) ? RingPlan{-1, 1} : plan;
+  if (plan.tile < 0) return plan;
+  const bool gated = output == RING_GATED;
+  const RingPlan other = gated ? plan : gemm_ring_plan(M, N, K, layout, output == RING_F32 ? RING_BF16 : RING_F32);
+  return whole_tiles_win(M, N, K, layout, gated, output == RING_BF16 ? other : plan, output == RING_BF16 ? plan : other) ? RingPlan{-1, 1} : plan;
 }
 // A gated product that the tiles run in parts where the kernel for many rows could run it: the finishing kernel writes its output, in
 // blocks of 16 rows too.
@@ -1633,8 +1643,9 @@ extern "C" int bh_gemm_bf16_then_norm(const void* a, const void* w, float* resid
 // K goes in parts through the kernel for many rows.  `sums`: parts * M * N floats.
 extern "C" int bh_gemm_bf16_bare_parts(int M, int N, int K, int layout) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (many_rows_plan(M, N, K, layout, RING_BF16).tile < 0) return 0;
   const RingPlan ring = gemm_ring_bare_plan(M, N, K, layout);
-  return ring.tile >= 0 && ring.parts > 1 && ring.parts <= MAX_RING_PARTS ? ring.parts : 0;
+  return ring.parts > 1 && ring.parts <= MAX_RING_PARTS ? ring.parts : 0;
 }
 extern "C" int bh_gemm_bf16_bare(const void* a, const void* w, float* sums, int M, int N, int K, int layout, hipStream_t stream) {
   const int parts = bh_gemm_bf16_bare_parts(M, N, K, layout);

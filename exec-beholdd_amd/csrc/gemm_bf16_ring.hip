@@ -260,10 +260,10 @@ double cost_us(int tile, int parts, int M, int W, int K, RingOutput output) {
   if (parts == 1) return t;
   // The parts' sums on their way to memory and back.  float32: the finishing kernel takes the place of the norm's launch.  bfloat16: it
   // is a launch more; wide products are the queries', keys' and values' projection as a rule, whose reader takes the parts as they are
-  // (gemm_ring_bare_plan), and at those what hides behind the next tiles is more: cheaper from 6,144 weight rows on (rather than
-  // at the price of the others: 768 x 7,168 x 5,120 75.9 against 79.9 us, 1,000 x 6,144 x 4,096 70.1 against 69.5).
+  // (gemm_ring_bare_plan), and at those what hides behind the next tiles is more: cheaper from 6,144 weight rows and k of 2,048 on
+  // (rather than at the price of the others: 768 x 7,168 x 5,120 75.9 against 79.9 us, 1,000 x 6,144 x 4,096 70.1 against 69.5).
   const double sums = parts * (double)M * W * 4.0;
-  return t + (output == RING_F32 ? sums / 3.0e6 : W >= 6144 ? sums / 7.0e6 : sums / 3.8e6 + 4.0);
+  return t + (output == RING_F32 ? sums / 3.0e6 : W >= 6144 && K >= 2048 ? sums / 6.4e6 : sums / 3.8e6 + 4.0);
 }
 
 template <int MODE>

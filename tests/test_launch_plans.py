@@ -130,6 +130,10 @@ def test_products_of_many_rows_take_the_tiles_that_were_measured_fastest(sizes):
     # gated products of few tiles: the whole tiles with K in parts
     assert plan(256, 1024, 4096, "gated") is None and plan(129, 2048, 2048, "gated") is None and plan(512, 768, 2048, "gated") is None
     assert plan(400, 2048, 2048, "gated") is not None and plan(129, 6912, 2560, "gated") is not None
+    # slices of k that make no equal parts, or none fine enough: the whole tiles again, whatever the product writes
+    for size in ((278, 960, 4544), (478, 768, 7232), (148, 2816, 4544), (264, 640, 1984), (675, 960, 3904), (862, 1344, 7744)):
+        assert plan(*size, "float32") is None and plan(*size, "bfloat16") is None, size
+    assert plan(1140, 1280, 2752, "float32") is not None
     assert plan(128, 4096, 4096, "float32") is None and plan(256, 4096, 512, "float32") is None      # for the slices; the tiles
 
 
