@@ -242,8 +242,9 @@ __global__ __launch_bounds__(256, KG == 4 ? 1 : 2) void gemm_f32_ring_kernel(con
 // ---- many rows, any K ----------------------------------------------------------------------------------
 // Four waves own 64 B x 64 B outputs (B = 1 or 2), a wave B x B tiles of v_mfma_f32_32x32x2_f32; a workgroup is one such group, or
 // KG of them that take the slices of k in turn (B = 1).  Slices of 32 k go through two LDS buffers, the next slice's loads on their way
-// while one is multiplied.  A row of a slice takes 36 floats of LDS, so that the 16-byte reads of 16 neighbouring rows fall on different banks; lane (row, half) reads four k at once and the
-// matrix instructions take k in that order, the same for both operands.  Every slice is summed on its own and then added.
+// while one is multiplied.  A row of a slice takes 36 floats of LDS, so that the 16-byte reads of 16 neighbouring rows fall on different
+// banks; lane (row, half) reads four k at once and the matrix instructions take k in that order, the same for both operands.  Every slice
+// is summed on its own and then added.
 // Bound by the matrix instructions (64 cycles a tile and two k) where the tiles fill the chip.
 // Measured: 695 x 6,144 x 1,024 in 104 us (84 TFLOP/s), 2,048 x 32,768 x 1,024 in 1.12 ms (122 TFLOP/s; a library product of 8,192
 // cubed reaches 154); 695 x 1,024 x 3,072 in 70 us, 87 with one group of waves a workgroup.
