@@ -1,0 +1,69 @@
+"""Products of up to 32 rows of packed weights at the edges of what a workgroup owns and a wave holds, against float64."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from beholdd.kernels import HipKernels
+    return HipKernels()
+
+
+def rel(got, want):
+    return float((got.double() - want).abs().max() / want.abs().max())
+
+
+# k: waves without a chunk, one and two chunks a wave and one more or less (all at once / in turn), the same for the four sets of the
+# spans of 8 rows (n of up to 2,048 from k of 1,536 on); n: spans of 16, 8, 20 and 24 rows, an odd number of workgroups, more than four
+# workgroups a compute unit and long k at more than 16 rows (the kernel that asks in bursts)
+@pytest.mark.parametrize("n,k", [(96, 64), (4096, 512), (2064, 960), (4080, 1024), (4112, 1088), (16, 1536), (1040, 1984), (2048, 2048),
+                                 (2032, 2112), (336, 5184), (5120, 448), (5120, 2112), (6144, 1024), (6144, 4160), (17408, 256), (2560, 2112)])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32])
+def test_products_of_few_rows(K, m, n, k):
+    """float32 with and without accumulation and a norm behind, bfloat16 behind prepared norm rows, squared, and gated, from rows and
+    from blocks whose rows behind the last hold NaN; the bounds are those of a sum of k float32 products and of bfloat16 roundings."""
+    from beholdd.kernels.library import BlockedRows
+    from beholdd.parts.base import NormRequest
+    g = torch.Generator(device="cuda:0").manual_seed(m + n + k)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device="cuda:0")
+    a, w = normal(m, k).to(torch.bfloat16), (normal(n, k) / k ** 0.5).to(torch.bfloat16)
+    packed, block_rows = K.pack_weight(w), int(K.lib.bh_gemm_bf16_reads_blocked(m, n, k, 1, 0))
+    assert block_rows == (8 if m <= 8 else 16)
+    x = BlockedRows(torch.full((BlockedRows.padded_rows(m, block_rows) * k,), float("nan"), dtype=torch.bfloat16, device="cuda:0"), m, k, block_rows)
+    K.to_blocked(a, x, block_rows)
+    want, bound = a.double() @ w.double().t(), 4 * math.sqrt(k) * 2.0 ** -24
+    empty = lambda dtype: torch.full((m, n), float("nan"), dtype=dtype, device="cuda:0")
+    out = empty(torch.float32)
+    K.gemm(x, packed, out)
+    assert rel(out, want) < bound
+    stream = torch.cuda.current_stream().cuda_stream
+    direct = empty(torch.float32)      # rows one after the other, which the entry takes as well
+    assert K.lib.bh_gemm_bf16(a.data_ptr(), packed.data.data_ptr(), direct.data_ptr(), 0, 0, m, n, k, 1, 0, None, 0, 0.0, None, 0, None, None, None,
+                              0, 0, 0, stream) == 0
+    assert torch.equal(direct, out)
+    base, weight, eps = normal(m, n), 1 + 0.3 * normal(n), 1e-5
+    total = base.clone()
+    prepared = K.gemm(x, packed, total, accumulate=True, then_norm=NormRequest(weight, eps))
+    assert rel(total, want + base.double()) < bound
+    assert rel(prepared.ss.sum(1), (total.double() ** 2).sum(-1)) < 1e-5
+    assert rel(prepared.rows, total.double() * weight.double()) < 4e-3
+    # prepared rows of width n in front of products of this shape turned round: the row factor
+    w2 = (normal(160, n) / n ** 0.5).to(torch.bfloat16)
+    if n % 64 == 0:
+        normed = total.double() / torch.sqrt((total.double() ** 2).mean(-1, keepdim=True) + eps) * weight.double()
+        rounded = torch.empty(m, 160, dtype=torch.bfloat16, device="cuda:0")
+        K.gemm(prepared, K.pack_weight(w2), rounded)
+        assert rel(rounded, normed @ w2.double().t()) < 1e-2
+    for rows in (0, block_rows) if n % 32 == 0 else (0,):
+        squared = empty(torch.bfloat16) if not rows else K.to_blocked(empty(torch.bfloat16), block_rows=rows)
+        if K.gemm_relu_squared(x, packed, squared):
+            assert rel(K.from_blocked(squared) if rows else squared, want.clamp(min=0) ** 2) < 4e-3 + 4 * bound
+    up = (normal(n, k) / k ** 0.5).to(torch.bfloat16)
+    gated = empty(torch.bfloat16)
+    K.gemm_swiglu(x, K.pack_weight(torch.cat([w, up])), gated)
+    assert rel(gated, want / (1 + torch.exp(-want)) * (a.double() @ up.double().t())) < 6e-3
