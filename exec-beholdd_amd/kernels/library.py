@@ -43,9 +43,10 @@ class NormedRows:
     1 / sqrt(total / width + eps).  Products (`gemm`, `gemm_swiglu`) take it in place of an activation
     matrix and apply the factor to their result; one that cannot (other operand types) runs the norm
     itself from `source`, which must still hold the norm's input then.  `shape` and `dtype` are those of
-    the matrix it stands for."""
+    the matrix it stands for.  Of float32 rows nothing is prepared (`ss` is None, `rows` the residual itself): the
+    product that reads them makes the norm from `source` as it goes."""
 
-    def __init__(self, rows: torch.Tensor, ss: torch.Tensor, eps: float, source: torch.Tensor, weight: torch.Tensor):
+    def __init__(self, rows: torch.Tensor, ss: torch.Tensor | None, eps: float, source: torch.Tensor, weight: torch.Tensor):
         self.rows, self.ss, self.eps = rows, ss, float(eps)
         self.source, self.weight = source, weight       # the norm's input and weight, for a product that cannot take this form
         self.shape, self.dtype, self.device = rows.shape, rows.dtype, rows.device
@@ -150,6 +151,8 @@ class KernelSizes:
             "bh_attention_f32_tiles": [i, i, i, i, i, i, p, p],
             "bh_gemm_f32_takes_gated": [i, i, i],
             "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
+            "bh_gemm_f32_takes_norm": [i, i, i],
+            "bh_gemm_f32_normed": [p, p, f, p, p, i, i, i, i, p],
             "bh_swiglu": [p, p, i, i, i, i, p],
             "bh_sample": [p, p, p, p, p, p, p, p, i, i, p],
             "bh_sample_scratch": [i, i],
@@ -607,17 +610,32 @@ class HipKernels(KernelSizes):
         n = w.shape[0]
         if w.shape[1] != k or tuple(out.shape) != (m, n):
             raise KernelError(f"gemm: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
-        if isinstance(a, NormedRows) and not self._takes_norm(a, w, n, 0):
+        if isinstance(a, NormedRows) and a.ss is None and not accumulate and self._normed_f32(a, w, out, n, 0):
+            return None
+        if isinstance(a, NormedRows) and (a.ss is None or not self._takes_norm(a, w, n, 0)):
             a = self._run_norm(a, w, n, 0)
         done, prepared = self._gemm_fast(a, w, out, accumulate, 0, then_norm)
         if done:
             return prepared
         if isinstance(a, BlockedRows):
             a = self.from_blocked(a)
+        if (then_norm is not None and a.dtype == out.dtype == then_norm.weight.dtype == torch.float32
+                and then_norm.weight.shape == (n,) and self.lib.bh_gemm_f32_takes_norm(m, 4, n)):
+            prepared = NormedRows(out, None, then_norm.eps, out, then_norm.weight)      # its reader norms the residual itself
         self._check(self.lib.bh_gemm_generic(
             self._ptr(a, "gemm a"), _code(a, "gemm a"), self._ptr(w, "gemm w"), _code(w, "gemm w"),
             self._ptr(out, "gemm out"), _code(out, "gemm out"), int(bool(accumulate)), m, n, k, self._stream()))
-        return None
+        return prepared
+
+    def _normed_f32(self, a, w, out, n, gate) -> bool:
+        """The product of float32 `NormedRows` with float32 weights, whose norm it makes itself; False where it does not go."""
+        m, k = a.shape
+        if (not isinstance(w, torch.Tensor) or not w.dtype == out.dtype == a.source.dtype == a.weight.dtype == torch.float32
+                or not self.lib.bh_gemm_f32_takes_norm(m, n, k) or (a.source.data_ptr() | w.data_ptr() | a.weight.data_ptr()) % 16):
+            return False
+        self._check(self.lib.bh_gemm_f32_normed(self._ptr(a.source, "gemm a"), self._ptr(a.weight, "norm weight"), a.eps, self._ptr(w, "gemm w"),
+                                                self._ptr(out, "gemm out"), m, n, k, gate, self._stream()))
+        return True
 
     def gemm_relu_squared(self, a, w, out) -> bool:
         """out[M, N] = max(a[M, K] @ w[N, K]^T, 0)^2 in one launch, where the library has a product of these operands that does
@@ -722,7 +740,9 @@ class HipKernels(KernelSizes):
         if tuple(w.shape) != (2 * width, k) or out.shape[0] != m or out.dtype != a.dtype:
             raise KernelError(f"gemm_swiglu: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} "
                               "do not fit")
-        if isinstance(a, NormedRows) and width % 16 == 0 and not self._takes_norm(a, w, width, 1):
+        if isinstance(a, NormedRows) and a.ss is None and self._normed_f32(a, w, out, width, self.GATES[gate]):
+            return
+        if isinstance(a, NormedRows) and (a.ss is None or (width % 16 == 0 and not self._takes_norm(a, w, width, 1))):
             a = self._run_norm(a, w, width, 1)
         if self._gemm_fast(a, w, out, False, 1, gate=self.GATES[gate])[0]:
             return

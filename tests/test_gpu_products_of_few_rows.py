@@ -67,3 +67,40 @@ def test_products_of_few_rows(K, m, n, k):
     gated = empty(torch.bfloat16)
     K.gemm_swiglu(x, K.pack_weight(torch.cat([w, up])), gated)
     assert rel(gated, want / (1 + torch.exp(-want)) * (a.double() @ up.double().t())) < 6e-3
+
+
+# rows around the groups of four and the last of the few; k: shorter than a wave's load, remainders of a chunk and of a trip, eight waves;
+# outputs: every split of a workgroup's rows
+@pytest.mark.parametrize("m,n,k", [(1, 5, 60), (3, 64, 64), (4, 2048, 1024), (5, 7, 68), (8, 4099, 256), (9, 130, 516), (16, 8200, 132),
+                                   (17, 33, 2052), (31, 516, 3072), (32, 16, 2048), (32, 1030, 1088)])
+def test_float32_products_norm_a_residual(K, m, n, k):
+    """A float32 product leaves the norm behind it to the product that reads it; both together against float64.  The bound: a sum of k
+    products, each of which is off by the roundings of its factors (the weight's, the row factor's with its sum of squares)."""
+    from beholdd.kernels import NormedRows
+    from beholdd.parts.base import NormRequest
+    g = torch.Generator(device="cuda:0").manual_seed(m + n + k)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device="cuda:0")
+    a, w_in, w, weight, eps = normal(m, 64), normal(k, 64) / 8, normal(2 * n, k) / k ** 0.5, 1 + 0.3 * normal(k), 1e-5
+    residual = normal(m, k)
+    want_residual = residual.double() + a.double() @ w_in.double().t()
+    prepared = K.gemm(a, w_in, residual, accumulate=True, then_norm=NormRequest(weight, eps))
+    assert isinstance(prepared, NormedRows) and prepared.ss is None and rel(residual, want_residual) < 64 * 2.0 ** -24
+    source = residual.double()
+    normed = source / torch.sqrt((source ** 2).mean(-1, keepdim=True) + eps) * weight.double()
+    bound = (k / 16 + 72) * 2.0 ** -24 * (normed.abs() @ w.double().abs().t())
+    out = torch.full((m, n), float("nan"), device="cuda:0")
+    half = w[:n].contiguous()
+    assert K.gemm(prepared, half, out) is None
+    assert bool(((out.double() - normed @ half.double().t()).abs() <= bound[:, :n]).all())
+    gated = torch.full((m, n), float("nan"), device="cuda:0")
+    K.gemm_swiglu(prepared, w, gated)
+    both = normed @ w.double().t()
+    gate, up = both[:, :n], both[:, n:]
+    # d(silu) is at most 1.1, and the function itself some roundings
+    slack = 1.1 * bound[:, :n] * up.abs() + bound[:, n:] * gate.abs() + 16 * 2.0 ** -24 * (gate * up).abs() + 1e-30
+    assert bool(((gated.double() - gate / (1 + torch.exp(-gate)) * up).abs() <= slack).all())
+    # one that adds to what is there runs the norm as a launch of its own
+    total = normal(m, n)
+    base = total.double()
+    K.gemm(prepared, half, total, accumulate=True)
+    assert bool(((total.double() - base - normed @ half.double().t()).abs() <= bound[:, :n] + 4 * 2.0 ** -24 * base.abs()).all())
