@@ -13,10 +13,13 @@
 // serial chain of FMAs.
 // A sequence's chunks have places of their own, floor(first row / 64) + sequence onward, which overlap no other sequence's: a step
 // needs rows / 64 + sequences places, and a window of them at a time has memory for its states.
-// Bound by the matrix instructions and the operands' reads from LDS beside them; a state is written once and read twice.
-// Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 88 us in all (26 + 18 +
-// 40 and the gaps between), 240 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 165 us, 610.  With the
-// values in LDS beside the keys, one workgroup a compute unit, about 20 and 50 us more.
+// Bound by the matrix instructions, of which lightning attention's outputs need 11 us below, and by what comes before and behind them: all
+// workgroups are at the same of a chunk's four phases at a time, and loads and stores alone take 17 us of the outputs' 34.  A state is
+// written once and read twice.
+// Measured, bfloat16 projections, one sequence of 2,048 rows: lightning attention with 16 heads of 128 x 128 70 us in all (25 + 11 +
+// 34), 240 as a walk of chunks; the state-space recurrence with 64 heads of 128 x 64 148 us, 610.  (88 and 165 with states by rows,
+// loads waited for one piece after the other, and heads of a group on different XCDs.)  With the values in LDS beside the keys, one
+// workgroup a compute unit, about 20 and 50 us more.
 #pragma once
 
 #include "common.h"
@@ -76,56 +79,102 @@ struct ScanDecays<false> {
   __device__ float from_start(int t) const { return exponential(sum[t]); }
 };
 
-// In: what the recurrence reads.  POWERS, SKIPS (with skip(head)), q4 / k4 / v4(row, head, i) (elements i .. i + 3 of the head's vector), and
-// prepare(decays, weights, chunk, head): called by a whole workgroup, which it leaves with a barrier to come.
-template <class In>
+// The place (of `places`) and head of a workgroup.  Heads that share their keys and queries (`shared` in a row) run at one place on one
+// XCD, one after the other, so that its L2 holds them (64 heads of 128 x 64 in groups of eight, 2,103 rows of three sequences: 164 -> 154 us); workgroups go to
+// the eight XCDs in turn.  The grid is of whole rounds (ds_grid); those beyond the last place and head have nothing to do.
+__device__ inline bool ds_where(int places, int H, int shared, int& place, int& head) {
+  const int turn = blockIdx.x / 8, unit = turn / shared * 8 + blockIdx.x % 8;
+  place = unit % places;
+  head = unit / places * shared + turn % shared;
+  return head < H;
+}
+inline unsigned ds_grid(int places, int H, int shared) { return ((unsigned)(places * (H / shared)) + 7) / 8 * 8 * shared; }
+
+// Where a workgroup's 512 threads find four neighbouring elements of the chunk's 64 vectors of 4 * `pieces` each: thread, then 512 on.
+struct ScanPieces {
+  int row, piece, pieces;
+  __device__ ScanPieces(int pieces) : row(threadIdx.x / pieces), piece(threadIdx.x % pieces), pieces(pieces) {}
+  __device__ void next() {
+    row += 512 / pieces;
+    piece += 512 % pieces;
+    if (piece >= pieces) piece -= pieces, ++row;
+  }
+};
+
+// A state lies in scratch memory as the matrix instructions hand it out and take it: 16 x 16 tiles, column after column of them, and in
+// a tile lane (j, g)'s four elements (rows 4 g .. + 3, column j) side by side, so that every load and store of one is 1 KB in a piece (by
+// rows, 64 bytes at a time, lightning attention's three kernels of 16 heads of 128 x 128 and 2,048 rows took 25 + 18 + 41 us).
+__device__ inline size_t ds_tile(int column_tile, int row_tile, int D) { return ((size_t)column_tile * (D / 16) + row_tile) * 256; }
+
+// In: what the recurrence reads.  POWERS, SKIPS (with skip(head)), shared() (heads in a row with the same keys and queries), Raw q4 / k4 / v4(row, head, i) (elements i .. i + 3 of the head's vector as
+// memory holds them) with float4 open(Raw), and prepare(decays, weights, chunk, head): called by a whole workgroup, which it leaves with
+// a barrier to come.  WIDE: vectors of more than 128 elements.  All of a chunk's loads are asked for before the first is waited for.
+template <class In, bool WIDE>
 __global__ __launch_bounds__(512) void scan_states_kernel(In in, const int32_t* __restrict__ seq_start, int n_seqs, int place0, int places,
                                                           float* __restrict__ states, float* __restrict__ factors, int H, int D, int V) {
   extern __shared__ __align__(16) float ds_lds[];
   __shared__ ScanDecays<In::POWERS> decays;
   __shared__ float weights[DS_ROWS];
-  const int head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + blockIdx.x);
+  constexpr int STEPS = WIDE ? 9 : 4;      // D of up to 288 fits the LDS
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int place, head;
+  if (!ds_where(places, H, in.shared(), place, head)) return;
+  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + place);
   if (at.rows == 0) return;
   const int ks = D + 4, vs = V + 4;
   float* k_lds = ds_lds;
   float* v_lds = k_lds + DS_ROWS * ks;
-  in.prepare(decays, weights, at, head);
-  for (int e = tid; e < DS_ROWS * V / 4; e += 512) {
-    const int r = e / (V / 4), i = 4 * (e % (V / 4));
-    *reinterpret_cast<float4*>(v_lds + r * vs + i) = r < at.rows ? in.v4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  __syncthreads();
-  for (int e = tid; e < DS_ROWS * D / 4; e += 512) {
-    const int r = e / (D / 4), i = 4 * (e % (D / 4));
-    float4 k = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (r < at.rows) {
-      k = in.k4(at.first + r, head, i);
-      const float w = weights[r] * decays.between(at.rows - 1, r);
-      k = make_float4(k.x * w, k.y * w, k.z * w, k.w * w);
+  typename In::Raw k_raw[STEPS], v_raw[STEPS];
+  {
+    ScanPieces k_at(D / 4), v_at(V / 4);
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u, k_at.next(), v_at.next()) {
+      if (k_at.row < at.rows) k_raw[u] = in.k4(at.first + k_at.row, head, 4 * k_at.piece);
+      if (v_at.row < at.rows) v_raw[u] = in.v4(at.first + v_at.row, head, 4 * v_at.piece);
     }
-    *reinterpret_cast<float4*>(k_lds + r * ks + i) = k;
   }
-  if (tid == 0) factors[(size_t)blockIdx.x * H + head] = decays.from_start(at.rows - 1);
+  in.prepare(decays, weights, at, head);
   __syncthreads();
-  // Z [D][V]: 32 x 16 elements at a time, rows of the chunk as the products' depth
+  const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+  ScanPieces k_at(D / 4), v_at(V / 4);
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u, k_at.next(), v_at.next()) {
+    if (k_at.row < DS_ROWS) {
+      float4 k = none;
+      if (k_at.row < at.rows) {
+        k = in.open(k_raw[u]);
+        const float w = weights[k_at.row] * decays.between(at.rows - 1, k_at.row);
+        k = make_float4(k.x * w, k.y * w, k.z * w, k.w * w);
+      }
+      *reinterpret_cast<float4*>(k_lds + k_at.row * ks + 4 * k_at.piece) = k;
+    }
+    if (v_at.row < DS_ROWS) *reinterpret_cast<float4*>(v_lds + v_at.row * vs + 4 * v_at.piece) = v_at.row < at.rows ? in.open(v_raw[u]) : none;
+  }
+  if (tid == 0) factors[(size_t)place * H + head] = decays.from_start(at.rows - 1);
+  __syncthreads();
+  // Z [D][V]: 32 x 16 elements at a time, rows of the chunk as the products' depth; a wave's values stay in registers while its columns
+  // do (V of 16, 32, 64, 128: always)
   const int j = lane & 15, g = lane >> 4, columns = V / 16;
-  float* out = states + ((size_t)blockIdx.x * H + head) * D * V;
+  float* out = states + ((size_t)place * H + head) * D * V;
+  float v[DS_ROWS / 4];
+  int held = -1;
   for (int unit = wave; unit < D / 32 * columns; unit += 8) {
-    const int d0 = unit / columns * 32, c0 = unit % columns * 16;
+    const int d0 = unit / columns * 32, column = unit % columns;
+    if (column != held) {
+      held = column;
+#pragma unroll
+      for (int s = 0; s < DS_ROWS / 4; ++s) v[s] = v_lds[(16 * (s / 4) + 4 * g + s % 4) * vs + 16 * column + j];
+    }
     ds_f32x4_t acc[2] = {};
 #pragma unroll
     for (int s = 0; s < DS_ROWS / 4; ++s) {
       const int row = 16 * (s / 4) + 4 * g + s % 4;      // four rows of 4 D + 16 floats apart: on banks of their own
       const float* k_row = k_lds + row * ks + d0 + j;
-      const float v = v_lds[row * vs + c0 + j];
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[0], v, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[16], v, acc[1], 0, 0, 0);
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[0], v[s], acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_row[16], v[s], acc[1], 0, 0, 0);
     }
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) out[(size_t)(d0 + 16 * x + 4 * g + r) * V + c0 + j] = acc[x][r];
+    for (int x = 0; x < 2; ++x) *reinterpret_cast<ds_f32x4_t*>(out + ds_tile(column, d0 / 16 + x, D) + 4 * lane) = acc[x];
   }
 }
 
@@ -134,49 +183,63 @@ template <int UNUSED = 0>
 __global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
                                                            int place0, int places, float* __restrict__ states,
                                                            const float* __restrict__ factors, float* __restrict__ home, long slot_stride,
-                                                           int H, int size) {
+                                                           int H, int D, int V) {
   constexpr int AHEAD = 8;
-  const int seq = blockIdx.x, head = blockIdx.y, e = 4 * (blockIdx.z * 256 + threadIdx.x);
+  const int seq = blockIdx.x, head = blockIdx.y, size = D * V, e = 4 * (blockIdx.z * 256 + threadIdx.x);
   if (e >= size) return;
   const int base = ds_place_of(seq_start, seq), chunks = (seq_start[seq + 1] - seq_start[seq] + DS_ROWS - 1) / DS_ROWS;
   const int from = max(0, place0 - base), upto = min(chunks, place0 + places - base);
   if (from >= upto) return;
-  float4* mine = reinterpret_cast<float4*>(home + (size_t)seq_slot[seq] * slot_stride + (size_t)head * size + e);
+  // the thread's four elements of a tile (ds_tile) in the sequence's region, which lies by rows
+  const int tile = e / 256, lane = e % 256 / 4, d = tile % (D / 16) * 16 + lane / 16 * 4, v = tile / (D / 16) * 16 + lane % 16;
+  float* mine = home + (size_t)seq_slot[seq] * slot_stride + (size_t)head * size + (size_t)d * V + v;
   const size_t apart = (size_t)H * size;
   float* z = states + ((size_t)(base + from - place0) * H + head) * size + e;
   const float* f = factors + (size_t)(base + from - place0) * H + head;
-  float4 state = *mine;
-  for (int c = 0; c < upto - from; c += AHEAD) {
-    float4 own[AHEAD];
-    float factor[AHEAD];
+  float4 state = make_float4(mine[0], mine[V], mine[2 * V], mine[3 * V]);
+  float4 own[2][AHEAD];
+  float factor[2][AHEAD];
+  auto ask = [&](int side, int c) {      // (beyond the last chunk the last one's again, which nobody uses)
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
       const int at = min(c + u, upto - from - 1);
-      own[u] = *reinterpret_cast<const float4*>(z + at * apart);
-      factor[u] = f[(size_t)at * H];
+      own[side][u] = *reinterpret_cast<const float4*>(z + at * apart);
+      factor[side][u] = f[(size_t)at * H];
     }
+  };
+  ask(0, 0);
+  for (int c0 = 0; c0 < upto - from; c0 += 2 * AHEAD)
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      if (c + u >= upto - from) break;
-      *reinterpret_cast<float4*>(z + (c + u) * apart) = state;      // what this chunk starts from
-      state.x = fmaf(factor[u], state.x, own[u].x);
-      state.y = fmaf(factor[u], state.y, own[u].y);
-      state.z = fmaf(factor[u], state.z, own[u].z);
-      state.w = fmaf(factor[u], state.w, own[u].w);
+    for (int side = 0; side < 2; ++side) {
+      const int c = c0 + side * AHEAD;
+      if (c >= upto - from) break;
+      if (c + AHEAD < upto - from) ask(1 - side, c + AHEAD);      // while this side's chunks are joined
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        if (c + u >= upto - from) break;
+        *reinterpret_cast<float4*>(z + (c + u) * apart) = state;      // what this chunk starts from
+        state.x = fmaf(factor[side][u], state.x, own[side][u].x);
+        state.y = fmaf(factor[side][u], state.y, own[side][u].y);
+        state.z = fmaf(factor[side][u], state.z, own[side][u].z);
+        state.w = fmaf(factor[side][u], state.w, own[side][u].w);
+      }
     }
-  }
-  *mine = state;
+  mine[0] = state.x, mine[V] = state.y, mine[2 * V] = state.z, mine[3 * V] = state.w;
 }
 
-template <class In>
-__global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t* __restrict__ seq_start, int n_seqs, int place0,
-                                                           const float* __restrict__ states, float* __restrict__ out, int H, int D, int V) {
+template <class In, bool WIDE>
+__global__ __launch_bounds__(512, WIDE ? 2 : 4) void scan_outputs_kernel(In in, const int32_t* __restrict__ seq_start, int n_seqs, int place0,
+                                                                         int places, const float* __restrict__ states, float* __restrict__ out,
+                                                                         int H, int D, int V) {
   extern __shared__ __align__(16) float ds_lds[];
   __shared__ ScanDecays<In::POWERS> decays;
   __shared__ float weights[DS_ROWS];
   __shared__ int any_spoilt;      // whether a value of the chunk is not finite
-  const int head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + blockIdx.x);
+  constexpr int STEPS = WIDE ? 9 : 4, DEPTH = WIDE ? 18 : 8;      // D of up to 288 fits the LDS
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int place, head;
+  if (!ds_where(places, H, in.shared(), place, head)) return;
+  const ScanChunk at = ds_find(seq_start, n_seqs, place0 + place);
   if (at.rows == 0) return;
   const int qs = D + 4, vs = V + 4;
   // The scores and the values take the keys' place once those have been multiplied (the values wait in registers), which lets two
@@ -185,20 +248,41 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
   float* k_lds = q_lds + DS_ROWS * qs;
   float* p_lds = k_lds;
   float* v_lds = p_lds + DS_SCORES;
-  in.prepare(decays, weights, at, head);
-  for (int e = tid; e < DS_ROWS * D / 4; e += 512) {
-    const int r = e / (D / 4), i = 4 * (e % (D / 4));
-    const bool there = r < at.rows;
-    *reinterpret_cast<float4*>(q_lds + r * qs + i) = there ? in.q4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
-    *reinterpret_cast<float4*>(k_lds + r * qs + i) = there ? in.k4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  float4 values[DS_MOST_VALUES / 32];
+  const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+  typename In::Raw v_raw[STEPS];
+  // the state that the chunk starts from: a wave's columns of it, asked for here and needed last
+  const float* start = states + ((size_t)place * H + head) * D * V;
+  const int columns = V / 16, halves = columns >= 8 ? 1 : 2;      // a wave has both halves of the rows where there are columns for every wave
+  ds_f32x4_t e[DEPTH];
+  auto ask_state = [&](int column) {
 #pragma unroll
-  for (int u = 0; u < DS_MOST_VALUES / 32; ++u) {
-    const int e = tid + 512 * u, r = e / (V / 4), i = 4 * (e % (V / 4));
-    values[u] = r < at.rows && e < DS_ROWS * V / 4 ? in.v4(at.first + r, head, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int b = 0; b < DEPTH; ++b)
+      if (16 * b < D) e[b] = *reinterpret_cast<const ds_f32x4_t*>(start + ds_tile(column, b, D) + 4 * lane);
+  };
+  {
+    typename In::Raw q_raw[STEPS], k_raw[STEPS];
+    ScanPieces asked(D / 4), v_at(V / 4), put(D / 4);
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u, asked.next()) {
+      if (asked.row < at.rows) {
+        q_raw[u] = in.q4(at.first + asked.row, head, 4 * asked.piece);
+        k_raw[u] = in.k4(at.first + asked.row, head, 4 * asked.piece);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u, v_at.next())
+      if (v_at.row < at.rows) v_raw[u] = in.v4(at.first + v_at.row, head, 4 * v_at.piece);
+    in.prepare(decays, weights, at, head);
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u, put.next()) {
+      if (put.row >= DS_ROWS) continue;
+      const bool there = put.row < at.rows;
+      *reinterpret_cast<float4*>(q_lds + put.row * qs + 4 * put.piece) = there ? in.open(q_raw[u]) : none;
+      *reinterpret_cast<float4*>(k_lds + put.row * qs + 4 * put.piece) = there ? in.open(k_raw[u]) : none;
+    }
   }
   if (tid == 0) any_spoilt = 0;
+  if (wave < halves * columns) ask_state(wave / halves);
   __syncthreads();
   // scores: the ten 16 x 16 tiles on and below the diagonal, a wave one or two.  A lane's 16 bytes are k 16 b + 4 g .. + 3 of its row
   // for either operand, which the matrix instructions take in turn.
@@ -213,6 +297,7 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
     const float* q_row = q_lds + (16 * tr + j) * qs + 4 * g;
     const float* k_row = k_lds + (16 * tc + j) * qs + 4 * g;
     ds_f32x4_t chain[4] = {};      // four sums side by side, added at the end
+#pragma unroll 2
     for (int b = 0; b < D; b += 32) {
       const ds_f32x4_t q0 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b), k0 = *reinterpret_cast<const ds_f32x4_t*>(k_row + b);
       const ds_f32x4_t q1 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b + 16), k1 = *reinterpret_cast<const ds_f32x4_t*>(k_row + b + 16);
@@ -241,38 +326,43 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
     }
   }
   float zero = 0.f;      // zero times every value: NaN where one is not finite
+  ScanPieces v_at(V / 4);
 #pragma unroll
-  for (int u = 0; u < DS_MOST_VALUES / 32; ++u) {
-    const int e = tid + 512 * u;
-    if (e < DS_ROWS * V / 4) *reinterpret_cast<float4*>(v_lds + e / (V / 4) * vs + 4 * (e % (V / 4))) = values[u];
-    zero = fmaf(values[u].w, 0.f, fmaf(values[u].z, 0.f, fmaf(values[u].y, 0.f, fmaf(values[u].x, 0.f, zero))));
+  for (int u = 0; u < STEPS; ++u, v_at.next()) {
+    if (v_at.row >= DS_ROWS) continue;
+    const float4 value = v_at.row < at.rows ? in.open(v_raw[u]) : none;
+    *reinterpret_cast<float4*>(v_lds + v_at.row * vs + 4 * v_at.piece) = value;
+    zero = fmaf(value.w, 0.f, fmaf(value.z, 0.f, fmaf(value.y, 0.f, fmaf(value.x, 0.f, zero))));
   }
   if (zero != 0.f) any_spoilt = 1;
   __syncthreads();
   const bool spoilt = any_spoilt;
   // outputs: 32 rows x 16 columns at a time
-  const float* start = states + ((size_t)blockIdx.x * H + head) * D * V;
-  for (int unit = wave; unit < 2 * (V / 16); unit += 8) {
-    const int r0 = 32 * (unit & 1), c0 = unit / 2 * 16;
-    ds_f32x4_t acc[2][2] = {}, from_state[2][2] = {};      // [side][upper or lower 16 rows]: two sums side by side
-    const float* q_row = q_lds + (r0 + j) * qs + 4 * g;
-    const float* e_row = start + (size_t)(4 * g) * V + c0 + j;
-#pragma unroll 4
-    for (int b = 0; b < D; b += 16) {
-      float e[4];
+  auto outputs = [&](int r0, int c0) {
+    ds_f32x4_t carried[2];
+    {
+      ds_f32x4_t from_state[2][2] = {};      // [side]: two sums side by side
+      const float* q_row = q_lds + (r0 + j) * qs + 4 * g;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) e[t] = e_row[(size_t)(b + t) * V];
-      const ds_f32x4_t q0 = *reinterpret_cast<const ds_f32x4_t*>(q_row + b), q1 = *reinterpret_cast<const ds_f32x4_t*>(q_row + 16 * qs + b);
+      for (int b = 0; b < DEPTH; ++b) {
+        if (16 * b >= D) break;
+        __builtin_amdgcn_sched_barrier(0);      // not all rows of q in registers at once
+        ds_f32x4_t q[2];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        from_state[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(q0[t], e[t], from_state[t & 1][0], 0, 0, 0);
-        from_state[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q1[t], e[t], from_state[t & 1][1], 0, 0, 0);
+        for (int x = 0; x < 2; ++x) q[x] = *reinterpret_cast<const ds_f32x4_t*>(q_row + 16 * x * qs + 16 * b);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int x = 0; x < 2; ++x) from_state[t & 1][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[x][t], e[b][t], from_state[t & 1][x], 0, 0, 0);
       }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) carried[x] = from_state[0][x] + from_state[1][x];
     }
-    const int tr = r0 / 16;
-    const float* p_row = p_lds + tr * (tr + 1) / 2 * 16 * DS_PSTRIDE + j * DS_PSTRIDE + 4 * g;      // the upper 16 rows' tiles; then the lower's
-    const float* p_lower = p_row + (tr + 1) * 16 * DS_PSTRIDE;
+    ds_f32x4_t acc[2][2] = {};
+    const int tile0 = r0 / 16;
+    auto p_tile = [&](int x, int column) { return p_lds + ((tile0 + x) * (tile0 + x + 1) / 2 + column) * 16 * DS_PSTRIDE; };
     auto add_rows = [&](auto guarded) {
+#pragma unroll 1
       for (int b = 0; b < r0 + 32; b += 16) {
         float v[4], own[4];      // own: what the tile on the diagonal takes
 #pragma unroll
@@ -280,16 +370,14 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
           v[t] = v_lds[(b + 4 * g + t) * vs + c0 + j];
           own[t] = !guarded || isfinite(v[t]) ? v[t] : 0.f;
         }
-        const ds_f32x4_t p1 = *reinterpret_cast<const ds_f32x4_t*>(p_lower + b * DS_PSTRIDE);
-        if (b <= r0) {      // the upper 16 rows see no later ones
-          const ds_f32x4_t p0 = *reinterpret_cast<const ds_f32x4_t*>(p_row + b * DS_PSTRIDE);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          if (b > r0 + 16 * x) continue;      // rows see no later ones
+          const ds_f32x4_t p = *reinterpret_cast<const ds_f32x4_t*>(p_tile(x, b / 16) + j * DS_PSTRIDE + 4 * g);
 #pragma unroll
           for (int t = 0; t < 4; ++t)
-            acc[t & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[t], guarded && b == r0 ? own[t] : v[t], acc[t & 1][0], 0, 0, 0);
+            acc[t & 1][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t], guarded && b == r0 + 16 * x ? own[t] : v[t], acc[t & 1][x], 0, 0, 0);
         }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          acc[t & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[t], guarded && b == r0 + 16 ? own[t] : v[t], acc[t & 1][1], 0, 0, 0);
       }
     };
     if (!spoilt) {
@@ -298,14 +386,14 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
       // Scores above the diagonal are zeros, but zero times infinity is not: a value that is not finite stays out of the product of
       // its own rows' tile and is added by itself, to its row and the later ones.
       add_rows(std::true_type{});
+#pragma unroll
       for (int x = 0; x < 2; ++x) {
-        const float* p_tile = p_lds + ((tr + x) * (tr + x + 1) / 2 + tr + x) * 16 * DS_PSTRIDE;
         for (int c = 0; c < 16; ++c) {
           const float v = v_lds[(r0 + 16 * x + c) * vs + c0 + j];
           if (isfinite(v)) continue;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float added = fmaf(p_tile[(4 * g + r) * DS_PSTRIDE + c], v, acc[0][x][r]);
+            const float added = fmaf(p_tile(x, tile0 + x)[(4 * g + r) * DS_PSTRIDE + c], v, acc[0][x][r]);
             if (c <= 4 * g + r) acc[0][x][r] = added;
           }
         }
@@ -317,16 +405,23 @@ __global__ __launch_bounds__(512) void scan_outputs_kernel(In in, const int32_t*
       for (int r = 0; r < 4; ++r) {
         const int t = r0 + 16 * x + 4 * g + r;
         if (t >= at.rows) continue;
-        float total = fmaf(from_state[0][x][r] + from_state[1][x][r], decays.from_start(t), acc[0][x][r] + acc[1][x][r]);
+        float total = fmaf(carried[x][r], decays.from_start(t), acc[0][x][r] + acc[1][x][r]);
         if (In::SKIPS) total = fmaf(in.skip(head), v_lds[t * vs + c0 + j], total);
         out[((size_t)(at.first + t) * H + head) * V + c0 + j] = total;
       }
+  };
+  for (int unit = wave; unit < halves * columns; unit += 8) {
+    if (unit != wave) ask_state(unit / halves);
+    const int first = halves == 2 ? unit % 2 * 32 : 0, last = halves == 2 ? first : 32;
+#pragma unroll 1
+    for (int r0 = first; r0 <= last; r0 += 32) outputs(r0, unit / halves * 16);
   }
 }
 
-__device__ inline float4 ds_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ inline float4 ds_load4(const bf16_t* p) {
-  const uint2 raw = *reinterpret_cast<const uint2*>(p);
+__device__ inline float4 ds_raw4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ inline uint2 ds_raw4(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
+__device__ inline float4 ds_widen(float4 raw) { return raw; }
+__device__ inline float4 ds_widen(uint2 raw) {
   return make_float4(bf16_bits_to_f32((uint16_t)raw.x), bf16_bits_to_f32((uint16_t)(raw.x >> 16)), bf16_bits_to_f32((uint16_t)raw.y),
                      bf16_bits_to_f32((uint16_t)(raw.y >> 16)));
 }
@@ -352,26 +447,34 @@ inline long ds_scratch_floats(int n_seqs, int n_rows, int H, int D, int V) {
   return (places < most ? places : most) * one;
 }
 
-template <class In>
-int ds_launch(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
+template <class In, bool WIDE>
+int ds_launch_as(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
               long scratch_floats, int n_seqs, int n_rows, int H, int D, int V, hipStream_t stream) {
   const long one = (long)H * ((long)D * V + 1), places = ds_places(n_seqs, n_rows);
   const int window = (int)(scratch_floats / one < places ? scratch_floats / one : places);
   BH_REQUIRE(window > 0, "scan: no scratch memory for a chunk's states");
-  BH_REQUIRE(n_seqs <= 2147483647 && ((long)D * V + 1023) / 1024 <= 65535, "scan: a state of %d x %d is too large", D, V);
+  BH_REQUIRE((long)window * H < (1L << 30) && ((long)D * V + 1023) / 1024 <= 65535, "scan: a state of %d x %d is too large", D, V);
   const size_t states_lds = ds_states_lds(D, V), outputs_lds = ds_outputs_lds(D, V);
-  bh_allow_lds<scan_states_kernel<In>>(states_lds);
-  bh_allow_lds<scan_outputs_kernel<In>>(outputs_lds);
+  bh_allow_lds<scan_states_kernel<In, WIDE>>(states_lds);
+  bh_allow_lds<scan_outputs_kernel<In, WIDE>>(outputs_lds);
   float* factors = scratch + (size_t)window * H * D * V;
   for (long place = 0; place < places; place += window) {
     const int here = (int)(places - place < window ? places - place : window);
-    scan_states_kernel<In><<<dim3(here, H), 512, states_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, factors, H, D, V);
+    scan_states_kernel<In, WIDE><<<ds_grid(here, H, in.shared()), 512, states_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, factors, H, D, V);
     if (int status = bh_check_launch("scan_states")) return status;
     scan_combine_kernel<0><<<dim3(n_seqs, H, (D * V + 1023) / 1024), 256, 0, stream>>>(seq_start, seq_slot, (int)place, here, scratch, factors, home,
-                                                                                     slot_stride, H, D * V);
+                                                                                     slot_stride, H, D, V);
     if (int status = bh_check_launch("scan_combine")) return status;
-    scan_outputs_kernel<In><<<dim3(here, H), 512, outputs_lds, stream>>>(in, seq_start, n_seqs, (int)place, scratch, out, H, D, V);
+    scan_outputs_kernel<In, WIDE><<<ds_grid(here, H, in.shared()), 512, outputs_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, out, H, D, V);
     if (int status = bh_check_launch("scan_outputs")) return status;
   }
   return 0;
+}
+
+template <class In>
+int ds_launch(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
+              long scratch_floats, int n_seqs, int n_rows, int H, int D, int V, hipStream_t stream) {
+  return D > 128 || V > 128
+             ? ds_launch_as<In, true>(in, seq_start, seq_slot, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream)
+             : ds_launch_as<In, false>(in, seq_start, seq_slot, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream);
 }

@@ -437,14 +437,16 @@ struct LightningRows {
   int stride, q_off, k_off, v_off;
   const float* decay;
   int dim, vdim;
-  __device__ float4 opened(int row, int column) const {
-    const float4 x = ds_load4(proj + (size_t)row * stride + column);
+  using Raw = decltype(ds_raw4((const T*)nullptr));
+  __device__ float4 open(Raw raw) const {
+    const float4 x = ds_widen(raw);
     return make_float4(silu_f32(x.x), silu_f32(x.y), silu_f32(x.z), silu_f32(x.w));
   }
-  __device__ float4 q4(int row, int head, int i) const { return opened(row, q_off + head * dim + i); }
-  __device__ float4 k4(int row, int head, int i) const { return opened(row, k_off + head * dim + i); }
-  __device__ float4 v4(int row, int head, int i) const { return opened(row, v_off + head * vdim + i); }
+  __device__ Raw q4(int row, int head, int i) const { return ds_raw4(proj + (size_t)row * stride + q_off + head * dim + i); }
+  __device__ Raw k4(int row, int head, int i) const { return ds_raw4(proj + (size_t)row * stride + k_off + head * dim + i); }
+  __device__ Raw v4(int row, int head, int i) const { return ds_raw4(proj + (size_t)row * stride + v_off + head * vdim + i); }
   __device__ float skip(int) const { return 0.f; }
+  BH_BOTH int shared() const { return 1; }
   __device__ void prepare(ScanDecays<true>& decays, float* weights, const ScanChunk&, int head) const {
     if (threadIdx.x > DS_ROWS) return;
     const double lambda = decay[head];

@@ -365,10 +365,13 @@ struct SsmRows {
   int proj_stride, dt_first;
   const float *dt_bias, *a_log, *d_skip;
   int H, vdim, N, G;
-  __device__ float4 q4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + H * vdim + (G + head / (H / G)) * N + i); }
-  __device__ float4 k4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + H * vdim + head / (H / G) * N + i); }
-  __device__ float4 v4(int row, int head, int i) const { return ds_load4(xbc + (size_t)row * stride + head * vdim + i); }
+  using Raw = float4;
+  __device__ float4 open(float4 raw) const { return raw; }
+  __device__ float4 q4(int row, int head, int i) const { return ds_raw4(xbc + (size_t)row * stride + H * vdim + (G + head / (H / G)) * N + i); }
+  __device__ float4 k4(int row, int head, int i) const { return ds_raw4(xbc + (size_t)row * stride + H * vdim + head / (H / G) * N + i); }
+  __device__ float4 v4(int row, int head, int i) const { return ds_raw4(xbc + (size_t)row * stride + head * vdim + i); }
   __device__ float skip(int head) const { return d_skip[head]; }
+  BH_BOTH int shared() const { return H / G; }
   __device__ void prepare(ScanDecays<false>& decays, float* weights, const ScanChunk& at, int head) const {
     const int t = threadIdx.x;
     if (t >= DS_ROWS) return;      // the first wave
