@@ -614,13 +614,24 @@ extern "C" int bh_attention_bf16_splits(int n_seqs, int max_rows_per_seq, int H,
   return (pages + per - 1) / per;
 }
 
-#define PREFILL_FROM_TILES 1024   // column tiles x kv heads x sequences from which the prefill kernel runs a step
+// Whether the prefill kernel runs a step: from 1,024 tiles of columns (over kv heads and sequences) on, and, where no cache is longer
+// than the seven pages up to which keys are never split, prompts of few pages and those whose tiles fill the
+// chip: its four waves share a page that goes through LDS once, where a workgroup of this file's kernel has four waves on as many pages
+// for 16 columns and a merge behind them.  us here / there: three prompts of 253 rows in all, 40 heads of 128 on 8 16.8 / 6.7, 128 rows of
+// 32 on 8 8.2 / 6.4, 16 rows of 32 on 8 7.6 / 5.4; of seven pages 96 tiles 8.3 / 8.9, 160 11.3 / 10.6, 512 24.9 / 11.3.  (A step of up to
+// eight rows has its output read in blocks of eight, which the prefill kernel does not write.)
+#define PREFILL_FROM_TILES 1024
+static bool prefill_wins(int n_seqs, int max_rows_per_seq, int H, int KVH, int max_position) {
+  const long columns = (long)max_rows_per_seq * (H / KVH), tiles = (columns + 15) / 16 * KVH * n_seqs;
+  const int pages = max_position / BH_PAGE + 1;
+  if (tiles >= PREFILL_FROM_TILES) return true;
+  return max_rows_per_seq > 8 && columns >= 16 && pages < 8 && (pages <= 4 || tiles >= bh_compute_units());
+}
 // Whether a step of these sizes goes to the kernel for many columns per sequence, which writes its output in rows
 // or in blocks of 16 rows x 32 columns (bh_blocked_index); the other steps' kernels write blocks of 8 or 16 rows.
 extern "C" int bh_attention_bf16_writes_blocked(int n_seqs, int max_rows_per_seq, int H, int KVH, int max_position) {
   if (n_seqs <= 0 || max_rows_per_seq <= 0 || H <= 0 || KVH <= 0 || H % KVH) return 0;
-  const long tiles = (long)((max_rows_per_seq * (H / KVH) + 15) / 16) * KVH * n_seqs;
-  return bh_attention_bf16_splits(n_seqs, max_rows_per_seq, H, KVH, max_position) == 1 && tiles >= PREFILL_FROM_TILES ? 1 : 0;
+  return bh_attention_bf16_splits(n_seqs, max_rows_per_seq, H, KVH, max_position) == 1 && prefill_wins(n_seqs, max_rows_per_seq, H, KVH, max_position) ? 1 : 0;
 }
 
 static int attention_bf16_run(const void* q, void* out, void* part_o, void* part_ml, const void* k_pages,
@@ -645,7 +656,7 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   const bool is_fused = fused.qkv != nullptr;
   BH_REQUIRE(!is_fused || (tiles == 1 && max_rows_per_seq == 1 && n_rows == n_seqs),
              "attention_bf16: the fused projection rows are taken in decode steps of at most 16 heads per kv head only");
-  if (!is_fused && n_splits == 1 && (long)tiles * KVH * n_seqs >= PREFILL_FROM_TILES) {   // many columns: the prefill kernel
+  if (!is_fused && n_splits == 1 && prefill_wins(n_seqs, max_rows_per_seq, H, KVH, max_position)) {
     BH_REQUIRE(out_blocked == 0 || out_blocked == 16, "attention_bf16: a step of many columns writes rows or blocks of 16 rows, not of %d", out_blocked);
     bh_attention_prefill_launch(q, out, k_pages, v_pages, page_table, table_stride, positions, seq_start, n_seqs,
                                 tiles, H, KVH, hd, form, window, out_blocked == 16, finish, stream);

@@ -1,0 +1,46 @@
+"""Attention of short prompts on both sides of the rule that sends a step to the kernel whose four waves share a page, against float64."""
+
+import math
+
+import pytest
+import torch
+
+from test_gpu_kernels import PAGE, K, Layout, attention_reference_rows, dev, make_cache, rel, stored      # noqa: F401  (K: the fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+# heads, kv heads, head size, rows and pasts of the sequences, which kernel: eight and nine rows; fewer than 16 columns; four and five
+# pages of few tiles; seven pages at 255 and 256 tiles, eight pages (whose keys may be split)
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim,news,pasts,shared", [
+    (8, 2, 128, [8, 3], [0, 60], 0), (8, 2, 128, [9, 3], [0, 60], 1), (2, 2, 64, [15, 2], [3, 0], 0), (2, 2, 64, [16, 2], [3, 0], 1),
+    (32, 8, 128, [100, 80, 73], [0, 0, 0], 1), (5, 1, 96, [40, 9], [216, 1], 1), (5, 1, 96, [40, 9], [217, 1], 0),
+    (4, 4, 32, [1008], [0], 0), (15, 15, 32, [272, 1], [176, 0], 1), (15, 15, 32, [16, 16], [401, 0], 0), (16, 16, 64, [100, 64, 33], [348, 0, 5], 1),
+    (16, 1, 256, [12, 130], [0, 100], 1), (4, 2, 160, [33, 1, 64], [7, 190, 64], 1)])
+def test_attention_of_short_prompts(K, n_heads, kv_heads, head_dim, news, pasts, shared):
+    dtype, scale = torch.bfloat16, 1 / math.sqrt(head_dim)
+    lengths = [p + n for p, n in zip(pasts, news)]
+    assert int(K.lib.bh_attention_bf16_writes_blocked(len(news), max(news), n_heads, kv_heads, max(lengths) - 1)) == shared
+    kp, vp, table, keys, values = make_cache(len(lengths), lengths, kv_heads, head_dim, dtype, seed=head_dim + n_heads)
+    for s, n in enumerate(lengths):      # nothing behind a sequence's last key may reach a sum
+        if n % PAGE:
+            kp[int(table[s, (n - 1) // PAGE]), :, n % PAGE:, :] = float("nan")
+            vp[int(table[s, (n - 1) // PAGE]), :, :, n % PAGE:] = float("nan")
+    kp, vp = stored(K, kp, vp)
+    n_rows = sum(news)
+    q = torch.randn(n_rows, n_heads * head_dim, generator=torch.Generator().manual_seed(n_rows)).to(dtype)
+    positions = torch.tensor([p + t for p, n in zip(pasts, news) for t in range(n)], dtype=torch.int32)
+    row_seq = torch.tensor([s for s, n in enumerate(news) for _ in range(n)], dtype=torch.int32)
+    starts = [sum(news[:s]) for s in range(len(news) + 1)]
+    layout = Layout(False, dev(torch.tensor(starts, dtype=torch.int32)), len(news), max(news), max(lengths) - 1)
+    for window in (0, 50):
+        out = torch.full((n_rows, n_heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+        blocks = K.to_blocked(out, block_rows=8 if n_rows <= 8 else 16) if (n_heads * head_dim) % 32 == 0 else None
+        for to in (out, blocks):
+            if to is not None:
+                K.attention(dev(q), to, kp, vp, dev(table), dev(row_seq), dev(positions), n_heads, kv_heads, head_dim, scale, window, layout=layout)
+        assert blocks is None or torch.equal(K.from_blocked(blocks), out)
+        for s in range(len(news)):
+            rows = slice(starts[s], starts[s + 1])
+            want = attention_reference_rows(q[rows], keys[s], values[s], positions[rows], n_heads, kv_heads, head_dim, scale, window)
+            assert rel(out[rows], want) < 8e-3, (s, window)      # probabilities and results of 8 bits
