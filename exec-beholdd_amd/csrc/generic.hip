@@ -496,13 +496,20 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
     int table_stride, int H, int KVH, int kv_order, int n_rows, int n_heads, int main_waves, int value_waves) {
   constexpr int HD = 8 * LPH, HPW = BH_WAVE / LPH;
   const int waves_per_row = (n_heads + HPW - 1) / HPW;
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / BH_WAVE), lane = threadIdx.x % BH_WAVE;
+  // The values' waves, which move the most each, are the first of the first blocks, one a block, so that no compute unit has four of them
+  // (256 rows of 40 and 8 heads of 128 in four parts: 12.2 -> 10.3 us); what blocks there are not enough for follows the others.
+  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / BH_WAVE), lane = threadIdx.x % BH_WAVE, block_at = blockIdx.x;
+  const int spread = min(value_waves, (int)gridDim.x);
+  const bool with_values = block_at < spread;
+  const int turn = with_values ? 3 * block_at + slot - 1 : 3 * spread + 4 * (block_at - spread) + slot;   // among the others
+  const int wave = with_values && slot == 0 ? main_waves + block_at : turn < main_waves ? turn : turn + spread;
   if (wave >= main_waves) {   // the values of eight rows and HPW kv heads
     if (wave - main_waves >= value_waves) return;   // the last block's waves beyond the work (none at all without write_kv)
-    const int chunks = (KVH + HPW - 1) / HPW, group = (wave - main_waves) / chunks;
+    const int chunks = (KVH + HPW - 1) / HPW, group = (wave - main_waves) / 2 / chunks;
+    const bool of_pieces = (wave - main_waves) % 2 == 0;   // two waves: one for a whole piece, one for the others, where there are any
     // lanes without a kv head of their own follow the last one and store nothing: every lane stays to the end,
     // because the rows' positions below are read out of the first 24 lanes' registers
-    const int wanted_head = ((wave - main_waves) % chunks) * HPW + lane / LPH, c = lane % LPH;
+    const int wanted_head = ((wave - main_waves) / 2 % chunks) * HPW + lane / LPH, c = lane % LPH;
     const bool mine = wanted_head < KVH;
     const int kv_head = mine ? wanted_head : KVH - 1;
     const size_t fused = (size_t)(H + 2 * KVH) * HD, part_stride = (size_t)n_rows * fused;
@@ -515,7 +522,20 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
     const int near_pos = positions[near], near_seq = row_seq[near];
     auto pos_of = [&](int row) { return __builtin_amdgcn_readlane(near_pos, __builtin_amdgcn_readfirstlane(row - base)); };
     auto seq_of = [&](int row) { return __builtin_amdgcn_readlane(near_seq, __builtin_amdgcn_readfirstlane(row - base)); };
-    for (int row = 8 * group; row < 8 * group + 8 && row < n_rows; ++row) {
+    const int near_page = page_table[(size_t)near_seq * table_stride + near_pos / BH_PAGE];
+    auto block_of = [&](int row) {
+      const int page = __builtin_amdgcn_readlane(near_page, __builtin_amdgcn_readfirstlane(row - base));
+      return v_pages + ((size_t)page * KVH + kv_head) * BH_PAGE * HD;
+    };
+    // Which of the eight rows starts a piece of eight tokens that the step holds as rows one after the other (at most one: -1, none), and
+    // which belong to no such piece, whose elements are then asked for together: row after row, the seven rows at a sequence's end were
+    // fourteen trips to memory, most of the kernel's time at 253 rows of three sequences.
+    int starts = -1;
+    unsigned single = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = 8 * group + i;
+      if (row >= n_rows) break;
       const int pos = pos_of(row), seq = seq_of(row);
       const int first = row - pos % 8;   // where the row of the piece's first token would lie
       bool whole = first >= 0 && first + 7 < n_rows;   // the piece's eight tokens are the rows first .. first + 7, in order
@@ -523,25 +543,16 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
 #pragma unroll
         for (int t = 0; t < 8; ++t) whole = whole && seq_of(first + t) == seq && pos_of(first + t) == pos - pos % 8 + t;
       }
-      if (whole && pos % 8 != 0) continue;   // the first row of the piece stores it
-      const int page = page_table[(size_t)seq * table_stride + pos / BH_PAGE];
-      uint16_t* block = v_pages + ((size_t)page * KVH + kv_head) * BH_PAGE * HD;
-      if (!whole) {
-        const size_t one_at[1] = {src + (size_t)row * fused};
-        uint4 one[1];
-        eight_of_each_row<PARTS, 1>(qkv, one_at, part_stride, parts, one);
-        const uint32_t words[4] = {one[0].x, one[0].y, one[0].z, one[0].w};
-        if (mine) {
+      if (!whole) single |= 1u << i;
+      else if (pos % 8 == 0) starts = row;
+    }
+    uint4 raw[8];
+    size_t raw_at[8];
+    if (of_pieces && starts >= 0) {      // raw: token t's dims 8 c .. 8 c + 7
+      uint16_t* block = block_of(starts);
+      const int token = pos_of(starts) % BH_PAGE;
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            block[bh_value_index(kv_order, pos % BH_PAGE, 8 * c + e, HD)] = (uint16_t)(words[e / 2] >> (16 * (e % 2)));
-        }
-        continue;
-      }
-      uint4 raw[8];   // token t's dims 8 c .. 8 c + 7
-      size_t raw_at[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) raw_at[t] = src + (size_t)(row + t) * fused;
+      for (int t = 0; t < 8; ++t) raw_at[t] = src + (size_t)(starts + t) * fused;
       eight_of_each_row<PARTS, 8>(qkv, raw_at, part_stride, parts, raw);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {   // dim 8 c + e of the eight tokens: the halves e % 2 of the words e / 2
@@ -554,7 +565,24 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
         piece.y = __builtin_amdgcn_perm(word[3], word[2], pick);
         piece.z = __builtin_amdgcn_perm(word[5], word[4], pick);
         piece.w = __builtin_amdgcn_perm(word[7], word[6], pick);
-        if (mine) *reinterpret_cast<uint4*>(block + bh_value_index(kv_order, pos % BH_PAGE, 8 * c + e, HD)) = piece;
+        if (mine) *reinterpret_cast<uint4*>(block + bh_value_index(kv_order, token, 8 * c + e, HD)) = piece;
+      }
+    }
+    if (!of_pieces && single) {      // raw: the eight rows' own, or, of those that are not written here, the first one's that is
+      const int needed = __builtin_ctz(single);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) raw_at[t] = src + (size_t)(8 * group + (single >> t & 1u ? t : needed)) * fused;
+      eight_of_each_row<PARTS, 8>(qkv, raw_at, part_stride, parts, raw);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (!(single >> i & 1u)) continue;
+        uint16_t* block = block_of(8 * group + i);
+        const int token = pos_of(8 * group + i) % BH_PAGE;
+        const uint32_t words[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+        if (mine) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) block[bh_value_index(kv_order, token, 8 * c + e, HD)] = (uint16_t)(words[e / 2] >> (16 * (e % 2)));
+        }
       }
     }
     return;
@@ -567,16 +595,19 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
   const bool is_q = head < H;
   // All of a wave's loads are asked for before anything is computed: RPW rows' 16 bytes, their positions and, behind
   // those, their angles.  (With one row per wave the three waits in a row, for so little data each, were the kernel's time.)
-  int pos[RPW];
+  int pos[RPW], seq[RPW], page[RPW];
   uint4 raw[RPW];
   size_t raw_at[RPW];
 #pragma unroll
   for (int r = 0; r < RPW; ++r) {
     const int row = min(first_row + r, n_rows - 1);
     pos[r] = positions[row];
+    seq[r] = is_q ? 0 : row_seq[row];
     raw_at[r] = ((size_t)row * (H + 2 * KVH) + head) * HD + 8 * c;
   }
   eight_of_each_row<PARTS, RPW>(qkv, raw_at, (size_t)n_rows * (H + 2 * KVH) * HD, parts, raw);
+#pragma unroll
+  for (int r = 0; r < RPW; ++r) page[r] = is_q ? 0 : page_table[(size_t)seq[r] * table_stride + pos[r] / BH_PAGE];
   const TW* weight = is_q ? q_weight : k_weight;
   float wv[8];
   if (weight != nullptr) load_eight(weight + 8 * c, wv);
@@ -623,9 +654,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
       *reinterpret_cast<uint4*>(q_out + ((size_t)row * H + head) * HD + 8 * c) = packed;
       continue;
     }
-    const int page = page_table[(size_t)row_seq[row] * table_stride + pos[r] / BH_PAGE];
     const int token = pos[r] % BH_PAGE, kv_head = head - H;
-    uint16_t* block = k_pages + ((size_t)page * KVH + kv_head) * BH_PAGE * HD;
+    uint16_t* block = k_pages + ((size_t)page[r] * KVH + kv_head) * BH_PAGE * HD;
     *reinterpret_cast<uint4*>(block + bh_key_index(kv_order, token, 8 * c, HD)) = packed;   // 8 dims lie together in both orders
   }
 }
@@ -643,7 +673,7 @@ static int qk_rows_form(const void* qkv, int parts, void* q_out, const void* q_w
   const int lanes_per_head = hd / 8, heads_per_wave = 64 / lanes_per_head, main_heads = write_kv ? H + KVH : H;
   constexpr int RPW = 4;
   const long main_waves = (long)((n_rows + RPW - 1) / RPW) * ((main_heads + heads_per_wave - 1) / heads_per_wave);
-  const long value_waves = write_kv ? (long)((n_rows + 7) / 8) * ((KVH + heads_per_wave - 1) / heads_per_wave) : 0;
+  const long value_waves = write_kv ? 2L * ((n_rows + 7) / 8) * ((KVH + heads_per_wave - 1) / heads_per_wave) : 0;
   BH_REQUIRE(main_waves + value_waves < (1L << 31), "qk_norm_rope: too many rows");
   BH_REQUIRE(w_dtype == BH_F32 || w_dtype == BH_BF16, "qk_norm_rope: unknown weight dtype %d", w_dtype);
   dim3 wide_grid((unsigned)((main_waves + value_waves + 3) / 4)), wide_block(4 * BH_WAVE);
