@@ -65,13 +65,31 @@ __global__ void embed_kernel(const int32_t* __restrict__ tokens, const int32_t* 
   for (int i = threadIdx.x; i < width; i += blockDim.x) dst[i] = to_f32(src[i]);
 }
 
+// The same in pieces of four elements, one a thread: with single elements in a loop a row of 4,096 is 16 trips to memory one after
+// the other (8 rows of a decode step 7.7 -> 3.7 us).
+template <typename T>
+__global__ __launch_bounds__(256) void embed_pieces_kernel(const int32_t* __restrict__ tokens, const int32_t* __restrict__ token_src,
+                                                           const int32_t* __restrict__ fed, const T* __restrict__ table,
+                                                           float* __restrict__ out, int width, int table_rows) {
+  const int row = blockIdx.x, i = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (i >= width) return;
+  int token = tokens[row];
+  if (token_src != nullptr && token_src[row] >= 0) token = fed[token_src[row]];
+  if (token < 0 || token >= table_rows) token = 0;
+  *reinterpret_cast<float4*>(out + (size_t)row * width + i) = load_four(table + (size_t)token * width + i);
+}
+
 extern "C" int bh_embed(const int32_t* tokens, const int32_t* token_src, const int32_t* fed, const void* table,
                         int table_dtype, float* out, int n_rows, int width, int table_rows, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0 && table_rows > 0, "embed: rows %d, width %d and table rows %d must be positive",
              n_rows, width, table_rows);
   BH_REQUIRE((token_src == nullptr) == (fed == nullptr), "embed: fed tokens and their row indices come together");
   dim3 grid(n_rows), block(256);
-  if (table_dtype == BH_F32)
+  if (width % 4 == 0 && (width + 1023) / 1024 <= 65535 && ((uintptr_t)table | (uintptr_t)out) % 16 == 0 && (table_dtype == BH_F32 || table_dtype == BH_BF16)) {
+    grid.y = (unsigned)((width + 1023) / 1024);
+    if (table_dtype == BH_F32) embed_pieces_kernel<float><<<grid, block, 0, stream>>>(tokens, token_src, fed, (const float*)table, out, width, table_rows);
+    else embed_pieces_kernel<bf16_t><<<grid, block, 0, stream>>>(tokens, token_src, fed, (const bf16_t*)table, out, width, table_rows);
+  } else if (table_dtype == BH_F32)
     embed_kernel<float><<<grid, block, 0, stream>>>(tokens, token_src, fed, (const float*)table, out, width, table_rows);
   else if (table_dtype == BH_BF16)
     embed_kernel<bf16_t><<<grid, block, 0, stream>>>(tokens, token_src, fed, (const bf16_t*)table, out, width,
