@@ -228,17 +228,23 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // workgroups than compute units, where the second workgroup is worth more than the overlap.
 // FORMED = scores are more than a scaled product (struct ScoreForm): they are made in full, and exponentials taken of them as they
 // are (scale_log2 is then log2(e)).
+// A workgroup of a FUSED step that is not LEAN has a fifth wave (heads of up to 128, whose pages leave two waves a SIMD their registers):
+// it norms and rotates the queries for all of them, while the others ask for their first pages and nothing else, and then takes the new
+// key, beside the pages.  (Every wave its own queries under its first page's loads, and the new key by the first wave behind its pages:
+// 4 sequences of 1,000 keys, 16 heads on 4 12.5 us, 11.0 now, of which the faster combining is 1.)
+__host__ __device__ constexpr bool fifth_wave(int ns, int fused, bool lean) { return fused && !lean && ns <= 4; }
 template <int NS, bool STREAM, int FUSED, bool LEAN = false, bool FORMED = false>
-__global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
+__global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 2 : 1)) void attention_mfma_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
     const int32_t* __restrict__ page_table, int table_stride, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ seq_start, int H, int KVH, float scale_log2, int window, int n_splits,
     int pages_per_split, int tile_groups, FusedQkv fused, int out_block_rows, HeadEnd finish, ScoreForm form) {
-  constexpr int HD = 32 * NS;
-  __shared__ float sm_m[4][16];
-  __shared__ float sm_l[4][16];
-  __shared__ float sm_o[4][16][HD + 1];
+  constexpr int HD = 32 * NS, WAVES = fifth_wave(NS, FUSED, LEAN) ? 5 : 4;
+  __shared__ u32x4_t sm_q[WAVES == 5 ? NS : 1][64];
+  __shared__ float sm_m[WAVES][16];
+  __shared__ float sm_l[WAVES][16];
+  __shared__ __attribute__((aligned(16))) float sm_o[WAVES][16][HD + 4];      // rows of 16-byte pieces, 4 banks apart
 
   const int tile = blockIdx.x % tile_groups, unit = blockIdx.x / tile_groups;
   const int kvh = unit % KVH, z = unit / KVH;
@@ -254,7 +260,8 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
   const int first_guess = split * pages_per_split + (int)(threadIdx.x / 64);
   const int page_guess = first_guess < table_stride ? table[first_guess] : 0;
 
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  // (a scalar: the fifth wave's way parts from the others', with a barrier on both)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int j = lane % 16, g = lane / 16;
   const int wanted = tile * 16 + j;
   const int c = wanted < n_cols ? wanted : n_cols - 1;
@@ -270,16 +277,20 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
   // FUSED: the raw rows and what norms and rotates them are asked for here and used once the first page's
   // loads are under way (q) and after the pages (the new key and value).
   u32x4_t q_raw[NS], k_raw[NS];
-  uint16_t new_value[2 * NS];   // dim 16 dt + j of the new value
+  uint16_t new_value[2 * NS];   // dim 16 dt + j of the new value, as the cache takes it
+  u32x2_t value_raw[2 * NS];    // dims 16 dt + 4 g .. + 3 of it, as the lane's sums do
   std::conditional_t<FUSED == 2, PairPrep<NS>, HeadPrep<NS>> q_prep, k_prep;
   bool q_ready = !FUSED;
-  const bool takes_new_key = FUSED && fused.write_kv && split == n_splits - 1 && wave == 0;
+  const bool new_key_here = FUSED && fused.write_kv && split == n_splits - 1, takes_new_key = new_key_here && wave == (WAVES == 5 ? 4 : 0);
   auto ask_new_key = [&]() {   // one row per sequence: every lane's row is this row
     const uint16_t* qkv_row = fused.qkv + (size_t)row * fused.row_stride;
 #pragma unroll
     for (int s = 0; s < NS; ++s) k_raw[s] = load16(qkv_row + fused.k_first + kvh * HD + 32 * s + 8 * g);
 #pragma unroll
-    for (int dt = 0; dt < 2 * NS; ++dt) new_value[dt] = qkv_row[fused.v_first + kvh * HD + 16 * dt + j];
+    for (int dt = 0; dt < 2 * NS; ++dt) {
+      new_value[dt] = qkv_row[fused.v_first + kvh * HD + 16 * dt + j];
+      value_raw[dt] = *reinterpret_cast<const u32x2_t*>(qkv_row + fused.v_first + kvh * HD + 16 * dt + 4 * g);
+    }
     // the rotation's numbers are q's, or (LEAN: q's are gone by then) asked for again
     if constexpr (FUSED == 2) {
       k_prep.ask(fused.k_weight, fused.weight_f32);
@@ -288,7 +299,7 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
       k_prep.ask(fused.k_weight, fused.weight_f32, LEAN ? fused.cos_table : nullptr, LEAN ? fused.sin_table : nullptr, pos_row, g);
     }
   };
-  if (FUSED) {
+  auto ask_q = [&]() {
     const uint16_t* qkv_row = fused.qkv + (size_t)row * fused.row_stride;
 #pragma unroll
     for (int s = 0; s < NS; ++s) q_raw[s] = load16(qkv_row + (size_t)head * HD + 32 * s + 8 * g);
@@ -298,7 +309,9 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
     } else {
       q_prep.ask(fused.q_weight, fused.weight_f32, fused.cos_table, fused.sin_table, pos_row, g);
     }
-    if (takes_new_key && !LEAN) ask_new_key();
+  };
+  if constexpr (FUSED) {
+    if (WAVES == 4) ask_q();
   } else {
     const uint16_t* qp = q + ((size_t)row * H + head) * HD + 8 * g;
 #pragma unroll
@@ -416,33 +429,9 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
     }
   };
 
-  // a page's number is asked for one page early
-  int page_ahead = (begin + wave < end) ? (begin + wave == first_guess ? page_guess : table[begin + wave]) : 0;
-  for (int p = begin + wave; p < end; p += 4) {
-    const int page = page_ahead;
-    if (p + 4 < end) page_ahead = table[p + 4];
-    const uint16_t* kb = k_pages + ((size_t)page * KVH + kvh) * BH_PAGE * HD;
-    const uint16_t* vb = v_pages + ((size_t)page * KVH + kvh) * HD * BH_PAGE;
-    u32x4_t k_vec[4][NS], v_vec[2 * NS][2];
-    // the cache lies in pieces (BH_KV_PIECES): every load instruction covers 1 KB of contiguous memory
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int s = 0; s < NS; ++s) k_vec[t][s] = load16_cache<STREAM>(kb + ((t * NS + s) * 64 + lane) * 8);
-#pragma unroll
-    for (int dt = 0; dt < 2 * NS; ++dt) {
-      v_vec[dt][0] = load16_cache<STREAM>(vb + ((dt * 2) * 64 + lane) * 8);
-      v_vec[dt][1] = load16_cache<STREAM>(vb + ((dt * 2 + 1) * 64 + lane) * 8);
-    }
-    if (FUSED && !q_ready) finish_q();   // under the page's loads
-    attend(k_vec, v_vec, p, pos, lo, pos_max, pos_min, lo_max);
-  }
-
-  if (takes_new_key) {
-    // The new key and value of this (sequence, kv head): normed and rotated here, attended to as a page in
-    // which only their own slot is visible, and written into the cache.
-    if (!q_ready) finish_q();
-    if (LEAN) ask_new_key();
+  // The new key and value of this (sequence, kv head): normed and rotated here, attended to, and written into the cache.  The key stands
+  // in all 16 rows of the product's operand, so that every lane has its column's score; the value is added in plain arithmetic.
+  auto take_new_key = [&]() {
     float x[NS][8];
     widen_head<NS>(x, k_raw);
     if (!LEAN) k_prep.take_angles(q_prep);
@@ -452,23 +441,26 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
       k_prep.apply(x, fused.k_weight != nullptr, fused.weight_f32, fused.eps, fused.cos_table != nullptr);
     u32x4_t new_key[NS];
     pack_head<NS>(new_key, x);
+    f32x4_t product = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; ++s) product = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(new_key[s]), q_vec[s], product, 0, 0, 0);
+    float score = product[0];
+    if constexpr (FORMED) {
+      score *= col_scale;
+      if (cap_rate > 0.f) score = capped_score(score, form.cap, cap_rate);
+    }
+    const float new_max = fmaxf(run_max, score);
+    const float shift = (new_max == -INFINITY) ? 0.f : -new_max * scale_log2;
+    const float alpha = (run_max == new_max) ? 1.0f : __builtin_amdgcn_exp2f((run_max - new_max) * scale_log2);
+    const float p = __builtin_amdgcn_exp2f(fmaf(score, scale_log2, shift));
+    run_sum = run_sum * alpha + (g == 0 ? p : 0.f);      // once for the column
+    run_max = new_max;
+#pragma unroll
+    for (int dt = 0; dt < 2 * NS; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[dt][r] = fmaf(p, bf16_bits_to_f32((uint16_t)(value_raw[dt][r / 2] >> (16 * (r % 2)))), o[dt][r] * alpha);
     const int token = pos_row % BH_PAGE;
     const int token_t = 2 * (token / 32) + (token / 4) % 2, token_j = 4 * ((token / 8) % 4) + token % 4;
-    const int token_u = token / 32, token_g = (token % 32) / 8, token_w = token % 8;
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    u32x4_t k_vec[4][NS], v_vec[2 * NS][2];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int s = 0; s < NS; ++s) k_vec[t][s] = (t == token_t && j == token_j) ? new_key[s] : zero;
-#pragma unroll
-    for (int dt = 0; dt < 2 * NS; ++dt) {
-      u32x4_t piece = zero;
-      piece[token_w / 2] = (uint32_t)new_value[dt] << (16 * (token_w % 2));
-      v_vec[dt][0] = (token_u == 0 && g == token_g) ? piece : zero;
-      v_vec[dt][1] = (token_u == 1 && g == token_g) ? piece : zero;
-    }
-    attend(k_vec, v_vec, pos_row / BH_PAGE, pos_row, pos_row, pos_row, pos_row, pos_row);
     const int page = table[pos_row / BH_PAGE];
     uint16_t* kb = fused.k_pages + ((size_t)page * KVH + kvh) * BH_PAGE * HD;
     uint16_t* vb = fused.v_pages + ((size_t)page * KVH + kvh) * HD * BH_PAGE;
@@ -481,9 +473,63 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
 #pragma unroll
       for (int dt = 0; dt < 2 * NS; ++dt) vb[bh_value_index(BH_KV_PIECES, token, 16 * dt + j, HD)] = new_value[dt];
     }
+  };
+
+  // a page's number is asked for one page early
+  int page_ahead = (begin + wave < end) ? (begin + wave == first_guess ? page_guess : table[begin + wave]) : 0;
+  u32x4_t k_vec[4][NS], v_vec[2 * NS][2];
+  auto ask_page = [&](int p) {
+    const int page = page_ahead;
+    if (p + 4 < end) page_ahead = table[p + 4];
+    const uint16_t* kb = k_pages + ((size_t)page * KVH + kvh) * BH_PAGE * HD;
+    const uint16_t* vb = v_pages + ((size_t)page * KVH + kvh) * HD * BH_PAGE;
+    // the cache lies in pieces (BH_KV_PIECES): every load instruction covers 1 KB of contiguous memory
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) k_vec[t][s] = load16_cache<STREAM>(kb + ((t * NS + s) * 64 + lane) * 8);
+#pragma unroll
+    for (int dt = 0; dt < 2 * NS; ++dt) {
+      v_vec[dt][0] = load16_cache<STREAM>(vb + ((dt * 2) * 64 + lane) * 8);
+      v_vec[dt][1] = load16_cache<STREAM>(vb + ((dt * 2 + 1) * 64 + lane) * 8);
+    }
+  };
+  // What the fifth wave hands over.  The barrier waits for LDS only: the first page stays on its way.
+  auto meet = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));      // vmcnt and expcnt as they are, lgkmcnt 0
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (WAVES == 5 && wave == 4) {
+    ask_q();
+    if (new_key_here) ask_new_key();
+    finish_q();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sm_q[s][lane] = __builtin_bit_cast(u32x4_t, q_vec[s]);
+    meet();
+  } else {
+    int p = begin + wave;
+    if (WAVES == 5) {
+      if (p < end) ask_page(p);
+      meet();
+#pragma unroll
+      for (int s = 0; s < NS; ++s) q_vec[s] = as_bf16x8(sm_q[s][lane]);
+    }
+    for (bool asked = WAVES == 5; p < end; p += 4, asked = false) {
+      if (!asked) ask_page(p);
+      if (FUSED && WAVES == 4 && !q_ready) finish_q();   // under the page's loads
+      attend(k_vec, v_vec, p, pos, lo, pos_max, pos_min, lo_max);
+    }
   }
 
-  // merge the four waves: lane (j, g) holds O^T[16dt + 4g + r, j]
+  if (takes_new_key) {
+    if (WAVES == 4) ask_new_key();
+    if (WAVES == 4 && !q_ready) finish_q();
+    take_new_key();
+  }
+
+  // merge the waves: lane (j, g) holds O^T[16dt + 4g + r, j]
   {
     float lane_sum = run_sum;
     lane_sum += __shfl_xor(lane_sum, 16, 64);
@@ -493,82 +539,116 @@ __global__ __launch_bounds__(256, (LEAN ? 2 : 1)) void attention_mfma_kernel(
       sm_l[wave][j] = lane_sum;
     }
 #pragma unroll
-    for (int dt = 0; dt < 2 * NS; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sm_o[wave][j][16 * dt + 4 * g + r] = o[dt][r];
+    for (int dt = 0; dt < 2 * NS; ++dt) *reinterpret_cast<f32x4_t*>(&sm_o[wave][j][16 * dt + 4 * g]) = o[dt];
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * HD; e += 256) {
-      const int col = e / HD, d = e % HD;
-      const int cc = tile * 16 + col;
-      if (cc >= n_cols) continue;
-      float top = fmaxf(fmaxf(sm_m[0][col], sm_m[1][col]), fmaxf(sm_m[2][col], sm_m[3][col]));
-      const float safe_top = (top == -INFINITY) ? 0.f : top;
-      float sum = 0.f, value = 0.f;
+    if (WAVES == 5 && wave == 4) return;
+    // 16 threads a column, each with neighbouring dimensions of it
+    constexpr int EACH = HD / 16;
+    const int col = threadIdx.x / 16, d0 = threadIdx.x % 16 * EACH, cc = tile * 16 + col;
+    if (cc >= n_cols) return;
+    float top = fmaxf(fmaxf(sm_m[0][col], sm_m[1][col]), fmaxf(sm_m[2][col], sm_m[3][col]));
+    if (WAVES == 5) top = fmaxf(top, sm_m[WAVES - 1][col]);
+    const float safe_top = (top == -INFINITY) ? 0.f : top;
+    float sum = 0.f, value[EACH];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float f = exp2f(sm_m[v][col] - safe_top);
-        sum += sm_l[v][col] * f;
-        value += sm_o[v][col][d] * f;
+    for (int d = 0; d < EACH; ++d) value[d] = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) {
+      if (v == 4 && !new_key_here) break;
+      const float f = exp2f(sm_m[v][col] - safe_top);
+      sum += sm_l[v][col] * f;
+#pragma unroll
+      for (int d = 0; d < EACH; d += 2) {
+        const float2 pair = *reinterpret_cast<const float2*>(&sm_o[v][col][d0 + d]);
+        value[d] += pair.x * f;
+        value[d + 1] += pair.y * f;
       }
-      const size_t column = (size_t)(row0 + cc / G) * H + kvh * G + cc % G;
-      if (n_splits == 1) {   // out_block_rows: the output [rows][H * HD] lies in blocks of that many rows (bh_rows_index)
-        // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
-        const int out_row = row0 + cc / G, out_head = kvh * G + cc % G;
-        if (finish.sinks) sum += exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top);
-        value *= head_gate<bf16_t>(finish, out_row, out_head);
-        out[bh_rows_index(out_block_rows, out_row, out_head * HD + d, H * HD)] = f32_to_bf16_bits(value / sum);
-      } else {
-        part_o[(column * n_splits + split) * HD + d] = value;
-        if (d == 0) {
-          part_ml[(column * n_splits + split) * 2] = top;
-          part_ml[(column * n_splits + split) * 2 + 1] = sum;
-        }
+    }
+    const int out_row = row0 + cc / G, out_head = kvh * G + cc % G;
+    const size_t column = (size_t)out_row * H + out_head;
+    if (n_splits == 1) {   // out_block_rows: the output [rows][H * HD] lies in blocks of that many rows (bh_rows_index)
+      // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
+      if (finish.sinks) sum += exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top);
+      const float gate = head_gate<bf16_t>(finish, out_row, out_head);
+#pragma unroll
+      for (int d = 0; d < EACH; d += 2)   // (two neighbours from an even dimension on are neighbours in blocks too)
+        *reinterpret_cast<uint32_t*>(out + bh_rows_index(out_block_rows, out_row, out_head * HD + d0 + d, H * HD)) =
+            (uint32_t)f32_to_bf16_bits(value[d] * gate / sum) | ((uint32_t)f32_to_bf16_bits(value[d + 1] * gate / sum) << 16);
+    } else {
+      float* to = part_o + (column * n_splits + split) * HD + d0;
+#pragma unroll
+      for (int d = 0; d < EACH; d += 2) *reinterpret_cast<float2*>(to + d) = make_float2(value[d], value[d + 1]);
+      if (d0 == 0) {
+        part_ml[(column * n_splits + split) * 2] = top;
+        part_ml[(column * n_splits + split) * 2 + 1] = sum;
       }
     }
   }
 }
 
-// One block per column.  Nothing here may wait for one split's numbers before asking for the next
-// one's: with 32 splits that is 32 trips to the L2 in a row.  So the lanes of a wave fetch the splits'
-// (maximum, sum) pairs side by side, and the partial outputs are fetched WIDTH splits at a time (8, or 4 where there are
-// no more); the sums run over the splits in their order either way.
-template <int WIDTH>
-__global__ void attention_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                         uint16_t* __restrict__ out, int n_splits, int HD, int H, int out_block_rows,
-                                         HeadEnd finish) {
+// One block per column, a group of 64 or 128 threads (a dimension each; heads of more take the others in turn) for every eight splits.
+// Nothing here may wait for one split's numbers before asking for the next one's, nor for the maxima before asking for the outputs: a
+// thread asks for all eight at once and makes their weights itself, from numbers that are the same for its wave.  The groups are merged
+// through LDS.  The sums run over the splits in their order.  (One group for all, by eights, and the maxima and sums over the lanes of a
+// wave: 3.1 us of a decode step's launches at up to eight splits, of which the launch is 1.7; 2.2 now.)
+#define COMBINE_SPLITS 8      // a group's; four where there are no more in all
+template <int SPLITS>
+__global__ __launch_bounds__(1024) void attention_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                                 uint16_t* __restrict__ out, int n_splits, int HD, int H, int out_block_rows,
+                                                                 HeadEnd finish, int dims) {
+  __shared__ float sm_value[COMBINE_SPLITS][256], sm_top[COMBINE_SPLITS], sm_sum[COMBINE_SPLITS];
+  const int row = blockIdx.x / H, head = blockIdx.x % H, groups = (n_splits + SPLITS - 1) / SPLITS;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / dims), dim = threadIdx.x % dims, first = group * SPLITS;
   const size_t column = blockIdx.x;
-  const float gate = head_gate<bf16_t>(finish, (int)(column / H), (int)(column % H));
   const float* ml = part_ml + column * n_splits * 2;
-  const int lane = threadIdx.x % BH_WAVE;
-  // the first splits' outputs are asked for beside the maxima and sums, not after them
-  float first_part[WIDTH];
+  const float* outputs = part_o + column * n_splits * HD;
+  float part[SPLITS], weight[SPLITS], share[SPLITS];
 #pragma unroll
-  for (int u = 0; u < WIDTH; ++u)
-    first_part[u] = threadIdx.x < HD ? part_o[(column * n_splits + (u < n_splits ? u : n_splits - 1)) * HD + threadIdx.x] : 0.f;
-  float top = -INFINITY;
-  for (int s = lane; s < n_splits; s += BH_WAVE) top = fmaxf(top, ml[2 * s]);
+  for (int u = 0; u < SPLITS; ++u) {
+    const int s = min(first + u, n_splits - 1);
+    part[u] = dim < HD ? outputs[s * HD + dim] : 0.f;
+    weight[u] = ml[2 * s];
+    share[u] = ml[2 * s + 1];
+  }
+  const float gate = head_gate<bf16_t>(finish, row, head);
+  float top = weight[0];
 #pragma unroll
-  for (int off = BH_WAVE / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, BH_WAVE));
-  float sum = 0.f;   // in the order: each lane its splits upwards, then the lanes pairwise
-  for (int s = lane; s < n_splits; s += BH_WAVE) sum += ml[2 * s + 1] * exp2f(ml[2 * s] - top);
+  for (int u = 1; u < SPLITS; ++u) top = fmaxf(top, weight[u]);
+  const float safe_top = top == -INFINITY ? 0.f : top;
+  float sum = 0.f;
 #pragma unroll
-  for (int off = BH_WAVE / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, BH_WAVE);
-  if (finish.sinks) sum += exp2f(finish.sinks[column % H] * 1.4426950408889634f - top);      // the sink's term, once for the whole row
-  const float inv = gate / sum;
-  for (int d = threadIdx.x; d < HD; d += blockDim.x) {
+  for (int u = 0; u < SPLITS; ++u) {
+    // (arguments <= 0; results below the normal range may be 0)
+    weight[u] = first + u < n_splits ? __builtin_amdgcn_exp2f(weight[u] - safe_top) : 0.f;
+    sum += share[u] * weight[u];
+  }
+  auto value_at = [&](int d) {
     float value = 0.f;
-    for (int s0 = 0; s0 < n_splits; s0 += WIDTH) {
-      float weight[WIDTH], part[WIDTH];
 #pragma unroll
-      for (int u = 0; u < WIDTH; ++u) {
-        const int s = s0 + u < n_splits ? s0 + u : n_splits - 1;
-        weight[u] = s0 + u < n_splits ? ml[2 * s] : -INFINITY;
-        part[u] = (s0 == 0 && d == threadIdx.x) ? first_part[u] : part_o[(column * n_splits + s) * HD + d];
-      }
-#pragma unroll
-      for (int u = 0; u < WIDTH; ++u) value += part[u] * exp2f(weight[u] - top);
-    }
-    out[bh_rows_index(out_block_rows, (int)(column / H), (int)(column % H) * HD + d, H * HD)] = f32_to_bf16_bits(value * inv);
+    for (int u = 0; u < SPLITS; ++u) value += (d == dim ? part[u] : outputs[min(first + u, n_splits - 1) * HD + d]) * weight[u];
+    return value;
+  };
+  auto write = [&](int d, float value, float total, float highest) {
+    // a sink: one more term exp(sinks[head]) in the softmax's sum
+    if (finish.sinks) total += exp2f(finish.sinks[head] * 1.4426950408889634f - highest);
+    out[bh_rows_index(out_block_rows, row, head * HD + d, H * HD)] = f32_to_bf16_bits(value * (gate / total));
+  };
+  if (groups == 1) {
+    for (int d = dim; d < HD; d += dims) write(d, value_at(d), sum, safe_top);
+    return;
+  }
+  for (int d = dim; d < HD; d += dims) sm_value[group][d] = value_at(d);
+  if (dim == 0) sm_top[group] = top, sm_sum[group] = sum;
+  __syncthreads();
+  if (group != 0) return;
+  for (int k = 1; k < groups; ++k) top = fmaxf(top, sm_top[k]);
+  const float highest = top == -INFINITY ? 0.f : top;
+  float total = 0.f;
+  for (int k = 0; k < groups; ++k) total += sm_sum[k] * __builtin_amdgcn_exp2f(sm_top[k] - highest);
+  for (int d = dim; d < HD; d += dims) {
+    float value = 0.f;
+    for (int k = 0; k < groups; ++k) value += sm_value[k][d] * __builtin_amdgcn_exp2f(sm_top[k] - highest);
+    write(d, value, total, highest);
   }
 }
 
@@ -666,9 +746,9 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
              "attention_bf16: the output's rows lie in blocks of 8 or 16, or one after the other (0), not %d", out_blocked);
   const int tile_groups = tiles, z_count = n_seqs * n_splits;
   const bool lean = (long)tiles * KVH * z_count > bh_compute_units();   // more workgroups than compute units: two of them per unit
-  dim3 grid(tile_groups * KVH * z_count), block(256);
+  dim3 grid(tile_groups * KVH * z_count);
 #define BH_ATT_ONE(NS, STREAM, FUSED, ...)                                                                      \
-  attention_mfma_kernel<NS, STREAM, FUSED, __VA_ARGS__><<<grid, block, 0, stream>>>(                          \
+  attention_mfma_kernel<NS, STREAM, FUSED, __VA_ARGS__><<<grid, is_fused && !lean && NS <= 4 ? 320 : 256, 0, stream>>>(        \
       (const uint16_t*)q, (uint16_t*)out, (float*)part_o, (float*)part_ml, (const uint16_t*)k_pages,            \
       (const uint16_t*)v_pages, page_table, table_stride, positions, seq_start, H, KVH, scale_log2, window,     \
       n_splits, per, tile_groups, fused, out_blocked, finish, form)
@@ -699,13 +779,14 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
 #undef BH_ATT_ONE
   if (int status = bh_check_launch("attention_mfma")) return status;
   if (n_splits > 1) {
-    const dim3 columns(n_rows * H), threads(hd >= 128 ? 128 : 64);
-    if (n_splits <= 4)
-      attention_combine_kernel<4><<<columns, threads, 0, stream>>>((const float*)part_o, (const float*)part_ml, (uint16_t*)out,
-                                                                   n_splits, hd, H, out_blocked, finish);
-    else
-      attention_combine_kernel<8><<<columns, threads, 0, stream>>>((const float*)part_o, (const float*)part_ml, (uint16_t*)out,
-                                                                   n_splits, hd, H, out_blocked, finish);
+    BH_REQUIRE(n_splits <= COMBINE_SPLITS * COMBINE_SPLITS, "attention_bf16: keys in %d splits, at most %d are combined", n_splits, COMBINE_SPLITS * COMBINE_SPLITS);
+    const int dims = hd >= 128 ? 128 : 64, groups = (n_splits + COMBINE_SPLITS - 1) / COMBINE_SPLITS;
+#define BH_COMBINE(SPLITS)                                                                                                                  \
+  attention_combine_kernel<SPLITS><<<n_rows * H, dims * groups, 0, stream>>>((const float*)part_o, (const float*)part_ml, (uint16_t*)out, \
+                                                                             n_splits, hd, H, out_blocked, finish, dims)
+    if (n_splits <= 4) BH_COMBINE(4);
+    else BH_COMBINE(COMBINE_SPLITS);
+#undef BH_COMBINE
     return bh_check_launch("attention_combine");
   }
   return 0;
