@@ -227,18 +227,18 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // in registers is gone while the pages stream, so that two workgroups fit a compute unit.  For launches of more
 // workgroups than compute units, where the second workgroup is worth more than the overlap.
 // FORMED = scores are more than a scaled product (struct ScoreForm): they are made in full, and exponentials taken of them as they
-// are (scale_log2 is then log2(e)).
+// are (scale_log2 is then log2(e)).  Otherwise a column's factor is in scale_log2 (ScoreForm::scaled_only).
 // A workgroup of a FUSED step that is not LEAN has a fifth wave (heads of up to 128, whose pages leave two waves a SIMD their registers):
 // it norms and rotates the queries for all of them, while the others ask for their first pages and nothing else, and then takes the new
 // key, beside the pages.  (Every wave its own queries under its first page's loads, and the new key by the first wave behind its pages:
 // 4 sequences of 1,000 keys, 16 heads on 4 12.5 us, 11.0 now, of which the faster combining is 1.)
 __host__ __device__ constexpr bool fifth_wave(int ns, int fused, bool lean) { return fused && !lean && ns <= 4; }
-template <int NS, bool STREAM, int FUSED, bool LEAN = false, bool FORMED = false>
+template <int NS, bool STREAM, int FUSED, bool LEAN = false, int FORMED = 0>
 __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 2 : 1)) void attention_mfma_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
     const int32_t* __restrict__ page_table, int table_stride, const int32_t* __restrict__ positions,
-    const int32_t* __restrict__ seq_start, int H, int KVH, float scale_log2, int window, int n_splits,
+    const int32_t* __restrict__ seq_start, int H, int KVH, int window, int n_splits,
     int pages_per_split, int tile_groups, FusedQkv fused, int out_block_rows, HeadEnd finish, ScoreForm form) {
   constexpr int HD = 32 * NS, WAVES = fifth_wave(NS, FUSED, LEAN) ? 5 : 4;
   __shared__ u32x4_t sm_q[WAVES == 5 ? NS : 1][64];
@@ -270,8 +270,9 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
   const bool new_key_apart = FUSED && fused.write_kv;   // the key at pos_row is not in the cache yet
   const int pos = new_key_apart ? pos_row - 1 : pos_row;   // the last key the row takes from the cache (-1: none)
   const int lo = bh_first_visible(pos_row, window);
-  // FORMED: what this lane's column makes of its products
-  const float col_scale = FORMED ? query_scale(form, pos_row) : 0.f, cap_rate = FORMED && form.cap > 0.f ? 2.0f * BH_LOG2E / form.cap : 0.f;
+  // what this lane's column makes of its products (FORMED), and of its scores or else its products into powers of two
+  const float scale_log2 = FORMED ? BH_LOG2E : query_scale(form, pos_row) * BH_LOG2E;
+  const float col_scale = FORMED ? query_scale(form, pos_row) : 0.f, cap_rate = FORMED == 2 ? 2.0f * BH_LOG2E / form.cap : 0.f;
   const float slope = FORMED && form.slopes ? form.slopes[head] : 0.f;
   bf16x8_t q_vec[NS];
   // FUSED: the raw rows and what norms and rotates them are asked for here and used once the first page's
@@ -366,7 +367,7 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
         for (int r = 0; r < 4; ++r) {
           const float off = slope * (float)(key0 + 32 * (t / 2) + 4 * (t % 2) + r - pos_row);
           const float s = st[t][r] * col_scale;
-          st[t][r] = (cap_rate > 0.f ? capped_score(s, form.cap, cap_rate) : s) + off;
+          st[t][r] = (FORMED == 2 ? capped_score(s, form.cap, cap_rate) : s) + off;
         }
     }
     // Online softmax with few instructions: the maximum is taken over the raw scores, the scale
@@ -447,7 +448,7 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
     float score = product[0];
     if constexpr (FORMED) {
       score *= col_scale;
-      if (cap_rate > 0.f) score = capped_score(score, form.cap, cap_rate);
+      if (FORMED == 2) score = capped_score(score, form.cap, cap_rate);
     }
     const float new_max = fmaxf(run_max, score);
     const float shift = (new_max == -INFINITY) ? 0.f : -new_max * scale_log2;
@@ -730,8 +731,7 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   const int tiles = (max_rows_per_seq * G + 15) / 16;
   const int pages = max_position / BH_PAGE + 1;
   const int per = (pages + n_splits - 1) / n_splits;
-  const bool formed = !form.plain();
-  const float scale_log2 = formed ? BH_LOG2E : form.scale * BH_LOG2E;
+  const int formed = bh_formed(form);
   BH_REQUIRE((long)tiles * KVH * n_seqs * n_splits < (1L << 31), "attention_bf16: too many workgroups");
   const bool is_fused = fused.qkv != nullptr;
   BH_REQUIRE(!is_fused || (tiles == 1 && max_rows_per_seq == 1 && n_rows == n_seqs),
@@ -750,20 +750,22 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
 #define BH_ATT_ONE(NS, STREAM, FUSED, ...)                                                                      \
   attention_mfma_kernel<NS, STREAM, FUSED, __VA_ARGS__><<<grid, is_fused && !lean && NS <= 4 ? 320 : 256, 0, stream>>>(        \
       (const uint16_t*)q, (uint16_t*)out, (float*)part_o, (float*)part_ml, (const uint16_t*)k_pages,            \
-      (const uint16_t*)v_pages, page_table, table_stride, positions, seq_start, H, KVH, scale_log2, window,     \
+      (const uint16_t*)v_pages, page_table, table_stride, positions, seq_start, H, KVH, window,                 \
       n_splits, per, tile_groups, fused, out_blocked, finish, form)
+#define BH_ATT_FORM(NS, STREAM, FUSED, LEAN)                                  \
+  do {                                                                        \
+    if (formed == 2) BH_ATT_ONE(NS, STREAM, FUSED, LEAN, 2);                  \
+    else if (formed) BH_ATT_ONE(NS, STREAM, FUSED, LEAN, 1);                  \
+    else BH_ATT_ONE(NS, STREAM, FUSED, LEAN, 0);                              \
+  } while (0)
 #define BH_ATT(NS)                                                                          \
   do {                                                                                      \
-    if (pairs && formed && lean && NS <= 4) BH_ATT_ONE(NS, true, 2, (NS <= 4), true);       \
-    else if (pairs && formed) BH_ATT_ONE(NS, true, 2, false, true);                         \
-    else if (pairs && lean && NS <= 4) BH_ATT_ONE(NS, true, 2, (NS <= 4), false);           \
-    else if (pairs) BH_ATT_ONE(NS, true, 2, false, false);                                  \
-    else if (is_fused && lean && NS <= 4) BH_ATT_ONE(NS, true, 1, (NS <= 4), false);        \
-    else if (is_fused) BH_ATT_ONE(NS, true, 1, false, false);                               \
-    else if (tile_groups == 1 && formed) BH_ATT_ONE(NS, true, 0, false, true);              \
-    else if (tile_groups == 1) BH_ATT_ONE(NS, true, 0, false, false);                       \
-    else if (formed) BH_ATT_ONE(NS, false, 0, false, true);                                 \
-    else BH_ATT_ONE(NS, false, 0, false, false);                                            \
+    if (pairs && lean && NS <= 4) BH_ATT_FORM(NS, true, 2, (NS <= 4));                      \
+    else if (pairs) BH_ATT_FORM(NS, true, 2, false);                                        \
+    else if (is_fused && lean && NS <= 4) BH_ATT_ONE(NS, true, 1, (NS <= 4), 0);            \
+    else if (is_fused) BH_ATT_ONE(NS, true, 1, false, 0);                                   \
+    else if (tile_groups == 1) BH_ATT_FORM(NS, true, 0, false);                             \
+    else BH_ATT_FORM(NS, false, 0, false);                                                  \
   } while (0)
   switch (hd / 32) {
     case 1: BH_ATT(1); break;
@@ -776,6 +778,7 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
     default: BH_ATT(8); break;
   }
 #undef BH_ATT
+#undef BH_ATT_FORM
 #undef BH_ATT_ONE
   if (int status = bh_check_launch("attention_mfma")) return status;
   if (n_splits > 1) {

@@ -48,12 +48,12 @@ __device__ inline float largest_of_column(float x) {
   return larger(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
 }
 
-template <int NS, int CTW, bool FORMED>      // FORMED: scores are more than a scaled product, and made in full (scale_log2 is log2(e))
+template <int NS, int CTW, int FORMED>      // FORMED: scores are more than a scaled product, and made in full (bh_formed)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2 : 1))) void attention_prefill_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, const uint16_t* __restrict__ k_pages,
     const uint16_t* __restrict__ v_pages, const int32_t* __restrict__ page_table, int table_stride,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_start, int H, int KVH,
-    float scale_log2, int window, int tile_groups, int n_seqs, int out_blocked, HeadEnd finish, ScoreForm form) {
+    int window, int tile_groups, int n_seqs, int out_blocked, HeadEnd finish, ScoreForm form) {
   constexpr int HD = 32 * NS;
   constexpr int PIECES = BH_PAGE * HD / 8;        // 16-byte pieces of one head's keys (or values) in a page
   constexpr int STAGE = 2 * PIECES / 256;         // pieces of a page (keys, then values) one thread copies
@@ -101,7 +101,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
   const bool wave_active = wave_tile0 * 16 < n_cols;
   int pos[CTW], lo[CTW];
   float col_scale[CTW], slope[CTW];      // FORMED: what a column makes of its products
-  const float cap_rate = FORMED && form.cap > 0.f ? 2.0f * BH_LOG2E / form.cap : 0.f;
+  float scale_log2[CTW];                 // of a column's scores (FORMED) or products into powers of two
+  const float cap_rate = FORMED == 2 ? 2.0f * BH_LOG2E / form.cap : 0.f;
   bf16x8_t q_vec[CTW][NS];
   int pos_max = 0, pos_min = 0x7fffffff, lo_min = 0x7fffffff, lo_max = 0;
 #pragma unroll
@@ -111,6 +112,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
     const int row = row0 + c / G, head = kvh * G + c % G;
     pos[ct] = positions[row];
     lo[ct] = bh_first_visible(pos[ct], window);
+    scale_log2[ct] = FORMED ? BH_LOG2E : query_scale(form, pos[ct]) * BH_LOG2E;
     if constexpr (FORMED) {
       col_scale[ct] = query_scale(form, pos[ct]);
       slope[ct] = form.slopes ? form.slopes[head] : 0.f;
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float off = fmaf(slope[ct], (float)(32 * (t / 2) + 4 * (t % 2) + r), nearest);
-          st[t][r] = cap_rate > 0.f ? capped_score(st[t][r] * col_scale[ct], form.cap, cap_rate) + off : fmaf(st[t][r], col_scale[ct], off);
+          st[t][r] = FORMED == 2 ? capped_score(st[t][r] * col_scale[ct], form.cap, cap_rate) + off : fmaf(st[t][r], col_scale[ct], off);
         }
     }
     if constexpr (decltype(masked)::value) {   // key k0 + d of the page is seen if lo <= k0 + d <= pos: two numbers per column, then constants
@@ -214,21 +216,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
     // The exponentials' reference moves only when the maximum has grown by more than SLACK powers of two (or
     // from nothing): until then probabilities may reach 2^SLACK, which float32 sums and bfloat16 operands
     // hold as well as numbers up to one, and what was summed so far needs no factor.
-    const bool stays = (new_max - run_max[ct]) * scale_log2 <= SLACK;   // false from -inf, and while nothing was seen
+    const bool stays = (new_max - run_max[ct]) * scale_log2[ct] <= SLACK;   // false from -inf, and while nothing was seen
     const float reference = stays ? run_max[ct] : new_max;
-    const float shift = (reference == -INFINITY) ? 0.f : -reference * scale_log2;
+    const float shift = (reference == -INFINITY) ? 0.f : -reference * scale_log2[ct];
     // exactly 1 while the reference stands still, 0 when nothing was seen before
     const float alpha =
-        (run_max[ct] == reference) ? 1.0f : __builtin_amdgcn_exp2f((run_max[ct] - reference) * scale_log2);
+        (run_max[ct] == reference) ? 1.0f : __builtin_amdgcn_exp2f((run_max[ct] - reference) * scale_log2[ct]);
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const int t = 2 * u + half;
-        const float e0 = __builtin_amdgcn_exp2f(fmaf(st[t][0], scale_log2, shift));
-        const float e1 = __builtin_amdgcn_exp2f(fmaf(st[t][1], scale_log2, shift));
-        const float e2 = __builtin_amdgcn_exp2f(fmaf(st[t][2], scale_log2, shift));
-        const float e3 = __builtin_amdgcn_exp2f(fmaf(st[t][3], scale_log2, shift));
+        const float e0 = __builtin_amdgcn_exp2f(fmaf(st[t][0], scale_log2[ct], shift));
+        const float e1 = __builtin_amdgcn_exp2f(fmaf(st[t][1], scale_log2[ct], shift));
+        const float e2 = __builtin_amdgcn_exp2f(fmaf(st[t][2], scale_log2[ct], shift));
+        const float e3 = __builtin_amdgcn_exp2f(fmaf(st[t][3], scale_log2[ct], shift));
         p_vec[u][2 * half] = pack_bf16(e0, e1);
         p_vec[u][2 * half + 1] = pack_bf16(e2, e3);
       }
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
     if (cc >= n_cols) continue;
     // a sink: one more term exp(sinks[head]) in the softmax's sum, taken against the exponentials' reference
     const int out_row = row0 + cc / G, out_head = kvh * G + cc % G, out_column = out_head * HD + 4 * g;
-    const float sunk = finish.sinks ? __builtin_amdgcn_exp2f((finish.sinks[out_head] * 1.4426950408889634f) - run_max[ct] * scale_log2) : 0.f;
+    const float sunk = finish.sinks ? __builtin_amdgcn_exp2f((finish.sinks[out_head] * 1.4426950408889634f) - run_max[ct] * scale_log2[ct]) : 0.f;
     const float inv = head_gate<bf16_t>(finish, out_row, out_head) / (run_sum[ct][0] + sunk);
 #pragma unroll
     for (int dt = 0; dt < 2 * NS; ++dt) {
@@ -358,17 +360,17 @@ void bh_attention_prefill_launch(const void* q, void* out, const void* k_pages, 
                                  const int32_t* page_table, int table_stride, const int32_t* positions,
                                  const int32_t* seq_start, int n_seqs, int tiles, int H, int KVH, int hd,
                                  const ScoreForm& form, int window, int out_blocked, const HeadEnd& finish, hipStream_t stream) {
-  const bool formed = !form.plain();
-  const float scale_log2 = formed ? BH_LOG2E : form.scale * BH_LOG2E;
+  const int formed = bh_formed(form);
 #define BH_PREFILL_ONE(NS, CTW, FORMED)                                                                      \
   attention_prefill_kernel<NS, CTW, FORMED><<<dim3(tile_groups * KVH * n_seqs), dim3(256), 0, stream>>>(     \
         (const uint16_t*)q, (uint16_t*)out, (const uint16_t*)k_pages, (const uint16_t*)v_pages, page_table,  \
-        table_stride, positions, seq_start, H, KVH, scale_log2, window, tile_groups, n_seqs, out_blocked, finish, form)
+        table_stride, positions, seq_start, H, KVH, window, tile_groups, n_seqs, out_blocked, finish, form)
 #define BH_PREFILL(NS, CTW)                                                                                  \
   do {                                                                                                       \
     const int tile_groups = (tiles + 4 * CTW - 1) / (4 * CTW);                                               \
-    if (formed) BH_PREFILL_ONE(NS, CTW, true);                                                               \
-    else BH_PREFILL_ONE(NS, CTW, false);                                                                     \
+    if (formed == 2) BH_PREFILL_ONE(NS, CTW, 2);                                                             \
+    else if (formed) BH_PREFILL_ONE(NS, CTW, 1);                                                             \
+    else BH_PREFILL_ONE(NS, CTW, 0);                                                                         \
   } while (0)
   // Two column tiles per wave while the accumulators leave room for two workgroups per compute unit; one
   // where that gives fewer than two workgroups per compute unit (a page costs a workgroup nearly the same

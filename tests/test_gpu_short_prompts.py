@@ -44,3 +44,30 @@ def test_attention_of_short_prompts(K, n_heads, kv_heads, head_dim, news, pasts,
             rows = slice(starts[s], starts[s + 1])
             want = attention_reference_rows(q[rows], keys[s], values[s], positions[rows], n_heads, kv_heads, head_dim, scale, window)
             assert rel(out[rows], want) < 8e-3, (s, window)      # probabilities and results of 8 bits
+
+
+@pytest.mark.parametrize("cap,sloped,coef,every", [(0.0, False, 0.3, 7), (0.0, False, -0.6, 5), (0.0, True, 0.0, 0), (1.5, False, 0.0, 0), (1.5, True, 0.3, 7)])
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim,new", [(4, 2, 128, 200), (8, 1, 64, 5), (2, 2, 32, 700)])
+def test_forms_of_scores(K, n_heads, kv_heads, head_dim, new, cap, sloped, coef, every):
+    """A query's factor stays out of the scores where it cannot be negative, and is in them where it is for late positions; slopes; a cap."""
+    dtype, scale, past = torch.bfloat16, 1 / math.sqrt(head_dim), 30
+    kp, vp, table, keys, values = make_cache(1, [past + new], kv_heads, head_dim, dtype, seed=new)
+    q = torch.randn(new, n_heads * head_dim, generator=torch.Generator().manual_seed(new)).to(dtype)
+    positions = torch.arange(past, past + new, dtype=torch.int32)
+    layout = Layout(False, dev(torch.tensor([0, new], dtype=torch.int32)), 1, new, past + new - 1)
+    out = torch.full((new, n_heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    kp, vp = stored(K, kp, vp)
+    slopes = torch.linspace(0.0, 0.25, n_heads) if sloped else None
+    K.attention(dev(q), out, kp, vp, dev(table), dev(torch.zeros(new, dtype=torch.int32)), dev(positions), n_heads, kv_heads, head_dim, scale, 0,
+                layout=layout, softcap=cap, slopes=None if slopes is None else dev(slopes), q_temp=(coef, every) if every else None)
+    factor = 1 + coef * torch.log(((positions + 1) // every).double() + 1) if every else torch.ones(new).double()
+    scores = torch.einsum("nhd,khd->nhk", q.double().view(new, n_heads, head_dim) * factor[:, None, None],
+                          keys[0].double().repeat_interleave(n_heads // kv_heads, 1)) * scale
+    if cap:
+        scores = cap * torch.tanh(scores / cap)
+    gap = positions[:, None] - torch.arange(past + new)
+    if sloped:
+        scores = scores - slopes.double()[:, None] * gap[:, None, :]
+    p = scores.masked_fill((gap < 0)[:, None, :], float("-inf")).softmax(-1)
+    want = torch.einsum("nhk,khd->nhd", p, values[0].double().repeat_interleave(n_heads // kv_heads, 1)).reshape(new, -1)
+    assert rel(out, want) < 8e-3                             # probabilities and results of 8 bits
