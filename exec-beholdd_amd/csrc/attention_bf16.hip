@@ -225,7 +225,8 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // LEAN (with FUSED) = the queries are normed and rotated before the first page is asked for, and the new key's
 // numbers are asked for after the last page: nothing of that overlaps with the pages any more, but what it needs
 // in registers is gone while the pages stream, so that two workgroups fit a compute unit.  For launches of more
-// workgroups than compute units, where the second workgroup is worth more than the overlap.
+// workgroups than compute units, where the second workgroup is worth more than the overlap; and for heads of more than 128, which
+// went to scratch memory with it (16 sequences of 1,000 to 2,000 keys, 16 heads on 8: of 256 122 -> 42 us, of 192 44 -> 34).
 // FORMED = scores are more than a scaled product (struct ScoreForm): they are made in full, and exponentials taken of them as they
 // are (scale_log2 is then log2(e)).  Otherwise a column's factor is in scale_log2 (ScoreForm::scaled_only).
 // A workgroup of a FUSED step that is not LEAN has a fifth wave (heads of up to 128, whose pages leave two waves a SIMD their registers):
@@ -234,7 +235,7 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // 4 sequences of 1,000 keys, 16 heads on 4 12.5 us, 11.0 now, of which the faster combining is 1.)
 __host__ __device__ constexpr bool fifth_wave(int ns, int fused, bool lean) { return fused && !lean && ns <= 4; }
 template <int NS, bool STREAM, int FUSED, bool LEAN = false, int FORMED = 0>
-__global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 2 : 1)) void attention_mfma_kernel(
+__global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN && NS <= 4 ? 2 : 1)) void attention_mfma_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
     const int32_t* __restrict__ page_table, int table_stride, const int32_t* __restrict__ positions,
@@ -275,13 +276,11 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
   const float col_scale = FORMED ? query_scale(form, pos_row) : 0.f, cap_rate = FORMED == 2 ? 2.0f * BH_LOG2E / form.cap : 0.f;
   const float slope = FORMED && form.slopes ? form.slopes[head] : 0.f;
   bf16x8_t q_vec[NS];
-  // FUSED: the raw rows and what norms and rotates them are asked for here and used once the first page's
-  // loads are under way (q) and after the pages (the new key and value).
+  // FUSED: the raw rows and what norms and rotates them.
   u32x4_t q_raw[NS], k_raw[NS];
   uint16_t new_value[2 * NS];   // dim 16 dt + j of the new value, as the cache takes it
   u32x2_t value_raw[2 * NS];    // dims 16 dt + 4 g .. + 3 of it, as the lane's sums do
   std::conditional_t<FUSED == 2, PairPrep<NS>, HeadPrep<NS>> q_prep, k_prep;
-  bool q_ready = !FUSED;
   const bool new_key_here = FUSED && fused.write_kv && split == n_splits - 1, takes_new_key = new_key_here && wave == (WAVES == 5 ? 4 : 0);
   auto ask_new_key = [&]() {   // one row per sequence: every lane's row is this row
     const uint16_t* qkv_row = fused.qkv + (size_t)row * fused.row_stride;
@@ -329,7 +328,6 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
     pack_head<NS>(packed, x);
 #pragma unroll
     for (int s = 0; s < NS; ++s) q_vec[s] = as_bf16x8(packed[s]);
-    q_ready = true;
   };
   if (FUSED && LEAN) finish_q();
   const int pos_max = wave_max_int(pos), pos_min = wave_min_int(pos);
@@ -519,14 +517,12 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN ? 
     }
     for (bool asked = WAVES == 5; p < end; p += 4, asked = false) {
       if (!asked) ask_page(p);
-      if (FUSED && WAVES == 4 && !q_ready) finish_q();   // under the page's loads
       attend(k_vec, v_vec, p, pos, lo, pos_max, pos_min, lo_max);
     }
   }
 
   if (takes_new_key) {
     if (WAVES == 4) ask_new_key();
-    if (WAVES == 4 && !q_ready) finish_q();
     take_new_key();
   }
 
@@ -760,10 +756,10 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   } while (0)
 #define BH_ATT(NS)                                                                          \
   do {                                                                                      \
-    if (pairs && lean && NS <= 4) BH_ATT_FORM(NS, true, 2, (NS <= 4));                      \
-    else if (pairs) BH_ATT_FORM(NS, true, 2, false);                                        \
-    else if (is_fused && lean && NS <= 4) BH_ATT_ONE(NS, true, 1, (NS <= 4), 0);            \
-    else if (is_fused) BH_ATT_ONE(NS, true, 1, false, 0);                                   \
+    if (pairs && lean) BH_ATT_FORM(NS, true, 2, true);                                      \
+    else if (pairs) BH_ATT_FORM(NS, true, 2, (NS > 4));                                     \
+    else if (is_fused && lean) BH_ATT_ONE(NS, true, 1, true, 0);                            \
+    else if (is_fused) BH_ATT_ONE(NS, true, 1, (NS > 4), 0);                                \
     else if (tile_groups == 1) BH_ATT_FORM(NS, true, 0, false);                             \
     else BH_ATT_FORM(NS, false, 0, false);                                                  \
   } while (0)
