@@ -120,10 +120,11 @@ struct ScoreForm {
   const float* slopes;   // [heads] or null
   float temp_coef;
   int temp_every;        // 0: none
-  // Whether a score is its product times a factor of the query that is not negative: then the largest product has the largest score, and
-  // the matrix-core kernels take the factor into the exponential instead of making the scores (2,048 rows, 32 heads of 128 on 8, which
-  // count the more the later they stand: 76 -> 53 us).  A factor that falls with the position may turn negative.
-  BH_BOTH bool scaled_only() const { return cap == 0.f && slopes == nullptr && (temp_every == 0 || (temp_coef >= 0.f && scale >= 0.f)); }
+  // Whether a score is its product times a positive factor of the query: then the largest product has the largest score, and the
+  // matrix-core kernels take the factor into the exponential instead of making the scores (2,048 rows, 32 heads of 128 on 8, which
+  // count the more the later they stand: 76 -> 53 us).  A factor that falls with the position may turn negative, and one of zero makes
+  // NaN of it: keys that are not seen stand at minus infinity, and nothing was summed before the first.
+  BH_BOTH bool scaled_only() const { return cap == 0.f && slopes == nullptr && scale > 0.f && (temp_every == 0 || temp_coef >= 0.f); }
 };
 // What the matrix-core kernels are compiled for: 0 scaled products only, 1 a factor and a distance's share, 2 a cap as well (asked of a number
 // at each score, both ways were made: 2,048 rows, 32 heads of 128 on 8 with slopes 79 -> 60 us, with a cap 93 -> 70).

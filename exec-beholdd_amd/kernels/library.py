@@ -1003,7 +1003,7 @@ class HipKernels(KernelSizes):
         if (qkv.dtype != torch.bfloat16 or k_pages.dtype != torch.bfloat16 or layout is None
                 or int(layout.max_rows_per_seq) != 1 or int(layout.n_seqs) != n_rows
                 or head_dim % 32 or head_dim > 256 or n_heads % n_kv_heads or n_heads // n_kv_heads > 16
-                or (cos is not None and (rot != head_dim or head_dim % 64))
+                or (cos is not None and (rot != head_dim or head_dim % 64)) or not scale > 0.0
                 or self.kv_order(k_pages.dtype, head_dim) != 1):
             return False
         if qkv.shape != (n_rows, (n_heads + 2 * n_kv_heads) * head_dim) or tuple(out.shape) != (n_rows, n_heads * head_dim) \

@@ -71,3 +71,37 @@ def test_forms_of_scores(K, n_heads, kv_heads, head_dim, new, cap, sloped, coef,
     p = scores.masked_fill((gap < 0)[:, None, :], float("-inf")).softmax(-1)
     want = torch.einsum("nhk,khd->nhd", p, values[0].double().repeat_interleave(n_heads // kv_heads, 1)).reshape(new, -1)
     assert rel(out, want) < 8e-3                             # probabilities and results of 8 bits
+
+
+@pytest.mark.parametrize("scale,coef,every", [(0.0, 0.3, 7), (0.0, 0.0, 0), (-0.2, 0.3, 7), (-0.2, 0.0, 0)])
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim,new,past", [(4, 2, 128, 200, 30), (8, 1, 64, 5, 30), (2, 2, 192, 1, 700)])
+def test_scores_whose_factor_is_not_positive(K, n_heads, kv_heads, head_dim, new, past, scale, coef, every):
+    """Nothing: the average of what is seen.  Negative: the smallest product has the largest score.  On the kernel of prompts, on the one of
+    few rows, and with keys in splits; then the last row once more as a decode step from the projection rows."""
+    dtype, length = torch.bfloat16, past + new
+    kp, vp, table, keys, values = make_cache(1, [length], kv_heads, head_dim, dtype, seed=new)
+    g = torch.Generator().manual_seed(new)
+    q = torch.randn(new, n_heads * head_dim, generator=g).to(dtype)
+    positions = torch.arange(past, length, dtype=torch.int32)
+    kp, vp = stored(K, kp, vp)
+    q_temp = (coef, every) if every else None
+    factor = 1 + coef * torch.log(((positions + 1) // every).double() + 1) if every else torch.ones(new).double()
+    scores = torch.einsum("nhd,khd->nhk", q.double().view(new, n_heads, head_dim) * factor[:, None, None],
+                          keys[0].double().repeat_interleave(n_heads // kv_heads, 1)) * scale
+    seen = positions[:, None] >= torch.arange(length)
+    want = torch.einsum("nhk,khd->nhd", scores.masked_fill(~seen[:, None, :], float("-inf")).softmax(-1),
+                        values[0].double().repeat_interleave(n_heads // kv_heads, 1)).reshape(new, -1)
+    out = torch.full((new, n_heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    layout = Layout(new == 1, dev(torch.tensor([0, new], dtype=torch.int32)), 1, new, length - 1)
+    K.attention(dev(q), out, kp, vp, dev(table), dev(torch.zeros(new, dtype=torch.int32)), dev(positions), n_heads, kv_heads, head_dim, scale, 0,
+                layout=layout, q_temp=q_temp)
+    assert rel(out, want) < 8e-3                             # probabilities and results of 8 bits
+    row = torch.cat([q[-1:], keys[0][-1:].reshape(1, -1), values[0][-1:].reshape(1, -1)], 1)
+    one = torch.full((1, n_heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    layout = Layout(True, dev(torch.tensor([0, 1], dtype=torch.int32)), 1, 1, length - 1)
+    assert K.attention_decode_pairs(dev(row), 0, one, None, None, 0.0, None, None, dev(positions[-1:]), kp, vp, dev(table), n_heads, kv_heads, head_dim,
+                                    scale, True, layout, q_temp=q_temp)
+    assert rel(one, want[-1:]) < 8e-3
+    if not every:      # the launch from whole fused rows has scaled products only, and leaves such steps to the two
+        assert not K.attention_decode_fused(dev(row), one, None, None, 0.0, None, None, dev(positions[-1:]), kp, vp, dev(table), n_heads, kv_heads,
+                                            head_dim, scale, 0, True, layout)
