@@ -498,7 +498,7 @@ extern "C" int bh_gemm_f32_normed(const float* a, const float* norm_weight, floa
   BH_REQUIRE(bh_gemm_f32_takes_norm(M, N, K) && bh_gemm_f32_takes(a, w, c, K) && ((uintptr_t)norm_weight % 16) == 0,
              "gemm: a float32 product that norms its rows takes up to %d of them, K a multiple of 4 and 16-byte aligned operands (M=%d K=%d)",
              BH_F32_FEW_ROWS, M, K);
-  BH_REQUIRE(norm_weight != nullptr && eps > 0.f, "gemm: a norm has a weight and an epsilon");
+  BH_REQUIRE(norm_weight != nullptr && eps >= 0.f, "gemm: a norm has a weight, and an epsilon that is not negative");
   BH_REQUIRE(gate == 0 || gate == BH_GATE_SILU || gate == BH_GATE_GELU_TANH, "gemm: unknown activation %d", gate);
   const GateForm form = bh_gate_form(gate);
   const RowNorm norm = {norm_weight, eps};

@@ -104,3 +104,23 @@ def test_float32_products_norm_a_residual(K, m, n, k):
     base = total.double()
     K.gemm(prepared, half, total, accumulate=True)
     assert bool(((total.double() - base - normed @ half.double().t()).abs() <= bound[:, :n] + 4 * 2.0 ** -24 * base.abs()).all())
+
+
+def test_float32_products_norm_without_an_epsilon(K):
+    """A norm's epsilon may be zero, as `rmsnorm` takes it, and one below the smallest float32 is."""
+    from beholdd.parts.base import NormRequest
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    a, w_in, w, weight = (torch.randn(*shape, generator=g, device="cuda:0") for shape in ((4, 64), (256, 64), (24, 256), (256,)))
+    for eps in (0.0, 1e-60):
+        residual = torch.randn(4, 256, generator=g, device="cuda:0")
+        prepared = K.gemm(a, w_in, residual, accumulate=True, then_norm=NormRequest(weight, eps))
+        assert prepared.ss is None
+        source = residual.double()
+        normed = source / source.square().mean(-1, keepdim=True).sqrt() * weight.double()
+        out, gated = torch.empty(4, 24, device="cuda:0"), torch.empty(4, 12, device="cuda:0")
+        K.gemm(prepared, w, out)
+        K.gemm_swiglu(prepared, w, gated)
+        both = normed @ w.double().t()
+        bound = (256 / 16 + 72) * 2.0 ** -24 * float((normed.abs() @ w.double().abs().t()).max())
+        assert float((out.double() - both).abs().max()) < bound
+        assert float((gated.double() - torch.nn.functional.silu(both[:, :12]) * both[:, 12:]).abs().max()) < 3 * bound * float(both.abs().max())
