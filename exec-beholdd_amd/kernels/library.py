@@ -628,8 +628,11 @@ class HipKernels(KernelSizes):
         return prepared
 
     def _normed_f32(self, a, w, out, n, gate) -> bool:
-        """The product of float32 `NormedRows` with float32 weights, whose norm it makes itself; False where it does not go."""
+        """The product of float32 `NormedRows` with float32 weights, whose norm it makes itself; False where it does not go (a product
+        that overwrites the rows it norms among them: its workgroups read all of them)."""
         m, k = a.shape
+        if out.data_ptr() < a.source.data_ptr() + 4 * m * k and a.source.data_ptr() < out.data_ptr() + 4 * m * n:
+            return False
         if (not isinstance(w, torch.Tensor) or not w.dtype == out.dtype == a.source.dtype == a.weight.dtype == torch.float32
                 or not self.lib.bh_gemm_f32_takes_norm(m, n, k) or (a.source.data_ptr() | w.data_ptr() | a.weight.data_ptr()) % 16):
             return False

@@ -124,3 +124,19 @@ def test_float32_products_norm_without_an_epsilon(K):
         bound = (256 / 16 + 72) * 2.0 ** -24 * float((normed.abs() @ w.double().abs().t()).max())
         assert float((out.double() - both).abs().max()) < bound
         assert float((gated.double() - torch.nn.functional.silu(both[:, :12]) * both[:, 12:]).abs().max()) < 3 * bound * float(both.abs().max())
+
+
+@pytest.mark.parametrize("n,first", [(512, 0), (256, 2048), (256, 0)])
+def test_float32_products_may_overwrite_what_they_norm(K, n, first):
+    """The output on the residual itself, on its last elements and on its first: the norm is then a launch of its own."""
+    from beholdd.parts.base import NormRequest
+    g = torch.Generator(device="cuda:0").manual_seed(n + first)
+    m, k = 8, 512
+    a, w_in, w, weight = (torch.randn(*shape, generator=g, device="cuda:0") for shape in ((m, 64), (k, 64), (n, k), (k,)))
+    residual = torch.randn(m, k, generator=g, device="cuda:0")
+    prepared = K.gemm(a, w_in, residual, accumulate=True, then_norm=NormRequest(weight, 1e-5))
+    source = residual.double()
+    want = source / (source.square().mean(-1, keepdim=True) + 1e-5).sqrt() * weight.double() @ w.double().t()
+    out = residual.view(-1)[first:first + m * n].view(m, n)
+    K.gemm(prepared, w, out)
+    assert float((out.double() - want).abs().max()) < (k / 16 + 72) * 2.0 ** -24 * float(want.abs().max()) * 8
