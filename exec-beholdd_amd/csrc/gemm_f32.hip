@@ -398,10 +398,12 @@ static void few_waves(const float* a, const float* w, float* c, int M, int N, in
       gemm_f32_few_kernel<R, C, 1, GATED, NORM><<<blocks, 64, 0, stream>>>(a, w, c, M, N, K, accumulate, form, norm);
       return;
     }
-  } else if (K >= 2048 && blocks < 2 * bh_compute_units()) {
+  } else if constexpr (!NORM || C < 8) {      // (norms of more than 16 rows: short K only, bh_gemm_f32_takes_norm)
     // Eight waves share a long K where four would leave a compute unit with fewer than two workgroups.
-    gemm_f32_few_kernel<R, C, 8, GATED, NORM><<<blocks, 512, 0, stream>>>(a, w, c, M, N, K, accumulate, form, norm);
-    return;
+    if (K >= 2048 && blocks < 2 * bh_compute_units()) {
+      gemm_f32_few_kernel<R, C, 8, GATED, NORM><<<blocks, 512, 0, stream>>>(a, w, c, M, N, K, accumulate, form, norm);
+      return;
+    }
   }
   gemm_f32_few_kernel<R, C, 4, GATED, NORM><<<blocks, 256, 0, stream>>>(a, w, c, M, N, K, accumulate, form, norm);
 }
@@ -491,22 +493,39 @@ extern "C" int bh_gemm_f32_gated(const float* a, const float* w, float* out, int
 }
 
 // The same products of RMSNorm(a; norm_weight, eps) in place of a, which is a residual as it stands, by one launch: c[M, N] = norm(a) W^T, or
-// gated (`gate`, a BhGate; N outputs).  For the float32 products of up to BH_F32_FEW_ROWS rows; bh_gemm_f32_takes_norm: whether these sizes go.
-extern "C" int bh_gemm_f32_takes_norm(int M, int N, int K) { return bh_gemm_f32_takes_gated(M, N, K); }
+// gated (`gate`, a BhGate; N outputs).
+// bh_gemm_f32_takes_norm: whether these sizes go.  It saves a launch of 2.5 us and costs every workgroup the squares of the rows and a
+// register or two for each number of them.  us, norm and product / one launch, chains of products of cold weights:
+//   up to 4 rows it wins at all sizes (1 x 7,268 x 748 9.4 / 7.2, 4 x 9,412 x 3,072 32.1 / 28.6, gated 4 x 1,848 x 6,044 26.3 / 23.7);
+//   up to 16 rows where a wave takes one or two groups of four outputs or a gated pair of them (8 x 2,608 x 668 7.7 / 5.6, 16 x 2,864 x 924
+//   11.2 / 9.7, 10 x 904 x 6,144 16.8 / 14.8, gated 8 x 2,720 x 1,564 15.2 / 13.2, 12 x 1,704 x 4,560 27.9 / 26.0); with more of them
+//   its registers leave room for a wave a SIMD less (gated 6 x 8,672 x 3,756 59.7 / 87.9, 12 x 11,000 x 260 11.1 / 15.0);
+//   up to 32 rows, whose squares are as much work as the products of a group, only where a wave has few of them and one workgroup is
+//   all that a compute unit has (24 x 448 x 140 6.4 / 5.7, gated 24 x 372 x 324 9.5 / 8.6; 28 x 1,488 x 2,600 22.2 / 26.4, 20 x 2,732 x 404
+//   9.6 / 14.0).
+// What does not go has its norm in front.
+extern "C" int bh_gemm_f32_takes_norm(int M, int N, int K, int gated) {
+  if (!bh_gemm_f32_takes_gated(M, N, K)) return 0;
+  if (M <= 4) return 1;
+  const int units = bh_compute_units(), group = (N + 3) / 4;      // groups of four outputs: of one a workgroup
+  if (M <= 16) return N < (gated ? 16 : 32) * units ? 1 : 0;
+  return group <= units && K <= 768 ? 1 : 0;
+}
 extern "C" int bh_gemm_f32_normed(const float* a, const float* norm_weight, float eps, const float* w, float* c, int M, int N, int K, int gate,
                                   hipStream_t stream) {
-  BH_REQUIRE(bh_gemm_f32_takes_norm(M, N, K) && bh_gemm_f32_takes(a, w, c, K) && ((uintptr_t)norm_weight % 16) == 0,
-             "gemm: a float32 product that norms its rows takes up to %d of them, K a multiple of 4 and 16-byte aligned operands (M=%d K=%d)",
-             BH_F32_FEW_ROWS, M, K);
+  BH_REQUIRE(bh_gemm_f32_takes_norm(M, N, K, gate != 0) && bh_gemm_f32_takes(a, w, c, K) && ((uintptr_t)norm_weight % 16) == 0,
+             "gemm: a float32 product of M=%d N=%d K=%d that norms its rows (bh_gemm_f32_takes_norm), from 16-byte aligned operands", M, N, K);
   BH_REQUIRE(norm_weight != nullptr && eps >= 0.f, "gemm: a norm has a weight, and an epsilon that is not negative");
   BH_REQUIRE(gate == 0 || gate == BH_GATE_SILU || gate == BH_GATE_GELU_TANH, "gemm: unknown activation %d", gate);
   const GateForm form = bh_gate_form(gate);
   const RowNorm norm = {norm_weight, eps};
   const int units = bh_compute_units();
-  if (gate && N >= 16 * units) few_rows<4, true, true>(a, w, c, M, N, K, 0, form, stream, norm);
+  if (gate && N >= 16 * units) few_waves<4, 1, true, true>(a, w, c, M, N, K, 0, form, norm, stream);
   else if (gate) few_rows<2, true, true>(a, w, c, M, N, K, 0, form, stream, norm);
-  else if (N >= 32 * units) few_rows<4, false, true>(a, w, c, M, N, K, 0, form, stream, norm);
-  else if (N >= 16 * units) few_rows<2, false, true>(a, w, c, M, N, K, 0, form, stream, norm);
-  else few_rows<1, false, true>(a, w, c, M, N, K, 0, form, stream, norm);
+  else if (N >= 32 * units) few_waves<4, 1, false, true>(a, w, c, M, N, K, 0, form, norm, stream);
+  else if (N < 16 * units) few_rows<1, false, true>(a, w, c, M, N, K, 0, form, stream, norm);
+  else if (M <= 4) few_waves<2, 1, false, true>(a, w, c, M, N, K, 0, form, norm, stream);
+  else if (M <= 8) few_waves<2, 2, false, true>(a, w, c, M, N, K, 0, form, norm, stream);
+  else few_waves<2, 4, false, true>(a, w, c, M, N, K, 0, form, norm, stream);
   return bh_check_launch("gemm_f32_few");
 }

@@ -151,7 +151,7 @@ class KernelSizes:
             "bh_attention_f32_tiles": [i, i, i, i, i, i, p, p],
             "bh_gemm_f32_takes_gated": [i, i, i],
             "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
-            "bh_gemm_f32_takes_norm": [i, i, i],
+            "bh_gemm_f32_takes_norm": [i, i, i, i],
             "bh_gemm_f32_normed": [p, p, f, p, p, i, i, i, i, p],
             "bh_swiglu": [p, p, i, i, i, i, p],
             "bh_sample": [p, p, p, p, p, p, p, p, i, i, p],
@@ -620,7 +620,7 @@ class HipKernels(KernelSizes):
         if isinstance(a, BlockedRows):
             a = self.from_blocked(a)
         if (then_norm is not None and a.dtype == out.dtype == then_norm.weight.dtype == torch.float32
-                and then_norm.weight.shape == (n,) and self.lib.bh_gemm_f32_takes_norm(m, 4, n)):
+                and then_norm.weight.shape == (n,) and self.lib.bh_gemm_f32_takes_gated(m, 4, n)):
             prepared = NormedRows(out, None, then_norm.eps, out, then_norm.weight)      # its reader norms the residual itself
         self._check(self.lib.bh_gemm_generic(
             self._ptr(a, "gemm a"), _code(a, "gemm a"), self._ptr(w, "gemm w"), _code(w, "gemm w"),
@@ -634,7 +634,7 @@ class HipKernels(KernelSizes):
         if out.data_ptr() < a.source.data_ptr() + 4 * m * k and a.source.data_ptr() < out.data_ptr() + 4 * m * n:
             return False
         if (not isinstance(w, torch.Tensor) or not w.dtype == out.dtype == a.source.dtype == a.weight.dtype == torch.float32
-                or not self.lib.bh_gemm_f32_takes_norm(m, n, k) or (a.source.data_ptr() | w.data_ptr() | a.weight.data_ptr()) % 16):
+                or not self.lib.bh_gemm_f32_takes_norm(m, n, k, int(gate != 0)) or (a.source.data_ptr() | w.data_ptr() | a.weight.data_ptr()) % 16):
             return False
         self._check(self.lib.bh_gemm_f32_normed(self._ptr(a.source, "gemm a"), self._ptr(a.weight, "norm weight"), a.eps, self._ptr(w, "gemm w"),
                                                 self._ptr(out, "gemm out"), m, n, k, gate, self._stream()))

@@ -140,3 +140,13 @@ def test_float32_products_may_overwrite_what_they_norm(K, n, first):
     out = residual.view(-1)[first:first + m * n].view(m, n)
     K.gemm(prepared, w, out)
     assert float((out.double() - want).abs().max()) < (k / 16 + 72) * 2.0 ** -24 * float(want.abs().max()) * 8
+
+
+# rows and outputs on both sides of each line of the rule (bh_gemm_f32_takes_norm): gated products stop at half as many outputs as plain ones
+@pytest.mark.parametrize("m,n,k,plain,gated", [(4, 8200, 132, 1, 1), (1, 8192, 68, 1, 1), (8, 4095, 260, 1, 1), (5, 4096, 64, 1, 0), (16, 8191, 64, 1, 0),
+                                               (9, 8192, 64, 0, 0), (17, 1024, 768, 1, 1), (32, 1025, 64, 0, 0), (24, 8, 772, 0, 0)])
+def test_float32_products_that_norm_and_those_that_leave_it(K, m, n, k, plain, gated):
+    takes = K.lib.bh_gemm_f32_takes_norm
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:      # the lines go by the compute units
+        assert (takes(m, n, k, 0), takes(m, n, k, 1)) == (plain, gated)
+    test_float32_products_norm_a_residual(K, m, n, k)
