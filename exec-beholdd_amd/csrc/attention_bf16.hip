@@ -493,11 +493,11 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
       v_vec[dt][1] = load16_cache<STREAM>(vb + ((dt * 2 + 1) * 64 + lane) * 8);
     }
   };
-  // What the fifth wave hands over.  The barrier waits for LDS only: the first page stays on its way.
+  // What the fifth wave hands over.  The barrier waits for LDS only: the first page stays on its way.  (One asm that may touch memory: the
+  // builtins are said to touch none, so that nothing would hold the stores of sm_q above and its loads below on their sides of them.)
   auto meet = [&]() {
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));      // vmcnt and expcnt as they are, lgkmcnt 0
-    __builtin_amdgcn_s_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
   if (WAVES == 5 && wave == 4) {
