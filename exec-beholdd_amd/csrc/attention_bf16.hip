@@ -723,6 +723,7 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   BH_REQUIRE(hd % 32 == 0 && hd >= 32 && hd <= 256, "attention_bf16: head size %d is not a multiple of 32 up to 256", hd);
   BH_REQUIRE(max_position >= 0, "attention_bf16: positions must not be negative");
   BH_REQUIRE(n_splits >= 1 && (n_splits == 1 || (part_o && part_ml)), "attention_bf16: split keys need scratch memory");
+  BH_REQUIRE(n_splits <= COMBINE_SPLITS * COMBINE_SPLITS, "attention_bf16: keys in %d splits, at most %d are combined", n_splits, COMBINE_SPLITS * COMBINE_SPLITS);
   const int G = H / KVH;
   const int tiles = (max_rows_per_seq * G + 15) / 16;
   const int pages = max_position / BH_PAGE + 1;
@@ -778,7 +779,6 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
 #undef BH_ATT_ONE
   if (int status = bh_check_launch("attention_mfma")) return status;
   if (n_splits > 1) {
-    BH_REQUIRE(n_splits <= COMBINE_SPLITS * COMBINE_SPLITS, "attention_bf16: keys in %d splits, at most %d are combined", n_splits, COMBINE_SPLITS * COMBINE_SPLITS);
     const int dims = hd >= 128 ? 128 : 64, groups = (n_splits + COMBINE_SPLITS - 1) / COMBINE_SPLITS;
 #define BH_COMBINE(SPLITS)                                                                                                                  \
   attention_combine_kernel<SPLITS><<<n_rows * H, dims * groups, 0, stream>>>((const float*)part_o, (const float*)part_ml, (uint16_t*)out, \

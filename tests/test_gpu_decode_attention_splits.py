@@ -41,6 +41,26 @@ def test_decode_attention_in_splits(K, heads, kv_heads, head_dim, context, bucke
             assert rel(got[s:s + 1], want) < 8e-3, (s, length)      # probabilities and results of 8 bits
 
 
+def test_splits_that_are_not_combined_are_refused_before_anything_runs(K):
+    """65 splits of a decode step that writes its new key: an error, and cache and output as they were."""
+    from beholdd.kernels import KernelError
+    heads, kv_heads, head_dim, n_splits, length = 2, 1, 64, 65, 65 * 64
+    kp, vp, table, _, _ = make_cache(1, [length], kv_heads, head_dim, torch.bfloat16, seed=1)
+    k_pages, v_pages = stored(K, kp, vp)
+    before = k_pages.clone(), v_pages.clone()
+    rows = torch.ones(1, (heads + 2 * kv_heads) * head_dim, dtype=torch.bfloat16, device="cuda:0")
+    out = torch.full((1, heads * head_dim), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    part_o, part_ml = torch.zeros(heads * n_splits * head_dim, device="cuda:0"), torch.zeros(heads * n_splits * 2, device="cuda:0")
+    table, positions = dev(table), torch.tensor([length - 1], dtype=torch.int32, device="cuda:0")
+    starts = torch.tensor([0, 1], dtype=torch.int32, device="cuda:0")
+    with pytest.raises(KernelError, match="65 splits"):
+        K._check(K.lib.bh_attention_decode_fused(
+            rows.data_ptr(), out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), table.data_ptr(),
+            table.shape[1], positions.data_ptr(), starts.data_ptr(), 1, heads, kv_heads, head_dim, 0.125, 0, length - 1, n_splits, None, None, 0,
+            0.0, None, None, 0, 0, 1, 0, K._stream()))
+    assert torch.equal(k_pages, before[0]) and torch.equal(v_pages, before[1]) and bool((out == 7.0).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [4, 6, 1020, 1024, 1028, 4100, 5120])
 def test_embedding_rows(K, dtype, width):
