@@ -567,10 +567,14 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
       // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
       if (finish.sinks) sum += exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top);
       const float gate = head_gate<bf16_t>(finish, out_row, out_head);
+      const bool pairs = ((uintptr_t)out & 3) == 0;
 #pragma unroll
-      for (int d = 0; d < EACH; d += 2)   // (two neighbours from an even dimension on are neighbours in blocks too)
-        *reinterpret_cast<uint32_t*>(out + bh_rows_index(out_block_rows, out_row, out_head * HD + d0 + d, H * HD)) =
-            (uint32_t)f32_to_bf16_bits(value[d] * gate / sum) | ((uint32_t)f32_to_bf16_bits(value[d + 1] * gate / sum) << 16);
+      for (int d = 0; d < EACH; d += 2) {   // (two neighbours from an even dimension on are neighbours in blocks too)
+        uint16_t* to = out + bh_rows_index(out_block_rows, out_row, out_head * HD + d0 + d, H * HD);
+        const uint16_t one = f32_to_bf16_bits(value[d] * gate / sum), two = f32_to_bf16_bits(value[d + 1] * gate / sum);
+        if (pairs) *reinterpret_cast<uint32_t*>(to) = (uint32_t)one | ((uint32_t)two << 16);
+        else to[0] = one, to[1] = two;
+      }
     } else {
       float* to = part_o + (column * n_splits + split) * HD + d0;
 #pragma unroll
@@ -733,7 +737,7 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   const bool is_fused = fused.qkv != nullptr;
   BH_REQUIRE(!is_fused || (tiles == 1 && max_rows_per_seq == 1 && n_rows == n_seqs),
              "attention_bf16: the fused projection rows are taken in decode steps of at most 16 heads per kv head only");
-  if (!is_fused && n_splits == 1 && prefill_wins(n_seqs, max_rows_per_seq, H, KVH, max_position)) {
+  if (!is_fused && n_splits == 1 && (uintptr_t)out % 8 == 0 && prefill_wins(n_seqs, max_rows_per_seq, H, KVH, max_position)) {   // it writes 8 bytes at a time
     BH_REQUIRE(out_blocked == 0 || out_blocked == 16, "attention_bf16: a step of many columns writes rows or blocks of 16 rows, not of %d", out_blocked);
     bh_attention_prefill_launch(q, out, k_pages, v_pages, page_table, table_stride, positions, seq_start, n_seqs,
                                 tiles, H, KVH, hd, form, window, out_blocked == 16, finish, stream);

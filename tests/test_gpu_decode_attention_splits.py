@@ -61,6 +61,31 @@ def test_splits_that_are_not_combined_are_refused_before_anything_runs(K):
     assert torch.equal(k_pages, before[0]) and torch.equal(v_pages, before[1]) and bool((out == 7.0).all())
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,context,new", [(4, 2, 128, 300, 1), (3, 3, 96, 300, 1), (4, 2, 256, 40, 1), (4, 2, 128, 60, 5), (4, 2, 64, 90, 40),
+                                                                 (4, 2, 128, 0, 300)])
+def test_attention_into_rows_that_stand_on_two_bytes(K, heads, kv_heads, head_dim, context, new):
+    """Decode steps, short steps and prompts that would else go to the kernel whose stores are 8 bytes: what lies around is as it was."""
+    dtype, scale, length = torch.bfloat16, 1 / math.sqrt(head_dim), context + new
+    kp, vp, table, keys, values = make_cache(1, [length], kv_heads, head_dim, dtype, seed=length)
+    k_pages, v_pages = stored(K, kp, vp)
+    q = torch.randn(new, heads * head_dim, generator=torch.Generator().manual_seed(length)).to(dtype)
+    positions = torch.arange(context, length, dtype=torch.int32)
+    want = attention_reference_rows(q, keys[0], values[0], positions, heads, kv_heads, head_dim, scale, 0)
+    layout = Layout(new == 1, dev(torch.tensor([0, new], dtype=torch.int32)), 1, new, length - 1)
+    for shift in (1, 2, 3):
+        space = torch.full((q.numel() + 8,), 7.0, dtype=dtype, device="cuda:0")
+        out = space[shift:shift + q.numel()].view(new, heads * head_dim)
+        K.attention(dev(q), out, k_pages, v_pages, dev(table), dev(torch.zeros(new, dtype=torch.int32)), dev(positions), heads, kv_heads, head_dim,
+                    scale, 0, layout=layout)
+        assert rel(out, want) < 8e-3                             # probabilities and results of 8 bits
+        assert bool((space[:shift] == 7.0).all()) and bool((space[shift + q.numel():] == 7.0).all())
+    if new == 1:
+        row = torch.cat([q, keys[0][-1:].reshape(1, -1), values[0][-1:].reshape(1, -1)], 1)
+        assert K.attention_decode_fused(dev(row), out, None, None, 0.0, None, None, dev(positions), k_pages, v_pages, dev(table), heads, kv_heads,
+                                        head_dim, scale, 0, True, layout)
+        assert rel(out, want) < 8e-3
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [4, 6, 1020, 1024, 1028, 4100, 5120])
 def test_embedding_rows(K, dtype, width):
