@@ -493,12 +493,14 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_waves_kernel(const fl
 // The same in pieces of 16 bytes of z and out, LANES lanes a group, all loads of a group before its sums: single elements are waited for
 // a few bytes at a time (2,048 rows of 32 heads of 128 in bfloat16 35 us, 23.9 now; 8,192 rows 124 -> 76).  Many small groups take
 // few lanes each and few large ones many, so that few lanes have nothing to do (3 groups of 512 on 32 lanes 28.7 us, on 64 16.2).
+// Eight lanes go with groups of a piece each: as an array of one, which stays in registers (8,192 rows of 64 groups of 32 in float32 59.5
+// -> 31.2 us, of 64 in bfloat16, 128 a row, 146 -> 108; of as many as 512 elements need, it lay in scratch memory or took 165 registers).
 template <typename T, int LANES, bool SPREAD>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_pieces_kernel(const float* __restrict__ y, const T* __restrict__ z, int z_stride,
                                                                         int z_first, const float* __restrict__ w, float eps,
                                                                         T* __restrict__ out, int n_rows, int width, int groups, int out_block_rows,
                                                                         int gate_after) {
-  constexpr int VEC = 16 / sizeof(T), PIECES = 512 / (VEC * LANES);
+  constexpr int VEC = 16 / sizeof(T), PIECES = LANES == 8 ? 1 : 512 / (VEC * LANES);
   const int row = bh_row_of_block<SPREAD>(), per = width / groups, lane = threadIdx.x % LANES;
   if (SPREAD && row >= n_rows) return;
   // a wave's lanes stay together (their sums are exchanged): those without a group take the last one's numbers and write nothing
