@@ -296,8 +296,7 @@ static void launch_rows(const void* a, const void* w, void* c, int accumulate, i
   if (gated) BH_FEW(1, true, false, 2);
   else if (span == 16) BH_FEW(1, false, false, 2);
   else if (span == 8) BH_FEW(1, false, true, 4);
-  else if (MB == 1 && sizeof(TC) == 4) BH_FEW(2, false, true, 4);
-  else BH_FEW(2, false, true, 2);
+  else BH_FEW(2, false, true, MB == 1 && sizeof(TC) == 4 ? 4 : 2);
 #undef BH_FEW
 }
 
