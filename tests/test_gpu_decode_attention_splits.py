@@ -1,12 +1,12 @@
 """Decode attention from the projection rows with keys in one to 64 splits, whose partial results groups of eight are combined from, and
-with last splits of no page, one page and four beside the new key, against float64; and the embedding at widths of whole and cut pieces."""
+with last splits of no page, one page and four beside the new key, against float64."""
 
 import math
 
 import pytest
 import torch
 
-from test_gpu_kernels import K, Layout, attention_reference_rows, dev, make_cache, rel, stored      # noqa: F401  (K: the fixture)
+from test_gpu_kernels import K, Layout, as_rows, attention_reference_rows, dev, make_cache, rel, stored      # noqa: F401  (K: the fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +39,66 @@ def test_decode_attention_in_splits(K, heads, kv_heads, head_dim, context, bucke
             key[-1], value[-1] = row[heads:heads + kv_heads], row[heads + kv_heads:]
             want = attention_reference_rows(row[:heads].reshape(1, -1), key, value, positions[s:s + 1], heads, kv_heads, head_dim, scale, 0)
             assert rel(got[s:s + 1], want) < 8e-3, (s, length)      # probabilities and results of 8 bits
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(2, 1, 128), (5, 1, 64), (4, 2, 192)])
+@pytest.mark.parametrize("context,bucket", [(1, 1), (449, 8), (2049, 33), (17000, 272)])
+def test_decode_attention_in_splits_norms_and_turns(K, heads, kv_heads, head_dim, context, bucket):
+    """The same with heads that are normed and rotated on the way (by the fifth wave, or, of more than 128, by all four), the key that
+    the cache gets among them."""
+    dtype, scale, eps = torch.bfloat16, 1 / math.sqrt(head_dim), 1e-5
+    lengths = [context, max(context // 3, 1), 1]
+    n = len(lengths)
+    kp, vp, table, keys, values = make_cache(n, lengths, kv_heads, head_dim, dtype, seed=context)
+    wide = torch.zeros(n, bucket, dtype=torch.int32)
+    wide[:, :table.shape[1]] = table
+    g = torch.Generator().manual_seed(context)
+    qkv = (3 * torch.randn(n, (heads + 2 * kv_heads) * head_dim, generator=g)).to(dtype)
+    weights = [(1 + 0.2 * torch.randn(head_dim, generator=g)).to(dtype) for _ in range(2)]
+    angles = torch.arange(bucket * 64, dtype=torch.float64)[:, None] / 1e4 ** (torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim)
+    positions = torch.tensor([length - 1 for length in lengths], dtype=torch.int32)
+    layout = Layout(True, dev(torch.arange(n + 1, dtype=torch.int32)), n, 1, bucket * 64 - 1)
+    k_pages, v_pages = stored(K, kp, vp)
+    out = torch.full((n, heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    assert K.attention_decode_fused(dev(qkv), out, dev(weights[0]), dev(weights[1]), eps, dev(angles.cos().float()), dev(angles.sin().float()),
+                                    dev(positions), k_pages, v_pages, dev(wide), heads, kv_heads, head_dim, scale, 0, True, layout)
+    k_rows, v_rows = as_rows(K, k_pages, v_pages)
+    for s, length in enumerate(lengths):
+        row = qkv[s].double().reshape(heads + 2 * kv_heads, head_dim)
+        made = []
+        for x, weight in ((row[:heads], weights[0]), (row[heads:heads + kv_heads], weights[1])):
+            x = x / (x.square().mean(-1, keepdim=True) + eps).sqrt() * weight.double()
+            low, high, cos, sin = x[:, :head_dim // 2], x[:, head_dim // 2:], angles[length - 1].cos(), angles[length - 1].sin()
+            made.append(torch.cat([low * cos - high * sin, high * cos + low * sin], 1).to(dtype))
+        key, value = keys[s].clone(), values[s].clone()
+        key[-1], value[-1] = made[1], qkv[s].reshape(-1, head_dim)[heads + kv_heads:]
+        page, token = int(wide[s, (length - 1) // 64]), (length - 1) % 64
+        assert rel(k_rows[page, :, token], made[1]) < 8e-3 and torch.equal(v_rows[page, :, :, token].to(dtype), value[-1])
+        want = attention_reference_rows(made[0].reshape(1, -1), key, value, positions[s:s + 1], heads, kv_heads, head_dim, scale, 0)
+        assert rel(out[s:s + 1], want) < 8e-3, (s, length)      # probabilities and results of 8 bits
+
+
+# keys in splits; more workgroups than compute units; heads of more than 128.  The last factor is negative from position 189 on.
+@pytest.mark.parametrize("heads,kv_heads,head_dim,n,context", [(4, 2, 128, 2, 3000), (32, 8, 128, 40, 150), (4, 2, 192, 2, 900), (4, 2, 64, 1, 40)])
+@pytest.mark.parametrize("coef,every", [(0.4, 16), (-0.3, 7)])
+def test_a_factor_of_the_query_alone_in_one_launch(K, heads, kv_heads, head_dim, n, context, coef, every):
+    dtype, scale = torch.bfloat16, 1 / math.sqrt(head_dim)
+    lengths = [context - 3 * s for s in range(n)]
+    kp, vp, table, keys, values = make_cache(n, lengths, kv_heads, head_dim, dtype, seed=context)
+    qkv = torch.randn(n, (heads + 2 * kv_heads) * head_dim, generator=torch.Generator().manual_seed(context)).to(dtype)
+    positions = torch.tensor([length - 1 for length in lengths], dtype=torch.int32)
+    layout = Layout(True, dev(torch.arange(n + 1, dtype=torch.int32)), n, 1, context - 1)
+    k_pages, v_pages = stored(K, kp, vp)
+    out = torch.full((n, heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    assert K.attention_decode_pairs(dev(qkv), 0, out, None, None, 0.0, None, None, dev(positions), k_pages, v_pages, dev(table), heads, kv_heads,
+                                    head_dim, scale, True, layout, q_temp=(coef, every))
+    for s, length in enumerate(lengths):
+        row = qkv[s].reshape(heads + 2 * kv_heads, head_dim)
+        key, value = keys[s].clone(), values[s].clone()
+        key[-1], value[-1] = row[heads:heads + kv_heads], row[heads + kv_heads:]
+        factor = 1 + coef * math.log(length // every + 1)
+        want = attention_reference_rows(row[:heads].double().reshape(1, -1) * factor, key, value, positions[s:s + 1], heads, kv_heads, head_dim, scale, 0)
+        assert rel(out[s:s + 1], want) < 8e-3, (s, length)
 
 
 def test_splits_that_are_not_combined_are_refused_before_anything_runs(K):
@@ -84,17 +144,3 @@ def test_attention_into_rows_that_stand_on_two_bytes(K, heads, kv_heads, head_di
         assert K.attention_decode_fused(dev(row), out, None, None, 0.0, None, None, dev(positions), k_pages, v_pages, dev(table), heads, kv_heads,
                                         head_dim, scale, 0, True, layout)
         assert rel(out, want) < 8e-3
-
-
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("width", [4, 6, 1020, 1024, 1028, 4100, 5120])
-def test_embedding_rows(K, dtype, width):
-    table = torch.randn(50, width, generator=torch.Generator().manual_seed(width)).to(dtype).cuda()
-    tokens = torch.tensor([3, 49, 0, -1, 50, 17, 17], dtype=torch.int32, device="cuda:0")      # ids outside the table read row 0
-    source = torch.tensor([-1, -1, 1, -1, -1, 0, -1], dtype=torch.int32, device="cuda:0")
-    fed = torch.tensor([8, 9], dtype=torch.int32, device="cuda:0")
-    out = torch.full((7, width), float("nan"), device="cuda:0")
-    K.embed(tokens, table, out)
-    assert torch.equal(out, table.float()[[3, 49, 0, 0, 0, 17, 17]])
-    K.embed(tokens, table, out, token_src=source, fed_tokens=fed)
-    assert torch.equal(out, table.float()[[3, 49, 9, 0, 0, 8, 17]])
