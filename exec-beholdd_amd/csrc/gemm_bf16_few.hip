@@ -16,7 +16,9 @@
 // Which rows (gemm_few_rows), us at 8 / 16 rows:
 //   16, the block of the layout.
 //   8 where blocks of 16 leave half of the compute units idle and k is 1,536 or more (2,048 x 6,144 8.2 / 9.9 -> 7.2 / 8.5, 1,024 x
-//   3,072 5.2 / 5.9 -> 5.0 / 5.3; 1,024 x 1,024 3.5 -> 3.7: there the launch is the time).  Both halves of a block are whole cache lines.
+//   3,072 5.2 / 5.9 -> 5.0 / 5.3; 1,024 x 1,024 3.5 -> 3.7: there the launch is the time).  At 17 to 32 rows too, where the blocks of
+//   16 went in bursts (32 rows: 2,048 x 2,048 5.2 -> 5.1, 1,024 x 3,072 6.9 -> 6.2, 2,048 x 6,144 11.3 -> 10.8, 512 x 12,288 18.4 ->
+//   17.6, 2,048 x 12,288 21.0 -> 20.0; the least is 512 x 2,048 with 4.7 -> 4.75).  Both halves of a block are whole cache lines.
 //   20 or 24 where the blocks of 16 are more than the compute units and fewer than twice as many: otherwise some compute units carry
 //   two blocks, the others one, and the product takes as long as one of twice the compute units' blocks.
 #include "gemm_bf16_few.h"
@@ -63,9 +65,18 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const uint16_t
     wp[t] = w + (size_t)tile * full * 1024;
     if (GATED) wp[NB + t] = w + (size_t)(tile + N / 16) * full * 1024;
   }
+  // A lane without a row of its own in a block loads nothing; or, where all of a wave's chunks are asked for at once, what the lane of the
+  // nearest owned row does, which brings no line more and goes nowhere: each load under a branch of its own costs more there (2,048 x
+  // 2,048 at 8 / 16 / 32 rows 4.1 / 4.4 / 5.3 us, 3.8 / 4.1 / 5.1 so).  In turn it is the other way round (2,048 x 12,288 at 32 rows
+  // 20.0 us, 20.7 so).
+  constexpr bool SWITCHED = MASKED && !SHORT;
   bool mine[NB];
+  int place[NB];
 #pragma unroll
-  for (int t = 0; t < NB; ++t) mine[t] = i >= lo[t] && i < hi[t];
+  for (int t = 0; t < NB; ++t) {
+    mine[t] = i >= lo[t] && i < hi[t];
+    place[t] = 8 * (MASKED && SHORT ? 16 * g + max(min(i, hi[t] - 1), lo[t]) : lane);
+  }
   // A lane's two pieces of a chunk are the pieces 2 g and 2 g + 1 of its two 32-wide steps (bh_rows_index): 16 lanes read 256
   // neighbouring bytes; of blocks of 8 rows 128, and lanes 8 to 15 take the second piece of rows 0 to 7, which lies right behind the
   // first ones, so that one load brings both and a lane move hands the second to the lane of its row.
@@ -94,11 +105,12 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const uint16_t
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
+      if (NB > 1 && SHORT && hi[t % NB] <= lo[t % NB]) continue;   // the same for the whole workgroup
       const uint16_t* p = wp[t] + (size_t)at * 1024;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const u32x4_t* from = reinterpret_cast<const u32x4_t*>(p + h * 512 + lane * 8);
-        wv[u][t][h] = (!MASKED || mine[t % NB]) ? __builtin_nontemporal_load(from) : zero;
+        const u32x4_t* from = reinterpret_cast<const u32x4_t*>(p + h * 512 + place[t % NB]);
+        wv[u][t][h] = (!SWITCHED || mine[t % NB]) ? __builtin_nontemporal_load(from) : zero;
       }
     }
   };
