@@ -58,4 +58,4 @@ __device__ inline float capped_score(float s, float cap, float two_log2e_over_ca
 void bh_attention_prefill_launch(const void* q, void* out, const void* k_pages, const void* v_pages,
                                  const int32_t* page_table, int table_stride, const int32_t* positions,
                                  const int32_t* seq_start, int n_seqs, int tiles, int H, int KVH, int hd,
-                                 const ScoreForm& form, int window, int out_blocked, const HeadEnd& finish, hipStream_t stream);
+                                 const ScoreForm& form, int window, int out_blocked, float slack, const HeadEnd& finish, hipStream_t stream);

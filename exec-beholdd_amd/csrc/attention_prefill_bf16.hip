@@ -53,12 +53,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, const uint16_t* __restrict__ k_pages,
     const uint16_t* __restrict__ v_pages, const int32_t* __restrict__ page_table, int table_stride,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_start, int H, int KVH,
-    int window, int tile_groups, int n_seqs, int out_blocked, HeadEnd finish, ScoreForm form) {
+    int window, int tile_groups, int n_seqs, int out_blocked, float slack, HeadEnd finish, ScoreForm form) {
   constexpr int HD = 32 * NS;
   constexpr int PIECES = BH_PAGE * HD / 8;        // 16-byte pieces of one head's keys (or values) in a page
   constexpr int STAGE = 2 * PIECES / 256;         // pieces of a page (keys, then values) one thread copies
   constexpr int GROUP_TILES = 4 * CTW;            // column tiles of a workgroup
-  constexpr float SLACK = 8.0f;
   __shared__ u32x4_t page_lds[2][2 * PIECES];
 
   // Workgroups go to the eight XCDs in turn, each with an L2 of its own: when the number of
@@ -213,10 +212,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
       local_max = larger(larger(local_max, st[t][3]), t < 3 ? st[t + 1][0] : run_max[ct]);
     }
     const float new_max = largest_of_column(local_max);               // raw (unscaled) scores, the earlier pages' too
-    // The exponentials' reference moves only when the maximum has grown by more than SLACK powers of two (or
-    // from nothing): until then probabilities may reach 2^SLACK, which float32 sums and bfloat16 operands
+    // The exponentials' reference moves only when the maximum has grown by more than `slack` powers of two (or
+    // from nothing): until then probabilities may reach 2^slack, which float32 sums and bfloat16 operands
     // hold as well as numbers up to one, and what was summed so far needs no factor.
-    const bool stays = (new_max - run_max[ct]) * scale_log2[ct] <= SLACK;   // false from -inf, and while nothing was seen
+    const bool stays = (new_max - run_max[ct]) * scale_log2[ct] <= slack;   // false from -inf, and while nothing was seen
     const float reference = stays ? run_max[ct] : new_max;
     const float shift = (reference == -INFINITY) ? 0.f : -reference * scale_log2[ct];
     // exactly 1 while the reference stands still, 0 when nothing was seen before
@@ -359,12 +358,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 4 ? 2
 void bh_attention_prefill_launch(const void* q, void* out, const void* k_pages, const void* v_pages,
                                  const int32_t* page_table, int table_stride, const int32_t* positions,
                                  const int32_t* seq_start, int n_seqs, int tiles, int H, int KVH, int hd,
-                                 const ScoreForm& form, int window, int out_blocked, const HeadEnd& finish, hipStream_t stream) {
+                                 const ScoreForm& form, int window, int out_blocked, float slack, const HeadEnd& finish, hipStream_t stream) {
   const int formed = bh_formed(form);
 #define BH_PREFILL_ONE(NS, CTW, FORMED)                                                                      \
   attention_prefill_kernel<NS, CTW, FORMED><<<dim3(tile_groups * KVH * n_seqs), dim3(256), 0, stream>>>(     \
         (const uint16_t*)q, (uint16_t*)out, (const uint16_t*)k_pages, (const uint16_t*)v_pages, page_table,  \
-        table_stride, positions, seq_start, H, KVH, window, tile_groups, n_seqs, out_blocked, finish, form)
+        table_stride, positions, seq_start, H, KVH, window, tile_groups, n_seqs, out_blocked, slack, finish, form)
 #define BH_PREFILL(NS, CTW)                                                                                  \
   do {                                                                                                       \
     const int tile_groups = (tiles + 4 * CTW - 1) / (4 * CTW);                                               \
