@@ -30,10 +30,11 @@
 
 // A decode step can hand the kernel the fused projection rows themselves (struct FusedQkv) instead of
 // finished queries and a cache that already holds the new keys: every workgroup then norms and rotates
-// its own queries, and one wave of the sequence's last split norms and rotates the new key, treats it and
-// the new value as one more page of a single visible key, and writes both into the cache for the steps
-// to come.  The keys that come from the cache end one position earlier.  This takes the place of the
-// launch of the norm/rotation/cache-write kernel.
+// its own queries (a fifth wave for the four with the pages, or, in the lean form, each wave for itself), and one
+// wave of the sequence's last split norms and rotates the new key, attends to it with one product of it and the
+// queries and to the new value in plain float32, and writes both into the cache for the steps to come.  The keys
+// that come from the cache end one position earlier.  This takes the place of the launch of the
+// norm/rotation/cache-write kernel.
 //
 // The rows' heads come in one of two forms.  Whole heads turned in split halves by tables over positions (FUSED 1: HeadPrep);
 // or the first `turned` dimensions in neighbouring pairs by cosines and sines of the step's rows (FUSED 2: PairPrep), with the
@@ -223,16 +224,17 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // STREAM = one workgroup per (sequence, kv head, split): each cache byte is read once, past the caches.
 // FUSED = the step is a decode step and `fused.qkv` is given, in form 1 or 2 (struct FusedQkv).
 // LEAN (with FUSED) = the queries are normed and rotated before the first page is asked for, and the new key's
-// numbers are asked for after the last page: nothing of that overlaps with the pages any more, but what it needs
-// in registers is gone while the pages stream, so that two workgroups fit a compute unit.  For launches of more
-// workgroups than compute units, where the second workgroup is worth more than the overlap; and for heads of more than 128, which
-// went to scratch memory with it (16 sequences of 1,000 to 2,000 keys, 16 heads on 8: of 256 122 -> 42 us, of 192 44 -> 34).
+// numbers are asked for after the last page: nothing of that overlaps with the pages any more, but four waves do with what they
+// have, so that two workgroups fit a compute unit (a fifth wave a workgroup would be a third one on some SIMDs, whose
+// registers are two waves').  For launches of more workgroups than compute units, where the second workgroup is worth more
+// than the overlap; and for heads of more than 128, which went to scratch memory with all of it in registers (16 sequences of
+// 1,000 to 2,000 keys, 16 heads on 8, the launch and its combining: of 256 119.8 -> 38.0 us, of 192 41.6 -> 29.8).
 // FORMED = scores are more than a scaled product (struct ScoreForm): they are made in full, and exponentials taken of them as they
 // are (scale_log2 is then log2(e)).  Otherwise a column's factor is in scale_log2 (ScoreForm::scaled_only).
 // A workgroup of a FUSED step that is not LEAN has a fifth wave (heads of up to 128, whose pages leave two waves a SIMD their registers):
 // it norms and rotates the queries for all of them, while the others ask for their first pages and nothing else, and then takes the new
 // key, beside the pages.  (Every wave its own queries under its first page's loads, and the new key by the first wave behind its pages:
-// 4 sequences of 1,000 keys, 16 heads on 4 12.5 us, 11.0 now, of which the faster combining is 1.)
+// 4 sequences of 1,000 keys, 16 heads on 4 11.5 us with the combining, 9.4 now, in a chain of such launches.)
 __host__ __device__ constexpr bool fifth_wave(int ns, int fused, bool lean) { return fused && !lean && ns <= 4; }
 template <int NS, bool STREAM, int FUSED, bool LEAN = false, int FORMED = 0>
 __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN && NS <= 4 ? 2 : 1)) void attention_mfma_kernel(
@@ -343,12 +345,11 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
   for (int dt = 0; dt < 2 * NS; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // One page of keys and values in operand order against the 16 columns: lane (j, g) holds keys
-  // 64 p + 8 g + 32 (t / 2) + 4 (t % 2) + r.  A column sees keys see_lo .. see_hi; the bounds over the
+  // 64 p + 8 g + 32 (t / 2) + 4 (t % 2) + r.  A column sees keys lo .. pos; the bounds over the
   // wave say whether anything has to be masked at all.
-  auto attend = [&](const u32x4_t (&k_vec)[4][NS], u32x4_t (&v_vec)[2 * NS][2], int p, int see_hi, int see_lo,
-                    int hi_max, int hi_min, int lo_most) {
+  auto attend = [&](const u32x4_t (&k_vec)[4][NS], u32x4_t (&v_vec)[2 * NS][2], int p) {
     const int key0 = p * BH_PAGE + 8 * g;
-    const bool mask_needed = (p * BH_PAGE + BH_PAGE - 1 > hi_min) || (p * BH_PAGE < lo_most);
+    const bool mask_needed = (p * BH_PAGE + BH_PAGE - 1 > pos_min) || (p * BH_PAGE < lo_max);
     f32x4_t st[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -377,7 +378,7 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int key = key0 + 32 * (t / 2) + 4 * (t % 2) + r;
-          if (key > see_hi || key < see_lo) st[t][r] = -INFINITY;
+          if (key > pos || key < lo) st[t][r] = -INFINITY;
         }
     }
     float local_max = fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3]));
@@ -407,8 +408,8 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
       }
     run_sum = run_sum * alpha + page_sum;
     run_max = new_max;
-    if (p * BH_PAGE + BH_PAGE - 1 > hi_max) {  // the page's tail was never written: zero it
-      const int valid = hi_max + 1 - key0;
+    if (p * BH_PAGE + BH_PAGE - 1 > pos_max) {  // the page's tail was never written: zero it
+      const int valid = pos_max + 1 - key0;
 #pragma unroll
       for (int dt = 0; dt < 2 * NS; ++dt) {
         v_vec[dt][0] = keep_first(v_vec[dt][0], valid);
@@ -517,7 +518,7 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
     }
     for (bool asked = WAVES == 5; p < end; p += 4, asked = false) {
       if (!asked) ask_page(p);
-      attend(k_vec, v_vec, p, pos, lo, pos_max, pos_min, lo_max);
+      attend(k_vec, v_vec, p);
     }
   }
 
@@ -591,7 +592,8 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
 // Nothing here may wait for one split's numbers before asking for the next one's, nor for the maxima before asking for the outputs: a
 // thread asks for all eight at once and makes their weights itself, from numbers that are the same for its wave.  The groups are merged
 // through LDS.  The sums run over the splits in their order.  (One group for all, by eights, and the maxima and sums over the lanes of a
-// wave: 3.1 us of a decode step's launches at up to eight splits, of which the launch is 1.7; 2.2 now.)
+// wave, in traces of decode steps, at the median: one sequence, 8 heads, eight splits 4.8 us, 3.8 now; eight sequences, 32 heads, four
+// splits 4.8, 4.7 now.)
 #define COMBINE_SPLITS 8      // a group's; four where there are no more in all
 template <int SPLITS>
 __global__ __launch_bounds__(1024) void attention_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
