@@ -568,13 +568,11 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
       // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
       if (finish.sinks) sum += exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top);
       const float gate = head_gate<bf16_t>(finish, out_row, out_head);
-      const bool pairs = ((uintptr_t)out & 3) == 0;
 #pragma unroll
       for (int d = 0; d < EACH; d += 2) {   // (two neighbours from an even dimension on are neighbours in blocks too)
         uint16_t* to = out + bh_rows_index(out_block_rows, out_row, out_head * HD + d0 + d, H * HD);
-        const uint16_t one = f32_to_bf16_bits(value[d] * gate / sum), two = f32_to_bf16_bits(value[d + 1] * gate / sum);
-        if (pairs) *reinterpret_cast<uint32_t*>(to) = (uint32_t)one | ((uint32_t)two << 16);
-        else to[0] = one, to[1] = two;
+        const uint32_t word = (uint32_t)f32_to_bf16_bits(value[d] * gate / sum) | ((uint32_t)f32_to_bf16_bits(value[d + 1] * gate / sum) << 16);
+        __builtin_memcpy(to, &word, sizeof word);      // (it need not stand on four bytes)
       }
     } else {
       float* to = part_o + (column * n_splits + split) * HD + d0;
