@@ -540,47 +540,78 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
     for (int dt = 0; dt < 2 * NS; ++dt) *reinterpret_cast<f32x4_t*>(&sm_o[wave][j][16 * dt + 4 * g]) = o[dt];
     __syncthreads();
     if (WAVES == 5 && wave == 4) return;
-    // 16 threads a column, each with neighbouring dimensions of it
+    // 16 threads a column, each with neighbouring dimensions of it; or, of finished results of at most four columns, 64, each with a pair
+    // (few query heads a kv head left most threads idle: 16 sequences of 200 keys, 8 heads on 4 9.6 us, 9.3 so)
     constexpr int EACH = HD / 16;
-    const int col = threadIdx.x / 16, d0 = threadIdx.x % 16 * EACH, cc = tile * 16 + col;
+    const bool few = n_splits == 1 && n_cols - tile * 16 <= 4;
+    const int col = few ? threadIdx.x / 64 : threadIdx.x / 16, place = few ? threadIdx.x % 64 : threadIdx.x % 16, cc = tile * 16 + col;
     if (cc >= n_cols) return;
     float top = fmaxf(fmaxf(sm_m[0][col], sm_m[1][col]), fmaxf(sm_m[2][col], sm_m[3][col]));
     if (WAVES == 5) top = fmaxf(top, sm_m[WAVES - 1][col]);
     const float safe_top = (top == -INFINITY) ? 0.f : top;
-    float sum = 0.f, value[EACH];
-#pragma unroll
-    for (int d = 0; d < EACH; ++d) value[d] = 0.f;
-#pragma unroll
-    for (int v = 0; v < WAVES; ++v) {
-      if (v == 4 && !new_key_here) break;
-      const float f = exp2f(sm_m[v][col] - safe_top);
-      sum += sm_l[v][col] * f;
-#pragma unroll
-      for (int d = 0; d < EACH; d += 2) {
-        const float2 pair = *reinterpret_cast<const float2*>(&sm_o[v][col][d0 + d]);
-        value[d] += pair.x * f;
-        value[d + 1] += pair.y * f;
-      }
-    }
     const int out_row = row0 + cc / G, out_head = kvh * G + cc % G;
     const size_t column = (size_t)out_row * H + out_head;
-    if (n_splits == 1) {   // out_block_rows: the output [rows][H * HD] lies in blocks of that many rows (bh_rows_index)
-      // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
-      if (finish.sinks) sum += exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top);
-      const float gate = head_gate<bf16_t>(finish, out_row, out_head);
+    float gate = 1.f;
+    auto finish_sum = [&](float sum) {      // a sink: one more term exp(sinks[head]) in the softmax's sum (`top` is in powers of two)
+      gate = head_gate<bf16_t>(finish, out_row, out_head);
+      return finish.sinks ? sum + exp2f(finish.sinks[out_head] * 1.4426950408889634f - safe_top) : sum;
+    };
+    // out_block_rows: the output [rows][H * HD] lies in blocks of that many rows (bh_rows_index); two neighbours from an even dimension on
+    // are neighbours there too.  Their word need not stand on four bytes.
+    auto write = [&](int d, float first, float second, float sum) {
+      uint16_t* to = out + bh_rows_index(out_block_rows, out_row, out_head * HD + d, H * HD);
+      const uint32_t word = (uint32_t)f32_to_bf16_bits(first * gate / sum) | ((uint32_t)f32_to_bf16_bits(second * gate / sum) << 16);
+      __builtin_memcpy(to, &word, sizeof word);
+    };
+    if (!few) {
+      const int d0 = place * EACH;
+      float sum = 0.f, value[EACH];
 #pragma unroll
-      for (int d = 0; d < EACH; d += 2) {   // (two neighbours from an even dimension on are neighbours in blocks too)
-        uint16_t* to = out + bh_rows_index(out_block_rows, out_row, out_head * HD + d0 + d, H * HD);
-        const uint32_t word = (uint32_t)f32_to_bf16_bits(value[d] * gate / sum) | ((uint32_t)f32_to_bf16_bits(value[d + 1] * gate / sum) << 16);
-        __builtin_memcpy(to, &word, sizeof word);      // (it need not stand on four bytes)
+      for (int d = 0; d < EACH; ++d) value[d] = 0.f;
+#pragma unroll
+      for (int v = 0; v < WAVES; ++v) {
+        if (v == 4 && !new_key_here) break;
+        const float f = exp2f(sm_m[v][col] - safe_top);
+        sum += sm_l[v][col] * f;
+#pragma unroll
+        for (int d = 0; d < EACH; d += 2) {
+          const float2 pair = *reinterpret_cast<const float2*>(&sm_o[v][col][d0 + d]);
+          value[d] += pair.x * f;
+          value[d + 1] += pair.y * f;
+        }
+      }
+      if (n_splits == 1) {
+        sum = finish_sum(sum);
+#pragma unroll
+        for (int d = 0; d < EACH; d += 2) write(d0 + d, value[d], value[d + 1], sum);
+      } else {
+        float* to = part_o + (column * n_splits + split) * HD + d0;
+#pragma unroll
+        for (int d = 0; d < EACH; d += 2) *reinterpret_cast<float2*>(to + d) = make_float2(value[d], value[d + 1]);
+        if (d0 == 0) {
+          part_ml[(column * n_splits + split) * 2] = top;
+          part_ml[(column * n_splits + split) * 2 + 1] = sum;
+        }
       }
     } else {
-      float* to = part_o + (column * n_splits + split) * HD + d0;
+      float sum = 0.f, weight[WAVES];
 #pragma unroll
-      for (int d = 0; d < EACH; d += 2) *reinterpret_cast<float2*>(to + d) = make_float2(value[d], value[d + 1]);
-      if (d0 == 0) {
-        part_ml[(column * n_splits + split) * 2] = top;
-        part_ml[(column * n_splits + split) * 2 + 1] = sum;
+      for (int v = 0; v < WAVES; ++v) {
+        weight[v] = v == 4 && !new_key_here ? 0.f : exp2f(sm_m[v][col] - safe_top);
+        sum += sm_l[v][col] * weight[v];
+      }
+      sum = finish_sum(sum);
+#pragma unroll
+      for (int d = 2 * place; d < HD; d += 128) {
+        float2 value = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int v = 0; v < WAVES; ++v) {
+          if (v == 4 && !new_key_here) break;
+          const float2 pair = *reinterpret_cast<const float2*>(&sm_o[v][col][d]);
+          value.x += pair.x * weight[v];
+          value.y += pair.y * weight[v];
+        }
+        write(d, value.x, value.y, sum);
       }
     }
   }
