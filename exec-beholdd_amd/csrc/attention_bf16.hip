@@ -782,7 +782,10 @@ static int attention_bf16_run(const void* q, void* out, void* part_o, void* part
   BH_REQUIRE(out_blocked == 0 || ((out_blocked == 8 || out_blocked == 16) && (H * hd) % 32 == 0),
              "attention_bf16: the output's rows lie in blocks of 8 or 16, or one after the other (0), not %d", out_blocked);
   const int tile_groups = tiles, z_count = n_seqs * n_splits;
-  const bool lean = (long)tiles * KVH * z_count > bh_compute_units();   // more workgroups than compute units: two of them per unit
+  // More workgroups than compute units: two of them per unit.  And long runs of pages, whose workgroups the fifth wave does not make faster
+  // (32 sequences of 5,000 keys, 79 pages a workgroup, 32 heads on 8 106.4 us before there was one, 108.9 with it, 106.7 lean, 8 heads on
+  // 8 101.6 / 106.4 / 102.8; at 31 and 40 pages within 2 % either way, at 16 and fewer up to 9 % for it where one page is all).
+  const bool lean = (long)tiles * KVH * z_count > bh_compute_units() || per > 24;
   dim3 grid(tile_groups * KVH * z_count);
 #define BH_ATT_ONE(NS, STREAM, FUSED, ...)                                                                      \
   attention_mfma_kernel<NS, STREAM, FUSED, __VA_ARGS__><<<grid, is_fused && !lean && NS <= 4 ? 320 : 256, 0, stream>>>(        \

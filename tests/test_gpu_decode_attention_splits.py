@@ -11,6 +11,29 @@ from test_gpu_kernels import K, Layout, as_rows, attention_reference_rows, dev, 
 pytestmark = pytest.mark.gpu
 
 
+# 24 and 25 pages a workgroup of one that has a compute unit for itself, and one column and five of them
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(4, 4, 32), (20, 4, 64), (4, 4, 128)])
+@pytest.mark.parametrize("context", [24 * 64, 24 * 64 + 1])
+def test_long_runs_of_pages(K, heads, kv_heads, head_dim, context):
+    dtype, scale, lengths = torch.bfloat16, 1 / math.sqrt(head_dim), [context] + [1, 70] * 31 + [context // 2]
+    n = len(lengths)
+    assert int(K.lib.bh_attention_bf16_splits(n, 1, heads, kv_heads, context - 1)) == 1
+    kp, vp, table, keys, values = make_cache(n, lengths, kv_heads, head_dim, dtype, seed=context)
+    qkv = torch.randn(n, (heads + 2 * kv_heads) * head_dim, generator=torch.Generator().manual_seed(context)).to(dtype)
+    positions = torch.tensor([length - 1 for length in lengths], dtype=torch.int32)
+    layout = Layout(True, dev(torch.arange(n + 1, dtype=torch.int32)), n, 1, context - 1)
+    k_pages, v_pages = stored(K, kp, vp)
+    out = torch.full((n, heads * head_dim), float("nan"), dtype=dtype, device="cuda:0")
+    assert K.attention_decode_fused(dev(qkv), out, None, None, 0.0, None, None, dev(positions), k_pages, v_pages, dev(table), heads, kv_heads,
+                                    head_dim, scale, 0, True, layout)
+    for s, length in enumerate(lengths):
+        row = qkv[s].reshape(heads + 2 * kv_heads, head_dim)
+        key, value = keys[s].clone(), values[s].clone()
+        key[-1], value[-1] = row[heads:heads + kv_heads], row[heads + kv_heads:]
+        want = attention_reference_rows(row[:heads].reshape(1, -1), key, value, positions[s:s + 1], heads, kv_heads, head_dim, scale, 0)
+        assert rel(out[s:s + 1], want) < 8e-3, (s, length)      # probabilities and results of 8 bits
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(2, 1, 128), (5, 1, 64), (4, 2, 256), (3, 3, 96)])
 @pytest.mark.parametrize("context,bucket", [(1, 1), (447, 7), (449, 8), (512, 16), (1100, 20), (1024, 32), (2049, 33), (4000, 72), (9000, 144), (17000, 272)])
 def test_decode_attention_in_splits(K, heads, kv_heads, head_dim, context, bucket):

@@ -107,7 +107,7 @@ def test_scores_whose_factor_is_not_positive(K, n_heads, kv_heads, head_dim, new
                                             head_dim, scale, 0, True, layout)
 
 
-@pytest.mark.parametrize("n_heads,kv_heads,head_dim,new", [(8, 2, 128, 448), (8, 2, 128, 256), (8, 4, 64, 256)])
+@pytest.mark.parametrize("n_heads,kv_heads,head_dim,new", [(16, 8, 128, 448), (8, 2, 128, 256), (8, 4, 64, 256)])
 def test_error_is_that_of_pages_by_their_own_maximum(K, n_heads, kv_heads, head_dim, new):
     """Scores spread by two, whose maximum grows by a little from page to page.  What else runs at these sizes rounds a page's probabilities
     against the page's own maximum, so that the largest is a one, and sums them unrounded: the error against float64 is held to that
