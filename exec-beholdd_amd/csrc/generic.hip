@@ -539,7 +539,11 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
     const int near = min(max(base + lane, 0), n_rows - 1);
     const int near_pos = positions[near], near_seq = row_seq[near];
     auto pos_of = [&](int row) { return __builtin_amdgcn_readlane(near_pos, __builtin_amdgcn_readfirstlane(row - base)); };
-    auto seq_of = [&](int row) { return __builtin_amdgcn_readlane(near_seq, __builtin_amdgcn_readfirstlane(row - base)); };
+    // bit i: row base + i holds the token behind that of the row before it (looked at token by token for each of the eight rows, this was
+    // most of what such a wave did: 4 prompts of 1,030 rows, 16 heads of 64 on 2 13.6 us, 12.0 so)
+    const int pos_before = __shfl_up(near_pos, 1, BH_WAVE), seq_before = __shfl_up(near_seq, 1, BH_WAVE);
+    const unsigned follows = (unsigned)__ballot(lane > 0 && lane < 24 && base + lane > 0 && base + lane < n_rows && near_seq == seq_before &&
+                                                near_pos == pos_before + 1);
     const int near_page = page_table[(size_t)near_seq * table_stride + near_pos / BH_PAGE];
     auto block_of = [&](int row) {
       const int page = __builtin_amdgcn_readlane(near_page, __builtin_amdgcn_readfirstlane(row - base));
@@ -554,13 +558,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
     for (int i = 0; i < 8; ++i) {
       const int row = 8 * group + i;
       if (row >= n_rows) break;
-      const int pos = pos_of(row), seq = seq_of(row);
-      const int first = row - pos % 8;   // where the row of the piece's first token would lie
-      bool whole = first >= 0 && first + 7 < n_rows;   // the piece's eight tokens are the rows first .. first + 7, in order
-      if (whole) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) whole = whole && seq_of(first + t) == seq && pos_of(first + t) == pos - pos % 8 + t;
-      }
+      const int pos = pos_of(row), first = 8 + i - pos % 8;   // where the row of the piece's first token would lie, from base on
+      const bool whole = (follows >> first & 0xfeu) == 0xfeu;   // the piece's eight tokens are the rows from there on, in order
       if (!whole) single |= 1u << i;
       else if (pos % 8 == 0) starts = row;
     }
