@@ -540,7 +540,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_rows_kernel(
     const int near_pos = positions[near], near_seq = row_seq[near];
     auto pos_of = [&](int row) { return __builtin_amdgcn_readlane(near_pos, __builtin_amdgcn_readfirstlane(row - base)); };
     // bit i: row base + i holds the token behind that of the row before it (looked at token by token for each of the eight rows, this was
-    // most of what such a wave did: 4 prompts of 1,030 rows, 16 heads of 64 on 2 13.6 us, 12.0 so)
+    // most of what such a wave did: 4 prompts of 1,030 rows, 16 heads of 64 on 2 13.6 us, 12.0 so; 253 rows of three, 40 heads of 128 on 8
+    // 7.2, 6.4 so)
     const int pos_before = __shfl_up(near_pos, 1, BH_WAVE), seq_before = __shfl_up(near_seq, 1, BH_WAVE);
     const unsigned follows = (unsigned)__ballot(lane > 0 && lane < 24 && base + lane > 0 && base + lane < n_rows && near_seq == seq_before &&
                                                 near_pos == pos_before + 1);

@@ -493,14 +493,15 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_waves_kernel(const fl
 // The same in pieces of 16 bytes of z and out, LANES lanes a group, all loads of a group before its sums: single elements are waited for
 // a few bytes at a time (2,048 rows of 32 heads of 128 in bfloat16 35 us, 23.9 now; 8,192 rows 124 -> 76).  Many small groups take
 // few lanes each and few large ones many, so that few lanes have nothing to do (3 groups of 512 on 32 lanes 28.7 us, on 64 16.2).
-// Eight lanes go with groups of a piece each: as an array of one, which stays in registers (8,192 rows of 64 groups of 32 in float32 59.5
-// -> 31.2 us, of 64 in bfloat16, 128 a row, 146 -> 108; of as many as 512 elements need, it lay in scratch memory or took 165 registers).
+// Eight lanes go with groups of a piece each, 16 with up to two: the arrays are no longer than that, and stay in registers (8,192 rows of
+// 64 groups of 32 in float32 59.5 -> 31.2 us, of 64 in bfloat16, 128 a row, 146 -> 108; of as many as 512 elements need, eight lanes had
+// scratch memory or 165 registers).
 template <typename T, int LANES, bool SPREAD>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_pieces_kernel(const float* __restrict__ y, const T* __restrict__ z, int z_stride,
                                                                         int z_first, const float* __restrict__ w, float eps,
                                                                         T* __restrict__ out, int n_rows, int width, int groups, int out_block_rows,
                                                                         int gate_after) {
-  constexpr int VEC = 16 / sizeof(T), PIECES = LANES == 8 ? 1 : 512 / (VEC * LANES);
+  constexpr int VEC = 16 / sizeof(T), PIECES = LANES <= 16 ? LANES / 8 : 512 / (VEC * LANES);
   const int row = bh_row_of_block<SPREAD>(), per = width / groups, lane = threadIdx.x % LANES;
   if (SPREAD && row >= n_rows) return;
   // a wave's lanes stay together (their sums are exchanged): those without a group take the last one's numbers and write nothing
@@ -558,18 +559,26 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_pieces_kernel(const f
 }
 
 // In blocks out's pieces are of 8 columns, so that 16 bytes of a row are contiguous there too.
+// Few small groups stay with a wave a group: in pieces most lanes would have nothing to do and the others four or eight elements one after
+// the other.  us at 8,192 rows, a wave a group / pieces: bfloat16 2 x 64 8.0 / 13.7, 4 x 128 13.6 / 20.9, 2 x 256 12.1 / 14.4, 4 x 384
+// 27.4 / 22.7, 8 x 64 17.2 / 21.6, 12 x 64 24.0 / 33.1, 6 x 128 21.2 / 19.5, 9 x 128 28.4 / 29.0; float32 2 x 64 8.1 / 9.4, 4 x 128 15.3 /
+// 15.7, 3 x 192 15.5 / 13.5, 6 x 32 14.6 / 12.3; at 128 rows bfloat16 4 x 128 3.3 / 3.5, 4 x 256 3.9 / 3.4, float32 2 x 64 2.8 / 3.1, 4 x
+// 128 3.15 / 3.0.  (Of many groups, more than two pieces for each of 16 lanes are better spread over 32: 8,192 rows of 17 x 256 in
+// float32 98.6 -> 82.6, 2,048 of them, which a wave a group took 22.6 for, 25.6 -> 21.4.)
 template <typename T>
 static void gated_group_rmsnorm_groups(const float* y, const T* z, int z_stride, int z_first, const float* w, float eps, T* out, int n_rows,
                                       int width, int groups, int out_block_rows, int gate_after, hipStream_t stream) {
   constexpr int VEC = 16 / sizeof(T);
-  const bool pieces = width / groups % VEC == 0 && z_stride % VEC == 0 && z_first % VEC == 0 &&
+  const int per = width / groups;
+  const bool pieces = per % VEC == 0 && z_stride % VEC == 0 && z_first % VEC == 0 &&
                       ((uintptr_t)y | (uintptr_t)w | (uintptr_t)z | (uintptr_t)out) % 16 == 0;
+  const bool idle = groups <= 4 ? per <= (n_rows < 2 * bh_compute_units() ? 16 : 32) * VEC : groups < 16 && VEC == 8 && per <= 64;
 #define BH_GROUPS(KERNEL, ...)                                                                                             \
   BH_BY_ROWS(T, n_rows, out_block_rows, 256, stream,                                                                       \
              (y, z, z_stride, z_first, w, eps, out, n_rows, width, groups, out_block_rows, gate_after), KERNEL, __VA_ARGS__)
-  if (!pieces) BH_GROUPS(gated_group_rmsnorm_waves_kernel, T);
-  else if (groups >= 16 && width / groups <= 8 * VEC) BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 8);
-  else if (groups >= 16) BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 16);
+  if (!pieces || idle) BH_GROUPS(gated_group_rmsnorm_waves_kernel, T);
+  else if (groups >= 16 && per <= 8 * VEC) BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 8);
+  else if (groups >= 16 && per <= 32 * VEC) BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 16);
   else if (groups > 4) BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 32);
   else BH_GROUPS(gated_group_rmsnorm_pieces_kernel, T, 64);
 #undef BH_GROUPS
