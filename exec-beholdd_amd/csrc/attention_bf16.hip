@@ -234,7 +234,9 @@ __device__ inline void pack_head(u32x4_t (&out)[NS], const float (&x)[NS][8]) {
 // A workgroup of a FUSED step that is not LEAN has a fifth wave (heads of up to 128, whose pages leave two waves a SIMD their registers):
 // it norms and rotates the queries for all of them, while the others ask for their first pages and nothing else, and then takes the new
 // key, beside the pages.  (Every wave its own queries under its first page's loads, and the new key by the first wave behind its pages:
-// 4 sequences of 1,000 keys, 16 heads on 4 11.5 us with the combining, 9.4 now, in a chain of such launches.)
+// 4 sequences of 1,000 keys, 16 heads on 4 11.5 us with the combining, 9.4 now, in a chain of such launches, of which more is the
+// combining's and the merge's.  The lean form in its place: 5 to 9 % of the launch slower where a page is all, within 5 % either way at up
+// to 24 pages a workgroup.)
 __host__ __device__ constexpr bool fifth_wave(int ns, int fused, bool lean) { return fused && !lean && ns <= 4; }
 template <int NS, bool STREAM, int FUSED, bool LEAN = false, int FORMED = 0>
 __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN && NS <= 4 ? 2 : 1)) void attention_mfma_kernel(
@@ -621,8 +623,8 @@ __global__ __launch_bounds__((fifth_wave(NS, FUSED, LEAN) ? 320 : 256), (LEAN &&
 // Nothing here may wait for one split's numbers before asking for the next one's, nor for the maxima before asking for the outputs: a
 // thread asks for all eight at once and makes their weights itself, from numbers that are the same for its wave.  The groups are merged
 // through LDS.  The sums run over the splits in their order.  (One group for all, by eights, and the maxima and sums over the lanes of a
-// wave, in traces of decode steps, at the median: one sequence, 8 heads, eight splits 4.8 us, 3.8 now; eight sequences, 32 heads, four
-// splits 4.8, 4.7 now.)
+// wave, took 4.8 us in traces of decode steps of one sequence with eight splits and of eight sequences with four; 3.8 to 4.7 now, and 4.7
+// to 4.8.)
 #define COMBINE_SPLITS 8      // a group's; four where there are no more in all
 template <int SPLITS>
 __global__ __launch_bounds__(1024) void attention_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
