@@ -148,6 +148,10 @@ class Engine:
         self._last_selection = self.sampler.select_async(logits, params, requests, steps)
         return self._last_selection
 
+    def kept_logits(self, logits):
+        """`logits` in memory of their own, which no later step writes."""
+        return logits.clone()
+
     # ---- the step function ----
     def step(self, entries: list, extras: dict | None = None):
         """Run the given tokens of each entry's sequence from the cache; return float32 logits

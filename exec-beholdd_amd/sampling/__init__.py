@@ -11,6 +11,7 @@ batch a request happens to be in.
 from __future__ import annotations
 
 import numbers
+import weakref
 from dataclasses import dataclass
 
 import torch
@@ -70,44 +71,70 @@ class Selection:
     `result()` waits for them and returns them as a list (raising for a row whose logits were not
     finite).  Until then, and afterwards, the tokens also stand in the sampler's device buffer:
     element i at row `device_rows[i]`, where the next step can read them without the host
-    (`StepEntry.fed_row`).  A selection is good until the sampler has made a few more."""
+    (`StepEntry.fed_row`), for as long as the sampler has made no other selection (`on_device`)."""
 
-    def __init__(self, host, event, device_rows, requests, steps):
-        self._host, self._event = host, event
+    def __init__(self, arrival, device_rows, requests, steps):
+        self._arrival = arrival
         self.device_rows, self.requests, self.steps = list(device_rows), list(requests), list(steps)
 
     def __len__(self):
         return len(self.device_rows)
 
+    @property
+    def on_device(self) -> bool:
+        """Whether the tokens still stand in the sampler's device buffer: no selection was made since."""
+        return self._arrival.newest()
+
     def take(self, positions):
         """The selection restricted to some of its elements."""
-        return Selection(self._host, self._event, [self.device_rows[i] for i in positions],
+        return Selection(self._arrival, [self.device_rows[i] for i in positions],
                          [self.requests[i] for i in positions], [self.steps[i] for i in positions])
 
     def token_at(self, device_row: int) -> int:
         """The token at a row of the device buffer, waited for; no check of the row's flag."""
-        if self._event is not None:
-            self._event.synchronize()
-        return int(self._host[0, device_row])
+        return int(self._arrival.rows()[0, device_row])
 
     def result(self) -> list:
-        if self._event is not None:
-            self._event.synchronize()
+        chosen, bad = self._arrival.rows()
         tokens = []
         for row, request, step in zip(self.device_rows, self.requests, self.steps):
-            if int(self._host[1, row]):
+            if bad[row]:
                 raise SamplingError(f"request {request}, step {step}: a logit is not finite")
-            tokens.append(int(self._host[0, row]))
+            tokens.append(int(chosen[row]))
         return tokens
+
+
+class _Arrival:
+    """One selection's tokens and flags on their way into a host buffer, read from it once: before the sampler
+    uses the buffer for another selection it asks a selection that somebody still holds to read its own."""
+
+    def __init__(self, sampler, host, event):
+        self._sampler, self._serial = weakref.ref(sampler), sampler.selections
+        self._host, self._event, self._rows = host, event, None
+
+    def rows(self):
+        """The buffer's two rows, tokens and flags, waited for: a copy, whatever becomes of the buffer."""
+        if self._rows is None:
+            if self._event is not None:
+                self._event.synchronize()
+            self._rows = self._host.numpy().copy()
+            self._host = self._event = None
+        return self._rows
+
+    def newest(self) -> bool:
+        sampler = self._sampler()
+        return sampler is not None and sampler.selections == self._serial
 
 
 class Sampler:
     """Runs the selection kernel on rows of float32 logits."""
 
-    RING = 4      # host buffers in turn: a selection stays readable while the next few are made
+    RING = 4      # host buffers in turn: a selection is not waited for while the next few are made
 
     def __init__(self, kernels, device, capacity: int = 64):
         self.kernels, self.device = kernels, torch.device(device)
+        self.selections = 0                       # how many were made
+        self._arrivals = [None] * self.RING       # weak references to what each host buffer was last used for
         self._allocate(int(capacity))
 
     def _allocate(self, capacity):
@@ -174,8 +201,12 @@ class Sampler:
             self.kernels.sample(logits, tokens, bad, temperature=on_device[0, :n_rows],
                                 top_k=counts_on_device[:n_rows] if any_k else None,
                                 top_p=on_device[1, :n_rows] if any_p else None, uniform=on_device[2, :n_rows])
-        host = self._hosts[self._turn]
-        self._turn = (self._turn + 1) % self.RING
+        turn = self._turn
+        self._turn = (turn + 1) % self.RING
+        before = self._arrivals[turn]() if self._arrivals[turn] is not None else None
+        if before is not None:
+            before.rows()
+        host = self._hosts[turn]
         event = None
         if self.device.type == "cuda":
             host.copy_(self.out, non_blocking=True)
@@ -183,7 +214,10 @@ class Sampler:
             event.record()
         else:
             host.copy_(self.out)
-        return Selection(host, event, range(n_rows), requests, steps)
+        self.selections += 1
+        arrival = _Arrival(self, host, event)
+        self._arrivals[turn] = weakref.ref(arrival)
+        return Selection(arrival, range(n_rows), requests, steps)
 
     def select(self, logits: torch.Tensor, params: list, requests: list, steps: list) -> list:
         """One token per row of `logits`, on the host."""

@@ -365,3 +365,77 @@ def test_generation_with_a_limit_on_a_steps_tokens():
         assert result.token_ids == expected_tokens(s, prompt, n)
     assert s.steps[:6] == [[(0, 5), (1, 3)], [(1, 8)], [(2, 8)], [(2, 8)], [(2, 1), (3, 1)], [(0, 1), (1, 1), (2, 1), (3, 1)]]
     assert s.state == {}
+
+
+class KeptStepper(ScriptedStepper):
+    """A stepper as the engine is one: logits in one buffer that every step writes again, the package's sampler (here on
+    the CPU), tokens read from its buffer by the next step, rows kept for a callback."""
+
+    class Kernels:
+        def sample(self, logits, tokens, bad, **numbers):
+            tokens.copy_(logits.argmax(dim=1))
+            bad.zero_()
+
+    def __init__(self, *args, **kwargs):
+        super().__init__(*args, **kwargs)
+        from beholdd.sampling import Sampler
+        self.sampler = Sampler(self.Kernels(), "cpu", capacity=self.max_slots)
+        self.buffer = torch.zeros(self.max_slots, self.vocab)
+        self.fed = self.fed_by_host = 0
+
+    def step(self, entries):
+        resolved = []
+        for e in entries:
+            if e.fed_row is not None:
+                self.fed += 1
+                e = type(e)(e.slot, [int(self.sampler.device_tokens[e.fed_row])], e.want)
+            elif self.state[e.slot] is not None:
+                self.fed_by_host += 1
+            resolved.append(e)
+        logits = super().step(resolved)
+        self.buffer[:len(logits)] = logits
+        return self.buffer[:len(logits)]
+
+    def select_async(self, logits, params, requests, steps):
+        return self.sampler.select_async(logits, params, requests, steps)
+
+    def kept_logits(self, logits):
+        return logits.clone()
+
+
+@pytest.mark.parametrize("nested", [0, 1, 9])      # selections that the callback makes for itself; nine: more than there are host buffers
+def test_the_loop_ahead_shows_a_callback_the_rows_each_token_was_chosen_from(nested):
+    prompts = [[1, 2, 3], [2, 2], [5], [7, 1], [3]]
+    free_run = [expected_tokens(ScriptedStepper(), p, 7) for p in prompts]
+    for stop in (free_run[1][2], free_run[0][0], free_run[4][6], 49):
+        outcomes = []
+        for s in (ScriptedStepper(), KeptStepper()):
+            seen = []
+
+            def on_logits(index, step, row):
+                seen.append((index, step, row.clone().tolist()))
+                for n in range(nested if isinstance(s, KeptStepper) else 0):
+                    assert s.select_async(torch.eye(s.vocab)[[n, 40, 41, 42, 43, 44]], [SamplingParams()] * 6, [0] * 6, [0] * 6).result()[0] == n
+
+            results = generate(s, prompts, [7, 7, 4, 7, 1], stop_token_ids=[stop], on_token=lambda i, t: seen.append((i, t)), on_logits=on_logits)
+            outcomes.append(([(r.token_ids, r.finish_reason, r.stop_token) for r in results], seen))
+            assert s.state == {} and sorted(s.free) == list(range(s.max_slots))
+        assert outcomes[0] == outcomes[1]
+        assert s.fed_by_host == 0 if nested == 0 else s.fed > 0 and s.fed_by_host > 0
+
+
+def test_nothing_runs_ahead_of_a_control_that_stands_beside_a_callback_for_logits():
+    log, s = [], KeptStepper()
+    generate(s, [[1], [2, 3]], 3, on_logits=lambda i, step, row: log.append((i, step)), control=lambda: log.append(len(s.steps)))
+    assert log == [0, (0, 0), (1, 0), 1, (0, 1), (1, 1), 2, (0, 2), (1, 2)] and s.fed == 0
+
+
+def test_a_selection_is_read_before_its_buffer_is_used_again():
+    s = KeptStepper()
+    rows = torch.eye(s.vocab)
+    held = s.sampler.select_async(rows[[3, 4]], [SamplingParams()] * 2, [0, 1], [0, 0])
+    assert held.on_device and held.take([1]).on_device
+    for n in range(2 * s.sampler.RING + 1):
+        later = s.sampler.select_async(rows[[n]], [SamplingParams()], [0], [0])
+    assert held.result() == [3, 4] and held.take([1]).result() == [4] and held.token_at(1) == 4 and not held.on_device
+    assert later.result() == [2 * s.sampler.RING] and later.on_device and later.token_at(1) == 4       # (row 1 of the buffer is still the first one's)
