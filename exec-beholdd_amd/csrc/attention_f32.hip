@@ -8,8 +8,9 @@
 // its own sums over its four tokens of each page; they are added over the lanes once, behind the last page.  The waves' softmax
 // sums are merged through LDS.
 // Bound by the pages' way from memory or the L2 (a page of a head of 128 is 64 KB): NR rows share it.
-// Measured (8 heads of 128 on 4): a decode step of 4 rows at 40 to 300 keys 8.2 us, 54 with a thread a key (generic.hip: every
-// lane its own line), 20 before a page's keys and values were asked for together; four prompts of 695 rows in all, up to 256 each,
+// Measured (8 heads of 128 on 4): a decode step of 4 rows at 40 to 300 keys with its norms, rotation and cache write 7.0 us in a chain of
+// such launches, 8.5 in two of them and 10.4 before eight waves took half pages (PARTS); the attention alone 54 with a thread a key
+// (generic.hip: every lane its own line), 20 before a page's keys and values were asked for together; four prompts of 695 rows in all, up to 256 each,
 // 41 us in waves of their own (30 in tiles of columns, see there), 94 in workgroups of four waves on four rows, 120 there.
 #include "common.h"
 #include <algorithm>
@@ -18,6 +19,17 @@
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 namespace {
+
+// A decode step's fused projection rows [q heads | k heads | v heads] in the place of finished queries and of a cache that holds the
+// new keys already: see attend_rows.
+struct F32Fused {
+  const float* qkv;
+  const float *q_weight, *k_weight;     // per-head RMSNorm weights [head size], or null for no norm
+  float eps;
+  const float *cos_table, *sin_table;   // [positions][head size / 2]: rotation over the whole head in split halves, or null for none
+  int write_kv;                         // 0: the cache entry belongs to another layer, which has written the new key already
+  float *k_pages, *v_pages;             // the cache again, to write into
+};
 
 struct F32Attention {
   const float* q;
@@ -30,6 +42,7 @@ struct F32Attention {
   ScoreForm form;
   int window;
   HeadEnd finish;
+  F32Fused fused;
 };
 
 __device__ inline floatx4 load4(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
@@ -40,60 +53,168 @@ struct Lds {
   float probs[WAVES][NR][BH_PAGE];
   float most[WAVES][NR], sum[WAVES][NR];
   float o[WAVES][NR][32 * P];
+  float new_score;      // of a decode step's new key
+};
+
+// A head as a wave's lanes hold it (elements 32 p + 4 dq + e; the eight lanes of other keys hold the same): RMSNorm, then split-half
+// rotation.  The partner of element i < HD / 2 is i + HD / 2, in the same lane, P / 2 slices on.
+template <int P>
+struct HeadTurn {
+  floatx4 weight[P], cos_v[P > 1 ? P / 2 : 1], sin_v[P > 1 ? P / 2 : 1];
+
+  __device__ void ask_weight(const float* of, int dq) {
+    if (of)
+#pragma unroll
+      for (int p = 0; p < P; ++p) weight[p] = load4(of + 32 * p + 4 * dq);
+  }
+  __device__ void ask_angles(const F32Fused& f, int pos, int dq) {
+    if (f.cos_table)
+#pragma unroll
+      for (int p = 0; p < P / 2; ++p) {
+        cos_v[p] = load4(f.cos_table + (size_t)pos * (16 * P) + 32 * p + 4 * dq);
+        sin_v[p] = load4(f.sin_table + (size_t)pos * (16 * P) + 32 * p + 4 * dq);
+      }
+  }
+  __device__ void apply(floatx4 (&x)[P], const F32Fused& f, const HeadTurn& angles) const {
+    if (f.q_weight) {
+      float ss = 0.f;
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += x[p][e] * x[p][e];
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) ss += __shfl_xor(ss, off, BH_WAVE);
+      const float inv = 1.0f / sqrtf(ss / (float)(32 * P) + f.eps);
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[p][e] = x[p][e] * inv * weight[p][e];
+    }
+    if (f.cos_table) {
+#pragma unroll
+      for (int p = 0; p < P / 2; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = x[p][e], hi = x[p + P / 2][e], c = angles.cos_v[p][e], s = angles.sin_v[p][e];
+          x[p][e] = lo * c - hi * s;
+          x[p + P / 2][e] = lo * s + hi * c;
+        }
+    }
+  }
 };
 
 // Rows row0 .. row0 + NR - 1, all of the sequence of row0.
-template <int P, int NR, int WAVES>
+// FUSED: a decode step (row s is sequence s's) from its projection rows, in place of the norm, rotation and cache write in a launch of
+// their own: every wave norms and rotates its query while its first page is on its way, whose number it asks for beside the position;
+// the last wave, which has the fewest pages, makes the new key and its score first.  In the merge that score and the new value are one
+// wave more.  The first head of a group writes both into the cache, whose keys are read to one position earlier.
+// PARTS: a wave takes a page's tokens in so many parts, a part at a time: of two parts a head of 96 or 128 fits the registers of eight waves
+// with all of a part's loads ahead, of whole pages those of four (decode steps with norms, rotation and cache write, us, whole pages and four
+// waves / half pages and eight: one row of 300 keys 9.1 / 7.0, 8 rows of 400 keys and 16 heads 10.0 / 7.9, 4 rows of 800 14.5 / 11.4).
+template <int P, int NR, int WAVES, bool FUSED = false, int PARTS = 1>
 __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int row0, int head) {
+  static_assert(!FUSED || NR == 1, "a decode step's rows are each of their own sequence");
+  static_assert(PARTS == 1 || PARTS == 2, "the sums over lanes are written for these");
+  constexpr int TOKENS = BH_PAGE / PARTS, GROUPS = TOKENS / 8;      // of a part, and its keys by eights
+  constexpr int TQ = TOKENS / 4, DL = 64 / TQ, ND = 32 * P / DL;    // lanes that share a dimension's values, dimensions a load, loads
   constexpr int HD = 32 * P;
   constexpr bool AHEAD = NR == 1 && P <= 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kl = lane >> 3, dq = lane & 7;    // keys: the lane's key among eight, its 16 bytes of each 32 dimensions
-  const int dl = lane >> 4, tq = lane & 15;   // values: the lane's dimension among four, its four tokens
+  const int dl = lane / TQ, tq = lane % TQ;   // values: the lane's dimension of a load's, its four tokens
   const int kv_head = head / (t.H / t.KVH);
-  const int32_t* table = t.page_table + (size_t)t.row_seq[row0] * t.table_stride;
+  const int32_t* table = t.page_table + (size_t)(FUSED ? row0 : t.row_seq[row0]) * t.table_stride;
   const float slope = t.form.slopes ? t.form.slopes[head] : 0.f;
 
-  int pos[NR], first[NR], from = 0x7fffffff, upto = 0;
+  const int page_guess = FUSED && wave / PARTS < t.table_stride ? table[wave / PARTS] : 0;      // the wave's first page if no window cuts the front off
+  const bool new_key_apart = FUSED && t.fused.write_kv, takes_new_key = new_key_apart && wave == WAVES - 1;
+  // pos: a row's own position; last: that of the last key it takes from the cache (-1: none)
+  int pos[NR], last[NR], first[NR], from = 0x7fffffff, upto = -1, new_page = 0;
   float scale[NR];
-  floatx4 q[NR][P];
+  floatx4 q[NR][P], new_key[FUSED ? P : 1];
+  HeadTurn<P> q_turn, k_turn;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     pos[r] = t.positions[row0 + r];
+    if constexpr (FUSED) {
+      const float* row = t.fused.qkv + (size_t)row0 * (t.H + 2 * t.KVH) * HD;
+#pragma unroll
+      for (int p = 0; p < P; ++p) q[0][p] = load4(row + head * HD + 32 * p + 4 * dq);
+      q_turn.ask_weight(t.fused.q_weight, dq);
+      if (takes_new_key) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) new_key[p] = load4(row + (t.H + kv_head) * HD + 32 * p + 4 * dq);
+        k_turn.ask_weight(t.fused.k_weight, dq);
+      }
+      q_turn.ask_angles(t.fused, pos[0], dq);
+      if (new_key_apart) new_page = table[pos[0] / BH_PAGE];
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p) q[r][p] = load4(t.q + ((size_t)(row0 + r) * t.H + head) * HD + 32 * p + 4 * dq);
+    }
+    last[r] = new_key_apart ? pos[r] - 1 : pos[r];
     first[r] = bh_first_visible(pos[r], t.window);
     scale[r] = query_scale(t.form, pos[r]);
     from = min(from, first[r]);
-    upto = max(upto, pos[r]);
+    upto = max(upto, last[r]);
+  }
+  const int last_part = upto >= 0 ? upto / TOKENS : -1;
+  bool ready = !FUSED;      // the query is what the scores are made with
+  auto finish_q = [&]() {
+    if constexpr (FUSED) {
+      if (ready) return;
+      ready = true;
+      q_turn.apply(q[0], t.fused, q_turn);
+    }
+  };
+  if constexpr (FUSED) {
+    if (takes_new_key) {      // before this wave's pages, if it has any: beside them there are not the registers
+      finish_q();
+      k_turn.apply(new_key, t.fused, q_turn);
+      float dot = 0.f;
 #pragma unroll
-    for (int p = 0; p < P; ++p) q[r][p] = load4(t.q + ((size_t)(row0 + r) * t.H + head) * HD + 32 * p + 4 * dq);
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dot = fmaf(q[0][p][e], new_key[p][e], dot);
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) dot += __shfl_xor(dot, off, BH_WAVE);
+      if (lane == 0) lds.new_score = dot * scale[0];
+      if (head % (t.H / t.KVH) == 0 && kl == 0) {
+        float* to = t.fused.k_pages + (((size_t)new_page * t.KVH + kv_head) * BH_PAGE + pos[0] % BH_PAGE) * HD + 4 * dq;
+#pragma unroll
+        for (int p = 0; p < P; ++p) *reinterpret_cast<floatx4*>(to + 32 * p) = new_key[p];
+      }
+    }
   }
 
-  float most[NR], sum[NR], acc[NR][8 * P];
+  float most[NR], sum[NR], acc[NR][ND];
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     most[r] = -INFINITY;
     sum[r] = 0.f;
 #pragma unroll
-    for (int d = 0; d < 8 * P; ++d) acc[r][d] = 0.f;
+    for (int d = 0; d < ND; ++d) acc[r][d] = 0.f;
   }
-  for (int page = from / BH_PAGE + wave; page <= upto / BH_PAGE; page += WAVES) {
-    const size_t block = ((size_t)table[page] * t.KVH + kv_head) * BH_PAGE * HD;
-    const float* keys = t.k_pages + block + kl * HD + 4 * dq;
-    const float* values = t.v_pages + block + dl * BH_PAGE + 4 * tq;
-    float s[NR][8];
-    floatx4 ahead[AHEAD ? 8 * P : 1];
+  for (int part = from / TOKENS + wave; part <= last_part; part += WAVES) {
+    const int page = part / PARTS, token0 = part % PARTS * TOKENS, at0 = part * TOKENS;      // its tokens in the page, and in the sequence
+    const size_t block = ((size_t)(FUSED && part == wave ? page_guess : table[page]) * t.KVH + kv_head) * BH_PAGE * HD;
+    const float* keys = t.k_pages + block + (token0 + kl) * HD + 4 * dq;
+    const float* values = t.v_pages + block + dl * BH_PAGE + token0 + 4 * tq;
+    float s[NR][GROUPS];
+    floatx4 ahead[AHEAD ? ND : 1];
     if constexpr (AHEAD) {
       // one row and a page or two a wave: the page's way from memory is the time, so all of it is asked for at once
-      floatx4 k[8][P];
+      floatx4 k[GROUPS][P];
 #pragma unroll
-      for (int g = 0; g < 8; ++g)
+      for (int g = 0; g < GROUPS; ++g)
 #pragma unroll
         for (int p = 0; p < P; ++p) k[g][p] = load4(keys + 8 * g * HD + 32 * p);
 #pragma unroll
-      for (int d = 0; d < 8 * P; ++d) ahead[d] = load4(values + 4 * d * BH_PAGE);
+      for (int d = 0; d < ND; ++d) ahead[d] = load4(values + DL * d * BH_PAGE);
       __builtin_amdgcn_sched_barrier(0);
+      finish_q();
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
+      for (int g = 0; g < GROUPS; ++g) {
         float dot = 0.f;
 #pragma unroll
         for (int p = 0; p < P; ++p)
@@ -102,8 +223,9 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
         s[0][g] = dot;
       }
     } else {
+      finish_q();
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
+      for (int g = 0; g < GROUPS; ++g) {
         floatx4 k[P];
 #pragma unroll
         for (int p = 0; p < P; ++p) k[p] = load4(keys + 8 * g * HD + 32 * p);
@@ -118,27 +240,28 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
         }
       }
     }
-    const int token = 8 * dq + kl, at = page * BH_PAGE + token;
+    const int token = PARTS == 1 ? 8 * dq + kl : 8 * (dq >> 1) + kl, at = at0 + token;
     float alpha[NR];
     floatx4 w[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
 #pragma unroll
-      for (int half = 4; half > 0; half >>= 1) {
-        const bool upper = dq & half;
+      for (int half = GROUPS / 2; half > 0; half >>= 1) {
+        const bool upper = dq & (half * PARTS);
 #pragma unroll
         for (int g = 0; g < half; ++g)
-          s[r][g] = (upper ? s[r][g + half] : s[r][g]) + __shfl_xor(upper ? s[r][g] : s[r][g + half], half, BH_WAVE);
+          s[r][g] = (upper ? s[r][g + half] : s[r][g]) + __shfl_xor(upper ? s[r][g] : s[r][g + half], half * PARTS, BH_WAVE);
       }
+      if (PARTS == 2) s[r][0] += __shfl_xor(s[r][0], 1, BH_WAVE);      // (two lanes then have the same key)
       float score = s[r][0] * scale[r];
       if (t.form.cap > 0.f) score = t.form.cap * tanhf(score / t.form.cap);
       score -= slope * (float)(pos[r] - at);
-      const bool seen = at >= first[r] && at <= pos[r];
+      const bool seen = at >= first[r] && at <= last[r];
       score = seen ? score : -INFINITY;
       const float now = fmaxf(most[r], wave_max(score));
       const float p = score == -INFINITY ? 0.f : expf(score - now);      // also where a seen key's score is: a page of those has now -inf
       alpha[r] = most[r] == -INFINITY ? 0.f : expf(most[r] - now);
-      sum[r] = sum[r] * alpha[r] + p;
+      sum[r] = sum[r] * alpha[r] + (PARTS == 2 && (dq & 1) ? 0.f : p);
       most[r] = now;
       lds.probs[wave][r][token] = p;
     }
@@ -149,17 +272,17 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
     for (int r = 0; r < NR; ++r) {
       w[r] = load4(&lds.probs[wave][r][4 * tq]);
 #pragma unroll
-      for (int d = 0; d < 8 * P; ++d) acc[r][d] *= alpha[r];
+      for (int d = 0; d < ND; ++d) acc[r][d] *= alpha[r];
     }
     // a key that a row does not see may hold anything (behind a sequence's end, or a later row's): it must not reach that row's
     // sums, not even times zero
     bool whole = true;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) whole = whole && first[r] <= page * BH_PAGE && pos[r] >= page * BH_PAGE + BH_PAGE - 1;
+    for (int r = 0; r < NR; ++r) whole = whole && first[r] <= at0 && last[r] >= at0 + TOKENS - 1;
     if (whole) {
 #pragma unroll
-      for (int d = 0; d < 8 * P; ++d) {
-        const floatx4 v = AHEAD ? ahead[AHEAD ? d : 0] : load4(values + 4 * d * BH_PAGE);
+      for (int d = 0; d < ND; ++d) {
+        const floatx4 v = AHEAD ? ahead[AHEAD ? d : 0] : load4(values + DL * d * BH_PAGE);
 #pragma unroll
         for (int r = 0; r < NR; ++r)
 #pragma unroll
@@ -167,26 +290,28 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
       }
     } else {
 #pragma unroll
-      for (int d = 0; d < 8 * P; ++d) {
-        const floatx4 v = AHEAD ? ahead[AHEAD ? d : 0] : load4(values + 4 * d * BH_PAGE);
+      for (int d = 0; d < ND; ++d) {
+        const floatx4 v = AHEAD ? ahead[AHEAD ? d : 0] : load4(values + DL * d * BH_PAGE);
 #pragma unroll
         for (int r = 0; r < NR; ++r)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int j = page * BH_PAGE + 4 * tq + e;
-            acc[r][d] = fmaf(w[r][e], j >= first[r] && j <= pos[r] ? v[e] : 0.f, acc[r][d]);
+            const int j = at0 + 4 * tq + e;
+            acc[r][d] = fmaf(w[r][e], j >= first[r] && j <= last[r] ? v[e] : 0.f, acc[r][d]);
           }
       }
     }
     __builtin_amdgcn_wave_barrier();
   }
+  finish_q();      // (a wave without a page)
 
-  // over the 16 lanes of a dimension: three halvings leave lane tq with P dimensions' sums over eight lanes, then its neighbour's
+  // over the lanes of a dimension: three halvings (two, of the eight lanes of half a page) leave lane tq with P dimensions' sums over half
+  // of the lanes, then its neighbour's
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
 #pragma unroll
-    for (int step = 0; step < 3; ++step) {
-      const int half = 4 * P >> step, bit = 8 >> step;
+    for (int step = 0; step < (PARTS == 1 ? 3 : 2); ++step) {
+      const int half = ND / 2 >> step, bit = TQ / 2 >> step;
       const bool upper = tq & bit;
 #pragma unroll
       for (int d = 0; d < half; ++d)
@@ -195,7 +320,7 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
 #pragma unroll
     for (int d = 0; d < P; ++d) {
       const float whole = acc[r][d] + __shfl_xor(acc[r][d], 1, BH_WAVE);
-      if ((tq & 1) == 0) lds.o[wave][r][4 * ((tq >> 1) * P + d) + dl] = whole;
+      if ((tq & 1) == 0) lds.o[wave][r][DL * ((tq >> 1) * P + d) + dl] = whole;
     }
     const float all = wave_sum(sum[r]);
     if (lane == 0) {
@@ -203,13 +328,32 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
       lds.sum[wave][r] = all;
     }
   }
+  constexpr int EACH = (NR * HD + 64 * WAVES - 1) / (64 * WAVES);      // elements that a thread merges
+  float new_value[EACH];
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) {
+      const int e = tid + u * 64 * WAVES;
+      new_value[u] = e < HD ? t.fused.qkv[((size_t)row0 * (t.H + 2 * t.KVH) + t.H + t.KVH + kv_head) * HD + e] : 0.f;
+    }
+  }
   __syncthreads();
-  for (int e = tid; e < NR * HD; e += 64 * WAVES) {
-    const int r = e / HD, d = e % HD;
+  const float new_score = new_key_apart ? lds.new_score : -INFINITY;
+#pragma unroll
+  for (int u = 0; u < EACH; ++u) {
+    const int e = tid + u * 64 * WAVES, r = e / HD, d = e % HD;
+    if (e >= NR * HD) break;
     float top = lds.most[0][r];
 #pragma unroll
     for (int s = 1; s < WAVES; ++s) top = fmaxf(top, lds.most[s][r]);
     float total = 0.f, all = 0.f;
+    if constexpr (FUSED) {
+      if (new_key_apart) {
+        top = fmaxf(top, new_score);
+        all = new_score == -INFINITY ? 0.f : expf(new_score - top);
+        total = new_value[u] * all;
+      }
+    }
 #pragma unroll
     for (int s = 0; s < WAVES; ++s) {
       const float share = lds.most[s][r] == -INFINITY ? 0.f : expf(lds.most[s][r] - top);
@@ -221,14 +365,27 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
     const int row = row0 + r;
     t.out[((size_t)row * t.H + head) * HD + d] = total / all * head_gate<float>(t.finish, row, head);
   }
+  if constexpr (FUSED) {
+    if (new_key_apart && head % (t.H / t.KVH) == 0) {
+      const size_t block = ((size_t)new_page * t.KVH + kv_head) * BH_PAGE * HD;
+      const int token = pos[0] % BH_PAGE;
+#pragma unroll
+      for (int u = 0; u < EACH; ++u) {
+        const int e = tid + u * 64 * WAVES;
+        if (e < HD) t.fused.v_pages[block + (size_t)e * BH_PAGE + token] = new_value[u];
+      }
+    }
+  }
 }
+
+constexpr int parts_of(int slices, int waves) { return slices >= 3 && waves == 8 ? 2 : 1; }
 
 template <int P, int NR, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(F32Attention t, int n_rows) {
   __shared__ __attribute__((aligned(16))) Lds<P, NR, WAVES> lds;
   const int row0 = blockIdx.x * NR, head = blockIdx.y;
   if constexpr (NR == 1) {
-    attend_rows<P, 1, WAVES>(t, lds, row0, head);
+    attend_rows<P, 1, WAVES, false, parts_of(P, WAVES)>(t, lds, row0, head);
   } else {
     bool together = row0 + NR <= n_rows;
     for (int r = 1; together && r < NR; ++r) together = t.row_seq[row0 + r] == t.row_seq[row0];
@@ -241,6 +398,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(F32Attention 
       __syncthreads();
     }
   }
+}
+
+template <int P, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attention_f32_fused_kernel(F32Attention t) {
+  __shared__ __attribute__((aligned(16))) Lds<P, 1, WAVES> lds;
+  attend_rows<P, 1, WAVES, true, parts_of(P, WAVES)>(t, lds, blockIdx.x, blockIdx.y);
 }
 
 // ---- prompts -------------------------------------------------------------------------------------------
@@ -456,6 +619,19 @@ bool tiles_pay(int n_rows, int n_seqs, int H, int KVH, int hd, int span, const i
   return 1.15 * in_tiles <= by_rows;
 }
 
+constexpr int many_waves(int slices) { return slices <= 4 ? 8 : 4; }
+
+// A decode step from its projection rows: as many waves a row and head as `launch` gives it.  In two launches / one, us, 8 rows of 100 keys,
+// 16 heads of 128 on 8 7.3 / 5.9, 4 rows of 300 keys, 4 heads of 64 on 2 7.5 / 5.6.
+template <int P>
+void launch_fused(const F32Attention& t, int n_rows, int most_pages, hipStream_t stream) {
+  const long units = bh_compute_units(), each = (long)n_rows * t.H;
+  const dim3 grid(n_rows, t.H);
+  if (most_pages <= 1 || (most_pages <= 4 && each >= 4 * units)) attention_f32_fused_kernel<P, 1><<<grid, 64, 0, stream>>>(t);
+  else if (each < 2 * units) attention_f32_fused_kernel<P, many_waves(P)><<<grid, 64 * many_waves(P), 0, stream>>>(t);
+  else attention_f32_fused_kernel<P, 4><<<grid, 256, 0, stream>>>(t);
+}
+
 template <int P>
 void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, bool tiled, hipStream_t stream) {
   constexpr int NR = P <= 4 ? 4 : P <= 7 ? 2 : 1;      // what the registers hold without spilling
@@ -481,7 +657,7 @@ void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, bool 
   }
   // Prompts: rows of one sequence share the pages' reads.  Else a row a workgroup, of eight waves where the rows and heads alone
   // leave compute units idle and the registers allow it: as many pages are then on their way together.
-  constexpr int MANY = P <= 3 ? 8 : 4;
+  constexpr int MANY = many_waves(P);
   if (prompts) attention_f32_kernel<P, NR, 4><<<dim3((n_rows + NR - 1) / NR, t.H), 256, 0, stream>>>(t, n_rows);
   else if ((long)n_rows * t.H < 2 * bh_compute_units())
     attention_f32_kernel<P, 1, MANY><<<dim3(n_rows, t.H), 64 * MANY, 0, stream>>>(t, n_rows);
@@ -512,7 +688,7 @@ extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages
   const ScoreForm form = {scale, cap, slopes, temp_coef, temp_every};
   if (const char* fault = bh_score_form_fault(form)) return bh_fail("attention: %s", fault);
   const F32Attention t = {q, out, k_pages, v_pages, page_table, table_stride, row_seq, positions, H, KVH, form, window,
-                          {sinks, gates, gate_stride, out_scale}};
+                          {sinks, gates, gate_stride, out_scale}, {}};
   const bool tiled = tiles_pay(n_rows, n_seqs, H, KVH, hd, window, host_start, host_past);
   switch (hd / 32) {
     case 1: launch<1>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
@@ -525,4 +701,38 @@ extern "C" int bh_attention_f32(const float* q, float* out, const float* k_pages
     default: launch<8>(t, n_rows, n_seqs, most_pages, tiled, stream); break;
   }
   return bh_check_launch("attention_f32");
+}
+
+// A decode step (row s is sequence s's) from its fused projection rows [q heads | k heads | v heads]: per-head RMSNorm of q and k (weights
+// may be null), rotation over the whole head at the row's position (tables may be null), the new key and value into the cache (unless
+// write_kv is 0: the entry is another layer's), and attention over the cache and the new key.  `most_pages` as above.
+extern "C" int bh_attention_f32_decode_fused(const float* qkv, float* out, float* k_pages, float* v_pages, const int32_t* page_table,
+                                             int table_stride, const int32_t* positions, int n_rows, int H, int KVH, int hd, float scale,
+                                             int window, int max_position, int most_pages, const float* q_weight, const float* k_weight, float eps,
+                                             const float* cos_table, const float* sin_table, int table_positions, int rot, int write_kv,
+                                             hipStream_t stream) {
+  BH_REQUIRE(n_rows > 0 && H > 0 && KVH > 0 && hd > 0 && max_position >= 0, "attention_decode_fused: sizes must be positive");
+  BH_REQUIRE(bh_attention_f32_takes(H, KVH, hd, BH_KV_ROWS), "attention_decode_fused: %d heads of %d on %d are not for the float32 kernel", H, hd, KVH);
+  BH_REQUIRE((((uintptr_t)qkv | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)cos_table |
+               (uintptr_t)sin_table) % 16) == 0, "attention_decode_fused: rows, cache, weights and tables must be 16-byte aligned");
+  BH_REQUIRE((q_weight == nullptr) == (k_weight == nullptr), "attention_decode_fused: give both norm weights or neither");
+  BH_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "attention_decode_fused: cos and sin tables come together");
+  BH_REQUIRE(cos_table == nullptr || (rot == hd && hd % 64 == 0),
+             "attention_decode_fused: the rotation must span the whole head (%d of %d) and the head be a multiple of 64", rot, hd);
+  BH_REQUIRE(cos_table == nullptr || max_position < table_positions,
+             "attention_decode_fused: position %d is outside the rotation table of %d positions", max_position, table_positions);
+  const F32Attention t = {nullptr, out, k_pages, v_pages, page_table, table_stride, nullptr, positions, H, KVH,
+                          ScoreForm{scale, 0.f, nullptr, 0.f, 0}, window, HeadEnd{},
+                          {qkv, q_weight, k_weight, eps, cos_table, sin_table, write_kv, k_pages, v_pages}};
+  switch (hd / 32) {
+    case 1: launch_fused<1>(t, n_rows, most_pages, stream); break;
+    case 2: launch_fused<2>(t, n_rows, most_pages, stream); break;
+    case 3: launch_fused<3>(t, n_rows, most_pages, stream); break;
+    case 4: launch_fused<4>(t, n_rows, most_pages, stream); break;
+    case 5: launch_fused<5>(t, n_rows, most_pages, stream); break;
+    case 6: launch_fused<6>(t, n_rows, most_pages, stream); break;
+    case 7: launch_fused<7>(t, n_rows, most_pages, stream); break;
+    default: launch_fused<8>(t, n_rows, most_pages, stream); break;
+  }
+  return bh_check_launch("attention_f32_decode_fused");
 }

@@ -148,6 +148,7 @@ class KernelSizes:
             "bh_attention_generic": [p, p, i, p, p, p, i, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32": [p, p, p, p, p, i, i, i, p, p, p, p, i, i, i, i, f, i, i, p, p, i, f, p, f, i, f, p],
             "bh_attention_f32_takes": [i, i, i, i],
+            "bh_attention_f32_decode_fused": [p, p, p, p, p, i, p, i, i, i, i, f, i, i, i, p, p, f, p, p, i, i, i, p],
             "bh_attention_f32_tiles": [i, i, i, i, i, i, p, p],
             "bh_gemm_f32_takes_gated": [i, i, i],
             "bh_gemm_f32_gated": [p, p, p, i, i, i, i, p],
@@ -1003,11 +1004,16 @@ class HipKernels(KernelSizes):
         (then call the two)."""
         n_rows = qkv.shape[0]
         rot = 2 * cos.shape[1] if cos is not None else 0
-        if (qkv.dtype != torch.bfloat16 or k_pages.dtype != torch.bfloat16 or layout is None
-                or int(layout.max_rows_per_seq) != 1 or int(layout.n_seqs) != n_rows
-                or head_dim % 32 or head_dim > 256 or n_heads % n_kv_heads or n_heads // n_kv_heads > 16
-                or (cos is not None and (rot != head_dim or head_dim % 64)) or not scale > 0.0
-                or self.kv_order(k_pages.dtype, head_dim) != 1):
+        if (k_pages.dtype != qkv.dtype or layout is None or int(layout.max_rows_per_seq) != 1 or int(layout.n_seqs) != n_rows
+                or (cos is not None and (rot != head_dim or head_dim % 64))):
+            return False
+        if qkv.dtype == torch.float32:      # the two launches take what this one does not
+            if (isinstance(out, BlockedRows) or not self.lib.bh_attention_f32_takes(n_heads, n_kv_heads, head_dim, self.kv_order(k_pages.dtype, head_dim))
+                    or any(w is not None and w.dtype != torch.float32 for w in (q_weight, k_weight))
+                    or any(t is not None and t.data_ptr() % 16 for t in (qkv, k_pages, v_pages, q_weight, k_weight, cos, sin))):
+                return False
+        elif (qkv.dtype != torch.bfloat16 or head_dim % 32 or head_dim > 256 or n_heads % n_kv_heads or n_heads // n_kv_heads > 16
+                or not scale > 0.0 or self.kv_order(k_pages.dtype, head_dim) != 1):
             return False
         if qkv.shape != (n_rows, (n_heads + 2 * n_kv_heads) * head_dim) or tuple(out.shape) != (n_rows, n_heads * head_dim) \
                 or out.dtype != qkv.dtype:
@@ -1025,6 +1031,15 @@ class HipKernels(KernelSizes):
         if cos is not None and (cos.shape != sin.shape or cos.dim() != 2):
             raise KernelError("attention_decode_fused: cos and sin tables must be matrices of one shape")
         self._check_pages(k_pages, v_pages, page_table, n_kv_heads, head_dim, qkv.dtype, "attention_decode_fused")
+        if qkv.dtype == torch.float32:
+            self._check(self.lib.bh_attention_f32_decode_fused(
+                self._ptr(qkv, "qkv"), self._ptr(out, "attention out"), self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
+                self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1], self._ptr(positions, "positions", (torch.int32,)),
+                n_rows, n_heads, n_kv_heads, head_dim, float(scale), int(window), int(layout.max_position),
+                self.furthest(layout.max_position, window) // self.page_size + 1, self._ptr(q_weight, "q_norm", None, True),
+                self._ptr(k_weight, "k_norm", None, True), float(eps), self._ptr(cos, "cos", (torch.float32,), True),
+                self._ptr(sin, "sin", (torch.float32,), True), cos.shape[0] if cos is not None else 0, rot, int(bool(write_kv)), self._stream()))
+            return True
         n_splits = int(self.lib.bh_attention_bf16_splits(n_rows, 1, n_heads, n_kv_heads, int(layout.max_position)))
         part_o = part_ml = None
         if n_splits > 1:
