@@ -9,7 +9,11 @@ kernel library's: the kernel that writes them and the attention kernels agree on
 cache itself never looks inside); a sequence's position p lives in page `table[p // page_size]`
 at token `p % page_size`, and a
 group with a window gives pages back once every position in them has left the window.  A
-state group holds [entries, max_slots, *shape] and a slot's rows are zero when it starts.
+state group holds [entries, max_slots, *shape] and a slot's rows are zero when it starts; or, *in banks*,
+[entries, 2 max_slots, *shape], two rows a slot of which one holds its state: a step reads that one and leaves the
+state in the other, and the commit says that the other holds it now.  Where layers cannot do that, or two runs of a
+step share an entry, the state is moved on in place and a step starts with a copy of its slots' rows (16 slots of 6
+layers of 2 MB: 75 us of a decode step of 990).
 
 Rules kept from the reference's single-sequence caches: a step first *reserves* room for all
 its new tokens or changes nothing (append refuses without mutating,
@@ -49,6 +53,7 @@ class GroupPlan:
     entries: list
     kv_bytes: int
     state_bytes: int
+    banked: bool = False      # two rows a slot, both in state_bytes
 
 
 @dataclass
@@ -83,6 +88,7 @@ class _Group:
         self.entries = list(entries)
         self.index_of = {entry: i for i, entry in enumerate(self.entries)}
         self.k = self.v = self.state = None
+        self.banked = False
         self.free_pages: list = []
         self.pages_of: dict = {}     # slot -> list of page ids (or -1 once released), position order
 
@@ -92,7 +98,8 @@ _MOST_SLOTS = 1 << 20     # every slot has a place in the free list and a row in
 
 class SequenceCache:
     def __init__(self, entry_needs: dict, max_tokens: int, dtype: torch.dtype, device, page_size: int,
-                 max_slots: int | None = None, max_position: int | None = None):
+                 max_slots: int | None = None, max_position: int | None = None, banks=()):
+        """`banks`: the entries whose state may stand in two rows a slot, if their layers say that they can (`CacheNeed.in_banks`)."""
         for name, value, optional in (("max_tokens", max_tokens, False), ("max_slots", max_slots, True),
                                       ("max_position", max_position, True)):
             if value is None and optional:
@@ -112,10 +119,13 @@ class SequenceCache:
         for entry in sorted(entry_needs):
             by_need.setdefault(entry_needs[entry], []).append(entry)
         self.groups = [_Group(need, entries) for need, entries in by_need.items()]
+        for g in self.groups:
+            g.banked = bool(g.need.in_banks and g.need.state_shape and all(entry in banks for entry in g.entries))
         self.group_of_entry = {entry: g for g in self.groups for entry in g.entries}
         self._free_slots = list(range(self.max_slots))
         heapq.heapify(self._free_slots)
         self._length: dict = {}      # live slot -> committed length
+        self._bank: dict = {}        # live slot -> which of its two rows holds its state, 0 or 1
         self._allocated = False
         self._slot_indices: dict = {}    # slots of a step, in order -> the same as a device tensor (a batch that is decoded repeats them)
         self._state_before: list = []    # (state, slot indices or None where it is the slots' own slice, its rows) before the running step
@@ -132,9 +142,12 @@ class SequenceCache:
                 count = 1
                 for axis in g.need.state_shape:
                     count *= axis
-                state = len(g.entries) * self.max_slots * count * _element_size(g.need.state_dtype)
-            plan.groups.append(GroupPlan(g.need, g.entries, kv, state))
+                state = len(g.entries) * self._rows(g) * count * _element_size(g.need.state_dtype)
+            plan.groups.append(GroupPlan(g.need, g.entries, kv, state, g.banked))
         return plan
+
+    def _rows(self, g) -> int:
+        return (2 if g.banked else 1) * self.max_slots
 
     def allocate(self, limit_bytes: int | None = None) -> CachePlan:
         plan = self.plan()
@@ -148,7 +161,7 @@ class SequenceCache:
                 g.v = torch.zeros((*head, g.need.head_dim, self.page_size), dtype=self.dtype, device=self.device)
                 g.free_pages = list(range(self.n_pages - 1, -1, -1))   # pop() hands out page 0 first
             if g.need.state_shape:
-                g.state = torch.zeros((len(g.entries), self.max_slots, *g.need.state_shape),
+                g.state = torch.zeros((len(g.entries), self._rows(g), *g.need.state_shape),
                                       dtype=g.need.state_dtype, device=self.device)
         self._allocated = True
         return plan
@@ -166,7 +179,7 @@ class SequenceCache:
         if not self._free_slots:
             raise CacheFull(f"all {self.max_slots} sequence slots are in use")
         slot = heapq.heappop(self._free_slots)
-        self._length[slot] = 0
+        self._length[slot] = self._bank[slot] = 0
         for g in self.groups:
             if g.need.kind == "kv":
                 g.pages_of[slot] = []
@@ -177,7 +190,7 @@ class SequenceCache:
     def free_slot(self, slot: int) -> None:
         if slot not in self._length:
             raise CacheError(f"slot {slot} is not in use (freed twice, or never given out)")
-        del self._length[slot]
+        del self._length[slot], self._bank[slot]
         for g in self.groups:
             if g.need.kind == "kv":
                 for page in g.pages_of.pop(slot):
@@ -228,14 +241,14 @@ class SequenceCache:
                 pages = g.pages_of[slot]
                 while len(pages) * self.page_size < self._length[slot] + n_new:
                     pages.append(g.free_pages.pop())
-        # State regions are updated in place while the step runs; keep what the step's slots held, so that a
+        # State regions that are not in banks are updated in place while the step runs; keep what the step's slots held, so that a
         # failed step can put it back (the key/value pages need no such copy: rows beyond a sequence's length are
         # never read).  Slots in a row, as a batch that started together has them, are copied as a slice of the state,
         # whose rows are whole and in order: 16 slots of 6 layers of 2 MB in 75 us where the gather by indices takes 118.
         self._state_before = []
         slots = tuple(slot for slot, _ in requests)
         for g in self.groups:
-            if g.state is None:
+            if g.state is None or g.banked:
                 continue
             first = slots[0] if slots else 0
             if slots == tuple(range(first, first + len(slots))):
@@ -259,6 +272,7 @@ class SequenceCache:
         self._state_before = []
         for slot, n_new in requests:
             self._length[slot] += n_new
+            self._bank[slot] ^= 1
         for g in self.groups:
             if g.need.kind != "kv" or not g.need.window:
                 continue
@@ -311,6 +325,11 @@ class SequenceCache:
             out[row, :] = 0
             out[row, :len(pages)] = [max(page, 0) for page in pages]
 
+    def state_rows(self, slots: list):
+        """([row that holds each slot's state], [row in which a step leaves it]) of the groups in banks."""
+        held = [slot + self.max_slots * self._bank[slot] for slot in slots]
+        return held, [2 * slot + self.max_slots - row for slot, row in zip(slots, held)]
+
     def page_tables(self, slots: list, min_width: int = 1) -> dict:
         """For each key/value group, an int32 device tensor [len(slots), width] of page ids."""
         import numpy as np
@@ -328,8 +347,8 @@ class SequenceCache:
         at = g.index_of[entry]
         if g.need.kind == "kv":
             return LayerCache(g.need, writes, k_pages=g.k[at], v_pages=g.v[at], page_table=tables[self.groups.index(g)],
-                              state=g.state[at] if g.state is not None else None)
-        return LayerCache(g.need, writes, state=g.state[at])
+                              state=g.state[at] if g.state is not None else None, banked=g.banked)
+        return LayerCache(g.need, writes, state=g.state[at], banked=g.banked)
 
     # ---- self-check, for tests ----
     def check_invariants(self) -> None:

@@ -128,7 +128,7 @@ def _generate(args: list, out) -> int:
 
         from .cache import SequenceCache
         from .engine import open_model, parse_dtype
-        from .engine.engine import GRAPH_LIMIT
+        from .engine.engine import GRAPH_LIMIT, entries_of_one_run
         from .engine.memory import plan_memory
         from .kernels import KernelSizes
 
@@ -138,7 +138,7 @@ def _generate(args: list, out) -> int:
         finally:
             weights.reader.close()
         cache = SequenceCache(model.entry_needs, max_tokens, parse_dtype(dtype), "cpu", page, max_slots=slots,
-                              max_position=model.max_position)
+                              max_position=model.max_position, banks=entries_of_one_run(model))
         capacity = cache.n_pages * cache.page_size
         # the kernel library's own account of what its calls allocate: host code, no GPU is touched
         plan = plan_memory(model, weight_bytes, cache.plan(), 2 if parse_dtype(dtype) == torch.bfloat16 else 4,

@@ -180,7 +180,7 @@ __global__ __launch_bounds__(512) void scan_states_kernel(In in, const int32_t* 
 
 // grid (sequences, heads, elements / 1024)
 template <int UNUSED = 0>
-__global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+__global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                                            int place0, int places, float* __restrict__ states,
                                                            const float* __restrict__ factors, float* __restrict__ home, long slot_stride,
                                                            int H, int D, int V) {
@@ -192,7 +192,9 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __rest
   if (from >= upto) return;
   // the thread's four elements of a tile (ds_tile) in the sequence's region, which lies by rows
   const int tile = e / 256, lane = e % 256 / 4, d = tile % (D / 16) * 16 + lane / 16 * 4, v = tile / (D / 16) * 16 + lane % 16;
-  float* mine = home + (size_t)seq_slot[seq] * slot_stride + (size_t)head * size + (size_t)d * V + v;
+  float* left = home + (size_t)seq_to[seq] * slot_stride + (size_t)head * size + (size_t)d * V + v;
+  // (a launch that goes on with a sequence goes on from what the one before left)
+  const float* mine = from > 0 ? left : home + (size_t)seq_slot[seq] * slot_stride + (size_t)head * size + (size_t)d * V + v;
   const size_t apart = (size_t)H * size;
   float* z = states + ((size_t)(base + from - place0) * H + head) * size + e;
   const float* f = factors + (size_t)(base + from - place0) * H + head;
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(const int32_t* __rest
         state.w = fmaf(factor[side][u], state.w, own[side][u].w);
       }
     }
-  mine[0] = state.x, mine[V] = state.y, mine[2 * V] = state.z, mine[3 * V] = state.w;
+  left[0] = state.x, left[V] = state.y, left[2 * V] = state.z, left[3 * V] = state.w;
 }
 
 template <class In, bool WIDE>
@@ -448,7 +450,7 @@ inline long ds_scratch_floats(int n_seqs, int n_rows, int H, int D, int V) {
 }
 
 template <class In, bool WIDE>
-int ds_launch_as(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
+int ds_launch_as(const In& in, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* home, long slot_stride, float* out, float* scratch,
               long scratch_floats, int n_seqs, int n_rows, int H, int D, int V, hipStream_t stream) {
   const long one = (long)H * ((long)D * V + 1), places = ds_places(n_seqs, n_rows);
   const int window = (int)(scratch_floats / one < places ? scratch_floats / one : places);
@@ -462,7 +464,7 @@ int ds_launch_as(const In& in, const int32_t* seq_start, const int32_t* seq_slot
     const int here = (int)(places - place < window ? places - place : window);
     scan_states_kernel<In, WIDE><<<ds_grid(here, H, in.shared()), 512, states_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, factors, H, D, V);
     if (int status = bh_check_launch("scan_states")) return status;
-    scan_combine_kernel<0><<<dim3(n_seqs, H, (D * V + 1023) / 1024), 256, 0, stream>>>(seq_start, seq_slot, (int)place, here, scratch, factors, home,
+    scan_combine_kernel<0><<<dim3(n_seqs, H, (D * V + 1023) / 1024), 256, 0, stream>>>(seq_start, seq_slot, seq_to, (int)place, here, scratch, factors, home,
                                                                                      slot_stride, H, D, V);
     if (int status = bh_check_launch("scan_combine")) return status;
     scan_outputs_kernel<In, WIDE><<<ds_grid(here, H, in.shared()), 512, outputs_lds, stream>>>(in, seq_start, n_seqs, (int)place, here, scratch, out, H, D, V);
@@ -472,9 +474,9 @@ int ds_launch_as(const In& in, const int32_t* seq_start, const int32_t* seq_slot
 }
 
 template <class In>
-int ds_launch(const In& in, const int32_t* seq_start, const int32_t* seq_slot, float* home, long slot_stride, float* out, float* scratch,
+int ds_launch(const In& in, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* home, long slot_stride, float* out, float* scratch,
               long scratch_floats, int n_seqs, int n_rows, int H, int D, int V, hipStream_t stream) {
   return D > 128 || V > 128
-             ? ds_launch_as<In, true>(in, seq_start, seq_slot, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream)
-             : ds_launch_as<In, false>(in, seq_start, seq_slot, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream);
+             ? ds_launch_as<In, true>(in, seq_start, seq_slot, seq_to, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream)
+             : ds_launch_as<In, false>(in, seq_start, seq_slot, seq_to, home, slot_stride, out, scratch, scratch_floats, n_seqs, n_rows, H, D, V, stream);
 }

@@ -4,7 +4,8 @@
 //   beta = sigmoid(b),  g = exp(-exp(A_log) softplus(a + dt_bias))        one of each a head
 //   S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q        (the read-out sees the token's own write)
 //   delta_prep   convolution, activation, unit lengths, beta, g and k.q of every row
-//   delta_scan   the recurrence over a sequence's rows of the step in order, from the state of the sequence's slot, which it moves on
+//   delta_scan   the recurrence over a sequence's rows of the step in order, from the state in row seq_slot, which it moves on into row
+//                seq_to (the same one, or one that no sequence of the step starts from)
 //   delta_step   all of it, the heads' norm and gate too, for a step of one row a sequence (a decode step), one launch
 // A slot's state: H states [dim][vdim], then the last taps - 1 projected rows of (q | k | v), oldest first.  Everything is float32 but the
 // projected rows, which come in the activation type.
@@ -263,7 +264,7 @@ template <int R, int SL, int C>
 __global__ __launch_bounds__(DR_WAVES * BH_WAVE) void delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ beside,
                                                                         float* __restrict__ state, long slot_stride,
                                                                         const int32_t* __restrict__ seq_start,
-                                                                        const int32_t* __restrict__ seq_slot, float* __restrict__ out, int H, int G,
+                                                                        const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, float* __restrict__ out, int H, int G,
                                                                         int dim, int vdim, DeltaChunks chunks) {
   constexpr int DP = R * SL, PER_WAVE = BH_WAVE / SL * C, COLS = DR_WAVES * PER_WAVE;
   constexpr int KQ = DR_STAGE * DP / 4;                              // 16-byte pieces of a stage's keys (and of its queries)
@@ -284,9 +285,9 @@ __global__ __launch_bounds__(DR_WAVES * BH_WAVE) void delta_scan_kernel(const fl
   const int local = threadIdx.x / BH_WAVE * PER_WAVE + lane / SL * C, column0 = tile0 + local;
   const int channels = 2 * G * dim + H * vdim, group = head / (H / G);
   const size_t head_state = (size_t)head * dim * vdim;
-  float* slot = state + (size_t)seq_slot[seq] * slot_stride + head_state;
+  const float* slot = state + (size_t)seq_slot[seq] * slot_stride + head_state;
   const size_t place = (size_t)(seq * chunks.count + chunk) * H + head;
-  float* values_to = apart ? chunks.states + place * dim * vdim : slot;
+  float* values_to = apart ? chunks.states + place * dim * vdim : state + (size_t)seq_to[seq] * slot_stride + head_state;
   float* moves_to = apart ? chunks.moves + place * dim * dim : nullptr;
 
   float S[C][R];
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(DR_WAVES * BH_WAVE) void delta_scan_kernel(const fl
 #define DC_STRIDE 20
 typedef float dr_f32x4_t __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void delta_combine_kernel(DeltaChunks chunks, float* __restrict__ state, long slot_stride,
-                                                            const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, int H,
+                                                            const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int H,
                                                             int dim, int vdim) {
   extern __shared__ float run[];           // [2][rows of 16-row tiles][DC_STRIDE]
   const int seq = blockIdx.x, head = blockIdx.y, v0 = blockIdx.z * DC_COLS;
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(256) void delta_combine_kernel(DeltaChunks chunks, 
     __syncthreads();
     now ^= 1;
   }
-  float* slot = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * dim * vdim + column;
+  float* slot = state + (size_t)seq_to[seq] * slot_stride + (size_t)head * dim * vdim + column;
   for (int d = threadIdx.x / 16; d < dim; d += 16)
     if (real) slot[(size_t)d * vdim] = run[now * half + d * DC_STRIDE + j];
 }
@@ -540,7 +541,7 @@ extern "C" int bh_delta_takes(int dim, int vdim) { return dim > 0 && dim <= 512 
 // that is less than max_rows (the rows of the longest sequence), scratch holds n_seqs * chunks * H * dim * (vdim + dim) +
 // n_rows * H * dim floats.
 extern "C" int bh_delta_scan(const float* qkv, const float* beside, float* state, long slot_stride, const int32_t* seq_start,
-                             const int32_t* seq_slot, float* out, int n_seqs, int H, int G, int dim, int vdim, int n_rows, int max_rows,
+                             const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_seqs, int H, int G, int dim, int vdim, int n_rows, int max_rows,
                              int chunk_rows, float* scratch, hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && H > 0 && G > 0 && dim > 0 && vdim > 0 && H % G == 0, "delta_scan: sizes must be positive, heads fall evenly to groups");
   BH_REQUIRE(bh_delta_takes(dim, vdim), "delta_scan: heads of %d key dimensions are above the limit of 512", dim);
@@ -560,7 +561,7 @@ extern "C" int bh_delta_scan(const float* qkv, const float* beside, float* state
   BH_REQUIRE((long)n_seqs * chunks.count < (1L << 31) && (most + columns - 1) / columns <= 65535, "delta_scan: too many chunks or columns");
   const dim3 grid(n_seqs * chunks.count, H, (most + columns - 1) / columns);
 #define BH_DR(R, SL, C)                                                                                                            \
-  delta_scan_kernel<R, SL, C><<<grid, DR_WAVES * BH_WAVE, 0, stream>>>(qkv, beside, state, slot_stride, seq_start, seq_slot, out, H, G, dim, \
+  delta_scan_kernel<R, SL, C><<<grid, DR_WAVES * BH_WAVE, 0, stream>>>(qkv, beside, state, slot_stride, seq_start, seq_slot, seq_to, out, H, G, dim, \
                                                                        vdim, chunks)
   if (dim <= 16) BH_DR(4, 4, 1);
   else if (dim <= 32) BH_DR(8, 4, 1);
@@ -573,7 +574,7 @@ extern "C" int bh_delta_scan(const float* qkv, const float* beside, float* state
   if (chunks.rows == 0) return 0;
   const size_t lds = (size_t)2 * ((dim + 15) / 16) * 16 * DC_STRIDE * sizeof(float);
   bh_allow_lds<delta_combine_kernel>(lds);
-  delta_combine_kernel<<<dim3(n_seqs, H, (vdim + DC_COLS - 1) / DC_COLS), 256, lds, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, H,
+  delta_combine_kernel<<<dim3(n_seqs, H, (vdim + DC_COLS - 1) / DC_COLS), 256, lds, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, seq_to, H,
                                                                                             dim, vdim);
   if (int status = bh_check_launch("delta_combine")) return status;
   return bh_chunk_carry(chunks.states, chunks.queries, chunks.rows, chunks.count, seq_start, out, n_seqs, H, dim, vdim, stream);
@@ -586,7 +587,7 @@ extern "C" int bh_delta_scan(const float* qkv, const float* beside, float* state
 // loads that were asked for before the convolutions; the slices' shares of S^T k and S^T q meet in LDS.
 template <typename T, int R, int TEAMS>
 __global__ __launch_bounds__(256 * TEAMS) void delta_step_kernel(const T* __restrict__ proj, DeltaRows in, int g_first,
-                                                                 const int32_t* __restrict__ seq_slot, const float* __restrict__ norm, float eps,
+                                                                 const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, const float* __restrict__ norm, float eps,
                                                                  T* __restrict__ out, int out_block_rows, int tiles) {
   extern __shared__ __align__(16) float lds[];
   const int H = in.H, G = in.G, dim = in.dim, vdim = in.vdim, per = H / G;
@@ -602,7 +603,8 @@ __global__ __launch_bounds__(256 * TEAMS) void delta_step_kernel(const T* __rest
   // (a wave's team, tile and slice are the same in all its lanes: the addresses of a state's rows stay out of the vector registers)
   const int lane = threadIdx.x % BH_WAVE, team_wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BH_WAVE), team = team_wave / 4, wave = team_wave % 4;
   const int column = (wave % tiles) * BH_WAVE + lane, slice = wave / tiles, d0 = slice * R;
-  float* slot = in.state + (size_t)seq_slot[seq] * in.slot_stride;
+  const float* slot = in.state + (size_t)seq_slot[seq] * in.slot_stride;
+  float* left = in.state + (size_t)seq_to[seq] * in.slot_stride;
   float S[R];
   auto load = [&](int i) {      // the state of the group's head i
     const float* from = slot + (size_t)(group * per + (i < per ? i : 0)) * dim * vdim;
@@ -616,7 +618,8 @@ __global__ __launch_bounds__(256 * TEAMS) void delta_step_kernel(const T* __rest
   load(team);
   // the convolutions, and the inputs they leave for the next step
   const int channels = in.channels(), mine = 2 * dim + per * vdim, keep = in.taps - 1;
-  float* old = slot + in.conv_offset;
+  const float* old = slot + in.conv_offset;
+  float* inputs = left + in.conv_offset;
   const T* x = proj + (size_t)row * in.row_stride;
   for (int e = threadIdx.x; e < mine; e += 256 * TEAMS) {
     const int c = e < dim ? group * dim + e : (e < 2 * dim ? (G + group) * dim + e - dim : 2 * G * dim + group * per * vdim + e - 2 * dim);
@@ -626,9 +629,9 @@ __global__ __launch_bounds__(256 * TEAMS) void delta_step_kernel(const T* __rest
     for (int j = 0; j < keep; ++j) {
       const float before = old[(size_t)j * channels + c];
       acc = fmaf(w[j], before, acc);
-      if (j > 0) old[(size_t)(j - 1) * channels + c] = before;
+      if (j > 0) inputs[(size_t)(j - 1) * channels + c] = before;
     }
-    if (keep > 0) old[(size_t)(keep - 1) * channels + c] = u;
+    if (keep > 0) inputs[(size_t)(keep - 1) * channels + c] = u;
     acc = dr_silu(fmaf(w[keep], u, acc));
     if (e < dim) q_s[e] = acc;
     else if (e < 2 * dim) k_s[e - dim] = acc;
@@ -685,7 +688,7 @@ __global__ __launch_bounds__(256 * TEAMS) void delta_step_kernel(const T* __rest
     sq *= q_scale;
     const float u = real ? beta * (v_s[i * vdim + column] - g * sk) : 0.f, o = real ? fmaf(kq, u, g * sq) : 0.f;
     const float ku = k_scale * u;
-    float* to = slot + (size_t)head * dim * vdim;
+    float* to = left + (size_t)head * dim * vdim;
     if (real) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -717,7 +720,7 @@ extern "C" int bh_delta_step_takes(int dim, int vdim) {
 // One row a sequence: proj [n_seqs][row_stride] (dtype) as for delta_prep, g from g_first; norm f32 [H * vdim]; out [n_seqs][H * vdim] (dtype; rows or
 // blocks of rows): the heads' read-outs over their root mean square, times norm, times silu(g).
 extern "C" int bh_delta_step(const void* proj, int dtype, int row_stride, int first, int g_first, int b_first, int a_first, const float* conv, int taps,
-                             float* state, long slot_stride, long conv_offset, const float* a_log, const float* dt_bias, const int32_t* seq_slot,
+                             float* state, long slot_stride, long conv_offset, const float* a_log, const float* dt_bias, const int32_t* seq_slot, const int32_t* seq_to,
                              const float* norm, float eps, void* out, int out_block_rows, int n_seqs, int H, int G, int dim, int vdim,
                              hipStream_t stream) {
   const DeltaRows in = {row_stride, first, b_first, a_first, conv, taps, state, slot_stride, conv_offset, a_log, dt_bias, H, G, dim, vdim};
@@ -734,7 +737,7 @@ extern "C" int bh_delta_step(const void* proj, int dtype, int row_stride, int fi
 #define BH_DS_ONE(T, RR, TEAMS)                                                                                                      \
   do {                                                                                                                               \
     bh_allow_lds<delta_step_kernel<T, RR, TEAMS>>(lds);                                                                              \
-    delta_step_kernel<T, RR, TEAMS><<<grid, 256 * TEAMS, lds, stream>>>((const T*)proj, in, g_first, seq_slot, norm, eps, (T*)out,   \
+    delta_step_kernel<T, RR, TEAMS><<<grid, 256 * TEAMS, lds, stream>>>((const T*)proj, in, g_first, seq_slot, seq_to, norm, eps, (T*)out,   \
                                                                         out_block_rows, tiles);                                      \
   } while (0)
 #define BH_DS(T, RR)                          \

@@ -3,8 +3,8 @@
 //   wkv (RWKV)               o_t = (S_(t-1) + diag(u) k_t v_t^T)^T r_t,   S_t = diag(a_t) S_(t-1) + k_t v_t^T,   a_t = exp(-exp(z_t + b)):
 //                            what a token reads are the tokens before it, and itself through the bonus u
 // (one a per key channel).
-//   gla_scan, wkv_scan   walk a sequence's rows of the step in order from the state that the sequence's slot holds and leave the
-//              state after the last row there; prompts, portions of prompts and decode steps are the same walk.
+//   gla_scan, wkv_scan   walk a sequence's rows of the step in order from the state in row seq_slot and leave the state after the
+//              last row in row seq_to (the same one, or one that no sequence of the step starts from); prompts, portions of prompts and decode steps are the same walk.
 // S is [dim][vdim] float32.  Decays (through the logarithm of the sigmoid, so that 1/tau is a factor), bonus, state, both
 // products and the read-out are float32; only q (r), k and v are read in the activations' type.
 #include "chunks.h"
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256, (R <= 16 ? 2 : 1)) void gla_scan_kernel(const 
                                                        const float* __restrict__ z, int z_stride, const float* __restrict__ bias,
                                                        float inv_tau, const float* __restrict__ bonus, float q_scale,
                                                        float* __restrict__ state, long slot_stride,
-                                                       const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                                       const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                                        float* __restrict__ out, int H, int dim, int vdim, int VT, GlaChunks chunks) {
   extern __shared__ __align__(16) float lds[];
   constexpr int GROUP = RULE == RULE_WKV ? GLA_GROUP / 2 : GLA_GROUP;      // (the old state is read beside the new one: more registers a row)
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256, (R <= 16 ? 2 : 1)) void gla_scan_kernel(const 
   if (chunk > 0 && chunk >= in_chunks) return;      // a shorter sequence has fewer chunks
   const bool apart = in_chunks > 1;
   float* mine = apart ? chunks.states + ((size_t)(seq * chunks.count + chunk) * H + head) * dim * vdim + v0 + col
-                      : state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * dim * vdim + v0 + col;
+                      : state + (size_t)seq_to[seq] * slot_stride + (size_t)head * dim * vdim + v0 + col;
   const float* from = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * dim * vdim + v0 + col;
   float S[R];
 #pragma unroll
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256, (R <= 16 ? 2 : 1)) void gla_scan_kernel(const 
 // S_in(c + 1) = A(c) S_in(c) + S_loc(c), A(c) the chunk's product of decays; a chunk's place in `states` then holds the state
 // it started from (for chunk_carry), and the state after the last chunk goes to the sequence's slot.
 __global__ __launch_bounds__(256) void gla_combine_kernel(GlaChunks chunks, float* __restrict__ state, long slot_stride,
-                                                          const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, int H,
+                                                          const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int H,
                                                           int dim, int vdim) {
   const int seq = blockIdx.y;
   const size_t per = (size_t)H * dim * vdim, e = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void gla_combine_kernel(GlaChunks chunks, floa
     *place = run;
     run = c == 0 ? local : fmaf(chunks.decays[(size_t)(seq * chunks.count + c) * H * dim + channel], run, local);
   }
-  state[(size_t)seq_slot[seq] * slot_stride + e] = run;
+  state[(size_t)seq_to[seq] * slot_stride + e] = run;
 }
 
 // out[row] += (carried query of the row) . S_in(the row's chunk), for the rows of every chunk but a sequence's first, on the float32
@@ -342,7 +342,7 @@ extern "C" int bh_gla_chunk_rows(int n_seqs, int max_rows, int H, int dim, int v
 template <int RULE>
 static int scan_run(const char* what, const void* q, const void* k, const void* v, int dtype, int row_stride, const float* z, int z_stride,
                     const float* bias, float inv_tau, const float* bonus, float q_scale, float* state, long slot_stride,
-                    const int32_t* seq_start, const int32_t* seq_slot, float* out, int n_seqs, int H, int dim, int vdim, int n_rows,
+                    const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_seqs, int H, int dim, int vdim, int n_rows,
                     int max_rows, int chunk_rows, float* scratch, hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && H > 0 && dim > 0 && vdim > 0, "%s: sizes must be positive", what);
   BH_REQUIRE(z_stride >= H * dim, "%s: the decays' rows hold %d numbers, %d are needed", what, z_stride, H * dim);
@@ -370,7 +370,7 @@ static int scan_run(const char* what, const void* q, const void* k, const void* 
   do {                                                                                                                       \
     bh_allow_lds<gla_scan_kernel<T, RR, RULE>>(lds);                                                                         \
     gla_scan_kernel<T, RR, RULE><<<grid, 256, lds, stream>>>((const T*)q, (const T*)k, (const T*)v, row_stride, z, z_stride, bias, \
-                                                             inv_tau, bonus, q_scale, state, slot_stride, seq_start, seq_slot, out, \
+                                                             inv_tau, bonus, q_scale, state, slot_stride, seq_start, seq_slot, seq_to, out, \
                                                              H, dim, vdim, VT, chunks);                                      \
   } while (0)
 #define BH_GLA_R(T)                  \
@@ -391,7 +391,7 @@ static int scan_run(const char* what, const void* q, const void* k, const void* 
   if (int status = bh_check_launch(what)) return status;
   if (chunks.rows == 0) return 0;
   const size_t per = (size_t)H * dim * vdim;
-  gla_combine_kernel<<<dim3((unsigned)((per + 255) / 256), n_seqs), 256, 0, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, H, dim, vdim);
+  gla_combine_kernel<<<dim3((unsigned)((per + 255) / 256), n_seqs), 256, 0, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, seq_to, H, dim, vdim);
   if (int status = bh_check_launch("gla_combine")) return status;
   return bh_chunk_carry(chunks.states, chunks.queries, chunks.rows, chunks.count, seq_start, out, n_seqs, H, dim, vdim, stream);
 }
@@ -403,7 +403,7 @@ static int scan_run(const char* what, const void* q, const void* k, const void* 
 // sequence's rows); where that is less than max_rows, scratch holds n_seqs * chunks * H * dim * (vdim + 1) + n_rows * H * dim floats.
 extern "C" int bh_gla_scan(const void* proj, int dtype, int proj_stride, int q_off, int k_off, int v_off, const float* z, int z_stride,
                            const float* bias, float tau, float q_scale, float* state, long slot_stride, const int32_t* seq_start,
-                           const int32_t* seq_slot, float* out, int n_seqs, int H, int dim, int vdim, int n_rows, int max_rows,
+                           const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_seqs, int H, int dim, int vdim, int n_rows, int max_rows,
                            int chunk_rows, float* scratch, hipStream_t stream) {
   BH_REQUIRE(tau > 0.f, "gla_scan: tau must be positive, got %f", (double)tau);
   BH_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && q_off + H * dim <= proj_stride && k_off + H * dim <= proj_stride &&
@@ -411,15 +411,15 @@ extern "C" int bh_gla_scan(const void* proj, int dtype, int proj_stride, int q_o
   const size_t element = dtype == BH_F32 ? 4 : 2;
   const char* rows = (const char*)proj;
   return scan_run<RULE_GLA>("gla_scan", rows + q_off * element, rows + k_off * element, rows + v_off * element, dtype, proj_stride, z, z_stride,
-                            bias, 1.0f / tau, nullptr, q_scale, state, slot_stride, seq_start, seq_slot, out, n_seqs, H, dim, vdim, n_rows,
+                            bias, 1.0f / tau, nullptr, q_scale, state, slot_stride, seq_start, seq_slot, seq_to, out, n_seqs, H, dim, vdim, n_rows,
                             max_rows, chunk_rows, scratch, stream);
 }
 
 // r, k [rows][row_stride] (dtype): H heads of `dim`; v: H heads of vdim; z, bias, state and the rest as above; bonus [H * dim] float32.
 extern "C" int bh_wkv_scan(const void* r, const void* k, const void* v, int dtype, int row_stride, const float* z, int z_stride, const float* bias,
-                           const float* bonus, float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot, float* out,
+                           const float* bonus, float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* out,
                            int n_seqs, int H, int dim, int vdim, int n_rows, int max_rows, int chunk_rows, float* scratch, hipStream_t stream) {
   BH_REQUIRE(bonus != nullptr && H * dim <= row_stride && H * vdim <= row_stride, "wkv_scan: r, k or v lie outside a row of %d", row_stride);
-  return scan_run<RULE_WKV>("wkv_scan", r, k, v, dtype, row_stride, z, z_stride, bias, 1.0f, bonus, 1.0f, state, slot_stride, seq_start, seq_slot,
+  return scan_run<RULE_WKV>("wkv_scan", r, k, v, dtype, row_stride, z, z_stride, bias, 1.0f, bonus, 1.0f, state, slot_stride, seq_start, seq_slot, seq_to,
                             out, n_seqs, H, dim, vdim, n_rows, max_rows, chunk_rows, scratch, stream);
 }

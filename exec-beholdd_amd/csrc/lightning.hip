@@ -37,7 +37,7 @@ __device__ inline float silu_f32(float x) { return x * __builtin_amdgcn_rcpf(1.0
 template <typename T, int DPT, int VT>
 __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_scan_kernel(const T* __restrict__ proj, int row_stride, int q_off, int k_off, int v_off,
                                       float* __restrict__ state, const float* __restrict__ decay,
-                                      const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                      const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                       float* __restrict__ out, int H, int dim, int vdim, int parts, int n_chunks,
                                       int chunk_rows, float* __restrict__ chunk_state) {
   extern __shared__ __align__(16) float lds[];
@@ -55,7 +55,6 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_scan_kernel(
   const int lo = seq_start[seq] + chunk * chunk_rows;
   if (lo >= seq_start[seq + 1]) return;      // the sequence has no such chunk
   const int hi = seq_start[seq + 1] < lo + chunk_rows ? seq_start[seq + 1] : lo + chunk_rows;
-  const int slot = seq_slot[seq];
   const float lambda = decay[head];
   const bool scaled = lambda >= LN_SCALED_FROM;
   if (threadIdx.x < LN_TOKENS) {
@@ -64,9 +63,10 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_scan_kernel(
     grow[threadIdx.x] = scaled ? power : 1.f;
     shrink[threadIdx.x] = scaled ? 1.0f / power : 1.f;
   }
-  float* mine = state + (((size_t)slot * H + head) * dim) * vdim;
+  const float* mine = state + (((size_t)seq_slot[seq] * H + head) * dim) * vdim;
   // where the end state goes: the cache, or with chunks the chunk's place in scratch memory
-  float* left = n_chunks > 1 ? chunk_state + ((((size_t)seq * n_chunks + chunk) * H + head) * dim) * vdim : mine;
+  float* left = n_chunks > 1 ? chunk_state + ((((size_t)seq * n_chunks + chunk) * H + head) * dim) * vdim
+                             : state + (((size_t)seq_to[seq] * H + head) * dim) * vdim;
   const bool live = column < vdim;
   float s[DPT];
 #pragma unroll
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_scan_kernel(
 template <typename T, int DPT, int VT>
 __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_step_kernel(
     const T* __restrict__ proj, int row_stride, int q_off, int k_off, int v_off, float* __restrict__ state,
-    const float* __restrict__ decay, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+    const float* __restrict__ decay, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
     float* __restrict__ out, int H, int dim, int vdim, int parts) {
   extern __shared__ __align__(16) float lds[];
   const int seq = blockIdx.x, head = blockIdx.y, tile = blockIdx.z;
@@ -213,7 +213,8 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_step_kernel(
   const int row = seq_start[seq];
   if (seq_start[seq + 1] <= row) return;
   const float lambda = decay[head];
-  float* mine = state + (((size_t)seq_slot[seq] * H + head) * dim) * vdim;
+  const float* mine = state + (((size_t)seq_slot[seq] * H + head) * dim) * vdim;
+  float* left = state + (((size_t)seq_to[seq] * H + head) * dim) * vdim;
   const bool live = column < vdim;
   float s[DPT];
 #pragma unroll
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_step_kernel(
 #pragma unroll
     for (int e = 0; e < DPT; ++e) {
       const int i = part * DPT + e;
-      if (i < dim) mine[(size_t)i * vdim + column] = s[e];
+      if (i < dim) left[(size_t)i * vdim + column] = s[e];
     }
   }
   __syncthreads();
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(DPT == 64 ? 1024 : 256) void lightning_step_kernel(
 __global__ __launch_bounds__(256) void lightning_combine_kernel(float* __restrict__ chunk_state, float* __restrict__ state,
                                                                 const float* __restrict__ decay,
                                                                 const int32_t* __restrict__ seq_start,
-                                                                const int32_t* __restrict__ seq_slot, int H, int size,
+                                                                const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int H, int size,
                                                                 int n_chunks, int chunk_rows) {
   const int seq = blockIdx.x, head = blockIdx.y, at = blockIdx.z * 256 + threadIdx.x;
   if (at >= size) return;
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256) void lightning_combine_kernel(float* __restric
     z[c * apart] = end;      // what chunk c should have started from
     end = fmaf(powf(lambda, (float)here), end, own);
   }
-  state[((size_t)seq_slot[seq] * H + head) * size + at] = end;
+  state[((size_t)seq_to[seq] * H + head) * size + at] = end;
 }
 
 // out[row] += decay^(t+1) E^T silu(q[row]) for the rows of every chunk but a sequence's first, E the state the chunk
@@ -354,7 +355,7 @@ extern "C" long bh_lightning_most_chunks(int n_seqs, int n_rows, int max_rows, i
 
 template <typename T, int DPT, int VT>
 static int launch_lightning(const void* proj, int row_stride, int q_off, int k_off, int v_off, float* state,
-                            const float* decay, const int32_t* seq_start, const int32_t* seq_slot, float* out, int n_seqs,
+                            const float* decay, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_seqs,
                             int n_rows, int H, int dim, int vdim, int n_chunks, int chunk_rows, float* chunk_state,
                             hipStream_t stream) {
   const int parts = (dim + DPT - 1) / DPT;
@@ -366,17 +367,17 @@ static int launch_lightning(const void* proj, int row_stride, int q_off, int k_o
   if (n_rows == n_seqs) {      // one row each
     const size_t lean = (size_t)(2 * parts * DPT + VT + parts * VT) * sizeof(float);
     lightning_step_kernel<T, DPT, VT><<<grid, block, lean, stream>>>((const T*)proj, row_stride, q_off, k_off, v_off, state, decay,
-                                                                     seq_start, seq_slot, out, H, dim, vdim, parts);
+                                                                     seq_start, seq_slot, seq_to, out, H, dim, vdim, parts);
     return bh_check_launch("lightning_step");
   }
   lightning_scan_kernel<T, DPT, VT><<<grid, block, smem, stream>>>((const T*)proj, row_stride, q_off, k_off, v_off, state, decay,
-                                                                   seq_start, seq_slot, out, H, dim, vdim, parts, n_chunks,
+                                                                   seq_start, seq_slot, seq_to, out, H, dim, vdim, parts, n_chunks,
                                                                    chunk_rows, chunk_state);
   if (int status = bh_check_launch("lightning_scan")) return status;
   if (n_chunks == 1) return 0;
   const int size = dim * vdim;
   lightning_combine_kernel<<<dim3(n_seqs, H, (size + 255) / 256), dim3(256), 0, stream>>>(chunk_state, state, decay, seq_start,
-                                                                                          seq_slot, H, size, n_chunks, chunk_rows);
+                                                                                          seq_slot, seq_to, H, size, n_chunks, chunk_rows);
   if (int status = bh_check_launch("lightning_combine")) return status;
   const int columns = vdim >= 256 ? 256 : (vdim + 63) / 64 * 64;
   dim3 carry(n_seqs * (n_chunks - 1) * (chunk_rows / LC_ROWS), H, (vdim + columns - 1) / columns);
@@ -387,9 +388,10 @@ static int launch_lightning(const void* proj, int row_stride, int q_off, int k_o
 
 // proj [n_rows][row_stride]: a row holds q (H x dim) from q_off, k (H x dim) from k_off, v (H x vdim) from v_off, all
 // before their silu.  state [slots][H][dim][vdim] float32; rows seq_start[b] .. seq_start[b + 1] - 1 belong to the
-// sequence in slot seq_slot[b], in order, and every sequence has at least one.  out [n_rows][H * vdim] float32.
+// sequence whose state is row seq_slot[b], in order, and every sequence has at least one; the state they leave is row seq_to[b] (the same
+// row, or one that no sequence of the step starts from, so that a step that fails leaves what it started from).  out [n_rows][H * vdim] float32.
 extern "C" int bh_lightning_scan(const void* proj, int dtype, int row_stride, int q_off, int k_off, int v_off, float* state,
-                                 const float* decay, const int32_t* seq_start, const int32_t* seq_slot, float* out,
+                                 const float* decay, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* out,
                                  int n_seqs, int n_rows, int max_rows, int H, int dim, int vdim, float* chunk_state,
                                  long chunk_state_floats, hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && n_rows >= n_seqs && H > 0 && dim > 0 && vdim > 0,
@@ -412,9 +414,9 @@ extern "C" int bh_lightning_scan(const void* proj, int dtype, int row_stride, in
   const int slice = (dim + 256 / vt - 1) / (256 / vt);      // slices of dim that make the workgroup four waves
 #define BH_LN(T, DPT)                                                                                                   \
   do {                                                                                                                  \
-    if (vt == 64) return launch_lightning<T, DPT, 64>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
-    if (vt == 32) return launch_lightning<T, DPT, 32>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
-    return launch_lightning<T, DPT, 16>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
+    if (vt == 64) return launch_lightning<T, DPT, 64>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, seq_to, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
+    if (vt == 32) return launch_lightning<T, DPT, 32>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, seq_to, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
+    return launch_lightning<T, DPT, 16>(proj, row_stride, q_off, k_off, v_off, state, decay, seq_start, seq_slot, seq_to, out, n_seqs, n_rows, H, dim, vdim, n_chunks, chunk_rows, chunk_state, stream); \
   } while (0)
 #define BH_LN_SIZES(T)            \
   if (slice <= 4) BH_LN(T, 4);    \
@@ -487,7 +489,7 @@ extern "C" long bh_lightning_products_most(int n_seqs, int n_rows, int max_rows,
 }
 // As bh_lightning_scan; proj, state and scratch lie on 16 bytes.
 extern "C" int bh_lightning_products(const void* proj, int dtype, int row_stride, int q_off, int k_off, int v_off, float* state,
-                                     const float* decay, const int32_t* seq_start, const int32_t* seq_slot, float* out, int n_seqs,
+                                     const float* decay, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_seqs,
                                      int n_rows, int max_rows, int H, int dim, int vdim, float* scratch, long scratch_floats,
                                      hipStream_t stream) {
   const long wanted = bh_lightning_products_scratch(n_seqs, n_rows, max_rows, H, dim, vdim, row_stride, q_off, k_off, v_off);
@@ -496,10 +498,10 @@ extern "C" int bh_lightning_products(const void* proj, int dtype, int row_stride
              "lightning: q, k and v do not lie inside a row of %d", row_stride);
   BH_REQUIRE((((uintptr_t)proj | (uintptr_t)state | (uintptr_t)scratch) % 16) == 0, "lightning: operands must be 16-byte aligned");
   if (dtype == BH_F32)
-    return ds_launch(LightningRows<float>{(const float*)proj, row_stride, q_off, k_off, v_off, decay, dim, vdim}, seq_start, seq_slot, state,
+    return ds_launch(LightningRows<float>{(const float*)proj, row_stride, q_off, k_off, v_off, decay, dim, vdim}, seq_start, seq_slot, seq_to, state,
                      (long)H * dim * vdim, out, scratch, scratch_floats, n_seqs, n_rows, H, dim, vdim, stream);
   if (dtype == BH_BF16)
-    return ds_launch(LightningRows<bf16_t>{(const bf16_t*)proj, row_stride, q_off, k_off, v_off, decay, dim, vdim}, seq_start, seq_slot, state,
+    return ds_launch(LightningRows<bf16_t>{(const bf16_t*)proj, row_stride, q_off, k_off, v_off, decay, dim, vdim}, seq_start, seq_slot, seq_to, state,
                      (long)H * dim * vdim, out, scratch, scratch_floats, n_seqs, n_rows, H, dim, vdim, stream);
   return bh_fail("lightning: unknown dtype %d", dtype);
 }

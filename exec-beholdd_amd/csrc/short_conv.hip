@@ -2,7 +2,8 @@
 // step through a state that holds the last taps - 1 inputs of each sequence:
 //   y[t][c] = sum_j w[c][j] * u[t - taps + 1 + j][c]  (+ bias[c])  (then silu),   zeros before a sequence starts.
 //   short_conv        the rows of a step; inputs that lie before the step come from the state
-//   short_conv_state  the state after the step (run it after every reader of the old state)
+//   short_conv_state  the state after the step (run it after every reader of the old state), left in the rows seq_to, which may be
+//                     those it is read from
 // State of one sequence: [taps - 1][channels] float32, the oldest input first, at `state + slot * slot_stride`.
 // Sums are float32; the result is float32.
 #include "common.h"
@@ -128,11 +129,12 @@ template <typename T>
 __global__ __launch_bounds__(256) void short_conv_state_kernel(const T* __restrict__ u, int row_stride, int first,
                                                                float* __restrict__ state, long slot_stride,
                                                                const int32_t* __restrict__ seq_start,
-                                                               const int32_t* __restrict__ seq_slot, int channels, int taps) {
+                                                               const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int channels, int taps) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, seq = blockIdx.y;
   if (c >= channels) return;
   const int start = seq_start[seq], n_new = seq_start[seq + 1] - start, keep = taps - 1;
-  float* mine = state + (size_t)seq_slot[seq] * slot_stride;
+  const float* mine = state + (size_t)seq_slot[seq] * slot_stride;
+  float* left = state + (size_t)seq_to[seq] * slot_stride;
   float next[SC_MAX_TAPS];
 #pragma unroll
   for (int s = 0; s < SC_MAX_TAPS; ++s) {
@@ -143,12 +145,12 @@ __global__ __launch_bounds__(256) void short_conv_state_kernel(const T* __restri
 #pragma unroll
   for (int s = 0; s < SC_MAX_TAPS; ++s) {
     if (s >= keep) break;
-    mine[(size_t)s * channels + c] = next[s];
+    left[(size_t)s * channels + c] = next[s];
   }
 }
 
 extern "C" int bh_short_conv_state(const void* u, int dtype, int row_stride, int first, float* state, long slot_stride,
-                                   const int32_t* seq_start, const int32_t* seq_slot, int n_seqs, int channels, int taps,
+                                   const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, int n_seqs, int channels, int taps,
                                    hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && channels > 0, "short_conv_state: sizes must be positive");
   BH_REQUIRE(taps >= 1 && taps <= SC_MAX_TAPS, "short_conv_state: 1 to %d taps, got %d", SC_MAX_TAPS, taps);
@@ -157,10 +159,10 @@ extern "C" int bh_short_conv_state(const void* u, int dtype, int row_stride, int
   dim3 grid((channels + 255) / 256, n_seqs);
   if (dtype == BH_F32)
     short_conv_state_kernel<float><<<grid, 256, 0, stream>>>((const float*)u, row_stride, first, state, slot_stride, seq_start,
-                                                             seq_slot, channels, taps);
+                                                             seq_slot, seq_to, channels, taps);
   else if (dtype == BH_BF16)
     short_conv_state_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)u, row_stride, first, state, slot_stride, seq_start,
-                                                              seq_slot, channels, taps);
+                                                              seq_slot, seq_to, channels, taps);
   else
     return bh_fail("short_conv_state: unknown dtype %d", dtype);
   return bh_check_launch("short_conv_state");

@@ -1,7 +1,8 @@
 // A selective state-space recurrence with a scalar decay per head (the "state-space duality" form), kept as a
 // recurrent state, and the gated norm behind it:
 //   ssm_scan            per (sequence, head): dt = softplus(dt_raw + dt_bias);  S <- exp(-exp(A_log) dt) S + dt B x^T;
-//                       y = S^T C + D x.   S is [N][vdim] float32 and lives in the sequence's state region.
+//                       y = S^T C + D x.   S is [N][vdim] float32, read from row seq_slot of the states and left in
+//                       row seq_to (the same one, or one that no sequence of the step starts from).
 //   gated_group_rmsnorm out = rms_g(y * silu(z)) * w, the root mean square taken in `groups` equal parts of a row; with
 //                       `gate_after` the statistic is y's alone: out = rms_g(y) * w * silu(z)
 // Everything but the reading of dt_raw and z is float32.  Prompts of aligned sizes go through decay_scan.h (chunks of 64 rows as
@@ -19,7 +20,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
                                                        int proj_stride, int dt_first, const float* __restrict__ dt_bias,
                                                        const float* __restrict__ a_log, const float* __restrict__ d_skip,
                                                        float* __restrict__ state, long slot_stride,
-                                                       const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                                       const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                                        float* __restrict__ y, int H, int vdim, int N, int G, int slices) {
   extern __shared__ float lds[];
   float* S = lds;                          // [N][vdim]
@@ -30,7 +31,8 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
   const int seq = blockIdx.x, head = blockIdx.y, group = head / (H / G);
   const int inner = H * vdim;
   const int start = seq_start[seq], stop = seq_start[seq + 1];
-  float* mine = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * N * vdim;
+  const float* mine = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * N * vdim;
+  float* left = state + (size_t)seq_to[seq] * slot_stride + (size_t)head * N * vdim;
   for (int e = threadIdx.x; e < N * vdim; e += blockDim.x) S[e] = mine[e];
   const int p = threadIdx.x % vdim, s = threadIdx.x / vdim;
   const bool works = s < slices;
@@ -67,12 +69,12 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
     }
     __syncthreads();
   }
-  for (int e = threadIdx.x; e < N * vdim; e += blockDim.x) mine[e] = S[e];
+  for (int e = threadIdx.x; e < N * vdim; e += blockDim.x) left[e] = S[e];
 }
 
 extern "C" int bh_ssm_scan(const float* xbc, int xbc_stride, const void* proj, int dtype, int proj_stride, int dt_first,
                            const float* dt_bias, const float* a_log, const float* d_skip, float* state, long slot_stride,
-                           const int32_t* seq_start, const int32_t* seq_slot, float* y, int n_seqs, int H, int vdim, int N, int G,
+                           const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* y, int n_seqs, int H, int vdim, int N, int G,
                            hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && H > 0 && vdim > 0 && N > 0 && G > 0, "ssm_scan: sizes must be positive");
   BH_REQUIRE(H % G == 0, "ssm_scan: %d heads do not fall into %d groups evenly", H, G);
@@ -87,11 +89,11 @@ extern "C" int bh_ssm_scan(const float* xbc, int xbc_stride, const void* proj, i
   if (dtype == BH_F32) {
     bh_allow_lds<ssm_scan_kernel<float>>(lds_bytes);
     ssm_scan_kernel<float><<<grid, 256, lds_bytes, stream>>>(xbc, xbc_stride, (const float*)proj, proj_stride, dt_first, dt_bias, a_log,
-                                                             d_skip, state, slot_stride, seq_start, seq_slot, y, H, vdim, N, G, slices);
+                                                             d_skip, state, slot_stride, seq_start, seq_slot, seq_to, y, H, vdim, N, G, slices);
   } else if (dtype == BH_BF16) {
     bh_allow_lds<ssm_scan_kernel<bf16_t>>(lds_bytes);
     ssm_scan_kernel<bf16_t><<<grid, 256, lds_bytes, stream>>>(xbc, xbc_stride, (const bf16_t*)proj, proj_stride, dt_first, dt_bias,
-                                                              a_log, d_skip, state, slot_stride, seq_start, seq_slot, y, H, vdim, N, G,
+                                                              a_log, d_skip, state, slot_stride, seq_start, seq_slot, seq_to, y, H, vdim, N, G,
                                                               slices);
   } else {
     return bh_fail("ssm_scan: unknown dtype %d", dtype);
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const float* __restrict_
                                                         const float* __restrict__ a_log, const float* __restrict__ d_skip,
                                                         float* __restrict__ state, long slot_stride, float* __restrict__ chunk_states,
                                                         float* __restrict__ chunk_decay, float* __restrict__ cum,
-                                                        const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                                        const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                                         float* __restrict__ y, int H, int vdim, int N, int G, int slices, int chunk_rows,
                                                         int chunks_per_seq) {
   extern __shared__ __align__(16) float lds[];
@@ -135,8 +137,9 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const float* __restrict_
   const bool works = s < slices;
   const int per = (N + slices - 1) / slices;
   const int n0 = s * per, n1 = n0 + per < N ? n0 + per : N;
-  float* home = MODE == 0 ? state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * N * vdim
-                          : chunk_states + ((size_t)blockIdx.x * H + head) * N * vdim;
+  const float* home = MODE == 0 ? state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * N * vdim
+                                : chunk_states + ((size_t)blockIdx.x * H + head) * N * vdim;
+  float* left = MODE == 0 ? state + (size_t)seq_to[seq] * slot_stride + (size_t)head * N * vdim : chunk_states + ((size_t)blockIdx.x * H + head) * N * vdim;
   float S[NPT];
 #pragma unroll
   for (int i = 0; i < NPT; ++i) S[i] = (MODE != 1 && works && n0 + i < n1) ? home[(size_t)(n0 + i) * vdim + p] : 0.f;
@@ -233,7 +236,7 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const float* __restrict_
   if (MODE != 2 && works) {
 #pragma unroll
     for (int i = 0; i < NPT; ++i)
-      if (n0 + i < n1) home[(size_t)(n0 + i) * vdim + p] = S[i];
+      if (n0 + i < n1) left[(size_t)(n0 + i) * vdim + p] = S[i];
   }
   if (MODE == 1 && threadIdx.x == 0) chunk_decay[(size_t)blockIdx.x * H + head] = run;
 }
@@ -241,12 +244,13 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(const float* __restrict_
 // grid (sequences, heads): a thread per state element walks the sequence's chunks in order.
 __global__ __launch_bounds__(256) void ssm_combine_kernel(float* __restrict__ state, long slot_stride, float* __restrict__ chunk_states,
                                                           const float* __restrict__ chunk_decay, const int32_t* __restrict__ seq_start,
-                                                          const int32_t* __restrict__ seq_slot, int H, int elements, int chunk_rows,
+                                                          const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int H, int elements, int chunk_rows,
                                                           int chunks_per_seq) {
   const int seq = blockIdx.x, head = blockIdx.y;
   const int n_rows = seq_start[seq + 1] - seq_start[seq];
   const int chunks = (n_rows + chunk_rows - 1) / chunk_rows;
-  float* home = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * elements;
+  const float* home = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * elements;
+  float* left = state + (size_t)seq_to[seq] * slot_stride + (size_t)head * elements;
   for (int e = threadIdx.x; e < elements; e += blockDim.x) {
     float S = home[e];
     for (int c = 0; c < chunks; ++c) {
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(256) void ssm_combine_kernel(float* __restrict__ st
       *slot = S;
       S = fmaf(expf(chunk_decay[at * H + head]), S, local);
     }
-    home[e] = S;
+    left[e] = S;
   }
 }
 
@@ -299,14 +303,14 @@ extern "C" int bh_ssm_fast_takes(int vdim, int N) {
 template <typename T, int NPT>
 static int ssm_fast_launch(const float* xbc, int xbc_stride, const T* proj, int proj_stride, int dt_first, const float* dt_bias,
                            const float* a_log, const float* d_skip, float* state, long slot_stride, float* chunk_states,
-                           float* chunk_decay, float* cum, const int32_t* seq_start, const int32_t* seq_slot, float* y, int n_seqs, int H,
+                           float* chunk_decay, float* cum, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* y, int n_seqs, int H,
                            int vdim, int N, int G, int slices, int chunk_rows, int chunks_per_seq, size_t lds, hipStream_t stream) {
   dim3 grid(n_seqs * chunks_per_seq, H);
 #define BH_SS(MODE)                                                                                                                 \
   do {                                                                                                                              \
     bh_allow_lds<ssm_chunk_kernel<T, NPT, MODE>>(lds);                                                                              \
     ssm_chunk_kernel<T, NPT, MODE><<<grid, 256, lds, stream>>>(xbc, xbc_stride, proj, proj_stride, dt_first, dt_bias, a_log, d_skip,   \
-                                                               state, slot_stride, chunk_states, chunk_decay, cum, seq_start, seq_slot, \
+                                                               state, slot_stride, chunk_states, chunk_decay, cum, seq_start, seq_slot, seq_to, \
                                                                y, H, vdim, N, G, slices, chunk_rows, chunks_per_seq);                \
   } while (0)
   if (chunks_per_seq == 1) {
@@ -314,7 +318,7 @@ static int ssm_fast_launch(const float* xbc, int xbc_stride, const T* proj, int 
     return bh_check_launch("ssm_scan");
   }
   BH_SS(1);
-  ssm_combine_kernel<<<dim3(n_seqs, H), 256, 0, stream>>>(state, slot_stride, chunk_states, chunk_decay, seq_start, seq_slot, H, N * vdim,
+  ssm_combine_kernel<<<dim3(n_seqs, H), 256, 0, stream>>>(state, slot_stride, chunk_states, chunk_decay, seq_start, seq_slot, seq_to, H, N * vdim,
                                                          chunk_rows, chunks_per_seq);
   BH_SS(2);
 #undef BH_SS
@@ -325,7 +329,7 @@ static int ssm_fast_launch(const float* xbc, int xbc_stride, const T* proj, int 
 // memory of the call (unused, and may be null, with one chunk a sequence).
 extern "C" int bh_ssm_scan_fast(const float* xbc, int xbc_stride, const void* proj, int dtype, int proj_stride, int dt_first,
                                 const float* dt_bias, const float* a_log, const float* d_skip, float* state, long slot_stride,
-                                float* chunk_states, float* chunk_decay, float* cum, const int32_t* seq_start, const int32_t* seq_slot,
+                                float* chunk_states, float* chunk_decay, float* cum, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to,
                                 float* y, int n_seqs, int H, int vdim, int N, int G, int chunk_rows, int chunks_per_seq,
                                 hipStream_t stream) {
   BH_REQUIRE(n_seqs > 0 && H > 0 && G > 0 && H % G == 0, "ssm_scan: %d heads in %d groups", H, G);
@@ -340,7 +344,7 @@ extern "C" int bh_ssm_scan_fast(const float* xbc, int xbc_stride, const void* pr
   const size_t lds = ((size_t)SS_STAGE * (2 * N + vdim + slices * vdim + 2)) * sizeof(float);
 #define BH_SF(T, NPT)                                                                                                              \
   return ssm_fast_launch<T, NPT>(xbc, xbc_stride, (const T*)proj, proj_stride, dt_first, dt_bias, a_log, d_skip, state, slot_stride, \
-                                 chunk_states, chunk_decay, cum, seq_start, seq_slot, y, n_seqs, H, vdim, N, G, slices, chunk_rows,   \
+                                 chunk_states, chunk_decay, cum, seq_start, seq_slot, seq_to, y, n_seqs, H, vdim, N, G, slices, chunk_rows,   \
                                  chunks_per_seq, lds, stream)
   if (dtype == BH_F32) {
     if (per <= 8) BH_SF(float, 8);
@@ -414,7 +418,7 @@ extern "C" long bh_ssm_products_most(int n_seqs, int n_rows, int max_rows, int H
 // As bh_ssm_scan; xbc, the state and its stride lie on 16 bytes.
 extern "C" int bh_ssm_products(const float* xbc, int xbc_stride, const void* proj, int dtype, int proj_stride, int dt_first,
                                const float* dt_bias, const float* a_log, const float* d_skip, float* state, long slot_stride,
-                               const int32_t* seq_start, const int32_t* seq_slot, float* y, int n_seqs, int H, int vdim, int N, int G,
+                               const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, float* y, int n_seqs, int H, int vdim, int N, int G,
                                int n_rows, int max_rows, float* scratch, long scratch_floats, hipStream_t stream) {
   const long wanted = bh_ssm_products_scratch(n_seqs, n_rows, max_rows, H, vdim, N, G, xbc_stride);
   BH_REQUIRE(wanted > 0 && scratch != nullptr && scratch_floats >= wanted, "ssm_scan: %d heads of %d with %d rows do not go as products", H, vdim, N);
@@ -424,10 +428,10 @@ extern "C" int bh_ssm_products(const float* xbc, int xbc_stride, const void* pro
              "ssm_scan: operands must be 16-byte aligned");
   if (dtype == BH_F32)
     return ds_launch(SsmRows<float>{xbc, xbc_stride, (const float*)proj, proj_stride, dt_first, dt_bias, a_log, d_skip, H, vdim, N, G}, seq_start,
-                     seq_slot, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
+                     seq_slot, seq_to, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
   if (dtype == BH_BF16)
     return ds_launch(SsmRows<bf16_t>{xbc, xbc_stride, (const bf16_t*)proj, proj_stride, dt_first, dt_bias, a_log, d_skip, H, vdim, N, G}, seq_start,
-                     seq_slot, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
+                     seq_slot, seq_to, state, slot_stride, y, scratch, scratch_floats, n_seqs, n_rows, H, N, vdim, stream);
   return bh_fail("ssm_scan: unknown dtype %d", dtype);
 }
 

@@ -40,11 +40,11 @@ __device__ inline void ts_store8(bf16_t* p, const float (&x)[8]) {
 // mixes lie in blocks of rows, a wave's lanes are the 16-byte pieces of a block in their order, so that its stores (and its loads, where h
 // lies in such blocks too) cover contiguous memory; otherwise they are neighbouring columns of a row.  Many rows: `turns` of them a thread.
 // The thread of a sequence's first row reads what the slot keeps of these columns and then
-// writes what it shall keep.
+// writes what it shall keep, to the row seq_to names (the same one or another).
 template <typename T>
 __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ h, int h_block_rows, const float* __restrict__ mu, int mixes,
                                                           float* __restrict__ state, long slot_stride, const int32_t* __restrict__ row_seq,
-                                                          const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, ShiftOuts outs,
+                                                          const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, ShiftOuts outs,
                                                           int out_block_rows, int n_rows, int width, int turns, int pieces) {
   const int piece = blockIdx.x * 256 + threadIdx.x;      // within a group of `apart` rows
   if (piece >= pieces) return;
@@ -57,13 +57,14 @@ __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ 
     float now[8], before[8];
     ts_load8(now, h + bh_rows_index(h_block_rows, row, column, width));
     if (opens == row) {
-      float* kept = state + (size_t)seq_slot[seq] * slot_stride + column;
+      const float* kept = state + (size_t)seq_slot[seq] * slot_stride + column;
+      float* keeps = state + (size_t)seq_to[seq] * slot_stride + column;
       float last[8];
       ts_load8(last, h + bh_rows_index(h_block_rows, seq_start[seq + 1] - 1, column, width));
 #pragma unroll
       for (int e = 0; e < 8; ++e) before[e] = kept[e];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) kept[e] = last[e];
+      for (int e = 0; e < 8; ++e) keeps[e] = last[e];
     } else {
       ts_load8(before, h + bh_rows_index(h_block_rows, row - 1, column, width));
     }
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ 
 template <typename T>
 __global__ __launch_bounds__(256) void token_shift_plain_kernel(const T* __restrict__ h, const float* __restrict__ mu, int mixes,
                                                                 float* __restrict__ state, long slot_stride, const int32_t* __restrict__ row_seq,
-                                                                const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot,
+                                                                const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
                                                                 ShiftOuts outs, int n_rows, int width) {
   const int column = blockIdx.x * 256 + threadIdx.x, row = blockIdx.y;
   if (column >= width) return;
@@ -91,9 +92,8 @@ __global__ __launch_bounds__(256) void token_shift_plain_kernel(const T* __restr
   const float now = to_f32(h[(size_t)row * width + column]);
   float before;
   if (seq_start[seq] == row) {
-    float* kept = state + (size_t)seq_slot[seq] * slot_stride + column;
-    before = *kept;
-    *kept = to_f32(h[(size_t)(seq_start[seq + 1] - 1) * width + column]);
+    before = state[(size_t)seq_slot[seq] * slot_stride + column];
+    state[(size_t)seq_to[seq] * slot_stride + column] = to_f32(h[(size_t)(seq_start[seq + 1] - 1) * width + column]);
   } else {
     before = to_f32(h[(size_t)(row - 1) * width + column]);
   }
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void token_shift_plain_kernel(const T* __restr
 // h [n_rows][width] (dtype; rows or blocks); mu f32 [mixes][width]; state: `width` floats a slot from state + slot * slot_stride; outs: `mixes`
 // matrices like h.
 extern "C" int bh_token_shift(const void* h, int dtype, int h_block_rows, const float* mu, int mixes, float* state, long slot_stride,
-                              const int32_t* row_seq, const int32_t* seq_start, const int32_t* seq_slot, void* const* outs, int out_block_rows,
+                              const int32_t* row_seq, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to, void* const* outs, int out_block_rows,
                               int n_rows, int width, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "token_shift: sizes must be positive");
   BH_REQUIRE(mixes >= 1 && mixes <= TS_MOST, "token_shift: 1 to %d mixes, not %d", TS_MOST, mixes);
@@ -123,10 +123,10 @@ extern "C" int bh_token_shift(const void* h, int dtype, int h_block_rows, const 
     const dim3 grid((pieces + 255) / 256, (groups + turns - 1) / turns);
     BH_REQUIRE(grid.y <= 65535, "token_shift: too many rows");
     if (dtype == BH_F32)
-      token_shift_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_block_rows, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, to,
+      token_shift_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_block_rows, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, seq_to, to,
                                                           out_block_rows, n_rows, width, turns, pieces);
     else if (dtype == BH_BF16)
-      token_shift_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, h_block_rows, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot,
+      token_shift_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, h_block_rows, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, seq_to,
                                                            to, out_block_rows, n_rows, width, turns, pieces);
     else return bh_fail("token_shift: unknown dtype %d", dtype);
     return bh_check_launch("token_shift");
@@ -134,10 +134,10 @@ extern "C" int bh_token_shift(const void* h, int dtype, int h_block_rows, const 
   BH_REQUIRE(n_rows <= 65535, "token_shift: %d rows of a width that is no multiple of 8", n_rows);
   const dim3 grid((width + 255) / 256, n_rows);
   if (dtype == BH_F32)
-    token_shift_plain_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, to, n_rows,
+    token_shift_plain_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, seq_to, to, n_rows,
                                                               width);
   else if (dtype == BH_BF16)
-    token_shift_plain_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, to, n_rows,
+    token_shift_plain_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, mu, mixes, state, slot_stride, row_seq, seq_start, seq_slot, seq_to, to, n_rows,
                                                                width);
   else return bh_fail("token_shift: unknown dtype %d", dtype);
   return bh_check_launch("token_shift");

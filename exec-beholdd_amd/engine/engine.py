@@ -77,7 +77,8 @@ class Engine:
 
         def make_cache(built):
             return SequenceCache(built.entry_needs, max_tokens, self.dtype, self.device, kernels.page_size,
-                                 max_slots=max_slots, max_position=built.max_position)
+                                 max_slots=max_slots, max_position=built.max_position,
+                                 banks=entries_of_one_run(built) if getattr(kernels, "state_in_banks", False) else ())
 
         def within_budget(weight_bytes, cache):
             capacity = cache.n_pages * cache.page_size
@@ -217,6 +218,12 @@ class Engine:
 
     def memory_plan(self) -> str:
         return f"{self.plan.describe()}\n{self.cache_plan.describe()}"
+
+
+def entries_of_one_run(model) -> set:
+    """The cache entries that one run of a layer alone uses in a step: what it leaves there nobody reads before the next step."""
+    runs = [entry for _layer, entry in getattr(model, "schedule", ())]
+    return {entry for entry in runs if runs.count(entry) == 1}
 
 
 def _model_tensors(model):

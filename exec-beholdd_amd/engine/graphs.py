@@ -60,8 +60,8 @@ class DecodeGraph:
         if self.copied is not None:
             self.copied.synchronize()     # the pinned buffer may not change under a copy in flight
         host = self.host_views
-        self.layout.fill(host, [_every_row_wanted(e) for e in entries], pasts)
         slots = [e.slot for e in entries]
+        self.layout.fill(host, [_every_row_wanted(e) for e in entries], pasts, cache.state_rows(slots))
         for index in self.layout.kv_groups:
             table = host["tables"][index]
             group = cache.groups[index]

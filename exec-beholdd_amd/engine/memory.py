@@ -55,7 +55,7 @@ def step_size(model, rows: int, seqs: int, act_size: int, max_position: int, siz
 
 def step_numbers_bytes(rows: int, seqs: int, kv_groups: int, table_width: int) -> int:
     """The step's integers on the device (`StepLayout.total` int32)."""
-    return _rounded(4 * (4 * rows + 3 * seqs + 1 + seqs + kv_groups * seqs * table_width))
+    return _rounded(4 * (4 * rows + 5 * seqs + 1 + seqs + kv_groups * seqs * table_width))
 
 
 def weights_as_kept(model, act_size: int, sizes) -> tuple:
@@ -117,7 +117,7 @@ def plan_memory(model, weight_bytes: int, cache_plan, act_size: int, sizes, max_
     plan.add("tables the parts build", tables_bytes(model))
     plan.add("cache", cache_plan.total_bytes)
     kv_groups = sum(1 for g in cache_plan.groups if g.need.kind == "kv")
-    state_bytes = sum(g.state_bytes for g in cache_plan.groups)
+    state_bytes = sum(g.state_bytes for g in cache_plan.groups if not g.banked)
     plan.add("state rows kept during a step, to put back if it fails", state_bytes)
     if hasattr(model, "working_bytes"):
         rows = int(max_rows_per_step)

@@ -73,13 +73,15 @@ class StepLayout:
     buffer with it and copies it to the device once; a captured decode step keeps a buffer of this layout for
     good and refreshes it before every replay.  A new piece is added here and nowhere else."""
 
-    PIECES = ("tokens", "positions", "row_seq", "seq_start", "seq_slot", "seq_past", "want_rows", "token_src")
+    PIECES = ("tokens", "positions", "row_seq", "seq_start", "seq_slot", "seq_past", "want_rows", "token_src",
+              "state_from", "state_to")
 
     def __init__(self, n_rows: int, n_seqs: int, n_want: int, kv_groups, table_width: int):
         self.n_rows, self.n_seqs, self.n_want = int(n_rows), int(n_seqs), int(n_want)
         self.kv_groups, self.table_width = list(kv_groups), int(table_width)
         sizes = {"tokens": n_rows, "positions": n_rows, "row_seq": n_rows, "seq_start": n_seqs + 1,
-                 "seq_slot": n_seqs, "seq_past": n_seqs, "want_rows": n_want, "token_src": n_rows}
+                 "seq_slot": n_seqs, "seq_past": n_seqs, "want_rows": n_want, "token_src": n_rows,
+                 "state_from": n_seqs, "state_to": n_seqs}
         self.place, at = {}, 0
         for name in self.PIECES:
             self.place[name] = (at, at + sizes[name])
@@ -97,8 +99,10 @@ class StepLayout:
                          for group, (lo, hi) in self.table_place.items()}
         return out
 
-    def fill(self, host, entries: list, pasts: list) -> None:
-        """Write everything but the page tables into the host views `host` (from `views`)."""
+    def fill(self, host, entries: list, pasts: list, state_rows=None) -> None:
+        """Write everything but the page tables into the host views `host` (from `views`).  `state_rows`: the rows in
+        which a cache with two rows a slot holds the sequences' states, and those in which the step leaves them."""
+        host["state_from"][:], host["state_to"][:] = state_rows if state_rows is not None else 2 * [[e.slot for e in entries]]
         if self.n_rows == self.n_seqs:       # one token each: whole pieces at once
             count = np.arange(self.n_seqs + 1, dtype=np.int32)
             host["tokens"][:] = [0 if e.fed_row is not None else e.tokens[0] for e in entries]
@@ -140,6 +144,7 @@ class StepLayout:
             host_seq_start=lists["seq_start"], host_seq_slot=lists["seq_slot"], host_seq_past=lists["seq_past"],
             is_decode=(self.n_rows == self.n_seqs), max_position=int(max_position),
             max_rows_per_seq=int(max_rows_per_seq),
+            state_from=device_views["state_from"], state_to=device_views["state_to"],
             token_src=device_views["token_src"] if fed_tokens is not None else None, fed_tokens=fed_tokens)
 
 
@@ -198,7 +203,7 @@ def build_step(kernels, act_dtype, device, cache, entries: list, staging: StepSt
     layout = StepLayout(n_rows, len(entries), sum(len(entry.want) for entry in entries), kv_groups, width)
     host_buffer = np.zeros(layout.total, dtype=np.int32)
     host = layout.views(host_buffer)
-    layout.fill(host, entries, pasts)
+    layout.fill(host, entries, pasts, cache.state_rows(slots))
     for group in kv_groups:
         cache.write_page_table(group, slots, host["tables"][group])
     if staging is not None and torch.device(device).type == "cuda":

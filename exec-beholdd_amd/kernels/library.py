@@ -181,10 +181,10 @@ class KernelSizes:
             "bh_relu_squared": [p, p, i, i, i, i, p],
             "bh_gemm_bf16_squared": [p, p, p, i, i, i, i, i, p],
             "bh_gemm_bf16_squares": [i, i, i],
-            "bh_lightning_scan": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
+            "bh_lightning_scan": [p, i, i, i, i, i, p, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
             "bh_lightning_chunks": [i, i, i, i, i, p],
-            "bh_lightning_products": [p, i, i, i, i, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
-            "bh_ssm_products": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, ctypes.c_long, p],
+            "bh_lightning_products": [p, i, i, i, i, i, p, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, p],
+            "bh_ssm_products": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, ctypes.c_long, p],
             "bh_gated_rmsnorm": [p, p, i, i, p, p, i, i, f, i, p],
             "bh_latent_write": [p, i, i, i, p, f, p, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, i, i, i, i, i, p, ctypes.c_long, i, f, p],
             "bh_heads_linear": [p, ctypes.c_long, i, i, p, p, ctypes.c_long, i, i, i, i, i, i, i, i, p],
@@ -203,17 +203,17 @@ class KernelSizes:
             "bh_rms_scale_add": [p, p, p, i, i, f, p],
             "bh_gelu_gate_table": [p, i, p, p, p, p, i, i, i, p, i, i, i, p],
             "bh_short_conv": [p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, p],
-            "bh_short_conv_state": [p, i, i, i, p, ctypes.c_long, p, p, i, i, i, p],
+            "bh_short_conv_state": [p, i, i, i, p, ctypes.c_long, p, p, p, i, i, i, p],
             "bh_whole_norm_rope_write": [p, p, p, f, p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, i, i, p],
             "bh_gate_heads": [p, i, i, p, i, i, p, i, i, i, i, i, p],
-            "bh_ssm_scan": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, i, i, i, i, i, p],
+            "bh_ssm_scan": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, p],
             "bh_gated_group_rmsnorm": [p, p, i, i, i, p, f, p, i, i, i, i, i, p],
             "bh_route_top_k": [p, i, p, p, p, p, i, i, i, i, p],
             "bh_experts_gate_up": [p, i, p, p, p, i, i, i, i, i, f, f, f, p, p],
             "bh_experts_down": [p, i, p, p, p, p, p, i, i, i, i, i, i, p],
             "bh_clamped_glu": [p, i, p, i, i, f, f, i, f, p],
             "bh_conv_norm_rope_write": [p, i, i, i, p, i, p, ctypes.c_long, p, p, p, p, f, p, i, p, p, p, p, p, p, i, i, i, i, i, i, i, i, i, p],
-            "bh_ssm_scan_fast": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, p, p, i, i, i, i, i, i, i, p],
+            "bh_ssm_scan_fast": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, p, p, p, i, i, i, i, i, i, i, p],
             "bh_ssm_chunk_rows": [i, i, i],
             "bh_ssm_fast_takes": [i, i],
             "bh_experts_products": [p, p, p, i, p, i, i, i, f, f, f, p],
@@ -225,14 +225,14 @@ class KernelSizes:
             "bh_experts_many": [p, i, p, i, p, p, p, i, i, i, i, i, f, f, f, p, p],
             "bh_experts_many_tile": [i, i, i, i, i],
             "bh_experts_gather": [p, i, i, p, i, p, p, p, p, i, i, i, p, p],
-            "bh_gla_scan": [p, i, i, i, i, i, p, i, p, f, f, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, p],
+            "bh_gla_scan": [p, i, i, i, i, i, p, i, p, f, f, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p],
             "bh_gla_chunk_rows": [i, i, i, i, i],
-            "bh_wkv_scan": [p, p, p, i, i, p, i, p, p, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, p, p],
-            "bh_token_shift": [p, i, i, p, i, p, ctypes.c_long, p, p, p, p, i, i, i, p],
+            "bh_wkv_scan": [p, p, p, i, i, p, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p],
+            "bh_token_shift": [p, i, i, p, i, p, ctypes.c_long, p, p, p, p, p, i, i, i, p],
             "bh_tanh_rows": [p, i, p, i, i, i, i, p],
             "bh_delta_prep": [p, i, i, i, i, i, p, i, p, ctypes.c_long, ctypes.c_long, p, p, p, p, p, p, p, i, i, i, i, i, p],
-            "bh_delta_scan": [p, p, p, ctypes.c_long, p, p, p, i, i, i, i, i, i, i, i, p, p],
-            "bh_delta_step": [p, i, i, i, i, i, i, p, i, p, ctypes.c_long, ctypes.c_long, p, p, p, p, f, p, i, i, i, i, i, i, p],
+            "bh_delta_scan": [p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, p, p],
+            "bh_delta_step": [p, i, i, i, i, i, i, p, i, p, ctypes.c_long, ctypes.c_long, p, p, p, p, p, f, p, i, i, i, i, i, i, p],
             "bh_delta_step_takes": [i, i],
             "bh_delta_chunk_rows": [i, i, i, i, i],
             "bh_delta_takes": [i, i],
@@ -370,6 +370,7 @@ class HipKernels(KernelSizes):
         self._device_index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self.device = torch.device("cuda", self._device_index)
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        self.state_in_banks = True      # the kernels that move a state on take `seq_to`, the rows to leave it in
         self._plans: dict = {}      # (m, n, k, packed, activation) -> what the library says of such a product
         self._squares: dict = {}    # (m, n, k) -> which product squares its output (`gemm_relu_squared`), or 0
         self._bare: dict = {}       # (m, n, k) -> the parts that `gemm_bare` leaves such a product in, or 0
@@ -415,6 +416,14 @@ class HipKernels(KernelSizes):
         if dtypes is not None and tensor.dtype not in dtypes:
             raise KernelError(f"{what}: dtype {tensor.dtype} is not one of {dtypes}")
         return tensor.data_ptr()
+
+    def _rows_to(self, seq_to, seq_slot):
+        """The rows of the state that a step's sequences leave theirs in: those they start from, or others of as many."""
+        if seq_to is None:
+            return self._ptr(seq_slot, "seq_slot", (torch.int32,))
+        if seq_to.shape != seq_slot.shape:
+            raise KernelError(f"a row to leave the state in for each sequence: {tuple(seq_to.shape)} for {tuple(seq_slot.shape)}")
+        return self._ptr(seq_to, "seq_to", (torch.int32,))
 
     def _product(self, m, n, k, packed, activation):
         """What the library says of a product of these sizes, asked once per shape: (blocks its activations are
@@ -1129,10 +1138,11 @@ class HipKernels(KernelSizes):
 
     # ---- linear attention with a decay, as a recurrence over a float32 state ----
     def lightning_scan(self, proj, q_off, k_off, v_off, state, decay, seq_start, seq_slot, out, n_heads, dim, vdim,
-                       max_rows_per_seq=None):
+                       max_rows_per_seq=None, seq_to=None):
         """For every sequence b of the step (rows seq_start[b] .. seq_start[b + 1] - 1 in order, state row seq_slot[b]) and
         head h: S <- decay[h] * S + k_t v_t^T, out_t = S^T q_t with q, k, v = silu of the row's slices from q_off, k_off,
-        v_off of `proj` [n, P].  state f32 [slots, H, dim, vdim] in place, out f32 [n, H * vdim].  `max_rows_per_seq`: no
+        v_off of `proj` [n, P].  state f32 [slots, H, dim, vdim] in place, or, as in all kernels that take `seq_to`, left in these rows (in
+        none of which a sequence of the step starts), out f32 [n, H * vdim].  `max_rows_per_seq`: no
         sequence of the step brings more rows (the step's total, if it is not given); long sequences go as products of matrices
         over chunks of rows where the sizes allow it, or, where they would leave the chip idle, are cut into chunks that are walked
         side by side; the chunks' states take scratch memory for the length of the call."""
@@ -1155,7 +1165,7 @@ class HipKernels(KernelSizes):
         self._check(entry(
             self._ptr(proj, "lightning proj"), _code(proj, "lightning proj"), stride, int(q_off), int(k_off), int(v_off),
             self._ptr(state, "lightning state", f32), self._ptr(decay, "lightning decay", f32),
-            self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._ptr(out, "lightning out", f32),
+            self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot), self._ptr(out, "lightning out", f32),
             n_seqs, n_rows, most, n_heads, dim, vdim, self._ptr(scratch, "chunk states", f32, True),
             scratch.numel() if scratch is not None else 0, self._stream()))
 
@@ -1174,7 +1184,7 @@ class HipKernels(KernelSizes):
 
     # ---- gated linear attention: a matrix state whose rows decay by factors that the token sets ----
     def gla_scan(self, proj, q_off, k_off, v_off, z, bias, tau, q_scale, state, seq_start, seq_slot, out, n_heads, dim, vdim,
-                 max_rows_per_seq=None):
+                 max_rows_per_seq=None, seq_to=None):
         """Per (sequence, head): S <- diag(alpha_t) S + k_t v_t^T, out_t = S^T (q_scale q_t), alpha_t = sigmoid(z_t + bias)^(1/tau),
         over the sequence's rows in order, from and into state[slot].  proj [n, P] holds q, k (H x dim) and v (H x vdim) from the
         given columns; z f32 [n, H dim]; bias f32 [H dim]; state f32 [slots, H, dim, vdim]; out f32 [n, H vdim].
@@ -1197,10 +1207,10 @@ class HipKernels(KernelSizes):
             self._ptr(proj, "gla_scan proj"), _code(proj, "gla_scan proj"), proj.shape[1], int(q_off), int(k_off), int(v_off),
             self._ptr(z, "gla_scan decays", f32), z.shape[1], self._ptr(bias, "gla_scan bias", f32), float(tau), float(q_scale),
             self._ptr(state, "gla_scan state", f32), n_heads * dim * vdim, self._ptr(seq_start, "seq_start", i32),
-            self._ptr(seq_slot, "seq_slot", i32), self._ptr(out, "gla_scan out", f32), n_seqs, n_heads, dim, vdim, n_rows, most,
+            self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot), self._ptr(out, "gla_scan out", f32), n_seqs, n_heads, dim, vdim, n_rows, most,
             chunk_rows, self._ptr(scratch, "gla_scan scratch", f32, True), self._stream()))
 
-    def wkv_scan(self, r, k, v, z, bias, bonus, state, state_offset, seq_start, seq_slot, out, n_heads, dim, vdim, max_rows_per_seq=None):
+    def wkv_scan(self, r, k, v, z, bias, bonus, state, state_offset, seq_start, seq_slot, out, n_heads, dim, vdim, max_rows_per_seq=None, seq_to=None):
         """Per (sequence, head): out_t = (S + diag(bonus) k_t v_t^T)^T r_t, then S <- diag(a_t) S + k_t v_t^T with a_t = exp(-exp(z_t + bias)),
         over the sequence's rows in order, from and into S [H, dim, vdim] f32 at `state_offset` floats into state[slot].  r, k [n, H dim]
         and v [n, H vdim] of one type and one row length (vdim = dim); z f32 [n, H dim]; bias, bonus f32 [H dim]; out f32 [n, H vdim]."""
@@ -1222,10 +1232,10 @@ class HipKernels(KernelSizes):
         self._check(self.lib.bh_wkv_scan(
             self._ptr(r, "wkv_scan r"), self._ptr(k, "wkv_scan k"), self._ptr(v, "wkv_scan v"), _code(r, "wkv_scan r"), width,
             self._ptr(z, "wkv_scan decays", f32), z.shape[1], self._ptr(bias, "wkv_scan bias", f32), self._ptr(bonus, "wkv_scan bonus", f32),
-            where, stride, self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._ptr(out, "wkv_scan out", f32),
+            where, stride, self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot), self._ptr(out, "wkv_scan out", f32),
             n_seqs, n_heads, dim, vdim, n_rows, most, chunk_rows, self._ptr(scratch, "wkv_scan scratch", f32, True), self._stream()))
 
-    def token_shift(self, h, mu, state, state_offset, row_seq, seq_start, seq_slot, outs):
+    def token_shift(self, h, mu, state, state_offset, row_seq, seq_start, seq_slot, outs, seq_to=None):
         """outs[s] = h + (h' - h) * mu[s], h' the row before in a row's sequence, or what state[slot] keeps (`state_offset` floats in) for a
         sequence's first row, where its last row of the step is left; h [n, D] (rows or `BlockedRows`), mu f32 [S, D], outs like h, all
         in one form."""
@@ -1240,7 +1250,7 @@ class HipKernels(KernelSizes):
         i32 = (torch.int32,)
         self._check(self.lib.bh_token_shift(
             self._ptr(h, "token_shift h"), _code(h, "token_shift h"), _block_rows(h), self._ptr(mu, "token_shift mu", (torch.float32,)), mixes,
-            where, stride, self._ptr(row_seq, "row_seq", i32), self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32),
+            where, stride, self._ptr(row_seq, "row_seq", i32), self._ptr(seq_start, "seq_start", i32), self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot),
             to, _block_rows(outs[0]), n_rows, width, self._stream()))
 
     def tanh_rows(self, x, out):
@@ -1278,7 +1288,7 @@ class HipKernels(KernelSizes):
             self._ptr(seq_slot, "seq_slot", i32), self._ptr(qkv, "delta q, k, v", f32), self._ptr(beside, "delta gates", f32), n_rows, n_heads,
             n_groups, dim, vdim, self._stream()))
 
-    def delta_scan(self, qkv, beside, state, seq_start, seq_slot, out, n_heads, n_groups, dim, vdim, max_rows_per_seq=None):
+    def delta_scan(self, qkv, beside, state, seq_start, seq_slot, out, n_heads, n_groups, dim, vdim, max_rows_per_seq=None, seq_to=None):
         """Per (sequence, head), its rows in order, from and into S [H, dim, vdim] f32 at the start of state[slot]: S <- g S, u = beta (v -
         S^T k), S <- S + k u^T, out = S^T q, of what `delta_prep` left; out f32 [n, H vdim].  `max_rows_per_seq` (the rows of the step's
         longest sequence; all rows where it is not said) lets long sequences be walked in chunks side by side, with scratch memory for
@@ -1298,11 +1308,11 @@ class HipKernels(KernelSizes):
         self._ptr(state, "delta_scan state", f32)
         self._check(self.lib.bh_delta_scan(
             self._ptr(qkv, "delta q, k, v", f32), self._ptr(beside, "delta gates", f32), where, stride, self._ptr(seq_start, "seq_start", i32),
-            self._ptr(seq_slot, "seq_slot", i32), self._ptr(out, "delta out", f32), n_seqs, n_heads, n_groups, dim, vdim, n_rows, most, chunk_rows,
+            self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot), self._ptr(out, "delta out", f32), n_seqs, n_heads, n_groups, dim, vdim, n_rows, most, chunk_rows,
             self._ptr(scratch, "delta scratch", f32, True), self._stream()))
 
     def delta_step(self, proj, first, g_first, b_first, a_first, conv_weight, state, conv_offset, a_log, dt_bias, seq_slot, norm_weight, eps, out,
-                   n_heads, n_groups, dim, vdim):
+                   n_heads, n_groups, dim, vdim, seq_to=None):
         """`delta_prep`, the convolution's state, `delta_scan` and the heads' gated norm in one launch for a step of one row a sequence (rows
         in the order of seq_slot): out [n, H vdim] (rows or `BlockedRows`) = rms(o per head) * norm_weight * silu(g), g from column
         g_first; norm_weight f32 [H vdim].  Returns False, having done nothing, where the kernel does not take heads of these sizes."""
@@ -1319,7 +1329,7 @@ class HipKernels(KernelSizes):
         self._check(self.lib.bh_delta_step(
             self._ptr(proj, "delta_step proj"), _code(proj, "delta_step proj"), proj.shape[1], int(first), int(g_first), int(b_first), int(a_first),
             self._ptr(conv_weight, "conv weight", f32), taps, where, stride, int(conv_offset), self._ptr(a_log, "A_log", f32),
-            self._ptr(dt_bias, "dt_bias", f32), self._ptr(seq_slot, "seq_slot", i32), self._ptr(norm_weight, "norm weight", f32), float(eps),
+            self._ptr(dt_bias, "dt_bias", f32), self._ptr(seq_slot, "seq_slot", i32), self._rows_to(seq_to, seq_slot), self._ptr(norm_weight, "norm weight", f32), float(eps),
             self._ptr(out, "delta_step out"), _block_rows(out), n_rows, n_heads, n_groups, dim, vdim, self._stream()))
         return True
 
@@ -1624,7 +1634,7 @@ class HipKernels(KernelSizes):
             self._ptr(seq_slot, "seq_slot", (torch.int32,)), self._ptr(out, "short_conv out", (torch.float32,)), n_rows, channels,
             taps, int(bool(silu)), self._stream()))
 
-    def short_conv_state(self, u, first, channels, taps, state, state_offset, seq_start, seq_slot):
+    def short_conv_state(self, u, first, channels, taps, state, state_offset, seq_start, seq_slot, seq_to=None):
         """The state after the step: the last taps - 1 inputs of every sequence (old ones where the step brought fewer)."""
         n_seqs = seq_slot.shape[0]
         if seq_start.shape != (n_seqs + 1,):
@@ -1633,7 +1643,7 @@ class HipKernels(KernelSizes):
         self._ptr(state, "short_conv state", (torch.float32,))
         self._check(self.lib.bh_short_conv_state(
             self._ptr(u, "short_conv_state u"), _code(u, "short_conv_state u"), u.shape[1], int(first), where, stride,
-            self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)), n_seqs, int(channels),
+            self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)), self._rows_to(seq_to, seq_slot), n_seqs, int(channels),
             int(taps), self._stream()))
 
     # ---- attention with queries and keys normed over the whole projection ----
@@ -1714,7 +1724,7 @@ class HipKernels(KernelSizes):
 
     # ---- a state-space recurrence with a scalar decay per head ----
     def ssm_scan(self, xbc, proj, dt_first, dt_bias, a_log, d_skip, state, state_offset, seq_start, seq_slot, out, n_heads, vdim,
-                 n_state, n_groups, max_rows_per_seq=None):
+                 n_state, n_groups, max_rows_per_seq=None, seq_to=None):
         """Per (sequence, head): S <- exp(-exp(a_log) dt) S + dt B x^T, y = S^T C + d_skip x with dt = softplus(proj[:, dt_first
         + head] + dt_bias); xbc f32 [n, H vdim + 2 G N] = [x | B | C], S [H, N, vdim] f32 at `state_offset` floats into
         state[slot], out f32 [n, H vdim].  `max_rows_per_seq` (the most rows any sequence brings; the step's rows if not
@@ -1730,7 +1740,7 @@ class HipKernels(KernelSizes):
         common = (self._ptr(xbc, "ssm_scan xbc", (torch.float32,)), xbc.shape[1], self._ptr(proj, "ssm_scan proj"), _code(proj, "ssm_scan proj"),
                   proj.shape[1], int(dt_first), self._ptr(dt_bias, "dt_bias", (torch.float32,)), self._ptr(a_log, "A_log", (torch.float32,)),
                   self._ptr(d_skip, "D", (torch.float32,)), where, stride)
-        rest = (self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)),
+        rest = (self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)), self._rows_to(seq_to, seq_slot),
                 self._ptr(out, "ssm_scan out", (torch.float32,)), n_seqs, n_heads, vdim, n_state, n_groups)
         most = int(max_rows_per_seq) if max_rows_per_seq else n_rows
         floats = 0

@@ -83,6 +83,8 @@ class CacheNeed:
                   convolution ahead of the keys, say), under the rules of kind "state".
     kind "state": one tensor of `state_shape` and `state_dtype` per sequence, of fixed size,
                   zero when a sequence starts.
+    `in_banks`: the part leaves the state a step moves on in the rows it is told to (`LayerCache.state_rows`), all of
+    each row, and reads it from others: a cache may then keep two rows a sequence.
     Layers whose needs are equal share one storage group.
     """
     kind: str
@@ -91,6 +93,7 @@ class CacheNeed:
     window: int = 0
     state_shape: tuple = ()
     state_dtype: torch.dtype = torch.float32
+    in_banks: bool = False
 
     def __post_init__(self):
         if self.kind not in ("kv", "state"):
@@ -135,6 +138,8 @@ class StepContext:
     max_position: int                      # largest absolute position in this step
     max_rows_per_seq: int = 1              # most tokens any one sequence brings
     token_src: torch.Tensor | None = None  # int32 [T]: >= 0 where a row's token is fed_tokens[token_src[row]]
+    state_from: torch.Tensor | None = None # int32 [B]: the row in which each sequence's state stands, in a cache with two rows a slot
+    state_to: torch.Tensor | None = None   # int32 [B]: the row in which the step leaves it
     fed_tokens: torch.Tensor | None = None # int32: tokens chosen on the device that the host has not read yet
     extras: dict = field(default_factory=dict)
     shared: dict = field(default_factory=dict)   # what a part makes once a forward for the parts after it (rotation angles of the rows); emptied by the model at both ends
@@ -217,6 +222,11 @@ class LayerCache:
     v_pages: torch.Tensor | None = None
     page_table: torch.Tensor | None = None
     state: torch.Tensor | None = None
+    banked: bool = False      # two rows of `state` a slot: index it with `state_rows` instead
+
+    def state_rows(self, ctx):
+        """(rows to read the state from, keywords that say in which rows a kernel leaves it, none where these are the same)."""
+        return (ctx.state_from, {"seq_to": ctx.state_to}) if self.banked else (ctx.seq_slot, {})
 
 
 # ---- registries ---------------------------------------------------------------------------------

@@ -82,7 +82,7 @@ class ConvGatedAttention:
 
     def cache_need(self):
         state = ((self.taps - 1) * self.conv_width,) if self.taps > 1 else ()
-        return CacheNeed(kind="kv", kv_heads=self.n_kv_heads, head_dim=self.pad, state_shape=state, state_dtype=torch.float32)
+        return CacheNeed(kind="kv", kv_heads=self.n_kv_heads, head_dim=self.pad, state_shape=state, state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         total = self.proj.working_bytes(step, step.rows)
@@ -99,21 +99,22 @@ class ConvGatedAttention:
         n = ctx.n_rows
         proj = self.proj.forward(ctx, x)
         state = cache.state if self.taps > 1 else None
+        rows, to = cache.state_rows(ctx)
         q = ctx.new_activations(n, self.n_heads * self.pad)
         freq = self.rotation.frequencies(ctx.device) if self.rotation is not None else None
         in_one = getattr(k, "conv_norm_rope_write", None)      # convolution, norm, rotation and cache write in one launch
         if in_one is not None:
-            in_one(proj, 0, self.conv_weight if self.taps else None, state, 0, ctx.seq_start, ctx.seq_slot, self.q_norm, self.k_norm,
+            in_one(proj, 0, self.conv_weight if self.taps else None, state, 0, ctx.seq_start, rows, self.q_norm, self.k_norm,
                    self.norm_eps, freq, self.turned, ctx.positions, ctx.row_seq, q, cache.k_pages, cache.v_pages, cache.page_table,
                    self.n_heads, self.n_kv_heads, self.dim, self.vdim, self.pad, cache.writes)
         else:
             conv = ctx.new_f32(n, self.conv_width)
-            k.short_conv(proj, 0, self.conv_weight, None, state, 0, ctx.row_seq, ctx.seq_start, ctx.seq_slot, conv)
+            k.short_conv(proj, 0, self.conv_weight, None, state, 0, ctx.row_seq, ctx.seq_start, rows, conv)
             k.whole_norm_rope_write(conv, self.q_norm, self.k_norm, self.norm_eps, freq, self.turned, ctx.positions, ctx.row_seq, q,
                                     cache.k_pages, cache.v_pages, cache.page_table, self.n_heads, self.n_kv_heads, self.dim, self.vdim,
                                     self.pad, cache.writes)
         if state is not None and cache.writes:      # after every reader of the old state
-            k.short_conv_state(proj, 0, self.conv_width, self.taps, state, 0, ctx.seq_start, ctx.seq_slot)
+            k.short_conv_state(proj, 0, self.conv_width, self.taps, state, 0, ctx.seq_start, rows, **to)
         attended = ctx.new_activations(n, self.n_heads * self.pad)
         k.attention(q, attended, cache.k_pages, cache.v_pages, cache.page_table, ctx.row_seq, ctx.positions, self.n_heads,
                     self.n_kv_heads, self.pad, self.scale, 0, layout=ctx)

@@ -75,7 +75,7 @@ class GatedDeltaRule:
         self.out.prepare(kernels)
 
     def cache_need(self):
-        return CacheNeed(kind="state", state_shape=(self.state_floats + (self.taps - 1) * self.channels,), state_dtype=torch.float32)
+        return CacheNeed(kind="state", state_shape=(self.state_floats + (self.taps - 1) * self.channels,), state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         chunks = 0
@@ -92,17 +92,18 @@ class GatedDeltaRule:
         proj = self.proj.forward(ctx, x)
         gated = ctx.new_activations(n, self.value_width, reader=self.out.reader())
         sizes = (self.n_heads, self.n_groups, self.dim, self.vdim)
+        rows, to = cache.state_rows(ctx)
         one_launch = getattr(k, "delta_step", None)
         if not (one_launch is not None and ctx.max_rows_per_seq == 1 and one_launch(
                 proj, 0, self.g_first, self.b_first, self.a_first, self.conv_weight, cache.state, self.state_floats, self.a_log, self.dt_bias,
-                ctx.seq_slot, self.norm_weight, self.norm_eps, gated, *sizes)):
+                rows, self.norm_weight, self.norm_eps, gated, *sizes, **to)):
             qkv, beside = ctx.new_f32(n, self.channels), ctx.new_f32(n, 4 * self.n_heads)
             k.delta_prep(proj, 0, self.b_first, self.a_first, self.conv_weight, cache.state, self.state_floats, self.a_log, self.dt_bias, ctx.row_seq,
-                         ctx.seq_start, ctx.seq_slot, qkv, beside, *sizes)
+                         ctx.seq_start, rows, qkv, beside, *sizes)
             if self.taps > 1:      # after every reader of the old state
-                k.short_conv_state(proj, 0, self.channels, self.taps, cache.state, self.state_floats, ctx.seq_start, ctx.seq_slot)
+                k.short_conv_state(proj, 0, self.channels, self.taps, cache.state, self.state_floats, ctx.seq_start, rows, **to)
             read = ctx.new_f32(n, self.value_width)
-            k.delta_scan(qkv, beside, cache.state, ctx.seq_start, ctx.seq_slot, read, *sizes, max_rows_per_seq=ctx.max_rows_per_seq)
+            k.delta_scan(qkv, beside, cache.state, ctx.seq_start, rows, read, *sizes, max_rows_per_seq=ctx.max_rows_per_seq, **to)
             k.gated_group_rmsnorm(read, proj, self.g_first, self.norm_weight, self.norm_eps, gated, self.n_heads, gate_after=True)
         self.out.forward(ctx, gated, out=hidden, accumulate=not fresh)
         return None

@@ -60,7 +60,7 @@ class GatedLinearAttention:
             linear.prepare(kernels)
 
     def cache_need(self):
-        return CacheNeed(kind="state", state_shape=(self.n_heads, self.dim, self.vdim), state_dtype=torch.float32)
+        return CacheNeed(kind="state", state_shape=(self.n_heads, self.dim, self.vdim), state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         width = self.n_heads * self.vdim
@@ -78,8 +78,9 @@ class GatedLinearAttention:
         proj = self.proj.forward(ctx, x)
         decays = self.decay_up.forward(ctx, self.decay_down.forward(ctx, x), out_dtype=torch.float32)
         mixed = ctx.new_f32(ctx.n_rows, width)
+        rows, to = cache.state_rows(ctx)
         k.gla_scan(proj, self.q_off, self.k_off, self.v_off, decays, self.decay_bias, self.tau, self.dim ** -0.5, cache.state,
-                   ctx.seq_start, ctx.seq_slot, mixed, self.n_heads, self.dim, self.vdim, max_rows_per_seq=ctx.max_rows_per_seq)
+                   ctx.seq_start, rows, mixed, self.n_heads, self.dim, self.vdim, max_rows_per_seq=ctx.max_rows_per_seq, **to)
         gated = ctx.new_activations(ctx.n_rows, width, reader=self.out.reader())
         k.gated_group_rmsnorm(mixed, proj, self.g_off, self.norm_weight, self.norm_eps, gated, self.n_heads, gate_after=True)
         self.out.forward(ctx, gated, out=hidden, accumulate=not fresh)

@@ -58,7 +58,7 @@ class LightningAttention:
         self.out.prepare(kernels)
 
     def cache_need(self):
-        return CacheNeed(kind="state", state_shape=(self.n_heads, self.dim, self.vdim), state_dtype=torch.float32)
+        return CacheNeed(kind="state", state_shape=(self.n_heads, self.dim, self.vdim), state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         width = self.n_heads * self.vdim
@@ -74,8 +74,9 @@ class LightningAttention:
         width = self.n_heads * self.vdim
         proj = self.proj.forward(ctx, x)
         mixed = ctx.new_f32(ctx.n_rows, width)
-        k.lightning_scan(proj, self.q_off, self.k_off, self.v_off, cache.state, self.decay, ctx.seq_start, ctx.seq_slot,
-                         mixed, self.n_heads, self.dim, self.vdim, max_rows_per_seq=ctx.max_rows_per_seq)
+        rows, to = cache.state_rows(ctx)
+        k.lightning_scan(proj, self.q_off, self.k_off, self.v_off, cache.state, self.decay, ctx.seq_start, rows,
+                         mixed, self.n_heads, self.dim, self.vdim, max_rows_per_seq=ctx.max_rows_per_seq, **to)
         gated = ctx.new_activations(ctx.n_rows, width, reader=self.out.reader())
         k.gated_rmsnorm(mixed, proj, self.g_off, self.norm_weight, self.norm_eps, gated)
         self.out.forward(ctx, gated, out=hidden, accumulate=not fresh)

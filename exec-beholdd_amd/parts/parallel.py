@@ -33,7 +33,7 @@ class ParallelMixers:
             raise ValueError("mixers side by side: at most one of them keeps pages and at most one a state")
         if paged and fixed:
             self._need = CacheNeed(kind="kv", kv_heads=paged[0].kv_heads, head_dim=paged[0].head_dim, window=paged[0].window,
-                                   state_shape=fixed[0].state_shape, state_dtype=fixed[0].state_dtype)
+                                   state_shape=fixed[0].state_shape, state_dtype=fixed[0].state_dtype, in_banks=fixed[0].in_banks)
         else:
             self._need = (paged or fixed or [None])[0]
 

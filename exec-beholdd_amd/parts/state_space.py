@@ -65,7 +65,7 @@ class StateSpaceScan:
         self.out.prepare(kernels)
 
     def cache_need(self):
-        return CacheNeed(kind="state", state_shape=(self.state_floats + (self.taps - 1) * self.conv_width,), state_dtype=torch.float32)
+        return CacheNeed(kind="state", state_shape=(self.state_floats + (self.taps - 1) * self.conv_width,), state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         chunks = 0
@@ -80,13 +80,14 @@ class StateSpaceScan:
         n = ctx.n_rows
         proj = self.proj.forward(ctx, x)
         xbc = ctx.new_f32(n, self.conv_width)
+        rows, to = cache.state_rows(ctx)
         k.short_conv(proj, self.inner, self.conv_weight, self.conv_bias, cache.state, self.state_floats, ctx.row_seq, ctx.seq_start,
-                     ctx.seq_slot, xbc, silu=True)
+                     rows, xbc, silu=True)
         if self.taps > 1:
-            k.short_conv_state(proj, self.inner, self.conv_width, self.taps, cache.state, self.state_floats, ctx.seq_start, ctx.seq_slot)
+            k.short_conv_state(proj, self.inner, self.conv_width, self.taps, cache.state, self.state_floats, ctx.seq_start, rows, **to)
         y = ctx.new_f32(n, self.inner)
-        k.ssm_scan(xbc, proj, self.dt_first, self.dt_bias, self.a_log, self.d_skip, cache.state, 0, ctx.seq_start, ctx.seq_slot, y,
-                   self.n_heads, self.vdim, self.n_state, self.n_groups, max_rows_per_seq=ctx.max_rows_per_seq)
+        k.ssm_scan(xbc, proj, self.dt_first, self.dt_bias, self.a_log, self.d_skip, cache.state, 0, ctx.seq_start, rows, y,
+                   self.n_heads, self.vdim, self.n_state, self.n_groups, max_rows_per_seq=ctx.max_rows_per_seq, **to)
         normed = ctx.new_activations(n, self.inner, reader=self.out.reader())
         k.gated_group_rmsnorm(y, proj, 0, self.norm_weight, self.norm_eps, normed, self.norm_groups)
         self.out.forward(ctx, normed, out=hidden, accumulate=True)

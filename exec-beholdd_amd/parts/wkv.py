@@ -63,7 +63,7 @@ class TimeMixing:
             linear.prepare(kernels)
 
     def cache_need(self):
-        return CacheNeed(kind="state", state_shape=(self.state_floats + self.hidden,), state_dtype=torch.float32)
+        return CacheNeed(kind="state", state_shape=(self.state_floats + self.hidden,), state_dtype=torch.float32, in_banks=True)
 
     def working_bytes(self, step) -> int:
         chunks = 0
@@ -81,15 +81,16 @@ class TimeMixing:
         n = ctx.n_rows
         reader = self.projections["r"].reader()
         mixed = {name: ctx.new_activations(n, self.hidden, reader=reader) for name in self.MIXES}
-        k.token_shift(x, self.mu, cache.state, self.state_floats, ctx.row_seq, ctx.seq_start, ctx.seq_slot, [mixed[name] for name in self.MIXES])
+        rows, to = cache.state_rows(ctx)
+        k.token_shift(x, self.mu, cache.state, self.state_floats, ctx.row_seq, ctx.seq_start, rows, [mixed[name] for name in self.MIXES], **to)
         projected = {name: linear.forward(ctx, mixed[name]) for name, linear in self.projections.items()}
         low = self.decay_down.forward(ctx, mixed["w"], out_dtype=torch.float32)
         bent = ctx.new_activations(n, self.decay_rank, reader=self.decay_up.reader())
         k.tanh_rows(low, bent)
         decays = self.decay_up.forward(ctx, bent, out_dtype=torch.float32)
         read = ctx.new_f32(n, self.width)
-        k.wkv_scan(projected["r"], projected["k"], projected["v"], decays, self.decay_bias, self.bonus, cache.state, 0, ctx.seq_start, ctx.seq_slot,
-                   read, self.n_heads, self.dim, self.dim, max_rows_per_seq=ctx.max_rows_per_seq)
+        k.wkv_scan(projected["r"], projected["k"], projected["v"], decays, self.decay_bias, self.bonus, cache.state, 0, ctx.seq_start, rows,
+                   read, self.n_heads, self.dim, self.dim, max_rows_per_seq=ctx.max_rows_per_seq, **to)
         gated = ctx.new_activations(n, self.width, reader=self.out.reader())
         k.gated_group_rmsnorm(read, projected["g"], 0, self.norm_weight, self.norm_eps, gated, self.n_heads, gate_after=True)
         self.out.forward(ctx, gated, out=hidden, accumulate=not fresh)
