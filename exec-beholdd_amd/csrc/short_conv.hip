@@ -6,17 +6,16 @@
 //                     those it is read from
 // State of one sequence: [taps - 1][channels] float32, the oldest input first, at `state + slot * slot_stride`.
 // Sums are float32; the result is float32.
-#include "common.h"
-
-#define SC_MAX_TAPS 16
+//                     A step that leaves it in other rows does so in short_conv itself (seq_to): the thread of a sequence's last row
+#include "short_conv.h"
 
 template <typename T>
 __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ u, int row_stride, int first,
                                                          const float* __restrict__ w, const float* __restrict__ bias,
-                                                         const float* __restrict__ state, long slot_stride,
+                                                         float* __restrict__ state, long slot_stride,
                                                          const int32_t* __restrict__ row_seq, const int32_t* __restrict__ seq_start,
-                                                         const int32_t* __restrict__ seq_slot, float* __restrict__ out,
-                                                         int n_rows, int channels, int taps, int silu) {
+                                                         const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
+                                                         float* __restrict__ out, int n_rows, int channels, int taps, int silu) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= channels) return;
   float wc[SC_MAX_TAPS];
@@ -39,6 +38,8 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ u
     }
     if (silu) acc = acc / (1.0f + expf(-acc));
     out[(size_t)row * channels + c] = acc;
+    if (seq_to && row + 1 == seq_start[seq + 1])
+      sc_leave_inputs(u, row_stride, first + c, row - t, t + 1, taps, old, state + (size_t)seq_to[seq] * slot_stride, channels, c);
   }
 }
 
@@ -50,10 +51,10 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ u
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void short_conv_walk_kernel(const T* __restrict__ u, int row_stride, int first,
                                                               const float* __restrict__ w, const float* __restrict__ bias,
-                                                              const float* __restrict__ state, long slot_stride,
+                                                              float* __restrict__ state, long slot_stride,
                                                               const int32_t* __restrict__ row_seq, const int32_t* __restrict__ seq_start,
-                                                              const int32_t* __restrict__ seq_slot, float* __restrict__ out,
-                                                              int n_rows, int channels, int silu) {
+                                                              const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
+                                                              float* __restrict__ out, int n_rows, int channels, int silu) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= channels) return;
   float wc[TAPS], win[TAPS];
@@ -83,12 +84,19 @@ __global__ __launch_bounds__(256) void short_conv_walk_kernel(const T* __restric
     for (int j = 0; j < TAPS; ++j) acc = fmaf(wc[j], win[j], acc);
     if (silu) acc = acc / (1.0f + expf(-acc));
     out[(size_t)row * channels + c] = acc;
+    if (seq_to && row + 1 == seq_start[seq + 1]) {      // the window's later inputs are what the next step starts with
+      float* to = state + (size_t)seq_to[seq] * slot_stride;
+#pragma unroll
+      for (int j = 1; j < TAPS; ++j) to[(size_t)(j - 1) * channels + c] = win[j];
+    }
   }
 }
 
+// seq_to [n_seqs]: the rows of the state to leave what the next step starts with in, none of which this step reads; or null: short_conv_state
+// does it.
 extern "C" int bh_short_conv(const void* u, int dtype, int row_stride, int first, const float* w, const float* bias,
-                             const float* state, long slot_stride, const int32_t* row_seq, const int32_t* seq_start,
-                             const int32_t* seq_slot, float* out, int n_rows, int channels, int taps, int silu,
+                             float* state, long slot_stride, const int32_t* row_seq, const int32_t* seq_start,
+                             const int32_t* seq_slot, const int32_t* seq_to, float* out, int n_rows, int channels, int taps, int silu,
                              hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && channels > 0, "short_conv: sizes must be positive");
   BH_REQUIRE(taps >= 1 && taps <= SC_MAX_TAPS, "short_conv: 1 to %d taps, got %d", SC_MAX_TAPS, taps);
@@ -99,7 +107,7 @@ extern "C" int bh_short_conv(const void* u, int dtype, int row_stride, int first
     dim3 walk((channels + 255) / 256, (n_rows + SC_ROWS - 1) / SC_ROWS);
 #define BH_SW(T, TAPS)                                                                                                              \
   short_conv_walk_kernel<T, TAPS><<<walk, 256, 0, stream>>>((const T*)u, row_stride, first, w, bias, state, slot_stride, row_seq, seq_start, \
-                                                            seq_slot, out, n_rows, channels, silu)
+                                                            seq_slot, seq_to, out, n_rows, channels, silu)
     if (dtype == BH_F32) {
       if (taps == 2) BH_SW(float, 2);
       else if (taps == 3) BH_SW(float, 3);
@@ -115,10 +123,10 @@ extern "C" int bh_short_conv(const void* u, int dtype, int row_stride, int first
   dim3 grid((channels + 255) / 256, n_rows < 4096 ? n_rows : 4096);
   if (dtype == BH_F32)
     short_conv_kernel<float><<<grid, 256, 0, stream>>>((const float*)u, row_stride, first, w, bias, state, slot_stride, row_seq,
-                                                       seq_start, seq_slot, out, n_rows, channels, taps, silu);
+                                                       seq_start, seq_slot, seq_to, out, n_rows, channels, taps, silu);
   else if (dtype == BH_BF16)
     short_conv_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)u, row_stride, first, w, bias, state, slot_stride, row_seq,
-                                                        seq_start, seq_slot, out, n_rows, channels, taps, silu);
+                                                        seq_start, seq_slot, seq_to, out, n_rows, channels, taps, silu);
   else
     return bh_fail("short_conv: unknown dtype %d", dtype);
   return bh_check_launch("short_conv");
@@ -132,21 +140,9 @@ __global__ __launch_bounds__(256) void short_conv_state_kernel(const T* __restri
                                                                const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to, int channels, int taps) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, seq = blockIdx.y;
   if (c >= channels) return;
-  const int start = seq_start[seq], n_new = seq_start[seq + 1] - start, keep = taps - 1;
-  const float* mine = state + (size_t)seq_slot[seq] * slot_stride;
-  float* left = state + (size_t)seq_to[seq] * slot_stride;
-  float next[SC_MAX_TAPS];
-#pragma unroll
-  for (int s = 0; s < SC_MAX_TAPS; ++s) {
-    if (s >= keep) break;
-    const int at = n_new + s - keep;        // index into the step's rows; negative: still an old input
-    next[s] = at >= 0 ? to_f32(u[(size_t)(start + at) * row_stride + first + c]) : mine[(size_t)(n_new + s) * channels + c];
-  }
-#pragma unroll
-  for (int s = 0; s < SC_MAX_TAPS; ++s) {
-    if (s >= keep) break;
-    left[(size_t)s * channels + c] = next[s];
-  }
+  const int start = seq_start[seq], n_new = seq_start[seq + 1] - start;
+  sc_leave_inputs(u, row_stride, first + c, start, n_new, taps, state + (size_t)seq_slot[seq] * slot_stride, state + (size_t)seq_to[seq] * slot_stride,
+                  channels, c);
 }
 
 extern "C" int bh_short_conv_state(const void* u, int dtype, int row_stride, int first, float* state, long slot_stride,

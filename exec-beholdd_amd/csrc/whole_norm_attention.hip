@@ -10,7 +10,7 @@
 //   gate_heads              out[row][h][i] = attended[row][h][i] * sigmoid(gate[row][h][i]) for i < vdim; the gate may be one
 //                           number a head (gate[row][h]) or absent (the heads' first vdim elements are put side by side)
 // Statistics, angles, cosines and sines are float32; the angle is the float32 product position * freq[i].
-#include "common.h"
+#include "short_conv.h"
 
 template <typename T>
 __global__ __launch_bounds__(256) void whole_norm_rope_write_kernel(
@@ -113,10 +113,13 @@ extern "C" int bh_whole_norm_rope_write(const float* qkv, const float* wq, const
 // The same from the projected rows themselves: the short convolution over time (csrc/short_conv.hip has its definition and
 // its state) is made on the way, a row's convolved channels stand in LDS as float32 and are never written to memory.
 // proj [n_rows][row_stride]: a row holds, from `first`, q, k and v; w_conv [q + k + v channels][taps] (taps 0: no convolution).
-template <typename T>
+// TAPS: four, whose loads are all asked for before the first is used, of a whole thread's channels where these are up to four (16 rows of 3,072
+// channels 9.8 us, 11.9 with a trip to memory a tap), or 0: any number.  seq_to: as in short_conv.hip.
+template <typename T, int TAPS>
 __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
-    const T* __restrict__ proj, int row_stride, int first, const float* __restrict__ w_conv, int taps, const float* __restrict__ state,
-    long slot_stride, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const float* __restrict__ wq,
+    const T* __restrict__ proj, int row_stride, int first, const float* __restrict__ w_conv, int taps, float* __restrict__ state,
+    long slot_stride, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
+    const float* __restrict__ wq,
     const float* __restrict__ wk, float eps, const float* __restrict__ freq, int turned, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ row_seq, T* __restrict__ q_out, T* __restrict__ k_pages, T* __restrict__ v_pages,
     const int32_t* __restrict__ page_table, int table_stride, int H, int G, int dim, int vdim, int pad, int kv_order, int write) {
@@ -135,6 +138,54 @@ __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
     sines[i] = sinf(angle);
   }
   float ss_q = 0.f, ss_k = 0.f;
+  const bool leaves = seq_to && row + 1 == seq_start[seq + 1];
+  float* left = leaves ? state + (size_t)seq_to[seq] * slot_stride : nullptr;
+  auto put = [&](int c, float acc) {
+    conv[c] = acc;
+    if (c < q_width) ss_q += acc * acc;
+    else if (c < q_width + k_width) ss_k += acc * acc;
+  };
+  if constexpr (TAPS > 0) {
+    constexpr int TOGETHER = 4;      // channels a thread
+    for (int c0 = threadIdx.x; c0 < channels; c0 += TOGETHER * blockDim.x) {
+      // (a row's input and an old one are both asked for, wherever they lie, and the one that counts is taken: no load waits for a branch)
+      T now[TOGETHER][TAPS];
+      float before[TOGETHER][TAPS], w[TOGETHER][TAPS], u[TOGETHER][TAPS];
+#pragma unroll
+      for (int i = 0; i < TOGETHER; ++i) {
+        const int c = min(c0 + i * (int)blockDim.x, channels - 1);
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+          const int back = TAPS - 1 - j;
+          w[i][j] = w_conv[(size_t)c * TAPS + j];
+          now[i][j] = proj[(size_t)(row - min(back, t)) * row_stride + first + c];
+          before[i][j] = 0.f;
+        }
+      }
+      if (t < TAPS - 1) {
+#pragma unroll
+        for (int i = 0; i < TOGETHER; ++i)
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j) before[i][j] = old[(size_t)min(t + j, TAPS - 2) * channels + min(c0 + i * (int)blockDim.x, channels - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < TOGETHER; ++i) {
+        const int c = c0 + i * (int)blockDim.x;
+        if (c >= channels) break;
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+          u[i][j] = TAPS - 1 - j <= t ? to_f32(now[i][j]) : before[i][j];
+          acc = fmaf(w[i][j], u[i][j], acc);
+        }
+        put(c, acc);
+        if (leaves) {
+#pragma unroll
+          for (int j = 1; j < TAPS; ++j) left[(size_t)(j - 1) * channels + c] = u[i][j];
+        }
+      }
+    }
+  } else
   for (int c = threadIdx.x; c < channels; c += blockDim.x) {
     float acc;
     if (taps <= 1) {
@@ -148,9 +199,8 @@ __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
         acc = fmaf(w_conv[(size_t)c * taps + j], u, acc);
       }
     }
-    conv[c] = acc;
-    if (c < q_width) ss_q += acc * acc;
-    else if (c < q_width + k_width) ss_k += acc * acc;
+    put(c, acc);
+    if (leaves) sc_leave_inputs(proj, row_stride, first + c, row - t, t + 1, taps, old, left, channels, c);
   }
   const float inv_q = 1.0f / sqrtf(block_sum(ss_q, scratch) / (float)q_width + eps);
   const float inv_k = 1.0f / sqrtf(block_sum(ss_k, scratch) / (float)k_width + eps);
@@ -195,8 +245,8 @@ __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
 }
 
 extern "C" int bh_conv_norm_rope_write(const void* proj, int dtype, int row_stride, int first, const float* w_conv, int taps,
-                                       const float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot,
-                                       const float* wq, const float* wk, float eps, const float* freq, int turned,
+                                       float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot,
+                                       const int32_t* seq_to, const float* wq, const float* wk, float eps, const float* freq, int turned,
                                        const int32_t* positions, const int32_t* row_seq, void* q_out, void* k_pages, void* v_pages,
                                        const int32_t* page_table, int table_stride, int n_rows, int H, int G, int dim, int vdim, int pad,
                                        int kv_order, int write, hipStream_t stream) {
@@ -213,16 +263,18 @@ extern "C" int bh_conv_norm_rope_write(const void* proj, int dtype, int row_stri
   const size_t lds = (size_t)(channels + turned) * sizeof(float);
   BH_REQUIRE(lds <= 128 * 1024, "conv_norm_rope_write: %d channels do not fit the local memory", channels);
   const int threads = n_rows < 2 * bh_compute_units() && channels >= 2048 ? 1024 : 256;      // few rows: more of the chip a row
-#define BH_CW(T)                                                                                                                   \
+#define BH_CW(T, TAPS)                                                                                                             \
   do {                                                                                                                             \
-    bh_allow_lds<conv_norm_rope_write_kernel<T>>(lds);                                                                             \
-    conv_norm_rope_write_kernel<T><<<n_rows, threads, lds, stream>>>((const T*)proj, row_stride, first, w_conv, taps, state, slot_stride,  \
-                                                                 seq_start, seq_slot, wq, wk, eps, freq, turned, positions, row_seq, \
+    bh_allow_lds<conv_norm_rope_write_kernel<T, TAPS>>(lds);                                                                       \
+    conv_norm_rope_write_kernel<T, TAPS><<<n_rows, threads, lds, stream>>>((const T*)proj, row_stride, first, w_conv, taps, state, slot_stride,  \
+                                                                 seq_start, seq_slot, seq_to, wq, wk, eps, freq, turned, positions, row_seq, \
                                                                  (T*)q_out, (T*)k_pages, (T*)v_pages, page_table, table_stride, H, G, \
                                                                  dim, vdim, pad, kv_order, write);                                  \
   } while (0)
-  if (dtype == BH_F32) BH_CW(float);
-  else if (dtype == BH_BF16) BH_CW(bf16_t);
+  if (dtype == BH_F32 && taps == 4) BH_CW(float, 4);
+  else if (dtype == BH_F32) BH_CW(float, 0);
+  else if (dtype == BH_BF16 && taps == 4) BH_CW(bf16_t, 4);
+  else if (dtype == BH_BF16) BH_CW(bf16_t, 0);
   else return bh_fail("conv_norm_rope_write: unknown dtype %d", dtype);
 #undef BH_CW
   return bh_check_launch("conv_norm_rope_write");

@@ -202,7 +202,7 @@ class KernelSizes:
             "bh_softcap": [p, ctypes.c_long, f, p],
             "bh_rms_scale_add": [p, p, p, i, i, f, p],
             "bh_gelu_gate_table": [p, i, p, p, p, p, i, i, i, p, i, i, i, p],
-            "bh_short_conv": [p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, p],
+            "bh_short_conv": [p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, p, i, i, i, i, p],
             "bh_short_conv_state": [p, i, i, i, p, ctypes.c_long, p, p, p, i, i, i, p],
             "bh_whole_norm_rope_write": [p, p, p, f, p, i, p, p, p, i, p, p, p, i, i, i, i, i, i, i, i, i, p],
             "bh_gate_heads": [p, i, i, p, i, i, p, i, i, i, i, i, p],
@@ -212,7 +212,7 @@ class KernelSizes:
             "bh_experts_gate_up": [p, i, p, p, p, i, i, i, i, i, f, f, f, p, p],
             "bh_experts_down": [p, i, p, p, p, p, p, i, i, i, i, i, i, p],
             "bh_clamped_glu": [p, i, p, i, i, f, f, i, f, p],
-            "bh_conv_norm_rope_write": [p, i, i, i, p, i, p, ctypes.c_long, p, p, p, p, f, p, i, p, p, p, p, p, p, i, i, i, i, i, i, i, i, i, p],
+            "bh_conv_norm_rope_write": [p, i, i, i, p, i, p, ctypes.c_long, p, p, p, p, p, f, p, i, p, p, p, p, p, p, i, i, i, i, i, i, i, i, i, p],
             "bh_ssm_scan_fast": [p, i, p, i, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, p, p, p, i, i, i, i, i, i, i, p],
             "bh_ssm_chunk_rows": [i, i, i],
             "bh_ssm_fast_takes": [i, i],
@@ -1615,10 +1615,11 @@ class HipKernels(KernelSizes):
             raise KernelError(f"{what}: {floats} floats at {offset} do not lie inside a slot's {per_slot}")
         return state.data_ptr() + 4 * int(offset), per_slot
 
-    def short_conv(self, u, first, weight, bias, state, state_offset, row_seq, seq_start, seq_slot, out, silu=False):
+    def short_conv(self, u, first, weight, bias, state, state_offset, row_seq, seq_start, seq_slot, out, silu=False, seq_to=None):
         """out[t, c] = sum_j weight[c, j] * u[t - taps + 1 + j, first + c] (+ bias[c]) (then silu) over the rows of each
         sequence of the step; inputs before the step come from the sequence's state region ([taps - 1, C] f32 at
-        `state_offset` floats into state[slot]).  u [n, W], weight f32 [C, taps], out f32 [n, C]."""
+        `state_offset` floats into state[slot]).  u [n, W], weight f32 [C, taps], out f32 [n, C].  With `seq_to` the state after the
+        step is left in these rows, none of which the step reads (without: `short_conv_state` moves it on afterwards)."""
         n_rows, channels = out.shape
         taps = weight.shape[1]
         if u.shape[0] != n_rows or weight.shape[0] != channels or (bias is not None and bias.shape != (channels,)):
@@ -1631,8 +1632,8 @@ class HipKernels(KernelSizes):
             self._ptr(u, "short_conv u"), _code(u, "short_conv u"), u.shape[1], int(first),
             self._ptr(weight, "short_conv weight", (torch.float32,)), self._ptr(bias, "short_conv bias", (torch.float32,), True),
             where, stride, self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(seq_start, "seq_start", (torch.int32,)),
-            self._ptr(seq_slot, "seq_slot", (torch.int32,)), self._ptr(out, "short_conv out", (torch.float32,)), n_rows, channels,
-            taps, int(bool(silu)), self._stream()))
+            self._ptr(seq_slot, "seq_slot", (torch.int32,)), self._rows_to(seq_to, seq_slot) if seq_to is not None else None,
+            self._ptr(out, "short_conv out", (torch.float32,)), n_rows, channels, taps, int(bool(silu)), self._stream()))
 
     def short_conv_state(self, u, first, channels, taps, state, state_offset, seq_start, seq_slot, seq_to=None):
         """The state after the step: the last taps - 1 inputs of every sequence (old ones where the step brought fewer)."""
@@ -1673,10 +1674,11 @@ class HipKernels(KernelSizes):
     CONV_ROW_IN_LDS = 30000   # channels of q, k and v together that the one launch keeps in local memory
 
     def conv_norm_rope_write(self, proj, first, conv_weight, state, state_offset, seq_start, seq_slot, q_weight, k_weight, eps, freq,
-                             turned, positions, row_seq, q_out, k_pages, v_pages, page_table, n_heads, n_kv_heads, dim, vdim, pad, write_kv):
+                             turned, positions, row_seq, q_out, k_pages, v_pages, page_table, n_heads, n_kv_heads, dim, vdim, pad, write_kv,
+                             seq_to=None):
         """`short_conv` of the q, k, v channels of `proj` (from column `first`; conv_weight f32 [channels, taps], or None for no
         convolution) and `whole_norm_rope_write` of the result in one launch: the convolved row is never written to memory.  The
-        state is read, not updated (`short_conv_state` afterwards).  A step of many rows runs the two kernels after all: the
+        state is read, not updated (`short_conv_state` afterwards), unless `seq_to` says in which other rows to leave it.  A step of many rows runs the two kernels after all: the
         convolution that walks down the rows loads every input once, where a workgroup per row loads it once per tap."""
         n_rows = proj.shape[0]
         channels = (n_heads + n_kv_heads) * dim + n_kv_heads * vdim
@@ -1684,7 +1686,8 @@ class HipKernels(KernelSizes):
         if walks or channels > self.CONV_ROW_IN_LDS:      # (a row of more channels does not fit the one launch's local memory)
             weight = conv_weight if conv_weight is not None else torch.ones((channels, 1), dtype=torch.float32, device=self.device)
             conv = torch.empty((n_rows, channels), dtype=torch.float32, device=self.device)
-            self.short_conv(proj, first, weight, None, state if weight.shape[1] > 1 else None, state_offset, row_seq, seq_start, seq_slot, conv)
+            self.short_conv(proj, first, weight, None, state if weight.shape[1] > 1 else None, state_offset, row_seq, seq_start, seq_slot, conv,
+                            seq_to=seq_to)
             self.whole_norm_rope_write(conv, q_weight, k_weight, eps, freq, turned, positions, row_seq, q_out, k_pages, v_pages, page_table,
                                        n_heads, n_kv_heads, dim, vdim, pad, write_kv)
             return
@@ -1705,7 +1708,7 @@ class HipKernels(KernelSizes):
         self._check(self.lib.bh_conv_norm_rope_write(
             self._ptr(proj, "proj"), _code(proj, "proj"), proj.shape[1], int(first), self._ptr(conv_weight, "conv weight", (torch.float32,), True),
             taps, where, stride, self._ptr(seq_start, "seq_start", (torch.int32,)), self._ptr(seq_slot, "seq_slot", (torch.int32,)),
-            self._ptr(q_weight, "q norm", (torch.float32,)), self._ptr(k_weight, "k norm", (torch.float32,)), float(eps),
+            self._rows_to(seq_to, seq_slot) if seq_to is not None else None, self._ptr(q_weight, "q norm", (torch.float32,)), self._ptr(k_weight, "k norm", (torch.float32,)), float(eps),
             self._ptr(freq, "frequencies", (torch.float32,), True), int(turned), self._ptr(positions, "positions", (torch.int32,)),
             self._ptr(row_seq, "row_seq", (torch.int32,)), self._ptr(q_out, "q_out"), self._ptr(k_pages, "k_pages"), self._ptr(v_pages, "v_pages"),
             self._ptr(page_table, "page_table", (torch.int32,)), page_table.shape[1], n_rows, n_heads, n_kv_heads, dim, vdim, pad,

@@ -100,21 +100,22 @@ class ConvGatedAttention:
         proj = self.proj.forward(ctx, x)
         state = cache.state if self.taps > 1 else None
         rows, to = cache.state_rows(ctx)
+        leaves = to if state is not None and cache.writes else {}      # rows of their own for the state: whoever convolves leaves it there
         q = ctx.new_activations(n, self.n_heads * self.pad)
         freq = self.rotation.frequencies(ctx.device) if self.rotation is not None else None
         in_one = getattr(k, "conv_norm_rope_write", None)      # convolution, norm, rotation and cache write in one launch
         if in_one is not None:
             in_one(proj, 0, self.conv_weight if self.taps else None, state, 0, ctx.seq_start, rows, self.q_norm, self.k_norm,
                    self.norm_eps, freq, self.turned, ctx.positions, ctx.row_seq, q, cache.k_pages, cache.v_pages, cache.page_table,
-                   self.n_heads, self.n_kv_heads, self.dim, self.vdim, self.pad, cache.writes)
+                   self.n_heads, self.n_kv_heads, self.dim, self.vdim, self.pad, cache.writes, **leaves)
         else:
             conv = ctx.new_f32(n, self.conv_width)
-            k.short_conv(proj, 0, self.conv_weight, None, state, 0, ctx.row_seq, ctx.seq_start, rows, conv)
+            k.short_conv(proj, 0, self.conv_weight, None, state, 0, ctx.row_seq, ctx.seq_start, rows, conv, **leaves)
             k.whole_norm_rope_write(conv, self.q_norm, self.k_norm, self.norm_eps, freq, self.turned, ctx.positions, ctx.row_seq, q,
                                     cache.k_pages, cache.v_pages, cache.page_table, self.n_heads, self.n_kv_heads, self.dim, self.vdim,
                                     self.pad, cache.writes)
-        if state is not None and cache.writes:      # after every reader of the old state
-            k.short_conv_state(proj, 0, self.conv_width, self.taps, state, 0, ctx.seq_start, rows, **to)
+        if state is not None and cache.writes and not leaves:      # after every reader of the old state
+            k.short_conv_state(proj, 0, self.conv_width, self.taps, state, 0, ctx.seq_start, rows)
         attended = ctx.new_activations(n, self.n_heads * self.pad)
         k.attention(q, attended, cache.k_pages, cache.v_pages, cache.page_table, ctx.row_seq, ctx.positions, self.n_heads,
                     self.n_kv_heads, self.pad, self.scale, 0, layout=ctx)

@@ -82,9 +82,9 @@ class StateSpaceScan:
         xbc = ctx.new_f32(n, self.conv_width)
         rows, to = cache.state_rows(ctx)
         k.short_conv(proj, self.inner, self.conv_weight, self.conv_bias, cache.state, self.state_floats, ctx.row_seq, ctx.seq_start,
-                     rows, xbc, silu=True)
-        if self.taps > 1:
-            k.short_conv_state(proj, self.inner, self.conv_width, self.taps, cache.state, self.state_floats, ctx.seq_start, rows, **to)
+                     rows, xbc, silu=True, **(to if self.taps > 1 else {}))
+        if self.taps > 1 and not to:      # (rows of their own for the state: the convolution has left it there)
+            k.short_conv_state(proj, self.inner, self.conv_width, self.taps, cache.state, self.state_floats, ctx.seq_start, rows)
         y = ctx.new_f32(n, self.inner)
         k.ssm_scan(xbc, proj, self.dt_first, self.dt_bias, self.a_log, self.d_skip, cache.state, 0, ctx.seq_start, rows, y,
                    self.n_heads, self.vdim, self.n_state, self.n_groups, max_rows_per_seq=ctx.max_rows_per_seq, **to)

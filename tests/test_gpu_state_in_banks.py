@@ -159,3 +159,42 @@ def test_an_engine_steps_the_same_after_a_step_that_failed(K, tmp_path):
             engine.graphs.step = replay
         seen.append([engine.step(rows_of(token)).clone() for token in (8, 9, 10)])
     assert all(torch.equal(a, b) for a, b in zip(*seen))
+
+
+# short sequences keep old inputs; steps of 128 rows and more walk down the rows
+@pytest.mark.parametrize("lengths", LENGTHS + [[2, 3, 1, 4], [40, 100, 2]])
+@pytest.mark.parametrize("taps", [2, 3, 4, 6])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(4, 2, 64), (24, 8, 128)])      # a few of a thread's channels, and all of them
+def test_convolutions_leave_their_state(K, lengths, taps, heads, kv_heads, dim):
+    n, (starts, row_seq) = sum(lengths), layout(lengths)
+    channels = (heads + 2 * kv_heads) * dim
+    u, weight = rows(n, channels + 8), dev(0.4 * torch.randn(channels, taps, generator=torch.Generator().manual_seed(1)))
+    norms = [dev(torch.ones(h * dim)) for h in (heads, kv_heads)]
+    position = dev(torch.cat([torch.arange(length) for length in lengths]).to(torch.int32))
+    pages = [-(-length // 64) for length in lengths]
+    table = torch.zeros(len(lengths), max(pages), dtype=torch.int32)
+    for s, count in enumerate(pages):
+        table[s, :count] = torch.arange(sum(pages[:s]), sum(pages[:s]) + count)
+
+    def alone(state, slot, seq_to=None):
+        out = torch.empty(n, channels, device="cuda:0")
+        K.short_conv(u, 0, weight, None, state, 16, row_seq, starts, slot, out, silu=True, **({"seq_to": seq_to} if seq_to is not None else {}))
+        if seq_to is None:
+            K.short_conv_state(u, 0, channels, taps, state, 16, starts, slot)
+        else:      # (sixteen floats that somebody else leaves)
+            state[seq_to.long(), :16] = state[slot.long(), :16]
+        return [out]
+
+    def with_heads(state, slot, seq_to=None):
+        q = torch.empty(n, heads * dim, dtype=torch.bfloat16, device="cuda:0")
+        keys, values = (torch.zeros(shape, dtype=torch.bfloat16, device="cuda:0") for shape in ((sum(pages), kv_heads, 64, dim), (sum(pages), kv_heads, dim, 64)))
+        K.conv_norm_rope_write(u, 0, weight, state, 16, starts, slot, *norms, 1e-6, None, 0, position, row_seq, q, keys, values, dev(table), heads, kv_heads, dim,
+                               dim, dim, True, **({"seq_to": seq_to} if seq_to is not None else {}))
+        if seq_to is None:
+            K.short_conv_state(u, 0, channels, taps, state, 16, starts, slot)
+        else:
+            state[seq_to.long(), :16] = state[slot.long(), :16]
+        return [q, keys, values]
+
+    both(alone, (16 + (taps - 1) * channels,), len(lengths))
+    both(with_heads, (16 + (taps - 1) * channels,), len(lengths))
