@@ -97,6 +97,7 @@ inline void bh_wide_row(int n_rows, int pieces, int* threads, int* per) {
 struct GateForm {
   float slope, cube;
   bool squared = false;
+  float limit = 0.f, shift = 0.f;   // a limit: the gate at most that, up between its negative and itself, and then moved by `shift`
 };
 enum BhGate { BH_GATE_SILU = 1, BH_GATE_GELU_TANH = 2 };
 inline GateForm bh_gate_form(int gate) {
@@ -107,6 +108,10 @@ __device__ inline float relu_squared(float x) {
   return v * v;
 }
 __device__ inline float gate_mul(float gate, float up, GateForm form) {
+  if (form.limit > 0.f) {      // (the same for the whole launch)
+    gate = fminf(gate, form.limit);
+    up = fminf(fmaxf(up, -form.limit), form.limit) + form.shift;
+  }
   return gate / (1.0f + expf(-gate * fmaf(form.cube, gate * gate, form.slope))) * up;
 }
 

@@ -39,7 +39,8 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
 // elements), 16 rows 4.1 us (8.6).
 template <typename TO, int PER>
 __global__ void layernorm_wide_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows, const float* __restrict__ w,
-                                      const float* __restrict__ b, TO* __restrict__ out, int n_rows, int width, float eps, int out_block_rows) {
+                                      const float* __restrict__ b, TO* __restrict__ out, int n_rows, int width, float eps, int out_block_rows,
+                                      TO* __restrict__ rows_out) {
   __shared__ float scratch[16];
   const int r = bh_row_of_block(out_block_rows), pieces = width / 4;
   if (r >= n_rows) return;
@@ -68,31 +69,35 @@ __global__ void layernorm_wide_kernel(const float* __restrict__ x, const int32_t
     if (i >= pieces) continue;
     const float4 f = reinterpret_cast<const float4*>(w)[i], c = b ? reinterpret_cast<const float4*>(b)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     // four neighbouring columns lie together in rows and in blocks alike
-    store_four(out + bh_rows_index(out_block_rows, r, 4 * i, width), held[k].x * inv * f.x + c.x, held[k].y * inv * f.y + c.y,
-               held[k].z * inv * f.z + c.z, held[k].w * inv * f.w + c.w);
+    const float4 y = make_float4(held[k].x * inv * f.x + c.x, held[k].y * inv * f.y + c.y, held[k].z * inv * f.z + c.z, held[k].w * inv * f.w + c.w);
+    store_four(out + bh_rows_index(out_block_rows, r, 4 * i, width), y.x, y.y, y.z, y.w);
+    if (rows_out) store_four(rows_out + (size_t)r * width + 4 * i, y.x, y.y, y.z, y.w);
   }
 }
 
 template <typename TO>
 static bool layernorm_wide(const float* x, const int32_t* rows, const float* w, const float* b, TO* out, int n_rows, int width, float eps,
-                           int out_block_rows, hipStream_t stream) {
-  if (width % 4 || width > 4 * 4 * 1024 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) % 16)) return false;
+                           int out_block_rows, TO* rows_out, hipStream_t stream) {
+  if (width % 4 || width > 4 * 4 * 1024 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out | (uintptr_t)rows_out) % 16)) return false;
   int threads, per;
   bh_wide_row(n_rows, width / 4, &threads, &per);
   const unsigned grid = bh_rows_grid(n_rows, out_block_rows);
-  if (per == 1) layernorm_wide_kernel<TO, 1><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
-  else if (per == 2) layernorm_wide_kernel<TO, 2><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
-  else layernorm_wide_kernel<TO, 4><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows);
+  if (per == 1) layernorm_wide_kernel<TO, 1><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows, rows_out);
+  else if (per == 2) layernorm_wide_kernel<TO, 2><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows, rows_out);
+  else layernorm_wide_kernel<TO, 4><<<grid, threads, 0, stream>>>(x, rows, w, b, out, n_rows, width, eps, out_block_rows, rows_out);
   return true;
 }
 
+// rows_out: a second output, row after row, for readers beside the one that `out` is laid out for, or null.
 extern "C" int bh_layernorm(const float* x, const int32_t* rows, const float* w, const float* b, void* out, int out_dtype,
-                            int n_rows, int width, float eps, int out_block_rows, hipStream_t stream) {
+                            int n_rows, int width, float eps, int out_block_rows, void* rows_out, hipStream_t stream) {
   BH_REQUIRE(n_rows > 0 && width > 0, "layernorm: sizes must be positive");
   BH_REQUIRE(out_block_rows == 0 || ((out_block_rows == 8 || out_block_rows == 16) && width % 32 == 0 && out_dtype == BH_BF16),
              "layernorm: rows in blocks of %d of width %d are not written", out_block_rows, width);
-  if (out_dtype == BH_F32 && layernorm_wide(x, rows, w, b, (float*)out, n_rows, width, eps, out_block_rows, stream)) return bh_check_launch("layernorm");
-  if (out_dtype == BH_BF16 && layernorm_wide(x, rows, w, b, (bf16_t*)out, n_rows, width, eps, out_block_rows, stream)) return bh_check_launch("layernorm");
+  if (out_dtype == BH_F32 && layernorm_wide(x, rows, w, b, (float*)out, n_rows, width, eps, out_block_rows, (float*)rows_out, stream)) return bh_check_launch("layernorm");
+  if (out_dtype == BH_BF16 && layernorm_wide(x, rows, w, b, (bf16_t*)out, n_rows, width, eps, out_block_rows, (bf16_t*)rows_out, stream)) return bh_check_launch("layernorm");
+  if (rows_out)
+    if (int status = bh_layernorm(x, rows, w, b, rows_out, out_dtype, n_rows, width, eps, 0, nullptr, stream)) return status;
   if (out_dtype == BH_F32)
     layernorm_kernel<float><<<n_rows, 256, 0, stream>>>(x, rows, w, b, (float*)out, width, eps, out_block_rows);
   else if (out_dtype == BH_BF16)

@@ -95,6 +95,19 @@ class BlockedRows:
         return -(-rows // unit) * unit
 
 
+class BothRows:
+    """A bfloat16 activation matrix that several kernels read, kept twice: row after row (`row_by_row`) and in the blocks of the
+    products among its readers (`blocks`).  `layernorm` writes both; `gemm` takes it and reads the form it reads best.  `shape` and
+    `dtype` are those of the matrix."""
+
+    def __init__(self, row_by_row: torch.Tensor, blocks: BlockedRows):
+        self.row_by_row, self.blocks = row_by_row, blocks
+        self.shape, self.dtype, self.device = tuple(row_by_row.shape), row_by_row.dtype, row_by_row.device
+
+    def dim(self):
+        return 2
+
+
 def _block_rows(x) -> int:
     """In blocks of how many rows a matrix lies (0: row after row)."""
     return x.block_rows if isinstance(x, BlockedRows) else 0
@@ -169,6 +182,7 @@ class KernelSizes:
             "bh_attention_bf16_writes_blocked": [i, i, i, i, i],
             "bh_attention_decode_fused": [p, p, p, p, p, p, p, i, p, p, i, i, i, i, f, i, i, i, p, p, i, f, p, p, i, i,
                                           i, i, p],
+            "bh_gemm_bf16_clamped_glu": [p, p, p, i, i, i, f, f, f, p, i, i, p],
             "bh_attention_decode_pairs": [p, i, i, p, p, p, p, p, p, i, p, p, i, i, i, i, f, i, i, i, p, p, i, f, p, p, i, i, i, i, p, p, i, f, p, f, i, f, p],
             "bh_row_angles": [p, p, f, p, p, i, i, p],
             "bh_kv_order": [i, i],
@@ -189,7 +203,7 @@ class KernelSizes:
             "bh_latent_write": [p, i, i, i, p, f, p, i, p, p, p, p, p, i, i, i, i, i, i, p, ctypes.c_long, i, i, i, i, i, p, ctypes.c_long, i, f, p],
             "bh_heads_linear": [p, ctypes.c_long, i, i, p, p, ctypes.c_long, i, i, i, i, i, i, i, i, p],
             "bh_rotate_heads": [p, ctypes.c_long, i, i, p, ctypes.c_long, i, i, i, p, i, p, i, i, i, p],
-            "bh_layernorm": [p, p, p, p, p, i, i, i, f, i, p],
+            "bh_layernorm": [p, p, p, p, p, i, i, i, f, i, p, p],
             "bh_cast_concat": [p, p, p, i, i, i, i, p],
             "bh_add_rmsnorm": [p, p, p, i, p, i, i, i, f, i, p],
             "bh_sum_layernorm": [p, p, f, p, p, p, i, i, i, f, i, p],
@@ -511,6 +525,8 @@ class HipKernels(KernelSizes):
 
     def _in_blocks_of(self, x, block_rows):
         """`x` (rows or `BlockedRows`) in blocks of `block_rows` rows (0: as rows), regrouped if it lies otherwise."""
+        if isinstance(x, BothRows):
+            x = x.blocks if x.blocks.block_rows == block_rows else x.row_by_row
         if _block_rows(x) == block_rows:
             return x
         rows = self.from_blocked(x) if isinstance(x, BlockedRows) else x
@@ -627,8 +643,7 @@ class HipKernels(KernelSizes):
         done, prepared = self._gemm_fast(a, w, out, accumulate, 0, then_norm)
         if done:
             return prepared
-        if isinstance(a, BlockedRows):
-            a = self.from_blocked(a)
+        a = self._in_blocks_of(a, 0)
         if (then_norm is not None and a.dtype == out.dtype == then_norm.weight.dtype == torch.float32
                 and then_norm.weight.shape == (n,) and self.lib.bh_gemm_f32_takes_gated(m, 4, n)):
             prepared = NormedRows(out, None, then_norm.eps, out, then_norm.weight)      # its reader norms the residual itself
@@ -648,6 +663,26 @@ class HipKernels(KernelSizes):
             return False
         self._check(self.lib.bh_gemm_f32_normed(self._ptr(a.source, "gemm a"), self._ptr(a.weight, "norm weight"), a.eps, self._ptr(w, "gemm w"),
                                                 self._ptr(out, "gemm out"), m, n, k, gate, self._stream()))
+        return True
+
+    def gemm_clamped_glu(self, a, w, out, limit, alpha, shift=1.0) -> bool:
+        """`gemm` of a [n, K] with w [2 ff, K] (gate rows, then up rows) and `clamped_glu` of the result into `out` [n, ff], in one product;
+        False, having done nothing, where the library has none of these operands that does so (then call the two)."""
+        if (not isinstance(w, PackedWeight) or isinstance(a, NormedRows) or a.dim() != 2 or a.dtype != torch.bfloat16 or out.dtype != torch.bfloat16
+                or a.shape[1] != w.shape[1] or not limit > 0.0 or out.shape[1] % 16):
+            return False
+        (m, k), width = a.shape, out.shape[1]
+        if tuple(out.shape) != (m, width) or w.shape[0] != 2 * width:
+            raise KernelError(f"gemm_clamped_glu: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
+        a_block_rows, writes, _, _, scratch_bytes, _ = self._product(m, width, k, 1, 1)
+        c_block_rows = _block_rows(out)
+        if c_block_rows and not (writes == 2 or (writes == 1 and c_block_rows == 16)):
+            return False
+        a = self._in_blocks_of(a, a_block_rows)
+        scratch = torch.empty(scratch_bytes // 4, dtype=torch.float32, device=self.device) if scratch_bytes else None
+        self._check(self.lib.bh_gemm_bf16_clamped_glu(
+            self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), m, width, k, float(limit), float(alpha), float(shift),
+            self._ptr(scratch, "gemm scratch", None, True), a_block_rows, c_block_rows, self._stream()))
         return True
 
     def gemm_relu_squared(self, a, w, out) -> bool:
@@ -764,8 +799,7 @@ class HipKernels(KernelSizes):
             self.gemm_swiglu(a, w, rows_out, gate)
             self.to_blocked(rows_out, out)
             return
-        if isinstance(a, BlockedRows):
-            a = self.from_blocked(a)
+        a = self._in_blocks_of(a, 0)
         if (a.dtype == w.dtype == torch.float32 and self.lib.bh_gemm_f32_takes_gated(m, width, k)
                 and (a.data_ptr() | w.data_ptr()) % 16 == 0):
             self._check(self.lib.bh_gemm_f32_gated(self._ptr(a, "gemm a"), self._ptr(w, "gemm w"), self._ptr(out, "gemm out"),
@@ -1412,8 +1446,11 @@ class HipKernels(KernelSizes):
     # ---- row-wise operations on the residual and on logits ----
     def layernorm(self, x, weight, bias, eps, out, rows=None):
         """out[r] = (x[row] - mean) / sqrt(var + eps) * weight + bias, row = rows[r] if rows is given else r; x f32 [*, D],
-        weight and bias f32 [D] (bias may be None), out [n, D] in rows or blocks of rows."""
+        weight and bias f32 [D] (bias may be None), out [n, D] in rows, blocks of rows or both (`BothRows`)."""
         n_rows, width = out.shape
+        beside = None
+        if isinstance(out, BothRows):
+            out, beside = out.blocks, out.row_by_row
         if x.dim() != 2 or x.shape[1] != width or weight.shape != (width,) or (bias is not None and bias.shape != (width,)):
             raise KernelError(f"layernorm: shapes x {tuple(x.shape)}, out {tuple(out.shape)} do not fit")
         if (rows is None and x.shape[0] != n_rows) or (rows is not None and rows.shape != (n_rows,)):
@@ -1421,7 +1458,13 @@ class HipKernels(KernelSizes):
         self._check(self.lib.bh_layernorm(
             self._ptr(x, "layernorm x", (torch.float32,)), self._ptr(rows, "layernorm rows", (torch.int32,), True),
             self._ptr(weight, "layernorm weight", (torch.float32,)), self._ptr(bias, "layernorm bias", (torch.float32,), True),
-            self._ptr(out, "layernorm out"), _code(out, "layernorm out"), n_rows, width, float(eps), _block_rows(out), self._stream()))
+            self._ptr(out, "layernorm out"), _code(out, "layernorm out"), n_rows, width, float(eps), _block_rows(out),
+            self._ptr(beside, "layernorm rows out", (out.dtype,), True), self._stream()))
+
+    def new_both_rows(self, rows, width, dtype, reader_outputs=None, reader_swiglu=False, reader_packed=True):
+        """`new_rows` for a matrix that kernels read row after row beside the product named: `BothRows` where that one reads blocks."""
+        blocks = self.new_rows(rows, width, dtype, reader_outputs, reader_swiglu, reader_packed)
+        return BothRows(torch.empty((int(rows), int(width)), dtype=dtype, device=self.device), blocks) if isinstance(blocks, BlockedRows) else blocks
 
     def sum_layernorm(self, hidden, y, alpha, weight, bias, eps, rounded=None):
         """hidden[r] <- layernorm(alpha * hidden[r] + y[r]) * weight + bias in place (all f32, the variance as the mean of

@@ -80,6 +80,10 @@ class PreNormBlock:
     @staticmethod
     def _normed(ctx, norm, consumer, hidden):
         reader = PreNormBlock._reader(norm, consumer)
+        if reader is None and getattr(norm, "serves_rows_too", False):      # rows, and blocks for the products among the consumer's kernels
+            products = getattr(consumer, "products_reader", None)
+            if products is not None:
+                return norm.forward(ctx, hidden, reader=products, rows_too=True)
         return norm.forward(ctx, hidden, reader=reader) if reader is not None else norm.forward(ctx, hidden)
 
     def entry_request(self, producer):

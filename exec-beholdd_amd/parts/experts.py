@@ -70,9 +70,11 @@ class ClampedGLU:
                 + self.down.working_bytes(step, step.rows, accumulate=True))
 
     def forward(self, ctx, x, hidden, then_norm=None):
-        both = self.gate_up.forward(ctx, x)
-        inner = ctx.new_activations(both.shape[0], self.ff, reader=self.down.reader())
-        ctx.kernels.clamped_glu(both, inner, self.limit, self.alpha)
+        inner = ctx.new_activations(x.shape[0], self.ff, reader=self.down.reader())
+        in_product = getattr(ctx.kernels, "gemm_clamped_glu", None)
+        if in_product is None or not in_product(x, self.gate_up.weight, inner, self.limit, self.alpha):
+            both = self.gate_up.forward(ctx, x)
+            ctx.kernels.clamped_glu(both, inner, self.limit, self.alpha)
         self.down.forward(ctx, inner, out=hidden, accumulate=True)
         return None
 
@@ -166,7 +168,7 @@ class RoutedExperts:
             self.for_products = [(kernels.pack_weight(self.w_gate_up[e]), kernels.pack_weight(self.w_down[e])) for e in range(self.n_experts)]
 
     def working_bytes(self, step) -> int:
-        total = self.router.working_bytes(step, step.rows, out_size=4)
+        total = self.router.working_bytes(step, step.rows, out_size=4) + step.matrix(step.rows, self.hidden, reader=self.router.reader_for_plan(step.act_size))
         if step.rows > self.WIDE_FROM_ROWS and self.router.out_features < self.WIDE_ROUTER:
             total = step.matrix(step.rows, self.WIDE_ROUTER, 4) + step.product(step.rows, self.WIDE_ROUTER, self.hidden)
         total += 2 * step.matrix(step.rows, self.top, 4)
@@ -177,16 +179,22 @@ class RoutedExperts:
             total += step.matrix(pairs, self.hidden) + step.matrix(pairs, 2 * self.ff) + step.matrix(pairs, 1, 4)
         return total + (self.shared.working_bytes(step) if self.shared is not None else 0)
 
+    @property
+    def products_reader(self):
+        """The product among the readers of this part's input, beside the kernels that read it row after row."""
+        return getattr(self.shared, "input_reader", None) or self.router.reader()
+
     def forward(self, ctx, x, hidden, then_norm=None, fresh=False):
         k = ctx.kernels
         n = x.shape[0]
+        whole, x = x, getattr(x, "row_by_row", x)      # what the products read, and what the others do
         routing = {"scoring": self.scoring} if self.scoring != "softmax" else {}
         if self.router_wide is not None and n > self.WIDE_FROM_ROWS:
             logits = ctx.new_f32(n, self.WIDE_ROUTER)
-            k.gemm(x, self.router_wide, logits)
+            k.gemm(whole, self.router_wide, logits)
             routing["experts"] = self.router.out_features
         else:
-            logits = self.router.forward(ctx, x, out_dtype=torch.float32)
+            logits = self.router.forward(ctx, whole, out_dtype=torch.float32)
         chosen = torch.empty((n, self.top), dtype=torch.int32, device=ctx.device)
         weights = ctx.new_f32(n, self.top)
         if self.correction is not None:
@@ -227,7 +235,7 @@ class RoutedExperts:
             else:
                 self._as_products(ctx, x, lists, counts, weights, hidden, adding)
         if self.shared is not None:
-            self.shared.forward(ctx, x, hidden)
+            self.shared.forward(ctx, whole, hidden)
         return None
 
     def _one_launch_is_faster(self, pairs: int) -> bool:

@@ -116,9 +116,13 @@ class LayerNorm:
         self.weight = get(self.name).to(torch.float32).contiguous()
         self.bias = get(self.bias_name).to(torch.float32).contiguous() if self.bias_name is not None else None
 
-    def forward(self, ctx, hidden, rows=None, reader=None):
+    serves_rows_too = True      # forward(..., rows_too=True): for kernels that read it row after row, beside the reader
+
+    def forward(self, ctx, hidden, rows=None, reader=None, rows_too=False):
         n = hidden.shape[0] if rows is None else rows.shape[0]
-        out = ctx.new_activations(n, self.width, reader=reader)
+        both = getattr(ctx.kernels, "new_both_rows", None) if rows_too and reader is not None and ctx.act_dtype == torch.bfloat16 else None
+        out = (both(n, self.width, ctx.act_dtype, reader.outputs, reader.swiglu, reader.packed) if both is not None
+               else ctx.new_activations(n, self.width, reader=None if rows_too else reader))
         ctx.kernels.layernorm(hidden, self.weight, self.bias, self.eps, out, rows=rows)
         return out
 
