@@ -1184,16 +1184,19 @@ extern "C" long bh_gemm_bf16_scratch(int M, int N, int K, int layout, int activa
 // bh_gemm_bf16_reads_blocked says this product reads them, or in rows (0).  c_block_rows: a SwiGLU's output goes out
 // that way (16 in the kernel for many rows; 0, 8 or 16 in the skinny one); behind_block_rows: so do the rows
 // prepared for a norm behind (the skinny kernel's).
-static int gemm_bf16_run(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K,
-                         int layout, int activation, const GateForm& form, const float* ahead_ss, int ahead_blocks, float ahead_eps,
-                         const void* behind_weight, int behind_weight_dtype, void* behind_rows,
-                         float* behind_ss, void* scratch, int a_block_rows, int c_block_rows, int behind_block_rows,
-                         hipStream_t stream) {
+extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K,
+                            int layout, int activation, const float* ahead_ss, int ahead_blocks, float ahead_eps,
+                            const void* behind_weight, int behind_weight_dtype, void* behind_rows,
+                            float* behind_ss, void* scratch, int a_block_rows, int c_block_rows, int behind_block_rows,
+                            hipStream_t stream) {
   BH_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_bf16: sizes M=%d N=%d K=%d must be positive", M, N, K);
   BH_REQUIRE(K % 8 == 0, "gemm_bf16: K=%d must be a multiple of 8", K);
   BH_REQUIRE(c_dtype == BH_F32 || c_dtype == BH_BF16, "gemm_bf16: unknown output dtype %d", c_dtype);
   BH_REQUIRE(((uintptr_t)a | (uintptr_t)w) % 16 == 0, "gemm_bf16: operands must be 16-byte aligned");
   BH_REQUIRE(layout == 0 || (layout == 1 && K % 64 == 0), "gemm_bf16: the tiles layout needs K=%d to be a multiple of 64", K);
+  BH_REQUIRE(activation == 0 || activation == BH_GATE_SILU || activation == BH_GATE_GELU_TANH, "gemm_bf16: unknown activation %d", activation);
+  const GateForm form = bh_gate_form(activation);
+  activation = activation != 0;      // from here on: gated or not
   BH_REQUIRE(activation == 0 || (N % 16 == 0 && !accumulate),
              "gemm_bf16: SwiGLU needs a multiple of 16 outputs (got %d) and no accumulation", N);
   BH_REQUIRE((M + 127) / 128 <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
@@ -1313,27 +1316,27 @@ static int gemm_bf16_run(const void* a, const void* w, void* c, int c_dtype, int
   return bh_check_launch("gemm_tiled");
 }
 
-extern "C" int bh_gemm_bf16(const void* a, const void* w, void* c, int c_dtype, int accumulate, int M, int N, int K,
-                            int layout, int activation, const float* ahead_ss, int ahead_blocks, float ahead_eps,
-                            const void* behind_weight, int behind_weight_dtype, void* behind_rows,
-                            float* behind_ss, void* scratch, int a_block_rows, int c_block_rows, int behind_block_rows,
-                            hipStream_t stream) {
-  BH_REQUIRE(activation == 0 || activation == BH_GATE_SILU || activation == BH_GATE_GELU_TANH, "gemm_bf16: unknown activation %d", activation);
-  return gemm_bf16_run(a, w, c, c_dtype, accumulate, M, N, K, layout, activation != 0, bh_gate_form(activation), ahead_ss, ahead_blocks, ahead_eps,
-                       behind_weight, behind_weight_dtype, behind_rows, behind_ss, scratch, a_block_rows, c_block_rows, behind_block_rows, stream);
-}
-
-// A SwiGLU of the kind g' sigmoid(alpha g') (u' + shift) with g' = min(g, limit) and u' = clamp(u, -limit, limit), as bfloat16 from packed
+// A SwiGLU of the kind g' sigmoid(alpha g') (u' + 1) with g' = min(g, limit) and u' = clamp(u, -limit, limit), as bfloat16 from packed
 // weights: the gate in the product, from its float32 sums, where an activation of its own read them back as bfloat16 (clamped_glu of
-// experts.hip; 2,100 rows of 3,072 outputs 12.7 us, 16 rows 4.6).
-extern "C" int bh_gemm_bf16_clamped_glu(const void* a, const void* w, void* c, int M, int N, int K, float limit, float alpha, float shift,
-                                        void* scratch, int a_block_rows, int c_block_rows, hipStream_t stream) {
+// experts.hip; 2,100 rows of 3,072 outputs 12.7 us, 16 rows 4.6).  Which products do: those of few rows and those of many that go in one
+// piece; 0 for the others.
+extern "C" int bh_gemm_bf16_clamps(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || N % 16 != 0) return 0;
+  if (const RingPlan ring = many_rows_plan(M, N, K, 1, RING_GATED); ring.tile >= 0) return ring.parts == 1 ? 1 : 0;
+  return skinny_first(M, N, K, 1, 1) && gemm_few_takes(M, N, K, true) ? 2 : 0;
+}
+extern "C" int bh_gemm_bf16_clamped_glu(const void* a, const void* w, void* c, int M, int N, int K, float limit, float alpha,
+                                        int a_block_rows, int c_block_rows, hipStream_t stream) {
+  const int kind = bh_gemm_bf16_clamps(M, N, K);
+  BH_REQUIRE(kind != 0, "gemm_bf16_clamped_glu: a product of M=%d N=%d K=%d does not clamp its gate", M, N, K);
   BH_REQUIRE(limit > 0.f, "gemm_bf16_clamped_glu: a limit is positive");
-  GateForm form = {alpha, 0.f};
-  form.limit = limit;
-  form.shift = shift;
-  return gemm_bf16_run(a, w, c, BH_BF16, 0, M, N, K, 1, 1, form, nullptr, 0, 0.f, nullptr, 0, nullptr, nullptr, scratch, a_block_rows, c_block_rows,
-                       0, stream);
+  BH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0, "gemm_bf16_clamped_glu: operands must be 16-byte aligned");
+  BH_REQUIRE(a_block_rows == bh_gemm_bf16_reads_blocked(M, N, K, 1, 1), "gemm_bf16_clamped_glu: the activations lie in blocks of %d rows", a_block_rows);
+  BH_REQUIRE(c_block_rows == 0 || (N % 32 == 0 && (c_block_rows == 16 || (c_block_rows == 8 && kind == 2))),
+             "gemm_bf16_clamped_glu: a product of M=%d N=%d does not write blocks of %d rows", M, N, c_block_rows);
+  const GateForm form = {alpha, limit};
+  if (kind == 1) return gemm_ring_launch(a, w, c, BH_BF16, 0, M, N, K, GATED_CLAMPED, many_rows_plan(M, N, K, 1, RING_GATED).tile, c_block_rows == 16, form, stream);
+  return gemm_few_launch(a, w, c, false, 0, M, N, K, GATED_CLAMPED, RidingNorm{}, {a_block_rows, c_block_rows, 0}, form, stream);
 }
 
 // C[M, N] = max(A W^T, 0)^2 as bfloat16 in one launch, from packed weights: what an activation of its own would read and write again

@@ -32,5 +32,5 @@ int gemm_few_rows(int N, int K, bool gated);
 // Whether the kernel is the better one for a product of up to 32 rows (N % 16 == 0, K % 64 == 0, W in the tiles layout): else the
 // kernel of gemm_bf16.hip that asks for its chunks in bursts, with 16 weight rows a workgroup.
 bool gemm_few_takes(int M, int N, int K, bool gated);
-int gemm_few_launch(const void* a, const void* w, void* c, bool f32, int accumulate, int M, int N, int K, bool gated, const RidingNorm& norm,
+int gemm_few_launch(const void* a, const void* w, void* c, bool f32, int accumulate, int M, int N, int K, int gated, const RidingNorm& norm,
                     const RowBlocks& blocks, GateForm form, hipStream_t stream);

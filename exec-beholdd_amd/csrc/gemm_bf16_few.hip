@@ -40,8 +40,8 @@ __device__ inline u32x4_t from_lane_plus_8(u32x4_t v) {
 
 #define FEW_WAVES 8
 // MB: blocks of 16 activation rows, which lie in blocks of XB rows.  NB: blocks of W that a span touches; MASKED: it is not the whole of
-// one.  SHORT: no wave has more than DEPTH chunks.
-template <int MB, typename TC, int XB, int NB, bool GATED, bool MASKED, int DEPTH, bool SHORT>
+// one.  SHORT: no wave has more than DEPTH chunks.  GATED: 1, or 2 with a clamped gate (gate_mul).
+template <int MB, typename TC, int XB, int NB, int GATED, bool MASKED, int DEPTH, bool SHORT>
 __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ w,
                                                                   TC* __restrict__ c, int M, int N, int K, int accumulate, int span,
                                                                   RidingNorm norm, RowBlocks blocks, GateForm form) {
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const uint16_t
       }
       if (!valid) continue;
       if constexpr (GATED) {
-        c[bh_rows_index(blocks.c, m, n, N)] = from_f32<TC>(gate_mul(sum[0], sum[GATED ? 1 : 0], form));
+        c[bh_rows_index(blocks.c, m, n, N)] = from_f32<TC>(gate_mul<GATED == 2>(sum[0], sum[GATED ? 1 : 0], form));
       } else if constexpr (OUT_EARLY) {
         const float value = accumulate ? before[pass][t] + sum[0] : sum[0];
         c[(size_t)m * N + n] = value;
@@ -289,7 +289,7 @@ bool gemm_few_takes(int M, int N, int K, bool gated) {
   return !many && (M <= 16 || K <= 2048);
 }
 
-template <int MB, typename TC, int XB, int NB, bool GATED, bool MASKED, int DEPTH>
+template <int MB, typename TC, int XB, int NB, int GATED, bool MASKED, int DEPTH>
 static void launch_depth(const void* a, const void* w, void* c, int accumulate, int M, int N, int K, int span, const RidingNorm& norm,
                          const RowBlocks& blocks, GateForm form, hipStream_t stream) {
 #define BH_FEW(SHORT)                                                                                                      \
@@ -301,18 +301,24 @@ static void launch_depth(const void* a, const void* w, void* c, int accumulate, 
 }
 
 template <int MB, typename TC, int XB>
-static void launch_rows(const void* a, const void* w, void* c, int accumulate, int M, int N, int K, bool gated, const RidingNorm& norm,
+static void launch_rows(const void* a, const void* w, void* c, int accumulate, int M, int N, int K, int gated, const RidingNorm& norm,
                         const RowBlocks& blocks, GateForm form, hipStream_t stream) {
   const int span = gemm_few_rows(N, K, gated);
 #define BH_FEW(...) launch_depth<MB, TC, XB, __VA_ARGS__>(a, w, c, accumulate, M, N, K, span, norm, blocks, form, stream)
-  if (gated) BH_FEW(1, true, false, 2);
-  else if (span == 16) BH_FEW(1, false, false, 2);
-  else if (span == 8) BH_FEW(1, false, true, 4);
-  else BH_FEW(2, false, true, MB == 1 && sizeof(TC) == 4 ? 4 : 2);
+  if constexpr (sizeof(TC) == 2) {
+    if (gated == GATED_CLAMPED) {
+      BH_FEW(1, 2, false, 2);
+      return;
+    }
+  }
+  if (gated) BH_FEW(1, 1, false, 2);
+  else if (span == 16) BH_FEW(1, 0, false, 2);
+  else if (span == 8) BH_FEW(1, 0, true, 4);
+  else BH_FEW(2, 0, true, MB == 1 && sizeof(TC) == 4 ? 4 : 2);
 #undef BH_FEW
 }
 
-int gemm_few_launch(const void* a, const void* w, void* c, bool f32, int accumulate, int M, int N, int K, bool gated, const RidingNorm& norm,
+int gemm_few_launch(const void* a, const void* w, void* c, bool f32, int accumulate, int M, int N, int K, int gated, const RidingNorm& norm,
                     const RowBlocks& blocks, GateForm form, hipStream_t stream) {
 #define BH_FEW_ARGS a, w, c, accumulate, M, N, K, gated, norm, blocks, form, stream
   if (blocks.a == 0 && M <= 16) {

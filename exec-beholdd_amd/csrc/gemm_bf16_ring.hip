@@ -72,7 +72,7 @@ __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int parts, in
 
 // MODE 0: bfloat16 output.  1: float32 output, optionally added to what is there; with parts, part p leaves the bare sums of its share
 // of k at c + p M N.  2: gated (the gate as `form` says), bfloat16 output of N columns; W has 2 N rows, gate rows then up rows, and a
-// wave's weight rows are the gate and the up rows of the same outputs.  3: as 0, squared behind a ReLU.  c_blocked (MODE 2 and 3): the
+// wave's weight rows are the gate and the up rows of the same outputs.  3: as 0, squared behind a ReLU.  4: as 2, clamped (gate_mul).  c_blocked (MODE 2 to 4): the
 // output in blocks of 16 rows.
 // A tile that sticks out of the matrix repeats its last blocks and stores only what exists; no block of A beyond the last row's is read.
 // K a multiple of 64 per part, so that a part has an even number of steps.
@@ -84,8 +84,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
                                                                     int c_blocked, GateForm form) {
   constexpr int WAVES = WM * WN, A_PIECES = XB * WM, W_PIECES = YB * WN, PIECES = A_PIECES + W_PIECES;
   constexpr int EACH = (PIECES + WAVES - 1) / WAVES;   // a wave's pieces of a step; those beyond the last repeat it, so that every wave's count of loads says how far they are
-  constexpr int ROWS = 16 * A_PIECES, OUTS = (MODE == 2 ? 8 : 16) * W_PIECES;
-  static_assert(MODE != 2 || YB % 2 == 0, "a wave's weight rows are gate and up rows of the same outputs");
+  constexpr bool GATED = MODE == 2 || MODE == 4;
+  constexpr int ROWS = 16 * A_PIECES, OUTS = (GATED ? 8 : 16) * W_PIECES;
+  static_assert(!GATED || YB % 2 == 0, "a wave's weight rows are gate and up rows of the same outputs");
   static_assert(R >= 4 && EACH * (R - 3) < 64, "the count of loads on their way fits s_waitcnt");
   __shared__ __attribute__((aligned(16))) u32x4_t rings[KG][R * PIECES * 64];     // [group][step in turn][A pieces, then W pieces][lane]
   const int lane = threadIdx.x % 64, wave_of_all = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
       from[i] = a + ((size_t)block * (K / 32) + k_first / 32) * 512 + lane * 8;
     } else {
       const int b = piece - A_PIECES, column = b / YB, y = b % YB;
-      const int block = MODE == 2 ? (y < YB / 2 ? 0 : N / 16) + min(tile_n * (W_PIECES / 2) + (YB / 2) * column + y % (YB / 2), N / 16 - 1)
+      const int block = GATED ? (y < YB / 2 ? 0 : N / 16) + min(tile_n * (W_PIECES / 2) + (YB / 2) * column + y % (YB / 2), N / 16 - 1)
                                   : min(tile_n * W_PIECES + b, N / 16 - 1);
       from[i] = w + ((size_t)block * (K / 64) + k_first / 64) * 1024 + w_lane;
     }
@@ -207,8 +208,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
     const int row = m0 + 16 * x;
     if (row >= M) continue;
 #pragma unroll
-    for (int y = 0; y < (MODE == 2 ? YB / 2 : YB); ++y) {
-      const int n = tile_n * OUTS + (MODE == 2 ? 8 : 16) * YB * wn + 16 * y + 4 * (lane / 16);
+    for (int y = 0; y < (GATED ? YB / 2 : YB); ++y) {
+      const int n = tile_n * OUTS + (GATED ? 8 : 16) * YB * wn + 16 * y + 4 * (lane / 16);
       if (n >= N) continue;
       if (MODE == 1) {
         f32x4_t* at = reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(c) + ((size_t)part * M + row) * N + n);
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void gemm_ring_kernel(const u
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          v[i] = MODE == 2 ? gate_mul(acc[x][y][i], acc[x][MODE == 2 ? y + YB / 2 : y][i], form) : MODE == 3 ? relu_squared(acc[x][y][i]) : acc[x][y][i];
+          v[i] = GATED ? gate_mul<MODE == 4>(acc[x][y][i], acc[x][GATED ? y + YB / 2 : y][i], form) : MODE == 3 ? relu_squared(acc[x][y][i]) : acc[x][y][i];
         u32x2_t packed;
         packed[0] = f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
         packed[1] = f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
@@ -269,7 +270,7 @@ double cost_us(int tile, int parts, int M, int W, int K, RingOutput output) {
 template <int MODE>
 int launch(int tile, int parts, const void* a, const void* w, void* c, int M, int N, int K, int accumulate, int c_blocked, GateForm form,
            hipStream_t stream) {
-  const int outs = SHAPES[tile].columns / (MODE == 2 ? 2 : 1), rows = SHAPES[tile].rows;
+  const int outs = SHAPES[tile].columns / (MODE == 2 || MODE == 4 ? 2 : 1), rows = SHAPES[tile].rows;
   const dim3 grid((unsigned)((long)((N + outs - 1) / outs) * ((M + rows - 1) / rows) * parts));
 #define BH_RING(XB, YB, WM, WN, R, KG, BM, BN)                                                                                 \
   gemm_ring_kernel<MODE, XB, YB, WM, WN, R, KG, BM, BN><<<grid, 64 * WM * WN * KG, 0, stream>>>(                               \
@@ -348,6 +349,7 @@ int gemm_ring_launch(const void* a, const void* w, void* c, int c_dtype, int acc
   BH_REQUIRE(!form.squared || (!activation && c_dtype == BH_BF16), "gemm_ring: a plain product squares its bfloat16 output");
   BH_REQUIRE(!c_blocked || ((activation || form.squared) && N % 32 == 0),
              "gemm_ring: only a gated or squared product writes its output in blocks, and N=%d must be a multiple of 32", N);
+  if (activation == GATED_CLAMPED) return launch<4>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);
   if (activation) return launch<2>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);
   if (c_dtype == BH_F32) return launch<1>(tile, 1, a, w, c, M, N, K, accumulate, 0, form, stream);
   if (form.squared) return launch<3>(tile, 1, a, w, c, M, N, K, 0, c_blocked, form, stream);

@@ -83,12 +83,13 @@ __device__ inline void tile_of_workgroup(int n_tiles, int m_tiles, int* tile_n, 
 // the same outputs).  3: as 0, squared behind a ReLU.  YB: blocks of 16 weight rows per wave.
 // A tile that would stick out of the weight rows is moved back inside and stores only what it owns.
 // A's buffer holds whole tiles of 256 rows, and a tile that sticks out below stays where it is and stores only the rows
-// that exist.  c_blocked (MODE 2 and 3): the output lies in blocks of 16 rows.
+// that exist.  4: as 2, clamped (gate_mul).  c_blocked (MODE 2 to 4): the output lies in blocks of 16 rows.
 template <int MODE, int YB>
 __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ w,
                                                       void* __restrict__ c, int M, int N, int K, int accumulate,
                                                       int c_blocked, GateForm form) {
-  constexpr int OUTS = MODE == 2 ? 16 * YB : 32 * YB;
+  constexpr bool GATED = MODE == 2 || MODE == 4;
+  constexpr int OUTS = GATED ? 16 * YB : 32 * YB;
   constexpr int CHUNKS = 16 + 2 * YB;
   constexpr int WL = YB / 2;   // W chunks per loading wave
   constexpr int R = 4;                 // steps that LDS holds (with five or six of them it ran no faster)
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 #pragma unroll
   for (int b = 0; b < WL; ++b) {
     const int rb = i4 * WL + b, gg = rb / YB, y = rb % YB;
-    const int nb = MODE == 2 ? (y < YB / 2 ? 0 : N / 16) + n0 / 16 + (YB / 2) * gg + y % (YB / 2) : n0 / 16 + rb;
+    const int nb = GATED ? (y < YB / 2 ? 0 : N / 16) + n0 / 16 + (YB / 2) * gg + y % (YB / 2) : n0 / 16 + rb;
     w_src[b] = w + ((size_t)nb * (K / 64) + k_first / 64) * 1024 + w_lane;
   }
   auto fetch_a = [&](int j, int region) {
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
   }
   // acc[x][y][i]: row 64 i4 + 16 x + lane % 16 of the tile, weight row 16 (YB g + y) + 4 (lane / 16) + i
   const int m = m0 + 64 * i4 + lane % 16;
-  if (MODE == 2) {
+  if (GATED) {
     uint16_t* out = reinterpret_cast<uint16_t*>(c);
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -211,8 +212,8 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
         const int n = n0 + 8 * YB * g + 16 * y + 4 * (lane / 16);
         if (n < n_own) continue;
         u32x2_t packed;
-        packed[0] = f32_to_bf16_bits(gate_mul(acc[x][y][0], acc[x][y + YB / 2][0], form)) | ((uint32_t)f32_to_bf16_bits(gate_mul(acc[x][y][1], acc[x][y + YB / 2][1], form)) << 16);
-        packed[1] = f32_to_bf16_bits(gate_mul(acc[x][y][2], acc[x][y + YB / 2][2], form)) | ((uint32_t)f32_to_bf16_bits(gate_mul(acc[x][y][3], acc[x][y + YB / 2][3], form)) << 16);
+        packed[0] = f32_to_bf16_bits(gate_mul<MODE == 4>(acc[x][y][0], acc[x][y + YB / 2][0], form)) | ((uint32_t)f32_to_bf16_bits(gate_mul<MODE == 4>(acc[x][y][1], acc[x][y + YB / 2][1], form)) << 16);
+        packed[1] = f32_to_bf16_bits(gate_mul<MODE == 4>(acc[x][y][2], acc[x][y + YB / 2][2], form)) | ((uint32_t)f32_to_bf16_bits(gate_mul<MODE == 4>(acc[x][y][3], acc[x][y + YB / 2][3], form)) << 16);
         *reinterpret_cast<u32x2_t*>(out + (c_blocked ? (size_t)bh_blocked_index(row, n, N) : (size_t)row * N + n)) = packed;
       }
     }
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(512) void gemm_turns_kernel(const uint16_t* __restr
 template <int MODE>
 void launch(const void* a, const void* w, void* c, int blocks, int M, int N, int K, int accumulate, int parts, int c_blocked, GateForm form,
             hipStream_t stream) {
-  const int outs = (MODE == 2 ? 16 : 32) * blocks;
+  const int outs = (MODE == 2 || MODE == 4 ? 16 : 32) * blocks;
   dim3 grid(((N + outs - 1) / outs) * ((M + 255) / 256), parts);
   if (blocks == 8)
     gemm_turns_kernel<MODE, 8><<<grid, 512, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, c, M, N, K, accumulate, c_blocked, form);
@@ -264,7 +265,7 @@ void launch(const void* a, const void* w, void* c, int blocks, int M, int N, int
 
 bool gemm_turns_can(int M, int N, int K, int mode, int blocks, int parts) {
   if (blocks != 8 && blocks != 6) return false;
-  const int outs = (mode == 2 ? 16 : 32) * blocks;
+  const int outs = (mode == 2 || mode == 4 ? 16 : 32) * blocks;
   return M > 0 && N >= outs && N % 16 == 0 && parts >= 1 && (mode == 1 || parts == 1) && K >= 128 * parts && K % (128 * parts) == 0 &&
          (long)((N + outs - 1) / outs) * ((M + 255) / 256) < (1L << 31);   // offsets into A, W and C are 64-bit
 }
@@ -273,6 +274,7 @@ int gemm_turns_launch(const void* a, const void* w, void* c, int mode, int accum
                       int c_blocked, GateForm form, hipStream_t stream) {
   BH_REQUIRE(gemm_turns_can(M, N, K, mode, blocks, parts), "gemm_turns: M=%d N=%d K=%d with %d blocks per wave in %d parts of K is not a product this kernel takes", M, N, K, blocks, parts);
   if (mode == 2) launch<2>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
+  else if (mode == 4) launch<4>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
   else if (mode == 1) launch<1>(a, w, c, blocks, M, N, K, accumulate, parts, 0, form, stream);
   else if (mode == 3) launch<3>(a, w, c, blocks, M, N, K, 0, 1, c_blocked, form, stream);
   else launch<0>(a, w, c, blocks, M, N, K, 0, 1, 0, form, stream);

@@ -182,7 +182,8 @@ class KernelSizes:
             "bh_attention_bf16_writes_blocked": [i, i, i, i, i],
             "bh_attention_decode_fused": [p, p, p, p, p, p, p, i, p, p, i, i, i, i, f, i, i, i, p, p, i, f, p, p, i, i,
                                           i, i, p],
-            "bh_gemm_bf16_clamped_glu": [p, p, p, i, i, i, f, f, f, p, i, i, p],
+            "bh_gemm_bf16_clamps": [i, i, i],
+            "bh_gemm_bf16_clamped_glu": [p, p, p, i, i, i, f, f, i, i, p],
             "bh_attention_decode_pairs": [p, i, i, p, p, p, p, p, p, i, p, p, i, i, i, i, f, i, i, i, p, p, i, f, p, p, i, i, i, i, p, p, i, f, p, f, i, f, p],
             "bh_row_angles": [p, p, f, p, p, i, i, p],
             "bh_kv_order": [i, i],
@@ -387,6 +388,7 @@ class HipKernels(KernelSizes):
         self.state_in_banks = True      # the kernels that move a state on take `seq_to`, the rows to leave it in
         self._plans: dict = {}      # (m, n, k, packed, activation) -> what the library says of such a product
         self._squares: dict = {}    # (m, n, k) -> which product squares its output (`gemm_relu_squared`), or 0
+        self._clamps: dict = {}     # (m, n, k) -> which gated product clamps (`gemm_clamped_glu`), or 0
         self._bare: dict = {}       # (m, n, k) -> the parts that `gemm_bare` leaves such a product in, or 0
         self.page_size = int(self.lib.bh_page_size())
         if self.page_size != _build.source_page_size():
@@ -665,7 +667,7 @@ class HipKernels(KernelSizes):
                                                 self._ptr(out, "gemm out"), m, n, k, gate, self._stream()))
         return True
 
-    def gemm_clamped_glu(self, a, w, out, limit, alpha, shift=1.0) -> bool:
+    def gemm_clamped_glu(self, a, w, out, limit, alpha) -> bool:
         """`gemm` of a [n, K] with w [2 ff, K] (gate rows, then up rows) and `clamped_glu` of the result into `out` [n, ff], in one product;
         False, having done nothing, where the library has none of these operands that does so (then call the two)."""
         if (not isinstance(w, PackedWeight) or isinstance(a, NormedRows) or a.dim() != 2 or a.dtype != torch.bfloat16 or out.dtype != torch.bfloat16
@@ -674,15 +676,16 @@ class HipKernels(KernelSizes):
         (m, k), width = a.shape, out.shape[1]
         if tuple(out.shape) != (m, width) or w.shape[0] != 2 * width:
             raise KernelError(f"gemm_clamped_glu: shapes a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
-        a_block_rows, writes, _, _, scratch_bytes, _ = self._product(m, width, k, 1, 1)
-        c_block_rows = _block_rows(out)
-        if c_block_rows and not (writes == 2 or (writes == 1 and c_block_rows == 16)):
+        clamps, c_block_rows = self._clamps.get((m, width, k)), _block_rows(out)
+        if clamps is None:
+            clamps = self._clamps[(m, width, k)] = int(self.lib.bh_gemm_bf16_clamps(m, width, k))
+        if not clamps or c_block_rows not in ((0, 16) if clamps == 1 else (0, 8, 16)):
             return False
+        a_block_rows = self._product(m, width, k, 1, 1)[0]
         a = self._in_blocks_of(a, a_block_rows)
-        scratch = torch.empty(scratch_bytes // 4, dtype=torch.float32, device=self.device) if scratch_bytes else None
         self._check(self.lib.bh_gemm_bf16_clamped_glu(
-            self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), m, width, k, float(limit), float(alpha), float(shift),
-            self._ptr(scratch, "gemm scratch", None, True), a_block_rows, c_block_rows, self._stream()))
+            self._ptr(a, "gemm a"), self._ptr(w.data, "gemm w"), self._ptr(out, "gemm out"), m, width, k, float(limit), float(alpha),
+            a_block_rows, c_block_rows, self._stream()))
         return True
 
     def gemm_relu_squared(self, a, w, out) -> bool:
