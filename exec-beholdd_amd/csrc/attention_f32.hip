@@ -378,7 +378,7 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
   }
 }
 
-constexpr int parts_of(int slices, int waves) { return slices >= 3 && waves == 8 ? 2 : 1; }
+constexpr int parts_of(int slices, int waves) { return slices >= 3 && (waves == 8 || waves == 2) ? 2 : 1; }
 
 template <int P, int NR, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(F32Attention t, int n_rows) {
@@ -620,6 +620,10 @@ bool tiles_pay(int n_rows, int n_seqs, int H, int KVH, int hd, int span, const i
 }
 
 constexpr int many_waves(int slices) { return slices <= 4 ? 8 : 4; }
+// Rows that see one page have work for one wave, or for two where the eight waves of longer rows take half pages: the parts and the order
+// in which their sums are added are then the same, so that a row's result does not hang on how many pages its step may see (a captured
+// step is launched for more than its rows hold; idle waves add zeros).
+constexpr int one_page_waves(int slices) { return parts_of(slices, many_waves(slices)); }
 
 // A decode step from its projection rows: as many waves a row and head as `launch` gives it.  In two launches / one, us, 8 rows of 100 keys,
 // 16 heads of 128 on 8 7.3 / 5.9, 4 rows of 300 keys, 4 heads of 64 on 2 7.5 / 5.6.
@@ -627,7 +631,8 @@ template <int P>
 void launch_fused(const F32Attention& t, int n_rows, int most_pages, hipStream_t stream) {
   const long units = bh_compute_units(), each = (long)n_rows * t.H;
   const dim3 grid(n_rows, t.H);
-  if (most_pages <= 1 || (most_pages <= 4 && each >= 4 * units)) attention_f32_fused_kernel<P, 1><<<grid, 64, 0, stream>>>(t);
+  if (most_pages <= 1 && each < 2 * units) attention_f32_fused_kernel<P, one_page_waves(P)><<<grid, 64 * one_page_waves(P), 0, stream>>>(t);
+  else if (most_pages <= 1 || (most_pages <= 4 && each >= 4 * units)) attention_f32_fused_kernel<P, 1><<<grid, 64, 0, stream>>>(t);
   else if (each < 2 * units) attention_f32_fused_kernel<P, many_waves(P)><<<grid, 64 * many_waves(P), 0, stream>>>(t);
   else attention_f32_fused_kernel<P, 4><<<grid, 256, 0, stream>>>(t);
 }
@@ -652,6 +657,8 @@ void launch(const F32Attention& t, int n_rows, int n_seqs, int most_pages, bool 
   if (most_pages <= 1 || (most_pages <= 4 && (long)n_rows * t.H >= (prompts ? 2L : 4L) * bh_compute_units())) {
     constexpr int FEW = P <= 4 ? 1 : NR;
     if (prompts) attention_f32_kernel<P, FEW, 1><<<dim3((n_rows + FEW - 1) / FEW, t.H), 64, 0, stream>>>(t, n_rows);
+    else if ((long)n_rows * t.H < 2 * bh_compute_units())
+      attention_f32_kernel<P, 1, one_page_waves(P)><<<dim3(n_rows, t.H), 64 * one_page_waves(P), 0, stream>>>(t, n_rows);
     else attention_f32_kernel<P, 1, 1><<<dim3(n_rows, t.H), 64, 0, stream>>>(t, n_rows);
     return;
   }

@@ -83,3 +83,30 @@ def test_float32_decode_attention_says_when_it_cannot(K):
     assert asked(rows, qw=weight) is False                           # weights of another type
     assert asked(rows, tables=(cos, cos)) is False                   # a rotation of half of the head
     assert asked(rows, step=Layout(True, layout.seq_start, 1, 2, 69)) is False
+
+
+@pytest.mark.parametrize("lengths,news", [([1, 64, 33], 1), ([2, 63], 2), ([64] * 3, 3)])
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(8, 4, 128), (4, 2, 96), (4, 2, 64), (2, 1, 160)])
+def test_float32_rows_of_one_page_whatever_the_step_may_see(K, heads, kv_heads, head_dim, lengths, news):
+    """A captured step is launched for more pages than its rows hold: the results are, bit for bit, those of a launch that knows how few."""
+    n, width = len(lengths), (heads + 2 * kv_heads) * head_dim
+    kp, vp, table, _, _ = make_cache(n, lengths, kv_heads, head_dim, torch.float32, seed=head_dim + n)
+    g = torch.Generator().manual_seed(head_dim)
+    positions = torch.cat([torch.arange(max(length - news, 0), length) for length in lengths]).int()
+    counts = [min(news, length) for length in lengths]
+    rows = sum(counts)
+    row_seq = torch.repeat_interleave(torch.arange(n), torch.tensor(counts)).int()
+    start = torch.tensor([0] + counts).cumsum(0).int()
+    q, qkv = torch.randn(rows, heads * head_dim, generator=g), torch.randn(rows, width, generator=g)
+    results = []
+    for furthest in (63, 1023):
+        out = torch.full((rows, heads * head_dim), float("nan"), device="cuda:0")
+        layout = Layout(news == 1, dev(start), n, news, furthest)
+        K.attention(dev(q), out, dev(kp), dev(vp), dev(table), dev(row_seq), dev(positions), heads, kv_heads, head_dim, 0.1, 0, layout=layout)
+        results.append([out])
+        if news == 1:
+            out, k_pages, v_pages = torch.full_like(out, float("nan")), dev(kp), dev(vp)
+            assert K.attention_decode_fused(dev(qkv), out, None, None, 1e-5, None, None, dev(positions), k_pages, v_pages, dev(table), heads, kv_heads,
+                                            head_dim, 0.1, 0, True, layout) is True
+            results[-1] += [out, k_pages, v_pages]
+    assert all(torch.equal(a, b) and not a.isnan().any() for a, b in zip(*results))
