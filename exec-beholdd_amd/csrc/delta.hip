@@ -247,19 +247,6 @@ struct DeltaChunks {
   float* queries;       // [n_rows][H][dim]
 };
 
-// x of the lane whose number differs in the bits of a group of 2, 4, 8 or 16 neighbours, added: all lanes of the group end with the sum
-template <int SL>
-__device__ inline float slices_sum(float x) {
-  auto moved = [](float v, auto ctrl) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  if constexpr (SL >= 2) x += moved(x, std::integral_constant<int, 0xB1>());      // neighbours swapped
-  if constexpr (SL >= 4) x += moved(x, std::integral_constant<int, 0x4E>());      // pairs swapped
-  if constexpr (SL >= 8) x += moved(x, std::integral_constant<int, 0x141>());     // halves of a row of 16 lanes mirrored
-  if constexpr (SL >= 16) x += moved(x, std::integral_constant<int, 0x140>());    // rows mirrored
-  return x;
-}
-
 template <int R, int SL, int C>
 __global__ __launch_bounds__(DR_WAVES * BH_WAVE) void delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ beside,
                                                                         float* __restrict__ state, long slot_stride,

@@ -223,6 +223,199 @@ __global__ __launch_bounds__(256, (R <= 16 ? 2 : 1)) void gla_scan_kernel(const 
   }
 }
 
+// The same walk for steps with many rows a sequence and rows of whole pieces of four: a thread keeps 16 elements of each of C columns, the SL
+// threads of a column are neighbouring lanes (elements in turns of four: slice, slice + SL, ...) and add their shares by data-parallel
+// moves.  What a row's decays, keys and queries cost in LDS reads, which bound the walk above, is shared by C columns, and no shares
+// go through LDS.  The first tile's workgroup makes the carried queries, a thread a key channel.  Bound by the multiplications (three an
+// element of the state and row, packed ones are not used) and, at one wave a SIMD, by a row's chain of them.  With the joining of the chunks, us:
+// wkv, 64 heads of 64, 2,048 rows 273 -> 128; eight prompts of 512 rows, 32 heads 271 -> 126; gla, 8 heads of 128, 2,048 rows 109 -> 86,
+// 16 heads of 256, 1,000 rows 1,275 -> 286.  Four columns a thread: 154, 165, 103, 334.
+#define GC_R 16
+template <typename T, int SL, int C, int WAVES, int RULE>
+__global__ __launch_bounds__(WAVES * BH_WAVE) void gla_columns_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int row_stride,
+                                                                      const float* __restrict__ z, int z_stride, const float* __restrict__ bias,
+                                                                      float inv_tau, const float* __restrict__ bonus, float q_scale,
+                                                                      float* __restrict__ state, long slot_stride, const int32_t* __restrict__ seq_start,
+                                                                      const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
+                                                                      float* __restrict__ out, int H, int dim, int vdim, GlaChunks chunks) {
+  constexpr int DP = GC_R * SL, PIECES = DP / 4, PER_WAVE = BH_WAVE / SL * C, COLS = WAVES * PER_WAVE, THREADS = WAVES * BH_WAVE;
+  constexpr int EACH = GLA_STAGE * PIECES / THREADS, V_PIECES = GLA_STAGE * COLS / 4, V_EACH = (V_PIECES + THREADS - 1) / THREADS;
+  constexpr int KEPT = (DP + THREADS - 1) / THREADS;
+  static_assert(EACH * THREADS == GLA_STAGE * PIECES && THREADS % PIECES == 0, "a thread's pieces are of the same key channels");
+  __shared__ float4 a_s[GLA_STAGE * PIECES], k_s[GLA_STAGE * PIECES], q_s[GLA_STAGE * PIECES];
+  __shared__ float4 v_s[V_PIECES];
+  __shared__ float own_s[GLA_STAGE];
+  const int seq = blockIdx.x / chunks.count, chunk = blockIdx.x % chunks.count, head = blockIdx.y, v0 = blockIdx.z * COLS;
+  const int seq_first = seq_start[seq], seq_stop = seq_start[seq + 1];
+  const int in_chunks = chunks.rows > 0 ? (seq_stop - seq_first + chunks.rows - 1) / chunks.rows : 1;
+  const int start = seq_first + chunk * chunks.rows;
+  const int stop = (chunks.rows > 0 && start + chunks.rows < seq_stop) ? start + chunks.rows : seq_stop;
+  if (chunk > 0 && chunk >= in_chunks) return;
+  const bool apart = in_chunks > 1, keeps = apart && blockIdx.z == 0;
+  const int lane = threadIdx.x % BH_WAVE, slice = lane % SL, local = threadIdx.x / BH_WAVE * PER_WAVE + lane / SL * C, column0 = v0 + local;
+  const bool has_columns = column0 < vdim;      // (all C of them: vdim is a multiple)
+  float* mine = apart ? chunks.states + ((size_t)(seq * chunks.count + chunk) * H + head) * dim * vdim
+                      : state + (size_t)seq_to[seq] * slot_stride + (size_t)head * dim * vdim;
+  const float* from = state + (size_t)seq_slot[seq] * slot_stride + (size_t)head * dim * vdim;
+  float S[C][GC_R];
+#pragma unroll
+  for (int r = 0; r < GC_R; ++r) {
+    const int d = 4 * (slice + SL * (r / 4)) + r % 4;
+#pragma unroll
+    for (int c = 0; c < C; ++c) S[c][r] = chunk == 0 && has_columns && d < dim ? from[(size_t)d * vdim + column0 + c] : 0.f;
+  }
+  auto decay_of = [&](float x) { return RULE == RULE_WKV ? expf(-expf(x)) : expf(log_sigmoid_f32(x) * inv_tau); };
+  float kept[KEPT];
+#pragma unroll
+  for (int j = 0; j < KEPT; ++j) kept[j] = 1.0f;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int my_d = threadIdx.x % PIECES * 4, my_t = threadIdx.x / PIECES;      // of a thread's pieces: key channels, and row of the first
+  const bool real = my_d < dim;
+  const float4 bias4 = real ? load_four(bias + head * dim + my_d) : zero;
+  const float4 bonus4 = RULE == RULE_WKV && real ? load_four(bonus + head * dim + my_d) : zero;
+  float4 z_ahead[EACH], k_ahead[EACH], q_ahead[EACH], v_ahead[V_EACH];
+  auto ask = [&](int row0) {
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const int row = row0 + my_t + i * (THREADS / PIECES);
+      z_ahead[i] = k_ahead[i] = q_ahead[i] = zero;
+      if (real && row < stop) {
+        const size_t at = (size_t)row * row_stride + head * dim + my_d;
+        z_ahead[i] = load_four(z + (size_t)row * z_stride + head * dim + my_d);
+        k_ahead[i] = load_four(k + at);
+        q_ahead[i] = load_four(q + at);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < V_EACH; ++i) {
+      const int e = threadIdx.x + THREADS * i, row = row0 + e / (COLS / 4), c = v0 + e % (COLS / 4) * 4;
+      v_ahead[i] = e < V_PIECES && row < stop && c < vdim ? load_four(v + (size_t)row * row_stride + head * vdim + c) : zero;
+    }
+  };
+  ask(start);
+  for (int row0 = start; row0 < stop; row0 += GLA_STAGE) {
+    const int n = stop - row0 < GLA_STAGE ? stop - row0 : GLA_STAGE;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const float4 x = z_ahead[i], kk = k_ahead[i];
+      float4 qq = q_ahead[i];
+      qq.x *= q_scale, qq.y *= q_scale, qq.z *= q_scale, qq.w *= q_scale;
+      const int e = threadIdx.x + THREADS * i;
+      a_s[e] = real ? make_float4(decay_of(x.x + bias4.x), decay_of(x.y + bias4.y), decay_of(x.z + bias4.z), decay_of(x.w + bias4.w)) : zero;
+      k_s[e] = kk;
+      q_s[e] = qq;
+      if constexpr (RULE == RULE_WKV) {
+        float own = fmaf(qq.x * bonus4.x, kk.x, fmaf(qq.y * bonus4.y, kk.y, fmaf(qq.z * bonus4.z, kk.z, qq.w * bonus4.w * kk.w)));
+#pragma unroll
+        for (int off = PIECES / 2; off > 0; off >>= 1) own += __shfl_xor(own, off, BH_WAVE);
+        if (my_d == 0) own_s[my_t + i * (THREADS / PIECES)] = own;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < V_EACH; ++i)
+      if (threadIdx.x + THREADS * i < V_PIECES) v_s[threadIdx.x + THREADS * i] = v_ahead[i];
+    lds_barrier();
+    if (row0 + GLA_STAGE < stop) ask(row0 + GLA_STAGE);
+    if (keeps) {
+      const float* decays = reinterpret_cast<const float*>(a_s);
+      const float* queries = reinterpret_cast<const float*>(q_s);
+#pragma unroll
+      for (int j = 0; j < KEPT; ++j) {
+        const int d = threadIdx.x + THREADS * j;
+        if (d >= dim) break;
+        float a[GLA_STAGE], x[GLA_STAGE];
+#pragma unroll
+        for (int t = 0; t < GLA_STAGE; ++t) a[t] = decays[t * DP + d], x[t] = queries[t * DP + d];
+#pragma unroll
+        for (int t = 0; t < GLA_STAGE; ++t) {
+          if (t >= n) break;
+          const float before = kept[j];
+          kept[j] *= a[t];
+          if (chunk > 0) chunks.queries[((size_t)(row0 + t) * H + head) * dim + d] = (RULE == RULE_WKV ? before : kept[j]) * x[t];
+        }
+      }
+    }
+    float o_kept[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) o_kept[c] = 0.f;
+    // a row's operands are asked for while the row before is walked
+    struct Row {
+      float4 a[GC_R / 4], k[GC_R / 4], q[GC_R / 4];
+      float v[C], own;
+    };
+    auto fetch = [&](Row& row, int t) {
+      t = t < GLA_STAGE ? t : GLA_STAGE - 1;
+#pragma unroll
+      for (int i = 0; i < GC_R / 4; ++i) {
+        const int at = t * PIECES + slice + SL * i;
+        row.a[i] = a_s[at], row.k[i] = k_s[at], row.q[i] = q_s[at];
+      }
+#pragma unroll
+      for (int c = 0; c < C; ++c) row.v[c] = reinterpret_cast<const float*>(v_s)[t * COLS + local + c];
+      row.own = RULE == RULE_WKV ? own_s[t] : 0.f;
+    };
+    auto walk = [&](const Row& row, int t) {
+      float sum[C][2];
+#pragma unroll
+      for (int c = 0; c < C; ++c) sum[c][0] = sum[c][1] = 0.f;
+#pragma unroll
+      for (int i = 0; i < GC_R / 4; ++i) {
+        const float a4[4] = {row.a[i].x, row.a[i].y, row.a[i].z, row.a[i].w}, k4[4] = {row.k[i].x, row.k[i].y, row.k[i].z, row.k[i].w};
+        const float q4[4] = {row.q[i].x, row.q[i].y, row.q[i].z, row.q[i].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int c = 0; c < C; ++c) {
+            float& s = S[c][4 * i + r];
+            if (RULE == RULE_WKV) sum[c][r & 1] = fmaf(s, q4[r], sum[c][r & 1]);
+            s *= a4[r];
+            s = fmaf(k4[r], row.v[c], s);
+            if (RULE == RULE_GLA) sum[c][r & 1] = fmaf(s, q4[r], sum[c][r & 1]);
+          }
+      }
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        float o = slices_sum<SL>(sum[c][0] + sum[c][1]);
+        if constexpr (RULE == RULE_WKV) o = fmaf(row.own, row.v[c], o);
+        if (slice == (t & (SL - 1))) o_kept[c] = o;
+      }
+      // every SL rows (and behind the last) each lane of a column writes the row it kept
+      if ((t & (SL - 1)) == SL - 1 || t == n - 1) {
+        const int kept_row = (t & ~(SL - 1)) + slice;
+        if (kept_row <= t && has_columns) {
+#pragma unroll
+          for (int c = 0; c < C; ++c) out[(size_t)(row0 + kept_row) * H * vdim + head * vdim + column0 + c] = o_kept[c];
+        }
+      }
+    };
+    Row even, odd;
+    fetch(even, 0);
+#pragma unroll 1
+    for (int t = 0; t < n; t += 2) {
+      fetch(odd, t + 1);
+      walk(even, t);
+      if (t + 1 >= n) break;
+      fetch(even, t + 2);
+      walk(odd, t + 1);
+    }
+    lds_barrier();      // the stage's LDS is written again
+  }
+#pragma unroll
+  for (int r = 0; r < GC_R; ++r) {
+    const int d = 4 * (slice + SL * (r / 4)) + r % 4;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (has_columns && d < dim) mine[(size_t)d * vdim + column0 + c] = S[c][r];
+  }
+  if (keeps) {
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j) {
+      const int d = threadIdx.x + THREADS * j;
+      if (d < dim) chunks.decays[((size_t)(seq * chunks.count + chunk) * H + head) * dim + d] = kept[j];
+    }
+  }
+}
+
 // One thread a state element (sequence, head, key channel, value column): through the sequence's chunks in order,
 // S_in(c + 1) = A(c) S_in(c) + S_loc(c), A(c) the chunk's product of decays; a chunk's place in `states` then holds the state
 // it started from (for chunk_carry), and the state after the last chunk goes to the sequence's slot.
@@ -338,6 +531,44 @@ extern "C" int bh_gla_chunk_rows(int n_seqs, int max_rows, int H, int dim, int v
   return rows >= max_rows ? max_rows : rows;
 }
 
+// The chunks' states joined, and what the later chunks' rows owe them.
+static int gla_join(const GlaChunks& chunks, float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to,
+                    float* out, int n_seqs, int H, int dim, int vdim, hipStream_t stream) {
+  if (chunks.rows == 0) return 0;
+  const size_t per = (size_t)H * dim * vdim;
+  gla_combine_kernel<<<dim3((unsigned)((per + 255) / 256), n_seqs), 256, 0, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, seq_to, H, dim, vdim);
+  if (int status = bh_check_launch("gla_combine")) return status;
+  return bh_chunk_carry(chunks.states, chunks.queries, chunks.rows, chunks.count, seq_start, out, n_seqs, H, dim, vdim, stream);
+}
+
+// Which steps share what is read between columns: long walks (a decode step is its state's way in and out) of which a compute unit has one at
+// least; below that a row's chain of steps is the time, and that of 16 elements a thread is the longer one (wkv, 64 heads of 64, 2,048 rows, us,
+// apart / in columns: 1,024 workgroups 273 / 128, 512 workgroups 266 / 195; one sequence of 100 rows, 64 heads, 64 workgroups 64 / 62; 32
+// heads, 128 workgroups 293 / 306; gla, 8 heads of 128, 64 workgroups 321 / 314; 20 heads of 48, 333 rows, 100 workgroups 59 / 70).
+#define GC_ROWS 64
+#define GC_C 2
+static bool gla_columns_take(long walks, int max_rows, int H, int dim, int vdim) {
+  return max_rows >= GC_ROWS && dim % 4 == 0 && dim > 32 && dim <= 256 && vdim % 4 == 0 && vdim > 32 &&
+         walks * H * ((vdim + 63) / 64) >= (long)bh_compute_units();
+}
+
+template <int RULE, typename T>
+static void gla_columns(const T* q, const T* k, const T* v, int row_stride, const float* z, int z_stride, const float* bias, float inv_tau,
+                        const float* bonus, float q_scale, float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot,
+                        const int32_t* seq_to, float* out, int n_seqs, int H, int dim, int vdim, const GlaChunks& chunks, hipStream_t stream) {
+#define BH_GC(SL, WAVES)                                                                                                                \
+  do {                                                                                                                                  \
+    static_assert((WAVES) * (BH_WAVE / (SL)) * GC_C == 64, "a tile is 64 columns");                                                     \
+    gla_columns_kernel<T, SL, GC_C, WAVES, RULE><<<dim3(n_seqs * chunks.count, H, (vdim + 63) / 64), (WAVES) * BH_WAVE, 0, stream>>>(   \
+        q, k, v, row_stride, z, z_stride, bias, inv_tau, bonus, q_scale, state, slot_stride, seq_start, seq_slot, seq_to, out, H, dim, vdim, \
+        chunks);                                                                                                                        \
+  } while (0)
+  if (dim <= 64) BH_GC(4, 2);
+  else if (dim <= 128) BH_GC(8, 4);
+  else BH_GC(16, 8);
+#undef BH_GC
+}
+
 // What both rules' entry points share.  q, k [rows][row_stride] (dtype): H heads of `dim` from a row's start; v: H heads of vdim.
 template <int RULE>
 static int scan_run(const char* what, const void* q, const void* k, const void* v, int dtype, int row_stride, const float* z, int z_stride,
@@ -359,6 +590,18 @@ static int scan_run(const char* what, const void* q, const void* k, const void* 
     chunks.queries = chunks.decays + (size_t)n_seqs * chunks.count * H * dim;
   }
   BH_REQUIRE((long)n_seqs * chunks.count < (1L << 31), "%s: too many chunks", what);
+  const size_t piece = 4 * (dtype == BH_F32 ? sizeof(float) : 2);
+  const bool in_columns = gla_columns_take((long)n_seqs * chunks.count, max_rows, H, dim, vdim) && row_stride % 4 == 0 && z_stride % 4 == 0 &&
+                          ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % piece == 0 && ((uintptr_t)z | (uintptr_t)bias | (uintptr_t)bonus) % 16 == 0;
+  if (in_columns) {
+    if (dtype == BH_F32) gla_columns<RULE>((const float*)q, (const float*)k, (const float*)v, row_stride, z, z_stride, bias, inv_tau, bonus, q_scale, state,
+                                           slot_stride, seq_start, seq_slot, seq_to, out, n_seqs, H, dim, vdim, chunks, stream);
+    else if (dtype == BH_BF16) gla_columns<RULE>((const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, row_stride, z, z_stride, bias, inv_tau, bonus, q_scale,
+                                                 state, slot_stride, seq_start, seq_slot, seq_to, out, n_seqs, H, dim, vdim, chunks, stream);
+    else return bh_fail("%s: unknown dtype %d", what, dtype);
+    if (int status = bh_check_launch(what)) return status;
+    return gla_join(chunks, state, slot_stride, seq_start, seq_slot, seq_to, out, n_seqs, H, dim, vdim, stream);
+  }
   const int VT = gla_tile((long)n_seqs * chunks.count, H, dim, vdim), SL = 256 / VT;
   int R = 1;
   while (R * SL < dim) R *= 2;
@@ -389,11 +632,7 @@ static int scan_run(const char* what, const void* q, const void* k, const void* 
 #undef BH_GLA_R
 #undef BH_GLA
   if (int status = bh_check_launch(what)) return status;
-  if (chunks.rows == 0) return 0;
-  const size_t per = (size_t)H * dim * vdim;
-  gla_combine_kernel<<<dim3((unsigned)((per + 255) / 256), n_seqs), 256, 0, stream>>>(chunks, state, slot_stride, seq_start, seq_slot, seq_to, H, dim, vdim);
-  if (int status = bh_check_launch("gla_combine")) return status;
-  return bh_chunk_carry(chunks.states, chunks.queries, chunks.rows, chunks.count, seq_start, out, n_seqs, H, dim, vdim, stream);
+  return gla_join(chunks, state, slot_stride, seq_start, seq_slot, seq_to, out, n_seqs, H, dim, vdim, stream);
 }
 
 // proj [rows][proj_stride] (dtype): a row holds H heads of q and of k (dim each) from q_off and k_off and H heads of v (vdim) from
