@@ -285,34 +285,51 @@ extern "C" int bh_clamped_glu(const void* gu, int dtype, void* out, int n_rows, 
 //   experts_gather    the pairs' input rows side by side, expert after expert, for products of many rows
 //   experts_combine   h_res[row] += sum_j weight_j * y[place of pair (row, j)], j in order
 
-// One workgroup an expert: it walks over all pairs in order and keeps those that chose it.
-__global__ __launch_bounds__(256) void experts_group_kernel(const int32_t* __restrict__ chosen, int n_pairs, int32_t* __restrict__ list,
-                                                            int capacity, int32_t* __restrict__ counts) {
-  __shared__ int wave_count[4];
-  const int e = blockIdx.x, lane = threadIdx.x & (BH_WAVE - 1), wave = threadIdx.x / BH_WAVE;
-  int base = 0;
-  for (int p0 = 0; p0 < n_pairs; p0 += 256) {
-    const int p = p0 + threadIdx.x;
-    const bool mine = p < n_pairs && chosen[p] == e;
-    const unsigned long long mask = __ballot(mine);
-    const int before = __popcll(mask & ((1ull << lane) - 1ull));
-    if (lane == 0) wave_count[wave] = __popcll(mask);
-    __syncthreads();
-    int offset = base, total = 0;
-    for (int w = 0; w < 4; ++w) {
-      if (w < wave) offset += wave_count[w];
-      total += wave_count[w];
+// One workgroup an expert.  Every wave takes a run of the pairs and goes over it twice, counting those that chose the expert and then
+// writing them behind those of the waves before it: two trips to memory and one barrier, whatever the number of pairs, since the
+// loads of a run do not wait for each other.  Bound by those trips.  8,400 pairs of 32 experts 6.0 us, 21.0 with a barrier every
+// 256 pairs.
+#define EG_AHEAD 4      // pieces of 64 pairs asked for together
+__global__ __launch_bounds__(1024) void experts_group_kernel(const int32_t* __restrict__ chosen, int n_pairs, int32_t* __restrict__ list,
+                                                             int capacity, int32_t* __restrict__ counts) {
+  __shared__ int wave_count[16];
+  const int e = blockIdx.x, lane = threadIdx.x & (BH_WAVE - 1), wave = threadIdx.x / BH_WAVE, waves = blockDim.x / BH_WAVE;
+  const int run = (n_pairs + EG_AHEAD * blockDim.x - 1) / (EG_AHEAD * blockDim.x) * (EG_AHEAD * BH_WAVE);      // pairs of a wave
+  const int first = wave * run, stop = first + run < n_pairs ? first + run : n_pairs;
+  auto each = [&](auto take) {      // take(pair, which lanes' pairs chose the expert)
+    for (int p0 = first; p0 < stop; p0 += EG_AHEAD * BH_WAVE) {
+      bool mine[EG_AHEAD];
+#pragma unroll
+      for (int i = 0; i < EG_AHEAD; ++i) {
+        const int p = p0 + i * BH_WAVE + lane;
+        mine[i] = chosen[p < stop ? p : stop - 1] == e && p < stop;
+      }
+#pragma unroll
+      for (int i = 0; i < EG_AHEAD; ++i) take(p0 + i * BH_WAVE + lane, __ballot(mine[i]));
     }
-    if (mine) list[(size_t)e * capacity + offset + before] = p;
-    base += total;
-    __syncthreads();
+  };
+  int count = 0;
+  each([&](int, unsigned long long mask) { count += __popcll(mask); });
+  if (lane == 0) wave_count[wave] = count;
+  __syncthreads();
+  int at = 0, total = 0;
+  for (int w = 0; w < waves; ++w) {
+    if (w < wave) at += wave_count[w];
+    total += wave_count[w];
   }
-  if (threadIdx.x == 0) counts[e] = base;
+  int32_t* to = list + (size_t)e * capacity;
+  each([&](int p, unsigned long long mask) {
+    if (mask >> lane & 1ull) to[at + __popcll(mask & ((1ull << lane) - 1ull))] = p;
+    at += __popcll(mask);
+  });
+  if (threadIdx.x == 0) counts[e] = total;
 }
 
 extern "C" int bh_experts_group(const int32_t* chosen, int n_pairs, int32_t* list, int capacity, int32_t* counts, int E, hipStream_t stream) {
   BH_REQUIRE(n_pairs > 0 && E > 0 && capacity > 0, "experts_group: sizes must be positive");
-  experts_group_kernel<<<E, 256, 0, stream>>>(chosen, n_pairs, list, capacity, counts);
+  // (a wave takes as many pairs as it asks for together, until there are sixteen)
+  const int waves = (n_pairs + EG_AHEAD * BH_WAVE - 1) / (EG_AHEAD * BH_WAVE);
+  experts_group_kernel<<<E, BH_WAVE * (waves < 16 ? waves : 16), 0, stream>>>(chosen, n_pairs, list, capacity, counts);
   return bh_check_launch("experts_group");
 }
 
