@@ -92,6 +92,97 @@ __global__ __launch_bounds__(256) void short_conv_walk_kernel(const T* __restric
   }
 }
 
+// The same in pieces of four channels: a thread asks for all inputs of its stretch of SC_FAR rows together and waits for them once, where the
+// walk above has a load a row and its wait.  A stretch in which a sequence starts is walked row by row.  Bound by its bytes (the inputs once,
+// 3 in 19 of them twice, float32 outputs) and, with few waves a compute unit, the way to memory.  2,100 rows of 6,144 and of 3,072 channels, on average 32.9 -> 23.8 us.
+#define SC_FAR 16
+
+template <typename T>
+struct FourOf {      // four channels' inputs as they come
+  float4 raw;
+  __device__ void load(const T* from) { raw = load_four(from); }
+  __device__ float4 values() const { return raw; }
+};
+template <>
+struct FourOf<bf16_t> {
+  uint2 raw;
+  __device__ void load(const bf16_t* from) { raw = *reinterpret_cast<const uint2*>(from); }
+  __device__ float4 values() const {
+    return make_float4(bf16_bits_to_f32((uint16_t)(raw.x & 0xffffu)), bf16_bits_to_f32((uint16_t)(raw.x >> 16)),
+                       bf16_bits_to_f32((uint16_t)(raw.y & 0xffffu)), bf16_bits_to_f32((uint16_t)(raw.y >> 16)));
+  }
+};
+
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void short_conv_pieces_kernel(const T* __restrict__ u, int row_stride, int first,
+                                                                const float* __restrict__ w, const float* __restrict__ bias,
+                                                                float* __restrict__ state, long slot_stride,
+                                                                const int32_t* __restrict__ row_seq, const int32_t* __restrict__ seq_start,
+                                                                const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_to,
+                                                                float* __restrict__ out, int n_rows, int channels, int silu) {
+  const int c = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+  if (c >= channels) return;
+  const int r0 = blockIdx.y * SC_FAR, r1 = r0 + SC_FAR < n_rows ? r0 + SC_FAR : n_rows;
+  const T* column = u + first + c;
+  FourOf<T> ahead[SC_FAR];
+#pragma unroll
+  for (int i = 0; i < SC_FAR; ++i) ahead[i].load(column + (size_t)(r0 + i < r1 ? r0 + i : r1 - 1) * row_stride);
+  float wc[4][TAPS], b[4], win[4][TAPS];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    b[v] = bias ? bias[c + v] : 0.f;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) wc[v][j] = w[(size_t)(c + v) * TAPS + j];
+  }
+  int seq = row_seq[r0], seq_stop = seq_start[seq + 1];
+  auto enter = [&](int row) {      // the inputs before a sequence's row
+    const int t = row - seq_start[seq];
+    const float* old = state + (size_t)seq_slot[seq] * slot_stride;
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int back = TAPS - 1 - j;
+      const float4 x = back <= t ? load_four(column + (size_t)(row - back) * row_stride) : make_float4(0.f, 0.f, 0.f, 0.f);
+      win[0][j] = x.x, win[1][j] = x.y, win[2][j] = x.z, win[3][j] = x.w;
+      if (back > t) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) win[v][j] = old[(size_t)(TAPS - 1 + t - back) * channels + c + v];
+      }
+    }
+  };
+  enter(r0);
+#pragma unroll
+  for (int i = 0; i < SC_FAR; ++i) {
+    const int row = r0 + i;
+    if (row >= r1) break;
+    if (row >= seq_stop) {
+      seq = row_seq[row], seq_stop = seq_start[seq + 1];
+      enter(row);
+    }
+    const float4 x = ahead[i].values();
+    win[0][TAPS - 1] = x.x, win[1][TAPS - 1] = x.y, win[2][TAPS - 1] = x.z, win[3][TAPS - 1] = x.w;
+    float y[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float acc = b[v];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc = fmaf(wc[v][j], win[v][j], acc);
+      y[v] = silu ? acc / (1.0f + expf(-acc)) : acc;
+    }
+    store_four(out + (size_t)row * channels + c, y[0], y[1], y[2], y[3]);
+    if (seq_to && row + 1 == seq_stop) {      // the window's later inputs are what the next step starts with
+      float* to = state + (size_t)seq_to[seq] * slot_stride;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 1; j < TAPS; ++j) to[(size_t)(j - 1) * channels + c + v] = win[v][j];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) win[v][j] = win[v][j + 1];
+  }
+}
+
 // seq_to [n_seqs]: the rows of the state to leave what the next step starts with in, none of which this step reads; or null: short_conv_state
 // does it.
 extern "C" int bh_short_conv(const void* u, int dtype, int row_stride, int first, const float* w, const float* bias,
@@ -104,6 +195,26 @@ extern "C" int bh_short_conv(const void* u, int dtype, int row_stride, int first
              first + channels, row_stride);
   BH_REQUIRE(taps == 1 || state != nullptr, "short_conv: more than one tap needs a state");
   if (n_rows >= 4 * SC_ROWS && taps >= 2 && taps <= 4 && (dtype == BH_F32 || dtype == BH_BF16)) {
+    const size_t piece = 4 * (dtype == BH_F32 ? sizeof(float) : 2);
+    if (channels % 4 == 0 && first % 4 == 0 && row_stride % 4 == 0 && (uintptr_t)u % piece == 0 && (uintptr_t)out % 16 == 0 &&
+        n_rows <= 65535 * SC_FAR) {
+      const int pieces = channels / 4, threads = (int)bh_piece_threads(pieces);
+      dim3 stretches((pieces + threads - 1) / threads, (n_rows + SC_FAR - 1) / SC_FAR);
+#define BH_SP(T, TAPS)                                                                                                              \
+  short_conv_pieces_kernel<T, TAPS><<<stretches, threads, 0, stream>>>((const T*)u, row_stride, first, w, bias, state, slot_stride, row_seq, \
+                                                                       seq_start, seq_slot, seq_to, out, n_rows, channels, silu)
+      if (dtype == BH_F32) {
+        if (taps == 2) BH_SP(float, 2);
+        else if (taps == 3) BH_SP(float, 3);
+        else BH_SP(float, 4);
+      } else {
+        if (taps == 2) BH_SP(bf16_t, 2);
+        else if (taps == 3) BH_SP(bf16_t, 3);
+        else BH_SP(bf16_t, 4);
+      }
+#undef BH_SP
+      return bh_check_launch("short_conv");
+    }
     dim3 walk((channels + 255) / 256, (n_rows + SC_ROWS - 1) / SC_ROWS);
 #define BH_SW(T, TAPS)                                                                                                              \
   short_conv_walk_kernel<T, TAPS><<<walk, 256, 0, stream>>>((const T*)u, row_stride, first, w, bias, state, slot_stride, row_seq, seq_start, \
