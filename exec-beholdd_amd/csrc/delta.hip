@@ -507,19 +507,29 @@ static DeltaShape delta_shape(int dim) {
   return {32, 16, 1};
 }
 
-// Rows of a chunk for a step whose longest sequence brings max_rows rows (max_rows and more: sequences are walked whole).  A walk is a
-// chain of rows, so long sequences are cut while the workgroups side by side do not fill the compute units; chunks but the first
-// carry dim more columns, which has to be worth it: three chunks at least.
+// Rows of a chunk for a step whose longest sequence brings max_rows rows (max_rows and more: sequences are walked whole): the number of chunks
+// with the least of an estimate.  A walk is a chain of rows, 0.33 us each until three workgroups share a compute unit, 0.14 us a workgroup
+// then; chunks but the first carry dim more columns, joining the chunks takes 7 us each, and what their rows owe 1 us for 1,600 rows of a head
+// of 128 x 128.  From 16 sizes, 8 to 96 heads of 128 x 128 and 512 to 4,096 rows, each at 7 to 10 numbers of chunks; us, with six workgroups a
+// compute unit wanted whatever a row costs then / by the estimate: 32 heads, 2,048 rows 384 / 349, 512 rows 143 / 117, 16 heads, 2,048
+// rows 252 / 215, 512 rows 108 / 91, 48 heads, 2,048 rows 501 / 455.
 extern "C" int bh_delta_chunk_rows(int n_seqs, int max_rows, int H, int dim, int vdim) {
   if (max_rows < 192 || n_seqs <= 0 || H <= 0 || dim <= 0 || vdim <= 0 || dim > 256) return max_rows;
   const int columns = delta_shape(dim).columns();
-  const long whole = (long)n_seqs * H * ((vdim + columns - 1) / columns), each = (long)n_seqs * H * ((vdim + dim + columns - 1) / columns);
-  long wanted = (6L * bh_compute_units() + each - 1) / each;
-  if (whole >= 4L * bh_compute_units() || wanted < 3) return max_rows;
-  if (wanted > max_rows / 64) wanted = max_rows / 64;
-  int rows = (int)((max_rows + wanted - 1) / wanted);
-  rows = (rows + DR_STAGE - 1) / DR_STAGE * DR_STAGE;
-  return rows >= max_rows ? max_rows : rows;
+  const long walks = (long)n_seqs * H, tiles = (vdim + columns - 1) / columns, later_tiles = (vdim + dim + columns - 1) / columns;
+  const auto chain = [](long workgroups) {
+    const long share = (workgroups + bh_compute_units() - 1) / bh_compute_units();
+    return share <= 2 ? 0.33 : 0.14 * (double)share;
+  };
+  const double owed = (double)walks * max_rows * dim * vdim / (16384.0 * 1600.0);
+  int best = max_rows;
+  double least = max_rows * chain(walks * tiles);
+  for (int wanted = 2; wanted <= max_rows / 64 && wanted <= 64; ++wanted) {
+    const int rows = ((max_rows + wanted - 1) / wanted + DR_STAGE - 1) / DR_STAGE * DR_STAGE, count = (max_rows + rows - 1) / rows;
+    const double cost = rows * chain(walks * (tiles + (count - 1) * later_tiles)) + owed + 7.0 * count;
+    if (rows < max_rows && cost < least) best = rows, least = cost;
+  }
+  return best;
 }
 
 extern "C" int bh_delta_takes(int dim, int vdim) { return dim > 0 && dim <= 512 && vdim > 0; }
