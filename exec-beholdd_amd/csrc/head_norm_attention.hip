@@ -95,6 +95,97 @@ __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_kerne
   }
 }
 
+// The same for steps of many rows, in pieces of four dimensions: the lanes of a head (pad / 4 of them, neighbours) keep it in registers, add its
+// squares up by exchanges and ask the mate of a half-split turn for its piece; a thread asks for the pieces of HN_HEADS heads at once.  The
+// kernel above goes through one head a wave after the other, an element a lane.  Bound by its bytes and, a third of it, the values,
+// whose tokens lie two bytes apart.  32 heads of 128 on 8, 64 dimensions turned: 2,048 rows 42.3 -> 29.6 us, 8,192 rows 144 -> 98.
+#define HN_HEADS 4
+template <typename T>
+__global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_pieces_kernel(
+    const T* __restrict__ proj, int row_stride, int first, const float* __restrict__ bias, const float* __restrict__ wq,
+    const float* __restrict__ wk, float eps, const float* __restrict__ freq, int turned, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ row_seq, T* __restrict__ q_out, T* __restrict__ k_pages, T* __restrict__ v_pages,
+    const int32_t* __restrict__ page_table, int table_stride, int H, int G, int dim, int vdim, int pad, int kv_order, int write,
+    int neighbours, float magnitude, int unit_norm, int values_are_keys, int n_rows) {
+  extern __shared__ float lds[];      // the cosines and sines of the row's turned pairs
+  const int row = bh_row_of_block<true>();      // 16 neighbours to an XCD: rows meet in the cache's lines
+  if (row >= n_rows) return;
+  const int half = turned / 2, lanes = pad / 4, lane = threadIdx.x % BH_WAVE, at_once = HN_WAVES * BH_WAVE / lanes;
+  const int i = threadIdx.x % lanes * 4, place = threadIdx.x / lanes, unit0 = blockIdx.y * HN_HEADS * at_once + place;
+  float* cosines = lds;
+  float* sines = lds + half;
+  const int pos = positions[row], token = pos % BH_PAGE;
+  int page = 0;
+  if (write) page = page_table[(size_t)row_seq[row] * table_stride + pos / BH_PAGE];
+  const T* x = proj + (size_t)row * row_stride + first;
+  const int q_width = H * dim, k_width = G * dim, heads = write ? (values_are_keys ? H + G : H + 2 * G) : H;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 held[HN_HEADS];
+#pragma unroll
+  for (int u = 0; u < HN_HEADS; ++u) {
+    const int unit = unit0 + u * at_once;
+    const bool is_value = unit >= H + G;
+    const int at = is_value ? q_width + k_width + (unit - H - G) * vdim + i : unit * dim + i;      // (the heads of k stand behind those of q)
+    held[u] = zero;
+    if (unit < heads && i < (is_value ? vdim : dim)) {
+      held[u] = load_four(x + at);
+      if (bias) {
+        const float4 b = load_four(bias + at);
+        held[u].x += b.x, held[u].y += b.y, held[u].z += b.z, held[u].w += b.w;
+      }
+    }
+  }
+  for (int j = threadIdx.x; j < half; j += blockDim.x) {
+    const float angle = (float)pos * freq[j];
+    cosines[j] = cosf(angle) * magnitude;
+    sines[j] = sinf(angle) * magnitude;
+  }
+  __syncthreads();
+  const bool turns = i < turned;
+  const int pair = neighbours ? i / 2 : (i < half ? i : i - half);      // the angles: of two pairs of neighbours, or of four halves' pairs
+  float c[4] = {1.f, 1.f, 1.f, 1.f}, s[4] = {0.f, 0.f, 0.f, 0.f};
+  if (turns) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = cosines[neighbours ? pair + j / 2 : pair + j], s[j] = sines[neighbours ? pair + j / 2 : pair + j];
+  }
+  const int mate_lane = neighbours || !turns ? lane : i < half ? lane + half / 4 : lane - half / 4;
+#pragma unroll
+  for (int u = 0; u < HN_HEADS; ++u) {
+    const int unit = unit0 + u * at_once;
+    const bool is_value = unit >= H + G, is_key = unit >= H && !is_value;
+    float ss = held[u].x * held[u].x + held[u].y * held[u].y + held[u].z * held[u].z + held[u].w * held[u].w;
+    for (int off = lanes / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, BH_WAVE);
+    const float* w = is_key ? wk : wq;
+    const float inv = w || unit_norm ? 1.0f / sqrtf(ss / (float)dim + eps) : 1.0f;
+    float y[4] = {0.f, 0.f, 0.f, 0.f};      // beyond dim, whatever the norm's factor is
+    if (i < dim) y[0] = held[u].x * inv, y[1] = held[u].y * inv, y[2] = held[u].z * inv, y[3] = held[u].w * inv;
+    if (w && i < dim) {
+      const float4 scale = load_four(w + i);
+      y[0] *= scale.x, y[1] *= scale.y, y[2] *= scale.z, y[3] *= scale.w;
+    }
+    float mate[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mate[j] = neighbours ? y[j ^ 1] : __shfl(y[j], mate_lane, BH_WAVE);
+    if (unit >= heads) continue;      // (a head's lanes together, behind their exchanges)
+    if (is_value || (is_key && values_are_keys)) {
+      T* values = v_pages + ((size_t)page * G + (is_value ? unit - H - G : unit - H)) * BH_PAGE * pad;
+      const float four[4] = {held[u].x, held[u].y, held[u].z, held[u].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) values[bh_value_index(kv_order, token, i + j, pad)] = from_f32<T>(four[j]);
+      if (is_value) continue;
+    }
+    if (turns) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool is_first = neighbours ? j % 2 == 0 : i < half;
+        y[j] = is_first ? y[j] * c[j] - mate[j] * s[j] : y[j] * c[j] + mate[j] * s[j];
+      }
+    }
+    if (is_key) store_four(k_pages + ((size_t)page * G + unit - H) * BH_PAGE * pad + bh_key_index(kv_order, token, i, pad), y[0], y[1], y[2], y[3]);
+    else store_four(q_out + ((size_t)row * H + unit) * pad + i, y[0], y[1], y[2], y[3]);
+  }
+}
+
 // proj [n_rows][row_stride]: a row holds, from `first`, H heads of q and G heads of k of `dim` and G heads of v of `vdim`;
 // bias f32 over those channels, or null; wq, wk f32 [dim], both or neither.  Pages as the attention kernels take them for G
 // kv heads of size `pad` (written when `write` is set); q_out [n_rows][H * pad].  `neighbours`: a turned pair is
@@ -118,6 +209,23 @@ extern "C" int bh_head_norm_rope_write(const void* proj, int dtype, int row_stri
   const size_t lds = (size_t)(turned + HN_WAVES * dim) * sizeof(float);
   BH_REQUIRE(lds <= 48 * 1024, "head_norm_rope_write: heads of %d dimensions do not fit the local memory", dim);
   const int heads = write ? (values_are_keys ? H + G : H + 2 * G) : H;
+  // Rows for every compute unit, whole pieces of four in both halves of a turn, heads of a power of two up to a wave's lanes.
+  const size_t piece = 4 * (dtype == BH_F32 ? sizeof(float) : 2);
+  if (n_rows >= bh_compute_units() && (pad == 32 || pad == 64 || pad == 128 || pad == 256) && dim % 4 == 0 && vdim % 4 == 0 && turned % (neighbours ? 4 : 8) == 0 &&
+      first % 4 == 0 && row_stride % 4 == 0 && ((uintptr_t)proj | (uintptr_t)q_out | (uintptr_t)k_pages) % piece == 0 &&
+      ((uintptr_t)bias | (uintptr_t)wq | (uintptr_t)wk) % 16 == 0 && (dtype == BH_F32 || dtype == BH_BF16)) {
+    const int at_once = HN_HEADS * HN_WAVES * BH_WAVE / (pad / 4);
+    const dim3 stretches(bh_rows_grid(n_rows, 16), (heads + at_once - 1) / at_once);
+    BH_REQUIRE(stretches.y <= 65535, "head_norm_rope_write: too many heads");
+#define BH_HNP(T)                                                                                                                  \
+  head_norm_rope_write_pieces_kernel<T><<<stretches, HN_WAVES * BH_WAVE, turned * sizeof(float), stream>>>(                        \
+      (const T*)proj, row_stride, first, bias, wq, wk, eps, freq, turned, positions, row_seq, (T*)q_out, (T*)k_pages, (T*)v_pages, page_table, \
+      table_stride, H, G, dim, vdim, pad, kv_order, write, neighbours, magnitude, unit_norm, values_are_keys, n_rows)
+    if (dtype == BH_F32) BH_HNP(float);
+    else BH_HNP(bf16_t);
+#undef BH_HNP
+    return bh_check_launch("head_norm_rope_write");
+  }
   const int per_group = n_rows >= 4 * bh_compute_units() ? 4 * HN_WAVES : HN_WAVES;      // many rows fill the chip by themselves
   const dim3 grid(n_rows, (heads + per_group - 1) / per_group);
   BH_REQUIRE(grid.y <= 65535, "head_norm_rope_write: too many heads");
