@@ -57,6 +57,7 @@ constexpr int STAGE_K = 256;             // K is cut into parts at multiples of 
 // 27.5, 96 rows qkv 21.2 / 20.5, down 33.4 / 32.1, o the same; the SwiGLU that finishes itself 48 rows 39.4 / 41.3, 64 rows
 // 47.3 / 44.5, 96 rows 50.7 / 55.4, so that one takes it at 49 to 64 rows only; a decode step of 64 sequences at context
 // 640 5.50 -> 5.40 ms.
+// KG = 2: two groups of WAVES waves, each with LDS of its own, take half of a part's k each.
 // GATED: SwiGLU with all of K in one workgroup (one part): waves 0 to 3 own four blocks of gate rows, waves 4 to 7 the
 // blocks of up rows of the same outputs (N / 16 blocks further on); at the end the up waves hand their sums over
 // through LDS and the gate waves write bfloat16(act(gate) * up), times the row factors of a norm ahead, into `gated`
@@ -71,22 +72,26 @@ struct GatedOut {
   GateForm form;          // what stands on the gate
 };
 
-template <int MB, int SC, int WAVES, bool GATED, bool DEEP = false>
-__global__ __launch_bounds__(64 * WAVES, GATED ? (WAVES + 3) / 4 : (MB > 4 || WAVES > 4) ? 2 : 4) void gemm_slices_kernel(const uint16_t* __restrict__ a,
+template <int MB, int SC, int WAVES, bool GATED, bool DEEP = false, int KG = 1>
+__global__ __launch_bounds__(64 * WAVES * KG, GATED ? (WAVES + 3) / 4 : (MB > 4 || WAVES > 4) ? 2 : 4) void gemm_slices_kernel(const uint16_t* __restrict__ a,
                                                                     const uint16_t* __restrict__ w,
                                                                     float* __restrict__ sums, int M, int w_rows, int K,
                                                                     int stages_per_part, GatedOut out) {
   constexpr int STEPS = 2 * SC, PIECES = MB * STEPS, MINE = (PIECES + WAVES - 1) / WAVES;   // per stage: steps of 32 k; 1 KB pieces; a wave's
-  __shared__ __attribute__((aligned(16))) u32x4_t xs[2][PIECES * 64];   // [stage in turn][block of 16 rows][step of 32 k][lane]
+  static_assert(KG == 1 || (KG == 2 && !GATED), "a product cut by k within its workgroups leaves bare sums");
+  __shared__ __attribute__((aligned(16))) u32x4_t xs_of[KG][2][PIECES * 64];   // [group][stage in turn][block of 16 rows][step of 32 k][lane]
   const int lane = threadIdx.x % 64;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int wave_of_all = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), group = KG > 1 ? wave_of_all / WAVES : 0, wave = wave_of_all - group * WAVES;
+  auto& xs = xs_of[group];
   const int blocks = w_rows / 16, chunks = K / 64, stages = chunks / SC;
   // GATED: blocks of gate rows 4 x .. 4 x + 3 and, `blocks / 2` further on, their up rows
   const int block_own = GATED ? blockIdx.x * (WAVES / 2) + wave % (WAVES / 2) + (wave / (WAVES / 2)) * (blocks / 2)
                               : blockIdx.x * WAVES + wave;
   const bool owned = GATED ? blockIdx.x * (WAVES / 2) + wave % (WAVES / 2) < blocks / 2 : block_own < blocks;
   const int block = owned ? block_own : blocks - 1;    // a wave beyond the last block repeats it and stores nothing
-  const int first = blockIdx.y * stages_per_part, end = min(stages, first + stages_per_part);
+  // (a part is whole pieces of STAGE_K, an even number of stages here: both groups have as many)
+  const int part_first = blockIdx.y * stages_per_part, part_end = min(stages, part_first + stages_per_part), mine = (part_end - part_first) / KG;
+  const int first = part_first + group * mine, end = first + mine;
   const uint16_t* wp = w + (size_t)block * chunks * 1024 + lane * 8;
   const int q = lane / 16, r = lane % 16;
   // Half u of a chunk holds, for lane group q, k 16 q + 8 u .. + 7 of the chunk's 64: in the activations' blocks
@@ -220,6 +225,19 @@ __global__ __launch_bounds__(64 * WAVES, GATED ? (WAVES + 3) / 4 : (MB > 4 || WA
     }
     return;
   }
+  if constexpr (KG > 1) {
+    static_assert(WAVES * MB <= 2 * PIECES, "the second group's sums fit where its activations stood");
+    f32x4_t* handed = reinterpret_cast<f32x4_t*>(&xs_of[1][0][0]) + wave * MB * 64 + lane;
+    MEET();   // everyone has read the last stage
+    if (group == 1) {
+#pragma unroll
+      for (int b = 0; b < MB; ++b) handed[b * 64] = acc[b];
+    }
+    MEET();
+    if (group == 1) return;
+#pragma unroll
+    for (int b = 0; b < MB; ++b) acc[b] += handed[b * 64];
+  }
   if (!owned) return;
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
@@ -321,13 +339,21 @@ int gemm_slices_launch(const void* a, const void* w, float* sums, int M, int N, 
 #undef BH_SLICES8
     return bh_check_launch("gemm_slices");
   }
-  const dim3 grid((w_rows / 16 + WAVES - 1) / WAVES, parts), block(64 * WAVES);
-#define BH_SLICES(MB) gemm_slices_kernel<MB, SC, WAVES, false, true><<<grid, block, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, sums, M, w_rows, K, each * (STAGE_K / 64 / SC), none)
+  // Parts of 512 k that leave compute units idle: a second group of four waves takes half of a workgroup's k, and hands its sums over through
+  // LDS.  Us with one group / with two, 64 rows: 2,560 x 2,560 (200 workgroups) 9.6 / 9.0, 2,048 x 2,048 (128) 8.9 / 8.3, 1,024 x 3,072 (96)
+  // 8.8 / 8.0; but 2,048 x 6,144 (384) 11.9 / 12.1, and at the chip's full number half as many parts of twice the waves lose, whose
+  // eight waves meet at each stage: 4,096 x 4,096 13.5 / 15.1, 4,096 x 12,288 26.8 / 30.0.
+  const int groups = (w_rows / 16 + WAVES - 1) / WAVES;
+  const bool in_halves = (long)groups * parts <= bh_compute_units();
+  const dim3 grid(groups, parts), block(64 * WAVES * (in_halves ? 2 : 1));
+#define BH_SLICES_OF(MB, KG) gemm_slices_kernel<MB, SC, WAVES, false, true, KG><<<grid, block, 0, stream>>>((const uint16_t*)a, (const uint16_t*)w, sums, M, w_rows, K, each * (STAGE_K / 64 / SC), none)
+#define BH_SLICES(MB) do { if (in_halves) BH_SLICES_OF(MB, 2); else BH_SLICES_OF(MB, 1); } while (0)
   if (M <= 32) BH_SLICES(2);
   else if (M <= 48) BH_SLICES(3);
   else if (M <= 64) BH_SLICES(4);
   else if (M <= 96) BH_SLICES(6);
   else BH_SLICES(8);
+#undef BH_SLICES_OF
 #undef BH_SLICES
   return bh_check_launch("gemm_slices");
 }
