@@ -509,24 +509,27 @@ static DeltaShape delta_shape(int dim) {
 
 // Rows of a chunk for a step whose longest sequence brings max_rows rows (max_rows and more: sequences are walked whole): the number of chunks
 // with the least of an estimate.  A walk is a chain of rows, 0.33 us each until three workgroups share a compute unit, 0.14 us a workgroup
-// then; chunks but the first carry dim more columns, joining the chunks takes 7 us each, and what their rows owe 1 us for 1,600 rows of a head
-// of 128 x 128.  From 16 sizes, 8 to 96 heads of 128 x 128 and 512 to 4,096 rows, each at 7 to 10 numbers of chunks; us, with six workgroups a
-// compute unit wanted whatever a row costs then / by the estimate: 32 heads, 2,048 rows 384 / 349, 512 rows 143 / 117, 16 heads, 2,048
-// rows 252 / 215, 512 rows 108 / 91, 48 heads, 2,048 rows 501 / 455.
+// then (with 8 elements a thread 0.65 of it; heads of more than 128, whose stages fill half of the LDS, run two at a time); chunks but
+// the first carry dim more columns, joining the chunks takes 7 us each at 128 (2.4 at 32), and what their rows owe 1 us for 1,600 rows of a head of
+// 128 x 128.  From 26 sizes, 8 to 96 heads of 32 to 256 and 512 to 4,096 rows, each at 7 to 10 numbers of chunks; us, with six workgroups a
+// compute unit wanted whatever a row costs then / by the estimate: 32 heads of 128, 2,048 rows 384 / 349, 512 rows 143 / 117, 16 heads, 2,048
+// rows 252 / 215, 512 rows 108 / 91, 48 heads, 2,048 rows 501 / 455; 8 heads of 256, 2,048 rows 579 / 492, 16 923 / 810; 16 heads of 64 122 / 97,
+// but 96 heads of 64 296 / 307.
 extern "C" int bh_delta_chunk_rows(int n_seqs, int max_rows, int H, int dim, int vdim) {
   if (max_rows < 192 || n_seqs <= 0 || H <= 0 || dim <= 0 || vdim <= 0 || dim > 256) return max_rows;
   const int columns = delta_shape(dim).columns();
   const long walks = (long)n_seqs * H, tiles = (vdim + columns - 1) / columns, later_tiles = (vdim + dim + columns - 1) / columns;
-  const auto chain = [](long workgroups) {
+  const double of_rows = delta_shape(dim).R < 16 ? 0.65 : 1.0, of_joining = 2.4 + 4.6 * dim * dim / 16384.0;
+  const auto chain = [&](long workgroups) {
     const long share = (workgroups + bh_compute_units() - 1) / bh_compute_units();
-    return share <= 2 ? 0.33 : 0.14 * (double)share;
+    return of_rows * (dim > 128 ? 0.33 * (double)((share + 1) / 2) : share <= 2 ? 0.33 : 0.14 * (double)share);
   };
   const double owed = (double)walks * max_rows * dim * vdim / (16384.0 * 1600.0);
   int best = max_rows;
   double least = max_rows * chain(walks * tiles);
   for (int wanted = 2; wanted <= max_rows / 64 && wanted <= 64; ++wanted) {
     const int rows = ((max_rows + wanted - 1) / wanted + DR_STAGE - 1) / DR_STAGE * DR_STAGE, count = (max_rows + rows - 1) / rows;
-    const double cost = rows * chain(walks * (tiles + (count - 1) * later_tiles)) + owed + 7.0 * count;
+    const double cost = rows * chain(walks * (tiles + (count - 1) * later_tiles)) + owed + of_joining * count;
     if (rows < max_rows && cost < least) best = rows, least = cost;
   }
   return best;
