@@ -148,15 +148,16 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
       }
       q_turn.ask_angles(t.fused, pos[0], dq);
       if (new_key_apart) new_page = table[pos[0] / BH_PAGE];
-    } else {
-#pragma unroll
-      for (int p = 0; p < P; ++p) q[r][p] = load4(t.q + ((size_t)(row0 + r) * t.H + head) * HD + 32 * p + 4 * dq);
     }
     last[r] = new_key_apart ? pos[r] - 1 : pos[r];
     first[r] = bh_first_visible(pos[r], t.window);
     scale[r] = query_scale(t.form, pos[r]);
     from = min(from, first[r]);
     upto = max(upto, last[r]);
+    if constexpr (!FUSED) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) q[r][p] = load4(t.q + ((size_t)(row0 + r) * t.H + head) * HD + 32 * p + 4 * dq);
+    }
   }
   const int last_part = upto >= 0 ? upto / TOKENS : -1;
   bool ready = !FUSED;      // the query is what the scores are made with
@@ -186,6 +187,10 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
       }
     }
   }
+
+  // Heads of 256: with the query's weights and angles carried into the loop there are not the registers to ask for much of a page at a time (8
+  // heads on 2, 4 rows of 300 keys 31.6 us, 13.8 so, 15.6 in two launches).  Heads of 160 to 224 have them, and lose: 4 rows of 100 keys of 160 7.9 / 16.7.
+  if constexpr (FUSED && P >= 8) finish_q();
 
   float most[NR], sum[NR], acc[NR][ND];
 #pragma unroll
@@ -303,7 +308,6 @@ __device__ void attend_rows(const F32Attention& t, Lds<P, NR, WAVES>& lds, int r
     }
     __builtin_amdgcn_wave_barrier();
   }
-  finish_q();      // (a wave without a page)
 
   // over the lanes of a dimension: three halvings (two, of the eight lanes of half a page) leave lane tq with P dimensions' sums over half
   // of the lanes, then its neighbour's
