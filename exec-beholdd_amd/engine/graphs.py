@@ -111,9 +111,9 @@ class DecodeGraph:
     def _capture(self, graph):
         """Capture the step into `graph`.  torch.cuda.graph() gives all cached device memory back beforehand (first decode steps,
         ms with it / without: 16 sequences of Gokazen 13 / 3.1, the float32 generation of four 16 / 9.6 of its whole call); here only
-        where memory runs short: the capture needs no more than what the step that just ran has left in the cache."""
+        where memory runs short (`_short_of_memory`)."""
         device = self.engine.device
-        if torch.cuda.mem_get_info(device)[0] < torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device):
+        if _short_of_memory(device, self.n_seqs * self.rows * self.engine.model.vocab * 4):
             torch.cuda.empty_cache()
         with torch.cuda.stream(self.stream if self.stream is not None else torch.cuda.Stream(device)):
             graph.capture_begin(*(() if self.pool is None else (self.pool,)))
@@ -121,6 +121,16 @@ class DecodeGraph:
                 self.logits = self._forward()
             finally:
                 graph.capture_end()
+
+
+def _short_of_memory(device, logits_bytes: int) -> bool:
+    """Whether the capture of the step that just ran might not get its memory beside what is cached, so that the allocator had to give
+    that back in the middle of it.  It takes what the step took: no more than is cached now, and the logits that are still held.  Its pool
+    may be new and then starts from whole segments (2 and 20 MB, pieces above 10 MB rounded to 2): twice that, and three segments."""
+    reserved = torch.cuda.memory_reserved(device)
+    free, total = torch.cuda.mem_get_info(device)
+    allowed = torch.cuda.get_per_process_memory_fraction(device) * total - reserved
+    return min(free, allowed) < 2 * (reserved - torch.cuda.memory_allocated(device) + logits_bytes) + (64 << 20)
 
 
 class _every_row_wanted:
@@ -142,8 +152,8 @@ class DecodeGraphs:
         self.graphs: dict = {}
         # One pool of device memory for all captures of the engine: only one of them runs at a time, on one
         # stream, so the temporaries of one step may stand where another's stood; what a capture returns (its
-        # logits) stays its own for as long as the capture lives.
-        self.pool = torch.cuda.graph_pool_handle()
+        # logits) stays its own for as long as the capture lives.  It lives with them: see `_live_pool`.
+        self.pool = None
         self.stream = None        # the stream that captures run on: temporaries of one may stand where another's stood on the same stream only
 
     def usable(self, ctx_entries) -> bool:
@@ -153,6 +163,16 @@ class DecodeGraphs:
                 and 1 <= rows <= self.rows_per_sequence and (rows == 1 or rows <= getattr(model, "graph_safe_rows", 1))
                 and all(len(e.tokens) == rows for e in ctx_entries)
                 and (rows == 1 or all(e.fed_row is None for e in ctx_entries)))
+
+    def _live_pool(self):
+        """The pool for the next capture.  A pool that no capture uses any more takes no other: what it held is given back and
+        another one is begun."""
+        if self.pool is not None and not any(graph.graph is not None for graph in self.graphs.values()):
+            torch.cuda.empty_cache()
+            self.pool = None
+        if self.pool is None:
+            self.pool = torch.cuda.graph_pool_handle()
+        return self.pool
 
     def step(self, entries, pasts, extras=None):
         cache = self.engine.cache
@@ -168,7 +188,9 @@ class DecodeGraphs:
                 self.graphs.pop(next(iter(self.graphs)))        # the least recently used
             if self.stream is None:
                 self.stream = torch.cuda.Stream(self.engine.device)
-            graph = DecodeGraph(self.engine, *key, pool=self.pool, stream=self.stream)
+            graph = DecodeGraph(self.engine, *key, stream=self.stream)
+        if graph.graph is None:
+            graph.pool = self._live_pool()
         self.graphs[key] = graph
         graph.fill(entries, pasts)
         logits = graph.run()
