@@ -96,11 +96,10 @@ __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_kerne
 }
 
 // The same for steps of many rows, in pieces of four dimensions: the lanes of a head (pad / 4 of them, neighbours) keep it in registers, add its
-// squares up by exchanges and ask the mate of a half-split turn for its piece; a thread asks for the pieces of HN_HEADS heads at once.  The
+// squares up by exchanges and ask the mate of a half-split turn for its piece; a thread asks for the pieces of HEADS heads at once.  The
 // kernel above goes through one head a wave after the other, an element a lane.  Bound by its bytes and, a third of it, the values,
 // whose tokens lie two bytes apart.  32 heads of 128 on 8, 64 dimensions turned: 2,048 rows 42.3 -> 29.6 us, 8,192 rows 144 -> 98.
-#define HN_HEADS 4
-template <typename T>
+template <typename T, int HEADS>
 __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_pieces_kernel(
     const T* __restrict__ proj, int row_stride, int first, const float* __restrict__ bias, const float* __restrict__ wq,
     const float* __restrict__ wk, float eps, const float* __restrict__ freq, int turned, const int32_t* __restrict__ positions,
@@ -110,8 +109,8 @@ __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_piece
   extern __shared__ float lds[];      // the cosines and sines of the row's turned pairs
   const int row = bh_row_of_block<true>();      // 16 neighbours to an XCD: rows meet in the cache's lines
   if (row >= n_rows) return;
-  const int half = turned / 2, lanes = pad / 4, lane = threadIdx.x % BH_WAVE, at_once = HN_WAVES * BH_WAVE / lanes;
-  const int i = threadIdx.x % lanes * 4, place = threadIdx.x / lanes, unit0 = blockIdx.y * HN_HEADS * at_once + place;
+  const int half = turned / 2, lanes = pad / 4, lane = threadIdx.x % BH_WAVE, at_once = blockDim.x / lanes;
+  const int i = threadIdx.x % lanes * 4, place = threadIdx.x / lanes, unit0 = blockIdx.y * HEADS * at_once + place;
   float* cosines = lds;
   float* sines = lds + half;
   const int pos = positions[row], token = pos % BH_PAGE;
@@ -120,9 +119,9 @@ __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_piece
   const T* x = proj + (size_t)row * row_stride + first;
   const int q_width = H * dim, k_width = G * dim, heads = write ? (values_are_keys ? H + G : H + 2 * G) : H;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 held[HN_HEADS];
+  float4 held[HEADS];
 #pragma unroll
-  for (int u = 0; u < HN_HEADS; ++u) {
+  for (int u = 0; u < HEADS; ++u) {
     const int unit = unit0 + u * at_once;
     const bool is_value = unit >= H + G;
     const int at = is_value ? q_width + k_width + (unit - H - G) * vdim + i : unit * dim + i;      // (the heads of k stand behind those of q)
@@ -150,7 +149,7 @@ __global__ __launch_bounds__(HN_WAVES * BH_WAVE) void head_norm_rope_write_piece
   }
   const int mate_lane = neighbours || !turns ? lane : i < half ? lane + half / 4 : lane - half / 4;
 #pragma unroll
-  for (int u = 0; u < HN_HEADS; ++u) {
+  for (int u = 0; u < HEADS; ++u) {
     const int unit = unit0 + u * at_once;
     const bool is_value = unit >= H + G, is_key = unit >= H && !is_value;
     float ss = held[u].x * held[u].x + held[u].y * held[u].y + held[u].z * held[u].z + held[u].w * held[u].w;
@@ -209,20 +208,32 @@ extern "C" int bh_head_norm_rope_write(const void* proj, int dtype, int row_stri
   const size_t lds = (size_t)(turned + HN_WAVES * dim) * sizeof(float);
   BH_REQUIRE(lds <= 48 * 1024, "head_norm_rope_write: heads of %d dimensions do not fit the local memory", dim);
   const int heads = write ? (values_are_keys ? H + G : H + 2 * G) : H;
-  // Rows for every compute unit, whole pieces of four in both halves of a turn, heads of a power of two up to a wave's lanes.
+  // Rows for every compute unit, heads that fill a wave or many rows, whole pieces of four in both halves of a turn, heads of a power of two up to a wave's
+  // lanes.  An element / four a thread, us, all dimensions turned, bfloat16: 16 heads of 128 on 4 256 rows 6.8 / 5.5, 4,096 rows 46 / 27; 4 of 64 on
+  // 2 256 rows 4.6 / 4.8, 4,096 rows 15.2 / 8.5; 2 of 32 on 1, half a wave, 4,096 rows 10.4 / 6.6, but 256 rows 4.3 / 4.8, 1,024 rows 5.1 / 5.2.
   const size_t piece = 4 * (dtype == BH_F32 ? sizeof(float) : 2);
-  if (n_rows >= bh_compute_units() && (pad == 32 || pad == 64 || pad == 128 || pad == 256) && dim % 4 == 0 && vdim % 4 == 0 && turned % (neighbours ? 4 : 8) == 0 &&
+  if (n_rows >= bh_compute_units() && bh_rows_spread(n_rows, 16) && (heads * (pad / 4) >= BH_WAVE || n_rows > 4 * bh_compute_units()) && (pad == 32 || pad == 64 || pad == 128 || pad == 256) && dim % 4 == 0 && vdim % 4 == 0 && turned % (neighbours ? 4 : 8) == 0 &&
       first % 4 == 0 && row_stride % 4 == 0 && ((uintptr_t)proj | (uintptr_t)q_out | (uintptr_t)k_pages) % piece == 0 &&
       ((uintptr_t)bias | (uintptr_t)wq | (uintptr_t)wk) % 16 == 0 && (dtype == BH_F32 || dtype == BH_BF16)) {
-    const int at_once = HN_HEADS * HN_WAVES * BH_WAVE / (pad / 4);
+    // As many heads a thread as leave no more than eight waves a row, and no waves without a head; rows that do not fill the chip: one.
+    const int lanes = heads * (pad / 4), most = HN_WAVES * BH_WAVE;
+    const int each = lanes <= most || n_rows < 4 * bh_compute_units() ? 1 : lanes <= 2 * most ? 2 : 4;
+    const int threads = std::min(most, ((lanes + each - 1) / each + BH_WAVE - 1) / BH_WAVE * BH_WAVE), at_once = each * (threads / (pad / 4));
     const dim3 stretches(bh_rows_grid(n_rows, 16), (heads + at_once - 1) / at_once);
     BH_REQUIRE(stretches.y <= 65535, "head_norm_rope_write: too many heads");
-#define BH_HNP(T)                                                                                                                  \
-  head_norm_rope_write_pieces_kernel<T><<<stretches, HN_WAVES * BH_WAVE, turned * sizeof(float), stream>>>(                        \
+#define BH_HNP(T, HEADS)                                                                                                           \
+  head_norm_rope_write_pieces_kernel<T, HEADS><<<stretches, threads, turned * sizeof(float), stream>>>(                            \
       (const T*)proj, row_stride, first, bias, wq, wk, eps, freq, turned, positions, row_seq, (T*)q_out, (T*)k_pages, (T*)v_pages, page_table, \
       table_stride, H, G, dim, vdim, pad, kv_order, write, neighbours, magnitude, unit_norm, values_are_keys, n_rows)
-    if (dtype == BH_F32) BH_HNP(float);
-    else BH_HNP(bf16_t);
+    if (dtype == BH_F32) {
+      if (each == 1) BH_HNP(float, 1);
+      else if (each == 2) BH_HNP(float, 2);
+      else BH_HNP(float, 4);
+    } else {
+      if (each == 1) BH_HNP(bf16_t, 1);
+      else if (each == 2) BH_HNP(bf16_t, 2);
+      else BH_HNP(bf16_t, 4);
+    }
 #undef BH_HNP
     return bh_check_launch("head_norm_rope_write");
   }

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void whole_norm_rope_write_pieces_kernel(
   float ss_q = 0.f, ss_k = 0.f;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int e = threadIdx.x + 256 * u, head = e / pieces, i = e % pieces * 4;
+    const int e = threadIdx.x + blockDim.x * u, head = e / pieces, i = e % pieces * 4;
     held[u] = e < units && i < dim ? load_four(x + head * dim + i) : zero;      // (the heads of k stand behind those of q)
   }
   for (int i = threadIdx.x; i < turned / 2; i += blockDim.x) {
@@ -122,14 +122,14 @@ __global__ __launch_bounds__(256) void whole_norm_rope_write_pieces_kernel(
   for (int u = 0; u < PER; ++u) {
     const float4 y = held[u];
     const float squares = y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w;
-    if (threadIdx.x + 256 * u < H * pieces) ss_q += squares;
+    if (threadIdx.x + blockDim.x * u < H * pieces) ss_q += squares;
     else ss_k += squares;
   }
   const float inv_q = 1.0f / sqrtf(block_sum(ss_q, scratch) / (float)q_width + eps);
   const float inv_k = 1.0f / sqrtf(block_sum(ss_k, scratch) / (float)k_width + eps);
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int e = threadIdx.x + 256 * u, head = e / pieces, i = e % pieces * 4;
+    const int e = threadIdx.x + blockDim.x * u, head = e / pieces, i = e % pieces * 4;
     if (e >= units) break;
     const bool is_key = head >= H;
     float4 y = zero;
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void whole_norm_rope_write_pieces_kernel(
     else if (write) store_four(k_pages + ((size_t)page * G + head - H) * BH_PAGE * pad + bh_key_index(kv_order, pos % BH_PAGE, i, pad), y.x, y.y, y.z, y.w);
   }
   if (!write) return;
-  for (int e = threadIdx.x; e < G * pieces; e += 256) {
+  for (int e = threadIdx.x; e < G * pieces; e += blockDim.x) {
     const int head = e / pieces, i = e % pieces * 4;
     const float4 y = i < vdim ? load_four(x + q_width + k_width + head * vdim + i) : zero;
     T* values = v_pages + ((size_t)page * G + head) * BH_PAGE * pad;
@@ -177,16 +177,23 @@ extern "C" int bh_whole_norm_rope_write(const float* qkv, const float* wq, const
   const size_t lds = (size_t)(turned > 0 ? turned : 1) * sizeof(float);
   // Rows for every compute unit, whole pieces of four, and no more of them than the threads hold.
   const int pieces = (H + G) * (pad / 4);
-  if (n_rows >= bh_compute_units() && dim % 4 == 0 && vdim % 4 == 0 && pad % 4 == 0 && pieces <= 8 * 256 && (dtype == BH_F32 || dtype == BH_BF16) &&
+  if (n_rows >= bh_compute_units() && bh_rows_spread(n_rows, 16) && dim % 4 == 0 && vdim % 4 == 0 && pad % 4 == 0 && pieces <= 8 * 256 && (dtype == BH_F32 || dtype == BH_BF16) &&
       ((uintptr_t)qkv | (uintptr_t)wq | (uintptr_t)wk | (uintptr_t)q_out | (uintptr_t)k_pages) % 16 == 0) {
+    const int threads = (int)bh_piece_threads(pieces), each = (pieces + threads - 1) / threads;
 #define BH_WNP(T, PER)                                                                                                          \
-  whole_norm_rope_write_pieces_kernel<T, PER><<<bh_rows_grid(n_rows, 16), 256, lds, stream>>>(qkv, wq, wk, eps, freq, turned, positions, row_seq, (T*)q_out, (T*)k_pages, \
+  whole_norm_rope_write_pieces_kernel<T, PER><<<bh_rows_grid(n_rows, 16), threads, lds, stream>>>(qkv, wq, wk, eps, freq, turned, positions, row_seq, (T*)q_out, (T*)k_pages, \
                                                                            (T*)v_pages, page_table, table_stride, H, G, dim, vdim, pad, kv_order, write, n_rows)
-    if (pieces <= 4 * 256) {
-      if (dtype == BH_F32) BH_WNP(float, 4);
-      else BH_WNP(bf16_t, 4);
-    } else if (dtype == BH_F32) BH_WNP(float, 8);
-    else BH_WNP(bf16_t, 8);
+#define BH_WNP_OF(T)               \
+  if (each <= 1) BH_WNP(T, 1);     \
+  else if (each <= 2) BH_WNP(T, 2); \
+  else if (each <= 4) BH_WNP(T, 4); \
+  else BH_WNP(T, 8)
+    if (dtype == BH_F32) {
+      BH_WNP_OF(float);
+    } else {
+      BH_WNP_OF(bf16_t);
+    }
+#undef BH_WNP_OF
 #undef BH_WNP
     return bh_check_launch("whole_norm_rope_write");
   }
