@@ -285,31 +285,33 @@ extern "C" int bh_clamped_glu(const void* gu, int dtype, void* out, int n_rows, 
 //   experts_gather    the pairs' input rows side by side, expert after expert, for products of many rows
 //   experts_combine   h_res[row] += sum_j weight_j * y[place of pair (row, j)], j in order
 
-// One workgroup an expert.  Every wave takes a run of the pairs and goes over it twice, counting those that chose the expert and then
-// writing them behind those of the waves before it: two trips to memory and one barrier, whatever the number of pairs, since the
-// loads of a run do not wait for each other.  Bound by those trips.  8,400 pairs of 32 experts 6.0 us, 21.0 with a barrier every
-// 256 pairs.
-#define EG_AHEAD 4      // pieces of 64 pairs asked for together
+// One workgroup an expert.  Every wave takes a run of the pairs and counts those that chose the expert, then writes them behind those of
+// the waves before it: one barrier, and a round of loads for every AHEAD x 64 pairs of a wave, twice where it has more than one round
+// (above 4,096 pairs).  Bound by those rounds.  8,400 pairs of 32 experts 6.0 us, 21.0 with a barrier every 256 pairs.
+template <int AHEAD>      // pieces of 64 pairs asked for together
 __global__ __launch_bounds__(1024) void experts_group_kernel(const int32_t* __restrict__ chosen, int n_pairs, int32_t* __restrict__ list,
                                                              int capacity, int32_t* __restrict__ counts) {
   __shared__ int wave_count[16];
   const int e = blockIdx.x, lane = threadIdx.x & (BH_WAVE - 1), wave = threadIdx.x / BH_WAVE, waves = blockDim.x / BH_WAVE;
-  const int run = (n_pairs + EG_AHEAD * blockDim.x - 1) / (EG_AHEAD * blockDim.x) * (EG_AHEAD * BH_WAVE);      // pairs of a wave
+  const int run = (n_pairs + AHEAD * blockDim.x - 1) / (AHEAD * blockDim.x) * (AHEAD * BH_WAVE);      // pairs of a wave
   const int first = wave * run, stop = first + run < n_pairs ? first + run : n_pairs;
-  auto each = [&](auto take) {      // take(pair, which lanes' pairs chose the expert)
-    for (int p0 = first; p0 < stop; p0 += EG_AHEAD * BH_WAVE) {
-      bool mine[EG_AHEAD];
+  unsigned long long masks[AHEAD] = {};      // of a round: which lanes' pairs chose the expert
+  auto ask = [&](int p0) {
+    int32_t found[AHEAD];
 #pragma unroll
-      for (int i = 0; i < EG_AHEAD; ++i) {
-        const int p = p0 + i * BH_WAVE + lane;
-        mine[i] = chosen[p < stop ? p : stop - 1] == e && p < stop;
-      }
-#pragma unroll
-      for (int i = 0; i < EG_AHEAD; ++i) take(p0 + i * BH_WAVE + lane, __ballot(mine[i]));
+    for (int i = 0; i < AHEAD; ++i) {
+      const int p = p0 + i * BH_WAVE + lane;
+      found[i] = chosen[p < stop ? p : stop - 1];
     }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) masks[i] = __ballot(found[i] == e && p0 + i * BH_WAVE + lane < stop);
   };
   int count = 0;
-  each([&](int, unsigned long long mask) { count += __popcll(mask); });
+  for (int p0 = first; p0 < stop; p0 += AHEAD * BH_WAVE) {
+    ask(p0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) count += __popcll(masks[i]);
+  }
   if (lane == 0) wave_count[wave] = count;
   __syncthreads();
   int at = 0, total = 0;
@@ -318,18 +320,24 @@ __global__ __launch_bounds__(1024) void experts_group_kernel(const int32_t* __re
     total += wave_count[w];
   }
   int32_t* to = list + (size_t)e * capacity;
-  each([&](int p, unsigned long long mask) {
-    if (mask >> lane & 1ull) to[at + __popcll(mask & ((1ull << lane) - 1ull))] = p;
-    at += __popcll(mask);
-  });
+  for (int p0 = first; p0 < stop; p0 += AHEAD * BH_WAVE) {
+    if (run > AHEAD * BH_WAVE) ask(p0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      if (masks[i] >> lane & 1ull) to[at + __popcll(masks[i] & ((1ull << lane) - 1ull))] = p0 + i * BH_WAVE + lane;
+      at += __popcll(masks[i]);
+    }
+  }
   if (threadIdx.x == 0) counts[e] = total;
 }
 
 extern "C" int bh_experts_group(const int32_t* chosen, int n_pairs, int32_t* list, int capacity, int32_t* counts, int E, hipStream_t stream) {
   BH_REQUIRE(n_pairs > 0 && E > 0 && capacity > 0, "experts_group: sizes must be positive");
-  // (a wave takes as many pairs as it asks for together, until there are sixteen)
-  const int waves = (n_pairs + EG_AHEAD * BH_WAVE - 1) / (EG_AHEAD * BH_WAVE);
-  experts_group_kernel<<<E, BH_WAVE * (waves < 16 ? waves : 16), 0, stream>>>(chosen, n_pairs, list, capacity, counts);
+  // Waves of 64 pairs until there are sixteen, then of 256.
+  const bool few = n_pairs <= 16 * BH_WAVE;
+  const int each = few ? BH_WAVE : 4 * BH_WAVE, waves = (n_pairs + each - 1) / each;
+  if (few) experts_group_kernel<1><<<E, BH_WAVE * waves, 0, stream>>>(chosen, n_pairs, list, capacity, counts);
+  else experts_group_kernel<4><<<E, BH_WAVE * (waves < 16 ? waves : 16), 0, stream>>>(chosen, n_pairs, list, capacity, counts);
   return bh_check_launch("experts_group");
 }
 
