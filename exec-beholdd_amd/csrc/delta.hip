@@ -11,6 +11,7 @@
 // projected rows, which come in the activation type.
 #include "chunks.h"
 #include "common.h"
+#include <cmath>
 
 #define DR_UNIT_EPS 1e-6f
 #define DR_MAX_TAPS 16
@@ -507,30 +508,58 @@ static DeltaShape delta_shape(int dim) {
   return {32, 16, 1};
 }
 
-// Rows of a chunk for a step whose longest sequence brings max_rows rows (max_rows and more: sequences are walked whole): the number of chunks
-// with the least of an estimate.  A walk is a chain of rows, 0.33 us each until three workgroups share a compute unit, 0.14 us a workgroup
-// then (with 8 elements a thread 0.65 of it; heads of more than 128, whose stages fill half of the LDS, run two at a time); chunks but
-// the first carry dim more columns, joining the chunks takes 7 us each at 128 (2.4 at 32), and what their rows owe 1 us for 1,600 rows of a head of
-// 128 x 128.  From 26 sizes, 8 to 96 heads of 32 to 256 and 512 to 4,096 rows, each at 7 to 10 numbers of chunks; us, with six workgroups a
-// compute unit wanted whatever a row costs then / by the estimate: 32 heads of 128, 2,048 rows 384 / 349, 512 rows 143 / 117, 16 heads, 2,048
-// rows 252 / 215, 512 rows 108 / 91, 48 heads, 2,048 rows 501 / 455; 8 heads of 256, 2,048 rows 579 / 492, 16 923 / 810; 16 heads of 64 122 / 97,
-// but 96 heads of 64 296 / 307.
-extern "C" int bh_delta_chunk_rows(int n_seqs, int max_rows, int H, int dim, int vdim) {
-  if (max_rows < 192 || n_seqs <= 0 || H <= 0 || dim <= 0 || vdim <= 0 || dim > 256) return max_rows;
-  const int columns = delta_shape(dim).columns();
-  const long walks = (long)n_seqs * H, tiles = (vdim + columns - 1) / columns, later_tiles = (vdim + dim + columns - 1) / columns;
-  const double of_rows = delta_shape(dim).R < 16 ? 0.65 : 1.0, of_joining = 2.4 + 4.6 * dim * dim / 16384.0;
-  const auto chain = [&](long workgroups) {
+// What a walk is estimated to take, for the number of chunks with the least of it.  A row of a workgroup's chain takes hypot(row, shared *
+// workgroups) us where so many of them stand on a compute unit, of which `resident` fit it (their stages in LDS, their registers); more come in
+// rounds.  A chunk but the first carries dim more columns.  The first's missing ones are felt where the number of chunks is odd: where
+// it is even, workgroups dealt to the eight XCDs in turn leave it all to some of them.  Joining takes 2 us a chunk and 4 more at heads of
+// 128 x 128, the launches behind the walk 16.
+// Fitted to 223 steps of 1 to 128 heads of 16 to 256, 256 to 8,192 rows in 1 to 16 sequences, each at up to 17 numbers of chunks: what it
+// chooses takes 1.004 times the best of these on average, 1.06 at most.  Six workgroups a compute unit wanted, whatever a row costs then, took 1.09;
+// us, so / by the estimate: 32 heads of 128, 2,048 rows 383 / 343, 512 rows 148 / 126, 16 heads, 2,048 rows 250 / 219, 48 heads 502 / 446; 8 heads of
+// 256 576 / 489; 16 heads of 64 125 / 102; 128 heads of 64 344 / 344; but 96 of 64, 8,192 rows 1,143 / 1,193, 8 of 256 1,983 / 2,106.
+struct DeltaCost {
+  double row, shared;
+  int resident;
+  long walks, tiles, later_tiles;
+  double joining;
+
+  DeltaCost(int n_seqs, int H, int dim, int vdim) {
+    const int columns = delta_shape(dim).columns();
+    if (dim <= 16) row = 0.2, shared = 0.054, resident = 8;
+    else if (dim <= 32) row = 0.223, shared = 0.075, resident = 6;
+    else if (dim <= 64) row = 0.2, shared = 0.083, resident = 6;
+    else if (dim <= 128) row = 0.306, shared = 0.121, resident = 4;
+    else row = 0.36, shared = 0.146, resident = 2;
+    walks = (long)n_seqs * H, tiles = (vdim + columns - 1) / columns, later_tiles = (vdim + dim + columns - 1) / columns;
+    joining = 2.0 + 3.9 * dim * dim / 16384.0;
+  }
+  double beside(long workgroups) const { return workgroups > 0 ? std::hypot(row, shared * (double)workgroups) : 0.0; }
+  double a_row(int chunks) const {
+    const long workgroups = walks * (chunks == 1 ? tiles : chunks % 2 == 0 ? chunks * later_tiles : tiles + (chunks - 1) * later_tiles);
     const long share = (workgroups + bh_compute_units() - 1) / bh_compute_units();
-    return of_rows * (dim > 128 ? 0.33 * (double)((share + 1) / 2) : share <= 2 ? 0.33 : 0.14 * (double)share);
-  };
-  const double owed = (double)walks * max_rows * dim * vdim / (16384.0 * 1600.0);
+    return (double)(share / resident) * beside(resident) + beside(share % resident);
+  }
+  // (of odd numbers above three the workgroups are left on some compute units one more than the average says)
+  static bool tried(int chunks) { return chunks <= 3 || chunks % 2 == 0; }
+  double behind(int chunks) const { return 16.0 + joining * chunks; }
+  // (the chunks' states of as many sequences are much memory for a last round's gain)
+  bool fills() const { return walks * tiles >= 4L * bh_compute_units(); }
+};
+#define DELTA_MOST_CHUNKS 64
+#define DELTA_CHUNK 64       // rows, at least
+
+// Rows of a chunk for a step whose longest sequence brings max_rows rows (max_rows and more: sequences are walked whole).
+extern "C" int bh_delta_chunk_rows(int n_seqs, int max_rows, int H, int dim, int vdim) {
+  if (max_rows < 3 * DELTA_CHUNK || n_seqs <= 0 || H <= 0 || dim <= 0 || vdim <= 0 || dim > 256) return max_rows;
+  const DeltaCost cost(n_seqs, H, dim, vdim);
+  if (cost.fills()) return max_rows;
   int best = max_rows;
-  double least = max_rows * chain(walks * tiles);
-  for (int wanted = 2; wanted <= max_rows / 64 && wanted <= 64; ++wanted) {
+  double least = max_rows * cost.a_row(1);
+  for (int wanted = 2; wanted <= max_rows / DELTA_CHUNK && wanted <= DELTA_MOST_CHUNKS; ++wanted) {
+    if (!DeltaCost::tried(wanted)) continue;
     const int rows = ((max_rows + wanted - 1) / wanted + DR_STAGE - 1) / DR_STAGE * DR_STAGE, count = (max_rows + rows - 1) / rows;
-    const double cost = rows * chain(walks * (tiles + (count - 1) * later_tiles)) + owed + of_joining * count;
-    if (rows < max_rows && cost < least) best = rows, least = cost;
+    const double takes = rows * cost.a_row(count) + cost.behind(count);
+    if (rows < max_rows && takes < least) best = rows, least = takes;
   }
   return best;
 }
