@@ -11,6 +11,7 @@
 // projected rows, which come in the activation type.
 #include "chunks.h"
 #include "common.h"
+#include <algorithm>
 #include <cmath>
 
 #define DR_UNIT_EPS 1e-6f
@@ -562,6 +563,39 @@ extern "C" int bh_delta_chunk_rows(int n_seqs, int max_rows, int H, int dim, int
     if (rows < max_rows && takes < least) best = rows, least = takes;
   }
   return best;
+}
+
+// Chunks of all sequences together, at most, over the steps of up to n_seqs sequences, n_rows rows and max_rows rows a sequence (0: no such
+// step is cut).  Fewer sequences are cut into more chunks each, and a number of chunks may be the best one at any number of rows: it is
+// left out where for the fewest and the most rows, and so, both costs being linear in them, for all between, fewer chunks cost less though their
+// rows are rounded up to a stage.
+extern "C" long bh_delta_most_chunks(int n_seqs, int n_rows, int max_rows, int H, int dim, int vdim) {
+  if (H <= 0 || dim <= 0 || vdim <= 0 || dim > 256) return 0;
+  long most = 0;
+  for (int n = 1; n <= n_seqs; ++n) {
+    const DeltaCost cost(n, H, dim, vdim);
+    const int longest = n_rows - n + 1 < max_rows ? n_rows - n + 1 : max_rows;      // the other sequences bring a row each
+    if (longest < 3 * DELTA_CHUNK || cost.fills()) break;
+    double a_row[DELTA_MOST_CHUNKS + 1];
+    const int pieces = longest / DELTA_CHUNK < DELTA_MOST_CHUNKS ? longest / DELTA_CHUNK : DELTA_MOST_CHUNKS;
+    for (int chunks = 1; chunks <= pieces; ++chunks) a_row[chunks] = cost.a_row(chunks);
+    const auto never = [&](int chunks) {
+      const int ends[2] = {std::max(chunks, 3) * DELTA_CHUNK, longest};
+      for (int fewer = 1; fewer < chunks; ++fewer) {
+        bool less = DeltaCost::tried(fewer);
+        for (int rows : ends) {
+          const double takes = (double)rows / chunks * a_row[chunks] + cost.behind(chunks);
+          less = less && (fewer == 1 ? rows * a_row[1] : ((double)rows / fewer + DR_STAGE) * a_row[fewer] + cost.behind(fewer)) < takes;
+        }
+        if (less) return true;
+      }
+      return false;
+    };
+    int chunks = pieces;
+    while (chunks > 1 && never(chunks)) --chunks;
+    if (chunks > 1) most = std::max(most, (long)n * chunks);
+  }
+  return most;
 }
 
 extern "C" int bh_delta_takes(int dim, int vdim) { return dim > 0 && dim <= 512 && vdim > 0; }

@@ -531,6 +531,21 @@ extern "C" int bh_gla_chunk_rows(int n_seqs, int max_rows, int H, int dim, int v
   return rows >= max_rows ? max_rows : rows;
 }
 
+// Chunks of all sequences together, at most, over the steps of up to n_seqs sequences, n_rows rows and max_rows rows a sequence (0: no such
+// step is cut): fewer sequences are cut into more chunks each.
+extern "C" long bh_gla_most_chunks(int n_seqs, int n_rows, int max_rows, int H, int dim, int vdim) {
+  if (dim > 256 * GLA_KEPT) return 0;
+  const long enough = 4L * bh_compute_units(), tiles = (vdim + 63) / 64;
+  long most = 0;
+  for (long n = 1; n <= n_seqs && n * H * tiles < enough; ++n) {
+    const long longest = n_rows - n + 1 < max_rows ? n_rows - n + 1 : max_rows;      // the other sequences bring a row each
+    if (longest < 128) break;
+    const long wanted = (enough + n * H * tiles - 1) / (n * H * tiles), pieces = longest / 64;
+    most = n * (wanted < pieces ? wanted : pieces) > most ? n * (wanted < pieces ? wanted : pieces) : most;
+  }
+  return most;
+}
+
 // The chunks' states joined, and what the later chunks' rows owe them.
 static int gla_join(const GlaChunks& chunks, float* state, long slot_stride, const int32_t* seq_start, const int32_t* seq_slot, const int32_t* seq_to,
                     float* out, int n_seqs, int H, int dim, int vdim, hipStream_t stream) {

@@ -262,7 +262,8 @@ class KernelSizes:
         lib.bh_gemm_bf16_scratch.argtypes = [i, i, i, i, i]
         lib.bh_gemm_bf16_scratch.restype = ctypes.c_long
         for query, count in ((lib.bh_lightning_products_scratch, 10), (lib.bh_ssm_products_scratch, 8), (lib.bh_lightning_products_most, 6),
-                             (lib.bh_ssm_products_most, 6), (lib.bh_lightning_most_chunks, 5), (lib.bh_ssm_most_chunks, 4)):
+                             (lib.bh_ssm_products_most, 6), (lib.bh_lightning_most_chunks, 5), (lib.bh_ssm_most_chunks, 4),
+                             (lib.bh_gla_most_chunks, 6), (lib.bh_delta_most_chunks, 6)):
             query.argtypes, query.restype = [i] * count, ctypes.c_long
         for query in (lib.bh_gemm_bf16_norm_blocks, lib.bh_gemm_bf16_takes_norm, lib.bh_gemm_bf16_turns_blocks,
                       lib.bh_gemm_bf16_reads_blocked, lib.bh_gemm_bf16_writes_blocked):
@@ -346,20 +347,16 @@ class KernelSizes:
         return _rounded(max(products, chunks * n_heads * dim * vdim) * 4)
 
     def gla_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, dim, vdim) -> int:
-        """Bytes of scratch memory that `gla_scan` allocates for a step of these sizes (long sequences cut into chunks)."""
-        chunk_rows = int(self.lib.bh_gla_chunk_rows(int(n_seqs), int(max_rows), int(n_heads), int(dim), int(vdim)))
-        if chunk_rows >= max_rows:
-            return 0
-        chunks = -(-int(max_rows) // chunk_rows)
-        return _rounded((n_seqs * chunks * n_heads * dim * (vdim + 1) + n_rows * n_heads * dim) * 4)
+        """Bytes of scratch memory that `gla_scan` and `wkv_scan` allocate at most in a step of up to so many sequences, rows and rows a
+        sequence (long sequences cut into chunks; fewer sequences may take more than many)."""
+        chunks = int(self.lib.bh_gla_most_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(dim), int(vdim)))
+        return _rounded((chunks * n_heads * dim * (vdim + 1) + n_rows * n_heads * dim) * 4) if chunks else 0
 
     def delta_chunk_bytes(self, n_seqs, n_rows, max_rows, n_heads, dim, vdim) -> int:
-        """Bytes of scratch memory that `delta_scan` allocates for a step of these sizes (long sequences cut into chunks)."""
-        chunk_rows = int(self.lib.bh_delta_chunk_rows(int(n_seqs), int(max_rows), int(n_heads), int(dim), int(vdim)))
-        if chunk_rows >= max_rows:
-            return 0
-        chunks = -(-int(max_rows) // chunk_rows)
-        return _rounded((n_seqs * chunks * n_heads * dim * (vdim + dim) + n_rows * n_heads * dim) * 4)
+        """Bytes of scratch memory that `delta_scan` allocates at most in a step of up to so many sequences, rows and rows a sequence
+        (long sequences cut into chunks; fewer sequences may take more than many)."""
+        chunks = int(self.lib.bh_delta_most_chunks(int(n_seqs), int(n_rows), int(max_rows), int(n_heads), int(dim), int(vdim)))
+        return _rounded((chunks * n_heads * dim * (vdim + dim) + n_rows * n_heads * dim) * 4) if chunks else 0
 
     def packs(self, rows, cols, act_size) -> bool:
         """Whether `pack_weight` regroups a matrix of this shape and element size."""

@@ -1,4 +1,4 @@
-"""The scratch memory that the byte plan counts for the recurrences with a scalar decay covers every smaller step, not only the largest
+"""The scratch memory that the byte plan counts for the recurrences covers every smaller step, not only the largest
 one: a step of one long sequence may take more than one of as many sequences as the engine holds."""
 
 import ctypes
@@ -49,3 +49,32 @@ def test_a_plan_covers_every_step_of_its_sizes(sizes, seqs, rows, longest, heads
                 assert ssm_takes(sizes.lib, n, r, most, heads, vdim, dim, stride) <= planned[1], (n, r, most, stride)
     if longest == 1:
         assert planned == (0, 0)      # captured decode steps take none
+
+
+def delta_takes(lib, seqs, rows, longest, heads, dim, vdim):
+    chunk = lib.bh_delta_chunk_rows(seqs, longest, heads, dim, vdim)
+    return (seqs * -(-longest // chunk) * heads * dim * (vdim + dim) + rows * heads * dim) * 4 if chunk < longest else 0
+
+
+def gla_takes(lib, seqs, rows, longest, heads, dim, vdim):
+    chunk = lib.bh_gla_chunk_rows(seqs, longest, heads, dim, vdim)
+    return (seqs * -(-longest // chunk) * heads * dim * (vdim + 1) + rows * heads * dim) * 4 if chunk < longest else 0
+
+
+# one sequence of many heads, many of few; heads of every kind of walk; sequences shorter than the step; steps that are never cut
+@pytest.mark.parametrize("seqs,rows,longest,heads,dim,vdim", [
+    (4, 8192, 8192, 8, 128, 128), (8, 8192, 8192, 32, 128, 128), (64, 2048, 2048, 32, 128, 128), (16, 8192, 4096, 16, 128, 128), (1, 300, 300, 8, 256, 256),
+    (8, 4096, 4096, 96, 64, 64), (64, 4096, 512, 16, 96, 64), (2, 8192, 8192, 4, 256, 250), (32, 16384, 8192, 4, 64, 64), (8, 1000, 1000, 32, 32, 32), (300, 700, 700, 2, 20, 48),
+    (4, 6000, 6000, 3, 300, 64), (64, 64, 1, 32, 128, 128)])
+def test_a_plan_covers_every_step_of_the_recurrences_that_are_joined(sizes, seqs, rows, longest, heads, dim, vdim):
+    rng = random.Random(rows + heads)
+    plans = sizes.delta_chunk_bytes(seqs, rows, longest, heads, dim, vdim), sizes.gla_chunk_bytes(seqs, rows, longest, heads, dim, vdim)
+    largest = [0, 0]
+    for n in range(1, seqs + 1):
+        most = min(longest, rows - n + 1)
+        for m in {most, max(most // 2, 1), *(rng.randint(1, most) for _ in range(3000 // seqs + 20)), *range(128, most + 1, 64)}:
+            for at, takes in enumerate((delta_takes, gla_takes)):
+                taken = takes(sizes.lib, n, min(rows, n * m), m, heads, dim, vdim)
+                assert taken <= plans[at], (n, m, at)
+                largest[at] = max(largest[at], taken)
+    assert all(plan <= 1.65 * most for plan, most in zip(plans, largest))      # and not much more: a limit on memory refuses by it
