@@ -21,7 +21,7 @@ from ..weights.binder import bind
 from ..weights.random_init import random_tensor_on_device
 from . import generation
 from .graphs import DecodeGraphs
-from .memory import plan_memory
+from .memory import kept_logits_bytes, plan_memory
 from .step import StepEntry, StepError, StepStaging, build_step, cache_for_runs, check_entries
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "fp32": torch.float32}
@@ -91,6 +91,9 @@ class Engine:
             if memory_limit_bytes is not None and self.plan.total_bytes > memory_limit_bytes:
                 raise MemoryBudgetError(f"the engine needs {self.plan.total_bytes} bytes, the limit is "
                                         f"{memory_limit_bytes}:\n{self.plan.describe()}")
+            self.kept_logits_bytes = kept_logits_bytes(cache.max_slots, getattr(model, "vocab", 0))
+            if memory_limit_bytes is not None and self.plan.total_bytes + self.kept_logits_bytes > memory_limit_bytes:
+                self.kept_logits = None      # generation then shows a callback each step's logits before it starts the next
 
         if model is None:
             if model_dir is None:
@@ -150,7 +153,8 @@ class Engine:
         return self._last_selection
 
     def kept_logits(self, logits):
-        """`logits` in memory of their own, which no later step writes."""
+        """`logits` in memory of their own, which no later step writes.  None in an engine whose limit leaves no room for two such
+        matrices beside its plan (`kept_logits_bytes`)."""
         return logits.clone()
 
     # ---- the step function ----
@@ -217,7 +221,8 @@ class Engine:
                                    batch_size, control, on_logits)
 
     def memory_plan(self) -> str:
-        return f"{self.plan.describe()}\n{self.cache_plan.describe()}"
+        beside = f"logits kept for a callback while a step runs ahead of it, beside the plan: {self.kept_logits_bytes if self.kept_logits else 0} bytes"
+        return f"{self.plan.describe()}\n{beside}\n{self.cache_plan.describe()}"
 
 
 def entries_of_one_run(model) -> set:

@@ -58,6 +58,11 @@ def step_numbers_bytes(rows: int, seqs: int, kv_groups: int, table_width: int) -
     return _rounded(4 * (4 * rows + 5 * seqs + 1 + seqs + kv_groups * seqs * table_width))
 
 
+def kept_logits_bytes(max_slots: int, vocab: int) -> int:
+    """What generation holds where it shows a callback the logits of a step behind the next step's launch: those of both steps."""
+    return 2 * _rounded(int(max_slots) * int(vocab) * 4)
+
+
 def weights_as_kept(model, act_size: int, sizes) -> tuple:
     """(bytes of the weights as the engine keeps them, bytes of the largest transient while loading): a matrix
     that the kernel library regroups has its rows padded to whole blocks, and while it is stacked from its

@@ -175,3 +175,22 @@ def test_an_engine_refuses_arguments_that_cannot_be_meant(model_dirs):
                 dict(memory_limit_bytes=1.5), dict(dtype="float16")):
         with pytest.raises(ValueError):
             make_engine(folder, **bad)
+
+
+def test_logits_are_kept_for_a_callback_only_where_the_limit_has_room_for_them(model_dirs):
+    folder = model_dirs("A", "float32")
+    free = make_engine(folder, max_tokens=256, max_slots=3)
+    need = 2 * 3 * free.model.vocab * 4      # both steps' rows, on whole units of 512 bytes
+    assert need % 512 == 0 and f"beside the plan: {need} bytes" in free.memory_plan()
+    prompts = schedules.random_requests(256, [9, 4, 17], seed=3)
+    outcomes = []
+    for limit, ahead in ((None, True), (free.plan.total_bytes + need, True), (free.plan.total_bytes + need - 1, False), (free.plan.total_bytes, False)):
+        engine = make_engine(folder, max_tokens=256, max_slots=3, memory_limit_bytes=limit)
+        assert (engine.kept_logits is not None) is ahead and (f"beside the plan: {need if ahead else 0} bytes" in engine.memory_plan())
+        log, step = [], engine.step
+        engine.step = lambda entries, *rest: log.append("step") or step(entries, *rest)
+        seen = []
+        results = engine.generate(prompts, max_new_tokens=4, on_logits=lambda index, at, row: (log.append("seen"), seen.append((index, at, row.clone().numpy().tolist()))))
+        assert (log[:2] == ["step", "step"]) is ahead      # the next step's launch before this one's callback, or after it
+        outcomes.append(([r.token_ids for r in results], seen))
+    assert all(outcome == outcomes[0] for outcome in outcomes) and len(outcomes[0][1]) == 12
