@@ -559,12 +559,20 @@ static int gla_join(const GlaChunks& chunks, float* state, long slot_stride, con
 // Which steps share what is read between columns: long walks (a decode step is its state's way in and out) of which a compute unit has one at
 // least; below that a row's chain of steps is the time, and that of 16 elements a thread is the longer one (wkv, 64 heads of 64, 2,048 rows, us,
 // apart / in columns: 1,024 workgroups 273 / 128, 512 workgroups 266 / 195; one sequence of 100 rows, 64 heads, 64 workgroups 64 / 62; 32
-// heads, 128 workgroups 293 / 306; gla, 8 heads of 128, 64 workgroups 321 / 314; 20 heads of 48, 333 rows, 100 workgroups 59 / 70).
+// heads, 128 workgroups 293 / 306; gla, 8 heads of 128, 64 workgroups 321 / 314; 20 heads of 48, 333 rows, 100 workgroups 59 / 70).  At the line, 256
+// workgroups, sequences of 64 / of 127 rows: wkv, 4 of 64 heads of 64 50.2 / 36.0 and 93.5 / 63.6, gla the same 40.4 / 39.6 and 77.0 / 71.4, 8 of 16 heads
+// of 128 62.9 / 42.5 and 122.0 / 77.2; but gla, 8 of 64 heads of 64, 64 rows, 512 workgroups 50.1 / 52.0.
 #define GC_ROWS 64
 #define GC_C 2
 static bool gla_columns_take(long walks, int max_rows, int H, int dim, int vdim) {
   return max_rows >= GC_ROWS && dim % 4 == 0 && dim > 32 && dim <= 256 && vdim % 4 == 0 && vdim > 32 &&
          walks * H * ((vdim + 63) / 64) >= (long)bh_compute_units();
+}
+
+// For tests: whether a step of operands on 16 bytes, in rows of whole pieces of four, is walked in columns.
+extern "C" int bh_gla_in_columns(int n_seqs, int max_rows, int H, int dim, int vdim) {
+  const int rows = bh_gla_chunk_rows(n_seqs, max_rows, H, dim, vdim);
+  return gla_columns_take((long)n_seqs * ((max_rows + rows - 1) / rows), max_rows, H, dim, vdim);
 }
 
 template <int RULE, typename T>

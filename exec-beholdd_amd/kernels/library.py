@@ -242,6 +242,7 @@ class KernelSizes:
             "bh_experts_gather": [p, i, i, p, i, p, p, p, p, i, i, i, p, p],
             "bh_gla_scan": [p, i, i, i, i, i, p, i, p, f, f, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p],
             "bh_gla_chunk_rows": [i, i, i, i, i],
+            "bh_gla_in_columns": [i, i, i, i, i],
             "bh_wkv_scan": [p, p, p, i, i, p, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p],
             "bh_token_shift": [p, i, i, p, i, p, ctypes.c_long, p, p, p, p, p, i, i, i, p],
             "bh_tanh_rows": [p, i, p, i, i, i, i, p],

@@ -29,15 +29,20 @@ def gla_recurrence(q, k, v, a, state):
     return o, s
 
 
+APART = [(260, 34, 34), (3, 64, 64), (300, 64, 64), (130, 132, 44)]      # what stays with the other walk of the sizes below
+
+
 # the sizes of a column's lanes (up to 64, 128, 256 key dimensions), tiles that values do not fill, stages and chunks that end early, sequences of
 # one row beside long ones; columns that are no multiple of four, few workgroups and short sequences stay with the other walk
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rule", ["wkv", "gla"])
 @pytest.mark.parametrize("heads,dim,vdim,lengths", [(64, 64, 64, [300, 17, 1, 64]), (260, 36, 36, [65]), (70, 68, 100, [79, 3, 90]), (130, 132, 44, [70]), (64, 256, 260, [66]),
+                                                    (260, 132, 44, [70]), (16, 128, 128, [1000, 5]), (9, 256, 252, [1000]), (33, 100, 64, [300, 260]),      # the last three in chunks
                                                     (260, 34, 34, [65]), (3, 64, 64, [200]), (300, 64, 64, [63, 5])])
 def test_walks_in_columns(K, dtype, rule, heads, dim, vdim, lengths):
     if rule == "wkv":
         vdim = dim
+    assert bool(K.lib.bh_gla_in_columns(len(lengths), max(lengths), heads, dim, vdim)) is ((heads, dim, vdim) not in APART)
     rng = np.random.default_rng(heads * dim + vdim)
     n, kw, vw, slots = sum(lengths), heads * dim, heads * vdim, len(lengths) + 1
     order = [int(i) for i in rng.permutation(slots)[:len(lengths)]]

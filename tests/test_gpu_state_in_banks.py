@@ -72,6 +72,17 @@ def test_state_space(K, lengths, heads, vdim, n_state, groups):
 @pytest.mark.parametrize("lengths", LENGTHS)
 @pytest.mark.parametrize("heads,dim", [(4, 64), (2, 32)])
 def test_time_mixing_and_gated_linear_attention(K, lengths, heads, dim):
+    time_mixing_and_gated_linear_attention(K, lengths, heads, dim)
+
+
+# steps whose walks go two columns a thread, whole and in chunks, a column over 4, 8 and 16 lanes
+@pytest.mark.parametrize("heads,dim,lengths", [(64, 64, [300, 17, 1, 64]), (260, 36, [65]), (16, 128, [1000, 5]), (8, 256, [1000, 1]), (64, 256, [66])])
+def test_time_mixing_and_gated_linear_attention_in_columns(K, lengths, heads, dim):
+    assert K.lib.bh_gla_in_columns(len(lengths), max(lengths), heads, dim, dim)
+    time_mixing_and_gated_linear_attention(K, lengths, heads, dim)
+
+
+def time_mixing_and_gated_linear_attention(K, lengths, heads, dim):
     n, (starts, row_seq), width = sum(lengths), layout(lengths), heads * dim
     proj, z, bias, bonus = rows(n, 3 * width), rows(n, width, torch.float32, 2, 0.5), dev(torch.linspace(-3.0, 0.0, width)), dev(torch.linspace(0.0, 1.0, width))
     mu, parts = dev(torch.rand(5, width, generator=torch.Generator().manual_seed(3))), [rows(n, width, seed=s) for s in (4, 5, 6)]
