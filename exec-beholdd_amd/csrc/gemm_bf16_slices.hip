@@ -341,7 +341,8 @@ int gemm_slices_launch(const void* a, const void* w, float* sums, int M, int N, 
   }
   // Parts of 512 k that leave compute units idle: a second group of four waves takes half of a workgroup's k, and hands its sums over through
   // LDS.  Us with one group / with two, 64 rows: 2,560 x 2,560 (200 workgroups) 9.6 / 9.0, 2,048 x 2,048 (128) 8.9 / 8.3, 1,024 x 3,072 (96)
-  // 8.8 / 8.0; but 2,048 x 6,144 (384) 11.9 / 12.1, and at the chip's full number half as many parts of twice the waves lose, whose
+  // 8.8 / 8.0; with the finishing launch, 33 rows of 2,560 x 2,560 10.6 / 9.8, 1,024 x 1,024 9.5 / 9.0, 128 rows 14.8 / 14.3, 12.5 / 11.8 (33 to 128 rows of
+  // 512 to 4,096 outputs and k of 512 to 8,192: none slower); but 2,048 x 6,144 (384) 11.9 / 12.1, and at the chip's full number half as many parts of twice the waves lose, whose
   // eight waves meet at each stage: 4,096 x 4,096 13.5 / 15.1, 4,096 x 12,288 26.8 / 30.0.
   const int groups = (w_rows / 16 + WAVES - 1) / WAVES;
   const bool in_halves = (long)groups * parts <= bh_compute_units();

@@ -1,12 +1,12 @@
 // A short causal convolution over time on every channel of a slice of a projected matrix, continued from step to
 // step through a state that holds the last taps - 1 inputs of each sequence:
 //   y[t][c] = sum_j w[c][j] * u[t - taps + 1 + j][c]  (+ bias[c])  (then silu),   zeros before a sequence starts.
-//   short_conv        the rows of a step; inputs that lie before the step come from the state
-//   short_conv_state  the state after the step (run it after every reader of the old state), left in the rows seq_to, which may be
-//                     those it is read from
+//   short_conv        the rows of a step; inputs that lie before the step come from the state.  With seq_to the thread of a sequence's
+//                     last row leaves the state after the step in these rows, which no sequence of the step reads
+//   short_conv_state  the state after the step, otherwise (run it after every reader of the old state), left in the rows seq_to, which
+//                     may be those it is read from
 // State of one sequence: [taps - 1][channels] float32, the oldest input first, at `state + slot * slot_stride`.
 // Sums are float32; the result is float32.
-//                     A step that leaves it in other rows does so in short_conv itself (seq_to): the thread of a sequence's last row
 #include "short_conv.h"
 
 template <typename T>
@@ -94,7 +94,9 @@ __global__ __launch_bounds__(256) void short_conv_walk_kernel(const T* __restric
 
 // The same in pieces of four channels: a thread asks for all inputs of its stretch of SC_FAR rows together and waits for them once, where the
 // walk above has a load a row and its wait.  A stretch in which a sequence starts is walked row by row.  Bound by its bytes (the inputs once,
-// 3 in 19 of them twice, float32 outputs) and, with few waves a compute unit, the way to memory.  2,100 rows of 6,144 and of 3,072 channels, on average 32.9 -> 23.8 us.
+// 3 in 19 of them twice, float32 outputs) and, with few waves a compute unit, the way to memory.  2,100 rows of 6,144 and of 3,072 channels, on average 32.9 -> 23.8 us; 1,024 rows of 6,144
+// 21.5 / 16.5; at the fewest, 128 rows of 512 channels 11.9 / 10.6, of 6,144 12.8 / 11.3 (512 to 6,144 channels, bfloat16 and float32, one and eight
+// sequences: 0.92 of the walk's time at worst).
 #define SC_FAR 16
 
 template <typename T>

@@ -213,8 +213,9 @@ extern "C" int bh_whole_norm_rope_write(const float* qkv, const float* wq, const
 // The same from the projected rows themselves: the short convolution over time (csrc/short_conv.hip has its definition and
 // its state) is made on the way, a row's convolved channels stand in LDS as float32 and are never written to memory.
 // proj [n_rows][row_stride]: a row holds, from `first`, q, k and v; w_conv [q + k + v channels][taps] (taps 0: no convolution).
-// TAPS: four, whose loads are all asked for before the first is used, of a whole thread's channels where these are up to four (16 rows of 3,072
-// channels 9.8 us, 11.9 with a trip to memory a tap), or 0: any number.  seq_to: as in short_conv.hip.
+// TAPS: four, whose loads are all asked for before the first is used, of a whole thread's channels where these are up to four, or 0: any
+// number, a trip to memory a tap (us, so / asked for together, 24 heads of 128 and 8 of keys and values: one row 11.7 / 9.7, 16 rows 12.0 / 10.1, a prompt of
+// 127 13.4 / 10.6; 64 and 8, 127 rows 21.6 / 14.8; 4 of 64 and 2, 16 rows 6.7 / 6.0).  seq_to: as in short_conv.hip.
 template <typename T, int TAPS>
 __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
     const T* __restrict__ proj, int row_stride, int first, const float* __restrict__ w_conv, int taps, float* __restrict__ state,
@@ -285,22 +286,23 @@ __global__ __launch_bounds__(1024) void conv_norm_rope_write_kernel(
         }
       }
     }
-  } else
-  for (int c = threadIdx.x; c < channels; c += blockDim.x) {
-    float acc;
-    if (taps <= 1) {
-      acc = to_f32(proj[(size_t)row * row_stride + first + c]) * (taps ? w_conv[c] : 1.f);
-    } else {
-      acc = 0.f;
-      for (int j = 0; j < taps; ++j) {
-        const int back = taps - 1 - j;
-        const float u = back <= t ? to_f32(proj[(size_t)(row - back) * row_stride + first + c])
-                                  : old[(size_t)(taps - 1 + t - back) * channels + c];
-        acc = fmaf(w_conv[(size_t)c * taps + j], u, acc);
+  } else {
+    for (int c = threadIdx.x; c < channels; c += blockDim.x) {
+      float acc;
+      if (taps <= 1) {
+        acc = to_f32(proj[(size_t)row * row_stride + first + c]) * (taps ? w_conv[c] : 1.f);
+      } else {
+        acc = 0.f;
+        for (int j = 0; j < taps; ++j) {
+          const int back = taps - 1 - j;
+          const float u = back <= t ? to_f32(proj[(size_t)(row - back) * row_stride + first + c])
+                                    : old[(size_t)(taps - 1 + t - back) * channels + c];
+          acc = fmaf(w_conv[(size_t)c * taps + j], u, acc);
+        }
       }
+      put(c, acc);
+      if (leaves) sc_leave_inputs(proj, row_stride, first + c, row - t, t + 1, taps, old, left, channels, c);
     }
-    put(c, acc);
-    if (leaves) sc_leave_inputs(proj, row_stride, first + c, row - t, t + 1, taps, old, left, channels, c);
   }
   const float inv_q = 1.0f / sqrtf(block_sum(ss_q, scratch) / (float)q_width + eps);
   const float inv_k = 1.0f / sqrtf(block_sum(ss_k, scratch) / (float)k_width + eps);

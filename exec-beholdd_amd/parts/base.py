@@ -38,10 +38,12 @@ A matrix that one product alone reads may be kept the way that product reads it 
     norm with `serves_reader = True`: forward(..., reader=) and request(reader) take that ProductReader.
     Inside a part, `ctx.new_activations(rows, width, reader=linear.reader())` asks for such a matrix between two
     of its own kernel calls.  Parts that say nothing get and give plain matrices.
-A mixer with a "state" cache need updates its rows of `cache.state` in place while it runs.  The cache keeps
-what the step's sequences held before the step and puts it back if the step fails, so a mixer needs no
-second bank; and the engine runs a part's forward exactly once per step, whether the step is launched kernel
-by kernel or replayed from a capture, so a state advances once per token.
+A mixer with a "state" cache need moves its rows of `cache.state` on while it runs: in place, at the rows `ctx.seq_slot`
+names, and the cache, which keeps what the step's sequences held before the step, puts it back if the step fails.  A mixer
+whose need says `in_banks` takes the rows from `cache.state_rows(ctx)` instead: those to read, and those to leave the whole
+state in, which are others where the cache keeps two rows a slot and no copy (what a failed step has left there does not
+count), and the same ones where it does not.  Either way the engine runs a part's forward exactly once per step, whether the
+step is launched kernel by kernel or replayed from a capture, so a state advances once per token.
 Every part may say what its forward allocates: working_bytes(step: StepSize) -> int, from sizes alone; the
 engine's byte plan adds them up before anything is allocated and names the parts that do not say.
 A part may declare `graph_safe = True`: its forward uses only the device tensors of the step
@@ -213,7 +215,8 @@ class LayerCache:
                 page_size], to be written and read through the kernel library only (it orders the
                 elements of a head inside a page as its attention kernels want them); page_table
                 int32 [n_seqs, width] for the sequences of this step, in batch order.
-    state need: state [max_slots, *state_shape]; index it with ctx.seq_slot.  A kv need with a state shape has both.
+    state need: state [max_slots, *state_shape]; index it with ctx.seq_slot, or, where the need says `in_banks`, with
+                `state_rows(ctx)` (if `banked`, there are 2 max_slots rows).  A kv need with a state shape has both.
     `writes` is False when the schedule lets this layer read another layer's entry.
     """
     need: CacheNeed

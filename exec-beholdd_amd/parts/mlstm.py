@@ -66,6 +66,7 @@ class MatrixMemory:
         self.out.prepare(kernels)
 
     def cache_need(self):
+        # (not in banks: its kernels leave the state in the row they read it from, behind the copy that the cache makes)
         return CacheNeed(kind="state", state_shape=(self.state_floats,), state_dtype=torch.float32)
 
     def working_bytes(self, step) -> int:
